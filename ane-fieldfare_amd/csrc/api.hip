@@ -78,6 +78,7 @@ struct ffmoe_ctx {
     // the 8-bit dense layers' GEMM form: the library handle and the fp32 sums [max_tokens][max(4 f, 2 d)]
     rocblas_handle blas = nullptr;
     float *gemm8_sums = nullptr;
+    SampleScratch sample{};          // what the sampled choice over long rows leaves between its two launches
     KernelTimer timer;
     std::vector<ffmoe_matrix *> matrices;   // resident matrices created on this context and not yet destroyed
     // the stream the scratch was last used on, and the event a call on another stream waits for (claim_scratch)
@@ -313,6 +314,8 @@ int ffmoe_create(int device, const ffmoe_shape *shape, ffmoe_ctx **out, char **e
                       ((size_t)ctx->max_pairs / 16 + ctx->pf.max_tiles + 2) * 16 * shape->f * sizeof(uint16_t));
     ctx->pf.act_blocks = ctx->max_pairs / 16 + ctx->pf.max_tiles + 2;
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&ctx->pf.partials), (size_t)ctx->max_pairs * shape->d * sizeof(uint16_t));
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&ctx->sample.group_keys), (size_t)FFMOE_MAX_VERIFY_ROWS * kSampleMaxGroups * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&ctx->sample.segments), (size_t)FFMOE_MAX_VERIFY_ROWS * kSampleMaxSegments * sizeof(SampleSegment));
     if (e == hipSuccess && shape->n_experts == 1 && shape->top_k == 1) {
         e = hipMalloc(reinterpret_cast<void **>(&ctx->dense_idx), (size_t)router_rows * sizeof(uint32_t));
         if (e == hipSuccess) e = hipMemset(ctx->dense_idx, 0, (size_t)router_rows * sizeof(uint32_t));
@@ -357,6 +360,8 @@ void ffmoe_destroy(ffmoe_ctx *ctx) {
     if (ctx->pf.acts) (void)hipFree(ctx->pf.acts);
     if (ctx->pf.partials) (void)hipFree(ctx->pf.partials);
     if (ctx->pf.act_scale) (void)hipFree(ctx->pf.act_scale);
+    if (ctx->sample.group_keys) (void)hipFree(ctx->sample.group_keys);
+    if (ctx->sample.segments) (void)hipFree(ctx->sample.segments);
     if (ctx->dense_idx) (void)hipFree(ctx->dense_idx);
     if (ctx->dense_w) (void)hipFree(ctx->dense_w);
     // matrices that outlive their context lose their device memory here; the handles stay valid to destroy
@@ -429,8 +434,9 @@ int ffmoe_sample_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_
         return fail(err, FFMOE_ERR_INVALID, "the sampled choice caps its logits: softcap must be positive and finite");
     if (rule->top_k > 256) return fail(err, FFMOE_ERR_INVALID, "top_k = %u outside 0...256", rule->top_k);
     if (rule->top_k && !(rule->top_p > 0.0f && rule->top_p <= 1.0f)) return fail(err, FFMOE_ERR_INVALID, "top_p outside (0, 1]");
+    claim_scratch(ctx, stream);
     FF_HIP(launch_sample_rows(static_cast<hipStream_t>(stream), logits, stride, rows, count, ids, rule->temperature, rule->top_p,
-                              rule->top_k, rule->key_base, rule->softcap, rule->seed, key_offset, out_tokens, out_prob));
+                              rule->top_k, rule->key_base, rule->softcap, rule->seed, key_offset, out_tokens, out_prob, ctx->sample));
     return FFMOE_OK;
 }
 

@@ -186,6 +186,21 @@ hipError_t launch_probe_stream(hipStream_t s, const uint8_t *arena_layer, ArenaG
 hipError_t launch_reduce_token_major(hipStream_t s, const uint16_t *partials, const uint16_t *weights,
                                      uint16_t *h2, uint32_t t, uint32_t top_k, uint32_t d, bool f16 = false);
 
+// What a sweep over long rows of fp32 logits by many blocks leaves for the launch that finishes the rows (the sampled and
+// the greedy choice: sample.hip, matrix.hip), per row: every 64-wide group's largest value (the truncated draw) and, per
+// block of kSampleSegment logits, its sums and its winner.
+constexpr uint32_t kSampleGroup = 64, kSampleSegment = 2048, kSampleMaxGroups = 8192;
+constexpr uint32_t kSampleMaxSegments = kSampleMaxGroups * kSampleGroup / kSampleSegment;
+struct SampleSegment {
+    unsigned long long best;
+    float top, sum;
+    uint32_t finite, pad;
+};
+struct SampleScratch {
+    uint32_t *group_keys = nullptr;      // [16][kSampleMaxGroups]
+    SampleSegment *segments = nullptr;   // [16][kSampleMaxSegments]
+};
+
 // matrix.hip: resident two-stream tiling of a [M][N] INT4 matrix, its multi-row GEMV and the greedy choice.
 // planes8: the weight is an 8-bit affine one, kept as two nibble planes per 16-row tile (csrc/matrix.hip)
 size_t matrix_tiles_bytes(uint32_t m, uint32_t n, bool planes8 = false);
@@ -254,6 +269,6 @@ hipError_t launch_gemv_int4(hipStream_t s, const uint8_t *w, const uint16_t *sca
 hipError_t launch_sample_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                               const uint32_t *ids, float temperature, float top_p, uint32_t top_k, uint32_t key_base,
                               float softcap, unsigned long long seed, const uint32_t *key_offset, uint32_t *out_tokens,
-                              float *out_prob);
+                              float *out_prob, SampleScratch sc);
 
 }  // namespace ffmoe

@@ -7,14 +7,22 @@
 // logits (ties to the lower index), of those the shortest prefix whose T = 1 probability mass reaches top_p, then
 // the draw at temperature T over the survivors.
 //
-// One block of 1,024 threads per row (a row is up to 262,144 logits: 1 MiB, which stays in the XCD's L2 across the
-// sweeps). Without truncation: two sweeps (the largest capped logit; the draw and the normaliser). With it the k-th
-// largest is found EXACTLY by a radix select over the order-preserving integer image of the capped logits - three
-// sweeps with LDS histograms of 11, 11 and 10 bits - instead of a histogram over the value range whose edge bin has to
-// fit a candidate buffer; a fourth sweep gathers the values above the threshold (any order: they are ranked
-// afterwards) and, of the values equal to it, the lowest indices (in index order, wave by wave). The <= 256
-// candidates are ranked by counting, thread 0 walks the top_p prefix, and the survivors draw.
+// Two forms with the same survivors. Long rows (use_scan below) take two launches: blocks of 2,048 logits sweep the row
+// ONCE - one wave per 64 logits leaves their largest capped value, a block its share of the normaliser (or, without
+// truncation, its own winner of the draw) - and one block per row finishes from those: the want-th largest of the 64-wide
+// groups' maxima is a lower bound of the want-th largest logit, only groups that reach it can hold a survivor, and
+// what those hold above the bound (a few hundred logits) is ranked exactly. One row of 262,144 logits, top_k = 64: 375 us as
+// one block's five sweeps (tanhf per logit and sweep, and LDS histograms whose few occupied bins serialise the
+// atomics) -> 17 us; sixteen rows without truncation 20 us.
+// Short rows, and rows whose groups tie at the bound in numbers that overflow the candidate lists, take one block of
+// 1,024 threads per row. Without truncation: two sweeps (the largest capped logit; the draw and the normaliser). With it
+// the k-th largest is found EXACTLY by a radix select over the order-preserving integer image of the capped logits -
+// three sweeps with LDS histograms of 11, 11 and 10 bits; a fourth sweep gathers the values above the threshold (any
+// order: they are ranked afterwards) and, of the values equal to it, the lowest indices (in index order, wave by wave).
+// The <= 256 candidates are ranked by counting, thread 0 walks the top_p prefix, and the survivors draw.
 #include <hip/hip_runtime.h>
+
+#include <cfloat>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -63,9 +71,7 @@ struct SampleShared {
     uint32_t wave_eq_n[kSampleWaves];
     float cand_v[kSampleMaxK], sorted_v[kSampleMaxK];
     uint32_t cand_i[kSampleMaxK], sorted_i[kSampleMaxK];
-    uint32_t n_above, bin, above, keep;
-    float f0;
-    unsigned long long k0;
+    uint32_t n_above, bin, above;
 };
 
 __device__ __forceinline__ float block_max_f(float v, SampleShared &sh) {
@@ -88,6 +94,25 @@ __device__ __forceinline__ float block_sum_f(float v, SampleShared &sh) {
     __syncthreads();
     float r = 0.0f;
     for (int w = 0; w < kSampleWaves; ++w) r += sh.red_f[w];
+    return r;
+}
+
+// two sums side by side
+__device__ __forceinline__ float2 block_sum_f2(float2 v, SampleShared &sh) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        v.x += __shfl_xor(v.x, o, 64);
+        v.y += __shfl_xor(v.y, o, 64);
+    }
+    float2 *red = reinterpret_cast<float2 *>(sh.red_k);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float2 r = make_float2(0.0f, 0.0f);
+    for (int w = 0; w < kSampleWaves; ++w) {
+        r.x += red[w].x;
+        r.y += red[w].y;
+    }
     return r;
 }
 
@@ -139,15 +164,101 @@ __device__ __forceinline__ void find_bin(SampleShared &sh, uint32_t bins, uint32
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t count,
-                                                                     const uint32_t *__restrict__ ids, SampleRule p,
-                                                                     const uint32_t *__restrict__ key_offset,
-                                                                     uint32_t *__restrict__ out_tokens, float *__restrict__ out_prob) {
-    __shared__ SampleShared sh;
-    const uint32_t r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float *row = logits + (size_t)r * stride;
+// The end of a truncated draw, called by the whole block: sh.sorted_v / sorted_i hold the n largest in order. The top_p prefix
+// over the T = 1 distribution within the top k (logit.metal:1213-1224; `total1` = the normaliser over the whole row), then
+// the draw at temperature T over the survivors. Wave 0 does it alone, four ranks per lane: no barrier in the chain.
+__device__ __forceinline__ void sample_finish(SampleShared &sh, const SampleRule &p, uint32_t n, float total1, unsigned long long seed,
+                                              uint32_t key, const uint32_t *__restrict__ ids, uint32_t *__restrict__ out_token,
+                                              float *__restrict__ out_prob) {
+    constexpr int kSlots = kSampleMaxK / 64;
+    const float invT = 1.0f / p.temperature;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const uint32_t lane = threadIdx.x;
+    float v[kSlots];                                            // lane l, slot u: rank 64 u + l
+    uint32_t at[kSlots];
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+        const uint32_t rank = min(64u * u + lane, n - 1);
+        v[u] = sh.sorted_v[rank];
+        at[u] = sh.sorted_i[rank];
+    }
+    const float top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(v[0])));
+    float share[kSlots], incl[kSlots];
+    float so_far = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+        share[u] = 64u * u + lane < n ? expf(v[u] - p.softcap) / total1 : 0.0f;
+        incl[u] = share[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+        if (64u * u >= n) break;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const float up = __shfl_up(incl[u], o, 64);
+            if (lane >= (uint32_t)o) incl[u] += up;
+        }
+        incl[u] += so_far;
+        so_far = __shfl(incl[u], 63, 64);
+    }
+    // The prefix is defined by the running sum that takes the shares one after the other. Two orders of adding <= 256
+    // positive shares that add to at most about 1 differ by less than 256 * 2^-24 * 2: where no prefix sum comes closer to
+    // top_p than that, the scan decides; else (equal logits whose shares meet top_p exactly) the sum itself runs.
+    constexpr float kClose = 4e-5f;
+    uint32_t keep = n;
+    bool close = false;
+#pragma unroll
+    for (int u = kSlots - 1; u >= 0; --u) {
+        if (64u * u >= n) continue;
+        const bool in = 64u * u + lane < n;
+        const unsigned long long over = __ballot(in && incl[u] >= p.top_p);
+        close = close || __ballot(in && fabsf(incl[u] - p.top_p) < kClose) != 0ull;
+        if (over) keep = 64u * u + (uint32_t)__builtin_ctzll(over) + 1;
+    }
+    if (close) {
+        keep = n;
+        float cum = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u)
+            for (uint32_t l = 0; l < 64 && 64u * u + l < n && keep == n; ++l) {
+                cum += __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(share[u]), (int)l));
+                if (cum >= p.top_p) keep = min(n, 64u * u + l + 1);
+            }
+    }
+    unsigned long long best = 0ull;
+    float esum = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+        if (64u * u >= keep) break;
+        const uint32_t rank = 64u * u + lane;
+        float e = 0.0f;
+        unsigned long long mine = 0ull;
+        if (rank < keep) {
+            e = expf((v[u] - top) * invT);
+            mine = ((unsigned long long)sample_key(v[u] * invT + sample_gumbel(seed, key, ids ? ids[at[u]] : at[u])) << 32) | (0xFFFFFFFFu - rank);
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            e += __shfl_xor(e, o, 64);
+            const unsigned long long other = __shfl_xor(mine, o, 64);
+            mine = other > mine ? other : mine;
+        }
+        esum += e;
+        best = mine > best ? mine : best;
+    }
+    if (lane == 0) {
+        const uint32_t bj = 0xFFFFFFFFu - (uint32_t)best;
+        *out_token = sh.sorted_i[bj];
+        *out_prob = expf((sh.sorted_v[bj] - top) * invT) / esum;
+    }
+}
+
+// One row by one block of kSampleThreads threads, whatever it holds.
+__device__ void sample_one_row(SampleShared &sh, const float *__restrict__ row, uint32_t count, const uint32_t *__restrict__ ids,
+                               const SampleRule &p, uint32_t key, uint32_t *__restrict__ out_token, float *__restrict__ out_prob) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float cap = p.softcap, invT = 1.0f / p.temperature;
-    const uint32_t key = p.key_base + (key_offset ? key_offset[0] : 0u) + r;
     const unsigned long long seed = ((unsigned long long)p.seed_hi << 32) | p.seed_lo;
     const bool truncated = p.top_k > 0u && p.top_k < count;
     auto token_of = [&](uint32_t i) { return ids ? ids[i] : i; };
@@ -170,8 +281,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float
         const float total = block_sum_f(sum, sh);
         if (tid == 0) {
             const uint32_t j = best ? 0xFFFFFFFFu - (uint32_t)best : 0xFFFFFFFFu;
-            out_tokens[r] = j;
-            out_prob[r] = (j == 0xFFFFFFFFu || !(total > 0.0f)) ? 0.0f : expf((sample_capped(row[j], cap) - m) * invT) / total;
+            *out_token = j;
+            *out_prob = (j == 0xFFFFFFFFu || !(total > 0.0f)) ? 0.0f : expf((sample_capped(row[j], cap) - m) * invT) / total;
         }
         return;
     }
@@ -195,8 +306,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float
     const uint32_t finite = (uint32_t)block_sum_f((float)n_finite, sh);      // counts up to 2^18 per row: exact in fp32
     if (finite == 0) {
         if (tid == 0) {
-            out_tokens[r] = 0xFFFFFFFFu;
-            out_prob[r] = 0.0f;
+            *out_token = 0xFFFFFFFFu;
+            *out_prob = 0.0f;
         }
         return;
     }
@@ -278,35 +389,296 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float
         sh.sorted_i[rank] = i;
     }
     __syncthreads();
-    // ---- top_p over the T = 1 distribution within the top k (logit.metal:1213-1224) ---------------------------
-    if (tid == 0) {
-        float cum = 0.0f;
-        uint32_t keep = 0;
-        while (keep < n) {
-            cum += expf(sh.sorted_v[keep] - cap) / total1;
-            keep += 1;
-            if (cum >= p.top_p) break;
+    sample_finish(sh, p, n, total1, seed, key, ids, out_token, out_prob);
+}
+
+__device__ __forceinline__ uint32_t sample_position_key(const SampleRule &p, const uint32_t *__restrict__ key_offset, uint32_t r) {
+    return p.key_base + (key_offset ? key_offset[0] : 0u) + r;
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t count,
+                                                                     const uint32_t *__restrict__ ids, SampleRule p,
+                                                                     const uint32_t *__restrict__ key_offset,
+                                                                     uint32_t *__restrict__ out_tokens, float *__restrict__ out_prob) {
+    __shared__ SampleShared sh;
+    const uint32_t r = blockIdx.x;
+    sample_one_row(sh, logits + (size_t)r * stride, count, ids, p, sample_position_key(p, key_offset, r), out_tokens + r, out_prob + r);
+}
+
+// ---- long rows: one sweep by many blocks, then one block per row -------------------------------------------------
+// Bound: the sweep is instruction issue (one tanhf and one expf, or the noise's two logf and 64-bit products, per logit),
+// spread over 128 blocks per full-vocabulary row; the second launch is a chain of LDS round trips.
+static_assert(kSampleMaxSegments <= kSampleThreads, "the finishing launches bring one segment per thread");
+constexpr int kScanThreads = 256, kScanPer = kSampleSegment / kScanThreads;
+static_assert(kSampleSegment % kScanThreads == 0 && kSampleGroup == 64, "a wave's load is one group");
+
+// TRUNCATED: every 64-wide group's largest capped logit as its key (0: nothing finite) and the block's share of the
+// T = 1 normaliser. Else: the block's largest capped logit, its tempered sum relative to that and its winner of the draw.
+template <bool TRUNCATED>
+__global__ __launch_bounds__(kScanThreads) void sample_scan_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t count,
+                                                                   const uint32_t *__restrict__ ids, SampleRule p,
+                                                                   const uint32_t *__restrict__ key_offset, SampleScratch sc) {
+    __shared__ float s_f[kScanThreads / 64];
+    __shared__ uint32_t s_n[kScanThreads / 64];
+    __shared__ unsigned long long s_k[kScanThreads / 64];
+    const uint32_t r = blockIdx.y, seg = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float *row = logits + (size_t)r * stride;
+    const float cap = p.softcap;
+    float c[kScanPer];
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) {
+        const uint32_t i = seg * kSampleSegment + u * kScanThreads + tid;
+        c[u] = i < count ? row[i] : -INFINITY;
+    }
+#pragma unroll
+    for (int u = 0; u < kScanPer; ++u) c[u] = sample_capped(c[u], cap);
+    if constexpr (TRUNCATED) {
+        float sum = 0.0f;
+        uint32_t finite = 0;
+        float top[kScanPer];
+#pragma unroll
+        for (int u = 0; u < kScanPer; ++u) {
+            top[u] = c[u];
+            if (c[u] != -INFINITY) {
+                sum += expf(c[u] - cap);
+                ++finite;
+            }
         }
-        sh.keep = max(keep, 1u);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+            for (int u = 0; u < kScanPer; ++u) top[u] = fmaxf(top[u], __shfl_xor(top[u], o, 64));
+            sum += __shfl_xor(sum, o, 64);
+            finite += (uint32_t)__shfl_xor((int)finite, o, 64);
+        }
+        uint32_t *keys = sc.group_keys + (size_t)r * kSampleMaxGroups + seg * (kSampleSegment / kSampleGroup);
+#pragma unroll
+        for (int u = 0; u < kScanPer; ++u)
+            if (lane == 0) keys[u * (kScanThreads / 64) + wave] = top[u] == -INFINITY ? 0u : sample_key(top[u]);
+        if (lane == 0) {
+            s_f[wave] = sum;
+            s_n[wave] = finite;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            SampleSegment out{};
+            for (int w = 0; w < kScanThreads / 64; ++w) {
+                out.sum += s_f[w];
+                out.finite += s_n[w];
+            }
+            sc.segments[(size_t)r * kSampleMaxSegments + seg] = out;
+        }
+    } else {
+        const float invT = 1.0f / p.temperature;
+        const uint32_t key = sample_position_key(p, key_offset, r);
+        const unsigned long long seed = ((unsigned long long)p.seed_hi << 32) | p.seed_lo;
+        float m = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < kScanPer; ++u) m = fmaxf(m, c[u]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        if (lane == 0) s_f[wave] = m;
+        __syncthreads();
+        for (int w = 0; w < kScanThreads / 64; ++w) m = fmaxf(m, s_f[w]);
+        __syncthreads();
+        float sum = 0.0f;
+        unsigned long long best = 0ull;
+#pragma unroll
+        for (int u = 0; u < kScanPer; ++u) {
+            if (c[u] == -INFINITY) continue;
+            const uint32_t i = seg * kSampleSegment + u * kScanThreads + tid;
+            sum += expf((c[u] - m) * invT);
+            const float g = c[u] * invT + sample_gumbel(seed, key, ids ? ids[i] : i);
+            const unsigned long long k = ((unsigned long long)sample_key(g) << 32) | (0xFFFFFFFFu - i);
+            best = k > best ? k : best;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            sum += __shfl_xor(sum, o, 64);
+            const unsigned long long other = __shfl_xor(best, o, 64);
+            best = other > best ? other : best;
+        }
+        if (lane == 0) {
+            s_f[wave] = sum;
+            s_k[wave] = best;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            SampleSegment out{};
+            out.top = m;
+            for (int w = 0; w < kScanThreads / 64; ++w) {
+                out.sum += s_f[w];
+                out.best = s_k[w] > out.best ? s_k[w] : out.best;
+            }
+            sc.segments[(size_t)r * kSampleMaxSegments + seg] = out;
+        }
+    }
+}
+
+// Without truncation: the segments' winners and sums merged, one block per row.
+__global__ __launch_bounds__(kSampleThreads) void sample_merge_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t n_seg,
+                                                                          SampleRule p, SampleScratch sc, uint32_t *__restrict__ out_tokens,
+                                                                          float *__restrict__ out_prob) {
+    __shared__ SampleShared sh;
+    const uint32_t r = blockIdx.x, tid = threadIdx.x;
+    const float invT = 1.0f / p.temperature;
+    SampleSegment mine{};
+    mine.top = -INFINITY;
+    if (tid < n_seg) mine = sc.segments[(size_t)r * kSampleMaxSegments + tid];
+    const float m = block_max_f(mine.top, sh);
+    const float total = block_sum_f(mine.best ? mine.sum * expf((mine.top - m) * invT) : 0.0f, sh);
+    const unsigned long long best = block_max_k(mine.best, sh);
+    if (tid == 0) {
+        const uint32_t j = best ? 0xFFFFFFFFu - (uint32_t)best : 0xFFFFFFFFu;
+        out_tokens[r] = j;
+        out_prob[r] = (j == 0xFFFFFFFFu || !(total > 0.0f)) ? 0.0f
+                                                            : expf((sample_capped(logits[(size_t)r * stride + j], p.softcap) - m) * invT) / total;
+    }
+}
+
+// With truncation: the bound from the groups' maxima, the candidates of the groups that reach it, the exact ranking.
+constexpr int kPickSlots = kSampleMaxGroups / kSampleThreads;
+constexpr uint32_t kPickMaxGroups = 1024, kPickMaxCands = 1024;
+
+__global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t count,
+                                                                     uint32_t n_seg, const uint32_t *__restrict__ ids, SampleRule p,
+                                                                     const uint32_t *__restrict__ key_offset, SampleScratch sc,
+                                                                     uint32_t *__restrict__ out_tokens, float *__restrict__ out_prob) {
+    __shared__ SampleShared sh;
+    __shared__ __align__(16) unsigned long long cand[kPickMaxCands];          // key << 32 | ~index: larger value first, then lower index
+    __shared__ uint32_t group_list[kPickMaxGroups];
+    __shared__ uint32_t n_list, n_cand;
+    const uint32_t r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float *row = logits + (size_t)r * stride;
+    const uint32_t n_groups = n_seg * (kSampleSegment / kSampleGroup);       // groups past the row's end hold key 0
+    uint32_t keys[kPickSlots];
+#pragma unroll
+    for (int s = 0; s < kPickSlots; ++s) {
+        const uint32_t g = s * kSampleThreads + tid;
+        keys[s] = g < n_groups ? sc.group_keys[(size_t)r * kSampleMaxGroups + g] : 0u;
+    }
+    SampleSegment mine{};
+    if (tid < n_seg) mine = sc.segments[(size_t)r * kSampleMaxSegments + tid];
+    if (tid == 0) n_list = n_cand = 0;
+    cand[tid] = 0ull;
+    const float2 sums = block_sum_f2(make_float2(mine.sum, (float)mine.finite), sh);
+    const float total1 = sums.x;
+    const uint32_t finite = (uint32_t)sums.y;                    // at most 2^19: exact in fp32
+    if (finite == 0) {
+        if (tid == 0) {
+            out_tokens[r] = 0xFFFFFFFFu;
+            out_prob[r] = 0.0f;
+        }
+        return;
+    }
+    const uint32_t want = min(p.top_k, finite);
+    // A bound that at least `want` groups reach, found by wave 0 on the threads' largest keys (a lower bound of the groups'
+    // own want-th largest), bit by bit from the top until it leaves out most of the others.
+    uint32_t most = 0;
+#pragma unroll
+    for (int s = 0; s < kPickSlots; ++s) most = max(most, keys[s]);
+    sh.hist[tid] = most;
+    __syncthreads();
+    if (wave == 0) {
+        uint32_t held[kSampleWaves];
+#pragma unroll
+        for (int s = 0; s < kSampleWaves; ++s) held[s] = sh.hist[64 * s + lane];
+        uint32_t low = 0, reach = kSampleThreads;
+#pragma unroll 1
+        for (int bit = 31; bit >= 0 && reach > want + want / 2; --bit) {
+            const uint32_t at = low | (1u << bit);
+            uint32_t c = 0;
+#pragma unroll
+            for (int s = 0; s < kSampleWaves; ++s) c += __popcll(__ballot(held[s] >= at));
+            if (c >= want) low = at, reach = c;
+        }
+        if (lane == 0) sh.bin = max(low, 1u);      // fewer finite groups than `want`: every finite logit is a candidate
     }
     __syncthreads();
-    const uint32_t keep = sh.keep;
-    // ---- the draw over the survivors --------------------------------------------------------------------------
-    unsigned long long best = 0ull;
-    float e = 0.0f;
-    if (tid < keep) {
-        const float v = sh.sorted_v[tid];
-        const float g = v * invT + sample_gumbel(seed, key, token_of(sh.sorted_i[tid]));
-        e = expf((v - sh.sorted_v[0]) * invT);
-        best = ((unsigned long long)sample_key(g) << 32) | (0xFFFFFFFFu - tid);
+    const uint32_t bound = sh.bin;
+    const uint32_t key = sample_position_key(p, key_offset, r);
+    // The candidates are first told apart by their raw value: `raw_low` is below every logit whose capped value reaches the
+    // bound (the inverse of the cap at the bound less a few thousand times tanhf's error), so that the cap itself is
+    // computed once per candidate and not for the other 63 logits of its group.
+    float raw_low = -FLT_MAX;
+    if (bound > 1u) {
+        const float at = __uint_as_float((bound & 0x80000000u) ? (bound & 0x7FFFFFFFu) : ~bound) / p.softcap;
+        const float z = fminf(at - 1e-4f * fabsf(at) - 1e-6f, 0.9999f);
+        if (z > -0.9999f) raw_low = p.softcap * atanhf(z);
     }
-    best = block_max_k(best, sh);
-    const float esum = block_sum_f(e, sh);
-    if (tid == 0) {
-        const uint32_t bj = 0xFFFFFFFFu - (uint32_t)best;
-        out_tokens[r] = sh.sorted_i[bj];
-        out_prob[r] = expf((sh.sorted_v[bj] - sh.sorted_v[0]) * invT) / esum;
+#pragma unroll
+    for (int s = 0; s < kPickSlots; ++s) {
+        const unsigned long long mask = __ballot(keys[s] >= bound);
+        if (mask == 0ull) continue;
+        uint32_t first = 0;
+        if (lane == 0) first = atomicAdd(&n_list, (uint32_t)__popcll(mask));
+        first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+        if (keys[s] >= bound && first < kPickMaxGroups) group_list[first] = s * kSampleThreads + tid;
     }
+    __syncthreads();
+    const uint32_t listed = n_list;
+    bool fits = listed <= kPickMaxGroups;
+    if (fits) {
+        constexpr int kAhead = 8;
+        for (uint32_t base = wave; base < listed; base += kAhead * kSampleWaves) {
+            float v[kAhead];
+            uint32_t at[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const uint32_t li = base + u * kSampleWaves;
+                at[u] = li < listed ? group_list[li] * kSampleGroup + lane : 0xFFFFFFFFu;
+                v[u] = at[u] < count ? row[at[u]] : NAN;
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const bool take = v[u] >= raw_low && v[u] <= FLT_MAX;
+                const unsigned long long mask = __ballot(take);
+                if (mask == 0ull) continue;
+                uint32_t first = 0;
+                if (lane == 0) first = atomicAdd(&n_cand, (uint32_t)__popcll(mask));
+                first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+                if (take && first < kPickMaxCands) cand[first] = ((unsigned long long)__float_as_uint(v[u]) << 32) | (0xFFFFFFFFu - at[u]);
+            }
+        }
+        __syncthreads();
+        fits = fits && n_cand <= kPickMaxCands;
+    }
+    if (!fits) {      // more ties at the bound than the lists hold
+        __syncthreads();
+        sample_one_row(sh, row, count, ids, p, key, out_tokens + r, out_prob + r);
+        return;
+    }
+    const uint32_t n = n_cand;
+    static_assert(kPickMaxCands == (uint32_t)kSampleThreads && kPickMaxCands % 4 == 0, "one candidate per thread");
+    if (tid < n) {
+        const unsigned long long raw = cand[tid];
+        const uint32_t q = sample_key(sample_capped(__uint_as_float((uint32_t)(raw >> 32)), p.softcap));
+        cand[tid] = q >= bound ? ((unsigned long long)q << 32) | (uint32_t)raw : 0ull;
+    }
+    // rank by counting: the threads of a candidate share the comparisons, four keys per read (all keys differ: they carry
+    // the index; the list ends in zeros)
+    const uint32_t parts = max(1u, (uint32_t)kSampleThreads / n), per = ((n + parts - 1) / parts + 3) & ~3u;
+    uint32_t *rank_of = sh.hist;
+    if (tid < n) rank_of[tid] = 0;
+    __syncthreads();
+    const uint32_t ci = tid % n, part = tid / n;
+    if (part < parts) {
+        const unsigned long long own = cand[ci];
+        uint32_t rank = 0;
+        for (uint32_t u = part * per; u < min(n, (part + 1) * per); u += 4) {
+            const ulonglong2 a = *reinterpret_cast<const ulonglong2 *>(&cand[u]), b = *reinterpret_cast<const ulonglong2 *>(&cand[u + 2]);
+            rank += (a.x > own ? 1u : 0u) + (a.y > own ? 1u : 0u) + (b.x > own ? 1u : 0u) + (b.y > own ? 1u : 0u);
+        }
+        if (rank) atomicAdd(&rank_of[ci], rank);
+    }
+    __syncthreads();
+    if (tid < n && rank_of[tid] < want && cand[tid]) {
+        const unsigned long long own = cand[tid];
+        const uint32_t q = (uint32_t)(own >> 32), rank = rank_of[tid];
+        sh.sorted_v[rank] = __uint_as_float((q & 0x80000000u) ? (q & 0x7FFFFFFFu) : ~q);
+        sh.sorted_i[rank] = 0xFFFFFFFFu - (uint32_t)own;
+    }
+    sample_finish(sh, p, want, total1, ((unsigned long long)p.seed_hi << 32) | p.seed_lo, key, ids, out_tokens + r, out_prob + r);
 }
 
 }  // namespace
@@ -314,8 +686,26 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float
 hipError_t launch_sample_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                               const uint32_t *ids, float temperature, float top_p, uint32_t top_k, uint32_t key_base,
                               float softcap, unsigned long long seed, const uint32_t *key_offset, uint32_t *out_tokens,
-                              float *out_prob) {
+                              float *out_prob, SampleScratch sc) {
     const SampleRule rule{temperature, top_p, top_k, key_base, softcap, (uint32_t)seed, (uint32_t)(seed >> 32)};
+    const bool truncated = top_k > 0u && top_k < count;
+    // the sweep by many blocks: rows long enough to fill several blocks, with at least twice as many groups as survivors
+    // (so that the bound leaves out most of the row), and no longer than the scratch holds groups for
+    const bool use_scan = sc.group_keys && count >= max(4096u, truncated ? 2u * kSampleGroup * top_k : 0u) &&
+                          count <= kSampleMaxGroups * kSampleGroup;
+    if (use_scan) {
+        const uint32_t n_seg = (count + kSampleSegment - 1) / kSampleSegment;
+        const dim3 grid(n_seg, rows);
+        if (truncated) {
+            hipLaunchKernelGGL(sample_scan_kernel<true>, grid, dim3(kScanThreads), 0, s, logits, stride, count, ids, rule, key_offset, sc);
+            hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(kSampleThreads), 0, s, logits, stride, count, n_seg, ids, rule, key_offset,
+                               sc, out_tokens, out_prob);
+        } else {
+            hipLaunchKernelGGL(sample_scan_kernel<false>, grid, dim3(kScanThreads), 0, s, logits, stride, count, ids, rule, key_offset, sc);
+            hipLaunchKernelGGL(sample_merge_kernel, dim3(rows), dim3(kSampleThreads), 0, s, logits, stride, n_seg, rule, sc, out_tokens, out_prob);
+        }
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(sample_rows_kernel, dim3(rows), dim3(kSampleThreads), 0, s, logits, stride, count, ids, rule, key_offset,
                        out_tokens, out_prob);
     return hipGetLastError();
