@@ -1062,7 +1062,7 @@ static int gemv_common(ffmoe_ctx *ctx, void *stream, const uint8_t *w, const uin
     if (ctx->f16 && (reinterpret_cast<uintptr_t>(x) % 16 || x_stride % 8))
         return fail(err, FFMOE_ERR_INVALID, "FP16 input rows must be 16-byte aligned with a stride that is a multiple of 8");
     FF_HIP(launch_gemv_int4(static_cast<hipStream_t>(stream), w, scales, biases, x, y, m, n, rows, x_stride, y_stride, y_f32, ids,
-                            ctx->f16));
+                            ctx->f16, ctx->n_cus));
     ctx->timer.mark(static_cast<hipStream_t>(stream), FFMOE_K_GEMV);
     ctx->timer.finish();
     return FFMOE_OK;
@@ -1367,8 +1367,9 @@ int ffmoe_argmax_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_
     if (stride < count) return fail(err, FFMOE_ERR_INVALID, "stride smaller than the row");
     if (!(softcap >= 0.0f) || std::isinf(softcap)) return fail(err, FFMOE_ERR_INVALID, "softcap must be finite and >= 0 (0 disables it)");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    claim_scratch(ctx, stream);
     ctx->timer.begin(s);
-    FF_HIP(launch_argmax_rows(s, logits, stride, rows, count, softcap, out_index, out_conf));
+    FF_HIP(launch_argmax_rows(s, logits, stride, rows, count, softcap, out_index, out_conf, ctx->sample));
     ctx->timer.mark(s, FFMOE_K_ARGMAX);
     ctx->timer.finish();
     return FFMOE_OK;

@@ -10,18 +10,19 @@
 // paired as (x[m], x[m+4]) to line up with ((w >> 4m) & 0x000F000F), and reused for every weight row.
 // Per chunk: acc = sum (128 + q) x by v_dot2_f32_bf16, then s * acc + (b - 128 s) * sum x, the factored
 // form of dequant_int4.metal:104-139. Rows are reduced across the wave by a xor-butterfly.
+// That kernel serves rows longer than a wave's K-slice holds; up to FFMOE_MATRIX_MAX_N the sums run on the matrix unit
+// (gemv_int4_mfma_kernel below).
 // Each input row accumulates independently of the others, so row r of a multi-row call equals the
 // single-row call bit for bit (the property DequantInt4SmallBatchTests.swift:74-78 asserts).
 #include "common.hpp"
 #include "kernels.hpp"
+#include "stream.hpp"
 
 namespace ffmoe {
 namespace {
 
 constexpr int kRowsPerWave = 8;
 constexpr int kRowTile = 4;   // input rows held in registers per pass
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 template <bool F16>
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
@@ -149,11 +150,142 @@ __global__ __launch_bounds__(256) void gemv_int4_kernel(const uint8_t *__restric
     }
 }
 
+// The same product on the matrix unit, for n <= 4 * kRing * 64. A block takes 16 weight rows at a time, its four waves split
+// K; a group's product is v_mfma_f32_16x16x32 of the (up to 16) input rows with the nibbles as 128 + q, then
+// s * acc + (b - 128 s) * sum x, as in the expert kernels (stream.hpp) but on the reference's row-major bytes: four
+// neighbouring lanes load the 32 bytes of a row's group (16 segments per request instead of 64) and ds_bpermute hands
+// each operand lane (row i, quarter q) its eight bytes, the values k = 16 q .. 16 q + 15 of the group. Nibble p of such a
+// dword is element p, so ((w >> 4 m) & 0x000F000F) pairs elements m and m + 4, and the input operand is paired the same way.
+// Bound: latency - row id, weights, products and the merge are one chain per 16 rows, and a hot list of a few thousand
+// rows is one such chain per compute unit. 4,099 listed rows x 2,816, 16 input rows: 50.8 us with the vector ALU's dot
+// products (four passes of four input rows over the weights) -> 7.5 us;
+// 32,768 rows: 19 us.
+template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16>
+__global__ __launch_bounds__(256, 2) void gemv_int4_mfma_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
+                                                                const uint16_t *__restrict__ biases, const uint16_t *__restrict__ x,
+                                                                void *__restrict__ y_, uint32_t m, uint32_t n_groups, uint32_t rows,
+                                                                uint32_t x_stride, uint32_t y_stride, const uint32_t *__restrict__ ids) {
+    __shared__ float s_red[2][kKSplit][4][64];
+    const uint32_t lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t j = lane & 15, jq = lane >> 4;                  // operand layout: row j, quarter jq
+    const uint32_t lrow = lane >> 2, lq = lane & 3;                // load layout: row lrow, quarter lq
+    const uint32_t n_blocks = (m + kTileRows - 1) / kTileRows;
+    const KSlice k = k_slice(n_groups, ks);
+    const size_t row_bytes = (size_t)n_groups * (kGroup / 2);
+    auto id_of = [&](uint32_t rb) {
+        const uint32_t o = min(rb * kTileRows + lrow, m - 1);
+        return ids ? ids[o] : o;
+    };
+    uint2 wt[kRing];
+    uint32_t sb[3];                                                 // scale | bias << 16 of groups g0 + 3 lq + 0 .. 2 of row lrow
+    auto load_w = [&](uint32_t row, int u) {
+        const uint8_t *p = w + row * row_bytes + (size_t)min(k.g0 + u, k.g_last) * (kGroup / 2) + 8 * lq;
+        if (ALIGNED) return *reinterpret_cast<const uint2 *>(p);
+        const uint16_t *h = reinterpret_cast<const uint16_t *>(p);  // 2-byte alignment is guaranteed
+        return make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+    };
+    auto load_s = [&](uint32_t row, int v) {
+        const size_t at = (size_t)row * n_groups + min(k.g0 + 3 * lq + v, k.g_last);
+        return (uint32_t)scales[at] | ((uint32_t)biases[at] << 16);
+    };
+    uint32_t rb = blockIdx.x;                                       // the grid has at most n_blocks blocks
+    uint32_t row = id_of(rb);
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) wt[u] = load_w(row, u);
+#pragma unroll
+    for (int v = 0; v < 3; ++v) sb[v] = load_s(row, v);
+    uint32_t next_id = id_of(min(rb + gridDim.x, n_blocks - 1));
+
+    // the input rows of this wave's K-slice in operand order, paired like the nibbles, and their sum per group
+    uint4 x0[kRing], x1[kRing];
+    f32x4 sx[kRing];
+    {
+        const uint16_t *xrow = x + (size_t)min(lrow, rows - 1) * x_stride + 16 * lq;
+#pragma unroll
+        for (int u = 0; u < kRing; ++u) {
+            const bool live = (uint32_t)u < k.ng;
+            const uint16_t *p = xrow + min(k.g0 + u, k.g_last) * kGroup;
+            x0[u] = live ? load_x8<X_ALIGNED>(p) : uint4{0, 0, 0, 0};
+            x1[u] = live ? load_x8<X_ALIGNED>(p + 8) : uint4{0, 0, 0, 0};
+        }
+        turn_token_rows(lane, x0, x1);
+        auto paired = [](const uint4 &d) {
+            return uint4{(d.x & 0xFFFFu) | (d.z << 16), (d.x >> 16) | (d.z & 0xFFFF0000u),
+                         (d.y & 0xFFFFu) | (d.w << 16), (d.y >> 16) | (d.w & 0xFFFF0000u)};
+        };
+#pragma unroll
+        for (int u = 0; u < kRing; ++u) {
+            x0[u] = paired(x0[u]);
+            x1[u] = paired(x1[u]);
+            sx[u] = group_input_sum<F16>(x0[u], x1[u]);
+        }
+    }
+    const int pull = (int)((4 * j + jq) * 4);
+    const uint32_t my_row = 4 * jq + ks;                            // the input row this lane finishes
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    for (int buf = 0; rb < n_blocks; rb += gridDim.x, buf ^= 1) {
+        row = next_id;
+        next_id = id_of(min(rb + 2 * gridDim.x, n_blocks - 1));
+        f32x4 tot = zero;
+#pragma unroll
+        for (int u = 0; u < kRing; ++u) {
+            uint2 t;
+            t.x = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].x);
+            t.y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].y);
+            uint32_t sc = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((4 * j + u / 3) * 4), (int)sb[u % 3]);
+            if ((uint32_t)u >= k.ng) sc = 0;
+            wt[u] = load_w(row, u);                                 // the next 16 rows (past the last: these again)
+            f32x4 acc = Act<F16>::mfma(x0[u], unpack8_offset<F16>(t.x), zero);
+            acc = Act<F16>::mfma(x1[u], unpack8_offset<F16>(t.y), acc);
+            const float s = bf16lo_to_f32(sc), b = bf16hi_to_f32(sc), tb = __builtin_fmaf(-Act<F16>::kOffset, s, b);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                tot[r] = __builtin_fmaf(s, acc[r], tot[r]);
+                tot[r] = __builtin_fmaf(tb, sx[u][r], tot[r]);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 3; ++v) sb[v] = load_s(row, v);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s_red[buf][ks][r][lane] = tot[r];
+        lds_barrier();
+        float v = s_red[buf][0][ks][lane];
+#pragma unroll
+        for (int o = 1; o < kKSplit; ++o) v += s_red[buf][o][ks][lane];
+        const uint32_t out = rb * kTileRows + j;
+        if (my_row < rows && out < m) {
+            const size_t at = (size_t)my_row * y_stride + out;
+            if (Y_F32) reinterpret_cast<float *>(y_)[at] = v;
+            else reinterpret_cast<uint16_t *>(y_)[at] = Act<F16>::round(v);
+        }
+    }
+}
+
 }  // namespace
 
 hipError_t launch_gemv_int4(hipStream_t s, const uint8_t *w, const uint16_t *scales, const uint16_t *biases,
                             const uint16_t *x, void *y, uint32_t m, uint32_t n, uint32_t rows,
-                            uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids, bool f16) {
+                            uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids, bool f16, uint32_t n_cus) {
+    if (n / kGroup <= (uint32_t)(kKSplit * kRing)) {
+        // every row count of such a width takes this form (the rows of a call equal single-row calls bit for bit)
+        const dim3 blocks(min((m + kTileRows - 1) / kTileRows, 2 * n_cus));
+        const bool wide_w = reinterpret_cast<uintptr_t>(w) % 8 == 0, wide_x = reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_stride % 8 == 0;
+        if (f16 && !wide_x) return hipErrorInvalidValue;     // FP16 rows come 16-byte aligned (checked at the boundary)
+#define FFMOE_GEMVM(A, X, Y, H)                                                                                                     \
+    hipLaunchKernelGGL((gemv_int4_mfma_kernel<A, X, Y, H>), blocks, dim3(256), 0, s, w, scales, biases, x, y, m, n / kGroup, rows, x_stride, \
+                       y_stride, ids)
+#define FFMOE_GEMVM_X(A, Y)                                                                             \
+    do {                                                                                                \
+        if (f16) FFMOE_GEMVM(A, true, Y, true);                                                         \
+        else if (wide_x) FFMOE_GEMVM(A, true, Y, false);                                                \
+        else FFMOE_GEMVM(A, false, Y, false);                                                           \
+    } while (0)
+        if (wide_w) { if (y_f32) FFMOE_GEMVM_X(true, true); else FFMOE_GEMVM_X(true, false); }
+        else { if (y_f32) FFMOE_GEMVM_X(false, true); else FFMOE_GEMVM_X(false, false); }
+#undef FFMOE_GEMVM_X
+#undef FFMOE_GEMVM
+        return hipGetLastError();
+    }
     const uint32_t waves = (m + kRowsPerWave - 1) / kRowsPerWave;
     const dim3 grid((waves + 3) / 4), block(256);
     const bool aligned = (reinterpret_cast<uintptr_t>(w) % 16 == 0) && ((n / 2) % 16 == 0);

@@ -227,7 +227,7 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
                                 float *out_conf = nullptr);
 // greedy choice (and the winner's softmax probability under the softcap) over rows of fp32 logits in memory
 hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count, float softcap,
-                              uint32_t *out, float *out_conf);
+                              uint32_t *out, float *out_conf, SampleScratch sc);
 
 // prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr.
 // Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
@@ -263,7 +263,7 @@ hipError_t launch_rmsnorm(hipStream_t s, const uint16_t *x, uint32_t x_stride, c
 // gemv.hip
 hipError_t launch_gemv_int4(hipStream_t s, const uint8_t *w, const uint16_t *scales, const uint16_t *biases,
                             const uint16_t *x, void *y, uint32_t m, uint32_t n, uint32_t rows,
-                            uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids = nullptr, bool f16 = false);
+                            uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids, bool f16, uint32_t n_cus);
 
 // sample.hip: the sampled choice over rows of fp32 logits (Gumbel-max draw, exact top-k, top-p prefix)
 hipError_t launch_sample_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,

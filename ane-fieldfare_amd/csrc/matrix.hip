@@ -311,28 +311,42 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     }
 }
 
+// The block's largest key, the same in every thread (4 or 16 waves: the waves' keys meet by a butterfly as well - one after
+// the other they were a chain of LDS reads).
 __device__ __forceinline__ unsigned long long block_max_key(unsigned long long k, unsigned long long *s_k) {
 #pragma unroll
     for (int mk = 32; mk >= 1; mk >>= 1) {
         const unsigned long long o = __shfl_xor(k, mk, 64);
         k = o > k ? o : k;
     }
+    const uint32_t waves = blockDim.x / 64;
     if ((threadIdx.x & 63) == 0) s_k[threadIdx.x >> 6] = k;
     __syncthreads();
-    k = s_k[0];
-    for (uint32_t v = 1; v < blockDim.x / 64; ++v) k = s_k[v] > k ? s_k[v] : k;
+    k = s_k[threadIdx.x & (waves - 1)];
+    for (uint32_t mk = waves >> 1; mk >= 1; mk >>= 1) {
+        const unsigned long long o = __shfl_xor(k, mk, 64);
+        k = o > k ? o : k;
+    }
     return k;
 }
 
-// The block's softmax pair, the same in every thread.
+// The block's softmax pair, the same in every thread: the largest value first, then the sums relative to it.
 __device__ __forceinline__ SoftmaxAcc block_softmax(SoftmaxAcc a, float2 *s_p) {
+    const uint32_t waves = blockDim.x / 64;
+    float m = a.m;
 #pragma unroll
-    for (int mk = 32; mk >= 1; mk >>= 1) a = softmax_merge(a, softmax_shuffle(a, mk));
-    if ((threadIdx.x & 63) == 0) s_p[threadIdx.x >> 6] = make_float2(a.m, a.s);
+    for (int mk = 32; mk >= 1; mk >>= 1) m = fmaxf(m, __shfl_xor(m, mk, 64));
+    float s = a.m > -INFINITY ? a.s * __expf(a.m - m) : 0.0f;
+#pragma unroll
+    for (int mk = 32; mk >= 1; mk >>= 1) s += __shfl_xor(s, mk, 64);
+    if ((threadIdx.x & 63) == 0) s_p[threadIdx.x >> 6] = make_float2(m, s);
     __syncthreads();
-    a = SoftmaxAcc{s_p[0].x, s_p[0].y};
-    for (uint32_t v = 1; v < blockDim.x / 64; ++v) a = softmax_merge(a, SoftmaxAcc{s_p[v].x, s_p[v].y});
-    return a;
+    const float2 own = s_p[threadIdx.x & (waves - 1)];
+    m = own.x;
+    for (uint32_t mk = waves >> 1; mk >= 1; mk >>= 1) m = fmaxf(m, __shfl_xor(m, mk, 64));
+    s = own.x > -INFINITY ? own.y * __expf(own.x - m) : 0.0f;
+    for (uint32_t mk = waves >> 1; mk >= 1; mk >>= 1) s += __shfl_xor(s, mk, 64);
+    return SoftmaxAcc{m, s};
 }
 
 // The winner's value from its key (argmax_key is a bijection on the finite values).
@@ -371,29 +385,74 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const unsigned long l
 }
 
 // argmax_rows_f32 (Metal/Sampling/logit.metal:946-1010): the greedy choice over rows of fp32 logits that are in
-// memory already (the listed GEMV's output: a drafter's hot vocabulary), one block per row: the largest finite value,
-// ties to the lowest position, 0xFFFFFFFF and confidence 0 when no value is finite; and the winner's probability
-// under the softcap.
-__global__ __launch_bounds__(256) void argmax_rows_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t count,
-                                                          float softcap, uint32_t *__restrict__ out, float *__restrict__ out_conf) {
-    __shared__ unsigned long long s_k[4];
-    __shared__ float2 s_p[4];
+// memory already (the listed GEMV's output: a drafter's hot vocabulary): the largest finite value, ties to the lowest
+// position, 0xFFFFFFFF and confidence 0 when no value is finite; and the winner's probability under the softcap.
+// One block per row; rows of more than kArgmaxOneBlock values (`segments` given) one block per kSampleSegment values, whose
+// winners argmax_merge_kernel joins. A thread requests eight values before it looks at the first, and adds their
+// exponentials relative to the largest of the eight (value by value it was a chain of exponentials: 16 rows of 4,099 took
+// 10.4 us with 256 threads each, 6.5 us now; 16 rows of 32,768 in segments: 4.9 + 3.9 us).
+constexpr int kArgmaxThreads = 1024, kArgmaxBatch = 8;
+constexpr uint32_t kArgmaxOneBlock = 8192;
+
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void argmax_rows_kernel(const float *__restrict__ logits, uint32_t stride, uint32_t count, uint32_t per_block,
+                                                              float softcap, uint32_t *__restrict__ out, float *__restrict__ out_conf,
+                                                              SampleSegment *__restrict__ segments) {
+    __shared__ unsigned long long s_k[THREADS / 64];
+    __shared__ float2 s_p[THREADS / 64];
     const float *row = logits + (size_t)blockIdx.x * stride;
+    const uint32_t lo = blockIdx.y * per_block, hi = min(count, lo + per_block);
     unsigned long long best = 0ull;
     SoftmaxAcc soft{-INFINITY, 0.0f};
-    for (uint32_t i = threadIdx.x; i < count; i += 256) {
-        const float v = row[i];
-        const unsigned long long k = argmax_key(v, i);
-        best = k > best ? k : best;
-        if (out_conf) softmax_take(soft, v, softcap);
+    for (uint32_t base = lo + threadIdx.x; base < hi; base += kArgmaxBatch * THREADS) {
+        float v[kArgmaxBatch];
+#pragma unroll
+        for (int u = 0; u < kArgmaxBatch; ++u) v[u] = base + u * THREADS < hi ? row[base + u * THREADS] : NAN;
+        float m = soft.m;
+#pragma unroll
+        for (int u = 0; u < kArgmaxBatch; ++u) {
+            const unsigned long long k = argmax_key(v[u], base + u * THREADS);
+            best = k > best ? k : best;
+            v[u] = k ? capped(v[u], softcap) : -INFINITY;       // non-finite values take no part
+            m = fmaxf(m, v[u]);
+        }
+        if (out_conf && m > -INFINITY) {
+            float sum = soft.s * __expf(soft.m - m);            // exp(-inf) = 0: nothing seen before
+#pragma unroll
+            for (int u = 0; u < kArgmaxBatch; ++u) sum += __expf(v[u] - m);
+            soft = SoftmaxAcc{m, sum};
+        }
     }
     best = block_max_key(best, s_k);
-    if (threadIdx.x == 0) out[blockIdx.x] = best ? 0xFFFFFFFFu - (uint32_t)best : 0xFFFFFFFFu;
-    if (out_conf) {
-        soft = block_softmax(soft, s_p);
-        if (threadIdx.x == 0) out_conf[blockIdx.x] = winner_confidence(best, soft, softcap);
+    if (out_conf) soft = block_softmax(soft, s_p);
+    if (threadIdx.x != 0) return;
+    if (segments) {
+        SampleSegment seg{};
+        seg.best = best;
+        seg.top = soft.m;
+        seg.sum = soft.s;
+        segments[(size_t)blockIdx.x * kSampleMaxSegments + blockIdx.y] = seg;
+        return;
     }
+    out[blockIdx.x] = best ? 0xFFFFFFFFu - (uint32_t)best : 0xFFFFFFFFu;
+    if (out_conf) out_conf[blockIdx.x] = winner_confidence(best, soft, softcap);
 }
+
+__global__ __launch_bounds__(256) void argmax_merge_kernel(const SampleSegment *__restrict__ segments, uint32_t n_seg, float softcap,
+                                                           uint32_t *__restrict__ out, float *__restrict__ out_conf) {
+    __shared__ unsigned long long s_k[4];
+    __shared__ float2 s_p[4];
+    SampleSegment mine{};
+    mine.top = -INFINITY;
+    if (threadIdx.x < n_seg) mine = segments[(size_t)blockIdx.x * kSampleMaxSegments + threadIdx.x];
+    const unsigned long long best = block_max_key(mine.best, s_k);
+    SoftmaxAcc soft{mine.top, mine.sum};
+    if (out_conf) soft = block_softmax(soft, s_p);
+    if (threadIdx.x != 0) return;
+    out[blockIdx.x] = best ? 0xFFFFFFFFu - (uint32_t)best : 0xFFFFFFFFu;
+    if (out_conf) out_conf[blockIdx.x] = winner_confidence(best, soft, softcap);
+}
+static_assert(kSampleMaxSegments <= 256, "one segment per thread of argmax_merge_kernel");
 
 }  // namespace
 
@@ -614,8 +673,16 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
 }
 
 hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count, float softcap,
-                              uint32_t *out, float *out_conf) {
-    hipLaunchKernelGGL(argmax_rows_kernel, dim3(rows), dim3(256), 0, s, logits, stride, count, softcap, out, out_conf);
+                              uint32_t *out, float *out_conf, SampleScratch sc) {
+    if (count > kArgmaxOneBlock && rows <= FFMOE_MAX_VERIFY_ROWS && count <= kSampleMaxSegments * kSampleSegment && sc.segments) {
+        const uint32_t n_seg = (count + kSampleSegment - 1) / kSampleSegment;
+        hipLaunchKernelGGL(argmax_rows_kernel<256>, dim3(rows, n_seg), dim3(256), 0, s, logits, stride, count, kSampleSegment, softcap, out,
+                           out_conf, sc.segments);
+        hipLaunchKernelGGL(argmax_merge_kernel, dim3(rows), dim3(256), 0, s, sc.segments, n_seg, softcap, out, out_conf);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(argmax_rows_kernel<kArgmaxThreads>, dim3(rows), dim3(kArgmaxThreads), 0, s, logits, stride, count, count, softcap, out,
+                       out_conf, (SampleSegment *)nullptr);
     return hipGetLastError();
 }
 

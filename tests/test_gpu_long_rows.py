@@ -1,0 +1,86 @@
+"""The forms that split long rows of logits over many blocks (sampled and greedy choice) and the matrix-unit form of the
+reference-layout GEMV, at the edges of their ranges, against the CPU oracle. Run on the GPU box: pytest -m gpu."""
+import numpy as np
+import pytest
+
+from helpers import bf16_tensor, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    assert torch.cuda.is_available()
+    return torch
+
+
+@pytest.fixture(scope="module")
+def ctx(torch):
+    import fieldfare_moe as ff
+    c = ff.Context(128, 64, 16, 8, n_layers=1, max_tokens=16)
+    yield c
+    c.close()
+
+
+# the last count of the one-block form and the first of the other, a last segment of one entry, one group more or less
+@pytest.mark.parametrize("count,top_k,top_p", [(4095, 0, 1.0), (4096, 0, 1.0), (8193, 0, 1.0), (8191, 64, 0.9), (8192, 64, 0.9),
+                                               (32768, 256, 0.95), (4097, 1, 1.0), (34817, 8, 1.0), (65599, 200, 1.0)])
+def test_sampled_choice_at_the_edges_of_the_split_form(ctx, oracle, torch, count, top_k, top_p):
+    rng = np.random.default_rng(count + top_k)
+    rows = rng.normal(0, 4, (6, count)).astype(np.float32)
+    rows[1] = np.round(rows[1])                                # ties at the top_k edge, over many groups
+    rows[2, :] = -1.25                                         # more ties than the candidate lists hold
+    rows[3, 3:] = np.nan                                       # fewer finite entries than top_k, in one group
+    rows[4] = np.sort(rows[4])                                 # every survivor in the last groups
+    rows[5, :] = -np.inf
+    logits = torch.from_numpy(rows).cuda()
+    want_tok, want_prob, gap = oracle.sample_rows(rows, 0.9, top_p, top_k, key_base=5, softcap=30.0, seed=11)
+    tok, prob = ctx.sample_rows(logits, 0.9, 30.0, 11, key_base=5, top_k=top_k, top_p=top_p)
+    tok, prob = tok.cpu().numpy().astype(np.uint32), prob.cpu().numpy().astype(np.float64)
+    clear = gap > 1e-4                                         # log and tanh of the two machines differ by less
+    assert clear.sum() >= 5 and np.array_equal(tok[clear], want_tok[clear]), (tok, want_tok, gap)
+    # exp of a difference of capped logits (|c| <= 30: 2^-24 * 30 * 2 absolute each) over a sum of `count` positive terms
+    same = tok == want_tok
+    assert (np.abs(prob[same] - want_prob[same]) <= 1e-5 + 2e-3 * want_prob[same]).all(), (prob, want_prob)
+
+
+@pytest.mark.parametrize("count", [1, 1023, 8192, 8193, 10241, 262144])
+def test_greedy_choice_over_long_rows(ctx, oracle, torch, count):
+    rng = np.random.default_rng(count)
+    rows = rng.normal(0, 3, (5, count)).astype(np.float32)
+    rows[1, :] = 2.0                                           # all equal: position 0
+    rows[2, :] = np.nan                                        # nothing finite
+    rows[3, count - 1] = 99.0                                  # the last entry wins
+    rows[4, : count // 2] = np.inf
+    logits = torch.from_numpy(rows).cuda()
+    for cap in (0.0, 30.0):
+        pos, conf = ctx.argmax_rows(logits, softcap=cap)
+        want_pos, want_conf = oracle.greedy_choice_rows(rows, cap)
+        assert np.array_equal(pos.cpu().numpy().astype(np.uint32), want_pos.astype(np.uint32))
+        assert np.abs(conf.cpu().numpy() - want_conf).max() <= 1e-5
+        assert np.array_equal(ctx.argmax_rows(logits, softcap=cap, want_conf=False).cpu().numpy(), pos.cpu().numpy())
+
+
+# tiles of 16 rows: one, one and a bit, more blocks than the grid holds; one group, a K-slice of two groups, the widest row
+@pytest.mark.parametrize("m,n,rows,off", [(1, 64, 1, 0), (17, 64, 16, 2), (33, 448, 3, 0), (8209, 192, 5, 0), (47, 2816, 16, 2),
+                                          (31, 2752, 9, 4), (20, 2880, 2, 0)])
+def test_reference_layout_gemv_at_the_edges(ctx, oracle, torch, m, n, rows, off):
+    g = oracle.seed_tree_key(m + n, f"gemv-edges-{rows}")
+    W, S, B = oracle.quantize_int4(g.uniform(-0.5, 0.5, m * n).reshape(m, n))
+    xb = oracle.bf16_bits(g.uniform(-1.0, 1.0, rows * (n + 8))).reshape(rows, n + 8)
+    raw = torch.from_numpy(np.concatenate([np.zeros(off, np.uint8), W.ravel()])).cuda()
+    Sd, Bd = (torch.from_numpy(a.view(np.int16)).cuda() for a in (S, B))
+    for start in (0, 1):                                       # 16-byte aligned input rows, and 2-byte aligned ones
+        x = bf16_tensor(torch, xb)[:, start:start + n]
+        y = ctx.gemv_int4(raw, Sd, Bd, x, f32_out=True, w_byte_offset=off).cpu().numpy()
+        for r in range(rows):
+            ref = oracle.gemv_int4_ref(W, S, B, oracle.bf16_to_float(xb[r, start:start + n]))
+            # the offset form's sums are about 17 times the result's terms, 64 roundings of 2^-24 per group
+            assert rel_err(y[r], ref) < 1e-4, (start, r)
+            one = ctx.gemv_int4(raw, Sd, Bd, x[r:r + 1], f32_out=True, w_byte_offset=off).cpu().numpy()[0]
+            assert np.array_equal(one.view(np.uint32), y[r].view(np.uint32))
+        ids = np.array([m - 1, 0, m // 2, 0], np.int32)
+        if off == 0:
+            listed = ctx.gemv_int4_listed(raw, Sd, Bd, torch.from_numpy(ids).cuda(), x).cpu().numpy()
+            assert np.array_equal(listed.view(np.uint32), y[:, ids].view(np.uint32))
