@@ -1,12 +1,16 @@
-"""ctypes binding of libfieldfare_moe_hip.so (the C ABI in include/fieldfare_moe.h).
+"""Binding of libfieldfare_moe_hip.so (the C ABI in include/fieldfare_moe.h).
 
 PyTorch is used for device memory and streams only: every method takes torch CUDA tensors, passes
-their raw device pointers through the C ABI, and enqueues on torch's current stream. There is no CPU
-or eager fallback: a missing library raises at import of the symbols, a missing GPU at Context().
+their raw device pointers through the C ABI, and enqueues on torch's current stream. The compute methods do
+that in native code (csrc/binding.cpp, the ffmoe_binding module built beside the library), the rest - creation, uploads,
+switches, reports - through ctypes. There is no CPU or eager fallback: a missing library raises at import of the symbols,
+a missing GPU at Context().
 """
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import subprocess
 from pathlib import Path
 
@@ -105,51 +109,33 @@ class Matrix:
             _check(self.L.ffmoe_matrix_create(ctx._h, raw(W, w_byte_offset), raw(S), raw(B), self.m, self.n, int(greedy),
                                               C.byref(h), C.byref(err)), err)
         self._h = h
+        self._hv = h.value
 
     def gemv(self, x, f32_out: bool = False, out=None):
-        import torch
-        rows = x.shape[0]
-        y = torch.empty((rows, self.m), dtype=torch.float32 if f32_out else self.ctx.act, device=x.device) if out is None else out
-        err = C.c_char_p()
-        _check(self.L.ffmoe_matrix_gemv(self._h, _stream(), _ptr(x), _row_stride(x), rows, _ptr(y), _row_stride(y),
-                                        int(f32_out), C.byref(err)), err)
-        return y
+        return _native.matrix_gemv(self._hv, x, self.m, self.ctx.act, f32_out, out)
 
     def rows(self, ids, out_scale: float = 1.0, out=None):
         """Dequantised rows `ids` (an int or an int32 / uint32 CUDA tensor) times out_scale: [count, N] of the activation type."""
         import torch
         single = isinstance(ids, int)
-        count = 1 if single else int(ids.shape[0])
-        y = torch.empty((count, self.n), dtype=self.ctx.act, device="cuda") if out is None else out
+        y = torch.empty((1 if single else int(ids.shape[0]), self.n), dtype=self.ctx.act, device="cuda") if out is None else out
+        if not single:
+            return _native.matrix_rows(self._hv, ids, out_scale, y)
         err = C.c_char_p()
-        _check(self.L.ffmoe_matrix_rows(self._h, _stream(), None if single else _ptr(ids), count, ids if single else 0,
-                                        out_scale, _ptr(y), _row_stride(y), C.byref(err)), err)
+        _check(self.L.ffmoe_matrix_rows(self._h, _stream(), None, 1, ids, out_scale, _ptr(y), _row_stride(y), C.byref(err)), err)
         return y
 
     def greedy(self, x):
-        import torch
-        rows = x.shape[0]
-        out = torch.empty((rows,), dtype=torch.int32, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_matrix_greedy(self._h, _stream(), _ptr(x), _row_stride(x), rows, _ptr(out), C.byref(err)),
-               err)
-        return out
+        return _native.matrix_greedy(self._hv, x)
 
     def greedy_conf(self, x, softcap: float = 0.0):
         """(tokens int32 [rows], confidence fp32 [rows]): the greedy choice and its softmax probability under the softcap."""
-        import torch
-        rows = x.shape[0]
-        out = torch.empty((rows,), dtype=torch.int32, device=x.device)
-        conf = torch.empty((rows,), dtype=torch.float32, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_matrix_greedy_conf(self._h, _stream(), _ptr(x), _row_stride(x), rows, softcap, _ptr(out), _ptr(conf),
-                                               C.byref(err)), err)
-        return out, conf
+        return _native.matrix_greedy_conf(self._hv, x, softcap)
 
     def close(self):
         if self._h:
             self.L.ffmoe_matrix_destroy(self._h)
-            self._h = None
+            self._h = self._hv = None
 
     def __del__(self):
         try:
@@ -158,6 +144,7 @@ class Matrix:
             pass
 
 
+BINDING_PATH = _PKG / "ffmoe_binding.so"
 HASH_PATH = LIB_PATH.with_suffix(".so.srchash")
 
 
@@ -165,7 +152,7 @@ def source_hash() -> str:
     """Digest of everything the library is compiled from (kernels, headers, Makefile, the C header)."""
     import hashlib
     h = hashlib.sha256()
-    files = sorted(p for p in CSRC.iterdir() if p.suffix in (".hip", ".hpp") or p.name == "Makefile")
+    files = sorted(p for p in CSRC.iterdir() if p.suffix in (".hip", ".hpp", ".cpp") or p.name == "Makefile")
     for p in files + [_PKG.parent / "include" / "fieldfare_moe.h"]:
         h.update(p.name.encode())
         h.update(p.read_bytes())
@@ -175,7 +162,7 @@ def source_hash() -> str:
 def is_stale() -> bool:
     """True when no library is built or the sources changed since it was (file times do not survive a copy of the tree,
     so the build leaves a digest of its sources beside the library)."""
-    return not (LIB_PATH.exists() and HASH_PATH.exists() and HASH_PATH.read_text().strip() == source_hash())
+    return not (LIB_PATH.exists() and BINDING_PATH.exists() and HASH_PATH.exists() and HASH_PATH.read_text().strip() == source_hash())
 
 
 def build(force: bool = True) -> Path:
@@ -193,19 +180,20 @@ def build(force: bool = True) -> Path:
 def ensure_built() -> Path:
     """Load what is built in-tree; compile only when nothing is, or when the sources are newer than the library."""
     if is_stale():
-        build(force=not LIB_PATH.exists())
+        build(force=not (LIB_PATH.exists() and BINDING_PATH.exists()))
     return LIB_PATH
 
 
 _lib = None
+_native = None      # the ffmoe_binding module
 
 
 def lib() -> C.CDLL:
-    global _lib
+    global _lib, _native
     if _lib is not None:
         return _lib
-    if not LIB_PATH.exists():
-        raise FileNotFoundError(f"{LIB_PATH} is not built; run __graft_entry__.build() (there is no fallback path)")
+    if not (LIB_PATH.exists() and BINDING_PATH.exists()):
+        raise FileNotFoundError(f"{LIB_PATH} or {BINDING_PATH.name} is not built; run __graft_entry__.build() (there is no fallback path)")
     if is_stale():
         raise RuntimeError(f"{LIB_PATH} was built from other sources than the ones in {CSRC}; run __graft_entry__.build() "
                            "or fieldfare_moe.ensure_built()")
@@ -270,7 +258,11 @@ def lib() -> C.CDLL:
     L.ffmoe_sample_rows.argtypes = [vp, vp, vp, u32, u32, u32, vp, C.POINTER(Sampling), vp, vp, vp, errp]
     L.ffmoe_route_verify_shared.argtypes = [vp, vp, vp, u32, u32, vp, u32, vp, u32, vp, u32, u32, vp, vp, errp]
     L.ffmoe_layer_tail_routed_shared.argtypes = [vp, vp, vp, vp, vp, u32, vp, vp, u32, C.c_float, C.c_float, errp]
-    _lib = L
+    loader = importlib.machinery.ExtensionFileLoader("ffmoe_binding", str(BINDING_PATH))
+    native = importlib.util.module_from_spec(importlib.util.spec_from_loader("ffmoe_binding", loader))
+    loader.exec_module(native)
+    native.bind(str(LIB_PATH), FieldfareError)
+    _native, _lib = native, L
     return L
 
 
@@ -311,6 +303,7 @@ class Context:
         self._h = C.c_void_p()
         err = C.c_char_p()
         _check(self.L.ffmoe_create(device, C.byref(self.shape), C.byref(self._h), C.byref(err)), err)
+        self._hv, self._d, self._k = self._h.value, d, top_k
         if act_dtype == "fp16":
             _check(self.L.ffmoe_set_activation_dtype(self._h, FP16, C.byref(err)), err)
 
@@ -327,6 +320,7 @@ class Context:
         if getattr(self, "_h", None) and self._h.value:
             self.L.ffmoe_destroy(self._h)
             self._h = C.c_void_p()
+            self._hv = None
 
     def __del__(self):
         try:
@@ -444,64 +438,28 @@ class Context:
     # -- router ----------------------------------------------------------------------------------
     def router(self, layer: int, router_x, want_logits: bool = False):
         """router_x: bf16 [T, stride>=d] CUDA tensor (rows may be strided). Returns (idx i32 [T,K], w bf16 [T,K][, logits])."""
-        import torch
-        assert router_x.dtype == self.act and router_x.is_cuda and router_x.stride(1) == 1
-        t = router_x.shape[0]
-        k, e = self.shape.top_k, self.shape.n_experts
-        idx = torch.empty((t, k), dtype=torch.int32, device=router_x.device)
-        w = torch.empty((t, k), dtype=self.act, device=router_x.device)
-        logits = torch.empty((t, e), dtype=torch.float32, device=router_x.device) if want_logits else None
-        err = C.c_char_p()
-        _check(self.L.ffmoe_router(self._h, _stream(), layer, _ptr(router_x), _row_stride(router_x), t, _ptr(idx), _ptr(w),
-                                   _ptr(logits), C.byref(err)), err)
-        return (idx, w, logits) if want_logits else (idx, w)
+        return _native.router(self._hv, layer, router_x, self.act, self._k, self.shape.n_experts, want_logits)
 
     # -- routed experts --------------------------------------------------------------------------
     def verify(self, layer: int, x, idx, w, residual=None, out=None):
         """Decode step (T = 1) or verify block (T <= 16): fused experts + weighted combine. x bf16 [T, stride]."""
-        import torch
-        t = x.shape[0]
-        y = out if out is not None else torch.empty((t, self.shape.d), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_verify(self._h, _stream(), layer, _ptr(x), _row_stride(x), t, _ptr(idx), _ptr(w), _ptr(residual),
-                                   _ptr(y), C.byref(err)), err)
-        return y
+        return _native.verify(self._hv, layer, x, idx, w, residual, out, self.act, self._d)
 
     def route_verify(self, layer: int, router_x, x, residual=None, out=None, combine: bool = True):
         """Router + expert pass of a block of <= 16 rows in one call. Returns (y, idx, w); combine=False leaves the
         routes' rows un-combined in the context (y is None) for layer_tail_routed."""
-        import torch
-        t, k = x.shape[0], self.shape.top_k
-        y = None if not combine else out if out is not None else torch.empty((t, self.shape.d), dtype=self.act, device=x.device)
-        idx = torch.empty((t, k), dtype=torch.int32, device=x.device)
-        w = torch.empty((t, k), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_route_verify(self._h, _stream(), layer, _ptr(router_x), _row_stride(router_x), _ptr(x), _row_stride(x),
-                                         t, _ptr(residual), _ptr(y), _ptr(idx), _ptr(w), C.byref(err)), err)
-        return y, idx, w
+        return _native.route_verify(self._hv, layer, router_x, x, residual, out, combine, self.act, self._k, self._d)
 
     def route_verify_shared(self, shared: "Context", layer: int, shared_layer: int, router_x, x, shared_x):
         """route_verify(..., combine=False) with the shared expert (the dense context `shared`, on shared_x) inside the
         same two launches. Returns (idx, w); the rows stay in the two contexts for layer_tail_routed_shared."""
-        import torch
-        t, k = x.shape[0], self.shape.top_k
-        idx = torch.empty((t, k), dtype=torch.int32, device=x.device)
-        w = torch.empty((t, k), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_route_verify_shared(self._h, shared._h, _stream(), layer, shared_layer, _ptr(router_x),
-                                                _row_stride(router_x), _ptr(x), _row_stride(x), _ptr(shared_x),
-                                                _row_stride(shared_x), t, _ptr(idx), _ptr(w), C.byref(err)), err)
-        return idx, w
+        return _native.route_verify_shared(self._hv, shared._hv, layer, shared_layer, router_x, x, shared_x, self.act, self._k)
 
     def verify_partials(self, layer: int, x, idx, w, partials=None):
-        import torch
-        t = x.shape[0]
         if partials is None:
-            partials = torch.zeros((t, self.shape.top_k, self.shape.d), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_verify_partials(self._h, _stream(), layer, _ptr(x), _row_stride(x), t, _ptr(idx), _ptr(w),
-                                            _ptr(partials), C.byref(err)), err)
-        return partials
+            import torch
+            partials = torch.zeros((x.shape[0], self._k, self._d), dtype=self.act, device=x.device)
+        return _native.verify_partials(self._hv, layer, x, idx, w, partials)
 
     def set_handover_timeout(self, ticks: int):
         """Ticks (100 MHz) a wave of route_verify's one-launch form waits for a hand-over word before it computes the
@@ -533,39 +491,19 @@ class Context:
         return int(n.value)
 
     def reduce_token_major(self, partials, weights):
-        import torch
-        t, k, d = partials.shape
-        h2 = torch.empty((t, d), dtype=self.act, device=partials.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_reduce_token_major(self._h, _stream(), _ptr(partials), _ptr(weights), _ptr(h2), t, k, d,
-                                               C.byref(err)), err)
-        return h2
+        return _native.reduce_token_major(self._hv, partials, weights, self.act)
 
     # -- prefill ---------------------------------------------------------------------------------
     def prefill(self, layer: int, x, idx, w, out=None):
-        import torch
-        t = x.shape[0]
-        y = out if out is not None else torch.empty((t, self.shape.d), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_prefill(self._h, _stream(), layer, _ptr(x), _row_stride(x), t, _ptr(idx), _ptr(w), _ptr(y),
-                                    C.byref(err)), err)
-        return y
+        return _native.prefill(self._hv, layer, x, idx, w, out, self.act, self._d)
 
     def dense_ffn(self, layer: int, x, out=None):
         """Shared expert: every row of x through expert 0 with weight 1 (context with n_experts = top_k = 1)."""
-        import torch
-        t = x.shape[0]
-        y = out if out is not None else torch.empty((t, self.shape.d), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_dense_ffn(self._h, _stream(), layer, _ptr(x), _row_stride(x), t, _ptr(y), C.byref(err)), err)
-        return y
+        return _native.dense_ffn(self._hv, layer, x, out, self.act, self._d)
 
     def prefill_pairs(self, layer: int, x, sorted_pairs, t: int, partials):
         """Guest contract: sorted_pairs int32 [n, 4] CUDA tensor of (token, expert, rank, weight bits)."""
-        err = C.c_char_p()
-        _check(self.L.ffmoe_prefill_pairs(self._h, _stream(), layer, _ptr(x), _row_stride(x), _ptr(sorted_pairs),
-                                          sorted_pairs.shape[0], t, _ptr(partials), C.byref(err)), err)
-        return partials
+        return _native.prefill_pairs(self._hv, layer, x, sorted_pairs, t, partials)
 
     def prefill_stats(self):
         """(pairs kept, M-tiles, pairs per expert) of the last prefill call."""
@@ -582,68 +520,29 @@ class Context:
                         out=None):
         """hidden (updated in place), attn: bf16 CUDA tensors [t, >= d] (row stride = their second stride);
         returns (dense_x, routed_x, router_x), each [t, d] unless `out` gives three tensors to fill."""
-        import torch
-        t = hidden.shape[0]
-        d = d or self.shape.d
-        outs = out if out is not None else tuple(torch.empty((t, d), dtype=self.act, device=hidden.device) for _ in range(3))
-        err = C.c_char_p()
-        _check(self.L.ffmoe_post_attn_setup(self._h, _stream(), _ptr(hidden), _row_stride(hidden), _ptr(attn), _row_stride(attn),
-                                            _ptr(outs[0]), _row_stride(outs[0]), _ptr(outs[1]), _row_stride(outs[1]),
-                                            _ptr(outs[2]), _row_stride(outs[2]), _ptr(w_post_attn), _ptr(w_pre_ffn),
-                                            _ptr(w_pre_ffn2), t, d, eps, C.byref(err)), err)
-        return outs
+        return _native.post_attn_setup(self._hv, hidden, attn, w_post_attn, w_pre_ffn, w_pre_ffn2, eps, d or self._d, out, self.act)
 
     def layer_tail(self, h2, h1, hidden, w_postffn2, w_postffn, layer_scalar: float, eps: float = 1e-6, d: int | None = None):
         """hidden = (hidden + norm(h1 + norm(h2))) * layer_scalar, in place; bf16 CUDA tensors [t, >= d]."""
-        t = hidden.shape[0]
-        d = d or self.shape.d
-        err = C.c_char_p()
-        _check(self.L.ffmoe_layer_tail(self._h, _stream(), _ptr(h2), _row_stride(h2), _ptr(h1), _row_stride(h1), _ptr(hidden),
-                                       _row_stride(hidden), _ptr(w_postffn2), _ptr(w_postffn), t, d, eps, layer_scalar,
-                                       C.byref(err)), err)
-        return hidden
+        return _native.layer_tail(self._hv, h2, h1, hidden, w_postffn2, w_postffn, layer_scalar, eps, d or self._d)
 
     def layer_tail_routed(self, route_w, h1, hidden, w_postffn2, w_postffn, layer_scalar: float, eps: float = 1e-6):
         """layer_tail on the rows the last route_verify(..., combine=False) left un-combined (weights: that call's w)."""
-        t = hidden.shape[0]
-        err = C.c_char_p()
-        _check(self.L.ffmoe_layer_tail_routed(self._h, _stream(), _ptr(route_w), _ptr(h1), _row_stride(h1), _ptr(hidden),
-                                              _row_stride(hidden), _ptr(w_postffn2), _ptr(w_postffn), t, eps, layer_scalar,
-                                              C.byref(err)), err)
-        return hidden
+        return _native.layer_tail_routed(self._hv, route_w, h1, hidden, w_postffn2, w_postffn, layer_scalar, eps)
 
     def layer_tail_routed_shared(self, shared: "Context", route_w, hidden, w_postffn2, w_postffn, layer_scalar: float,
                                  eps: float = 1e-6):
         """layer_tail on the rows the last route_verify_shared left in this context (routed) and in `shared` (h1)."""
-        t = hidden.shape[0]
-        err = C.c_char_p()
-        _check(self.L.ffmoe_layer_tail_routed_shared(self._h, shared._h, _stream(), _ptr(route_w), _ptr(hidden),
-                                                     _row_stride(hidden), _ptr(w_postffn2), _ptr(w_postffn), t, eps,
-                                                     layer_scalar, C.byref(err)), err)
-        return hidden
+        return _native.layer_tail_routed_shared(self._hv, shared._hv, route_w, hidden, w_postffn2, w_postffn, layer_scalar, eps)
 
     def layer_tail_norms(self, h2, h1, hidden, w_postffn1, w_postffn2, w_postffn, layer_scalar: float, w_next=None,
                          eps: float = 1e-6, d: int | None = None):
         """The tail with h1 taken before its post-FFN-1 norm; with w_next also returns the next layer's input norm."""
-        import torch
-        t = hidden.shape[0]
-        d = d or self.shape.d
-        normed = torch.empty((t, d), dtype=self.act, device=hidden.device) if w_next is not None else None
-        err = C.c_char_p()
-        _check(self.L.ffmoe_layer_tail_norms(self._h, _stream(), _ptr(h2), _row_stride(h2), _ptr(h1), _row_stride(h1), _ptr(hidden),
-                                             _row_stride(hidden), _ptr(w_postffn1), _ptr(w_postffn2), _ptr(w_postffn), _ptr(w_next),
-                                             _ptr(normed), d, t, d, eps, layer_scalar, C.byref(err)), err)
-        return normed
+        return _native.layer_tail_norms(self._hv, h2, h1, hidden, w_postffn1, w_postffn2, w_postffn, layer_scalar, w_next, eps,
+                                        d or self._d, self.act)
 
     def rmsnorm(self, x, w, eps: float = 1e-6, d: int | None = None, out=None):
-        import torch
-        t = x.shape[0]
-        d = d or self.shape.d
-        y = out if out is not None else torch.empty((t, d), dtype=self.act, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_rmsnorm(self._h, _stream(), _ptr(x), _row_stride(x), _ptr(w), _ptr(y), _row_stride(y), t, d, eps,
-                                    C.byref(err)), err)
-        return y
+        return _native.rmsnorm(self._hv, x, w, eps, d or self._d, out, self.act)
 
     # -- generic GEMV ----------------------------------------------------------------------------
     def matrix(self, W, S, B, greedy: bool = False, w_byte_offset: int = 0):
@@ -660,60 +559,23 @@ class Context:
 
     def gelu_mul(self, gate, up, out=None):
         """out = round16(gelu_tanh(gate) * up), rows of the activation type (2-D tensors of one shape)."""
-        import torch
-        rows, count = gate.shape
-        out = torch.empty((rows, count), dtype=gate.dtype, device=gate.device) if out is None else out
-        err = C.c_char_p()
-        _check(self.L.ffmoe_gelu_mul(self._h, _stream(), _ptr(gate), _row_stride(gate), _ptr(up), _row_stride(up), _ptr(out),
-                                     _row_stride(out), rows, count, C.byref(err)), err)
-        return out
+        return _native.gelu_mul(self._hv, gate, up, out)
 
     def argmax_rows(self, logits, count: int | None = None, softcap: float = 0.0, want_conf: bool = True):
         """Greedy position per row of fp32 logits [rows, >= count] (int32, -1 when no value is finite) and, with
         want_conf, the winner's softmax probability under the softcap."""
-        import torch
-        rows = logits.shape[0]
-        count = count or logits.shape[1]
-        out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
-        conf = torch.empty((rows,), dtype=torch.float32, device=logits.device) if want_conf else None
-        err = C.c_char_p()
-        _check(self.L.ffmoe_argmax_rows(self._h, _stream(), _ptr(logits), _row_stride(logits), rows, count, softcap, _ptr(out),
-                                        _ptr(conf), C.byref(err)), err)
-        return (out, conf) if want_conf else out
+        return _native.argmax_rows(self._hv, logits, count or 0, softcap, want_conf)
 
     def sample_rows(self, logits, temperature: float, softcap: float, seed: int, key_base: int = 0, top_k: int = 0,
                     top_p: float = 1.0, ids=None, key_offset=None, count: int | None = None):
         """The sampled choice per row of fp32 logits [rows, >= count]: (position int32 [-1: nothing finite], probability)."""
-        import torch
-        rows = logits.shape[0]
-        count = count or logits.shape[1]
-        out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
-        prob = torch.empty((rows,), dtype=torch.float32, device=logits.device)
-        rule = Sampling(temperature, top_p, top_k, key_base, softcap, seed)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_sample_rows(self._h, _stream(), _ptr(logits), _row_stride(logits), rows, count, _ptr(ids),
-                                        C.byref(rule), _ptr(key_offset), _ptr(out), _ptr(prob), C.byref(err)), err)
-        return out, prob
+        return _native.sample_rows(self._hv, logits, temperature, softcap, seed, key_base, top_k, top_p, ids, key_offset, count or 0)
 
     def gemv_int4_listed(self, W, S, B, ids, x):
         """GEMV over the weight rows listed in `ids` (int32 CUDA tensor [m]): y fp32 [R, m], y[:, o] = row ids[o]."""
-        import torch
-        m, n, rows = ids.shape[0], S.shape[1] * GROUP, x.shape[0]
-        y = torch.empty((rows, m), dtype=torch.float32, device=x.device)
-        err = C.c_char_p()
-        _check(self.L.ffmoe_gemv_int4_listed(self._h, _stream(), _ptr(W), _ptr(S), _ptr(B), _ptr(ids), _ptr(x), _ptr(y), m, n,
-                                             rows, _row_stride(x), m, C.byref(err)), err)
-        return y
+        return _native.gemv_int4_listed(self._hv, W, S, B, ids, x)
 
     def gemv_int4(self, W, S, B, x, f32_out: bool = False, w_byte_offset: int = 0):
         """W uint8 [M, N/2] (optionally starting `w_byte_offset` bytes into a larger buffer), S/B bf16-bit
         int16/uint16 tensors [M, N/64], x bf16 [R, stride]. Returns y [R, M]."""
-        import torch
-        m, n = S.shape[0], S.shape[1] * GROUP
-        rows = x.shape[0]
-        y = torch.empty((rows, m), dtype=torch.float32 if f32_out else self.act, device=x.device)
-        err = C.c_char_p()
-        wp = C.c_void_p(W.data_ptr() + w_byte_offset)
-        _check(self.L.ffmoe_gemv_int4(self._h, _stream(), wp, _ptr(S), _ptr(B), _ptr(x), _ptr(y), m, n, rows,
-                                      _row_stride(x), m, int(f32_out), C.byref(err)), err)
-        return y
+        return _native.gemv_int4(self._hv, W, S, B, x, f32_out, w_byte_offset, self.act)
