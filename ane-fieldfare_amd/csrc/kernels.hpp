@@ -229,6 +229,17 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
 hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count, float softcap,
                               uint32_t *out, float *out_conf, SampleScratch sc);
 
+// The most pairs per expert, on average, at which a prefill chunk takes the streaming product, and the M-tiles that a
+// scratch for `max_pairs` pairs has to hold: that product's tiles go down to 32 pairs (prefill_tile_shift, prefill.hip).
+constexpr uint32_t kPrefillStreamPairs = 48;
+constexpr uint32_t kDenseTileStreamRows = 896;       // and the most rows at which a dense FFN's chunk does
+inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts) {
+    const uint32_t whole = max_pairs / FFMOE_PREFILL_TILE_M;
+    // 32 pairs a tile up to 28 per expert, 64 up to 48: fewer than n_experts full tiles
+    const uint32_t small = n_experts == 1 ? kDenseTileStreamRows / 32 : n_experts;
+    return (whole > small ? whole : small) + n_experts + 1;
+}
+
 // prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr.
 // Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,

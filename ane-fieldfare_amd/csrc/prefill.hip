@@ -20,6 +20,7 @@
 // fix) unnecessary.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "stream.hpp"
 
 namespace ffmoe {
 namespace {
@@ -72,7 +73,9 @@ constexpr int kScanKeep = 16;
 __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad,
                                                                     uint32_t *__restrict__ block_cnt,
                                                                     PrefillPlan *__restrict__ plan,
-                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles) {
+                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles,
+                                                                    uint32_t tile_shift) {
+    const uint32_t bm = 1u << tile_shift;        // pairs per M-tile
     __shared__ uint32_t total[FFMOE_MAX_EXPERTS];
     __shared__ uint32_t offset[FFMOE_MAX_EXPERTS + 1];
     __shared__ uint32_t tile_off[FFMOE_MAX_EXPERTS + 1];
@@ -113,7 +116,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
     if (threadIdx.x < FFMOE_MAX_EXPERTS) {
         const uint32_t i = threadIdx.x, lane = i & 63, wv = i >> 6;
         const uint32_t n = i < n_experts ? total[i] : 0;
-        const unsigned long long own = ((unsigned long long)((n + kBM - 1) / kBM) << 32) | n;
+        const unsigned long long own = ((unsigned long long)((n + bm - 1) >> tile_shift) << 32) | n;
         unsigned long long inc = own;
 #pragma unroll
         for (int sh = 1; sh < 64; sh <<= 1) {
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
             unsigned long long all = ex;
             if (i != n_experts) {
                 const uint32_t n = total[i];
-                all += ((unsigned long long)((n + kBM - 1) / kBM) << 32) | n;
+                all += ((unsigned long long)((n + bm - 1) >> tile_shift) << 32) | n;
                 offset[n_experts] = (uint32_t)all;
                 tile_off[n_experts] = (uint32_t)(all >> 32);
             }
@@ -155,11 +158,11 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
     // anywhere in the expert order). Where an expert's shorter tile goes takes a look at every other expert's: the
     // threads of an expert share that out (one thread alone is a chain of two thousand instructions).
     if (live) {
-        const uint32_t rest = total[e] % kBM, per_o = (e_pad + chunks - 1) / chunks;
+        const uint32_t rest = (total[e] & (bm - 1)), per_o = (e_pad + chunks - 1) / chunks;
         const uint32_t o_lo = min(e_pad, ch * per_o), o_hi = min(e_pad, o_lo + per_o);
         uint32_t all = 0, in_front = 0, above = 0;
         for (uint32_t o = o_lo; o < o_hi; ++o) {
-            const uint32_t r = total[o] % kBM;          // experts past n_experts hold zero
+            const uint32_t r = (total[o] & (bm - 1));          // experts past n_experts hold zero
             const uint32_t has = r != 0 ? 1u : 0u;
             all += has;
             in_front += has & (o < e ? 1u : 0u);
@@ -188,7 +191,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
     plan->expert_offset[e] = offset[e];
     plan->expert_count[e] = total[e];
     // a tile keeps its number in row order, which places its activation blocks
-    const uint32_t nt = (total[e] + kBM - 1) / kBM, n_full = total[e] / kBM;
+    const uint32_t nt = (total[e] + bm - 1) >> tile_shift, n_full = total[e] >> tile_shift;
     const uint32_t shorter_tiles = shorter[0][e], shorter_in_front = shorter[1][e], ranked_above = shorter[2][e];
     const uint32_t full_in_front = tile_off[e] - shorter_in_front, full_tiles = tile_off[n_experts] - shorter_tiles;
     for (uint32_t i = 0; i < nt; ++i) {
@@ -196,8 +199,8 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
         if (ti < max_tiles) {
             PrefillTile tl;
             tl.expert = e;
-            tl.row_start = offset[e] + i * kBM;
-            tl.rows = min((uint32_t)kBM, total[e] - i * kBM);
+            tl.row_start = offset[e] + i * bm;
+            tl.rows = min(bm, total[e] - i * bm);
             tl.order = tile_off[e] + i;
             tiles[ti] = tl;
         }
@@ -246,7 +249,8 @@ __global__ __launch_bounds__(kSortBlock) void prefill_scatter_kernel(ItemSource 
 
 // A dense FFN's chunk needs no sort: one expert, route r = row r. One launch writes what the three above would: the
 // identity tables and the chunk cut into M-tiles.
-__global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t t, PrefillPlan *__restrict__ plan,
+__global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t t, uint32_t tile_shift,
+                                                                       PrefillPlan *__restrict__ plan,
                                                                        PrefillTile *__restrict__ tiles,
                                                                        uint32_t *__restrict__ sorted_token,
                                                                        uint32_t *__restrict__ sorted_out_row) {
@@ -255,12 +259,12 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
         sorted_token[i] = i;
         sorted_out_row[i] = i;
     }
-    const uint32_t n_tiles = (t + kBM - 1) / kBM;
+    const uint32_t bm = 1u << tile_shift, n_tiles = (t + bm - 1) >> tile_shift;
     if (i < n_tiles) {
         PrefillTile tl;
         tl.expert = 0;
-        tl.row_start = i * kBM;
-        tl.rows = min((uint32_t)kBM, t - i * kBM);
+        tl.row_start = i * bm;
+        tl.rows = min(bm, t - i * bm);
         tl.order = i;
         tiles[i] = tl;
     }
@@ -621,6 +625,22 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const ArenaGeom &g
     }
 }
 
+// Consecutive block ids go to consecutive XCDs. Many experts: all N-blocks of an M-tile share an XCD (its L2 holds
+// the tile's A rows). One expert (the dense FFN: few M-tiles, every one against the same weights): all M-tiles of
+// an N-block share an XCD instead, so each XCD reads its eighth of the weights once and every XCD is equally full.
+__device__ __forceinline__ bool prefill_block(uint32_t n_nblocks, bool nb_major, uint32_t &tile, uint32_t &nb) {
+    const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    if (nb_major) {
+        const uint32_t per_xcd = (n_nblocks + 7) / 8;
+        tile = slot / per_xcd;
+        nb = (slot % per_xcd) * 8 + xcd;
+        return nb < n_nblocks;
+    }
+    tile = (slot / n_nblocks) * 8 + xcd;
+    nb = slot % n_nblocks;
+    return true;
+}
+
 // F16: a context in FP16 mode - FP16 rows in, FP16 tiles, block-scaled FP16 activations, FP16 per-route rows out
 template <bool GATE_UP, bool F16 = false, bool DUMP = false>
 __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
@@ -634,21 +654,8 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(const uint8_t *__r
                                                               uint4 *__restrict__ dump = nullptr) {
     __shared__ __align__(16) uint4 wb[4][kTilesPerBlock][2][2][kWave];   // [buffer][tile][stream][k-half][lane]: group g lives in buffer g % 4
 
-    // Consecutive block ids go to consecutive XCDs. Many experts: all N-blocks of an M-tile share an XCD (its L2 holds
-    // the tile's A rows). One expert (the dense FFN: few M-tiles, every one against the same weights): all M-tiles of
-    // an N-block share an XCD instead, so each XCD reads its eighth of the weights once and every XCD is equally full.
-    const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     uint32_t ti, nb;
-    if (nb_major) {
-        const uint32_t per_xcd = (n_nblocks + 7) / 8;
-        ti = slot / per_xcd;
-        nb = (slot % per_xcd) * 8 + xcd;
-        if (nb >= n_nblocks) return;
-    } else {
-        ti = (slot / n_nblocks) * 8 + xcd;
-        nb = slot % n_nblocks;
-    }
-    if (ti >= plan->n_tiles) return;
+    if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;
     GemmWave gw;
     gw.tile = tiles[ti];
     gw.lane = threadIdx.x & 63;
@@ -681,6 +688,317 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(const uint8_t *__r
         case 3: gemm_wave<GATE_UP, 3, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
         default: gemm_wave<GATE_UP, 4, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
     }
+}
+
+// ---------------------------------------------------------------------------------------------------
+// Grouped product for chunks whose experts hold few pairs each (a short prompt): same tiles, same N-blocks and same
+// activation layout as the GEMM above, another way through them. There the expansion to 16-bit weights (some 120 vector
+// instructions per 1 KiB tile, whatever the pairs) bounds the launch below about 50 pairs per expert: 90 us for the
+// 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s. Here a wave owns one arena tile row for the whole of K, streams its
+// packed tiles through a ring of four and multiplies them in the offset form of the decode kernels (stream.hpp): about 75
+// vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. The pairs' rows go through LDS in
+// operand order, two groups at a time in two buffers, so that every wave of the block reads the same fragments and the
+// registers hold one chunk's 16-byte pieces in flight; the weights stay in flight across the barriers. Gate/up of 37 rows
+// 90 -> 55 us, of 301 rows 103 -> 70. What bounds it then is the weights' bytes (32 pairs per tile) and the matrix and
+// vector instructions together (64).
+// A pair's arithmetic does not depend on its tile: any two launches of this kernel give the same row bit for bit.
+// ---------------------------------------------------------------------------------------------------
+constexpr int kStreamDepth = 4;                                             // weight tiles in flight per wave
+constexpr int kStreamChunk = 2;                                             // groups whose rows are in LDS at a time, twice
+constexpr uint32_t kStreamStageRow = 2 * kTilesPerBlock * kTileRows * 2 + 16;   // bytes: 128 output columns + padding
+
+// The eight nibbles of a dword as matrix operands. bf16: 128 + q, as in the decode kernels. FP16: the nibble's bits as they
+// lie, i.e. the subnormal q * 2^-24 (exact, and the matrix unit takes FP16 subnormals): no offset to cancel. With 1024 + q
+// the fp32 sums of a group carry 1024 * sum x through their roundings, which made a 2,816-wide row's error against 64 bits
+// 3.60e-4 where the rounded weights of the GEMM have 3.58e-4.
+constexpr float kNibbleUnit = 16777216.0f;      // 2^24
+template <bool F16>
+__device__ __forceinline__ uint4 unpack8_stream(uint32_t w) {
+    if constexpr (!F16) return unpack8_offset<false>(w);
+    const uint32_t mask = 0x000F000Fu;
+    return make_uint4(w & mask, (w >> 4) & mask, (w >> 8) & mask, (w >> 12) & mask);
+}
+
+template <bool GATE_UP, int NM, bool F16>
+__device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom &g, const TileSource &src, uint32_t tile0,
+                                            uint4 *__restrict__ lds, const uint32_t *__restrict__ sorted_token,
+                                            const uint32_t *__restrict__ sorted_out_row, uint16_t *__restrict__ out,
+                                            float *__restrict__ act_scale) {
+    constexpr int CHUNK = kStreamChunk;
+    static_assert(2 * CHUNK % kStreamDepth == 0, "a group's ring slot follows from its place in a pair of chunks");
+    constexpr int kFrags = 2 * CHUNK;                     // operand fragments of a 16-pair block in a chunk
+    constexpr int kRowPieces = 8 * CHUNK;                 // 16-byte pieces of a row in a chunk
+    constexpr int kPassRows = 256 / kRowPieces;           // rows that the block's threads load at a time
+    constexpr int kPieces = 16 * NM / kPassRows;          // pieces of A per thread and chunk
+    constexpr int kBuf = NM * kFrags * kWave;             // one LDS buffer, in pieces
+    const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4, tid = threadIdx.x;
+    const uint32_t n_groups = gw.n_groups, last = n_groups - 1;
+    const uint32_t n_chunks = (n_groups + CHUNK - 1) / CHUNK;
+
+    // Where this thread's pieces of a chunk come from and go to.
+    // GATE_UP: row tid / kRowPieces + kPassRows k of the tile, piece tid % kRowPieces of its contiguous bytes; in LDS piece p of row r sits
+    // in fragment p / 4 at (p % 4, (r + p) % 16): the 16 pieces that 16 neighbouring lanes store then fall on 16
+    // different 16-byte columns, and so do the 16 rows that a fragment read takes.
+    // else: the activations are in fragment order already, the chunk of a 16-pair block is contiguous.
+    const uint16_t *from[GATE_UP ? kPieces : 1];
+    const uint32_t p = tid % kRowPieces, row0 = tid / kRowPieces;
+    if constexpr (GATE_UP) {
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            const uint32_t row = min(row0 + kPassRows * k, gw.tile.rows - 1);
+            from[k] = gw.a + (size_t)sorted_token[gw.tile.row_start + row] * gw.a_stride + (p & 7) * 8;
+        }
+    } else {
+        from[0] = gw.a + (size_t)gw.act_block0 * n_groups * (2 * kWave * 8) + (tid & 127) * 8;
+    }
+    u32x4_t stage[kPieces];        // (a native vector type: it stays in registers)
+    float rel[kPieces];
+    auto load_a = [&](uint32_t chunk) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            if constexpr (GATE_UP) {
+                const uint32_t grp = min(chunk * CHUNK + (p >> 3), last);        // past the end: the last group again, never used
+                stage[k] = *reinterpret_cast<const u32x4_t *>(from[k] + grp * kGroup);
+            } else {
+                const uint32_t grp = min(chunk * CHUNK + 2 * k % CHUNK + (tid >> 7), last);
+                stage[k] = *reinterpret_cast<const u32x4_t *>(from[0] + ((size_t)(2 * k / CHUNK) * n_groups + grp) * (2 * kWave * 8));
+                if constexpr (F16) rel[k] = act_scale[((size_t)(gw.act_block0 + 2 * k / CHUNK) * n_groups + grp) * 16 + (tid & 15)];
+            }
+        }
+    };
+    auto store_a = [&](uint32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            if constexpr (GATE_UP) {
+                const uint32_t row = row0 + kPassRows * k;
+                lds[buf * kBuf + ((row >> 4) * kFrags + (p >> 2)) * kWave + (p & 3) * 16 + ((row + p) & 15)] = __builtin_bit_cast(uint4, stage[k]);
+            } else {
+                uint4 v = __builtin_bit_cast(uint4, stage[k]);
+                if constexpr (F16) {
+                    const _Float16 r = (_Float16)rel[k];
+                    const f16x2 r2 = {r, r};
+                    v.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.x) * r2);
+                    v.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.y) * r2);
+                    v.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.z) * r2);
+                    v.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.w) * r2);
+                }
+                lds[buf * kBuf + 256 * k + tid] = v;
+            }
+        }
+    };
+    // fragment f of 16-pair block m, this lane's 16 bytes of it
+    auto frag = [&](uint32_t buf, int m, int f) __attribute__((always_inline)) {
+        const uint32_t at = GATE_UP ? jq * 16 + ((j + jq + 4 * (f & 3)) & 15) : lane;
+        return lds[buf * kBuf + (m * kFrags + f) * kWave + at];
+    };
+
+    uint4 ring_t[kStreamDepth];
+    uint2 ring_s[kStreamDepth];
+    auto fill = [&](int u, uint32_t grp) __attribute__((always_inline)) {
+        const uint32_t tile = __builtin_amdgcn_readfirstlane(tile0 + min(grp, last));
+        const u32x4_t t = __builtin_amdgcn_raw_buffer_load_b128(src.tiles, (int)(lane * 16u), (int)(tile * kTileBytes), 0);
+        const u32x2_t s = __builtin_amdgcn_raw_buffer_load_b64(src.scales, (int)(j * 8u), (int)(tile * kTileScaleBytes), 0);
+        ring_t[u] = make_uint4(t.x, t.y, t.z, t.w);
+        ring_s[u] = make_uint2(s.x, s.y);
+    };
+    TwoStreamAcc tot[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) tot[m].a = tot[m].b = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    auto step = [&](uint32_t buf, int gl, int u, uint32_t refill) __attribute__((always_inline)) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        const uint4 tile = ring_t[u];
+        const uint2 sc = ring_s[u];
+        fill(u, refill);
+        const uint4 wa0 = unpack8_stream<F16>(tile.x), wa1 = unpack8_stream<F16>(tile.y);
+        const uint4 wb0 = unpack8_stream<F16>(tile.z), wb1 = unpack8_stream<F16>(tile.w);
+        float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y), ta = bf16hi_to_f32(sc.x), tb = bf16hi_to_f32(sc.y);
+        if constexpr (F16) {
+            sa *= kNibbleUnit;
+            sb *= kNibbleUnit;
+        } else {
+            ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ta);
+            tb = __builtin_fmaf(-Act<F16>::kOffset, sb, tb);
+        }
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const uint4 x0 = frag(buf, m, 2 * gl), x1 = frag(buf, m, 2 * gl + 1);
+            const f32x4 sx = group_input_sum<F16>(x0, x1);
+            f32x4 aa = Act<F16>::mfma(x0, wa0, zero);
+            aa = Act<F16>::mfma(x1, wa1, aa);
+            f32x4 ab = Act<F16>::mfma(x0, wb0, zero);
+            ab = Act<F16>::mfma(x1, wb1, ab);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                tot[m].a[r] = __builtin_fmaf(sa, aa[r], tot[m].a[r]);
+                tot[m].a[r] = __builtin_fmaf(ta, sx[r], tot[m].a[r]);
+                tot[m].b[r] = __builtin_fmaf(sb, ab[r], tot[m].b[r]);
+                tot[m].b[r] = __builtin_fmaf(tb, sx[r], tot[m].b[r]);
+            }
+            // pinned: left alone, the compiler collects the scale-and-bias arithmetic of several groups and carries all
+            // their matrix results there, which does not fit the register budget
+#pragma unroll
+            for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(tot[m].a[r]), "+v"(tot[m].b[r]));
+        }
+    };
+
+    load_a(0);
+#pragma unroll
+    for (int u = 0; u < kStreamDepth; ++u) fill(u, u);
+    store_a(0);
+    load_a(min(1u, n_chunks - 1));
+    lds_barrier();
+    // chunk c from LDS buffer c % 2; chunk c + 1 goes from registers into the other one, chunk c + 2 into the registers.
+    // One barrier per chunk: the stores of chunk c + 1 in front of their reads, the reads of chunk c in front of the stores of
+    // chunk c + 2 into the same buffer.
+    auto chunk = [&](uint32_t c, auto parity, auto whole) __attribute__((always_inline)) {
+        constexpr int kFirst = decltype(parity)::value * CHUNK;
+        const uint32_t buf = c & 1;
+        store_a(buf ^ 1);               // (past the last chunk: a buffer nobody reads)
+        load_a(min(c + 2, n_chunks - 1));
+#pragma unroll
+        for (int gl = 0; gl < CHUNK; ++gl) {
+            const uint32_t grp = c * CHUNK + gl;
+            if (decltype(whole)::value || grp < n_groups) step(buf, gl, (kFirst + gl) % kStreamDepth, grp + kStreamDepth);
+        }
+        lds_barrier();
+    };
+    using Even = std::integral_constant<int, 0>;
+    using Odd = std::integral_constant<int, 1>;
+    using Whole = std::integral_constant<bool, true>;
+    using Part = std::integral_constant<bool, false>;
+    uint32_t c = 0;
+    for (; (c + 2) * CHUNK <= n_groups; c += 2) {
+        chunk(c, Even{}, Whole{});
+        chunk(c + 1, Odd{}, Whole{});
+    }
+    if (c < n_chunks) chunk(c, Even{}, Part{});
+    if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
+
+    // lane (j, jq) holds, per stream, weight row j of the tile row for pairs 4 jq .. 4 jq + 3 of every 16-pair block. The
+    // last chunk ended with a barrier: the LDS is free.
+    uint16_t *half = reinterpret_cast<uint16_t *>(lds);
+    if constexpr (GATE_UP) {
+        float h[NM][4];
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) h[m][r] = gelu_tanh_fast(tot[m].a[r]) * tot[m].b[r];
+        if constexpr (F16) {
+            // the block scale of a pair's 64 activations, as in gemm_wave's epilogue: sixteen lanes hold a quarter of them
+            float *peaks = reinterpret_cast<float *>(lds + NM * 2 * kWave);             // [wave][pair]
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = fabsf(h[m][r]);
+#pragma unroll
+                    for (int x = 1; x < 16; x <<= 1) v = fmaxf(v, __shfl_xor(v, x, 64));
+                    if (j == 0) peaks[wave * (16 * NM) + 16 * m + 4 * jq + r] = v;
+                }
+            lds_barrier();
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t pair = 16 * m + 4 * jq + r;
+                    float peak = 0.0f;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) peak = fmaxf(peak, peaks[v * (16 * NM) + pair]);
+                    int e = 0;
+                    (void)frexpf(peak, &e);
+                    e = max(e, -100);
+                    h[m][r] *= ldexpf(1.0f, 14 - e);
+                    if (wave == 0 && j == 0)
+                        act_scale[((size_t)(gw.act_block0 + m) * g.gf + gw.nb) * 16 + 4 * jq + r] = ldexpf(1.0f, e - 14);
+                }
+        }
+        // this wave's k = 16 wave + j of the block's group of F: k-half wave / 2, operand lane (pair, 2 (wave % 2) + j / 8)
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                half[((m * 2 + (wave >> 1)) * kWave + ((wave & 1) * 2 + (j >> 3)) * 16 + 4 * jq + r) * 8 + (j & 7)] = Act<F16>::round(h[m][r]);
+        lds_barrier();
+        for (uint32_t i = tid; i < (uint32_t)NM * 2 * kWave; i += 256) {
+            const uint32_t m = i / (2 * kWave), at = i % (2 * kWave);
+            *reinterpret_cast<uint4 *>(out + (((size_t)(gw.act_block0 + m) * g.gf + gw.nb) * 2 * kWave + at) * 8) = lds[i];
+        }
+        return;
+    }
+    uint8_t *rows = reinterpret_cast<uint8_t *>(lds);
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t pair = 16 * m + 4 * jq + r;
+            float va = tot[m].a[r], vb = tot[m].b[r];
+            if constexpr (F16) {
+                const float largest = act_scale[(size_t)gw.act_blocks * g.gf * 16 + (gw.act_block0 + m) * 16 + 4 * jq + r];
+                va *= largest;
+                vb *= largest;
+            }
+            uint16_t *dst = reinterpret_cast<uint16_t *>(rows + pair * kStreamStageRow) + 32 * wave + j;
+            dst[0] = Act<F16>::round(va);
+            dst[16] = Act<F16>::round(vb);
+        }
+    lds_barrier();
+    const uint32_t piece = tid & 15;
+    if (gw.nb * kTilesPerBlock + (piece >> 2) < gw.n_arena_tiles) {
+#pragma unroll
+        for (int k = 0; k < NM; ++k) {
+            const uint32_t row = (tid >> 4) + 16 * k;
+            if (row < gw.tile.rows)
+                *reinterpret_cast<uint4 *>(out + (size_t)sorted_out_row[gw.tile.row_start + row] * g.d +
+                                           gw.nb * (2 * kTilesPerBlock * kTileRows) + 8 * piece) =
+                    *reinterpret_cast<const uint4 *>(rows + row * kStreamStageRow + 16 * piece);
+        }
+    }
+}
+
+// MAX_NM: 16-pair blocks of the largest tile the plan cut
+template <bool GATE_UP, int MAX_NM, bool F16, int WAVES>
+__global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
+                                                                    const PrefillPlan *__restrict__ plan,
+                                                                    const PrefillTile *__restrict__ tiles,
+                                                                    const uint32_t *__restrict__ sorted_token,
+                                                                    const uint32_t *__restrict__ sorted_out_row,
+                                                                    const uint16_t *__restrict__ a, uint32_t a_stride,
+                                                                    uint16_t *__restrict__ out, uint32_t n_nblocks, bool nb_major,
+                                                                    float *__restrict__ act_scale, uint32_t act_blocks) {
+    __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave];
+    static_assert(16 * MAX_NM * kStreamStageRow <= sizeof(lds), "the down epilogue's rows fit");
+    uint32_t ti, nb;
+    if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;
+    GemmWave gw;
+    gw.tile = tiles[ti];
+    gw.lane = threadIdx.x & 63;
+    gw.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    gw.n_groups = GATE_UP ? g.gd : g.gf;
+    gw.n_arena_tiles = GATE_UP ? g.gu_rb : g.dn_rbp;
+    gw.nb = nb;
+    gw.a = a;
+    gw.a_stride = a_stride;
+    gw.act_block0 = gw.tile.row_start / 16 + gw.tile.order;
+    gw.act_blocks = act_blocks;
+    gw.w_tiles = gw.w_scales = nullptr;
+    // the tile row this wave multiplies; past the last one the last again (never stored)
+    const uint32_t at = min(nb * kTilesPerBlock + gw.wave, gw.n_arena_tiles - 1);
+    const uint8_t *expert_base = arena_layer + (size_t)__builtin_amdgcn_readfirstlane(gw.tile.expert) * g.expert_bytes;
+    const size_t n_tiles = (size_t)gw.n_arena_tiles * gw.n_groups;
+    const TileSource src = make_tile_source(expert_base + (GATE_UP ? g.gu_tiles_off : g.dn_tiles_off), n_tiles * kTileBytes,
+                                            expert_base + (GATE_UP ? g.gu_scales_off : g.dn_scales_off), n_tiles * kTileScaleBytes);
+    const uint32_t tile0 = at * gw.n_groups;
+#define FFMOE_STREAM(N)                                                                                                      \
+    if constexpr (N <= MAX_NM)                                                                                               \
+        stream_tile<GATE_UP, N, F16>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale)
+    switch (__builtin_amdgcn_readfirstlane((gw.tile.rows + 15) / 16)) {
+        case 1: FFMOE_STREAM(1); break;
+        case 2: FFMOE_STREAM(2); break;
+        case 3: FFMOE_STREAM(3); break;
+        default: FFMOE_STREAM(4); break;
+    }
+#undef FFMOE_STREAM
 }
 
 // Between the two GEMMs of the FP16 prefill: a pair's block scales divided by its largest (powers of two: exact), the
@@ -768,6 +1086,30 @@ __global__ void prefill_dump_plan_kernel(uint32_t expert, PrefillPlan *plan, Pre
     sorted_out_row[0] = 0;
 }
 
+// Pairs per M-tile, as a shift: below 8 (256 pairs) the chunk goes through prefill_stream_kernel. The line is drawn by the
+// pairs per expert on average, from the chunk's size alone: the counts themselves are only known on the device, and a pair
+// list's rows do not depend on how many of the chunk's pairs it names. Router table to combined rows, 128 experts, top-8,
+// 2,816 x 704, us at 32 | 64 | 256 pairs per tile, bf16 (FP16): 37 rows 97 | 101 | 143 (106 | 110 | 174), 301 rows
+// 120 | 126 | 172 (130 | 137 | 191), 400 rows (25 pairs) 129 | 137 | 177, 512 rows (32) 152 | 147 | 182, 700 rows (44)
+// 196 | 170 | 195 (215 | 183 | 211), 1,000 rows (62, where many experts take two tiles) 218 | 220 | 219. Tiles of 16 pairs
+// gain nothing over 32 (37 rows: 99), tiles of 128 lose everywhere (1,000 rows: 227, two waves per SIMD).
+uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts) {
+    if (n_items <= 28 * n_experts) return 5;
+    if (n_items <= kPrefillStreamPairs * n_experts) return 6;
+    return 8;
+}
+
+// The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths). 2,816 -> 2,112 -> 2,816, us at
+// 32 | 64 | 256 rows per tile, bf16 (FP16): 512 rows 51 | 64 | 79 (70 | 84 | 109), 700 rows 66 | 71 | 79 (86 | 93 | 109),
+// 1,000 rows 80 | 83 | 80 (101 | 106 | 109).
+uint32_t dense_tile_shift(uint32_t t) { return t <= kDenseTileStreamRows ? 5 : 8; }
+
+template <bool GATE_UP>
+auto stream_kernel(uint32_t tile_shift, bool f16) {
+    if (tile_shift == 5) return f16 ? prefill_stream_kernel<GATE_UP, 2, true, 4> : prefill_stream_kernel<GATE_UP, 2, false, 4>;
+    return f16 ? prefill_stream_kernel<GATE_UP, 4, true, 3> : prefill_stream_kernel<GATE_UP, 4, false, 3>;
+}
+
 }  // namespace
 
 uint32_t prefill_dump_fragments(const ArenaGeom &g, bool gate_up) {
@@ -812,44 +1154,49 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     src.t = t;
     if (src.n_items == 0) return hipSuccess;
     const uint32_t n_blocks = (src.n_items + kSortBlock - 1) / kSortBlock;
+    const uint32_t tile_shift = dense ? dense_tile_shift(t) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts);
+    const bool streamed = tile_shift < 8;
     if (dense) {
-        hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, sc.plan, sc.tiles, sc.sorted_token,
+        hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_shift, sc.plan, sc.tiles, sc.sorted_token,
                            sc.sorted_out_row);
     } else {
         hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
         uint32_t e_pad = 1;
         while (e_pad < n_experts) e_pad <<= 1;          // n_experts <= FFMOE_MAX_EXPERTS = 256 <= kScanThreads
         hipLaunchKernelGGL(prefill_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, n_blocks, n_experts, e_pad, sc.block_cnt,
-                           sc.plan, sc.tiles, sc.max_tiles);
+                           sc.plan, sc.tiles, sc.max_tiles, tile_shift);
         hipLaunchKernelGGL(prefill_scatter_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt, sc.sorted_token,
                            sc.sorted_out_row);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     timer->mark(s, FFMOE_K_PREFILL_SORT);
-    const uint32_t tile_cap = min(sc.max_tiles, (src.n_items + kBM - 1) / kBM + n_experts);
+    const uint32_t tile_cap = min(sc.max_tiles, (src.n_items >> tile_shift) + n_experts);
     const uint32_t tile_slots = (tile_cap + 7) / 8 * 8;
     const uint32_t nb_gu = (g.gu_rb + kTilesPerBlock - 1) / kTilesPerBlock, nb_dn = (g.dn_rbp + kTilesPerBlock - 1) / kTilesPerBlock;
     if (f16 && !sc.act_scale) return hipErrorInvalidValue;      // allocated when the context was switched to FP16
     // grid: (N-blocks x tile slots) in either order of the kernel's block map
     const bool nb_major = n_experts == 1;
     auto grid_of = [&](uint32_t n_nblocks) { return nb_major ? 8 * ((n_nblocks + 7) / 8) * tile_cap : n_nblocks * tile_slots; };
-    if (f16)
-        hipLaunchKernelGGL((prefill_gemm_kernel<true, true>), dim3(grid_of(nb_gu)), dim3(256), 0, s, arena_layer, g, sc.plan,
-                           sc.tiles, sc.sorted_token, sc.sorted_out_row, x, x_stride, sc.acts, nb_gu, nb_major, sc.act_scale, sc.act_blocks);
-    else
-        hipLaunchKernelGGL((prefill_gemm_kernel<true, false>), dim3(grid_of(nb_gu)), dim3(256), 0, s, arena_layer, g, sc.plan,
-                           sc.tiles, sc.sorted_token, sc.sorted_out_row, x, x_stride, sc.acts, nb_gu, nb_major, nullptr, 0u);
-    timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
     uint16_t *partials = partials_out ? partials_out : sc.partials;
+    float *act_scale = f16 ? sc.act_scale : nullptr;
+    const uint32_t act_blocks = f16 ? sc.act_blocks : 0u;
+#define FFMOE_GEMM(GU, A, STRIDE, OUT, NB)                                                                                    \
+    hipLaunchKernelGGL((f16 ? prefill_gemm_kernel<GU, true> : prefill_gemm_kernel<GU, false>), dim3(grid_of(NB)), dim3(256), 0, s, \
+                       arena_layer, g, sc.plan, sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major,    \
+                       act_scale, act_blocks, nullptr)
+#define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
+    hipLaunchKernelGGL(stream_kernel<GU>(tile_shift, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
+                       sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major, act_scale, act_blocks)
+    if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);
+    else FFMOE_GEMM(true, x, x_stride, sc.acts, nb_gu);
+    timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
     if (f16)
         hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap), dim3(kBM), 0, s, sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale);
-    if (f16)
-        hipLaunchKernelGGL((prefill_gemm_kernel<false, true>), dim3(grid_of(nb_dn)), dim3(256), 0, s, arena_layer, g, sc.plan,
-                           sc.tiles, sc.sorted_token, sc.sorted_out_row, sc.acts, g.f, partials, nb_dn, nb_major, sc.act_scale, sc.act_blocks);
-    else
-        hipLaunchKernelGGL((prefill_gemm_kernel<false, false>), dim3(grid_of(nb_dn)), dim3(256), 0, s, arena_layer, g, sc.plan,
-                           sc.tiles, sc.sorted_token, sc.sorted_out_row, sc.acts, g.f, partials, nb_dn, nb_major, nullptr, 0u);
+    if (streamed) FFMOE_STREAM(false, sc.acts, g.f, partials, nb_dn);
+    else FFMOE_GEMM(false, sc.acts, g.f, partials, nb_dn);
+#undef FFMOE_GEMM
+#undef FFMOE_STREAM
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     timer->mark(s, FFMOE_K_PREFILL_DOWN);

@@ -1,0 +1,108 @@
+"""The prefill's streaming product (chunks whose experts hold few pairs): experts with 0, 1 and every count around a 16-pair
+block, around a tile of 32 and of 64 pairs, K of whole and of ragged chunks, output columns that do not fill an N-block, both
+activation types, and the line between it and the grouped GEMMs. Run on the GPU box: pytest -m gpu."""
+import numpy as np
+import pytest
+
+from helpers import bf16_tensor, bits_of, cosine, make_layer, rel_err, to_ff_offsets
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = (0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 97, 130)
+
+
+def _routes(rng, counts, e):
+    """One route per token (top_k = 1), counts[i] tokens for expert i, tokens shuffled."""
+    idx = np.repeat(np.arange(e, dtype=np.uint32), counts)
+    rng.shuffle(idx)
+    return idx[:, None]
+
+
+# d, f: (groups of d, groups of f) = whole pairs of chunks, one ragged chunk, three groups past a pair; 320 columns = 2.5 N-blocks
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,scale", [(256, 128, 1), (320, 192, 1), (448, 64, 2), (64, 704, 2)])
+def test_tile_edges_against_the_oracle(oracle, act, d, f, scale):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    e = len(COUNTS) * scale                       # scale 1: 38 pairs per expert on average (tiles of 64), 2: 19 (tiles of 32)
+    counts = np.array(COUNTS + (0,) * (e - len(COUNTS)))
+    rng, pool, _ = make_layer(oracle, 77 + d, d, f, e, align=1)
+    idx = _routes(rng, counts, e)
+    t = idx.shape[0]
+    assert t <= 48 * e
+    ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt)
+        w = torch.from_numpy(rng.uniform(0.2, 1.0, (t, 1)).astype(np.float32)).to(dt)
+        gi = torch.from_numpy(idx.view(np.int32)).cuda()
+        y = ctx.prefill(0, x.cuda(), gi, w.cuda()).float().cpu().numpy()
+        n_pairs, n_tiles, got_counts = ctx.prefill_stats()
+        assert n_pairs == t and np.array_equal(got_counts, counts)
+        xf, wf = x.float().numpy(), w.float().numpy()
+        ref, spread = np.zeros((t, d), np.float64), np.zeros((t, d), np.float64)
+        for ex in range(e):
+            rows = np.flatnonzero(idx[:, 0] == ex)
+            if len(rows):
+                g, u, dn = (oracle.dequantize_int4(*pool.sub(ex, n)).astype(np.float64) for n in ("gate", "up", "down"))
+                gate, up = xf[rows] @ g.T, xf[rows] @ u.T
+                act_rows = 0.5 * gate * (1 + np.tanh(0.7978845608028654 * (gate + 0.044715 * gate ** 3))) * up
+                ref[rows] = wf[rows] * (act_rows @ dn.T)
+                spread[rows] = wf[rows] * (np.abs(act_rows) @ np.abs(dn.T))
+        # element by element: every activation rounded once (unit 2^-8 in bf16, 2^-11 in FP16, through the down product's
+        # absolute sum), the per-route row and the weighted row once each; a tenth on top for the fp32 sums in the offset form
+        unit = 2.0 ** (-8 if act == "bf16" else -11)
+        assert np.all(np.abs(y - ref) <= 1.1 * unit * (spread + 2 * np.abs(ref)) + 1e-6 * np.abs(ref).max())
+        # a pair's row does not depend on the pairs beside it: the chunk's first half alone, in tiles cut elsewhere
+        half = t // 2
+        part = ctx.prefill(0, x[:half].cuda(), gi[:half].contiguous(), w[:half].cuda()).float().cpu().numpy()
+        assert np.array_equal(part, y[:half])
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("t", [47, 48, 49])
+def test_the_line_to_the_grouped_gemms(oracle, t):
+    # four experts, top-4: t pairs each; 48 per expert is the last chunk that streams. Either side to the same bar.
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, e = 128, 128, 4
+    rng, pool, _ = make_layer(oracle, 5, d, f, e, align=1)
+    ctx = ff.Context(d, f, e, 4, n_layers=1, max_tokens=64)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        xb = oracle.bf16_bits(rng.normal(0, 1, (t, d)).astype(np.float32))
+        idx = np.stack([rng.permutation(4) for _ in range(t)]).astype(np.uint32)
+        wb = oracle.bf16_bits(rng.dirichlet(np.ones(4), size=t).astype(np.float32))
+        y = oracle.bf16_to_float(bits_of(ctx.prefill(0, bf16_tensor(torch, xb), torch.from_numpy(idx.view(np.int32)).cuda(), bf16_tensor(torch, wb))))
+        ref = oracle.moe_experts(pool, xb, idx, oracle.bf16_to_float(wb))
+        assert rel_err(y, ref) <= 1e-2 and cosine(y, ref) >= 0.9999
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("t", [385, 895, 896, 897])
+def test_dense_chunks_beyond_the_gemv(oracle, act, t):
+    # a dense FFN's chunk: tiles of 32 rows up to 896 rows, the GEMMs from there on
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f = 192, 320
+    g = oracle.seed_tree_key(0x5EED, f"dense-tiles-{t}")
+    parts = tuple(oracle.quantize_int4(g.uniform(-0.3, 0.3, r * c).reshape(r, c)) for r, c in ((f, d), (f, d), (d, f)))
+    x = torch.from_numpy(g.uniform(-1.0, 1.0, t * d).reshape(t, d).astype(np.float32)).to(torch.bfloat16 if act == "bf16" else torch.float16)
+    ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_expert_parts(0, 0, *parts)
+        y = ctx.dense_ffn(0, x.cuda()).float().cpu().numpy()
+        gw, uw, dw = (oracle.dequantize_int4(*p).astype(np.float64) for p in parts)
+        xf = x.float().numpy()
+        gate, up = xf @ gw.T, xf @ uw.T
+        ref = (0.5 * gate * (1 + np.tanh(0.7978845608028654 * (gate + 0.044715 * gate ** 3))) * up) @ dw.T
+        assert rel_err(y, ref) <= 1e-2 and cosine(y, ref) >= 0.9999
+    finally:
+        ctx.close()
