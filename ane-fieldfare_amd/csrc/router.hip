@@ -15,7 +15,9 @@
 namespace ffmoe {
 namespace {
 
-// Decode / verify router logits (T <= 16). grid = (E, ceil(T / 4)); the four waves of a block are the
+constexpr uint32_t kRouterSmallRows = 160;     // the most rows that take the form below where the two-pass form could serve
+
+// Decode / verify / short-prompt router logits. grid = (E, ceil(T / 4)); the four waves of a block are the
 // four sub-accumulators of one expert row for four tokens; wave 0 combines them. (A variant whose last
 // block also selected the top-k behind a device-scope counter measured 2.5x slower: every block paid
 // for the same-address atomic and the L2 write-back of its release fence.)
@@ -491,7 +493,14 @@ hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uin
     timer->begin(s);
     const bool x_aligned = (reinterpret_cast<uintptr_t>(x) % 8 == 0) && (x_stride % 4 == 0);
     if (f16 && !x_aligned) return hipErrorInvalidValue;     // FP16 rows come 8-byte aligned (checked at the boundary)
-    if (t <= FFMOE_MAX_VERIFY_ROWS) {
+    const bool two_pass = rw.w_frag && !rw.w_is_f32 && !rw.effective_scale && !want_logits && d % 256 == 0 && d <= 1024 * kExactSteps &&
+                          n_experts % 16 == 0 && n_experts <= 128 && top_k <= 8 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                          x_stride % 8 == 0 && scratch;
+    // The two passes of the prefill form are two chains of round trips, 19 us (FP16: 22) however few the rows; one block per
+    // expert and four rows costs the router's weights once more from the caches for every four rows. 2,816 x 128, two-pass
+    // form against this one, us, bf16 (FP16): 17 rows 18.6 | 8.0 (22.2 | 7.9), 64 rows 18.8 | 10.3, 128 rows 19.1 | 14.8
+    // (22.5 | 14.7), 160 rows 19.3 | 16.9, 200 rows 19.6 | 19.8 (22.8 | 19.9). Same pinned sums: same routes bit for bit.
+    if (t <= FFMOE_MAX_VERIFY_ROWS || (two_pass && t <= kRouterSmallRows)) {
         const dim3 grid(n_experts, (t + kChunkTokens - 1) / kChunkTokens);
 #define FFMOE_ROUTER(WF, XA)                                                                                 \
     hipLaunchKernelGGL((router_small_kernel<WF, XA>), grid, dim3(256), 0, s, rw.w, rw.effective_scale, x,   \
@@ -506,8 +515,7 @@ hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uin
         timer->finish();
         return hipGetLastError();
     }
-    if (rw.w_frag && !rw.w_is_f32 && !rw.effective_scale && !want_logits && d % 256 == 0 && d <= 1024 * kExactSteps &&
-        n_experts % 16 == 0 && n_experts <= 128 && top_k <= 8 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_stride % 8 == 0 && scratch) {
+    if (two_pass) {
         // approximate logits of every expert on the matrix unit, the pinned ones only where the select can tell
         const uint32_t t_pad = (t + 63) & ~63u;
         float *xnorm2 = scratch, *approx = scratch + (size_t)kApproxKParts * t_pad;
