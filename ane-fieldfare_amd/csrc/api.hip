@@ -31,12 +31,18 @@ struct ffmoe_layer {
     // the same weights as hi + lo rows of the activation type for the library GEMM that serves large row counts
     // ([4 f][d] and [2 d][f]); null when the context's max_tokens stays below the row count from which it is used
     uint16_t *gate_up8_hilo = nullptr, *down8_hilo = nullptr;
+    // and as the integer operands of the GEMMs that serve the largest (dense8.hip); null below their row count likewise
+    uint8_t *gate_up8_ops = nullptr, *down8_ops = nullptr;
 };
 
 // From this many rows on an 8-bit dense layer goes through the library's dense GEMM on hi / lo rows instead of one
 // streaming pass per 16 rows (measured at 2816 -> 2112 -> 2816: streaming 19 us at 32 rows + 8.8 us per 32 more, 42 us at
 // 127; the GEMM form 50 us at 128, 58 at 192, 67 at 256, 100 at 1,024, 244 at 3,072).
 constexpr uint32_t kGemm8MinRows = 192;
+// And from this many the GEMMs on integer operands (dense8.hip), which do half the products; below, their blocks are too few to
+// hide a group's round trip. Library form | integer form, us: 301 rows 48 | 61, 512 rows 61 | 65, 700 rows 74 | 69, 1,000 rows
+// 97 | 85, 1,500 rows 124 | 102, 3,072 rows 248 | 181.
+constexpr uint32_t kDense8MinRows = 640;
 // Up to this many rows a 4-bit dense layer streams its arena tiles through the resident-matrix GEMV (a grid row per 16
 // input rows) instead of the grouped products (which beat it from about 200 rows on in bf16 and 370 in FP16: 384 rows 66 us
 // against 45 and 64; the rows of a chunk and of a part of it are equal bit for bit up to here, so the line stays put).
@@ -78,7 +84,8 @@ struct ffmoe_ctx {
     bool f16 = false;                // activations are FP16 (ffmoe_set_activation_dtype)
     // the 8-bit dense layers' GEMM form: the library handle and the fp32 sums [max_tokens][max(4 f, 2 d)]
     rocblas_handle blas = nullptr;
-    float *gemm8_sums = nullptr;
+    float *gemm8_sums = nullptr;                                // sums of kDense8MinRows rows at most
+    uint8_t *dense8_x = nullptr, *dense8_acts = nullptr;        // the integer form's inputs as operands, max_tokens rows
     SampleScratch sample{};          // what the sampled choice over long rows leaves between its two launches
     KernelTimer timer;
     std::vector<ffmoe_matrix *> matrices;   // resident matrices created on this context and not yet destroyed
@@ -212,15 +219,24 @@ void drop_int8_form(ffmoe_layer &l) {
     if (l.gate_up8_hilo) (void)hipFree(l.gate_up8_hilo);
     if (l.down8_hilo) (void)hipFree(l.down8_hilo);
     l.gate_up8_hilo = l.down8_hilo = nullptr;
+    if (l.gate_up8_ops) (void)hipFree(l.gate_up8_ops);
+    if (l.down8_ops) (void)hipFree(l.down8_ops);
+    l.gate_up8_ops = l.down8_ops = nullptr;
 }
 
-// (Re)makes the hi / lo rows of an 8-bit layer in the context's activation type from its nibble planes. Blocking.
+// (Re)makes the GEMM forms of an 8-bit layer in the context's activation type from its nibble planes. Blocking.
 hipError_t expand_int8_layer(ffmoe_ctx *ctx, ffmoe_layer &l) {
     if (!l.gate_up8_hilo) return hipSuccess;
     hipError_t e = launch_expand_planes8(nullptr, l.gate_up8->tiles, l.gate_up8->scales, ctx->shape.f, ctx->shape.d, true,
                                          l.gate_up8_hilo, ctx->f16);
     if (e == hipSuccess)
         e = launch_expand_planes8(nullptr, l.down8->tiles, l.down8->scales, ctx->shape.d, ctx->shape.f, false, l.down8_hilo, ctx->f16);
+    if (l.gate_up8_ops) {
+        if (e == hipSuccess)
+            e = launch_dense8_weights(nullptr, l.gate_up8->tiles, l.gate_up8->scales, 2 * ctx->shape.f, ctx->shape.d, l.gate_up8_ops, ctx->f16);
+        if (e == hipSuccess)
+            e = launch_dense8_weights(nullptr, l.down8->tiles, l.down8->scales, ctx->shape.d, ctx->shape.f, l.down8_ops, ctx->f16);
+    }
     if (e == hipSuccess) e = hipDeviceSynchronize();
     return e;
 }
@@ -339,6 +355,8 @@ void ffmoe_destroy(ffmoe_ctx *ctx) {
     (void)hipDeviceSynchronize();
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
     if (ctx->gemm8_sums) (void)hipFree(ctx->gemm8_sums);
+    if (ctx->dense8_x) (void)hipFree(ctx->dense8_x);
+    if (ctx->dense8_acts) (void)hipFree(ctx->dense8_acts);
     for (auto &l : ctx->layers) {
         // the layer's own 8-bit matrices: nobody else holds their handles
         drop_int8_form(l);
@@ -819,6 +837,17 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
             return fail(err, FFMOE_ERR_INVALID, "x must be 16-byte aligned with a stride that is a multiple of 8 and >= d");
         hipStream_t s = static_cast<hipStream_t>(stream);
         claim_scratch(ctx, stream);
+        if (t >= kDense8MinRows && l.gate_up8_ops) {
+            const uint32_t f = ctx->shape.f, d = ctx->shape.d;
+            ctx->timer.begin(s);
+            FF_HIP(launch_dense8_rows(s, x, x_stride, t, d, f, ctx->dense8_x, ctx->dense8_acts, ctx->f16));
+            FF_HIP(launch_dense8_gemm(s, l.gate_up8_ops, 2 * f, d, true, ctx->dense8_x, t, ctx->dense8_acts, 0, ctx->f16));
+            ctx->timer.mark(s, FFMOE_K_GATE_UP);
+            FF_HIP(launch_dense8_gemm(s, l.down8_ops, d, f, false, ctx->dense8_acts, t, y, d, ctx->f16));
+            ctx->timer.mark(s, FFMOE_K_DOWN);
+            ctx->timer.finish();
+            return FFMOE_OK;
+        }
         if (t >= kGemm8MinRows && l.gate_up8_hilo) {
             // many rows: two dense GEMMs of the library on the hi / lo rows (fp32 sums), each followed by the pass that adds
             // a weight row's two columns and rounds as the streaming form does
@@ -1252,7 +1281,14 @@ int ffmoe_upload_expert_parts_int8(ffmoe_ctx *ctx, uint32_t layer, const ffmoe_p
         hipError_t e = hipSuccess;
         if (!ctx->gemm8_sums)
             e = hipMalloc(reinterpret_cast<void **>(&ctx->gemm8_sums),
-                          (size_t)sh.max_tokens * std::max(4 * (size_t)sh.f, 2 * (size_t)sh.d) * sizeof(float));
+                          (size_t)std::min(sh.max_tokens, kDense8MinRows) * std::max(4 * (size_t)sh.f, 2 * (size_t)sh.d) * sizeof(float));
+        if (sh.max_tokens >= kDense8MinRows) {
+            if (e == hipSuccess && !ctx->dense8_x) e = hipMalloc(reinterpret_cast<void **>(&ctx->dense8_x), dense8_operand_bytes(sh.max_tokens, sh.d));
+            if (e == hipSuccess && !ctx->dense8_acts)
+                e = hipMalloc(reinterpret_cast<void **>(&ctx->dense8_acts), dense8_operand_bytes(sh.max_tokens, sh.f));
+            if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&l.gate_up8_ops), dense8_weight_bytes(2 * sh.f, sh.d));
+            if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&l.down8_ops), dense8_weight_bytes(sh.d, sh.f));
+        }
         if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&l.gate_up8_hilo), (size_t)4 * sh.f * sh.d * sizeof(uint16_t));
         if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&l.down8_hilo), (size_t)2 * sh.d * sh.f * sizeof(uint16_t));
         if (e == hipSuccess) e = expand_int8_layer(ctx, l);

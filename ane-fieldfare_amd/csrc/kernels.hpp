@@ -240,6 +240,16 @@ inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts) {
     return (whole > small ? whole : small) + n_experts + 1;
 }
 
+// dense8.hip: the 8-bit dense FFN at many rows. `stored_rows` = rows of the resident matrix as stored (the gated one: 2 f).
+size_t dense8_weight_bytes(uint32_t stored_rows, uint32_t n);
+size_t dense8_operand_bytes(uint32_t rows, uint32_t n);
+hipError_t launch_dense8_weights(hipStream_t s, const uint8_t *tiles, const uint8_t *scales, uint32_t stored_rows, uint32_t n, void *out,
+                                 bool f16);
+hipError_t launch_dense8_rows(hipStream_t s, const uint16_t *x, uint32_t x_stride, uint32_t t, uint32_t d, uint32_t f, void *x_ops,
+                              void *act_ops, bool f16);
+hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t stored_rows, uint32_t n, bool gated, const void *ops, uint32_t t,
+                              void *out, uint32_t out_stride, bool f16);
+
 // prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr.
 // Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,

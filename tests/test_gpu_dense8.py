@@ -1,0 +1,69 @@
+"""The 8-bit dense layer's GEMMs on integer operands (640 rows and more): ragged row tiles either side of the tile sizes, an
+output width that fills half a block of columns, widths of an odd number of groups, both activation types, inputs with a large
+common part (so that the bias columns carry most of a sum), rows that overflow. Run on the GPU box: pytest -m gpu."""
+import numpy as np
+import pytest
+
+from helpers import cosine, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _gelu(x):
+    return 0.5 * x * (1 + np.tanh(0.7978845608028654 * (x + 0.044715 * x ** 3)))
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,t", [(128, 64, 640), (192, 320, 641), (64, 704, 703), (192, 1472, 1088), (448, 192, 1089), (2816, 128, 1153)])
+def test_rows_against_float64(oracle, act, d, f, t):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    g = oracle.seed_tree_key(0x1A8, f"dense8-{d}-{f}-{t}")
+    parts = tuple(oracle.quantize_int8(g.uniform(-0.2, 0.2, r * c).reshape(r, c)) for r, c in ((f, d), (f, d), (d, f)))
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    x = torch.from_numpy((g.uniform(-1.0, 1.0, t * d) + 0.5).reshape(t, d).astype(np.float32)).to(dt)
+    ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_expert_parts(0, 0, *parts, int8=True)
+        y = ctx.dense_ffn(0, x.cuda())
+        yf = y.float().cpu().numpy()
+        gw, uw, dw = (oracle.dequantize_int8(*p).astype(np.float64) for p in parts)
+        xf = x.double().numpy()
+        # as the layer rounds: gate and up to the activation type, the product once more, the output row
+        rnd = lambda a: torch.from_numpy(a).to(torch.float32).to(dt).double().numpy()
+        a = rnd(_gelu(rnd(xf @ gw.T)) * rnd(xf @ uw.T))
+        ref, spread = a @ dw.T, np.abs(a) @ np.abs(dw.T)
+        # where a sum falls near a rounding's middle, the fp32 sum may round the other way: one unit (2^-8 bf16, 2^-11 FP16) of
+        # gate, up and the activation each (gelu' is below 1.13), through the down product; then the output's own half unit
+        unit = 2.0 ** (-8 if act == "bf16" else -11)
+        assert np.all(np.abs(yf - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
+        assert cosine(yf, ref) > 0.99999 and rel_err(yf, ref) < (1e-2 if act == "bf16" else 1.5e-3)
+        # a row does not depend on the rows beside it (both tile sizes sum in one order)
+        if t > 1088:
+            part = ctx.dense_ffn(0, x[:1088].cuda()).float().cpu().numpy()
+            assert np.array_equal(part, yf[:1088])
+        # other rows are untouched by one that is not finite
+        x[7, 3] = float("inf")
+        got = ctx.dense_ffn(0, x.cuda()).float().cpu().numpy()
+        assert not np.isfinite(got[7]).any() and np.array_equal(np.delete(got, 7, 0), np.delete(yf, 7, 0))
+    finally:
+        ctx.close()
+
+
+def test_the_form_follows_the_activation_type(oracle):
+    # the operands are remade when the context changes type, and given back with a 4-bit upload
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, t = 128, 192, 650
+    g = oracle.seed_tree_key(0x1A8, "dense8-types")
+    parts = tuple(oracle.quantize_int8(g.uniform(-0.2, 0.2, r * c).reshape(r, c)) for r, c in ((f, d), (f, d), (d, f)))
+    x = torch.from_numpy(g.uniform(-1.0, 1.0, t * d).reshape(t, d).astype(np.float32))
+    outs = {}
+    for act in ("bf16", "fp16"):
+        ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+        ctx.upload_expert_parts(0, 0, *parts, int8=True)
+        outs[act] = ctx.dense_ffn(0, x.to(torch.bfloat16 if act == "bf16" else torch.float16).cuda()).float().cpu().numpy()
+        ctx.close()
+    assert rel_err(outs["bf16"], outs["fp16"]) < 2e-2 and not np.array_equal(outs["bf16"], outs["fp16"])
