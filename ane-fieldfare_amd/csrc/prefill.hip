@@ -68,8 +68,10 @@ __global__ __launch_bounds__(kSortBlock) void prefill_hist_kernel(ItemSource src
 // of sort blocks, so the counts of a whole column are in flight at once and - up to kScanKeep per thread -
 // stay in registers between the summing pass and the pass that writes the bases.
 constexpr int kScanThreads = 1024;
-constexpr int kScanKeep = 32;         // 8,192 rows x 8 routes with 128 experts: 15.4 -> 10.3 us (16 kept half of a run, the rest was read twice)
+// (kScanKeep: 16, or 32 where a thread's run is longer - 8,192 rows x 8 routes with 128 experts: 15.4 -> 10.3 us, the second half of
+// a run was read twice; short runs pay for the longer unrolled passes, 443.1 against 441.4 us for a plugin chunk of 3,079 rows)
 
+template <int kScanKeep>
 __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad,
                                                                     uint32_t *__restrict__ block_cnt,
                                                                     PrefillPlan *__restrict__ plan,
@@ -1163,8 +1165,9 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
         hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
         uint32_t e_pad = 1;
         while (e_pad < n_experts) e_pad <<= 1;          // n_experts <= FFMOE_MAX_EXPERTS = 256 <= kScanThreads
-        hipLaunchKernelGGL(prefill_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, n_blocks, n_experts, e_pad, sc.block_cnt,
-                           sc.plan, sc.tiles, sc.max_tiles, tile_shift);
+        const uint32_t run = (n_blocks + kScanThreads / e_pad - 1) / (kScanThreads / e_pad);     // sort blocks per thread
+        hipLaunchKernelGGL((run <= 16 ? prefill_scan_kernel<16> : prefill_scan_kernel<32>), dim3(1), dim3(kScanThreads), 0, s, n_blocks,
+                           n_experts, e_pad, sc.block_cnt, sc.plan, sc.tiles, sc.max_tiles, tile_shift);
         hipLaunchKernelGGL(prefill_scatter_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt, sc.sorted_token,
                            sc.sorted_out_row);
     }
