@@ -124,6 +124,24 @@ __device__ __forceinline__ uint4 unpack8_offset(uint32_t w) {
     return r;
 }
 
+// The same with less to cancel, where the sums are wanted to fp32's own accuracy. bf16: 16 + q (ulp 1/8 at 16: the nibble at
+// mantissa bits 3..6), an eighth of the offset for one more shift. FP16: the nibble's bits as they lie, i.e. the subnormal
+// q * 2^-24 (exact, and the matrix unit takes FP16 subnormals): no offset at all, the scale carries 2^24.
+template <bool F16> struct FineNibble {
+    static constexpr float kOffset = F16 ? 0.0f : 16.0f, kUnit = F16 ? 16777216.0f : 1.0f;
+};
+template <bool F16>
+__device__ __forceinline__ uint4 unpack8_fine(uint32_t w) {
+    if constexpr (F16) {
+        const uint32_t mask = 0x000F000Fu;
+        return make_uint4(w & mask, (w >> 4) & mask, (w >> 8) & mask, (w >> 12) & mask);
+    }
+    uint32_t mask = 0x00780078u, c = 0x41804180u;
+    asm("" : "+s"(mask));
+    asm("" : "+v"(c));
+    return make_uint4(((w << 3) & mask) | c, ((w >> 1) & mask) | c, ((w >> 5) & mask) | c, ((w >> 9) & mask) | c);
+}
+
 // Workgroup barrier that waits for this wave's LDS traffic only. __syncthreads() also drains every
 // outstanding global load, which would serialise a register prefetch that is meant to stay in flight
 // across the barrier; here the compiler's own counters still guard each prefetched register at its use.

@@ -709,16 +709,13 @@ constexpr int kStreamDepth = 4;                                             // w
 constexpr int kStreamChunk = 2;                                             // groups whose rows are in LDS at a time, twice
 constexpr uint32_t kStreamStageRow = 2 * kTilesPerBlock * kTileRows * 2 + 16;   // bytes: 128 output columns + padding
 
-// The eight nibbles of a dword as matrix operands. bf16: 128 + q, as in the decode kernels. FP16: the nibble's bits as they
-// lie, i.e. the subnormal q * 2^-24 (exact, and the matrix unit takes FP16 subnormals): no offset to cancel. With 1024 + q
-// the fp32 sums of a group carry 1024 * sum x through their roundings, which made a 2,816-wide row's error against 64 bits
-// 3.60e-4 where the rounded weights of the GEMM have 3.58e-4.
-constexpr float kNibbleUnit = 16777216.0f;      // 2^24
+// The eight nibbles of a dword as matrix operands. bf16: 128 + q, as in the decode kernels. FP16: the subnormal q * 2^-24. With
+// 1024 + q the fp32 sums of a group carry 1024 * sum x through their roundings, which made a 2,816-wide row's error against 64
+// bits 3.60e-4 where the rounded weights of the GEMM have 3.58e-4.
 template <bool F16>
 __device__ __forceinline__ uint4 unpack8_stream(uint32_t w) {
-    if constexpr (!F16) return unpack8_offset<false>(w);
-    const uint32_t mask = 0x000F000Fu;
-    return make_uint4(w & mask, (w >> 4) & mask, (w >> 8) & mask, (w >> 12) & mask);
+    if constexpr (F16) return unpack8_fine<true>(w);
+    else return unpack8_offset<false>(w);
 }
 
 template <bool GATE_UP, int NM, bool F16>
@@ -816,8 +813,8 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         const uint4 wb0 = unpack8_stream<F16>(tile.z), wb1 = unpack8_stream<F16>(tile.w);
         float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y), ta = bf16hi_to_f32(sc.x), tb = bf16hi_to_f32(sc.y);
         if constexpr (F16) {
-            sa *= kNibbleUnit;
-            sb *= kNibbleUnit;
+            sa *= FineNibble<true>::kUnit;
+            sb *= FineNibble<true>::kUnit;
         } else {
             ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ta);
             tb = __builtin_fmaf(-Act<F16>::kOffset, sb, tb);
