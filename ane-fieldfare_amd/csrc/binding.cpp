@@ -77,6 +77,17 @@ uint32_t u32(PyObject *o) {
     if (v == (unsigned long)-1 && PyErr_Occurred()) throw PythonError{};
     return (uint32_t)v;
 }
+// the address `offset` bytes from a tensor's first; the offset has the pointer's width (a buffer that holds a model's weights is
+// larger than 4 GiB) and, as in Python's own address arithmetic, is an int that may be negative
+const uint8_t *address(PyObject *o, PyObject *offset) {
+    if (!PyLong_Check(offset)) {
+        PyErr_Format(PyExc_TypeError, "a byte offset is an int, got %.100s", Py_TYPE(offset)->tp_name);
+        throw PythonError{};
+    }
+    const long long bytes = PyLong_AsLongLong(offset);
+    if (bytes == -1 && PyErr_Occurred()) throw PythonError{};
+    return reinterpret_cast<const uint8_t *>(reinterpret_cast<uintptr_t>(pointer<uint8_t>(o)) + (uintptr_t)bytes);
+}
 float f32(PyObject *o) {
     const double v = PyFloat_AsDouble(o);
     if (v == -1.0 && PyErr_Occurred()) throw PythonError{};
@@ -401,9 +412,10 @@ PyObject *gemv_int4(Args a) {        // handle, W, S, B, x, f32_out, w_byte_offs
     const at::Tensor &s = tensor(a[2]), &x = tensor(a[4]);
     const uint32_t m = dim_of(s, 0), n = dim_of(s, 1) * FFMOE_GROUP;
     const bool wide = truth(a[5]);
+    const uint8_t *w = address(a[1], a[6]);
     at::Tensor y = fresh(x, wide ? at::kFloat : dtype(a[7]), x.size(0), m);
     char *err = nullptr;
-    check(g_calls.ffmoe_gemv_int4(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint8_t>(a[1]) + u32(a[6]), pointer<uint16_t>(s),
+    check(g_calls.ffmoe_gemv_int4(handle<ffmoe_ctx>(a[0]), stream(), w, pointer<uint16_t>(s),
                                   pointer<uint16_t>(a[3]), pointer<uint16_t>(x), y.data_ptr(), m, n, dim_of(x, 0), row_stride(x), m, wide, &err), err);
     return wrap(y);
 }

@@ -84,3 +84,20 @@ def test_reference_layout_gemv_at_the_edges(ctx, oracle, torch, m, n, rows, off)
         if off == 0:
             listed = ctx.gemv_int4_listed(raw, Sd, Bd, torch.from_numpy(ids).cuda(), x).cpu().numpy()
             assert np.array_equal(listed.view(np.uint32), y[:, ids].view(np.uint32))
+
+
+@pytest.mark.parametrize("view", ["host address", "end of the buffer"])
+def test_weight_offsets_have_the_width_of_a_pointer(ctx, oracle, torch, view):
+    # gemv_int4's w_byte_offset counts from W's first byte: as far as from an address on the host to the weights on the GPU (some
+    # 2^46 either way), and backwards from a view that starts behind the weights
+    m, n = 33, 128
+    g = oracle.seed_tree_key(0x0FF, "gemv-offset")
+    W, S, B = oracle.quantize_int4(g.uniform(-0.5, 0.5, m * n).reshape(m, n))
+    x = bf16_tensor(torch, oracle.bf16_bits(g.uniform(-1.0, 1.0, n)).reshape(1, n))
+    raw = torch.from_numpy(np.concatenate([W.ravel(), np.zeros(64, np.uint8)])).cuda()
+    Sd, Bd = (torch.from_numpy(a.view(np.int16)).cuda() for a in (S, B))
+    base = torch.zeros(16, dtype=torch.uint8) if view == "host address" else raw[W.size:]
+    off = raw.data_ptr() - base.data_ptr()
+    assert abs(off) > (1 << 32) or view != "host address"
+    y = ctx.gemv_int4(base, Sd, Bd, x, f32_out=True, w_byte_offset=off)
+    assert torch.equal(y, ctx.gemv_int4(raw, Sd, Bd, x, f32_out=True))
