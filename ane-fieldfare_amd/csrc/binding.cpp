@@ -11,6 +11,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <dlfcn.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -426,14 +427,14 @@ PyObject *method(PyObject *, PyObject *const *args, Py_ssize_t n) {
         PyErr_Format(PyExc_TypeError, "%d arguments are wanted, got %zd", N, n);
         return nullptr;
     }
+    // what torch throws arrives as from torch's own calls (torch.OutOfMemoryError from an allocation, IndexError, ...)
+    HANDLE_TH_ERRORS
     try {
         return F(args);
     } catch (const PythonError &) {
         return nullptr;
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
     }
+    END_HANDLE_TH_ERRORS
 }
 
 // bind(path of the loaded library, exception class)

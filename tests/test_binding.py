@@ -19,3 +19,10 @@ def _gemv_int4(native, offset):
 def test_a_byte_offset_is_taken_whole_or_refused(native, offset, error):
     with pytest.raises(error):
         _gemv_int4(native, offset)
+
+
+def test_errors_keep_the_types_torch_gives_them(native):
+    import torch
+    flat = torch.zeros(64, dtype=torch.bfloat16)              # one dimension where rows are wanted
+    with pytest.raises(IndexError):
+        native.gemv_int4_listed(None, flat, flat, flat, flat, flat)
