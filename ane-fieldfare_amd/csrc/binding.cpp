@@ -39,6 +39,20 @@ struct Calls {
 } g_calls;
 #undef FFMOE_POINTER
 
+// While one lives the interpreter lock is given up: a launch that waits for room in its queue, a library's first use, an
+// allocation that waits for the device do not hold up the program's other threads. Python objects are read before, results
+// wrapped after.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+template <typename... P, typename... A>
+int call(int (*f)(P...), A... args) {
+    const Unlocked unlocked;
+    return f(args...);
+}
+
 void check(int code, char *&err) {      // by reference: the call that fills it is the first argument
     if (code == FFMOE_OK) return;
     PyObject *args = Py_BuildValue("(is)", code, err ? err : "(no message)");
@@ -111,10 +125,13 @@ uint32_t dim_of(const at::Tensor &t, int64_t dim) { return (uint32_t)t.size(dim)
 uint32_t row_stride(const at::Tensor &t) { return (uint32_t)(t.size(0) > 1 ? t.stride(0) : std::max(t.stride(0), t.size(1))); }
 void *stream() { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 
-at::Tensor fresh(const at::Tensor &like, at::ScalarType type, int64_t a) { return at::detail::empty_cuda({a}, type, like.device(), std::nullopt); }
-at::Tensor fresh(const at::Tensor &like, at::ScalarType type, int64_t a, int64_t b) {
-    return at::detail::empty_cuda({a, b}, type, like.device(), std::nullopt);
+at::Tensor allocate(const at::Tensor &like, at::ScalarType type, at::IntArrayRef sizes) {
+    const at::Device device = like.device();
+    const Unlocked unlocked;
+    return at::detail::empty_cuda(sizes, type, device, std::nullopt);
 }
+at::Tensor fresh(const at::Tensor &like, at::ScalarType type, int64_t a) { return allocate(like, type, at::IntArrayRef{a}); }
+at::Tensor fresh(const at::Tensor &like, at::ScalarType type, int64_t a, int64_t b) { return allocate(like, type, {a, b}); }
 PyObject *wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
 // the caller's output tensor, or a new one
 struct Out {
@@ -147,16 +164,16 @@ PyObject *matrix_gemv(Args a) {      // handle, x, m, act, f32_out, out
     const bool wide = truth(a[4]);
     Out y = output(a[5], x, wide ? at::kFloat : dtype(a[3]), x.size(0), (int64_t)u32(a[2]));
     char *err = nullptr;
-    check(g_calls.ffmoe_matrix_gemv(handle<ffmoe_matrix>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0), y.t.data_ptr(),
-                                    row_stride(y.t), wide, &err), err);
+    check(call(g_calls.ffmoe_matrix_gemv, handle<ffmoe_matrix>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0), y.t.data_ptr(),
+               row_stride(y.t), wide, &err), err);
     return y.result();
 }
 
 PyObject *matrix_rows(Args a) {      // handle, ids (a tensor), out_scale, out (a tensor)
     const at::Tensor &ids = tensor(a[1]), &y = tensor(a[3]);
     char *err = nullptr;
-    check(g_calls.ffmoe_matrix_rows(handle<ffmoe_matrix>(a[0]), stream(), pointer<uint32_t>(ids), dim_of(ids, 0), 0u, f32(a[2]),
-                                    pointer<uint16_t>(y), row_stride(y), &err), err);
+    check(call(g_calls.ffmoe_matrix_rows, handle<ffmoe_matrix>(a[0]), stream(), pointer<uint32_t>(ids), dim_of(ids, 0), 0u, f32(a[2]),
+               pointer<uint16_t>(y), row_stride(y), &err), err);
     Py_INCREF(a[3]);
     return a[3];
 }
@@ -165,8 +182,8 @@ PyObject *matrix_greedy(Args a) {    // handle, x
     const at::Tensor &x = tensor(a[1]);
     at::Tensor out = fresh(x, at::kInt, x.size(0));
     char *err = nullptr;
-    check(g_calls.ffmoe_matrix_greedy(handle<ffmoe_matrix>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
-                                      pointer<uint32_t>(out), &err), err);
+    check(call(g_calls.ffmoe_matrix_greedy, handle<ffmoe_matrix>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
+               pointer<uint32_t>(out), &err), err);
     return wrap(out);
 }
 
@@ -174,8 +191,8 @@ PyObject *matrix_greedy_conf(Args a) {      // handle, x, softcap
     const at::Tensor &x = tensor(a[1]);
     at::Tensor out = fresh(x, at::kInt, x.size(0)), conf = fresh(x, at::kFloat, x.size(0));
     char *err = nullptr;
-    check(g_calls.ffmoe_matrix_greedy_conf(handle<ffmoe_matrix>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0), f32(a[2]),
-                                           pointer<uint32_t>(out), pointer<float>(conf), &err), err);
+    check(call(g_calls.ffmoe_matrix_greedy_conf, handle<ffmoe_matrix>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0), f32(a[2]),
+               pointer<uint32_t>(out), pointer<float>(conf), &err), err);
     return tuple({wrap(out), wrap(conf)});
 }
 
@@ -191,8 +208,8 @@ PyObject *router(Args a) {           // handle, layer, router_x, act, top_k, n_e
     at::Tensor idx = fresh(x, at::kInt, t, k), w = fresh(x, act, t, k), logits;
     if (want) logits = fresh(x, at::kFloat, t, (int64_t)u32(a[5]));
     char *err = nullptr;
-    check(g_calls.ffmoe_router(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), (uint32_t)t,
-                               pointer<uint32_t>(idx), pointer<uint16_t>(w), want ? pointer<float>(logits) : nullptr, &err), err);
+    check(call(g_calls.ffmoe_router, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), (uint32_t)t,
+               pointer<uint32_t>(idx), pointer<uint16_t>(w), want ? pointer<float>(logits) : nullptr, &err), err);
     if (want) return tuple({wrap(idx), wrap(w), wrap(logits)});
     return tuple({wrap(idx), wrap(w)});
 }
@@ -201,8 +218,8 @@ PyObject *verify(Args a) {           // handle, layer, x, idx, w, residual, out,
     const at::Tensor &x = tensor(a[2]);
     Out y = output(a[6], x, dtype(a[7]), x.size(0), (int64_t)u32(a[8]));
     char *err = nullptr;
-    check(g_calls.ffmoe_verify(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
-                               pointer<uint32_t>(a[3]), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]), pointer<uint16_t>(y.t), &err), err);
+    check(call(g_calls.ffmoe_verify, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
+               pointer<uint32_t>(a[3]), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]), pointer<uint16_t>(y.t), &err), err);
     return y.result();
 }
 
@@ -215,9 +232,9 @@ PyObject *route_verify(Args a) {     // handle, layer, router_x, x, residual, ou
     if (combine) y = output(a[5], x, act, t, (int64_t)u32(a[9]));
     at::Tensor idx = fresh(x, at::kInt, t, k), w = fresh(x, act, t, k);
     char *err = nullptr;
-    check(g_calls.ffmoe_route_verify(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(rx), row_stride(rx), pointer<uint16_t>(x),
-                                     row_stride(x), (uint32_t)t, pointer<uint16_t>(a[4]), combine ? pointer<uint16_t>(y.t) : nullptr,
-                                     pointer<uint32_t>(idx), pointer<uint16_t>(w), &err), err);
+    check(call(g_calls.ffmoe_route_verify, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(rx), row_stride(rx), pointer<uint16_t>(x),
+               row_stride(x), (uint32_t)t, pointer<uint16_t>(a[4]), combine ? pointer<uint16_t>(y.t) : nullptr,
+               pointer<uint32_t>(idx), pointer<uint16_t>(w), &err), err);
     if (!combine) Py_INCREF(Py_None);
     return tuple({combine ? y.result() : Py_None, wrap(idx), wrap(w)});
 }
@@ -227,17 +244,17 @@ PyObject *route_verify_shared(Args a) {     // handle, shared handle, layer, sha
     const int64_t t = x.size(0), k = u32(a[8]);
     at::Tensor idx = fresh(x, at::kInt, t, k), w = fresh(x, dtype(a[7]), t, k);
     char *err = nullptr;
-    check(g_calls.ffmoe_route_verify_shared(handle<ffmoe_ctx>(a[0]), handle<ffmoe_ctx>(a[1]), stream(), u32(a[2]), u32(a[3]),
-                                            pointer<uint16_t>(rx), row_stride(rx), pointer<uint16_t>(x), row_stride(x), pointer<uint16_t>(sx),
-                                            row_stride(sx), (uint32_t)t, pointer<uint32_t>(idx), pointer<uint16_t>(w), &err), err);
+    check(call(g_calls.ffmoe_route_verify_shared, handle<ffmoe_ctx>(a[0]), handle<ffmoe_ctx>(a[1]), stream(), u32(a[2]), u32(a[3]),
+               pointer<uint16_t>(rx), row_stride(rx), pointer<uint16_t>(x), row_stride(x), pointer<uint16_t>(sx),
+               row_stride(sx), (uint32_t)t, pointer<uint32_t>(idx), pointer<uint16_t>(w), &err), err);
     return tuple({wrap(idx), wrap(w)});
 }
 
 PyObject *verify_partials(Args a) {  // handle, layer, x, idx, w, partials (a tensor)
     const at::Tensor &x = tensor(a[2]);
     char *err = nullptr;
-    check(g_calls.ffmoe_verify_partials(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
-                                        pointer<uint32_t>(a[3]), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]), &err), err);
+    check(call(g_calls.ffmoe_verify_partials, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
+               pointer<uint32_t>(a[3]), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]), &err), err);
     Py_INCREF(a[5]);
     return a[5];
 }
@@ -246,8 +263,8 @@ PyObject *reduce_token_major(Args a) {      // handle, partials, weights, act
     const at::Tensor &p = tensor(a[1]);
     at::Tensor h2 = fresh(p, dtype(a[3]), p.size(0), p.size(2));
     char *err = nullptr;
-    check(g_calls.ffmoe_reduce_token_major(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(p), pointer<uint16_t>(a[2]),
-                                           pointer<uint16_t>(h2), dim_of(p, 0), dim_of(p, 1), dim_of(p, 2), &err), err);
+    check(call(g_calls.ffmoe_reduce_token_major, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(p), pointer<uint16_t>(a[2]),
+               pointer<uint16_t>(h2), dim_of(p, 0), dim_of(p, 1), dim_of(p, 2), &err), err);
     return wrap(h2);
 }
 
@@ -255,8 +272,8 @@ PyObject *prefill(Args a) {          // handle, layer, x, idx, w, out, act, d
     const at::Tensor &x = tensor(a[2]);
     Out y = output(a[5], x, dtype(a[6]), x.size(0), (int64_t)u32(a[7]));
     char *err = nullptr;
-    check(g_calls.ffmoe_prefill(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
-                                pointer<uint32_t>(a[3]), pointer<uint16_t>(a[4]), pointer<uint16_t>(y.t), &err), err);
+    check(call(g_calls.ffmoe_prefill, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
+               pointer<uint32_t>(a[3]), pointer<uint16_t>(a[4]), pointer<uint16_t>(y.t), &err), err);
     return y.result();
 }
 
@@ -264,16 +281,16 @@ PyObject *dense_ffn(Args a) {        // handle, layer, x, out, act, d
     const at::Tensor &x = tensor(a[2]);
     Out y = output(a[3], x, dtype(a[4]), x.size(0), (int64_t)u32(a[5]));
     char *err = nullptr;
-    check(g_calls.ffmoe_dense_ffn(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
-                                  pointer<uint16_t>(y.t), &err), err);
+    check(call(g_calls.ffmoe_dense_ffn, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x), dim_of(x, 0),
+               pointer<uint16_t>(y.t), &err), err);
     return y.result();
 }
 
 PyObject *prefill_pairs(Args a) {    // handle, layer, x, sorted_pairs, t, partials (a tensor)
     const at::Tensor &x = tensor(a[2]), &pairs = tensor(a[3]);
     char *err = nullptr;
-    check(g_calls.ffmoe_prefill_pairs(handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x),
-                                      pointer<ffmoe_pair>(pairs), dim_of(pairs, 0), u32(a[4]), pointer<uint16_t>(a[5]), &err), err);
+    check(call(g_calls.ffmoe_prefill_pairs, handle<ffmoe_ctx>(a[0]), stream(), u32(a[1]), pointer<uint16_t>(x), row_stride(x),
+               pointer<ffmoe_pair>(pairs), dim_of(pairs, 0), u32(a[4]), pointer<uint16_t>(a[5]), &err), err);
     Py_INCREF(a[5]);
     return a[5];
 }
@@ -296,10 +313,10 @@ PyObject *post_attn_setup(Args a) {  // handle, hidden, attn, w_post_attn, w_pre
         }
     }
     char *err = nullptr;
-    check(g_calls.ffmoe_post_attn_setup(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(attn),
-                                        row_stride(attn), pointer<uint16_t>(outs[0]), row_stride(outs[0]), pointer<uint16_t>(outs[1]),
-                                        row_stride(outs[1]), pointer<uint16_t>(outs[2]), row_stride(outs[2]), pointer<uint16_t>(a[3]),
-                                        pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]), (uint32_t)t, (uint32_t)d, f32(a[6]), &err), err);
+    check(call(g_calls.ffmoe_post_attn_setup, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(attn),
+               row_stride(attn), pointer<uint16_t>(outs[0]), row_stride(outs[0]), pointer<uint16_t>(outs[1]),
+               row_stride(outs[1]), pointer<uint16_t>(outs[2]), row_stride(outs[2]), pointer<uint16_t>(a[3]),
+               pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]), (uint32_t)t, (uint32_t)d, f32(a[6]), &err), err);
     if (given) {
         Py_INCREF(given);
         return given;
@@ -310,9 +327,9 @@ PyObject *post_attn_setup(Args a) {  // handle, hidden, attn, w_post_attn, w_pre
 PyObject *layer_tail(Args a) {       // handle, h2, h1, hidden, w_postffn2, w_postffn, layer_scalar, eps, d
     const at::Tensor &h2 = tensor(a[1]), &h1 = tensor(a[2]), &hidden = tensor(a[3]);
     char *err = nullptr;
-    check(g_calls.ffmoe_layer_tail(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(h2), row_stride(h2), pointer<uint16_t>(h1), row_stride(h1),
-                                   pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]),
-                                   dim_of(hidden, 0), u32(a[8]), f32(a[7]), f32(a[6]), &err), err);
+    check(call(g_calls.ffmoe_layer_tail, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(h2), row_stride(h2), pointer<uint16_t>(h1), row_stride(h1),
+               pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]),
+               dim_of(hidden, 0), u32(a[8]), f32(a[7]), f32(a[6]), &err), err);
     Py_INCREF(a[3]);
     return a[3];
 }
@@ -320,9 +337,9 @@ PyObject *layer_tail(Args a) {       // handle, h2, h1, hidden, w_postffn2, w_po
 PyObject *layer_tail_routed(Args a) {       // handle, route_w, h1, hidden, w_postffn2, w_postffn, layer_scalar, eps
     const at::Tensor &h1 = tensor(a[2]), &hidden = tensor(a[3]);
     char *err = nullptr;
-    check(g_calls.ffmoe_layer_tail_routed(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(a[1]), pointer<uint16_t>(h1), row_stride(h1),
-                                          pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]),
-                                          dim_of(hidden, 0), f32(a[7]), f32(a[6]), &err), err);
+    check(call(g_calls.ffmoe_layer_tail_routed, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(a[1]), pointer<uint16_t>(h1), row_stride(h1),
+               pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]), pointer<uint16_t>(a[5]),
+               dim_of(hidden, 0), f32(a[7]), f32(a[6]), &err), err);
     Py_INCREF(a[3]);
     return a[3];
 }
@@ -330,9 +347,9 @@ PyObject *layer_tail_routed(Args a) {       // handle, route_w, h1, hidden, w_po
 PyObject *layer_tail_routed_shared(Args a) {       // handle, shared handle, route_w, hidden, w_postffn2, w_postffn, layer_scalar, eps
     const at::Tensor &hidden = tensor(a[3]);
     char *err = nullptr;
-    check(g_calls.ffmoe_layer_tail_routed_shared(handle<ffmoe_ctx>(a[0]), handle<ffmoe_ctx>(a[1]), stream(), pointer<uint16_t>(a[2]),
-                                                 pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]),
-                                                 pointer<uint16_t>(a[5]), dim_of(hidden, 0), f32(a[7]), f32(a[6]), &err), err);
+    check(call(g_calls.ffmoe_layer_tail_routed_shared, handle<ffmoe_ctx>(a[0]), handle<ffmoe_ctx>(a[1]), stream(), pointer<uint16_t>(a[2]),
+               pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]),
+               pointer<uint16_t>(a[5]), dim_of(hidden, 0), f32(a[7]), f32(a[6]), &err), err);
     Py_INCREF(a[3]);
     return a[3];
 }
@@ -343,11 +360,11 @@ PyObject *layer_tail_norms(Args a) { // handle, h2, h1, hidden, w_postffn1, w_po
     at::Tensor normed;
     if (a[8] != Py_None) normed = fresh(hidden, dtype(a[11]), hidden.size(0), d);
     char *err = nullptr;
-    check(g_calls.ffmoe_layer_tail_norms(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(h2), row_stride(h2), pointer<uint16_t>(h1),
-                                         row_stride(h1), pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]),
-                                         pointer<uint16_t>(a[5]), pointer<uint16_t>(a[6]), pointer<uint16_t>(a[8]),
-                                         normed.defined() ? pointer<uint16_t>(normed) : nullptr, d, dim_of(hidden, 0), d, f32(a[9]), f32(a[7]),
-                                         &err), err);
+    check(call(g_calls.ffmoe_layer_tail_norms, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(h2), row_stride(h2), pointer<uint16_t>(h1),
+               row_stride(h1), pointer<uint16_t>(hidden), row_stride(hidden), pointer<uint16_t>(a[4]),
+               pointer<uint16_t>(a[5]), pointer<uint16_t>(a[6]), pointer<uint16_t>(a[8]),
+               normed.defined() ? pointer<uint16_t>(normed) : nullptr, d, dim_of(hidden, 0), d, f32(a[9]), f32(a[7]),
+               &err), err);
     if (normed.defined()) return wrap(normed);
     Py_RETURN_NONE;
 }
@@ -357,8 +374,8 @@ PyObject *rmsnorm(Args a) {          // handle, x, w, eps, d, out, act
     const uint32_t d = u32(a[4]);
     Out y = output(a[5], x, dtype(a[6]), x.size(0), d);
     char *err = nullptr;
-    check(g_calls.ffmoe_rmsnorm(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), pointer<uint16_t>(a[2]),
-                                pointer<uint16_t>(y.t), row_stride(y.t), dim_of(x, 0), d, f32(a[3]), &err), err);
+    check(call(g_calls.ffmoe_rmsnorm, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(x), row_stride(x), pointer<uint16_t>(a[2]),
+               pointer<uint16_t>(y.t), row_stride(y.t), dim_of(x, 0), d, f32(a[3]), &err), err);
     return y.result();
 }
 
@@ -366,8 +383,8 @@ PyObject *gelu_mul(Args a) {         // handle, gate, up, out
     const at::Tensor &gate = tensor(a[1]), &up = tensor(a[2]);
     Out y = output(a[3], gate, gate.scalar_type(), gate.size(0), gate.size(1));
     char *err = nullptr;
-    check(g_calls.ffmoe_gelu_mul(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(gate), row_stride(gate), pointer<uint16_t>(up),
-                                 row_stride(up), pointer<uint16_t>(y.t), row_stride(y.t), dim_of(gate, 0), dim_of(gate, 1), &err), err);
+    check(call(g_calls.ffmoe_gelu_mul, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(gate), row_stride(gate), pointer<uint16_t>(up),
+               row_stride(up), pointer<uint16_t>(y.t), row_stride(y.t), dim_of(gate, 0), dim_of(gate, 1), &err), err);
     return y.result();
 }
 
@@ -378,8 +395,8 @@ PyObject *argmax_rows(Args a) {      // handle, logits, count (0: the whole row)
     at::Tensor out = fresh(l, at::kInt, l.size(0)), conf;
     if (want) conf = fresh(l, at::kFloat, l.size(0));
     char *err = nullptr;
-    check(g_calls.ffmoe_argmax_rows(handle<ffmoe_ctx>(a[0]), stream(), pointer<float>(l), row_stride(l), dim_of(l, 0), count ? count : dim_of(l, 1),
-                                    f32(a[3]), pointer<uint32_t>(out), want ? pointer<float>(conf) : nullptr, &err), err);
+    check(call(g_calls.ffmoe_argmax_rows, handle<ffmoe_ctx>(a[0]), stream(), pointer<float>(l), row_stride(l), dim_of(l, 0), count ? count : dim_of(l, 1),
+               f32(a[3]), pointer<uint32_t>(out), want ? pointer<float>(conf) : nullptr, &err), err);
     if (want) return tuple({wrap(out), wrap(conf)});
     return wrap(out);
 }
@@ -392,9 +409,9 @@ PyObject *sample_rows(Args a) {      // handle, logits, temperature, softcap, se
     const ffmoe_sampling rule{f32(a[2]), f32(a[7]), u32(a[6]), u32(a[5]), f32(a[3]), (uint64_t)seed};
     at::Tensor out = fresh(l, at::kInt, l.size(0)), prob = fresh(l, at::kFloat, l.size(0));
     char *err = nullptr;
-    check(g_calls.ffmoe_sample_rows(handle<ffmoe_ctx>(a[0]), stream(), pointer<float>(l), row_stride(l), dim_of(l, 0), count ? count : dim_of(l, 1),
-                                    pointer<uint32_t>(a[8]), &rule, pointer<uint32_t>(a[9]), pointer<uint32_t>(out), pointer<float>(prob),
-                                    &err), err);
+    check(call(g_calls.ffmoe_sample_rows, handle<ffmoe_ctx>(a[0]), stream(), pointer<float>(l), row_stride(l), dim_of(l, 0), count ? count : dim_of(l, 1),
+               pointer<uint32_t>(a[8]), &rule, pointer<uint32_t>(a[9]), pointer<uint32_t>(out), pointer<float>(prob),
+               &err), err);
     return tuple({wrap(out), wrap(prob)});
 }
 
@@ -403,9 +420,9 @@ PyObject *gemv_int4_listed(Args a) { // handle, W, S, B, ids, x
     const uint32_t m = dim_of(ids, 0), n = dim_of(s, 1) * FFMOE_GROUP;
     at::Tensor y = fresh(x, at::kFloat, x.size(0), m);
     char *err = nullptr;
-    check(g_calls.ffmoe_gemv_int4_listed(handle<ffmoe_ctx>(a[0]), stream(), pointer<uint8_t>(a[1]), pointer<uint16_t>(s), pointer<uint16_t>(a[3]),
-                                         pointer<uint32_t>(ids), pointer<uint16_t>(x), pointer<float>(y), m, n, dim_of(x, 0), row_stride(x), m,
-                                         &err), err);
+    check(call(g_calls.ffmoe_gemv_int4_listed, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint8_t>(a[1]), pointer<uint16_t>(s), pointer<uint16_t>(a[3]),
+               pointer<uint32_t>(ids), pointer<uint16_t>(x), pointer<float>(y), m, n, dim_of(x, 0), row_stride(x), m,
+               &err), err);
     return wrap(y);
 }
 
@@ -416,8 +433,8 @@ PyObject *gemv_int4(Args a) {        // handle, W, S, B, x, f32_out, w_byte_offs
     const uint8_t *w = address(a[1], a[6]);
     at::Tensor y = fresh(x, wide ? at::kFloat : dtype(a[7]), x.size(0), m);
     char *err = nullptr;
-    check(g_calls.ffmoe_gemv_int4(handle<ffmoe_ctx>(a[0]), stream(), w, pointer<uint16_t>(s),
-                                  pointer<uint16_t>(a[3]), pointer<uint16_t>(x), y.data_ptr(), m, n, dim_of(x, 0), row_stride(x), m, wide, &err), err);
+    check(call(g_calls.ffmoe_gemv_int4, handle<ffmoe_ctx>(a[0]), stream(), w, pointer<uint16_t>(s),
+               pointer<uint16_t>(a[3]), pointer<uint16_t>(x), y.data_ptr(), m, n, dim_of(x, 0), row_stride(x), m, wide, &err), err);
     return wrap(y);
 }
 

@@ -24,3 +24,41 @@ def test_a_failed_allocation_is_torch_s_own_error(ctx):
             ctx.gemv_int4(w, s, s, x, f32_out=True)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def test_a_call_that_waits_lets_other_threads_run(ctx):
+    # with profiling on a call waits for its kernel, here behind some 100 ms of products: the other thread's clock goes on
+    import threading
+    import time
+    import numpy as np
+    import torch
+    rng = np.random.default_rng(0)
+    mx = ctx.matrix(rng.integers(0, 256, (64, 64), dtype=np.uint8), *(np.full((64, 2), 0x3C00, np.uint16) for _ in range(2)))
+    x = torch.zeros((1, 128), dtype=torch.bfloat16, device="cuda")
+    big = torch.zeros((8192, 8192), dtype=torch.bfloat16, device="cuda")
+    out = torch.empty_like(big)
+    ctx.set_profiling(True)
+    mx.gemv(x)
+    torch.mm(big, big, out=out)
+    torch.cuda.synchronize()
+    stamps, stop = [], threading.Event()
+
+    def clock():
+        while not stop.is_set():
+            stamps.append(time.perf_counter())
+            time.sleep(0.001)
+
+    for _ in range(150):
+        torch.mm(big, big, out=out)
+    th = threading.Thread(target=clock)
+    th.start()
+    time.sleep(0.005)
+    begin = time.perf_counter()
+    mx.gemv(x)
+    end = time.perf_counter()
+    stop.set()
+    th.join()
+    inside = [begin] + [s for s in stamps if begin < s < end] + [end]
+    assert end - begin > 0.02, "the call did not wait"
+    assert max(b - a for a, b in zip(inside, inside[1:])) < 0.5 * (end - begin)
+    mx.close()
