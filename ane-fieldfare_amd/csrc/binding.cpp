@@ -120,6 +120,11 @@ at::ScalarType dtype(PyObject *o) {
     }
     return reinterpret_cast<THPDtype *>(o)->scalar_type;
 }
+void rank(const at::Tensor &t, int64_t dims) {      // where the shape is taken apart whole
+    if (t.dim() == dims) return;
+    PyErr_Format(PyExc_ValueError, "a tensor of %lld dimensions is wanted, got %lld", (long long)dims, (long long)t.dim());
+    throw PythonError{};
+}
 uint32_t dim_of(const at::Tensor &t, int64_t dim) { return (uint32_t)t.size(dim); }
 // row stride in elements; a single-row tensor may report any stride for its size-1 dimension
 uint32_t row_stride(const at::Tensor &t) { return (uint32_t)(t.size(0) > 1 ? t.stride(0) : std::max(t.stride(0), t.size(1))); }
@@ -261,6 +266,7 @@ PyObject *verify_partials(Args a) {  // handle, layer, x, idx, w, partials (a te
 
 PyObject *reduce_token_major(Args a) {      // handle, partials, weights, act
     const at::Tensor &p = tensor(a[1]);
+    rank(p, 3);
     at::Tensor h2 = fresh(p, dtype(a[3]), p.size(0), p.size(2));
     char *err = nullptr;
     check(call(g_calls.ffmoe_reduce_token_major, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(p), pointer<uint16_t>(a[2]),
@@ -302,7 +308,9 @@ PyObject *post_attn_setup(Args a) {  // handle, hidden, attn, w_post_attn, w_pre
     PyObject *given = a[8] == Py_None ? nullptr : a[8];
     for (int i = 0; i < 3; ++i) {
         if (given) {
-            PyObject *item = PySequence_GetItem(given, i);
+            // given[i]: three tensors in a sequence, or one of [3, t, >= d]
+            PyObject *index = PyLong_FromLong(i), *item = index ? PyObject_GetItem(given, index) : nullptr;
+            Py_XDECREF(index);
             if (!item) throw PythonError{};
             outs[i] = THPVariable_Check(item) ? THPVariable_Unpack(item) : at::Tensor();
             if (!THPVariable_Check(item)) PyErr_SetString(PyExc_TypeError, "out holds three tensors");
@@ -381,6 +389,7 @@ PyObject *rmsnorm(Args a) {          // handle, x, w, eps, d, out, act
 
 PyObject *gelu_mul(Args a) {         // handle, gate, up, out
     const at::Tensor &gate = tensor(a[1]), &up = tensor(a[2]);
+    rank(gate, 2);
     Out y = output(a[3], gate, gate.scalar_type(), gate.size(0), gate.size(1));
     char *err = nullptr;
     check(call(g_calls.ffmoe_gelu_mul, handle<ffmoe_ctx>(a[0]), stream(), pointer<uint16_t>(gate), row_stride(gate), pointer<uint16_t>(up),

@@ -26,3 +26,28 @@ def test_errors_keep_the_types_torch_gives_them(native):
     flat = torch.zeros(64, dtype=torch.bfloat16)              # one dimension where rows are wanted
     with pytest.raises(IndexError):
         native.gemv_int4_listed(None, flat, flat, flat, flat, flat)
+
+
+def test_ranks_are_the_methods_own(native):
+    import torch
+    rows = torch.zeros((2, 64), dtype=torch.bfloat16)
+    for gate in (rows[0], rows[None]):
+        with pytest.raises(ValueError):
+            native.gelu_mul(None, gate, gate, gate)
+    for partials in (rows, rows[None, None]):
+        with pytest.raises(ValueError):
+            native.reduce_token_major(None, partials, rows, torch.bfloat16)
+
+
+@pytest.mark.skipif("__import__('torch').cuda.is_available()", reason="on the CPU the call ends at the device, past its arguments")
+def test_setup_outputs_may_come_in_any_container(native):
+    # three tensors in a sequence or one tensor of three: both get as far as the device; two do not
+    import torch
+    h = torch.zeros((2, 64), dtype=torch.bfloat16)
+    setup = lambda out: native.post_attn_setup(None, h, h, h[0], h[0], h[0], 1e-6, 64, out, torch.bfloat16)
+    for out in ((h, h, h), [h, h, h], torch.zeros((3, 2, 64), dtype=torch.bfloat16), {0: h, 1: h, 2: h}):
+        with pytest.raises(RuntimeError, match="(?i)no .*(device|gpu)"):
+            setup(out)
+    for out, error in (((h, h), IndexError), ((h, h, 3), TypeError)):
+        with pytest.raises(error):
+            setup(out)

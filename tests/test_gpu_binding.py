@@ -62,3 +62,15 @@ def test_a_call_that_waits_lets_other_threads_run(ctx):
     assert end - begin > 0.02, "the call did not wait"
     assert max(b - a for a, b in zip(inside, inside[1:])) < 0.5 * (end - begin)
     mx.close()
+
+
+def test_setup_outputs_in_one_tensor(ctx):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    hidden, attn = (torch.randn((5, 128), device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    w = [torch.rand(128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(3)]
+    out = torch.zeros((3, 5, 128), dtype=torch.bfloat16, device="cuda")
+    want = ctx.post_attn_setup(hidden.clone(), attn, *w)
+    assert ctx.post_attn_setup(hidden.clone(), attn, *w, out=out) is out
+    assert all(torch.equal(a, b) for a, b in zip(out, want))
