@@ -146,39 +146,60 @@ class Matrix:
 
 BINDING_PATH = _PKG / "ffmoe_binding.so"
 HASH_PATH = LIB_PATH.with_suffix(".so.srchash")
+BINDING_HASH_PATH = BINDING_PATH.with_suffix(".so.srchash")
+
+
+def _digest(files, *more: str) -> str:
+    import hashlib
+    h = hashlib.sha256()
+    for p in files:
+        h.update(p.name.encode())
+        h.update(p.read_bytes())
+    for text in more:
+        h.update(text.encode())
+    return h.hexdigest()
 
 
 def source_hash() -> str:
     """Digest of everything the library is compiled from (kernels, headers, Makefile, the C header)."""
-    import hashlib
-    h = hashlib.sha256()
-    files = sorted(p for p in CSRC.iterdir() if p.suffix in (".hip", ".hpp", ".cpp") or p.name == "Makefile")
-    for p in files + [_PKG.parent / "include" / "fieldfare_moe.h"]:
-        h.update(p.name.encode())
-        h.update(p.read_bytes())
-    return h.hexdigest()
+    files = sorted(p for p in CSRC.iterdir() if p.suffix in (".hip", ".hpp") or p.name == "Makefile")
+    return _digest(files + [_PKG.parent / "include" / "fieldfare_moe.h"])
+
+
+def binding_hash() -> str:
+    """The same of the native module, with the torch and the Python it is compiled against: a module that was built for
+    other ones is not loaded."""
+    import sysconfig
+    import torch
+    return _digest([CSRC / "Makefile", CSRC / "binding.cpp", _PKG.parent / "include" / "fieldfare_moe.h"], torch.__version__,
+                   str(sysconfig.get_config_var("SOABI")))
+
+
+def _matches(built: Path, digest: Path, want) -> bool:
+    return built.exists() and digest.exists() and digest.read_text().strip() == want()
 
 
 def is_stale() -> bool:
-    """True when no library is built or the sources changed since it was (file times do not survive a copy of the tree,
-    so the build leaves a digest of its sources beside the library)."""
-    return not (LIB_PATH.exists() and BINDING_PATH.exists() and HASH_PATH.exists() and HASH_PATH.read_text().strip() == source_hash())
+    """True when the library or the native module is not built, or was built from other sources (file times do not survive
+    a copy of the tree, so the build leaves a digest beside each)."""
+    return not (_matches(LIB_PATH, HASH_PATH, source_hash) and _matches(BINDING_PATH, BINDING_HASH_PATH, binding_hash))
 
 
 def build(force: bool = True) -> Path:
-    """Compile the library for gfx950 with the Makefile in csrc/ (hipcc cross-compiles without a GPU). `force` recompiles
-    every source; otherwise make rebuilds what its dependencies say changed. A failed build raises with the compiler's
-    messages."""
-    cmd = ["make", "-C", str(CSRC), "-j8"] + (["-B"] if force else [])
+    """Compile the library for gfx950 and the native module with the Makefile in csrc/ (hipcc cross-compiles without a GPU).
+    `force` recompiles every source; otherwise make rebuilds what its dependencies say changed, and everything where that
+    leaves a digest that does not match. A failed build raises with the compiler's messages."""
+    cmd = ["make", "-C", str(CSRC), "-j8", "all"] + (["-B"] if force else [])
     run = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if run.returncode != 0:
         raise RuntimeError(f"building {LIB_PATH.name} failed ({' '.join(cmd)}):\n{run.stdout[-6000:]}")
-    HASH_PATH.write_text(source_hash() + "\n")
+    if not force and is_stale():
+        return build()
     return LIB_PATH
 
 
 def ensure_built() -> Path:
-    """Load what is built in-tree; compile only when nothing is, or when the sources are newer than the library."""
+    """Load what is built in-tree; compile only when nothing is, or when it was built from something else."""
     if is_stale():
         build(force=not (LIB_PATH.exists() and BINDING_PATH.exists()))
     return LIB_PATH
@@ -195,8 +216,8 @@ def lib() -> C.CDLL:
     if not (LIB_PATH.exists() and BINDING_PATH.exists()):
         raise FileNotFoundError(f"{LIB_PATH} or {BINDING_PATH.name} is not built; run __graft_entry__.build() (there is no fallback path)")
     if is_stale():
-        raise RuntimeError(f"{LIB_PATH} was built from other sources than the ones in {CSRC}; run __graft_entry__.build() "
-                           "or fieldfare_moe.ensure_built()")
+        raise RuntimeError(f"{LIB_PATH} or {BINDING_PATH.name} was built from other sources than the ones in {CSRC}, or for another "
+                           "torch or Python; run __graft_entry__.build() or fieldfare_moe.ensure_built()")
     # torch ships its own HIP runtime: it has to be in the process before this library resolves
     # libamdhip64, or two runtimes end up loaded and the second one finds no device
     import torch  # noqa: F401
