@@ -201,6 +201,21 @@ void claim_scratch(ffmoe_ctx *ctx, void *stream) {
     }
 }
 
+// The scratch of a choice over rows of logits, claimed for the call, or none: a call that needs none orders no streams, and
+// one under capture gets none - its replays claim nothing, and beside another call of the context they would share the scratch.
+// The choice then takes one block per row and writes to the caller's buffers alone (one row of 262,144 logits, top_k = 64:
+// 375 us instead of 17).
+SampleScratch choice_scratch(ffmoe_ctx *ctx, void *stream, bool wanted) {
+    if (!wanted) return SampleScratch{};
+    hipStreamCaptureStatus now = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &now) != hipSuccess || now != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return SampleScratch{};
+    }
+    claim_scratch(ctx, stream);
+    return ctx->sample;
+}
+
 int check_layer(ffmoe_ctx *ctx, uint32_t layer, bool need_experts, bool need_router, char **err) {
     if (layer >= ctx->shape.n_layers)
         return fail(err, FFMOE_ERR_INVALID, "layer %u out of range (n_layers = %u)", layer, ctx->shape.n_layers);
@@ -453,9 +468,9 @@ int ffmoe_sample_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_
         return fail(err, FFMOE_ERR_INVALID, "the sampled choice caps its logits: softcap must be positive and finite");
     if (rule->top_k > 256) return fail(err, FFMOE_ERR_INVALID, "top_k = %u outside 0...256", rule->top_k);
     if (rule->top_k && !(rule->top_p > 0.0f && rule->top_p <= 1.0f)) return fail(err, FFMOE_ERR_INVALID, "top_p outside (0, 1]");
-    claim_scratch(ctx, stream);
+    const SampleScratch sc = choice_scratch(ctx, stream, sample_takes_scratch(count, rule->top_k));
     FF_HIP(launch_sample_rows(static_cast<hipStream_t>(stream), logits, stride, rows, count, ids, rule->temperature, rule->top_p,
-                              rule->top_k, rule->key_base, rule->softcap, rule->seed, key_offset, out_tokens, out_prob, ctx->sample));
+                              rule->top_k, rule->key_base, rule->softcap, rule->seed, key_offset, out_tokens, out_prob, sc));
     return FFMOE_OK;
 }
 
@@ -1408,9 +1423,9 @@ int ffmoe_argmax_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_
     if (stride < count) return fail(err, FFMOE_ERR_INVALID, "stride smaller than the row");
     if (!(softcap >= 0.0f) || std::isinf(softcap)) return fail(err, FFMOE_ERR_INVALID, "softcap must be finite and >= 0 (0 disables it)");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    claim_scratch(ctx, stream);
+    const SampleScratch sc = choice_scratch(ctx, stream, argmax_takes_scratch(rows, count));
     ctx->timer.begin(s);
-    FF_HIP(launch_argmax_rows(s, logits, stride, rows, count, softcap, out_index, out_conf, ctx->sample));
+    FF_HIP(launch_argmax_rows(s, logits, stride, rows, count, softcap, out_index, out_conf, sc));
     ctx->timer.mark(s, FFMOE_K_ARGMAX);
     ctx->timer.finish();
     return FFMOE_OK;

@@ -225,7 +225,9 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
                                 const uint16_t *x, uint32_t x_stride, uint32_t rows, unsigned long long *partials,
                                 uint32_t *out, uint32_t n_cus, bool f16, KernelTimer *timer, float softcap = 0.0f,
                                 float *out_conf = nullptr);
-// greedy choice (and the winner's softmax probability under the softcap) over rows of fp32 logits in memory
+// greedy choice (and the winner's softmax probability under the softcap) over rows of fp32 logits in memory; without a scratch
+// one block per row, whatever its length
+bool argmax_takes_scratch(uint32_t rows, uint32_t count);
 hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count, float softcap,
                               uint32_t *out, float *out_conf, SampleScratch sc);
 
@@ -286,7 +288,9 @@ hipError_t launch_gemv_int4(hipStream_t s, const uint8_t *w, const uint16_t *sca
                             const uint16_t *x, void *y, uint32_t m, uint32_t n, uint32_t rows,
                             uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids, bool f16, uint32_t n_cus);
 
-// sample.hip: the sampled choice over rows of fp32 logits (Gumbel-max draw, exact top-k, top-p prefix)
+// sample.hip: the sampled choice over rows of fp32 logits (Gumbel-max draw, exact top-k, top-p prefix); without a scratch one
+// block per row, whatever its length
+bool sample_takes_scratch(uint32_t count, uint32_t top_k);
 hipError_t launch_sample_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                               const uint32_t *ids, float temperature, float top_p, uint32_t top_k, uint32_t key_base,
                               float softcap, unsigned long long seed, const uint32_t *key_offset, uint32_t *out_tokens,

@@ -672,9 +672,13 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
     return hipGetLastError();
 }
 
+bool argmax_takes_scratch(uint32_t rows, uint32_t count) {
+    return count > kArgmaxOneBlock && rows <= FFMOE_MAX_VERIFY_ROWS && count <= kSampleMaxSegments * kSampleSegment;
+}
+
 hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count, float softcap,
                               uint32_t *out, float *out_conf, SampleScratch sc) {
-    if (count > kArgmaxOneBlock && rows <= FFMOE_MAX_VERIFY_ROWS && count <= kSampleMaxSegments * kSampleSegment && sc.segments) {
+    if (sc.segments && argmax_takes_scratch(rows, count)) {
         const uint32_t n_seg = (count + kSampleSegment - 1) / kSampleSegment;
         hipLaunchKernelGGL(argmax_rows_kernel<256>, dim3(rows, n_seg), dim3(256), 0, s, logits, stride, count, kSampleSegment, softcap, out,
                            out_conf, sc.segments);

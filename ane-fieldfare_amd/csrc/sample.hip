@@ -683,16 +683,20 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
 
 }  // namespace
 
+// The sweep by many blocks: rows long enough to fill several blocks, with at least twice as many groups as survivors (so that
+// the bound leaves out most of the row), and no longer than the scratch holds groups for.
+bool sample_takes_scratch(uint32_t count, uint32_t top_k) {
+    const bool truncated = top_k > 0u && top_k < count;
+    return count >= max(4096u, truncated ? 2u * kSampleGroup * top_k : 0u) && count <= kSampleMaxGroups * kSampleGroup;
+}
+
 hipError_t launch_sample_rows(hipStream_t s, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                               const uint32_t *ids, float temperature, float top_p, uint32_t top_k, uint32_t key_base,
                               float softcap, unsigned long long seed, const uint32_t *key_offset, uint32_t *out_tokens,
                               float *out_prob, SampleScratch sc) {
     const SampleRule rule{temperature, top_p, top_k, key_base, softcap, (uint32_t)seed, (uint32_t)(seed >> 32)};
     const bool truncated = top_k > 0u && top_k < count;
-    // the sweep by many blocks: rows long enough to fill several blocks, with at least twice as many groups as survivors
-    // (so that the bound leaves out most of the row), and no longer than the scratch holds groups for
-    const bool use_scan = sc.group_keys && count >= max(4096u, truncated ? 2u * kSampleGroup * top_k : 0u) &&
-                          count <= kSampleMaxGroups * kSampleGroup;
+    const bool use_scan = sc.group_keys && sample_takes_scratch(count, top_k);
     if (use_scan) {
         const uint32_t n_seg = (count + kSampleSegment - 1) / kSampleSegment;
         const dim3 grid(n_seg, rows);

@@ -371,7 +371,9 @@ int ffmoe_matrix_greedy_conf(ffmoe_matrix *mx, void *stream, const uint16_t *x, 
 /* The greedy choice over rows of fp32 logits that are in memory already - the output of ffmoe_gemv_int4_listed for a
  * drafter's hot vocabulary: out_index[r] = position of the largest finite value of logits[r][0..count), ties to the
  * lowest position, 0xFFFFFFFF when none is finite; out_conf (may be NULL) as above. The caller maps a position
- * through its id list. Replaces argmax_rows_f32 as LMHeadChainInt4.encodeHotGreedyRows dispatches it
+ * through its id list. Rows of more than 8,192 values are split over many blocks, which meet in the context's scratch; shorter
+ * ones, and any under graph capture, take a block per row and write to the caller's buffers alone, so that such calls on
+ * several streams, and replays of a captured one, need no ordering among themselves. Replaces argmax_rows_f32 as LMHeadChainInt4.encodeHotGreedyRows dispatches it
  * (LMHeadChainInt4.swift:144-186,209-223). */
 int ffmoe_argmax_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                       float softcap, uint32_t *out_index, float *out_conf, char **err);
@@ -399,7 +401,9 @@ typedef struct ffmoe_sampling {
  * uint32 added to key_base, for a base that lives on the GPU. Replaces sample_rows_f32 as
  * LMHeadChainInt4.encodeChoice dispatches it (Metal/Sampling/logit.metal:1010-1259,
  * Kernels/Fusions/LMHeadChainInt4.swift:192-223). The top_k set is found exactly (a radix select), where the
- * reference gathers the histogram's edge bin into at most 1,024 candidates. rows <= 16. */
+ * reference gathers the histogram's edge bin into at most 1,024 candidates. Rows of 4,096 logits and more (with top_k:
+ * of 128 top_k and more; up to 524,288) go through the context's scratch, others and any under graph capture do not, as
+ * above; the survivors and the drawn position are the same, the probability agrees to the order of its sums. rows <= 16. */
 int ffmoe_sample_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                       const uint32_t *ids, const ffmoe_sampling *rule, const uint32_t *key_offset, uint32_t *out_tokens,
                       float *out_prob, char **err);

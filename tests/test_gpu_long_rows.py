@@ -101,3 +101,61 @@ def test_weight_offsets_have_the_width_of_a_pointer(ctx, oracle, torch, view):
     assert abs(off) > (1 << 32) or view != "host address"
     y = ctx.gemv_int4(base, Sd, Bd, x, f32_out=True, w_byte_offset=off)
     assert torch.equal(y, ctx.gemv_int4(raw, Sd, Bd, x, f32_out=True))
+
+
+def _choices(ctx, logits, key):
+    return [t.clone() for t in (*ctx.sample_rows(logits, 0.9, 30.0, 11, key_base=key, top_k=64, top_p=0.9),
+                                *ctx.sample_rows(logits, 0.9, 30.0, 11, key_base=key), *ctx.argmax_rows(logits, softcap=30.0))]
+
+
+def test_captured_choices_replay_beside_eager_calls(ctx, torch):
+    # a captured choice over long rows uses nothing of the context: its replays on one stream and the context's eager choices on
+    # another, over other rows and in no order, leave what each leaves alone
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    mine, other = (4 * torch.randn((3, 40961), device="cuda", generator=gen) for _ in range(2))
+    want, want_other = _choices(ctx, mine, 7), _choices(ctx, other, 900)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        captured = _choices(ctx, mine, 7)
+    eager = []
+    for replay in range(12):
+        with torch.cuda.stream(side):
+            graph.replay()
+        eager += [_choices(ctx, other, 900) for _ in range(3)]
+        if replay % 3 == 2:
+            torch.cuda.synchronize()
+            for got in eager:
+                assert all(torch.equal(a, b) for a, b in zip(got, want_other))
+            eager.clear()
+            for i, (got, alone) in enumerate(zip(captured, want)):
+                # positions the same; a probability is a sum in another order over up to 40,961 terms
+                assert torch.equal(got, alone) if i % 2 == 0 else torch.allclose(got, alone, rtol=1e-4, atol=1e-7), (replay, i)
+            for got in captured:
+                got.zero_()
+
+
+def test_choices_that_need_no_scratch_order_no_streams(ctx, torch):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    long_rows, short = torch.randn((1, 16384), device="cuda", generator=gen), torch.randn((2, 1024), device="cuda", generator=gen)
+    big = torch.zeros((8192, 8192), dtype=torch.bfloat16, device="cuda")
+    out = torch.empty_like(big)
+    busy, quick = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.mm(big, big, out=out)
+    with torch.cuda.stream(quick):
+        _choices(ctx, short, 1)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        _choices(ctx, long_rows, 1)                            # the context's scratch is this stream's
+        for _ in range(150):
+            torch.mm(big, big, out=out)
+        end = torch.cuda.Event()
+        end.record()
+    with torch.cuda.stream(quick):
+        _choices(ctx, short, 1)
+    quick.synchronize()
+    assert not end.query(), "the short rows waited for the other stream's work"
+    torch.cuda.synchronize()
