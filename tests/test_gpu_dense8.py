@@ -51,19 +51,71 @@ def test_rows_against_float64(oracle, act, d, f, t):
         ctx.close()
 
 
+def _parts(oracle, d, f, key):
+    g = oracle.seed_tree_key(0x1A8, key)
+    weights = [g.uniform(-0.2, 0.2, r * c).reshape(r, c) for r, c in ((f, d), (f, d), (d, f))]
+    return g, tuple(oracle.quantize_int8(w) for w in weights), tuple(oracle.quantize_int4(w) for w in weights)
+
+
 def test_the_form_follows_the_activation_type(oracle):
-    # the operands are remade when the context changes type, and given back with a 4-bit upload
+    # one context through both types and back, a 4-bit upload and an 8-bit one again: every state gives the bits of a context that
+    # was made for it, so the operands are remade when the context changes type and go with a 4-bit upload
     import torch
     import fieldfare_moe as ff
     ff.lib()
     d, f, t = 128, 192, 650
-    g = oracle.seed_tree_key(0x1A8, "dense8-types")
-    parts = tuple(oracle.quantize_int8(g.uniform(-0.2, 0.2, r * c).reshape(r, c)) for r, c in ((f, d), (f, d), (d, f)))
+    g, int8, int4 = _parts(oracle, d, f, "dense8-types")
     x = torch.from_numpy(g.uniform(-1.0, 1.0, t * d).reshape(t, d).astype(np.float32))
-    outs = {}
+    run = lambda c, act: c.dense_ffn(0, x.to(torch.bfloat16 if act == "bf16" else torch.float16).cuda()).float().cpu().numpy()
+    alone = {}
     for act in ("bf16", "fp16"):
-        ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
-        ctx.upload_expert_parts(0, 0, *parts, int8=True)
-        outs[act] = ctx.dense_ffn(0, x.to(torch.bfloat16 if act == "bf16" else torch.float16).cuda()).float().cpu().numpy()
+        for bits, parts in ((8, int8), (4, int4)):
+            ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+            ctx.upload_expert_parts(0, 0, *parts, int8=bits == 8)
+            alone[act, bits] = run(ctx, act)
+            ctx.close()
+    assert rel_err(alone["bf16", 8], alone["fp16", 8]) < 2e-2 and not np.array_equal(alone["bf16", 8], alone["fp16", 8])
+    assert not np.array_equal(alone["bf16", 8], alone["bf16", 4])
+    ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t)
+    try:
+        for step, (act, upload, bits) in enumerate((("bf16", int8, 8), ("fp16", None, 8), ("bf16", None, 8), ("bf16", int4, 4), ("fp16", None, 4),
+                                                    ("fp16", int8, 8), ("bf16", None, 8))):
+            ctx.set_act_dtype(act)
+            if upload:
+                ctx.upload_expert_parts(0, 0, *upload, int8=bits == 8)
+            assert np.array_equal(run(ctx, act), alone[act, bits]), (step, act, bits)
+    finally:
         ctx.close()
-    assert rel_err(outs["bf16"], outs["fp16"]) < 2e-2 and not np.array_equal(outs["bf16"], outs["fp16"])
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("t", [640, 1153])
+def test_the_gemms_in_a_graph(oracle, act, t):
+    # replayed with new rows in the input and eager calls of the context (another row count, the streaming form) in between
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f = 192, 320
+    g, int8, _ = _parts(oracle, d, f, f"dense8-graph-{t}")
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_expert_parts(0, 0, *int8, int8=True)
+        rows = [torch.from_numpy(g.uniform(-1.0, 1.0, t * d).reshape(t, d).astype(np.float32)).to(dt).cuda() for _ in range(4)]
+        want = [ctx.dense_ffn(0, r) for r in rows]
+        x, y = rows[0].clone(), torch.empty((t, d), dtype=dt, device="cuda")
+        torch.cuda.synchronize()
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=side):
+            ctx.dense_ffn(0, x, out=y)
+        for r, alone in zip(rows, want):
+            x.copy_(r)
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), alone.view(torch.int16))
+            ctx.dense_ffn(0, rows[1][:640])
+            ctx.dense_ffn(0, rows[2][:33])
+            torch.cuda.synchronize()
+    finally:
+        ctx.close()
