@@ -943,7 +943,7 @@ int ffmoe_prefill_plan_stats(ffmoe_ctx *ctx, void *stream, uint32_t *n_pairs, ui
     FF_HIP(hipMemcpy(&host, ctx->pf.plan, sizeof(PrefillPlan), hipMemcpyDeviceToHost));
     if (n_pairs) *n_pairs = host.n_pairs;
     if (n_tiles) {
-        // tiles of FFMOE_PREFILL_TILE_M pairs, whichever size the chunk's own plan cut
+        // counted from the routes, whichever size of tile the chunk's own plan cut
         *n_tiles = 0;
         for (uint32_t e = 0; e < ctx->shape.n_experts; ++e) *n_tiles += (host.expert_count[e] + FFMOE_PREFILL_TILE_M - 1) / FFMOE_PREFILL_TILE_M;
     }

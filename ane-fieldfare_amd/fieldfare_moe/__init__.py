@@ -527,7 +527,7 @@ class Context:
         return _native.prefill_pairs(self._hv, layer, x, sorted_pairs, t, partials)
 
     def prefill_stats(self):
-        """(pairs kept, M-tiles, pairs per expert) of the last prefill call."""
+        """(pairs kept, M-tiles of PREFILL_TILE_M pairs that they make, pairs per expert) of the last prefill call."""
         import numpy as np
         n_pairs, n_tiles = C.c_uint32(), C.c_uint32()
         counts = np.zeros(self.shape.n_experts, np.uint32)

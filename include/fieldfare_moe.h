@@ -47,7 +47,8 @@ enum { FFMOE_GATE = 0, FFMOE_UP = 1, FFMOE_DOWN = 2 };
 #define FFMOE_MAX_VERIFY_ROWS 16 /* maxVerifyTokens, Runtime/Inference/RealForwardRunner.swift:414 */
 #define FFMOE_MAX_EXPERTS 256    /* router limit, Kernels/MoE/MoE.swift:137 */
 #define FFMOE_PREFILL_TILE_M 256 /* pairs per M-tile of the prefill GEMMs (the role of groupTokenExpertPairs' tileM,
-                                    Kernels/Prefill/MoE/PrefillMoEGrouping.swift:49); ffmoe_prefill_plan_stats counts these */
+                                    Kernels/Prefill/MoE/PrefillMoEGrouping.swift:49), and the unit in which
+                                    ffmoe_prefill_plan_stats counts a chunk's tiles; a short chunk's own are smaller */
 
 typedef struct ffmoe_ctx ffmoe_ctx;
 
@@ -251,7 +252,8 @@ int ffmoe_prefill(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t *
 int ffmoe_prefill_pairs(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t *x, uint32_t x_stride,
                         const ffmoe_pair *pairs, uint32_t n_pairs, uint32_t t, uint16_t *partials, char **err);
 
-/* Pairs kept and M-tiles run by the last prefill call on `stream`, and pairs per expert (`counts`,
+/* Pairs kept by the last prefill call on `stream`, the M-tiles of FFMOE_PREFILL_TILE_M pairs that they make, expert by expert
+ * (a property of the routes: the form that ran a short chunk may have cut smaller tiles), and pairs per expert (`counts`,
  * n_experts entries, may be NULL). Waits for the stream. For reporting (the reference's
  * prefillRouted* counters, RealForwardRunner.swift:171-203). */
 int ffmoe_prefill_plan_stats(ffmoe_ctx *ctx, void *stream, uint32_t *n_pairs, uint32_t *n_tiles,
@@ -371,10 +373,10 @@ int ffmoe_matrix_greedy_conf(ffmoe_matrix *mx, void *stream, const uint16_t *x, 
 /* The greedy choice over rows of fp32 logits that are in memory already - the output of ffmoe_gemv_int4_listed for a
  * drafter's hot vocabulary: out_index[r] = position of the largest finite value of logits[r][0..count), ties to the
  * lowest position, 0xFFFFFFFF when none is finite; out_conf (may be NULL) as above. The caller maps a position
- * through its id list. Rows of more than 8,192 values are split over many blocks, which meet in the context's scratch; shorter
- * ones, and any under graph capture, take a block per row and write to the caller's buffers alone, so that such calls on
- * several streams, and replays of a captured one, need no ordering among themselves. Replaces argmax_rows_f32 as LMHeadChainInt4.encodeHotGreedyRows dispatches it
- * (LMHeadChainInt4.swift:144-186,209-223). */
+ * through its id list. Rows of more than 8,192 values are split over many blocks, which meet in the context's scratch;
+ * shorter ones, and any under graph capture, take a block per row and write to the caller's buffers alone, so that such
+ * calls on several streams, and replays of a captured one, need no ordering among themselves. Replaces argmax_rows_f32
+ * as LMHeadChainInt4.encodeHotGreedyRows dispatches it (LMHeadChainInt4.swift:144-186,209-223). */
 int ffmoe_argmax_rows(ffmoe_ctx *ctx, void *stream, const float *logits, uint32_t stride, uint32_t rows, uint32_t count,
                       float softcap, uint32_t *out_index, float *out_conf, char **err);
 

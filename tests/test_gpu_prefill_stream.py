@@ -41,6 +41,7 @@ def test_tile_edges_against_the_oracle(oracle, act, d, f, scale):
         y = ctx.prefill(0, x.cuda(), gi, w.cuda()).float().cpu().numpy()
         n_pairs, n_tiles, got_counts = ctx.prefill_stats()
         assert n_pairs == t and np.array_equal(got_counts, counts)
+        assert n_tiles == int(np.sum((counts + ff.PREFILL_TILE_M - 1) // ff.PREFILL_TILE_M))       # the routes', not the chunk's own
         xf, wf = x.float().numpy(), w.float().numpy()
         ref, spread = np.zeros((t, d), np.float64), np.zeros((t, d), np.float64)
         for ex in range(e):
