@@ -856,9 +856,9 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
             const uint32_t f = ctx->shape.f, d = ctx->shape.d;
             ctx->timer.begin(s);
             FF_HIP(launch_dense8_rows(s, x, x_stride, t, d, f, ctx->dense8_x, ctx->dense8_acts, ctx->f16));
-            FF_HIP(launch_dense8_gemm(s, l.gate_up8_ops, 2 * f, d, true, ctx->dense8_x, t, ctx->dense8_acts, 0, ctx->f16));
+            FF_HIP(launch_dense8_gemm(s, l.gate_up8_ops, 2 * f, d, true, ctx->dense8_x, t, ctx->dense8_acts, 0, ctx->f16, ctx->n_cus));
             ctx->timer.mark(s, FFMOE_K_GATE_UP);
-            FF_HIP(launch_dense8_gemm(s, l.down8_ops, d, f, false, ctx->dense8_acts, t, y, d, ctx->f16));
+            FF_HIP(launch_dense8_gemm(s, l.down8_ops, d, f, false, ctx->dense8_acts, t, y, d, ctx->f16, ctx->n_cus));
             ctx->timer.mark(s, FFMOE_K_DOWN);
             ctx->timer.finish();
             return FFMOE_OK;

@@ -346,13 +346,19 @@ hipError_t launch_dense8_rows(hipStream_t s, const uint16_t *x, uint32_t x_strid
 }
 
 hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t stored_rows, uint32_t n, bool gated, const void *ops, uint32_t t,
-                              void *out, uint32_t out_stride, bool f16) {
+                              void *out, uint32_t out_stride, bool f16, uint32_t n_cus) {
     const uint32_t n_blocks = n_blocks_of(stored_rows), row_blocks = (t + 15) / 16;
     const float *scales = reinterpret_cast<const float *>(static_cast<const uint8_t *>(weights) +
                                                           (size_t)n_blocks * all_groups_of(n) * (kBFrags * kWave * sizeof(uint4)));
-    // Tiles of 64 rows until 128-row tiles give every compute unit a block: whole FFN, 64 | 128 rows per tile, us: 704 rows
-    // 69 | 75, 1,000 rows 85 | 90, 1,250 rows 111 | 91, 2,000 rows 141 | 125, 3,072 rows 212 | 181, 4,096 rows 266 | 217.
-    const bool small = t <= 1088;
+    // Tiles of 64 rows while a compute unit holds few of them: 128-row tiles halve the weights' way through LDS but leave a
+    // chip that is not full to fewer blocks. The line is drawn on the XCD that has the most N-blocks (all row tiles of one run
+    // there), at blocks of 64 rows per compute unit: 3 for the gated product, 1.75 for the plain one. Whole FFN,
+    // 64 | 128 rows per tile in both products, us: 2,816 -> 2,112 -> 2,816, 640 rows (1.6 and 0.9 blocks) 72 | 78, 1,024 rows
+    // (2.5, 1.5) 88 | 91, 1,280 rows (3.1, 1.9) 114 | 94, 3,072 rows 222 | 186; 2,816 -> 704, 1,024 rows (1, 1.5) 52 | 61, 2,048
+    // rows (2, 3) 66 | 67; 704 -> 2,816, 1,152 rows (3.4, 0.6) 63 | 66, and 58 with 128 gated and 64 plain; 512 -> 512, 2,048
+    // rows (1, 1) 26 | 30. Either gives the same bits.
+    const uint32_t m64 = (row_blocks + 3) / 4;
+    const bool small = 4 * ((n_blocks + 7) / 8) * m64 <= (gated ? 12u : 7u) * (n_cus / 8);
     const uint32_t tile_blocks = small ? 4 : 8, m_tiles = (row_blocks + tile_blocks - 1) / tile_blocks;
     const dim3 grid(8 * ((n_blocks + 7) / 8) * m_tiles);
 #define FFMOE_DENSE8(N, W)                                                                                                              \

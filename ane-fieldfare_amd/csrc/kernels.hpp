@@ -250,7 +250,7 @@ hipError_t launch_dense8_weights(hipStream_t s, const uint8_t *tiles, const uint
 hipError_t launch_dense8_rows(hipStream_t s, const uint16_t *x, uint32_t x_stride, uint32_t t, uint32_t d, uint32_t f, void *x_ops,
                               void *act_ops, bool f16);
 hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t stored_rows, uint32_t n, bool gated, const void *ops, uint32_t t,
-                              void *out, uint32_t out_stride, bool f16);
+                              void *out, uint32_t out_stride, bool f16, uint32_t n_cus);
 
 // prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr.
 // Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.

@@ -14,7 +14,9 @@ def _gelu(x):
 
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
-@pytest.mark.parametrize("d,f,t", [(128, 64, 640), (192, 320, 641), (64, 704, 703), (192, 1472, 1088), (448, 192, 1089), (2816, 128, 1153)])
+# the last four: 64-row tiles in both products, 128 in the plain one alone, in the gated one alone, in both
+@pytest.mark.parametrize("d,f,t", [(128, 64, 640), (192, 320, 641), (64, 704, 703), (192, 1472, 1088), (448, 192, 1089), (2816, 128, 1153),
+                                   (192, 2816, 1025), (2112, 2112, 1217)])
 def test_rows_against_float64(oracle, act, d, f, t):
     import torch
     import fieldfare_moe as ff
@@ -40,9 +42,9 @@ def test_rows_against_float64(oracle, act, d, f, t):
         assert np.all(np.abs(yf - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
         assert cosine(yf, ref) > 0.99999 and rel_err(yf, ref) < (1e-2 if act == "bf16" else 1.5e-3)
         # a row does not depend on the rows beside it (both tile sizes sum in one order)
-        if t > 1088:
-            part = ctx.dense_ffn(0, x[:1088].cuda()).float().cpu().numpy()
-            assert np.array_equal(part, yf[:1088])
+        if t > 640:
+            part = ctx.dense_ffn(0, x[:640].cuda()).float().cpu().numpy()
+            assert np.array_equal(part, yf[:640])
         # other rows are untouched by one that is not finite
         x[7, 3] = float("inf")
         got = ctx.dense_ffn(0, x.cuda()).float().cpu().numpy()
