@@ -39,10 +39,6 @@ struct ffmoe_layer {
 // streaming pass per 16 rows (measured at 2816 -> 2112 -> 2816: streaming 19 us at 32 rows + 8.8 us per 32 more, 42 us at
 // 127; the GEMM form 50 us at 128, 58 at 192, 67 at 256, 100 at 1,024, 244 at 3,072).
 constexpr uint32_t kGemm8MinRows = 192;
-// And from this many the GEMMs on integer operands (dense8.hip), which do half the products; below, their blocks are too few to
-// hide a group's round trip. Library form | integer form, us: 301 rows 48 | 61, 512 rows 61 | 65, 700 rows 74 | 69, 1,000 rows
-// 97 | 85, 1,500 rows 124 | 102, 3,072 rows 248 | 181.
-constexpr uint32_t kDense8MinRows = 640;
 // Up to this many rows a 4-bit dense layer streams its arena tiles through the resident-matrix GEMV (a grid row per 16
 // input rows) instead of the grouped products (which beat it from about 200 rows on in bf16 and 370 in FP16: 384 rows 66 us
 // against 45 and 64; the rows of a chunk and of a part of it are equal bit for bit up to here, so the line stays put).
@@ -84,7 +80,7 @@ struct ffmoe_ctx {
     bool f16 = false;                // activations are FP16 (ffmoe_set_activation_dtype)
     // the 8-bit dense layers' GEMM form: the library handle and the fp32 sums [max_tokens][max(4 f, 2 d)]
     rocblas_handle blas = nullptr;
-    float *gemm8_sums = nullptr;                                // sums of kDense8MinRows rows at most
+    float *gemm8_sums = nullptr;                                // fewer rows than dense8_min_rows
     uint8_t *dense8_x = nullptr, *dense8_acts = nullptr;        // the integer form's inputs as operands, max_tokens rows
     SampleScratch sample{};          // what the sampled choice over long rows leaves between its two launches
     KernelTimer timer;
@@ -852,7 +848,7 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
             return fail(err, FFMOE_ERR_INVALID, "x must be 16-byte aligned with a stride that is a multiple of 8 and >= d");
         hipStream_t s = static_cast<hipStream_t>(stream);
         claim_scratch(ctx, stream);
-        if (t >= kDense8MinRows && l.gate_up8_ops) {
+        if (l.gate_up8_ops && t >= dense8_min_rows(ctx->shape.d, ctx->shape.f)) {
             const uint32_t f = ctx->shape.f, d = ctx->shape.d;
             ctx->timer.begin(s);
             FF_HIP(launch_dense8_rows(s, x, x_stride, t, d, f, ctx->dense8_x, ctx->dense8_acts, ctx->f16));
@@ -1294,10 +1290,11 @@ int ffmoe_upload_expert_parts_int8(ffmoe_ctx *ctx, uint32_t layer, const ffmoe_p
             return fail(err, FFMOE_ERR_RUNTIME, "rocblas_create_handle failed");
         }
         hipError_t e = hipSuccess;
+        const uint32_t min_rows8 = dense8_min_rows(sh.d, sh.f);
         if (!ctx->gemm8_sums)
             e = hipMalloc(reinterpret_cast<void **>(&ctx->gemm8_sums),
-                          (size_t)std::min(sh.max_tokens, kDense8MinRows) * std::max(4 * (size_t)sh.f, 2 * (size_t)sh.d) * sizeof(float));
-        if (sh.max_tokens >= kDense8MinRows) {
+                          (size_t)std::min(sh.max_tokens, min_rows8) * std::max(4 * (size_t)sh.f, 2 * (size_t)sh.d) * sizeof(float));
+        if (sh.max_tokens >= min_rows8) {
             if (e == hipSuccess && !ctx->dense8_x) e = hipMalloc(reinterpret_cast<void **>(&ctx->dense8_x), dense8_operand_bytes(sh.max_tokens, sh.d));
             if (e == hipSuccess && !ctx->dense8_acts)
                 e = hipMalloc(reinterpret_cast<void **>(&ctx->dense8_acts), dense8_operand_bytes(sh.max_tokens, sh.f));

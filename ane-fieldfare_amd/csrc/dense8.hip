@@ -320,6 +320,19 @@ uint32_t n_blocks_of(uint32_t stored_rows) { return (stored_rows / 16 + kTilesN 
 
 }  // namespace
 
+// While its blocks are fewer than the compute units hold, a GEMM here takes one block's chain of groups, 0.7 us each however few
+// the rows (a group's round trip), where the library's two take 22 us and 12.5 us per 1,000 rows and 10^6 weights of a
+// projection: the lines cross where rows * d f / 10^6 is 68 times the groups of both products less 2,000 (fitted at 18
+// widths, GPU time). Library form | this one, us: 2,816 -> 2,112, 576 rows 65 | 67, 704 rows 76 | 70, 3,072 rows 248 | 178; 2,816
+// -> 704, 640 rows 41 | 50, 896 rows 53 | 52; 1,024 -> 2,816, 704 rows 52 | 57, 896 rows 59 | 59, 1,024 rows 67 | 60; 2,816 -> 2,816,
+// 576 rows 78 | 77; 512 -> 512, 640 rows 24 | 22. Not below 640 rows, where the forms meet at the widest, nor beyond 1,024, where
+// the narrowest (2,816 -> 256, 38 | 47) still cross, but in a call that the library's own 41 us on the host bound.
+uint32_t dense8_min_rows(uint32_t d, uint32_t f) {
+    const uint32_t groups = all_groups_of(d) + all_groups_of(f);
+    const uint64_t line = groups * 68ull <= 2000ull ? 0 : (groups * 68ull - 2000ull) * 1000000ull / ((uint64_t)d * f);
+    return (uint32_t)(line < 640 ? 640 : line > 1024 ? 1024 : line);
+}
+
 size_t dense8_weight_bytes(uint32_t stored_rows, uint32_t n) {
     const size_t blocks = (size_t)n_blocks_of(stored_rows) * all_groups_of(n);
     return blocks * (kBFrags * kWave * sizeof(uint4) + 16 * kTilesN * sizeof(float));

@@ -243,6 +243,8 @@ inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts) {
 }
 
 // dense8.hip: the 8-bit dense FFN at many rows. `stored_rows` = rows of the resident matrix as stored (the gated one: 2 f).
+// dense8_min_rows: from how many rows on; below, the library's GEMMs on hi / lo rows (matrix.hip) are the faster form
+uint32_t dense8_min_rows(uint32_t d, uint32_t f);
 size_t dense8_weight_bytes(uint32_t stored_rows, uint32_t n);
 size_t dense8_operand_bytes(uint32_t rows, uint32_t n);
 hipError_t launch_dense8_weights(hipStream_t s, const uint8_t *tiles, const uint8_t *scales, uint32_t stored_rows, uint32_t n, void *out,

@@ -42,9 +42,9 @@ def test_rows_against_float64(oracle, act, d, f, t):
         assert np.all(np.abs(yf - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
         assert cosine(yf, ref) > 0.99999 and rel_err(yf, ref) < (1e-2 if act == "bf16" else 1.5e-3)
         # a row does not depend on the rows beside it (both tile sizes sum in one order)
-        if t > 640:
-            part = ctx.dense_ffn(0, x[:640].cuda()).float().cpu().numpy()
-            assert np.array_equal(part, yf[:640])
+        first = 1024 if t > 1024 else 640                    # from 1,024 rows on every width takes this form
+        part = ctx.dense_ffn(0, x[:first].cuda()).float().cpu().numpy()
+        assert np.array_equal(part, yf[:first])
         # other rows are untouched by one that is not finite
         x[7, 3] = float("inf")
         got = ctx.dense_ffn(0, x.cuda()).float().cpu().numpy()
@@ -88,6 +88,27 @@ def test_the_form_follows_the_activation_type(oracle):
             assert np.array_equal(run(ctx, act), alone[act, bits]), (step, act, bits)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("d,f,line", [(2816, 128, 1024), (1024, 1984, 689), (128, 192, 640)])
+def test_the_line_to_the_library_form(oracle, d, f, line):
+    # the row before and the row after the line that the widths draw, in a context for more rows and in one for the row before alone
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    g, int8, _ = _parts(oracle, d, f, f"dense8-line-{d}")
+    x = torch.from_numpy(g.uniform(-1.0, 1.0, line * d).reshape(line, d).astype(np.float32)).to(torch.bfloat16).cuda()
+    outs = []
+    for cap in (line, line - 1):
+        ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=cap)
+        ctx.upload_expert_parts(0, 0, *int8, int8=True)
+        outs += [ctx.dense_ffn(0, x[:t]).float().cpu().numpy() for t in (line - 1, line) if t <= cap]
+        ctx.close()
+    library, integers, alone = outs
+    assert np.array_equal(library, alone)                    # the same form, whatever the context could also do
+    assert not np.array_equal(library, integers[:-1])        # another one
+    # 16-bit results of one rounding each way, of sums whose weights have 16 significant bits or all of them
+    assert rel_err(library, integers[:-1]) < 2e-2 and cosine(library, integers[:-1]) > 0.9999
 
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
