@@ -15,7 +15,17 @@
 namespace ffmoe {
 namespace {
 
-constexpr uint32_t kRouterSmallRows = 160;     // the most rows that take the form below where the two-pass form could serve
+// Whether a prompt of t rows takes the form below where the two-pass form could serve. The two passes of the prefill form are
+// chains of round trips, 6.3 us + 30 ns per expert + 3.2 ns per column (FP16 rows 4.4) however few the rows; one block per
+// expert and four rows costs the router's weights once more from the caches for every four rows, 5.5 us + 0.58 ns per row and
+// expert whatever the columns (fitted at 8 tables). Two-pass form | this one, us, bf16: 2,816 x 128, 17 rows
+// 18.9 | 7.6, 64 rows 19.3 | 10.6, 128 rows 19.3 | 15.1, 160 rows 19.4 | 17.3; 2,048 x 128, 128 rows 16.3 | 14.9, 160 rows
+// 16.5 | 17.1; 1,024 x 64, 160 rows 11.7 | 11.3; 256 x 128, 64 rows 10.6 | 10.1, 128 rows 10.7 | 14.5; 512 x 16, 160 rows
+// 7.9 | 7.1; FP16, 2,816 x 128, 160 rows 22.8 | 17.4; 2,048 x 128, 160 rows 18.5 | 17.0; 256 x 128, 128 rows 11.9 | 14.5. Same
+// pinned sums: same routes bit for bit.
+bool router_small_rows(uint32_t t, uint32_t n_experts, uint32_t d, bool f16) {      // (in units of 20 ps)
+    return t <= 160 && 29u * n_experts * t <= 40000u + 1500u * n_experts + (f16 ? 220u : 160u) * d;
+}
 
 // Decode / verify / short-prompt router logits. grid = (E, ceil(T / 4)); the four waves of a block are the
 // four sub-accumulators of one expert row for four tokens; wave 0 combines them. (A variant whose last
@@ -496,11 +506,7 @@ hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uin
     const bool two_pass = rw.w_frag && !rw.w_is_f32 && !rw.effective_scale && !want_logits && d % 256 == 0 && d <= 1024 * kExactSteps &&
                           n_experts % 16 == 0 && n_experts <= 128 && top_k <= 8 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                           x_stride % 8 == 0 && scratch;
-    // The two passes of the prefill form are two chains of round trips, 19 us (FP16: 22) however few the rows; one block per
-    // expert and four rows costs the router's weights once more from the caches for every four rows. 2,816 x 128, two-pass
-    // form against this one, us, bf16 (FP16): 17 rows 18.6 | 8.0 (22.2 | 7.9), 64 rows 18.8 | 10.3, 128 rows 19.1 | 14.8
-    // (22.5 | 14.7), 160 rows 19.3 | 16.9, 200 rows 19.6 | 19.8 (22.8 | 19.9). Same pinned sums: same routes bit for bit.
-    if (t <= FFMOE_MAX_VERIFY_ROWS || (two_pass && t <= kRouterSmallRows)) {
+    if (t <= FFMOE_MAX_VERIFY_ROWS || (two_pass && router_small_rows(t, n_experts, d, f16))) {
         const dim3 grid(n_experts, (t + kChunkTokens - 1) / kChunkTokens);
 #define FFMOE_ROUTER(WF, XA)                                                                                 \
     hipLaunchKernelGGL((router_small_kernel<WF, XA>), grid, dim3(256), 0, s, rw.w, rw.effective_scale, x,   \
