@@ -237,8 +237,8 @@ constexpr uint32_t kPrefillStreamPairs = 48;
 constexpr uint32_t kDenseTileStreamRows = 896;       // and the most rows at which a dense FFN's chunk does
 inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts) {
     const uint32_t whole = max_pairs / FFMOE_PREFILL_TILE_M;
-    // 32 pairs a tile up to 28 per expert, 64 up to 48: fewer than n_experts full tiles
-    const uint32_t small = n_experts == 1 ? kDenseTileStreamRows / 32 : n_experts;
+    // tiles of 32 pairs or more up to 48 per expert: 1.5 n_experts full ones at most
+    const uint32_t small = n_experts == 1 ? kDenseTileStreamRows / 32 : kPrefillStreamPairs * n_experts / 32;
     return (whole > small ? whole : small) + n_experts + 1;
 }
 
@@ -259,7 +259,7 @@ hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t store
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,
                           const uint16_t *x, uint32_t x_stride, uint32_t t, const uint32_t *idx, const uint16_t *w,
                           const ffmoe_pair *pairs, uint32_t n_pairs_in, uint16_t *y, uint16_t *partials_out,
-                          PrefillScratch sc, KernelTimer *timer, bool f16 = false, bool dense = false);
+                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16 = false, bool dense = false);
 
 // Test hook: the weight fragments of one expert's gate/up (or down) tiles as the grouped GEMM's matrix instructions
 // read them from LDS: [N-block][group][fragment 0..15][lane] x 16 bytes, `prefill_dump_fragments` fragments in all.

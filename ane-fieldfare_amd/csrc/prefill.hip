@@ -1087,15 +1087,25 @@ __global__ void prefill_dump_plan_kernel(uint32_t expert, PrefillPlan *plan, Pre
 
 // Pairs per M-tile, as a shift: below 8 (256 pairs) the chunk goes through prefill_stream_kernel. The line is drawn by the
 // pairs per expert on average, from the chunk's size alone: the counts themselves are only known on the device, and a pair
-// list's rows do not depend on how many of the chunk's pairs it names. Router table to combined rows, 128 experts, top-8,
-// 2,816 x 704, us at 32 | 64 | 256 pairs per tile, bf16 (FP16): 37 rows 97 | 101 | 143 (106 | 110 | 174), 301 rows
-// 120 | 126 | 172 (130 | 137 | 191), 400 rows (25 pairs) 129 | 137 | 177, 512 rows (32) 152 | 147 | 182, 700 rows (44)
-// 196 | 170 | 195 (215 | 183 | 211), 1,000 rows (62, where many experts take two tiles) 218 | 220 | 219. Tiles of 16 pairs
-// gain nothing over 32 (37 rows: 99), tiles of 128 lose everywhere (1,000 rows: 227, two waves per SIMD).
-uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts) {
+// list's rows do not depend on how many of the chunk's pairs it names. Up to 28 the streaming product wins at every width.
+// Beyond, up to 48: tiles of 32 pairs still where a tile from every expert would not fill the chip (its blocks then run at once,
+// and a shorter tile is a shorter chain); tiles of 64 where K is long enough to pay for a block's start and end; else the
+// grouped GEMMs, which have to expand little there. Router table to combined rows, us at 32 | 64 | 256 pairs per tile, bf16 (FP16):
+// 128 experts, top-8, 2,816 x 704: 37 rows 97 | 101 | 143 (106 | 110 | 174), 301 rows 120 | 126 | 172 (130 | 137 | 191), 512 rows
+// (32 pairs) 166 | 152 | 186 (178 | 165 | 203), 704 rows (44) 207 | 178 | 203 (220 | 192 | 215), 768 rows (48) 220 | 184 | 208
+// (232 | 202 | 224), 1,000 rows (62, where many experts take two tiles) 218 | 220 | 219. 8 experts, 4,096 x 1,536: 28 pairs 56 | 62 | 69,
+// 40 pairs 66 | 72 | 70 (76 | 87 | 83); 16 experts, 2,816 x 704, 48 pairs 54 | 55 | 54 (61 | 67 | 63). 64 experts, 1,024 x 512:
+// 32 pairs 39 | 38 | 42 (49 | 45 | 48), 48 pairs 51 | 45 | 45 (57 | 53 | 51); 64 experts, 1,536 x 768, 48 pairs 77 | 71 | 74 (85 | 80 |
+// 84); 256 experts, 512 x 256, 28 pairs 48 | 49 | 52, 40 pairs 59 | 56 | 53 (64 | 65 | 59).
+// Skewed routes move nothing: at the first shape with Zipf popularity of exponent 0.6, 1.1 and 1.6 the streaming form wins at
+// every size up to 48 pairs (448 rows 146 | 159 | 166 against 186 | 201 | 196 for the GEMMs, 768 rows 192 | 201 | 212 against 225 |
+// 226 | 232). Tiles of 16 pairs gain nothing over 32 (37 rows: 99), tiles of 128 lose everywhere (1,000 rows: 227, two waves per
+// SIMD).
+uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts, uint32_t d, uint32_t n_nblocks, uint32_t n_cus, bool f16) {
     if (n_items <= 28 * n_experts) return 5;
-    if (n_items <= kPrefillStreamPairs * n_experts) return 6;
-    return 8;
+    if (n_items > kPrefillStreamPairs * n_experts) return 8;
+    if (n_nblocks * n_experts <= n_cus) return 5;
+    return n_items <= 32 * n_experts || d >= (f16 ? 1536u : 1024u) ? 6 : 8;
 }
 
 // The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths). 2,816 -> 2,112 -> 2,816, us at
@@ -1139,7 +1149,7 @@ hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, 
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,
                           const uint16_t *x, uint32_t x_stride, uint32_t t, const uint32_t *idx, const uint16_t *w,
                           const ffmoe_pair *pairs, uint32_t n_pairs_in, uint16_t *y, uint16_t *partials_out,
-                          PrefillScratch sc, KernelTimer *timer, bool f16, bool dense) {
+                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16, bool dense) {
     // dense: the caller vouches for a dense FFN's chunk - one expert, top_k = 1, every row routed to it at weight 1
     dense = dense && n_experts == 1 && top_k == 1 && !pairs && !y;
     timer->begin(s);
@@ -1153,7 +1163,9 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     src.t = t;
     if (src.n_items == 0) return hipSuccess;
     const uint32_t n_blocks = (src.n_items + kSortBlock - 1) / kSortBlock;
-    const uint32_t tile_shift = dense ? dense_tile_shift(t) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts);
+    const uint32_t nb_gu = (g.gu_rb + kTilesPerBlock - 1) / kTilesPerBlock, nb_dn = (g.dn_rbp + kTilesPerBlock - 1) / kTilesPerBlock;
+    const uint32_t tile_shift =
+        dense ? dense_tile_shift(t) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts, g.d, nb_gu, n_cus, f16);
     const bool streamed = tile_shift < 8;
     if (dense) {
         hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_shift, sc.plan, sc.tiles, sc.sorted_token,
@@ -1173,7 +1185,6 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     timer->mark(s, FFMOE_K_PREFILL_SORT);
     const uint32_t tile_cap = min(sc.max_tiles, (src.n_items >> tile_shift) + n_experts);
     const uint32_t tile_slots = (tile_cap + 7) / 8 * 8;
-    const uint32_t nb_gu = (g.gu_rb + kTilesPerBlock - 1) / kTilesPerBlock, nb_dn = (g.dn_rbp + kTilesPerBlock - 1) / kTilesPerBlock;
     if (f16 && !sc.act_scale) return hipErrorInvalidValue;      // allocated when the context was switched to FP16
     // grid: (N-blocks x tile slots) in either order of the kernel's block map
     const bool nb_major = n_experts == 1;
