@@ -1108,10 +1108,18 @@ uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts, uint32_t d, ui
     return n_items <= 32 * n_experts || d >= (f16 ? 1536u : 1024u) ? 6 : 8;
 }
 
-// The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths). 2,816 -> 2,112 -> 2,816, us at
-// 32 | 64 | 256 rows per tile, bf16 (FP16): 512 rows 51 | 64 | 79 (70 | 84 | 109), 700 rows 66 | 71 | 79 (86 | 93 | 109),
-// 1,000 rows 80 | 83 | 80 (101 | 106 | 109).
-uint32_t dense_tile_shift(uint32_t t) { return t <= kDenseTileStreamRows ? 5 : 8; }
+// The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths): tiles of 32 rows while the gate/up
+// launch is one round (four blocks per compute unit on the XCD with the most N-blocks), or while a chunk's products are few
+// enough that the GEMMs' expansion of every weight for each 256 rows still costs more; at most kDenseTileStreamRows.
+// us at 32 | 256 rows per tile, bf16 (FP16): 2,816 -> 2,112, 512 rows 54 | 78 (71 | 107), 800 rows 69 | 79 (88 | 108), 896 rows
+// 78 | 79 (98 | 108); 2,816 -> 2,816, 672 rows 70 | 87, 832 rows 87 | 88, 896 rows 94 | 88 (114 | 121); 4,096 -> 2,816, 672 rows 96 |
+// 106, 704 rows 109 | 106 (126 | 140), 896 rows 129 | 108 (147 | 142); 2,816 -> 704, 896 rows 40 | 64 (48 | 76). Tiles of 64 gain
+// nothing (2,816 -> 2,112, 700 rows 71 | 66 at 32).
+uint32_t dense_tile_shift(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, bool f16) {
+    if (t > kDenseTileStreamRows) return 8;
+    const bool one_round = (n_nblocks + 7) / 8 * ((t + 31) / 32) <= 4 * (n_cus / 8);
+    return one_round || (uint64_t)t * g.d * g.f <= (f16 ? 9600000000ull : 6600000000ull) ? 5 : 8;
+}
 
 template <bool GATE_UP>
 auto stream_kernel(uint32_t tile_shift, bool f16) {
@@ -1165,7 +1173,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     const uint32_t n_blocks = (src.n_items + kSortBlock - 1) / kSortBlock;
     const uint32_t nb_gu = (g.gu_rb + kTilesPerBlock - 1) / kTilesPerBlock, nb_dn = (g.dn_rbp + kTilesPerBlock - 1) / kTilesPerBlock;
     const uint32_t tile_shift =
-        dense ? dense_tile_shift(t) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts, g.d, nb_gu, n_cus, f16);
+        dense ? dense_tile_shift(t, g, nb_gu, n_cus, f16) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts, g.d, nb_gu, n_cus, f16);
     const bool streamed = tile_shift < 8;
     if (dense) {
         hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_shift, sc.plan, sc.tiles, sc.sorted_token,

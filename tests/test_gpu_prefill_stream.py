@@ -87,14 +87,15 @@ def test_the_line_to_the_grouped_gemms(oracle, t):
         ctx.close()
 
 
+# 2,944 -> 2,816 (wider than the GEMV's ring, so from 17 rows on): one round of gate/up blocks up to 672 rows, bf16's products
+# up to 796
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
-@pytest.mark.parametrize("t", [385, 895, 896, 897])
-def test_dense_chunks_beyond_the_gemv(oracle, act, t):
-    # a dense FFN's chunk: tiles of 32 rows up to 896 rows, the GEMMs from there on
+@pytest.mark.parametrize("d,f,t", [(192, 320, 385), (192, 320, 895), (192, 320, 896), (192, 320, 897), (2944, 2816, 673), (2944, 2816, 797)])
+def test_dense_chunks_beyond_the_gemv(oracle, act, d, f, t):
+    # a dense FFN's chunk: tiles of 32 rows up to 896 rows, fewer where wide, the GEMMs from there on
     import torch
     import fieldfare_moe as ff
     ff.lib()
-    d, f = 192, 320
     g = oracle.seed_tree_key(0x5EED, f"dense-tiles-{t}")
     parts = tuple(oracle.quantize_int4(g.uniform(-0.3, 0.3, r * c).reshape(r, c)) for r, c in ((f, d), (f, d), (d, f)))
     x = torch.from_numpy(g.uniform(-1.0, 1.0, t * d).reshape(t, d).astype(np.float32)).to(torch.bfloat16 if act == "bf16" else torch.float16)
