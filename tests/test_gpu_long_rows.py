@@ -113,7 +113,7 @@ def test_captured_choices_replay_beside_eager_calls(ctx, torch):
     # another, over other rows and in no order, leave what each leaves alone
     gen = torch.Generator(device="cuda")
     gen.manual_seed(5)
-    mine, other = (4 * torch.randn((3, 40961), device="cuda", generator=gen) for _ in range(2))
+    mine, other = (4 * torch.randn((8, 262143), device="cuda", generator=gen) for _ in range(2))
     want, want_other = _choices(ctx, mine, 7), _choices(ctx, other, 900)
     side = torch.cuda.Stream()
     torch.cuda.synchronize()
@@ -131,10 +131,28 @@ def test_captured_choices_replay_beside_eager_calls(ctx, torch):
                 assert all(torch.equal(a, b) for a, b in zip(got, want_other))
             eager.clear()
             for i, (got, alone) in enumerate(zip(captured, want)):
-                # positions the same; a probability is a sum in another order over up to 40,961 terms
+                # positions the same; a probability is a sum in another order over up to 262,143 terms
                 assert torch.equal(got, alone) if i % 2 == 0 else torch.allclose(got, alone, rtol=1e-4, atol=1e-7), (replay, i)
             for got in captured:
                 got.zero_()
+
+
+def test_a_captured_choice_is_one_kernel(ctx, torch):
+    # the split form's two launches meet in the context's scratch; under capture there is one launch per call and no meeting
+    import ctypes as C
+    hip = C.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    logits = torch.zeros((2, 32768), device="cuda")
+    side = torch.cuda.Stream()
+    for call in (lambda: ctx.sample_rows(logits, 0.9, 30.0, 11, top_k=64, top_p=0.9), lambda: ctx.sample_rows(logits, 0.9, 30.0, 11),
+                 lambda: ctx.argmax_rows(logits, softcap=30.0)):
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=side):
+            call()
+        nodes = C.c_size_t()
+        assert hip.hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(nodes)) == 0
+        assert nodes.value == 1
 
 
 def test_choices_that_need_no_scratch_order_no_streams(ctx, torch):
@@ -143,10 +161,12 @@ def test_choices_that_need_no_scratch_order_no_streams(ctx, torch):
     long_rows, short = torch.randn((1, 16384), device="cuda", generator=gen), torch.randn((2, 1024), device="cuda", generator=gen)
     big = torch.zeros((8192, 8192), dtype=torch.bfloat16, device="cuda")
     out = torch.empty_like(big)
-    busy, quick = torch.cuda.Stream(), torch.cuda.Stream()
+    # several quick streams: one of them may share the busy stream's hardware queue, all do not
+    busy, quick = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(6)]
     torch.mm(big, big, out=out)
-    with torch.cuda.stream(quick):
-        _choices(ctx, short, 1)
+    for q in quick:
+        with torch.cuda.stream(q):
+            _choices(ctx, short, 1)
     torch.cuda.synchronize()
     with torch.cuda.stream(busy):
         _choices(ctx, long_rows, 1)                            # the context's scratch is this stream's
@@ -154,8 +174,13 @@ def test_choices_that_need_no_scratch_order_no_streams(ctx, torch):
             torch.mm(big, big, out=out)
         end = torch.cuda.Event()
         end.record()
-    with torch.cuda.stream(quick):
-        _choices(ctx, short, 1)
-    quick.synchronize()
-    assert not end.query(), "the short rows waited for the other stream's work"
+    done = [torch.cuda.Event() for _ in quick]
+    for q, event in zip(quick, done):
+        with torch.cuda.stream(q):
+            _choices(ctx, short, 1)
+            event.record()
+    early = 0
+    while not end.query():
+        early = sum(event.query() for event in done)
+    assert early, "the short rows waited for the other stream's work"
     torch.cuda.synchronize()
