@@ -147,6 +147,31 @@ __device__ __forceinline__ uint4 unpack8_fine(uint32_t w) {
 // across the barrier; here the compiler's own counters still guard each prefetched register at its use.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Workgroup barrier behind which every load into LDS that any wave of the block asked for is there, but for each wave's last
+// IN_FLIGHT global loads. It does not wait for the waves' own LDS reads: whoever fills a buffer behind it again has to know that
+// their results were used.
+template <int IN_FLIGHT> __device__ __forceinline__ void vmem_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IN_FLIGHT) : "memory");
+}
+
+// Global memory to LDS with no register in between: lane l's 16 (4) bytes go to LDS byte `to` + 16 l (4 l), `to` wave-uniform.
+// Inline, because the compiler otherwise waits for every such load in front of the next LDS read, whatever buffer that reads;
+// the caller waits (vmem_barrier) before anything of the block reads the data.
+__device__ __forceinline__ void global_to_lds_16(const void *from, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
+}
+// (the same from a wave-uniform base and a byte offset per lane)
+__device__ __forceinline__ void global_to_lds_16(const void *base, uint32_t offset, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
+}
+__device__ __forceinline__ void global_to_lds_4(const void *from, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(from), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
+}
+
+__device__ __forceinline__ void global_to_lds_4(const void *base, uint32_t offset, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
+}
+
 // xor-butterfly sum across the 64 lanes (masks 32,16,8,4,2,1): every lane ends with the same value, and
 // every addition has the operands v[i] and v[i ^ mask] - the order the CPU oracle restates. The partners
 // come through register-to-register lane moves (gfx950 row swaps for 32 and 16, DPP rotations and quad

@@ -262,7 +262,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
                           PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16 = false, bool dense = false);
 
 // Test hook: the weight fragments of one expert's gate/up (or down) tiles as the grouped GEMM's matrix instructions
-// read them from LDS: [N-block][group][fragment 0..15][lane] x 16 bytes, `prefill_dump_fragments` fragments in all.
+// receive them: [N-block][group][fragment 0..15][lane] x 16 bytes, `prefill_dump_fragments` fragments in all.
 // Fragment u = arena tile (u % 8) / 2 of the N-block, stream u % 2, k-half u / 8; lane l holds row l % 16 of the
 // stream and k = 32 * (k-half) + 8 * (l / 16) .. + 7 of the group.
 uint32_t prefill_dump_fragments(const ArenaGeom &g, bool gate_up);

@@ -1,5 +1,5 @@
 // Prefill routed experts: expert-sorted (token, expert) pairs, then two grouped GEMMs on the matrix
-// units whose weight tiles are dequantised INT4 -> bf16 into LDS.
+// units whose weight tiles are dequantised INT4 -> bf16 on the way into their operands.
 //
 // Replaces the host-side pair sort of PrefillMoEGrouping.groupTokenExpertPairs
 // (Kernels/Prefill/MoE/PrefillMoEGrouping.swift:49-110), prefill_routed_gate_up_tensorops /
@@ -11,10 +11,9 @@
 // order the reference's comparator produces (PrefillMoEGrouping.swift:66-75). Only integer counting uses
 // LDS atomics; every position comes from prefix sums, so the result does not depend on timing.
 //
-// GEMM: one block = one M-tile of up to 256 same-expert pairs x 128 weight rows (4 arena tiles per
-// 64-wide group). Per group the four tiles' weights are expanded once to bf16(fma(q, scale, bias)) - the
-// reference's 16-bit tile weight (prefill.metal:581-590) - into LDS in the register layout
-// v_mfma_f32_16x16x32_bf16 wants; the pairs' inputs go from global memory straight into that layout.
+// GEMM: items of one M-tile of up to 256 same-expert pairs x 256 weight rows, a block per compute unit walking a list of them. Every
+// wave expands its own arena tile to bf16(fma(q, scale, bias)) - the reference's 16-bit tile weight (prefill.metal:581-590) - in
+// the register layout v_mfma_f32_16x16x32_bf16 wants; the pairs' inputs and the packed tiles go from global memory straight into LDS.
 // fp32 accumulation; GELU-tanh(gate) * up in the epilogue.
 // bf16 activations make the reference's power-of-two block scaling (prefill.metal:593-598, an FP16 range
 // fix) unnecessary.
@@ -280,18 +279,25 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Grouped GEMM. One block = one M-tile (up to 256 pairs of one expert) x one N-block (4 arena tiles =
-// 128 weight rows); block ids are laid out so that all N-blocks of an M-tile run on one XCD and find the
-// tile's A rows in that XCD's L2. The M-tile's 16-row blocks are dealt round-robin to the four waves
-// (wave w owns blocks w, w + 4, ...), so a short tile still loads all four matrix units evenly.
-//   A: every lane loads its own MFMA fragments straight from global memory (16 B per fragment), one
-//      64-wide group ahead, into registers - the rows are private to the wave, LDS would add nothing.
-//   B: wave w expands arena tile w of the next group to bf16(fma(q, scale, bias)) into the other half of
-//      a double-buffered LDS area while all waves multiply from the current half; one barrier per group.
+// Grouped GEMM. One block = one M-tile (up to 256 pairs of one expert) x one N-block (8 arena tiles = 256 weight rows), a wave
+// per arena tile: its 32 weight rows against all pairs of the tile.
+//   Weights: a lane's 16 bytes of an arena tile are its share of four matrix operands already, so they are expanded to
+//      bf16(fma(q, scale, bias)) register to register, an operand set ahead of the products, once per M-tile; the packed tiles go
+//      from memory straight into LDS, kRingW groups ahead.
+//   Pairs: a 64-wide group of their rows goes from memory straight into LDS as well (three buffers), and every wave reads each
+//      16-pair fragment once and multiplies it with its two row blocks.
+// One block of eight waves per compute unit walks a list of such items (prefill_gemm_kernel), the loads running on from one to the next.
+// What bounds it: 192 pairs per expert make 48 matrix instructions per wave and group, i.e. 1,536 cycles of a SIMD's matrix unit
+// of the 2,150 that a group takes; beside them 82 vector instructions (the expansion, 68 of them, shrinks with every pair a
+// wave multiplies its weights with), 26 LDS reads and one barrier. Run back to back the card also lowers its clock under it.
+// Weights through LDS instead (a wave expands a tile for all waves to read) costs the same however the waves split a block:
+// 215 to 235 us where this takes 183; 64 weight rows x 128 pairs per wave, every tile expanded twice, 209. Gate/up and down of a
+// 3,072-row chunk 222 + 115 -> 183 + 110 us, of 8,192 skewed rows 7.5 % less per layer, of 1,000 FP16 rows 144 + 78 -> 112 + 80; 256 pairs in each of 128
+// experts 275 + 133 -> 216 + 137 us (1,200 TFLOP/s in gate/up). A second pass of bf16 products by the vendor's library on ready-made
+// weights reaches 1,250 on this card.
 // GATE_UP: A rows are gathered token rows of x; streams are gate / up; out = the activations, stored in the order the
 //          down GEMM's matrix instructions want them (below).
-// else:    A = those activations, loaded straight into operand registers (1 KiB contiguous per wave and fragment, no
-//          cross-lane re-layout); streams are two 16-row blocks; out = partials[out_row][D] (16-bit).
+// else:    A = those activations; streams are two 16-row blocks; out = partials[out_row][D] (16-bit).
 // Activation layout: [16-pair block][group of F][k-half][lane (j, jq)] x 8 values = pair j of the block at
 // k = 32 * (k-half) + 8 * jq .. + 7 of the group. The 16-pair blocks of an M-tile start at block row_start / 16 + its number
 // in row order: consecutive tiles never share a block (a tile adds at most one block of slack), so the buffer holds
@@ -299,7 +305,6 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
 // ---------------------------------------------------------------------------------------------------
 
 struct GemmWave {
-    const uint8_t *w_tiles, *w_scales;    // this wave's arena tile row
     const uint16_t *a;                    // A matrix
     uint32_t a_stride, n_groups, n_arena_tiles, nb, wave, lane;
     uint32_t act_blocks;                  // 16-pair blocks the activation buffer holds (the scale tables' extent)
@@ -307,320 +312,358 @@ struct GemmWave {
     PrefillTile tile;
 };
 
-// The k-loop and epilogue of one wave that owns NMB 16-row blocks (a compile-time count: the MFMA
-// sequence has no branches, so the scheduler can interleave it with the expansion of the next tile).
-// DUMP: a test instantiation that also copies every weight fragment out of LDS, read exactly as the matrix
-// instructions read it, so that a test can hold the expanded tile itself against the reference's 16-bit weight.
+constexpr int kGemmTiles = 8;                               // arena tiles per N-block = waves per block
+constexpr int kRingA = 3, kRingW = 5;                       // groups of A, and of packed tiles at most, in LDS
+constexpr int kMaxLoads = kBM / 64;                         // KiB of A per wave and group, a whole M-tile
+constexpr uint32_t kFragBytes = kWave * 16;                 // one matrix operand of a wave
+constexpr uint32_t kGemmABytes = kBM / 16 * 2 * kFragBytes;
+constexpr uint32_t kGemmWBytes = kTileBytes + 2 * kTileScaleBytes;            // packed tile of one wave (a 64-lane load brings the scales twice)
+constexpr uint32_t kGemmWAt = kRingA * kGemmABytes, kGemmRowAt = kGemmWAt + kRingW * kGemmTiles * kGemmWBytes;
+// (down product: the pairs' output rows and largest scales, two items' worth, and the block scales of the groups of A)
+constexpr uint32_t kGemmRowBytes = kBM * 4, kGemmLargestAt = kGemmRowAt + 2 * kGemmRowBytes, kGemmRelAt = kGemmLargestAt + 2 * kGemmRowBytes;
+// the epilogues work in the buffer of the item's last group of A: the next item's first two are in the others
+constexpr int kTurnBlocks = 3;                              // 16-pair blocks that a wave turns at a time
+constexpr uint32_t kGemmTurnRow = 2 * kTileRows * 2 + 16, kGemmTurnBytes = 16 * kGemmTurnRow;
+static_assert(kGemmTiles * kTurnBlocks * kGemmTurnBytes <= kGemmABytes && kGemmTiles * kBM * 4 <= kGemmABytes, "staging rows or peaks fit a buffer");
+constexpr uint32_t gemm_lds_bytes(bool gate_up, bool f16) { return gate_up ? kGemmRowAt : f16 ? kGemmRelAt + kRingA * kGemmRowBytes : kGemmLargestAt; }
+
+// One M-tile x N-block, and what a wave needs to ask for its rows: `from` = GATE_UP: in bytes from the first row's start (WIDE, where
+// the rows span 4 GiB or more: in 16-byte pieces); else: in KiB, wave-uniform.
+struct GemmItem {
+    bool valid;
+    uint32_t parity;                      // of its number among the block's
+    PrefillTile tile;
+    uint32_t nb, act_block0, loads;
+    uint32_t from[kMaxLoads];
+    const uint8_t *w_tiles, *w_scales;    // this wave's arena tile
+};
+
+// How many fragments of A a wave has in flight or in use, `most` or fewer: a divisor of the 2 NM of a group, so that a fragment's
+// registers are known at compile time, and at most NM + 1, so that none of the next group is read in a group's first half.
+constexpr int gemm_queue(int nm, int most) {
+    if ((nm == 11 || nm == 13) && most > 4) return nm;
+    int q = 2;
+    for (int d = 3; d <= most; ++d)
+        if (2 * nm % d == 0 && d <= nm + 1) q = d;
+    return q;
+}
+
+// NM: 16-pair blocks of the tile, all of them this wave's (a compile-time count: the matrix instructions have no branches
+// between them); 0 for a wave past the last arena tile, which only brings its share of A. LOADS: KiB of A per wave and group.
+// DUMP: a test instantiation that also copies every weight operand out, so that a test can hold the expanded tile itself
+// against the reference's 16-bit weight.
 // F16: the reference's FP16 prefill (prefill.metal:581-598,685-702,723-777): FP16 rows against FP16 tile weights
 // half(fma(q, scale, bias)), fp32 sums; the activations between the two GEMMs are FP16 with a power-of-two scale per
 // pair and 64-wide block of F (`act_scale[pair][block]`; the block's largest magnitude lands below 2^14), so values
 // past FP16's range keep FP16's relative precision; the down GEMM brings every block of a pair to the pair's largest
 // scale as it takes it in (exact unless a value falls below FP16's normal range relative to that largest) and
 // applies that scale to the pair's sums.
-template <bool GATE_UP, int NMB, bool F16, bool DUMP = false>
-__device__ __forceinline__ void gemm_wave(const GemmWave &gw, const ArenaGeom &g, uint4 (*wb)[kTilesPerBlock][2][2][kWave],
-                                          const uint32_t *__restrict__ sorted_token,
-                                          const uint32_t *__restrict__ sorted_out_row, uint16_t *__restrict__ out,
-                                          float *__restrict__ act_scale, uint4 *__restrict__ dump = nullptr) {
-    constexpr int NA = NMB > 0 ? NMB : 1;
-    const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4;
-    const uint32_t n_groups = gw.n_groups;
-    const uint16_t *arow[NA];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-        if (!GATE_UP) {
-            // the activations are stored fragment by fragment: block, group, k-half, then 16 bytes per lane
-            arow[i] = gw.a + ((size_t)(gw.act_block0 + wave + 4 * i) * n_groups * 2) * (kWave * 8) + lane * 8;
-            continue;
-        }
-        // load layout: four neighbouring lanes read 64 contiguous bytes of one row (row lane / 4, 8-element
-        // chunk lane % 4), so a load touches 16 half-lines instead of 64 scattered 16-byte pieces
-        const uint32_t prow = min((wave + 4 * i) * 16 + (lane >> 2), gw.tile.rows - 1);
-        const uint32_t src = sorted_token[gw.tile.row_start + prow];
-        // rows 8..15 take their four chunks rotated by two: the lanes a half-wave then pulls from in the re-layout
-        // below fall on 32 different LDS banks (in natural order rows r and r + 8 collide on every bank)
-        arow[i] = gw.a + (size_t)src * gw.a_stride + 8 * (((lane & 3) - 2 * (lane >> 5)) & 3);
+// Where a wave is in the rings, as byte offsets into LDS: they turn on from one item to the next.
+struct GemmRings {
+    uint32_t cur, next, before;           // A of the group at hand, of the next one, of the one before (and of the group after the next)
+    uint32_t slot, first_slot, end_slot;  // this wave's packed tile of the group at hand; where its slots begin and end
+    uint32_t depth;                       // slots in use
+    __device__ __forceinline__ uint32_t next_slot() const {
+        const uint32_t s = slot + kGemmTiles * kGemmWBytes;
+        return s == end_slot ? first_slot : s;
     }
-    // MFMA layout: lane (j, jq) needs row j, chunk jq = what load-layout lane 4 j + ((jq + 2 (j / 8)) % 4) holds
-    const int pull = (int)((4 * j + ((jq + 2 * (j >> 3)) & 3)) * 4);
-    // FP16 down GEMM: the pair a lane holds in row block i (operand lane (j, jq) = pair j of the block), its largest
-    // block scale and the reciprocal (powers of two: exact)
-    // FP16: the block scales are laid out like the activations - act_scale[(16-pair block * groups of F + group) * 16 + j],
-    // pair j of the block - so a lane's address is a wave-uniform base plus 4 j. The down GEMM finds them already
-    // divided by the pair's largest (prefill_pair_scale_kernel ran in between: powers of two <= 1), and the largest
-    // itself in a second table behind the first, [block * 16 + j].
-    auto scale_at = [&](int i, uint32_t grp) { return ((size_t)(gw.act_block0 + wave + 4 * i) * g.gf + grp) * 16 + j; };
-    auto to_frag = [&](const uint4 &v, float rel) {
-        if (!GATE_UP) {                                           // already in operand order
-            if constexpr (!F16) return v;
-            const _Float16 r = (_Float16)rel;
-            const f16x2 r2 = {r, r};
-            uint4 o;
-            o.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.x) * r2);
-            o.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.y) * r2);
-            o.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.z) * r2);
-            o.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.w) * r2);
-            return o;
-        }
-        uint4 r;
-        r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.x);
-        r.y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.y);
-        r.z = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.z);
-        r.w = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w);
-        return r;
-    };
-    f32x4 acc[NA][2 * kTilesPerBlock];
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-#pragma unroll
-        for (int nf = 0; nf < 2 * kTilesPerBlock; ++nf) acc[i][nf] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __device__ __forceinline__ void turn() {
+        const uint32_t c = cur;
+        cur = next, next = before, before = c;
+        slot = next_slot();
+    }
+};
 
-    // this wave's packed tile of the next kSlots groups to expand, in flight: group g waits in slot g % kSlots
-    // (one slot where the row blocks leave no registers for a second: the steps are long enough there)
-    constexpr int kSlots = ((GATE_UP || F16) && NMB >= 4) ? 1 : 2;      // (the FP16 down GEMM carries the pairs' block scales besides)
-    uint4 wraw[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-    uint2 sraw[2] = {{0, 0}, {0, 0}};
-    auto load_b = [&](uint32_t grp, int slot) {
-        wraw[slot] = reinterpret_cast<const uint4 *>(gw.w_tiles + (size_t)grp * kTileBytes)[lane];
-        sraw[slot] = reinterpret_cast<const uint2 *>(gw.w_scales + (size_t)grp * kTileScaleBytes)[j];
-    };
-    // Expansion of the packed tile in `wcur` into wb[buf], cut into 16 pieces of about five VALU
-    // instructions (piece 4 c + q = output dword q of packed word c; the word's last piece stores it).
-    uint32_t wcur[4];
-    float sc[2], bi[2];
-    uint32_t lo = 0, hi = 0;
-    uint4 ex = {0, 0, 0, 0};
-    auto expand_begin = [&](int slot) {
-        wcur[0] = wraw[slot].x, wcur[1] = wraw[slot].y, wcur[2] = wraw[slot].z, wcur[3] = wraw[slot].w;
-        sc[0] = bf16lo_to_f32(sraw[slot].x), bi[0] = bf16hi_to_f32(sraw[slot].x);
-        sc[1] = bf16lo_to_f32(sraw[slot].y), bi[1] = bf16hi_to_f32(sraw[slot].y);
-    };
-    auto expand_piece = [&](int buf, int piece) {
-        const int c = piece >> 2, q = piece & 3;
-        const float s_ = sc[c >> 1], b_ = bi[c >> 1];
-        if (q == 0) {
-            // even / odd nibbles as bytes; the empty asm keeps the masks as written (one v_cvt_f32_ubyteN per byte)
-            lo = wcur[c] & 0x0F0F0F0Fu, hi = (wcur[c] >> 4) & 0x0F0F0F0Fu;
-            asm("" : "+v"(lo), "+v"(hi));
-            ex.x = Act<F16>::pack(__builtin_fmaf((float)(lo & 0xFFu), s_, b_), __builtin_fmaf((float)((lo >> 16) & 0xFFu), s_, b_));
-        } else if (q == 1) {
-            ex.y = Act<F16>::pack(__builtin_fmaf((float)(hi & 0xFFu), s_, b_), __builtin_fmaf((float)((hi >> 16) & 0xFFu), s_, b_));
-        } else if (q == 2) {
-            ex.z = Act<F16>::pack(__builtin_fmaf((float)((lo >> 8) & 0xFFu), s_, b_), __builtin_fmaf((float)(lo >> 24), s_, b_));
-        } else {
-            ex.w = Act<F16>::pack(__builtin_fmaf((float)((hi >> 8) & 0xFFu), s_, b_), __builtin_fmaf((float)(hi >> 24), s_, b_));
-            wb[buf][wave][c >> 1][c & 1][lane] = ex;
-        }
-    };
-    uint4 araw[NA][2];      // A in load layout, in flight: [.][0] k-half 0, [.][1] k-half 1
-    uint4 af[NA][2];        // A as MFMA fragments
-    float ablock[NA][2];    // FP16 down GEMM: the block scale of the group araw[.][half] belongs to
-    auto load_a = [&](uint32_t grp, int half) {
-        if (NMB == 0) return;
+// The loads of one group: the k-th KiB of a wave's share of A, its packed tile (k = 0) and that tile's scales (k = 1).
+template <bool GATE_UP, bool F16, bool WIDE>
+__device__ __forceinline__ void gemm_load_a(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, const float *__restrict__ act_scale,
+                                            uint32_t grp, uint32_t at, uint32_t rel_buf, int k) {
+    if (F16 && !GATE_UP && k == 0) {
+        // the scales of four 16-pair blocks (the second four waves repeat the first's, so that all count alike)
+        const uint32_t block = min(4 * (gw.wave & 3) + (gw.lane >> 4), (it.tile.rows - 1) / 16);
+        global_to_lds_4(act_scale + ((size_t)(it.act_block0 + block) * gw.n_groups + grp) * 16 + (gw.lane & 15),
+                        lds_base + kGemmRelAt + rel_buf * kGemmRowBytes + (gw.wave & 3) * (kWave * 4));
+    }
+    const uint32_t to = lds_base + at + (gw.wave + kGemmTiles * k) * kFragBytes;
+    if constexpr (GATE_UP && WIDE) global_to_lds_16(gw.a + grp * kGroup + (size_t)it.from[k] * 8, to);
+    else if constexpr (GATE_UP) global_to_lds_16(gw.a + grp * kGroup, it.from[k], to);
+    else global_to_lds_16(gw.a + ((size_t)it.from[k] + 2 * grp) * (kWave * 8), gw.lane * 16, to);
+}
+__device__ __forceinline__ void gemm_load_w(uint32_t lane, const uint8_t *w_tiles, const uint8_t *w_scales, uint32_t to, int k) {
+    if (k == 0) global_to_lds_16(w_tiles, lane * 16, to);
+    else global_to_lds_4(w_scales, lane * 4 % kTileScaleBytes, to + kTileBytes);
+}
+// what an item's first step counts on: two groups of A, as many packed tiles as the ring holds
+template <bool GATE_UP, bool F16, bool WIDE>
+__device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, const GemmRings &rings,
+                                         const float *__restrict__ act_scale) {
 #pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            araw[i][half] = GATE_UP ? *reinterpret_cast<const uint4 *>(arow[i] + grp * kGroup + 32 * half)
-                                    : *reinterpret_cast<const uint4 *>(arow[i] + (size_t)(grp * 2 + half) * (kWave * 8));
-            if constexpr (F16 && !GATE_UP) ablock[i][half] = act_scale[scale_at(i, grp)];
+    for (uint32_t grp = 0; grp < kRingW; ++grp) {
+        const bool live = grp < rings.depth;
+        const uint32_t to = lds_base + rings.first_slot + grp * kGemmTiles * kGemmWBytes;
+        if (live) {
+            gemm_load_w(gw.lane, it.w_tiles + grp * kTileBytes, it.w_scales + grp * kTileScaleBytes, to, 0);
+            gemm_load_w(gw.lane, it.w_tiles + grp * kTileBytes, it.w_scales + grp * kTileScaleBytes, to, 1);
+        }
+        if (grp < 2 && live) {
+#pragma unroll
+            for (int k = 0; k < kMaxLoads; ++k)
+                if ((uint32_t)k < it.loads)
+                    gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, act_scale, grp, grp ? rings.next : rings.cur, (grp ? rings.next : rings.cur) / kGemmABytes, k);
+        }
+    }
+}
+
+template <bool GATE_UP, int NM, int LOADS, bool F16, bool WIDE, bool DUMP>
+__device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it, const GemmItem &next_item, GemmRings &rings, const ArenaGeom &g,
+                                          uint8_t *__restrict__ lds, uint32_t lds_base, const uint32_t *__restrict__ sorted_out_row,
+                                          uint16_t *__restrict__ out, float *__restrict__ act_scale, uint4 *__restrict__ dump = nullptr) {
+    constexpr int NA = NM > 0 ? NM : 1;
+    constexpr int kQueue = gemm_queue(NA, F16 ? 4 : 8);     // (FP16 has the block scales and their products in registers besides)
+    constexpr bool kScaled = F16 && !GATE_UP;               // a pair's blocks come with scales of their own
+    const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4, n_groups = gw.n_groups;
+    const uint32_t tile = it.nb * kGemmTiles + wave;        // this wave's arena tile
+    if constexpr (!GATE_UP) {
+        // the pairs' output rows (and largest scales), for the epilogue; waves 4.. repeat what waves 0..3 bring
+        const uint32_t pair = min((wave & 3) * kWave + lane, it.tile.rows - 1);
+        global_to_lds_4(sorted_out_row + it.tile.row_start + pair, lds_base + kGemmRowAt + it.parity * kGemmRowBytes + (wave & 3) * (kWave * 4));
+        if constexpr (F16)
+            global_to_lds_4(act_scale + (size_t)gw.act_blocks * g.gf * 16 + it.act_block0 * 16 + pair, lds_base + kGemmLargestAt + it.parity * kGemmRowBytes + (wave & 3) * (kWave * 4));
+    }
+    uint4 wraw = {0, 0, 0, 0};
+    uint2 sraw = {0, 0};
+    auto read_w = [&](uint32_t slot) __attribute__((always_inline)) {
+        const uint8_t *at = lds + slot;
+        wraw = *reinterpret_cast<const uint4 *>(at + lane * 16);
+        sraw = *reinterpret_cast<const uint2 *>(at + kTileBytes + j * 8);
+    };
+    // Expansion: bits 0..3 and 4..7 of each half of a dword are FP16 subnormals q 2^-24 and q 2^-20 as they lie, and one
+    // v_fma_mix_f32 takes such a half with fp32 scale (times 2^24, 2^20: exact) and bias: 17 vector instructions for eight
+    // weights instead of 23 with byte conversions, the same fp32 value to the bit.
+    float s24[2], s20[2], bias[2];
+    auto take_scales = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const uint32_t sb = st ? sraw.y : sraw.x;
+            s24[st] = bf16lo_to_f32(sb) * 16777216.0f;
+            s20[st] = bf16lo_to_f32(sb) * 1048576.0f;
+            bias[st] = bf16hi_to_f32(sb);
         }
     };
-    auto frag_a = [&](int half) {
-        if (NMB == 0) return;
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            float rel = 1.0f;
-            if constexpr (F16 && !GATE_UP) rel = ablock[i][half];
-            af[i][half] = to_frag(araw[i][half], rel);
-        }
+    uint4 wf[2][2];                     // operands: k-half, stream
+    auto expand_piece = [&](int half, int piece) __attribute__((always_inline)) {
+        // half of a dword: two packed pairs at a time, so that the conversion of one stands behind the products of the other
+        const int st = piece >> 1;
+        const uint32_t w = st ? (half ? wraw.w : wraw.z) : (half ? wraw.y : wraw.x), b = piece & 1 ? w >> 8 : w;
+        const f16x2 u = __builtin_bit_cast(f16x2, b & 0x000F000Fu), v = __builtin_bit_cast(f16x2, b & 0x00F000F0u);
+        const float u0 = __builtin_fmaf((float)u[0], s24[st], bias[st]), u1 = __builtin_fmaf((float)u[1], s24[st], bias[st]);
+        const float v0 = __builtin_fmaf((float)v[0], s20[st], bias[st]), v1 = __builtin_fmaf((float)v[1], s20[st], bias[st]);
+        uint32_t lo = Act<F16>::pack(u0, u1), hi = Act<F16>::pack(v0, v1);
+        asm volatile("" : "+v"(lo), "+v"(hi));     // here, among the products, and not where the operand is first used
+        if (piece & 1) wf[half][st].z = lo, wf[half][st].w = hi;
+        else wf[half][st].x = lo, wf[half][st].y = hi;
     };
-    // One 64-wide group = 16 units; unit u multiplies weight fragment (nf = u % 8, k-half u / 8) with the NA
-    // row blocks, and is followed by one piece of the next group's expansion, so the matrix pipe and the
-    // VALU run side by side inside the wave (a scheduling fence after every unit keeps the order as
-    // written). On entry: af[.][0] = k-half 0 of this group; araw[.][1] = its k-half 1 in load layout;
-    // araw[.][0] = k-half 0 of the next group in flight; wraw/sraw[grp % kSlots] = packed tile of the group after next
-    // (it is expanded during this step, and its slot is reloaded at once with the group kSlots further on: with
-    // two slots a packed tile has two steps to arrive); wb[buf] = expanded tiles of this group, the next group's are
-    // there as well. The k-half 1 fragments are made at the start of the
-    // step and the next k-half 0 fragments in its middle, each as soon as the registers they replace have
-    // had their last use, with 8 units of MFMAs to cover the cross-lane latency; every register that a
-    // conversion frees is reloaded at once for the following group. Loads past the last group run on clamped
-    // indices and are never used: with no branch around them the compiler counts the loads in flight exactly.
-    // The last two steps are a second instantiation without the expansion (their groups are in LDS already).
-    // The expanded tiles sit in four LDS buffers (group g in buffer g % 4) and the expansion runs two groups ahead of the products, so one barrier per PAIR of groups orders both
-    // the first read of a buffer behind its last write and its next write behind its last read.
-    auto step = [&](uint32_t grp, auto expand_ahead, auto parity) {
-        constexpr bool kExpand = decltype(expand_ahead)::value;     // false in the last two steps: nothing is left to expand
-        constexpr int kSlot = decltype(parity)::value;              // grp % 2, known at compile time: the slots are registers
-        const int buf = grp & 3;
-        frag_a(1);
-        load_a(min(grp + 1, n_groups - 1), 1);
-        if (kExpand) {
-            expand_begin(kSlot % kSlots);                           // group grp + 2
-            load_b(min(grp + 2 + kSlots, n_groups - 1), kSlot % kSlots);
-        }
-        uint4 bq[3];
-        auto read_b = [&](int u) { bq[u % 3] = wb[buf][(u & 7) >> 1][u & 1][u >> 3][lane]; };
-        if (DUMP && wave == 0) {
-            // fragment u of group grp of this N-block, as unit u of the loop below receives it
+
+    f32x4 acc[NA][2];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                read_b(u);
-                dump[(((size_t)gw.nb * n_groups + grp) * 16 + u) * kWave + lane] = bq[u % 3];
-            }
-        }
-        if (NMB > 0) {
-            read_b(0);
-            read_b(1);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < NA; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 xq[kQueue];
+    uint32_t rq[kQueue];
+    // fragment f (k-half f / NM of 16-pair block f % NM) of a group
+    const uint32_t at0 = GATE_UP ? j * 128 + 16 * (jq ^ (j & 7)) : lane * 16;
+    auto read_a = [&](uint32_t from, int f) __attribute__((always_inline)) {
+        const int half = f / NA, i = f % NA;
+        const uint32_t at = GATE_UP ? at0 ^ (64 * half) : at0 + half * kFragBytes;
+        xq[f % kQueue] = *reinterpret_cast<const uint4 *>(lds + from + i * (2 * kFragBytes) + at);
+        if constexpr (kScaled) rq[f % kQueue] = *reinterpret_cast<const uint32_t *>(lds + kGemmRelAt + (from / kGemmABytes) * kGemmRowBytes + (i * 16 + j) * 4);
+    };
+    // One step = one group, its k-halves one after the other: the products with the four pieces of the next operand set's
+    // expansion between them (a scheduling fence behind each product keeps them there) and the fragments of A kQueue - 1 ahead.
+    // In its middle the next group's A, asked for in the step before, has to be there, and a barrier makes it the whole block's; the
+    // last fragments' reads then run ahead into that group, and the buffer of the group before is filled again.
+    // What a step asks for goes out between its products: all at once, the waves queue for the address unit (11 ns per KiB of
+    // rows) in front of their products. Behind an item's last group comes the next item's first, so that its packed tiles and, in
+    // the last two steps, its A are on their way before this one ends; without a next item the packed tiles of this one once more.
+    const bool run_on = next_item.valid && n_groups > 1;
+    const uint8_t *const next_w_tiles = next_item.valid ? next_item.w_tiles : it.w_tiles, *const next_w_scales = next_item.valid ? next_item.w_scales : it.w_scales;
+    uint32_t own_w = n_groups - rings.depth;                        // groups of this item whose packed tiles are still to be asked for
+    const uint8_t *ask_tiles = own_w ? it.w_tiles + rings.depth * kTileBytes : next_w_tiles;
+    const uint8_t *ask_scales = own_w ? it.w_scales + rings.depth * kTileScaleBytes : next_w_scales;
+    auto step = [&](uint32_t grp, auto is_steady) __attribute__((always_inline)) {
+        constexpr bool kSteady = decltype(is_steady)::value;        // not one of the last two: A is this item's, and no branches
+        constexpr int kUnits = 2 * NA;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            if (NMB > 0) {
-                if (u + 2 < 16) read_b(u + 2);
-#pragma unroll
-                for (int i = 0; i < NA; ++i)
-                    // weights as the first operand: the lane ends up with four consecutive weight rows of
-                    // one pair, which the epilogue packs into one 8-byte piece of that pair's output row
-                    acc[i][u & 7] = Act<F16>::mfma(bq[u % 3], af[i][u >> 3], acc[i][u & 7]);
-            }
-            if (kExpand) expand_piece((buf + 2) & 3, u);
-            __builtin_amdgcn_sched_barrier(0);
-            if (u == 7) {
-                frag_a(0);
-                load_a(min(grp + 2, n_groups - 1), 0);
+        for (int half = 0; half < 2; ++half) {
+            if (half == 1) {
+                if (DUMP) vmem_barrier<0>();
+                else if (kSteady || run_on) vmem_barrier<2>();      // (the packed tile asked for in the first half)
+                else vmem_barrier<0>();
+                if (NM > 0) read_w(rings.next_slot());
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (DUMP && NM > 0) {
+#pragma unroll
+                for (int st = 0; st < 2; ++st)
+                    dump[(((size_t)(tile / kTilesPerBlock) * n_groups + grp) * 16 + half * 8 + tile % kTilesPerBlock * 2 + st) * kWave + lane] = wf[half][st];
+            }
+            constexpr int kFirst = NA > 2 ? 4 : 0;
+            const int first = half == 1 ? kFirst : 0;               // (the packed tile is on its way from LDS)
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                const int f = half * NM + i, ahead = f + kQueue - 1;
+                uint4 x = {0, 0, 0, 0};
+                if (NM > 0) {
+                    if (ahead < 2 * NM) read_a(rings.cur, ahead);
+                    else read_a(rings.next, ahead - 2 * NM);
+                    x = xq[f % kQueue];
+                    if constexpr (kScaled) {
+                        const f16x2 r2 = __builtin_bit_cast(f16x2, rq[f % kQueue]);
+                        x.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.x) * r2);
+                        x.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.y) * r2);
+                        x.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.z) * r2);
+                        x.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.w) * r2);
+                    }
+                }
+#pragma unroll
+                for (int st = 0; st < 2; ++st) {
+                    // weights as the first operand: the lane ends up with four consecutive weight rows of
+                    // one pair, which the epilogue packs into one 8-byte piece of that pair's output row
+                    if (NM > 0) acc[i][st] = Act<F16>::mfma(wf[half][st], x, acc[i][st]);
+                    const int at = 2 * i + st, u = at - first;
+                    if (half == 1 && kSteady) {
+#pragma unroll
+                        for (int k = 0; k < LOADS; ++k)
+                            if (at == max((k + 1) * kUnits / (LOADS + 1) - 1, 0)) gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, act_scale, grp + 2, rings.before, rings.before / kGemmABytes, k);
+                    } else if (half == 1) {
+#pragma unroll
+                        for (int k = 0; k < kMaxLoads; ++k)
+                            if (at == max((k + 1) * kUnits / (kMaxLoads + 1) - 1, 0) && run_on && (uint32_t)k < next_item.loads)
+                                gemm_load_a<GATE_UP, F16, WIDE>(gw, next_item, lds_base, act_scale, grp + 2 - n_groups, rings.before, rings.before / kGemmABytes, k);
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 2; ++k)
+                            if (at == max((k + 1) * kUnits / 3 - 1, 0) && (kSteady || run_on))     // (this group's went to registers in the step before)
+                                gemm_load_w(lane, ask_tiles, ask_scales, lds_base + rings.slot, k);
+                    }
+                    if (NM > 0) {
+                        if (half == 1 && u == 0) take_scales();
+#pragma unroll
+                        for (int p = max(u, 0) * 4 / (kUnits - first); p < max(u + 1, 0) * 4 / (kUnits - first); ++p) expand_piece(half ^ 1, p);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
         }
-        // one barrier per pair of groups: the expansion runs two groups ahead (the tail steps, which use no slot,
-        // are one instantiation and look at the group's parity itself)
-        if (kExpand && kSlots == 2 ? kSlot != 0 : (grp & 1) != 0) lds_barrier();
     };
-    using Ahead = std::integral_constant<bool, true>;
-    using Tail = std::integral_constant<bool, false>;
-    using Even = std::integral_constant<int, 0>;
-    using Odd = std::integral_constant<int, 1>;
-
-    load_b(0, 0);
-    if (kSlots == 2) load_b(min(1u, n_groups - 1), 1);
-    load_a(0, 0);
-    load_a(0, 1);
-    expand_begin(0);
-    load_b(min((uint32_t)kSlots, n_groups - 1), 0);
+    if (NM > 0) {
+        read_w(rings.slot);
+        take_scales();
 #pragma unroll
-    for (int piece = 0; piece < 16; ++piece) expand_piece(0, piece);
-    expand_begin(1 % kSlots);
-    load_b(min(1u + kSlots, n_groups - 1), 1 % kSlots);
+        for (int p = 0; p < 4; ++p) expand_piece(0, p);
 #pragma unroll
-    for (int piece = 0; piece < 16; ++piece) expand_piece(1, piece);
-    frag_a(0);
-    load_a(min(1u, n_groups - 1), 0);
-    lds_barrier();
-    // steps in pairs (the slot of a group's packed tile and the barrier follow the group's parity); the last two
-    // steps multiply only: their groups were expanded two steps earlier
-    const uint32_t n_ahead = n_groups > 2 ? n_groups - 2 : 0;
-    uint32_t grp = 0;
-    if constexpr (kSlots == 2) {
-        for (; grp + 2 <= n_ahead; grp += 2) {
-            step(grp, Ahead{}, Even{});
-            step(grp + 1, Ahead{}, Odd{});
-        }
-        if (grp < n_ahead) {             // an odd number of groups: one more expanding step
-            step(grp, Ahead{}, Even{});
-            ++grp;
-        }
-    } else {
-        for (; grp < n_ahead; ++grp) step(grp, Ahead{}, Even{});
+        for (int f = 0; f < kQueue - 1; ++f) read_a(rings.cur, f);
     }
-    for (; grp < n_groups; ++grp) step(grp, Tail{}, Even{});
-    if (n_groups & 1) lds_barrier();     // the last pair was half a pair
-    if (NMB == 0) return;
+    auto turn_rings = [&]() __attribute__((always_inline)) {
+        rings.turn();
+        ask_tiles += kTileBytes;
+        ask_scales += kTileScaleBytes;
+        if (--own_w == 0) ask_tiles = next_w_tiles, ask_scales = next_w_scales;
+    };
+    uint32_t grp = 0;
+#pragma nounroll
+    for (; grp + 2 < n_groups; ++grp) {
+        step(grp, std::true_type{});
+        turn_rings();
+    }
+#pragma nounroll
+    for (; grp < n_groups; ++grp) {
+        step(grp, std::false_type{});
+        turn_rings();
+    }
+    lds_barrier();                      // nobody reads the last group's A any more
+    uint8_t *const stage = lds + rings.before;
+    if (n_groups == 1 && next_item.valid) gemm_ask<GATE_UP, F16, WIDE>(gw, next_item, lds_base, rings, act_scale);
 
-    // epilogue: lane (j, jq) holds pair 16 (w + 4 i) + j, weight rows 4 jq .. 4 jq + 3 of every fragment
-    if (GATE_UP) {
+    // epilogue: lane (j, jq) holds pair j of every 16-pair block, weight rows 4 jq .. 4 jq + 3 of both row blocks
+    if constexpr (GATE_UP) {
+        // this wave's arena tile is k = 16 (tile % 4) .. + 15 of group tile / 4 of F: k-half tile / 2 % 2, operand lane
+        // (j, 2 (tile % 2) + jq / 2), values 4 (jq % 2) .. + 3 of that lane's eight
 #pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            const uint32_t prow = (wave + 4 * i) * 16 + j;
-            if (prow >= gw.tile.rows) continue;
-            // this N-block is group nb of F (four arena tiles = 64 activations); arena tile tl holds k = 16 tl .. + 15
-            // of it, this lane the four values from k = 16 tl + 4 jq: k-half tl / 2, operand lane (j, 2 (tl % 2) + jq / 2),
-            // values 4 (jq % 2) .. + 3 of that lane's eight
-            uint16_t *oblk = out + ((size_t)(gw.act_block0 + wave + 4 * i) * g.gf + gw.nb) * 2 * (kWave * 8);
-            float h[kTilesPerBlock][4];
+        for (int i = 0; i < NA; ++i)
 #pragma unroll
-            for (int tl = 0; tl < kTilesPerBlock; ++tl)
+            for (int r = 0; r < 4; ++r) acc[i][0][r] = gelu_tanh_fast(acc[i][0][r]) * acc[i][1][r];
+        if constexpr (F16) {
+            // a pair's 64 activations of a group sit in the four lanes (j, 0..3) of four waves: their largest magnitude
+            // peak < 2^e goes to 2^14 (frexp / ldexp as prefill.metal:689-702)
+            float *peaks = reinterpret_cast<float *>(stage);                // [wave][pair]
 #pragma unroll
-                for (int r = 0; r < 4; ++r) h[tl][r] = gelu_tanh_fast(acc[i][2 * tl][r]) * acc[i][2 * tl + 1][r];
-            if constexpr (F16) {
-                // the pair's 64 activations of this block sit in the four lanes (j, 0..3), sixteen each: their
-                // largest magnitude peak < 2^e goes to 2^14 (frexp / ldexp as prefill.metal:689-702)
+            for (int i = 0; i < NM; ++i) {
                 float peak = 0.0f;
 #pragma unroll
-                for (int tl = 0; tl < kTilesPerBlock; ++tl)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) peak = fmaxf(peak, fabsf(h[tl][r]));
+                for (int r = 0; r < 4; ++r) peak = fmaxf(peak, fabsf(acc[i][0][r]));
                 peak = fmaxf(peak, __shfl_xor(peak, 16, 64));
                 peak = fmaxf(peak, __shfl_xor(peak, 32, 64));
+                if (jq == 0) peaks[wave * (16 * NM) + 16 * i + j] = peak;
+            }
+            lds_barrier();
+#pragma unroll
+            for (int i = 0; i < NM; ++i) {
+                float peak = 0.0f;
+#pragma unroll
+                for (uint32_t v = 0; v < 4; ++v) peak = fmaxf(peak, peaks[((wave & 4) + v) * (16 * NM) + 16 * i + j]);
                 int e = 0;
                 (void)frexpf(peak, &e);
                 e = max(e, -100);                                   // 2^(14 - e) stays finite for a block of denormal size
                 const float to_half = ldexpf(1.0f, 14 - e);
 #pragma unroll
-                for (int tl = 0; tl < kTilesPerBlock; ++tl)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) h[tl][r] *= to_half;
-                if (jq == 0) act_scale[scale_at(i, gw.nb)] = ldexpf(1.0f, e - 14);
+                for (int r = 0; r < 4; ++r) acc[i][0][r] *= to_half;
+                if (jq == 0 && (wave & 3) == 0 && 16 * i + j < it.tile.rows)
+                    act_scale[((size_t)(it.act_block0 + i) * g.gf + tile / kTilesPerBlock) * 16 + j] = ldexpf(1.0f, e - 14);
             }
+        }
 #pragma unroll
-            for (int tl = 0; tl < kTilesPerBlock; ++tl) {
-                uint16_t *dst = oblk + (tl >> 1) * (kWave * 8) + (((tl & 1) * 2 + (jq >> 1)) * 16 + j) * 8 + (jq & 1) * 4;
-                *reinterpret_cast<uint2 *>(dst) = make_uint2(Act<F16>::pack(h[tl][0], h[tl][1]), Act<F16>::pack(h[tl][2], h[tl][3]));
-            }
+        for (int i = 0; i < NM; ++i) {
+            if (16 * i + j >= it.tile.rows) continue;
+            uint16_t *oblk = out + (((size_t)(it.act_block0 + i) * g.gf + tile / kTilesPerBlock) * 2 + (tile >> 1 & 1)) * (kWave * 8);
+            *reinterpret_cast<uint2 *>(oblk + (((tile & 1) * 2 + (jq >> 1)) * 16 + j) * 8 + (jq & 1) * 4) =
+                make_uint2(Act<F16>::pack(acc[i][0][0], acc[i][0][1]), Act<F16>::pack(acc[i][0][2], acc[i][0][3]));
         }
         return;
     }
-    // Down projection: a 16-pair block of this N-block is 16 rows x 256 B. Each wave turns its blocks
-    // through a private LDS area (the weight buffers are free: the last step ended with a barrier) so that
-    // 16 lanes store one row's 256 contiguous bytes, instead of 8-byte pieces 32 B apart per instruction.
-    constexpr uint32_t kStageRow = 2 * kTilesPerBlock * kTileRows * 2 + 16;     // bytes: 128 columns + padding
-    static_assert(4 * 16 * kStageRow <= sizeof(uint4) * 4 * kTilesPerBlock * 2 * 2 * kWave, "staging fits the weight buffers");
-    uint8_t *stage = reinterpret_cast<uint8_t *>(wb) + wave * 16 * kStageRow;
-    const uint32_t rsub = lane >> 4, chunk = lane & 15;                         // read side: row 4 p + rsub, columns 8 chunk ..
-    const bool col_ok = gw.nb * kTilesPerBlock + (chunk >> 2) < gw.n_arena_tiles;
-    float pair_largest[NA];
-    if constexpr (F16) {
+    // Down projection: a 16-pair block of this wave's columns is 16 rows x 64 B. Each wave turns its blocks through a private piece
+    // of LDS, so that four lanes store 64 contiguous bytes of a row, instead of 8-byte pieces 32 B apart per instruction.
+    uint8_t *turn = stage + wave * (kTurnBlocks * kGemmTurnBytes);
+    const uint32_t row = lane >> 2, chunk = lane & 3;                           // read side
 #pragma unroll
-        for (int i = 0; i < NA; ++i) pair_largest[i] = act_scale[(size_t)gw.act_blocks * g.gf * 16 + (gw.act_block0 + wave + 4 * i) * 16 + j];
-    }
-    uint32_t orow_idx[NA][4];
+    for (int i0 = 0; i0 < NM; i0 += kTurnBlocks) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i)
+        for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i) {
+            float pair_largest = 1.0f;
+            if constexpr (F16) pair_largest = *reinterpret_cast<const float *>(lds + kGemmLargestAt + it.parity * kGemmRowBytes + (16 * i + j) * 4);
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint32_t prow = (wave + 4 * i) * 16 + 4 * p + rsub;
-            orow_idx[i][p] = sorted_out_row[gw.tile.row_start + min(prow, gw.tile.rows - 1)];
-        }
+            for (int st = 0; st < 2; ++st) {
+                f32x4 v = acc[i][st];
+                if constexpr (F16) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-#pragma unroll
-        for (int nf = 0; nf < 2 * kTilesPerBlock; ++nf) {
-            f32x4 v = acc[i][nf];
-            if constexpr (F16) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] *= pair_largest[i];      // the pair's sums back to their scale
+                    for (int r = 0; r < 4; ++r) v[r] *= pair_largest;         // the pair's sums back to their scale
+                }
+                *reinterpret_cast<uint2 *>(turn + (i - i0) * kGemmTurnBytes + j * kGemmTurnRow + st * 32 + 8 * jq) =
+                    make_uint2(Act<F16>::pack(v[0], v[1]), Act<F16>::pack(v[2], v[3]));
             }
-            *reinterpret_cast<uint2 *>(stage + j * kStageRow + nf * 32 + 8 * jq) =
-                make_uint2(Act<F16>::pack(v[0], v[1]), Act<F16>::pack(v[2], v[3]));
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint4 v[kTurnBlocks];
+        uint32_t orow[kTurnBlocks];
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint32_t row = 4 * p + rsub, prow = (wave + 4 * i) * 16 + row;
-            const uint4 v = *reinterpret_cast<const uint4 *>(stage + row * kStageRow + 16 * chunk);
-            if (prow < gw.tile.rows && col_ok)
-                *reinterpret_cast<uint4 *>(out + (size_t)orow_idx[i][p] * g.d + gw.nb * (2 * kTilesPerBlock * kTileRows) + 8 * chunk) = v;
+        for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i) {
+            v[i - i0] = *reinterpret_cast<const uint4 *>(turn + (i - i0) * kGemmTurnBytes + row * kGemmTurnRow + 16 * chunk);
+            orow[i - i0] = *reinterpret_cast<const uint32_t *>(lds + kGemmRowAt + it.parity * kGemmRowBytes + (16 * i + row) * 4);
         }
+#pragma unroll
+        for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i)
+            if (16 * i + row < it.tile.rows) *reinterpret_cast<uint4 *>(out + (size_t)orow[i - i0] * g.d + tile * (2 * kTileRows) + 8 * chunk) = v[i - i0];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -644,51 +687,138 @@ __device__ __forceinline__ bool prefill_block(uint32_t n_nblocks, bool nb_major,
 }
 
 // F16: a context in FP16 mode - FP16 rows in, FP16 tiles, block-scaled FP16 activations, FP16 per-route rows out
-template <bool GATE_UP, bool F16 = false, bool DUMP = false>
-__global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
-                                                              const PrefillPlan *__restrict__ plan,
-                                                              const PrefillTile *__restrict__ tiles,
-                                                              const uint32_t *__restrict__ sorted_token,
-                                                              const uint32_t *__restrict__ sorted_out_row,
-                                                              const uint16_t *__restrict__ a, uint32_t a_stride,
-                                                              uint16_t *__restrict__ out, uint32_t n_nblocks,
-                                                              bool nb_major, float *__restrict__ act_scale, uint32_t act_blocks,
-                                                              uint4 *__restrict__ dump = nullptr) {
-    __shared__ __align__(16) uint4 wb[4][kTilesPerBlock][2][2][kWave];   // [buffer][tile][stream][k-half][lane]: group g lives in buffer g % 4
-
-    uint32_t ti, nb;
-    if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;
+// A block per compute unit, which works off its share of the XCD's items one after the other: an item's first loads then travel
+// during the epilogue of the one before.
+template <bool GATE_UP, bool F16 = false, bool WIDE = false, bool DUMP = false>
+__global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
+                                                                          const PrefillPlan *__restrict__ plan,
+                                                                          const PrefillTile *__restrict__ tiles,
+                                                                          const uint32_t *__restrict__ sorted_token,
+                                                                          const uint32_t *__restrict__ sorted_out_row,
+                                                                          const uint16_t *__restrict__ a, uint32_t a_stride,
+                                                                          uint16_t *__restrict__ out, bool nb_major,
+                                                                          float *__restrict__ act_scale, uint32_t act_blocks,
+                                                                          uint4 *__restrict__ dump = nullptr) {
+    __shared__ __align__(16) uint8_t lds[gemm_lds_bytes(GATE_UP, F16)];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     GemmWave gw;
-    gw.tile = tiles[ti];
     gw.lane = threadIdx.x & 63;
     gw.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // wave-uniform: branches on it stay scalar
     gw.n_groups = GATE_UP ? g.gd : g.gf;
     gw.n_arena_tiles = GATE_UP ? g.gu_rb : g.dn_rbp;
-    gw.nb = nb;
     gw.a = a;
     gw.a_stride = a_stride;
-    gw.act_block0 = gw.tile.row_start / 16 + gw.tile.order;
     gw.act_blocks = act_blocks;
-    // the arena tile row this wave expands; past the last one it expands the last again (never stored)
-    const uint32_t at = min(nb * kTilesPerBlock + gw.wave, gw.n_arena_tiles - 1);
-    const uint8_t *expert_base = arena_layer + (size_t)gw.tile.expert * g.expert_bytes;
-    gw.w_tiles = expert_base + (GATE_UP ? g.gu_tiles_off : g.dn_tiles_off) + (size_t)at * gw.n_groups * kTileBytes;
-    gw.w_scales = expert_base + (GATE_UP ? g.gu_scales_off : g.dn_scales_off) + (size_t)at * gw.n_groups * kTileScaleBytes;
 
-    const uint32_t n_mb = (gw.tile.rows + 15) / 16;
-    const uint32_t my_mb = n_mb > gw.wave ? (n_mb - gw.wave + 3) / 4 : 0;    // 16-row blocks of this wave
-    if (DUMP) {
-        // the test launch runs one pair: wave 0 owns its row block, the others only expand their tiles
-        if (my_mb) gemm_wave<GATE_UP, 1, F16, true>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale, dump);
-        else gemm_wave<GATE_UP, 0, F16, true>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale, dump);
-        return;
-    }
-    switch (my_mb) {
-        case 0: gemm_wave<GATE_UP, 0, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
-        case 1: gemm_wave<GATE_UP, 1, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
-        case 2: gemm_wave<GATE_UP, 2, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
-        case 3: gemm_wave<GATE_UP, 3, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
-        default: gemm_wave<GATE_UP, 4, F16>(gw, g, wb, sorted_token, sorted_out_row, out, act_scale); break;
+    // The XCD's items, largest first: full N-blocks tile by tile, then the tiles' last N-blocks where those are not full, then its
+    // share of the tiles that do not make up a set of eight.
+    // Many experts: an M-tile's items are all on one XCD (its L2 holds the tile's A rows), tile t on XCD t % 8, but for the last few. One
+    // expert (the dense FFN: few M-tiles, every one against the same weights): the N-blocks one after the other, an eighth of the
+    // list per XCD, so that each reads its eighth of the weights once.
+    const uint32_t xcd = blockIdx.x & 7, mine = blockIdx.x >> 3, per_xcd = gridDim.x >> 3;
+    const uint32_t n_tiles = plan->n_tiles, n_full = gw.n_arena_tiles / kGemmTiles, n_nb = (gw.n_arena_tiles + kGemmTiles - 1) / kGemmTiles;
+    const uint32_t all = n_tiles * n_nb, tiles_x = n_tiles / 8, over = n_tiles % 8 * n_nb;
+    const uint32_t first = nb_major ? (uint32_t)((uint64_t)all * xcd / 8) : 0;
+    const uint32_t n_items = nb_major ? (uint32_t)((uint64_t)all * (xcd + 1) / 8) - first : tiles_x * n_nb + (over + 7 - xcd) / 8;
+    // round r of this block: the rounds run forth and back over the blocks, so that who had a large item gets a small one
+    auto item_at = [&](uint32_t r) __attribute__((always_inline)) {
+        GemmItem it;
+        const uint32_t q = r * per_xcd + (r & 1 ? per_xcd - 1 - mine : mine);
+        it.valid = q < n_items;
+        it.parity = r & 1;
+        if (!it.valid) return it;
+        uint32_t ti;
+        if (nb_major) {
+            ti = (first + q) % n_tiles;
+            it.nb = (first + q) / n_tiles;
+        } else if (q < tiles_x * n_full) {
+            ti = q / n_full * 8 + xcd;
+            it.nb = q % n_full;
+        } else if (q < tiles_x * n_nb) {
+            ti = (q - tiles_x * n_full) * 8 + xcd;
+            it.nb = n_full;
+        } else {
+            const uint32_t o = (q - tiles_x * n_nb) * 8 + xcd;
+            ti = tiles_x * 8 + o / n_nb;
+            it.nb = o % n_nb;
+        }
+        ti = __builtin_amdgcn_readfirstlane(ti);
+        it.nb = __builtin_amdgcn_readfirstlane(it.nb);
+        it.tile = tiles[ti];
+        it.tile.rows = __builtin_amdgcn_readfirstlane(it.tile.rows);
+        it.act_block0 = it.tile.row_start / 16 + it.tile.order;
+        const uint32_t last_block = (it.tile.rows - 1) / 16;
+        it.loads = last_block / 4 + 1;
+        // A to LDS, 1 KiB at a time. GATE_UP: eight rows of 128 bytes, eight neighbouring lanes per row; 16-byte piece c of row r lies
+        // at piece c ^ (r % 8) of the row, so that the sixteen rows of a fragment read fall on different banks. else: the
+        // activations are stored fragment by fragment.
+#pragma unroll
+        for (int k = 0; k < kMaxLoads; ++k) {
+            const uint32_t piece = gw.wave + kGemmTiles * k;
+            if constexpr (GATE_UP) {
+                const uint32_t row = min(piece * 8 + (gw.lane >> 3), it.tile.rows - 1);
+                it.from[k] = (sorted_token[it.tile.row_start + row] * (gw.a_stride / 8) + ((gw.lane & 7) ^ (gw.lane >> 3))) * (WIDE ? 1u : 16u);
+            } else {
+                it.from[k] = __builtin_amdgcn_readfirstlane((it.act_block0 + min(piece >> 1, last_block)) * gw.n_groups * 2 + (piece & 1));
+            }
+        }
+        // this wave's arena tile; past the last one the last again (read and left at that)
+        const uint32_t at = min(it.nb * kGemmTiles + gw.wave, gw.n_arena_tiles - 1) * gw.n_groups;
+        const uint8_t *expert_base = arena_layer + (size_t)__builtin_amdgcn_readfirstlane(it.tile.expert) * g.expert_bytes;
+        it.w_tiles = expert_base + (GATE_UP ? g.gu_tiles_off : g.dn_tiles_off) + (size_t)at * kTileBytes;
+        it.w_scales = expert_base + (GATE_UP ? g.gu_scales_off : g.dn_scales_off) + (size_t)at * kTileScaleBytes;
+        return it;
+    };
+    GemmItem it = item_at(0);
+    if (!it.valid) return;
+    GemmRings rings;
+    rings.depth = min((uint32_t)kRingW, gw.n_groups);
+    rings.cur = 0, rings.next = kGemmABytes, rings.before = 2 * kGemmABytes;
+    rings.slot = rings.first_slot = kGemmWAt + gw.wave * kGemmWBytes;
+    rings.end_slot = rings.first_slot + rings.depth * (kGemmTiles * kGemmWBytes);
+    gemm_ask<GATE_UP, F16, WIDE>(gw, it, lds_base, rings, act_scale);
+    vmem_barrier<0>();
+    for (uint32_t r = 1;; ++r) {
+        const GemmItem next = item_at(r);
+        const uint32_t n_mb = (it.tile.rows + 15) / 16;
+        const bool owns = it.nb * kGemmTiles + gw.wave < gw.n_arena_tiles;
+        // (waves that own no tile take part in the loads and the barriers, which are the same in all instantiations of one LOADS)
+#define FFMOE_GEMM_WAVE(N, L) gemm_wave<GATE_UP, N, L, F16, WIDE, DUMP>(gw, it, next, rings, g, lds, lds_base, sorted_out_row, out, act_scale, dump)
+        if constexpr (DUMP) {
+            // the test launch runs one pair
+            if (owns) FFMOE_GEMM_WAVE(1, 1);
+            else FFMOE_GEMM_WAVE(0, 1);
+        } else if (!owns) {
+            switch ((n_mb + 3) / 4) {
+                case 1: FFMOE_GEMM_WAVE(0, 1); break;
+                case 2: FFMOE_GEMM_WAVE(0, 2); break;
+                case 3: FFMOE_GEMM_WAVE(0, 3); break;
+                default: FFMOE_GEMM_WAVE(0, 4); break;
+            }
+        } else {
+            switch (n_mb) {
+                case 1: FFMOE_GEMM_WAVE(1, 1); break;
+                case 2: FFMOE_GEMM_WAVE(2, 1); break;
+                case 3: FFMOE_GEMM_WAVE(3, 1); break;
+                case 4: FFMOE_GEMM_WAVE(4, 1); break;
+                case 5: FFMOE_GEMM_WAVE(5, 2); break;
+                case 6: FFMOE_GEMM_WAVE(6, 2); break;
+                case 7: FFMOE_GEMM_WAVE(7, 2); break;
+                case 8: FFMOE_GEMM_WAVE(8, 2); break;
+                case 9: FFMOE_GEMM_WAVE(9, 3); break;
+                case 10: FFMOE_GEMM_WAVE(10, 3); break;
+                case 11: FFMOE_GEMM_WAVE(11, 3); break;
+                case 12: FFMOE_GEMM_WAVE(12, 3); break;
+                case 13: FFMOE_GEMM_WAVE(13, 4); break;
+                case 14: FFMOE_GEMM_WAVE(14, 4); break;
+                case 15: FFMOE_GEMM_WAVE(15, 4); break;
+                default: FFMOE_GEMM_WAVE(16, 4); break;
+            }
+        }
+#undef FFMOE_GEMM_WAVE
+        if (!next.valid || gw.n_groups == 1) vmem_barrier<0>();     // (no load into LDS outlives the block)
+        if (!next.valid) return;
+        it = next;
     }
 }
 
@@ -774,8 +904,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
             } else {
                 uint4 v = __builtin_bit_cast(uint4, stage[k]);
                 if constexpr (F16) {
-                    const _Float16 r = (_Float16)rel[k];
-                    const f16x2 r2 = {r, r};
+                    const f16x2 r2 = __builtin_bit_cast(f16x2, rel[k]);
                     v.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.x) * r2);
                     v.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.y) * r2);
                     v.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.z) * r2);
@@ -980,7 +1109,6 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_
     gw.a_stride = a_stride;
     gw.act_block0 = gw.tile.row_start / 16 + gw.tile.order;
     gw.act_blocks = act_blocks;
-    gw.w_tiles = gw.w_scales = nullptr;
     // the tile row this wave multiplies; past the last one the last again (never stored)
     const uint32_t at = min(nb * kTilesPerBlock + gw.wave, gw.n_arena_tiles - 1);
     const uint8_t *expert_base = arena_layer + (size_t)__builtin_amdgcn_readfirstlane(gw.tile.expert) * g.expert_bytes;
@@ -1016,7 +1144,8 @@ __global__ __launch_bounds__(kBM) void prefill_pair_scale_kernel(const PrefillPl
     float largest = 0.0f;
     for (uint32_t b = 0; b < groups; ++b) largest = fmaxf(largest, s[b * 16]);
     const float inv = 1.0f / largest;          // a scale is 2^(e - 14) with e >= -100: never zero
-    for (uint32_t b = 0; b < groups; ++b) s[b * 16] *= inv;
+    // kept as the FP16 pair that the down products multiply by
+    for (uint32_t b = 0; b < groups; ++b) s[b * 16] = __uint_as_float(Act<true>::pack(s[b * 16] * inv, s[b * 16] * inv));
     act_scale[(size_t)act_blocks * groups * 16 + block * 16 + j] = largest;
 }
 
@@ -1141,13 +1270,13 @@ hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, 
                        sc.sorted_out_row);
     // the pair's input row is whatever row 0 of the scratch holds: only the weight side is looked at
 #define FFMOE_DUMP(GU, H, A, STRIDE, OUT, NB)                                                                              \
-    hipLaunchKernelGGL((prefill_gemm_kernel<GU, H, true>), dim3((NB) * 8), dim3(256), 0, s, arena_layer, g, sc.plan, sc.tiles,  \
-                       sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, false, sc.act_scale, sc.act_blocks, static_cast<uint4 *>(dump))
+    hipLaunchKernelGGL((prefill_gemm_kernel<GU, H, false, true>), dim3((NB) * 8), dim3(64 * kGemmTiles), 0, s, arena_layer, g, sc.plan, sc.tiles,  \
+                       sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, false, sc.act_scale, sc.act_blocks, static_cast<uint4 *>(dump))
     if (gate_up) {
-        const uint32_t nb = (g.gu_rb + kTilesPerBlock - 1) / kTilesPerBlock;
+        const uint32_t nb = (g.gu_rb + kGemmTiles - 1) / kGemmTiles;
         if (f16) FFMOE_DUMP(true, true, sc.partials, g.d, sc.acts, nb); else FFMOE_DUMP(true, false, sc.partials, g.d, sc.acts, nb);
     } else {
-        const uint32_t nb = (g.dn_rbp + kTilesPerBlock - 1) / kTilesPerBlock;
+        const uint32_t nb = (g.dn_rbp + kGemmTiles - 1) / kGemmTiles;
         if (f16) FFMOE_DUMP(false, true, sc.acts, g.f, sc.partials, nb); else FFMOE_DUMP(false, false, sc.acts, g.f, sc.partials, nb);
     }
 #undef FFMOE_DUMP
@@ -1197,23 +1326,27 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     // grid: (N-blocks x tile slots) in either order of the kernel's block map
     const bool nb_major = n_experts == 1;
     auto grid_of = [&](uint32_t n_nblocks) { return nb_major ? 8 * ((n_nblocks + 7) / 8) * tile_cap : n_nblocks * tile_slots; };
+    const uint32_t gemm_gu = (g.gu_rb + kGemmTiles - 1) / kGemmTiles, gemm_dn = (g.dn_rbp + kGemmTiles - 1) / kGemmTiles;
     uint16_t *partials = partials_out ? partials_out : sc.partials;
     float *act_scale = f16 ? sc.act_scale : nullptr;
     const uint32_t act_blocks = f16 ? sc.act_blocks : 0u;
+    // (a row's address is 32 bits from the first row's where that reaches the last)
+    const bool wide = (uint64_t)t * x_stride * 2 > 0xFFFFFFFFull;
 #define FFMOE_GEMM(GU, A, STRIDE, OUT, NB)                                                                                    \
-    hipLaunchKernelGGL((f16 ? prefill_gemm_kernel<GU, true> : prefill_gemm_kernel<GU, false>), dim3(grid_of(NB)), dim3(256), 0, s, \
-                       arena_layer, g, sc.plan, sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major,    \
+    hipLaunchKernelGGL((GU && wide ? (f16 ? prefill_gemm_kernel<GU, true, GU> : prefill_gemm_kernel<GU, false, GU>)                    \
+                                   : (f16 ? prefill_gemm_kernel<GU, true> : prefill_gemm_kernel<GU, false>)), dim3(8 * min((n_cus + 7) / 8, tile_slots * (NB))), dim3(64 * kGemmTiles), 0, s, \
+                       arena_layer, g, sc.plan, sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, nb_major,    \
                        act_scale, act_blocks, nullptr)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
     hipLaunchKernelGGL(stream_kernel<GU>(tile_shift, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
                        sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major, act_scale, act_blocks)
     if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);
-    else FFMOE_GEMM(true, x, x_stride, sc.acts, nb_gu);
+    else FFMOE_GEMM(true, x, x_stride, sc.acts, gemm_gu);
     timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
     if (f16)
         hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap), dim3(kBM), 0, s, sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale);
     if (streamed) FFMOE_STREAM(false, sc.acts, g.f, partials, nb_dn);
-    else FFMOE_GEMM(false, sc.acts, g.f, partials, nb_dn);
+    else FFMOE_GEMM(false, sc.acts, g.f, partials, gemm_dn);
 #undef FFMOE_GEMM
 #undef FFMOE_STREAM
     e = hipGetLastError();

@@ -437,7 +437,7 @@ class Context:
         return out
 
     def prefill_tiles(self, layer: int, expert: int, which: int):
-        """The 16-bit weights of one sub-tensor as the grouped GEMM's matrix instructions read them from LDS, put
+        """The 16-bit weights of one sub-tensor as the grouped GEMM's matrix instructions receive them, put
         back into [rows][cols] order: a CUDA tensor of the context's activation type - bf16(fma(q, s, b)), or
         half(fma(q, s, b)) for a context in FP16 mode (ffmoe_prefill_dump_tiles)."""
         import torch

@@ -1,0 +1,87 @@
+"""The prefill's grouped GEMMs: M-tiles of every number of 16-pair blocks (and one, two and no pairs past a block), plans whose
+largest tile is at most half a tile (deeper rings of packed tiles), K of one group, of fewer and of more than the rings hold,
+N-blocks that are full, half full and a quarter full, fewer and more items than compute units, both activation types; rows that
+span more than 4 GiB. Run on the GPU box: pytest -m gpu."""
+import numpy as np
+import pytest
+
+from helpers import make_layer, to_ff_offsets
+
+pytestmark = pytest.mark.gpu
+
+LONG = (1, 16, 33, 64, 80, 96, 112, 113, 128, 129, 144, 160, 176, 177, 192, 208, 224, 240, 241, 255, 256, 257, 0, 300)
+SHORT = (1, 15, 17, 32, 33, 64, 65, 80, 96, 97, 112, 113, 127, 128, 128, 0)
+
+
+def _check(oracle, pool, e, idx, x, w, y, act):
+    """Element by element against 64-bit products of the 16-bit tile weights: every activation rounded once (unit 2^-8 in bf16,
+    2^-11 in FP16, through the down product's absolute sum), the per-route row and the weighted row once each; a tenth on top
+    for the fp32 sums."""
+    t, d = x.shape
+    dt = x.dtype
+    import torch
+    unit = 2.0 ** (-8 if act == "bf16" else -11)
+    xf, wf = x.double().numpy(), w.double().numpy()
+    ref, spread = np.zeros((t, d)), np.zeros((t, d))
+    for ex in range(e):
+        rows = np.flatnonzero(idx[:, 0] == ex)
+        if not len(rows):
+            continue
+        g, u, dn = (torch.from_numpy(oracle.dequantize_int4(*pool.sub(ex, n))).to(dt).double().numpy() for n in ("gate", "up", "down"))
+        gate, up = xf[rows] @ g.T, xf[rows] @ u.T
+        act_rows = 0.5 * gate * (1 + np.tanh(0.7978845608028654 * (gate + 0.044715 * gate ** 3))) * up
+        ref[rows] = wf[rows] * (act_rows @ dn.T)
+        spread[rows] = wf[rows] * (np.abs(act_rows) @ np.abs(dn.T))
+    assert np.all(np.abs(y - ref) <= 1.1 * unit * (spread + 2 * np.abs(ref)) + 1e-6 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,counts", [(64, 2816, LONG), (128, 1408, LONG), (192, 320, LONG), (704, 192, LONG), (2816, 64, LONG),
+                                        (1408, 128, LONG), (320, 704, LONG), (704, 320, SHORT), (2816, 128, SHORT), (192, 2816, SHORT)])
+def test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    e = len(counts)
+    rng, pool, _ = make_layer(oracle, 31 + d + f, d, f, e, align=1)
+    idx = np.repeat(np.arange(e, dtype=np.uint32), counts)
+    rng.shuffle(idx)
+    idx = idx[:, None]
+    t = idx.shape[0]
+    assert t > 48 * e
+    ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt)
+        w = torch.from_numpy(rng.uniform(0.2, 1.0, (t, 1)).astype(np.float32)).to(dt)
+        gi = torch.from_numpy(idx.view(np.int32)).cuda()
+        y = ctx.prefill(0, x.cuda(), gi, w.cuda())
+        _check(oracle, pool, e, idx, x, w, y.float().cpu().numpy(), act)
+        # the chunk backwards: other pairs in every tile, the same rows
+        back = ctx.prefill(0, x.flip(0).cuda(), gi.flip(0).contiguous(), w.flip(0).cuda())
+        assert torch.equal(back.flip(0), y)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+def test_rows_that_span_four_gigabytes(oracle, act):
+    # 99 rows of 2^25 elements' stride: a row's place does not fit 32 bits
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, e, t, stride = 256, 192, 2, 99, 1 << 25
+    rng, pool, _ = make_layer(oracle, 9, d, f, e, align=1)
+    ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt).cuda()
+        idx = torch.from_numpy(rng.integers(0, e, (t, 1)).astype(np.int32)).cuda()
+        w = torch.from_numpy(rng.uniform(0.2, 1.0, (t, 1)).astype(np.float32)).to(dt).cuda()
+        far = torch.empty(((t - 1) * stride + d,), dtype=dt, device="cuda").as_strided((t, d), (stride, 1))
+        far.copy_(x)
+        assert torch.equal(ctx.prefill(0, far, idx, w), ctx.prefill(0, x, idx, w))
+    finally:
+        ctx.close()
