@@ -663,7 +663,7 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
         }
 #pragma unroll
         for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i)
-            if (16 * i + row < it.tile.rows) *reinterpret_cast<uint4 *>(out + (size_t)orow[i - i0] * g.d + tile * (2 * kTileRows) + 8 * chunk) = v[i - i0];
+            if (16 * i + row < it.tile.rows && (!DUMP || tile < gw.n_arena_tiles)) *reinterpret_cast<uint4 *>(out + (size_t)orow[i - i0] * g.d + tile * (2 * kTileRows) + 8 * chunk) = v[i - i0];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -781,7 +781,9 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
     for (uint32_t r = 1;; ++r) {
         const GemmItem next = item_at(r);
         const uint32_t n_mb = (it.tile.rows + 15) / 16;
-        const bool owns = it.nb * kGemmTiles + gw.wave < gw.n_arena_tiles;
+        // (the test's tiles past the last, up to a set of four, are the last once more)
+        const uint32_t owned = DUMP ? (gw.n_arena_tiles + kTilesPerBlock - 1) / kTilesPerBlock * kTilesPerBlock : gw.n_arena_tiles;
+        const bool owns = it.nb * kGemmTiles + gw.wave < owned;
         // (waves that own no tile take part in the loads and the barriers, which are the same in all instantiations of one LOADS)
 #define FFMOE_GEMM_WAVE(N, L) gemm_wave<GATE_UP, N, L, F16, WIDE, DUMP>(gw, it, next, rings, g, lds, lds_base, sorted_out_row, out, act_scale, dump)
         if constexpr (DUMP) {

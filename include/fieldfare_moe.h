@@ -118,7 +118,7 @@ int ffmoe_dequant_expert(ffmoe_ctx *ctx, void *stream, uint32_t layer, uint32_t 
                          uint16_t *out_bf16, char **err);
 
 /* Test hook for the grouped GEMM of ffmoe_prefill: runs one pair of `expert` through the gate/up (gate_up != 0) or
- * the down GEMM and copies out every weight fragment exactly as the matrix instructions read it from LDS:
+ * the down GEMM and copies out every weight fragment exactly as the matrix instructions receive it:
  * out[N-block][group][fragment 0..15][lane 0..63] x 8 bf16, where an N-block is four 32-row arena tiles, fragment u is
  * arena tile (u % 8) / 2 of the N-block, stream u % 2 (gate / up rows 16 * tile + r; down rows 32 * tile + 16 * stream + r),
  * k-half u / 8, and lane l holds row r = l % 16 at k = 64 * group + 32 * (u / 8) + 8 * (l / 16) .. + 7. Tiles past the last
