@@ -237,8 +237,9 @@ constexpr uint32_t kPrefillStreamPairs = 48;
 constexpr uint32_t kDenseTileStreamRows = 896;       // and the most rows at which a dense FFN's chunk does
 inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts) {
     const uint32_t whole = max_pairs / FFMOE_PREFILL_TILE_M;
-    // tiles of 32 pairs or more up to 48 per expert: 1.5 n_experts full ones at most
-    const uint32_t small = n_experts == 1 ? kDenseTileStreamRows / 32 : kPrefillStreamPairs * n_experts / 32;
+    // tiles of 32 pairs or more up to 48 per expert: 1.5 n_experts full ones at most; a dense FFN's down to 64 rows beyond the streamed
+    const uint32_t dense = kDenseTileStreamRows / 32 > max_pairs / 64 ? kDenseTileStreamRows / 32 : max_pairs / 64;
+    const uint32_t small = n_experts == 1 ? dense : kPrefillStreamPairs * n_experts / 32;
     return (whole > small ? whole : small) + n_experts + 1;
 }
 

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kSortBlock) void prefill_scatter_kernel(ItemSource 
 
 // A dense FFN's chunk needs no sort: one expert, route r = row r. One launch writes what the three above would: the
 // identity tables and the chunk cut into M-tiles.
-__global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t t, uint32_t tile_shift,
+__global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t t, uint32_t bm,
                                                                        PrefillPlan *__restrict__ plan,
                                                                        PrefillTile *__restrict__ tiles,
                                                                        uint32_t *__restrict__ sorted_token,
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
         sorted_token[i] = i;
         sorted_out_row[i] = i;
     }
-    const uint32_t bm = 1u << tile_shift, n_tiles = (t + bm - 1) >> tile_shift;
+    const uint32_t n_tiles = (t + bm - 1) / bm;          // bm: a multiple of 16, at most kBM
     if (i < n_tiles) {
         PrefillTile tl;
         tl.expert = 0;
@@ -1241,15 +1241,33 @@ uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts, uint32_t d, ui
 
 // The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths): tiles of 32 rows while the gate/up
 // launch is one round (four blocks per compute unit on the XCD with the most N-blocks), or while a chunk's products are few
-// enough that the GEMMs' expansion of every weight for each 256 rows still costs more; at most kDenseTileStreamRows.
-// us at 32 | 256 rows per tile, bf16 (FP16): 2,816 -> 2,112, 512 rows 54 | 78 (71 | 107), 800 rows 69 | 79 (88 | 108), 896 rows
-// 78 | 79 (98 | 108); 2,816 -> 2,816, 672 rows 70 | 87, 832 rows 87 | 88, 896 rows 94 | 88 (114 | 121); 4,096 -> 2,816, 672 rows 96 |
-// 106, 704 rows 109 | 106 (126 | 140), 896 rows 129 | 108 (147 | 142); 2,816 -> 704, 896 rows 40 | 64 (48 | 76). Tiles of 64 gain
-// nothing (2,816 -> 2,112, 700 rows 71 | 66 at 32).
+// enough that it cost less than the GEMMs at 256 rows per tile did; at most kDenseTileStreamRows. With tiles of fewer rows the
+// GEMMs are now the faster ones from some 640 rows on (2,816 -> 2,112, 897 rows 62 us, FP16 85, where 896 streamed ones take 78
+// and 98), but their weights are rounded to 16 bits and the streamed ones' are not: a chunk that had the smaller error keeps it.
+// us at 32 | 256 rows per tile, bf16 (FP16): 2,816 -> 2,112, 512 rows 54 | 78 (71 | 107), 800 rows 69 | 79 (88 | 108); 2,816 ->
+// 2,816, 672 rows 70 | 87, 896 rows 94 | 88 (114 | 121); 4,096 -> 2,816, 672 rows 96 | 106, 896 rows 129 | 108 (147 | 142).
+// Streamed tiles of 64 gain nothing (2,816 -> 2,112, 700 rows 71 | 66 at 32).
 uint32_t dense_tile_shift(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, bool f16) {
     if (t > kDenseTileStreamRows) return 8;
     const bool one_round = (n_nblocks + 7) / 8 * ((t + 31) / 32) <= 4 * (n_cus / 8);
     return one_round || (uint64_t)t * g.d * g.f <= (f16 ? 9600000000ull : 6600000000ull) ? 5 : 8;
+}
+
+// Rows per M-tile of a dense FFN's GEMMs: 16 n, n chosen so that the items fill their last round. A compute unit takes (10 + n) / 10 of
+// about 1,000 cycles per group of an item and the time of some six groups around them; the lists' last N-blocks are counted as
+// full ones. 2,816 -> 2,112 -> 2,816, us of the call at 256 rows per tile | the rule's: 102 | 62 at 897 rows (n = 4), 104 | 82 at
+// 2,048 (9), 112 | 103 at 3,072 (13), 170 | 147 at 4,096 (12), 292 | 259 at 8,192 (13); FP16 inputs 144 | 85, 148 | 113, 154 | 141,
+// 220 | 188 and 367 | 323. Of n = 6..16 each, the rule's is the fastest at these sizes or within 3% of it.
+uint32_t dense_tile_rows(uint32_t t, const ArenaGeom &g, uint32_t n_cus) {
+    uint32_t best = kBM;
+    uint64_t least = ~0ull;
+    for (uint32_t n = kBM / 16; n >= 4; --n) {
+        const uint32_t m = (t + 16 * n - 1) / (16 * n);
+        auto rounds = [&](uint32_t arena_tiles) { return (uint64_t)((m * ((arena_tiles + kGemmTiles - 1) / kGemmTiles) + n_cus - 1) / n_cus); };
+        const uint64_t cost = (10 + n) * (rounds(g.gu_rb) * (g.gd + 6) + rounds(g.dn_rbp) * (g.gf + 6));
+        if (cost < least) least = cost, best = 16 * n;
+    }
+    return best;
 }
 
 template <bool GATE_UP>
@@ -1306,8 +1324,9 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     const uint32_t tile_shift =
         dense ? dense_tile_shift(t, g, nb_gu, n_cus, f16) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts, g.d, nb_gu, n_cus, f16);
     const bool streamed = tile_shift < 8;
+    const uint32_t dense_rows = dense && !streamed ? dense_tile_rows(t, g, n_cus) : 1u << tile_shift;
     if (dense) {
-        hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_shift, sc.plan, sc.tiles, sc.sorted_token,
+        hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, dense_rows, sc.plan, sc.tiles, sc.sorted_token,
                            sc.sorted_out_row);
     } else {
         hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
@@ -1322,7 +1341,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     timer->mark(s, FFMOE_K_PREFILL_SORT);
-    const uint32_t tile_cap = min(sc.max_tiles, (src.n_items >> tile_shift) + n_experts);
+    const uint32_t tile_cap = min(sc.max_tiles, dense ? (t + dense_rows - 1) / dense_rows : (src.n_items >> tile_shift) + n_experts);
     const uint32_t tile_slots = (tile_cap + 7) / 8 * 8;
     if (f16 && !sc.act_scale) return hipErrorInvalidValue;      // allocated when the context was switched to FP16
     // grid: (N-blocks x tile slots) in either order of the kernel's block map

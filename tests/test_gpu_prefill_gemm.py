@@ -85,3 +85,29 @@ def test_rows_that_span_four_gigabytes(oracle, act):
         assert torch.equal(ctx.prefill(0, far, idx, w), ctx.prefill(0, x, idx, w))
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,rows", [(704, 1408, (897, 1025, 1500, 1601, 2049, 2300, 2800, 3000, 3600, 4000, 4400, 5000)),
+                                      (1408, 1408, (913, 1700, 4801, 5000, 5600))])
+def test_dense_tiles_of_the_row_count(oracle, act, d, f, rows):
+    """A dense FFN's tiles have as many rows as fill the last round of blocks (64 to 256): the largest chunk against 64-bit products,
+    every other one, cut elsewhere, to the same bits."""
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    rng, pool, _ = make_layer(oracle, 77 + d, d, f, 1, align=1)
+    t = max(rows)
+    ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt)
+        y = ctx.dense_ffn(0, x.cuda())
+        # (the reference's cost bounds the rows compared: the first and last of the chunk, which every tile size cuts differently)
+        some = np.r_[0:200, t - 200:t]
+        _check(oracle, pool, 1, np.zeros((len(some), 1), np.uint32), x[some], torch.ones((len(some), 1), dtype=dt), y.float().cpu().numpy()[some], act)
+        for n in rows:
+            assert torch.equal(ctx.dense_ffn(0, x[:n].cuda()), y[:n]), n
+    finally:
+        ctx.close()
