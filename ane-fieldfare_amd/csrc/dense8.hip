@@ -17,13 +17,12 @@
 namespace ffmoe {
 namespace {
 
-constexpr int kTilesN = 8;                                  // 16-row tiles per N-block
-constexpr int kBFrags = kTilesN * 2;                        // weight fragments per N-block and group
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+constexpr int kTilesN = 8;                                  // 16-row tiles per 128-row block
+constexpr int kBFrags = kTilesN * 2;                        // weight fragments of it per group
 
 __device__ __forceinline__ uint32_t ext_groups(uint32_t n_groups) { return (3 * n_groups + kGroup - 1) / kGroup; }
 
-// Column c of the bias columns, row j of a 16-row block: where it stands behind the block's (or N-block tile's) groups.
+// Column c of the bias columns, row j of a 16-row block: where it stands behind the block's (or tile's) groups.
 __device__ __forceinline__ uint32_t ext_lane(uint32_t c, uint32_t j) { return ((c & 31) >> 3) * 16 + j; }
 
 // a row's group sum as three bf16 values that add up to its 24 significant bits
@@ -45,7 +44,7 @@ __global__ __launch_bounds__(256) void dense8_weights_kernel(const uint8_t *__re
     for (size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x; gid < total; gid += (size_t)gridDim.x * 256) {
         const uint32_t piece = (uint32_t)(gid & 7), grp = (uint32_t)(gid / 8 % all_groups), row = (uint32_t)(gid / 8 / all_groups);
         const uint32_t tr = row >> 4, i = row & 15, jq = piece & 3, kh = piece >> 2;
-        const bool real = tr < n_tiles;                     // tiles past the matrix (half an N-block): zeros
+        const bool real = tr < n_tiles;                     // tiles past the matrix (half a block): zeros
         uint32_t w[4] = {0, 0, 0, 0};
         float sc = 1.0f;                                    // the bias columns' scale
         if (grp < n_groups) {
@@ -117,216 +116,288 @@ __global__ __launch_bounds__(256) void dense8_rows_kernel(const uint16_t *__rest
     }
 }
 
-// One block = 16 NMB (4 / WN) rows x one N-block of 128 weight rows; wave (wm, wn) owns every (4 / WN)th 16-row block from wm on
-// and the tiles (8 / WN) wn ... Weights of a group (16 KiB) go through LDS in two buffers, a group ahead in registers; the inputs
-// are in operand order and go straight to registers, a group ahead. Two fma of the tile before stand behind each product, so
-// that the vector unit works in the matrix unit's shadow. GATED: out = the activations as the second GEMM's operands (with
-// their group sums); else out = the output rows.
-// Bound: the compute unit's LDS and load paths beside the matrix unit (at 128 rows and WN = 1, per group: 1,088 cycles of LDS
-// for 512 of products on each SIMD; WN = 2 halves the fragment reads and loads every input twice, 218 us at 3,072 rows where
-// WN = 1 takes 174). 3,072 rows of 2,816 -> 2,112 -> 2,816, whole FFN: 174-181 us against 248 for two library GEMMs on hi / lo
-// rows with their epilogue passes. Measured and not kept: three groups of loads in flight (no change; two waves per SIMD
-// fewer), 192-row tiles (178 us, and 251 against 206 at 4,096 rows, whose blocks they spread badly).
-template <bool GATED, int NMB, int WN, bool F16>
-__global__ __launch_bounds__(256, 2) void dense8_gemm_kernel(const uint16_t *__restrict__ weights, const float *__restrict__ scales,
-                                                             uint32_t n_groups, uint32_t n_blocks, uint32_t n_cols,
-                                                             const uint16_t *__restrict__ a, uint32_t t, uint16_t *__restrict__ out,
-                                                             uint32_t out_stride) {
-    __shared__ __align__(16) uint4 wb[2][kBFrags * kWave];
-    __shared__ __align__(16) float sb[2][16 * kTilesN];
+// The GEMMs. An item = 16 NM rows x one N-block of 256 weight rows, a block of eight waves: wave w has the two 16-row tiles 2 w and
+// 2 w + 1 (GATED: gate and up of the same 16 activations) for all the rows. Inputs and weights lie in operand order and go straight
+// into LDS, a fragment (1 KiB) per instruction, two groups ahead: the inputs into a ring of three groups that the block shares,
+// a wave's 4 KiB of weights into two slots of its own, from where they go to registers. One barrier per group; it stands where the
+// last of a group's fragments have been read, so that reads run on into the next group and the buffer can be filled again.
+// Two fma per product bring a group's sums into the running ones with their scale: those of a 16-row block stand between the
+// products of the next (a group's last block: of the next group's first). GATED: out = the activations as the second GEMM's
+// operands (with their group sums); else out = the output rows.
+// Bound: the matrix unit and, with it on all compute units, the card's power: the products, their fma and the fragment reads
+// alone take 53 us where the gated product of 13 blocks takes 65 on 68 compute units and 80 on 255 (with inputs of zeros 72). The
+// barrier and the weights' reads are 6 of the difference, the loads into LDS 8; nearer loads change nothing, nor do four products
+// in a row with a raised wave priority, weights in two register sets without moves, or offsets in vector registers. 2,816 ->
+// 2,112 -> 2,816, us of gate/up + down where four waves took 64 or 128 rows and 128 weight rows with weights through registers and
+// a barrier before every group's reads | now: 640 rows 42 + 27 | 30 + 21, 1,024 rows 55 + 32 | 38 + 23, 3,072 rows 115 + 61 | 80 +
+// 46, 8,192 rows 261 + 130 | 230 + 118; FP16 alike. 704 -> 2,816, 1,024 rows 21 + 31 | 17 + 25; 2,816 -> 256, 4,096 rows 45 + 16 |
+// 28 + 15.
+
+// LDS of a block: three groups of inputs (2 NM KiB each), then every wave's two groups of weights and of their scales. The
+// epilogue's images take the same bytes.
+constexpr int kWaves8 = 8;
+constexpr uint32_t kFrag8 = kWave * 16;                     // bytes of a fragment
+constexpr uint32_t kSlot8 = 4 * kFrag8, kScaleSlot8 = kWave * 4;
+template <int NM> struct Lds8 {
+    static constexpr uint32_t a_bytes = 2 * NM * kFrag8, w_at = 3 * a_bytes, s_at = w_at + 2 * kWaves8 * kSlot8,
+                              bytes = s_at + 2 * kWaves8 * kScaleSlot8;
+};
+constexpr int kMaxBlocks8 = 15, kMinBlocks8 = 3;            // 16-row blocks per item
+
+// Fragments of inputs in flight or in use per wave: a divisor of a group's 2 NM, so that a fragment's registers are known at compile time.
+constexpr int queue8(int nm) {
+    int q = 2;
+    for (int d = 3; d <= (nm == 11 || nm == 13 ? nm : 8); ++d)
+        if (2 * nm % d == 0) q = d;
+    return q;
+}
+
+template <bool GATED, int NM, bool F16>
+__global__ __launch_bounds__(64 * kWaves8, 2) void dense8_gemm_kernel(const uint8_t *__restrict__ weights, const float *__restrict__ scales,
+                                                                      uint32_t n_groups, uint32_t n_blocks, uint32_t n_cols,
+                                                                      const uint8_t *__restrict__ a, uint32_t t, uint16_t *__restrict__ out,
+                                                                      uint32_t out_stride) {
+    using L = Lds8<NM>;
+    __shared__ __align__(16) uint8_t lds[L::bytes];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, jq = lane >> 4;
-    constexpr int WM = 4 / WN;                              // waves side by side over the rows, over the tiles
-    const uint32_t wm = wave % WM, wn = wave / WM;
-    // all row tiles of an N-block on one XCD: its weights are read into one L2
-    const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, per_xcd = (n_blocks + 7) / 8;
-    const uint32_t mt = slot / per_xcd, nb = (slot % per_xcd) * 8 + xcd;
-    if (nb >= n_blocks) return;
-    const uint32_t ge = ext_groups(n_groups), all_groups = n_groups + ge, row_blocks = (t + 15) / 16;
-    const u32x4_t *wsrc = reinterpret_cast<const u32x4_t *>(weights) + (size_t)nb * all_groups * (kBFrags * kWave) + tid;
-    const float *ssrc = scales + (size_t)nb * all_groups * (16 * kTilesN) + (tid & 127);
-    const uint4 *asrc[NMB];
-    uint32_t blk[NMB];
+    // the items N-block by N-block, an eighth of the list per XCD: each reads its eighth of the weights into its L2 once
+    const uint32_t row_blocks = (t + 15) / 16, m_tiles = (row_blocks + NM - 1) / NM, n_nb = (n_blocks + 1) / 2, all = m_tiles * n_nb;
+    const uint32_t xcd = blockIdx.x & 7, first = (uint32_t)((uint64_t)all * xcd / 8);
+    const uint32_t item = first + (blockIdx.x >> 3);
+    if (item >= (uint32_t)((uint64_t)all * (xcd + 1) / 8)) return;
+    const uint32_t nb = item / m_tiles, block0 = item % m_tiles * NM;
+    const uint32_t all_groups = n_groups + ext_groups(n_groups), last = all_groups - 1;
+    // this wave's 128-row block of weights, of which it has tiles 2 (wave % 4) and the next; past the last block the last again
+    const bool owns = nb * 2 + (wave >> 2) < n_blocks;
+    const size_t wblock = (size_t)min(nb * 2 + (wave >> 2), n_blocks - 1) * all_groups;
+    const uint8_t *const w = weights + (wblock * kBFrags + (wave & 3) * 4) * kFrag8;
+    const float *const sc_src = scales + wblock * (16 * kTilesN) + (wave & 3) * 2;
+    const uint32_t sc_lane = ((lane & 31) >> 1) * (kTilesN * 4) + (lane & 1) * 4;        // row by row, both tiles
+    constexpr int kLoadsA = (2 * NM + kWaves8 - 1) / kWaves8;                              // KiB per wave and group
+    constexpr int kLoads = kLoadsA + 5;
+    uint32_t from[kLoadsA], to[kLoadsA];
 #pragma unroll
-    for (int i = 0; i < NMB; ++i) {
-        blk[i] = mt * (WM * NMB) + wm + WM * i;
-        // blocks past the last read it again (never stored)
-        asrc[i] = reinterpret_cast<const uint4 *>(a) + (size_t)min(blk[i], row_blocks - 1) * all_groups * (2 * kWave) + lane;
+    for (int k = 0; k < kLoadsA; ++k) {
+        // (what does not divide by the waves, the last fragment several times; blocks past the last are the last again, never stored)
+        const uint32_t piece = min(wave + kWaves8 * k, 2u * NM - 1);
+        from[k] = min(block0 + (piece >> 1), row_blocks - 1) * all_groups * 2 + (piece & 1);
+        to[k] = piece * kFrag8;
     }
-    const uint32_t last = all_groups - 1;                   // loads past the end fetch the last group again, never used
-    u32x4_t wst[4];
-    float sst = 0.0f;
-    auto load_b = [&](uint32_t grp) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) wst[k] = wsrc[(size_t)grp * (kBFrags * kWave) + 256 * k];
-        sst = ssrc[grp * (16 * kTilesN)];
+    auto load_w = [&](uint32_t grp, uint32_t slot, int k) __attribute__((always_inline)) {
+        if (k < 4) global_to_lds_16(w + (size_t)grp * (kBFrags * kFrag8) + k * kFrag8, lane * 16, lds_base + L::w_at + (slot * kWaves8 + wave) * kSlot8 + k * kFrag8);
+        else global_to_lds_4(sc_src + grp * (16 * kTilesN), sc_lane, lds_base + L::s_at + (slot * kWaves8 + wave) * kScaleSlot8);
     };
-    auto store_b = [&](uint32_t buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) reinterpret_cast<u32x4_t *>(wb[buf])[256 * k + tid] = wst[k];
-        if (tid < 16 * kTilesN) sb[buf][tid] = sst;
+    auto load_a = [&](uint32_t grp, uint32_t buf, int k) __attribute__((always_inline)) {
+        global_to_lds_16(a + ((size_t)from[k] + 2 * grp) * kFrag8, lane * 16, lds_base + buf + to[k]);
     };
-    uint4 an[NMB][2];
-    auto load_a = [&](uint32_t grp) __attribute__((always_inline)) {
+    uint4 wf[2][2];                     // operands: tile, k-half
+    float sc[2][2] = {};                // of the group before, of this one
+    uint4 wn[2][2];
+    float sn[2];
+    auto read_w = [&](uint32_t slot) __attribute__((always_inline)) {
+        const uint8_t *at = lds + L::w_at + (slot * kWaves8 + wave) * kSlot8;
 #pragma unroll
-        for (int i = 0; i < NMB; ++i)
+        for (int st = 0; st < 2; ++st)
 #pragma unroll
-            for (int kh = 0; kh < 2; ++kh) an[i][kh] = asrc[i][(grp * 2 + kh) * kWave];
+            for (int kh = 0; kh < 2; ++kh) wn[st][kh] = *reinterpret_cast<const uint4 *>(at + (st * 2 + kh) * kFrag8 + lane * 16);
+        const float2 v = *reinterpret_cast<const float2 *>(lds + L::s_at + (slot * kWaves8 + wave) * kScaleSlot8 + j * 8);
+        sn[0] = v.x, sn[1] = v.y;
     };
-    constexpr int kTiles = kTilesN / WN;                    // of this wave
-    f32x4 tot[NMB][kTiles];
+    constexpr int kFrags = 2 * NM, kQueue = queue8(NM), kLate = 2;
+    uint4 xq[kQueue];
+    auto read_a = [&](uint32_t buf, int f) __attribute__((always_inline)) {
+        xq[f % kQueue] = *reinterpret_cast<const uint4 *>(lds + buf + f * kFrag8 + lane * 16);
+    };
+    f32x4 tot[NM][2];
 #pragma unroll
-    for (int i = 0; i < NMB; ++i)
+    for (int i = 0; i < NM; ++i) tot[i][0] = tot[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // a block's products of one group, in flight while the block before is added up (a group's last during the next one's first)
+    f32x4 part[3][2];
+    part[2][0] = part[2][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto part_of = [](int i) __attribute__((always_inline)) { return i == NM - 1 ? 2 : i & 1; };
+    auto add = [&](int i, int m, int which) __attribute__((always_inline)) {              // two of a block's eight sums
+        const int st = m >> 1;
 #pragma unroll
-        for (int nf = 0; nf < kTiles; ++nf) tot[i][nf] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int r = 2 * (m & 1); r < 2 * (m & 1) + 2; ++r) tot[i][st][r] = __builtin_fmaf(sc[st][which], part[part_of(i)][st][r], tot[i][st][r]);
+    };
+    uint32_t cur = 0, next = L::a_bytes, before = 2 * L::a_bytes, slot = 0;
 
     // H: the element type of this group's operands (the bias columns are bf16 in either mode)
     auto step = [&](uint32_t grp, auto type) __attribute__((always_inline)) {
         constexpr bool H = decltype(type)::value;
-        const uint32_t buf = grp & 1;
-        uint4 af[NMB][2];
 #pragma unroll
-        for (int i = 0; i < NMB; ++i) af[i][0] = an[i][0], af[i][1] = an[i][1];
-        store_b(buf ^ 1);                                   // group grp + 1 (past the last: a buffer nobody reads)
-        load_b(min(grp + 2, last));
-        load_a(min(grp + 1, last));
-        float sc[kTiles];
+        for (int st = 0; st < 2; ++st) wf[st][0] = wn[st][0], wf[st][1] = wn[st][1], sc[st][0] = sc[st][1], sc[st][1] = sn[st];
+        constexpr int kBarrier = kFrags - kQueue + 1 + kLate;
 #pragma unroll
-        for (int nf = 0; nf < kTiles; nf += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(&sb[buf][j * kTilesN + kTiles * wn + nf]);
-            sc[nf] = v[0], sc[nf + 1] = v[1], sc[nf + 2] = v[2], sc[nf + 3] = v[3];
-        }
-        // tile by tile: its products, and the sums of the tile before between them, two fma behind each product
-        // (a wave alone on its SIMD asks for all its fragments first: their latency is then paid once per group)
-        constexpr int kQueue = WN == 2 ? kTiles : 2;
-        uint4 bq[kQueue][2];
-        auto read_b = [&](int nf) __attribute__((always_inline)) {
+        for (int f = 0; f < kFrags; ++f) {
+            const int i = f >> 1, kh = f & 1, ahead = f + kQueue - 1;
+            if (f == kBarrier) {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory");
+                read_w(slot ^ 1);
 #pragma unroll
-            for (int kh = 0; kh < 2; ++kh) bq[nf % kQueue][kh] = wb[buf][((kTiles * wn + nf) * 2 + kh) * kWave + lane];
-        };
-        f32x4 part[2][NMB];
-        auto add = [&](int nf, int f) __attribute__((always_inline)) {
-            tot[f >> 2][nf][f & 3] = __builtin_fmaf(sc[nf], part[nf & 1][f >> 2][f & 3], tot[f >> 2][nf][f & 3]);
-        };
+                for (int n = 0; n < kLate; ++n) read_a(next, n);
+            }
+            if (ahead < kFrags) read_a(cur, ahead);
+            else if (f >= kBarrier) read_a(next, ahead - kFrags);
 #pragma unroll
-        for (int nf = 0; nf < kQueue - 1; ++nf) read_b(nf);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int nf = 0; nf < kTiles; ++nf) {
-            if (nf + kQueue - 1 < kTiles) read_b(nf + kQueue - 1);
-#pragma unroll
-            for (int m = 0; m < 2 * NMB; ++m) {
-                const int i = m % NMB, kh = m / NMB;
+            for (int st = 0; st < 2; ++st) {
                 const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-                part[nf & 1][i] = Act<H>::mfma(af[i][kh], bq[nf % kQueue][kh], kh ? part[nf & 1][i] : zero);
-                if (nf > 0) {
-                    add(nf - 1, 2 * m);
-                    add(nf - 1, 2 * m + 1);
-                }
+                part[part_of(i)][st] = Act<H>::mfma(xq[f % kQueue], wf[st][kh], kh ? part[part_of(i)][st] : zero);
+                // the sums of the block before, three products behind their last one
+                const int at = 2 * f + st, m = at & 3;
+                if (m > 0) add((i + NM - 1) % NM, m - 1, i > 0);
+                else if (at > 0) add((i + NM - 2) % NM, 3, i > 1);
+#pragma unroll
+                for (int k = 0; k < 5; ++k)
+                    if (at == 2 + k * (2 * kBarrier - 2) / 5) load_w(min(grp + 2, last), slot, k);
+#pragma unroll
+                for (int k = 0; k < kLoadsA; ++k)
+                    if (at == 2 * kBarrier + 1 + k * (2 * (kFrags - kBarrier) - 1) / kLoadsA) load_a(min(grp + 3, last), cur, k);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-#pragma unroll
-        for (int f = 0; f < 4 * NMB; ++f) add(kTiles - 1, f);
-        lds_barrier();
+        add((2 * NM - 2) % NM, 3, 1);
+        const uint32_t c = cur;
+        cur = next, next = before, before = c;
+        slot ^= 1;
     };
-    load_b(0);
-    load_a(0);
-    store_b(0);
-    load_b(min(1u, last));
-    lds_barrier();
+#pragma unroll
+    for (uint32_t g = 0; g < 3; ++g) {
+#pragma unroll
+        for (int k = 0; k < kLoadsA; ++k) load_a(min(g, last), g * L::a_bytes, k);
+#pragma unroll
+        for (int k = 0; k < 5; ++k)
+            if (g < 2) load_w(min(g, last), g, k);
+    }
+    vmem_barrier<kLoads + kLoadsA>();
+    read_w(0);
+#pragma unroll
+    for (int f = 0; f < kQueue - 1; ++f) read_a(cur, f);
+#pragma nounroll
     for (uint32_t grp = 0; grp < n_groups; ++grp) step(grp, std::integral_constant<bool, F16>{});
+#pragma nounroll
     for (uint32_t grp = n_groups; grp < all_groups; ++grp) step(grp, std::integral_constant<bool, false>{});
+#pragma unroll
+    for (int m = 0; m < 4; ++m) add(NM - 1, m, 1);
+    // (an fp32 value like the others' and then a 16-bit one: not both in one instruction with one rounding)
+    asm volatile("" : "+v"(tot[NM - 1][0]), "+v"(tot[NM - 1][1]));
+    vmem_barrier<0>();                                      // no load is on its way into what the epilogue writes
+    lds_barrier();
 
-    // lane (j, jq) holds weight row j of every tile for rows 4 jq .. 4 jq + 3 of every 16-row block; each wave turns its blocks
-    // through a piece of the weight buffers of its own (the last step ended with a barrier)
-    constexpr uint32_t kStageRow = kTiles * 32 + 16;        // bytes: 64 columns + padding
-    constexpr uint32_t kStageBytes = 4 * 16 * kStageRow, kRows = 16 * WM * NMB;
-    static_assert(kStageBytes + 2 * kRows * sizeof(float) <= sizeof(wb), "staging and row sums fit the weight buffers");
-    uint8_t *stage = reinterpret_cast<uint8_t *>(wb) + wave * 16 * kStageRow;
-    float *row_sums = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(wb) + kStageBytes);      // [k-half][row of the tile]
-    auto wave_sync = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    const uint32_t f_groups = n_blocks, f_all = f_groups + ext_groups(f_groups);         // (GATED: an N-block is a group of F)
+    // lane (j, jq) holds weight row j of both tiles for rows 4 jq .. 4 jq + 3 of every 16-row block
+    if constexpr (GATED) {
+        // gate and up of 16 activations: a quarter of group 2 nb + wave / 4 of F, k-half (wave / 2) % 2. The operands are put together
+        // in LDS ([group][16-row block][k-half][lane]), stored from there, and their groups summed there.
+        uint16_t *img = reinterpret_cast<uint16_t *>(lds);
 #pragma unroll
-    for (int i = 0; i < NMB; ++i) {
-        if (blk[i] >= row_blocks) continue;                 // wave-uniform
-        if constexpr (GATED) {
-            // tiles 2 tl and 2 tl + 1 of this wave: gate and up of 16 activations; its share of group nb is k-half wn, or both
-            uint16_t *img = reinterpret_cast<uint16_t *>(stage);
-            float sum[2 / WN][4] = {};             // per k-half, so that both splits of the tiles add up alike
+        for (int i = 0; i < NM; ++i)
 #pragma unroll
-            for (int tl = 0; tl < kTiles / 2; ++tl)
+            for (int r = 0; r < 4; ++r) {
+                const float g = Act<F16>::widen(Act<F16>::round(tot[i][0][r])), u = Act<F16>::widen(Act<F16>::round(tot[i][1][r]));
+                img[((((wave >> 2) * NM + i) * 2 + (wave >> 1 & 1)) * kWave + ((wave & 1) * 2 + (j >> 3)) * 16 + 4 * jq + r) * 8 + (j & 7)] =
+                    Act<F16>::round(gelu_tanh_fast(g) * u);
+            }
+        lds_barrier();
+        const uint32_t f_groups = n_blocks, f_all = f_groups + ext_groups(f_groups), groups = min(2u, f_groups - 2 * nb);
+        for (uint32_t p = tid; p < groups * NM * 2 * kWave; p += 64 * kWaves8) {
+            const uint32_t gi = p / (NM * 2 * kWave), i = p / (2 * kWave) % NM;
+            if (block0 + i < row_blocks)
+                reinterpret_cast<uint4 *>(out)[((size_t)(block0 + i) * f_all + 2 * nb + gi) * (2 * kWave) + p % (2 * kWave)] = reinterpret_cast<const uint4 *>(lds)[p];
+        }
+        // the group sums of the activations as they were rounded, into the second GEMM's bias columns: a thread per row and group
+        for (uint32_t p = tid; p < groups * NM * 16; p += 64 * kWaves8) {
+            const uint32_t gi = p / (NM * 16), i = p / 16 % NM, row = p & 15;
+            if (block0 + i >= row_blocks) continue;
+            float sum[2];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float g = Act<F16>::widen(Act<F16>::round(tot[i][2 * tl][r])), u = Act<F16>::widen(Act<F16>::round(tot[i][2 * tl + 1][r]));
-                    const uint16_t v = Act<F16>::round(gelu_tanh_fast(g) * u);
-                    sum[tl >> 1][r] += Act<F16>::widen(v);
-                    img[((tl >> 1) * kWave + ((tl & 1) * 2 + (j >> 3)) * 16 + 4 * jq + r) * 8 + (j & 7)] = v;
+            for (int kh = 0; kh < 2; ++kh) {
+                const uint4 *at = reinterpret_cast<const uint4 *>(lds) + ((gi * NM + i) * 2 + kh) * kWave + row;
+                float v[16];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const uint4 x = at[16 * c], y = at[16 * (c + 2)];
+                    const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, yw[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        v[8 * c + 2 * q] = Act<F16>::lo(xw[q]) + Act<F16>::lo(yw[q]);
+                        v[8 * c + 2 * q + 1] = Act<F16>::hi(xw[q]) + Act<F16>::hi(yw[q]);
+                    }
                 }
 #pragma unroll
-            for (int h = 0; h < 2 / WN; ++h)
+                for (int m = 1; m < 16; m <<= 1)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
+                    for (int q = 0; q < 16; q += 2 * m) v[q] += v[q + m];
+                sum[kh] = v[0];
+            }
+            uint16_t part[3];
+            split_sum(sum[0] + sum[1], part);
+            uint16_t *dst = out + (size_t)(block0 + i) * f_all * 2 * (kWave * 8);
 #pragma unroll
-                    for (int m = 1; m < 16; m <<= 1) sum[h][r] += __shfl_xor(sum[h][r], m, 64);
-                    if (j == 0) row_sums[(wn + h) * kRows + (wm + WM * i) * 16 + 4 * jq + r] = sum[h][r];
-                }
-            wave_sync();
+            for (int q = 0; q < 3; ++q) {
+                const uint32_t c = 3 * (2 * nb + gi) + q;
+                dst[((size_t)(f_groups + (c >> 6)) * 2 + ((c & 63) >> 5)) * (kWave * 8) + ext_lane(c, row) * 8 + (c & 7)] = part[q];
+            }
+        }
+    } else {
+        // a 16-row block of this wave's columns is 16 rows x 64 bytes: each wave turns its blocks through a piece of LDS of its own
+        constexpr uint32_t kStageRow = 64 + 16, kStage = 16 * kStageRow;                 // bytes: 32 columns + padding
+        constexpr int kTurn = 4;
+        static_assert(kWaves8 * kTurn * kStage <= L::bytes, "staging fits the rings");
+        uint8_t *stage = lds + wave * (kTurn * kStage);
+        const uint32_t sub = lane >> 2, chunk = lane & 3, col = nb * 256 + wave * 32 + 8 * chunk;
+        if (!owns) return;
 #pragma unroll
-            for (int h = 0; h < 2 / WN; ++h)
-                reinterpret_cast<uint4 *>(out)[(((size_t)blk[i] * f_all + nb) * 2 + wn + h) * kWave + lane] =
-                    reinterpret_cast<const uint4 *>(stage)[h * kWave + lane];
-            wave_sync();
-        } else {
+        for (int i0 = 0; i0 < NM; i0 += kTurn) {
 #pragma unroll
-            for (int nf = 0; nf < kTiles; ++nf)
+            for (int i = i0; i < i0 + kTurn && i < NM; ++i)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    *reinterpret_cast<uint16_t *>(stage + (4 * jq + r) * kStageRow + nf * 32 + 2 * j) = Act<F16>::round(tot[i][nf][r]);
-            wave_sync();
+                for (int st = 0; st < 2; ++st)
 #pragma unroll
-            for (int p = 0; p < 4 / WN; ++p) {
-                constexpr uint32_t kChunks = 2 * kTiles;                                 // 16-byte pieces of a staged row
-                const uint32_t sub = (kWave / kChunks) * p + lane / kChunks, chunk = lane % kChunks, row = blk[i] * 16 + sub;
-                const uint32_t col = nb * (kTilesN * 16) + wn * (kTiles * 16) + 8 * chunk;
-                const uint4 v = *reinterpret_cast<const uint4 *>(stage + sub * kStageRow + 16 * chunk);
+                    for (int r = 0; r < 4; ++r)
+                        *reinterpret_cast<uint16_t *>(stage + (i - i0) * kStage + (4 * jq + r) * kStageRow + st * 32 + 2 * j) = Act<F16>::round(tot[i][st][r]);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int i = i0; i < i0 + kTurn && i < NM; ++i) {
+                const uint32_t row = (block0 + i) * 16 + sub;
+                const uint4 v = *reinterpret_cast<const uint4 *>(stage + (i - i0) * kStage + sub * kStageRow + 16 * chunk);
                 if (row < t && col < n_cols) *reinterpret_cast<uint4 *>(out + (size_t)row * out_stride + col) = v;
             }
-            wave_sync();
-        }
-    }
-    if constexpr (GATED) {
-        // the group sums of the activations as they were rounded, into the second GEMM's bias columns
-        lds_barrier();
-        const uint32_t block = mt * (WM * NMB) + (tid >> 4);
-        if (tid < kRows && block < row_blocks) {
-            uint16_t part[3];
-            split_sum(row_sums[tid] + row_sums[kRows + tid], part);
-            uint16_t *dst = out + (size_t)block * f_all * 2 * (kWave * 8);
-#pragma unroll
-            for (int p = 0; p < 3; ++p) {
-                const uint32_t c = 3 * nb + p;
-                dst[((size_t)(f_groups + (c >> 6)) * 2 + ((c & 63) >> 5)) * (kWave * 8) + ext_lane(c, tid & 15) * 8 + (c & 7)] = part[p];
-            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     }
 }
 
 uint32_t all_groups_of(uint32_t n) { return n / kGroup + (3 * (n / kGroup) + kGroup - 1) / kGroup; }
+// 16-row blocks per item: as many as make the rounds of items over the compute units cheapest, an item of n costing n + 6 (2,816 wide,
+// one round: 28.7 us at 3, 68.2 at 15). Of 3..15 each, the rule's is the fastest or within 4% of it, gate/up of 2,112 at 640 rows
+// (3: 29 us, 8: 45), 1,024 (5: 36, 4: 61 in two rounds), 2,048 (9: 56, 8: 92), 3,072 (13: 80, 12: 125, 7: 90), 4,096 (9: 108, 12:
+// 122), 8,192 (12: 203, 9: 214, 13: 222); down at 3,072 (9: 44, 8: 70, 13: 54), 4,096 (12: 54, 11: 89). 15 is what LDS holds; below 3
+// a group's 32 KiB of weights take longer than its products. Any gives the same bits.
+uint32_t dense8_blocks(uint32_t row_blocks, uint32_t n_nb, uint32_t n_cus) {
+    uint32_t best = kMaxBlocks8;
+    uint64_t least = ~0ull;
+    for (uint32_t n = kMaxBlocks8; n >= (uint32_t)kMinBlocks8; --n) {
+        const uint64_t rounds = ((row_blocks + n - 1) / n * n_nb + n_cus - 1) / n_cus, cost = rounds * (6 + n);
+        if (cost < least) least = cost, best = n;
+    }
+    return best;
+}
 uint32_t n_blocks_of(uint32_t stored_rows) { return (stored_rows / 16 + kTilesN - 1) / kTilesN; }
 
 }  // namespace
 
-// While its blocks are fewer than the compute units hold, a GEMM here takes one block's chain of groups, 0.7 us each however few
-// the rows (a group's round trip), where the library's two take 22 us and 12.5 us per 1,000 rows and 10^6 weights of a
-// projection: the lines cross where rows * d f / 10^6 is 68 times the groups of both products less 2,000 (fitted at 18
-// widths, GPU time). Library form | this one, us: 2,816 -> 2,112, 576 rows 65 | 67, 704 rows 76 | 70, 3,072 rows 248 | 178; 2,816
-// -> 704, 640 rows 41 | 50, 896 rows 53 | 52; 1,024 -> 2,816, 704 rows 52 | 57, 896 rows 59 | 59, 1,024 rows 67 | 60; 2,816 -> 2,816,
-// 576 rows 78 | 77; 512 -> 512, 640 rows 24 | 22. Not below 640 rows, where the forms meet at the widest, nor beyond 1,024, where
-// the narrowest (2,816 -> 256, 38 | 47) still cross, but in a call that the library's own 41 us on the host bound.
+// While its items are fewer than the compute units, a GEMM here takes one item's chain of groups however few the rows, where the
+// library's two take 22 us and 12.5 us per 1,000 rows and 10^6 weights of a projection: the lines cross where rows * d f / 10^6 is 68
+// times the groups of both products less 2,000 (fitted at 18 widths, GPU time, when a group of the chain took 0.7 us). A group is
+// 0.5 us now and the forms cross lower: library form | this one, us: 2,816 -> 2,112, 704 rows 76 | 56, 3,072 rows 248 | 140; 2,816 ->
+// 704, 1,024 rows 55 | 45; 1,024 -> 2,816, 1,024 rows 67 | 50. The line stays: a chunk keeps the form, and with it the bits, that
+// it had. Not below 640 rows, where the forms met at the widest, nor beyond 1,024, where the narrowest (2,816 -> 256) still
+// crossed, but in a call that the library's own 41 us on the host bound.
 uint32_t dense8_min_rows(uint32_t d, uint32_t f) {
     const uint32_t groups = all_groups_of(d) + all_groups_of(f);
     const uint64_t line = groups * 68ull <= 2000ull ? 0 : (groups * 68ull - 2000ull) * 1000000ull / ((uint64_t)d * f);
@@ -363,24 +434,31 @@ hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t store
     const uint32_t n_blocks = n_blocks_of(stored_rows), row_blocks = (t + 15) / 16;
     const float *scales = reinterpret_cast<const float *>(static_cast<const uint8_t *>(weights) +
                                                           (size_t)n_blocks * all_groups_of(n) * (kBFrags * kWave * sizeof(uint4)));
-    // Tiles of 64 rows while a compute unit holds few of them: 128-row tiles halve the weights' way through LDS but leave a
-    // chip that is not full to fewer blocks. The line is drawn on the XCD that has the most N-blocks (all row tiles of one run
-    // there), at blocks of 64 rows per compute unit: 3 for the gated product, 1.75 for the plain one. Whole FFN,
-    // 64 | 128 rows per tile in both products, us: 2,816 -> 2,112 -> 2,816, 640 rows (1.6 and 0.9 blocks) 72 | 78, 1,024 rows
-    // (2.5, 1.5) 88 | 91, 1,280 rows (3.1, 1.9) 114 | 94, 3,072 rows 222 | 186; 2,816 -> 704, 1,024 rows (1, 1.5) 52 | 61, 2,048
-    // rows (2, 3) 66 | 67; 704 -> 2,816, 1,152 rows (3.4, 0.6) 63 | 66, and 58 with 128 gated and 64 plain; 512 -> 512, 2,048
-    // rows (1, 1) 26 | 30. Either gives the same bits.
-    const uint32_t m64 = (row_blocks + 3) / 4;
-    const bool small = 4 * ((n_blocks + 7) / 8) * m64 <= (gated ? 12u : 7u) * (n_cus / 8);
-    const uint32_t tile_blocks = small ? 4 : 8, m_tiles = (row_blocks + tile_blocks - 1) / tile_blocks;
-    const dim3 grid(8 * ((n_blocks + 7) / 8) * m_tiles);
-#define FFMOE_DENSE8(N, W)                                                                                                              \
-    hipLaunchKernelGGL((gated ? (f16 ? dense8_gemm_kernel<true, N, W, true> : dense8_gemm_kernel<true, N, W, false>)                      \
-                              : (f16 ? dense8_gemm_kernel<false, N, W, true> : dense8_gemm_kernel<false, N, W, false>)),                  \
-                       grid, dim3(256), 0, s, static_cast<const uint16_t *>(weights), scales, n / kGroup, n_blocks, stored_rows,          \
-                       static_cast<const uint16_t *>(ops), t, static_cast<uint16_t *>(out), out_stride)
-    if (small) FFMOE_DENSE8(2, 2);
-    else FFMOE_DENSE8(2, 1);
+    const uint32_t nm = dense8_blocks(row_blocks, (n_blocks + 1) / 2, n_cus), all = (row_blocks + nm - 1) / nm * ((n_blocks + 1) / 2);
+    const dim3 grid((all + 7) / 8 * 8);
+    auto launch = [&](auto blocks) {
+        constexpr int N = decltype(blocks)::value;
+        hipLaunchKernelGGL((gated ? (f16 ? dense8_gemm_kernel<true, N, true> : dense8_gemm_kernel<true, N, false>)
+                                  : (f16 ? dense8_gemm_kernel<false, N, true> : dense8_gemm_kernel<false, N, false>)),
+                           grid, dim3(64 * kWaves8), 0, s, static_cast<const uint8_t *>(weights), scales, n / kGroup, n_blocks, stored_rows,
+                           static_cast<const uint8_t *>(ops), t, static_cast<uint16_t *>(out), out_stride);
+    };
+#define FFMOE_DENSE8(N) case N: launch(std::integral_constant<int, N>{}); break
+    switch (nm) {
+        FFMOE_DENSE8(3);
+        FFMOE_DENSE8(4);
+        FFMOE_DENSE8(5);
+        FFMOE_DENSE8(6);
+        FFMOE_DENSE8(7);
+        FFMOE_DENSE8(8);
+        FFMOE_DENSE8(9);
+        FFMOE_DENSE8(10);
+        FFMOE_DENSE8(11);
+        FFMOE_DENSE8(12);
+        FFMOE_DENSE8(13);
+        FFMOE_DENSE8(14);
+        default: launch(std::integral_constant<int, 15>{}); break;
+    }
 #undef FFMOE_DENSE8
     return hipGetLastError();
 }

@@ -142,3 +142,35 @@ def test_the_gemms_in_a_graph(oracle, act, t):
             torch.cuda.synchronize()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+# every number of 16-row blocks per tile (3 to 15) in both products, last tiles of one block and more; odd numbers of 128-row blocks
+@pytest.mark.parametrize("d,f,rows", [(448, 2112, (1024, 1206, 1457, 1682, 1927, 2165, 2403, 2657, 2886, 3124, 3377)),
+                                      (2112, 448, (1025, 1346, 1794, 2242, 2691, 3138, 3586, 4034, 4482, 4930, 5378, 5826)),
+                                      (704, 1408, (1024, 1108)), (2816, 64, (5154,))])
+def test_tiles_of_the_row_count(oracle, act, d, f, rows):
+    # the largest chunk against 64-bit products (first and last rows), every other one, cut elsewhere, to the same bits
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    g, int8, _ = _parts(oracle, d, f, f"dense8-tiles-{d}")
+    t = max(rows)
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    x = torch.from_numpy((g.uniform(-1.0, 1.0, t * d) + 0.25).reshape(t, d).astype(np.float32)).to(dt)
+    ctx = ff.Context(d, f, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_expert_parts(0, 0, *int8, int8=True)
+        y = ctx.dense_ffn(0, x.cuda())
+        some = np.r_[0:260, t - 260:t]
+        gw, uw, dw = (oracle.dequantize_int8(*p).astype(np.float64) for p in int8)
+        xf = x[some].double().numpy()
+        rnd = lambda a: torch.from_numpy(a).to(torch.float32).to(dt).double().numpy()
+        a = rnd(_gelu(rnd(xf @ gw.T)) * rnd(xf @ uw.T))
+        ref, spread = a @ dw.T, np.abs(a) @ np.abs(dw.T)
+        unit = 2.0 ** (-8 if act == "bf16" else -11)         # the bound of test_rows_against_float64
+        assert np.all(np.abs(y[some].float().cpu().numpy() - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
+        for n in rows:
+            assert torch.equal(ctx.dense_ffn(0, x[:n].cuda()), y[:n]), n
+    finally:
+        ctx.close()
