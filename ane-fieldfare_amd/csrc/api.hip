@@ -35,13 +35,13 @@ struct ffmoe_layer {
     uint8_t *gate_up8_ops = nullptr, *down8_ops = nullptr;
 };
 
-// From this many rows on an 8-bit dense layer goes through the library's dense GEMM on hi / lo rows instead of one
-// streaming pass per 16 rows (measured at 2816 -> 2112 -> 2816: streaming 19 us at 32 rows + 8.8 us per 32 more, 42 us at
-// 127; the GEMM form 50 us at 128, 58 at 192, 67 at 256, 100 at 1,024, 244 at 3,072).
+// From this many rows on an 8-bit dense layer goes through the library's dense GEMM on hi / lo rows instead of the resident-matrix
+// products (drawn where those were a pass per 16 rows, and kept with the bits on either side: 2,816 -> 2,112 -> 2,816, 190 rows 43 us
+// in bands of rows, 66 in passes; the GEMM form 50 us at 128, 58 at 192, 67 at 256).
 constexpr uint32_t kGemm8MinRows = 192;
-// Up to this many rows a 4-bit dense layer streams its arena tiles through the resident-matrix GEMV (a grid row per 16
-// input rows) instead of the grouped products (which beat it from about 200 rows on in bf16 and 370 in FP16: 384 rows 66 us
-// against 45 and 64; the rows of a chunk and of a part of it are equal bit for bit up to here, so the line stays put).
+// Up to this many rows a 4-bit dense layer takes the resident-matrix products on its arena tiles (bands of input rows) instead of
+// the grouped products: 2,816 -> 2,112 -> 2,816, 301 rows 39 us against 41 in bf16 and 58 in FP16, 384 rows 46 against 45 and 63.
+// The rows of a chunk and of a part of it are equal bit for bit up to here.
 constexpr uint32_t kDenseStreamMaxRows = 384;
 
 // A resident matrix: the re-tiled copy of one [m][n] INT4 weight plus the scratch of its greedy choice.
@@ -886,8 +886,7 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
             ctx->timer.finish();
             return FFMOE_OK;
         }
-        // two launches whatever the row count: a grid row per 16 input rows, each a pass of its own over the weights
-        // (from the caches after the first); the activation rows of a block of more than 16 go to the prefill scratch
+        // two launches whatever the row count; the activation rows of a block of more than 16 go to the prefill scratch
         uint16_t *acts = t <= FFMOE_MAX_VERIFY_ROWS ? ctx->acts : ctx->pf.acts;
         ctx->timer.begin(s);
         FF_HIP(launch_matrix_gemv(s, l.gate_up8->tiles, l.gate_up8->scales, ctx->shape.f, ctx->shape.d, x, x_stride, t, acts,
@@ -908,7 +907,7 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
         // 17 rows to a few hundred (a short prompt, a chunk's ragged end): below the row count at which the grouped GEMMs'
         // fixed cost (the weights' expansion per M-tile) is paid back, the resident-matrix GEMV streams the expert's arena
         // tiles as they lie - a gate/up tile's two streams are a gate and an up row block, a down tile is a plain 4-bit
-        // matrix tile - with one grid row per 16 input rows: two launches.
+        // matrix tile - in bands of input rows: two launches.
         if (int rc = check_layer(ctx, layer, true, false, err)) return rc;
         const uint32_t cap = std::max<uint32_t>(ctx->shape.max_tokens, FFMOE_MAX_VERIFY_ROWS);
         if (!x || t > cap) return fail(err, FFMOE_ERR_INVALID, "t = %u exceeds max_tokens = %u", t, cap);

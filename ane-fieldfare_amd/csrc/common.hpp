@@ -154,6 +154,11 @@ template <int IN_FLIGHT> __device__ __forceinline__ void vmem_barrier() {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IN_FLIGHT) : "memory");
 }
 
+// The same where what the block reads of LDS next may be written by such loads: nobody's reads are under way either.
+template <int IN_FLIGHT> __device__ __forceinline__ void ring_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(IN_FLIGHT) : "memory");
+}
+
 // Global memory to LDS with no register in between: lane l's 16 (4) bytes go to LDS byte `to` + 16 l (4 l), `to` wave-uniform.
 // Inline, because the compiler otherwise waits for every such load in front of the next LDS read, whatever buffer that reads;
 // the caller waits (vmem_barrier) before anything of the block reads the data.

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * kWaves8, 2) void dense8_gemm_kernel(const uint
         for (int f = 0; f < kFrags; ++f) {
             const int i = f >> 1, kh = f & 1, ahead = f + kQueue - 1;
             if (f == kBarrier) {
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory");
+                ring_barrier<kLoads>();
                 read_w(slot ^ 1);
 #pragma unroll
                 for (int n = 0; n < kLate; ++n) read_a(next, n);

@@ -177,13 +177,9 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     __shared__ float s_red[2][kKSplit][8][64];
     static_assert(!(PLANES8 && GREEDY), "the greedy choice is built for the 4-bit head only");
     static_assert((GLU == 1) ? PLANES8 : true, "tile pairs are the 8-bit planes' gated form");
-    static_assert((GLU == 2) ? !PLANES8 && !GREEDY : true, "gate and up as a tile's two streams is the 4-bit gated form");
-    // GLU == 2: a 4-bit tile's stream A holds 16 rows of a gate projection and its stream B the same rows of the up
-    // projection - the expert arena's gate/up tiles - and `m` counts the outputs gelu_tanh(gate . x) * (up . x), both sums
-    // fp32 in front of the activation as in the expert kernels (moe.metal:496).
     // GLU == 1: tiles 2 p and 2 p + 1 hold rows 16 p ... 16 p + 15 of a gate and of an up projection; a block takes whole
     // pairs, and `m` counts the outputs gelu_tanh(gate . x) * (up . x)
-    const uint32_t n_tiles = GLU == 1 ? 2 * ((m + 15) / 16) : (PLANES8 || GLU == 2) ? (m + 15) / 16 : (m + 31) / 32;
+    const uint32_t n_tiles = GLU == 1 ? 2 * ((m + 15) / 16) : PLANES8 ? (m + 15) / 16 : (m + 31) / 32;
     uint32_t rb0, rb1;
     split_range(GLU == 1 ? n_tiles / 2 : n_tiles, gridDim.x, blockIdx.x, rb0, rb1);
     if (GLU == 1) {
@@ -202,15 +198,6 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     const uint32_t g_last = g1 > g0 ? g1 - 1 : n_groups - 1;
     const TileSource src = make_tile_source(tiles, (size_t)n_tiles * n_groups * kTileBytes, scales,
                                             (size_t)n_tiles * n_groups * kTileScaleBytes);
-    // more than 16 input rows (the plain forms only): grid row y takes rows 16 y ... 16 y + 15 - the same pass over the
-    // weights again, which then come from the caches
-    if (!GREEDY && blockIdx.y != 0) {
-        x += (size_t)blockIdx.y * FFMOE_MAX_VERIFY_ROWS * x_stride;
-        y_ = Y_F32 ? static_cast<void *>(reinterpret_cast<float *>(y_) + (size_t)blockIdx.y * FFMOE_MAX_VERIFY_ROWS * y_stride)
-                   : static_cast<void *>(reinterpret_cast<uint16_t *>(y_) + (size_t)blockIdx.y * FFMOE_MAX_VERIFY_ROWS * y_stride);
-    }
-    if (!GREEDY) rows = min((uint32_t)FFMOE_MAX_VERIFY_ROWS, rows - blockIdx.y * FFMOE_MAX_VERIFY_ROWS);
-
     WeightRing ring;
 #pragma unroll
     for (int u = 0; u < kRing; ++u) ring_fill(ring, u, src, rb0 * n_groups + min(g0 + u, g_last), lane);
@@ -251,14 +238,7 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
             va += s_red[buf][o][ks][lane];
             vb += s_red[buf][o][4 + ks][lane];
         }
-        if (GLU == 2) {
-            const uint32_t col = rb * kTileRows + j;
-            if (my_row < rows && col < m) {
-                const float act = gelu_tanh_fast(va) * vb;
-                if (Y_F32) y32[(size_t)my_row * y_stride + col] = act;
-                else y16[(size_t)my_row * y_stride + col] = Act<F16>::round(act);
-            }
-        } else if (GLU == 1) {
+        if (GLU == 1) {
             // both projections are rounded to 16 bits in front of the activation, as shared_int8_gate_up_act_simd does
             // (Metal/Quant/dequant_int8.metal:131-136) and as two separate calls with the activation between them would
             const float v = Act<F16>::widen(Act<F16>::round(va + vb));
@@ -307,6 +287,197 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
 #pragma unroll
             for (int mk = 8; mk >= 1; mk >>= 1) soft = softmax_merge(soft, softmax_shuffle(soft, mk));
             if (j == 0 && my_row < rows) conf_part[(size_t)my_row * gridDim.x + blockIdx.x] = make_float2(soft.m, soft.s);
+        }
+    }
+}
+
+// The same sums for more than 16 input rows, 16 R of them per block: there the GEMV's grid rows each read the weights and every
+// block its input rows again. A block has 8 / PARTS tiles and PARTS parts of K, a wave one of each: it expands a tile's nibbles
+// once for R blocks of rows. The rows of all parts and the waves' tiles go straight into LDS, a ring of chunks of one or two
+// groups ahead (all scales at once: a load of them per group takes the address unit as long as one of a tile); rows in
+// 128-byte lines whose 16-byte piece c lies at c ^ (row % 8), so that the sixteen rows of an operand fall on different
+// banks. A part of K is one or two of the GEMV's slices of K: each is summed by itself and the four are added in its order, so
+// that a row has the GEMV's bits.
+// GLU == 2: a 4-bit tile's stream A holds 16 rows of a gate projection and its stream B the same rows of the up projection - the
+// expert arena's gate/up tiles - and `m` counts the outputs gelu_tanh(gate . x) * (up . x), both sums fp32 in front of the
+// activation as in the expert kernels (moe.metal:496). GLU == 1 and PLANES8 as in the GEMV.
+// Bound: up to some 100 rows the chain of groups of one item (0.36 us each at one block of rows: the barrier, the expansion,
+// the products and their sums one behind the other), beyond that the products and the sums themselves, a third of the products
+// being the inputs' own sums, which every wave makes anew. Kept out, as they change nothing: the sums between the products or
+// behind six of them, with and without a raised wave priority. 2,816 -> 2,112 -> 2,816, 4 bits, us of gate/up + down with the GEMV's
+// passes of 16 rows | now: 17 rows 10 + 7 | 9 + 8, 96 rows 17 + 12 | 12 + 10, 190 rows 28 + 18 | 17 + 12, 301 rows 39 + 24 | 22 +
+// 17, 384 rows 46 + 29 | 25 + 20; 8 bits, 37 rows 14 + 13 | 14 + 10, 190 rows 36 + 30 | 25 + 20.
+constexpr int kBandWaves = 8, kBandMax = 5;
+template <int PARTS, int R> struct Band {
+    static constexpr int tiles = kBandWaves / PARTS, slices = kKSplit / PARTS;
+    static constexpr int groups = R <= 3 ? 2 : 1;                                   // of a chunk
+    static constexpr int scale_loads = (slices * kRing * kTileScaleBytes + 1023) / 1024;
+    static constexpr uint32_t x_bytes = PARTS * R * 2048, group_bytes = x_bytes + kBandWaves * kTileBytes;
+    static constexpr uint32_t scales_at = 0, ring_at = kBandWaves * scale_loads * 1024, chunk_bytes = groups * group_bytes;
+    static constexpr int room = (int)((160 * 1024 - ring_at) / chunk_bytes), depth = room < 6 ? room : 6;
+    static constexpr uint32_t bytes = ring_at + depth * chunk_bytes;
+    static constexpr int x_loads = (2 * R + tiles - 1) / tiles, loads = groups * (x_loads + 1);     // per wave and chunk
+};
+
+template <bool F16, bool PLANES8, int GLU, int PARTS, int R>
+__global__ __launch_bounds__(64 * kBandWaves, 2) void matrix_band_kernel(const uint8_t *__restrict__ tiles, const uint8_t *__restrict__ scales,
+                                                                         uint32_t m, uint32_t n_groups, const uint16_t *__restrict__ x,
+                                                                         uint32_t x_stride, uint32_t rows, uint16_t *__restrict__ y,
+                                                                         uint32_t y_stride) {
+    using B = Band<PARTS, R>;
+    static_assert(B::depth >= 2, "a chunk in use and one on its way");
+    static_assert(B::tiles * (kKSplit - B::slices) * R * 8 * kWave * sizeof(float) <= B::bytes, "the other parts' sums fit");
+    __shared__ __align__(16) uint8_t lds[B::bytes];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, jq = lane >> 4;
+    const uint32_t unit = wave % B::tiles, part = wave / B::tiles;
+    const uint32_t n_tiles = GLU == 1 ? 2 * ((m + 15) / 16) : (PLANES8 || GLU == 2) ? (m + 15) / 16 : (m + 31) / 32;
+    // the items tile set by tile set, an eighth of the list per XCD: each reads its eighth of the weights into its L2 once
+    const uint32_t bands = ((rows + 15) / 16 + R - 1) / R, all = bands * ((n_tiles + B::tiles - 1) / B::tiles);
+    const uint32_t xcd = blockIdx.x & 7, item = (uint32_t)((uint64_t)all * xcd / 8) + (blockIdx.x >> 3);
+    if (item >= (uint32_t)((uint64_t)all * (xcd + 1) / 8)) return;
+    const uint32_t row0 = item % bands * (16 * R), tile = item / bands * B::tiles + unit;
+    const size_t at = (size_t)min(tile, n_tiles - 1) * n_groups;              // (past the last tile the last again, not stored)
+    const uint8_t *const w_tiles = tiles + at * kTileBytes, *const w_scales = scales + at * kTileScaleBytes;
+    const uint32_t per = (n_groups + kKSplit - 1) / kKSplit, g0 = part * B::slices * per, steps = B::slices * per;
+    // the scales of the part's groups (past the last group the last bytes again, not used)
+    const uint32_t scales_lds = wave * (B::scale_loads * 1024);
+#pragma unroll
+    for (int k = 0; k < B::scale_loads; ++k)
+        global_to_lds_16(w_scales, min(g0 * kTileScaleBytes + k * 1024 + lane * 16, n_groups * kTileScaleBytes - 16), lds_base + B::scales_at + scales_lds + k * 1024);
+    const uint16_t *from[B::x_loads];
+    uint32_t to[B::x_loads];
+#pragma unroll
+    for (int k = 0; k < B::x_loads; ++k) {
+        // 8 rows x 128 bytes per load (what does not divide by the waves, the last piece twice; rows past the last, the last)
+        const uint32_t piece = min(unit + B::tiles * k, 2u * R - 1), row = min(row0 + piece * 8 + (lane >> 3), rows - 1);
+        from[k] = x + (size_t)row * x_stride + 8 * ((lane & 7) ^ (lane >> 3));
+        to[k] = part * (R * 2048) + piece * 1024;
+    }
+    auto load = [&](uint32_t step, uint32_t slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < B::groups; ++c) {
+            const uint32_t grp = min(g0 + step + c, n_groups - 1), base = lds_base + slot + c * B::group_bytes;      // (past the last: read, not used)
+            global_to_lds_16(w_tiles + (size_t)grp * kTileBytes, lane * 16, base + B::x_bytes + wave * kTileBytes);
+#pragma unroll
+            for (int k = 0; k < B::x_loads; ++k) global_to_lds_16(from[k] + grp * kGroup, base + to[k]);
+        }
+    };
+    TwoStreamAcc tot[B::slices][R];
+    TwoStreamAcc sum[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        sum[i].a = sum[i].b = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < B::slices; ++q) tot[q][i].a = tot[q][i].b = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const uint32_t x_at = part * (R * 2048) + j * 128 + 16 * (jq ^ (j & 7));
+#pragma unroll
+    for (int d = 0; d < B::depth - 1; ++d) load(d * B::groups, B::ring_at + d * B::chunk_bytes);
+    uint32_t slot = B::ring_at, before = B::ring_at + (B::depth - 1) * B::chunk_bytes;
+#pragma nounroll
+    for (uint32_t s = 0; s < steps; s += B::groups) {
+        ring_barrier<(B::depth - 2) * B::loads>();          // this chunk's loads are there, and nobody reads the one before any more
+        load(s + (B::depth - 1) * B::groups, before);
+#pragma unroll
+        for (int c = 0; c < B::groups; ++c) {
+            if (B::slices == 2 && s + c == per) {
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    tot[0][i] = sum[i];
+                    sum[i].a = sum[i].b = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+            if (s + c >= steps || g0 + s + c >= n_groups) continue;        // wave-uniform: the last slices may be short
+            const uint8_t *const here = lds + slot + c * B::group_bytes;
+            const uint4 t = *reinterpret_cast<const uint4 *>(here + B::x_bytes + wave * kTileBytes + lane * 16);
+            const uint2 sc = *reinterpret_cast<const uint2 *>(lds + B::scales_at + scales_lds + (s + c) * kTileScaleBytes + j * 8);
+            const uint4 a0 = unpack8_offset<F16>(t.x), a1 = unpack8_offset<F16>(t.y), b0 = unpack8_offset<F16>(t.z), b1 = unpack8_offset<F16>(t.w);
+            const float sa = bf16lo_to_f32(sc.x), ba = bf16hi_to_f32(sc.x), sb = bf16lo_to_f32(sc.y), bb = bf16hi_to_f32(sc.y);
+            const float ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ba), tb = __builtin_fmaf(-Act<F16>::kOffset, sb, bb);
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const uint4 x0 = *reinterpret_cast<const uint4 *>(here + x_at + i * 2048), x1 = *reinterpret_cast<const uint4 *>(here + (x_at ^ 64) + i * 2048);
+                const f32x4 sx = group_input_sum<F16>(x0, x1);
+                const f32x4 acc_a = Act<F16>::mfma(x1, a1, Act<F16>::mfma(x0, a0, zero)), acc_b = Act<F16>::mfma(x1, b1, Act<F16>::mfma(x0, b0, zero));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sum[i].a[r] = __builtin_fmaf(ta, sx[r], __builtin_fmaf(sa, acc_a[r], sum[i].a[r]));
+                    sum[i].b[r] = __builtin_fmaf(tb, sx[r], __builtin_fmaf(sb, acc_b[r], sum[i].b[r]));
+                }
+            }
+        }
+        before = slot;
+        slot = slot + B::chunk_bytes == B::bytes ? B::ring_at : slot + B::chunk_bytes;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) tot[B::slices - 1][i] = sum[i];
+    vmem_barrier<0>();                                      // no load is on its way into what follows
+    lds_barrier();
+    // the later parts' slices to the first part's waves
+    constexpr int kOthers = kKSplit - B::slices;
+    float *const sums = reinterpret_cast<float *>(lds) + unit * (kOthers * R * 8 * kWave) + lane;
+    if (part) {
+#pragma unroll
+        for (int q = 0; q < B::slices; ++q)
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float *const to_q = sums + (((part - 1) * B::slices + q) * R + i) * (8 * kWave);
+                    to_q[r * kWave] = tot[q][i].a[r];
+                    to_q[(4 + r) * kWave] = tot[q][i].b[r];
+                }
+    }
+    lds_barrier();
+    if (!part) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float va = tot[0][i].a[r], vb = tot[0][i].b[r];
+                if (B::slices == 2) va += tot[B::slices - 1][i].a[r], vb += tot[B::slices - 1][i].b[r];
+#pragma unroll
+                for (int q = 0; q < kOthers; ++q) {
+                    va += sums[(q * R + i) * (8 * kWave) + r * kWave];
+                    vb += sums[(q * R + i) * (8 * kWave) + (4 + r) * kWave];
+                }
+                const uint32_t row = row0 + i * 16 + 4 * jq + r;
+                uint16_t *const yr = y + (size_t)row * y_stride;
+                if (GLU == 1) {
+                    // gate or up, rounded as the GEMV rounds them; the pair's other wave has the other
+                    sums[i * (8 * kWave) + r * kWave] = Act<F16>::widen(Act<F16>::round(va + vb));
+                } else if (row < rows && tile < n_tiles) {
+                    if (GLU == 2) {
+                        const uint32_t col = tile * kTileRows + j;
+                        if (col < m) yr[col] = Act<F16>::round(gelu_tanh_fast(va) * vb);
+                    } else if (PLANES8) {
+                        const uint32_t col = tile * kTileRows + j;
+                        if (col < m) yr[col] = Act<F16>::round(va + vb);
+                    } else {
+                        const uint32_t col = tile * 2 * kTileRows + j;
+                        if (col < m) yr[col] = Act<F16>::round(va);
+                        if (col + kTileRows < m) yr[col + kTileRows] = Act<F16>::round(vb);
+                    }
+                }
+            }
+    }
+    if (GLU == 1) {
+        lds_barrier();
+        if (part || tile >= n_tiles) return;
+        // both waves of a pair have both projections in reach: each finishes every other of its rows' blocks of 16
+        const float *const gate = reinterpret_cast<const float *>(lds) + (unit & ~1u) * (kOthers * R * 8 * kWave) + lane, *const up = gate + kOthers * R * 8 * kWave;
+        const uint32_t col = (tile >> 1) * kTileRows + j;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if ((i & 1) != (int)(unit & 1)) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t row = row0 + i * 16 + 4 * jq + r;
+                const float act = gelu_tanh_fast(gate[i * (8 * kWave) + r * kWave]) * up[i * (8 * kWave) + r * kWave];
+                if (row < rows && col < m) y[(size_t)row * y_stride + col] = Act<F16>::round(act);
+            }
         }
     }
 }
@@ -462,6 +633,25 @@ size_t matrix_tiles_bytes(uint32_t m, uint32_t n, bool planes8) {
 size_t matrix_scales_bytes(uint32_t m, uint32_t n, bool planes8) {
     return (size_t)(planes8 ? (m + 15) / 16 : (m + 31) / 32) * (n / kGroup) * kTileScaleBytes;
 }
+// Parts of K per block and 16-row blocks per band: the pair whose rounds of items over the compute units cost least, an item's
+// time being 5 us + 0.18 us per group of its chain and (row block + 1). 2,816 -> 2 x 2,112 gated, 4 bits, us at parts.blocks: 37 rows
+// 4.1 9, 4.3 14, 2.1 13; 96 rows 4.1 17 (two rounds), 4.2 12, 2.1 14; 190 rows 4.3 25, 2.2 17, 2.3 22; 301 rows 4.3 26, 2.3 22, 2.4
+// 25; 384 rows 2.3 38, 2.4 25. Any gives the same bits.
+struct BandShape {
+    uint32_t parts, blocks;
+};
+static BandShape band_shape(uint32_t rows, uint32_t n_tiles, uint32_t n_groups, uint32_t n_cus) {
+    const uint32_t row_blocks = (rows + 15) / 16, per = (n_groups + kKSplit - 1) / kKSplit;
+    BandShape best = {2, kBandMax};
+    uint64_t least = ~0ull;
+    for (uint32_t parts = 4; parts >= 2; parts -= 2)
+        for (uint32_t r = 1; r <= (parts == 4 ? 3u : (uint32_t)kBandMax); ++r) {
+            const uint32_t per_block = kBandWaves / parts, items = (row_blocks + r - 1) / r * ((n_tiles + per_block - 1) / per_block);
+            const uint64_t cost = (uint64_t)((items + n_cus - 1) / n_cus) * (28 + kKSplit / parts * per * (1 + r));
+            if (cost < least) least = cost, best = BandShape{parts, r};
+        }
+    return best;
+}
 bool matrix_shape_ok(uint32_t n) { return n % kGroup == 0 && (n / kGroup + kKSplit - 1) / kKSplit <= (uint32_t)kRing; }
 
 hipError_t launch_matrix_repack(hipStream_t s, const uint8_t *w, const uint16_t *scales, const uint16_t *biases,
@@ -480,20 +670,44 @@ hipError_t launch_matrix_repack(hipStream_t s, const uint8_t *w, const uint16_t 
 hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t *scales, uint32_t m, uint32_t n,
                               const uint16_t *x, uint32_t x_stride, uint32_t rows, void *y, uint32_t y_stride,
                               bool y_f32, uint32_t n_cus, bool f16, bool planes8, int glu) {
-    // glu: 0 plain, 1 the 8-bit planes' tile pairs, 2 a 4-bit tile's two streams as gate and up (m = the gated outputs)
+    // glu: 0 plain, 1 the 8-bit planes' tile pairs, 2 a 4-bit tile's two streams as gate and up (m = the gated outputs; more than 16
+    // rows: up to there such a matrix is an expert's and takes the expert kernels)
     if (glu == 2 && (planes8 || y_f32)) return hipErrorInvalidValue;
     const uint32_t n_tiles = (planes8 || glu == 2) ? (m + 15) / 16 : (m + 31) / 32;      // glu == 1: pairs of tiles
-    if (rows == 0 || (rows + FFMOE_MAX_VERIFY_ROWS - 1) / FFMOE_MAX_VERIFY_ROWS > 65535u) return hipErrorInvalidValue;
-    dim3 grid(min(2 * n_cus, n_tiles), (rows + FFMOE_MAX_VERIFY_ROWS - 1) / FFMOE_MAX_VERIFY_ROWS);
-    // several grid rows: a multiple of 8 blocks per row keeps a tile on one XCD (blocks go to the XCDs round robin), whose L2
-    // then serves every pass after the first; the blocks past the tile count leave at once
-    if (grid.y > 1) grid.x = (grid.x + 7) / 8 * 8;
+    if (rows == 0 || rows > (1u << 20) || (rows > FFMOE_MAX_VERIFY_ROWS ? y_f32 : glu == 2)) return hipErrorInvalidValue;
+    const uint32_t all_tiles = glu == 1 ? 2 * n_tiles : n_tiles;
+    if (rows > FFMOE_MAX_VERIFY_ROWS) {
+        const BandShape shape = band_shape(rows, all_tiles, n / kGroup, n_cus);
+        const uint32_t bands = ((rows + 15) / 16 + shape.blocks - 1) / shape.blocks, per_block = kBandWaves / shape.parts;
+        const dim3 grid((bands * ((all_tiles + per_block - 1) / per_block) + 7) / 8 * 8);
+        auto launch = [&](auto parts, auto blocks) {
+            constexpr int P = decltype(parts)::value, N = decltype(blocks)::value;
+            auto kernel = glu == 2   ? (f16 ? matrix_band_kernel<true, false, 2, P, N> : matrix_band_kernel<false, false, 2, P, N>)
+                          : glu == 1 ? (f16 ? matrix_band_kernel<true, true, 1, P, N> : matrix_band_kernel<false, true, 1, P, N>)
+                          : planes8  ? (f16 ? matrix_band_kernel<true, true, 0, P, N> : matrix_band_kernel<false, true, 0, P, N>)
+                                     : (f16 ? matrix_band_kernel<true, false, 0, P, N> : matrix_band_kernel<false, false, 0, P, N>);
+            hipLaunchKernelGGL(kernel, grid, dim3(64 * kBandWaves), 0, s, tiles, scales, m, n / kGroup, x, x_stride, rows,
+                               static_cast<uint16_t *>(y), y_stride);
+        };
+#define FFMOE_BAND(P, N) launch(std::integral_constant<int, P>{}, std::integral_constant<int, N>{})
+        switch (shape.parts * 8 + shape.blocks) {
+            case 4 * 8 + 1: FFMOE_BAND(4, 1); break;
+            case 4 * 8 + 2: FFMOE_BAND(4, 2); break;
+            case 4 * 8 + 3: FFMOE_BAND(4, 3); break;
+            case 2 * 8 + 1: FFMOE_BAND(2, 1); break;
+            case 2 * 8 + 2: FFMOE_BAND(2, 2); break;
+            case 2 * 8 + 3: FFMOE_BAND(2, 3); break;
+            case 2 * 8 + 4: FFMOE_BAND(2, 4); break;
+            default: FFMOE_BAND(2, kBandMax); break;
+        }
+#undef FFMOE_BAND
+        return hipGetLastError();
+    }
+    const dim3 grid(min(2 * n_cus, n_tiles));
 #define FFMOE_MGEMV(Y, H, P, G)                                                                                             \
     hipLaunchKernelGGL((matrix_gemv_kernel<Y, H, false, false, P, G>), grid, dim3(256), 0, s, tiles, scales, m, n / kGroup, x, x_stride, \
                        rows, y, y_stride)
-    if (glu == 2) {
-        if (f16) FFMOE_MGEMV(false, true, false, 2); else FFMOE_MGEMV(false, false, false, 2);
-    } else if (glu == 1) {
+    if (glu == 1) {
         if (f16) { if (y_f32) FFMOE_MGEMV(true, true, true, 1); else FFMOE_MGEMV(false, true, true, 1); }
         else { if (y_f32) FFMOE_MGEMV(true, false, true, 1); else FFMOE_MGEMV(false, false, true, 1); }
     } else if (planes8) {
