@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kSortBlock) void prefill_hist_kernel(ItemSource src
     if (threadIdx.x < src.n_experts) block_cnt[(size_t)blockIdx.x * src.n_experts + threadIdx.x] = cnt[threadIdx.x];
 }
 
-// One block of 1024 threads: per expert, turn the per-block counts into per-block bases, then lay out the
+// For a block of 1024 threads: per expert, turn the per-block counts (in memory or LDS) into per-block bases, then lay out the
 // experts one after the other and cut each into M-tiles. Thread (expert e, chunk c) owns a contiguous run
 // of sort blocks, so the counts of a whole column are in flight at once and - up to kScanKeep per thread -
 // stay in registers between the summing pass and the pass that writes the bases.
@@ -71,11 +71,9 @@ constexpr int kScanThreads = 1024;
 // a run was read twice; short runs pay for the longer unrolled passes, 443.1 against 441.4 us for a plugin chunk of 3,079 rows)
 
 template <int kScanKeep>
-__global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad,
-                                                                    uint32_t *__restrict__ block_cnt,
-                                                                    PrefillPlan *__restrict__ plan,
-                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles,
-                                                                    uint32_t tile_shift) {
+__device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad, uint32_t *__restrict__ block_cnt,
+                                             PrefillPlan *__restrict__ plan, PrefillTile *__restrict__ tiles, uint32_t max_tiles,
+                                             uint32_t tile_shift) {
     const uint32_t bm = 1u << tile_shift;        // pairs per M-tile
     __shared__ uint32_t total[FFMOE_MAX_EXPERTS];
     __shared__ uint32_t offset[FFMOE_MAX_EXPERTS + 1];
@@ -104,7 +102,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
     __syncthreads();
     if (ch == 0 && live) {
         uint32_t run = 0;
-        for (uint32_t c = 0; c < chunks; ++c) {
+        for (uint32_t c = 0; c < min(chunks, n_blocks); ++c) {      // (the chunks behind hold nothing)
             const uint32_t v = part[c * e_pad + e];
             part[c * e_pad + e] = run;
             run += v;
@@ -176,7 +174,8 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
         }
     }
     __syncthreads();
-    if (!live) return;
+    const uint32_t n_pairs = offset[n_experts];
+    if (!live) return n_pairs;
     uint32_t run = offset[e] + part[threadIdx.x];
 #pragma unroll
     for (int u = 0; u < kScanKeep; ++u) {
@@ -188,7 +187,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
         block_cnt[(size_t)b * n_experts + e] = run;
         run += c;
     }
-    if (ch != 0) return;
+    if (ch != 0) return n_pairs;
     plan->expert_offset[e] = offset[e];
     plan->expert_count[e] = total[e];
     // a tile keeps its number in row order, which places its activation blocks
@@ -206,35 +205,33 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
             tiles[ti] = tl;
         }
     }
+    return n_pairs;
 }
 
-__global__ __launch_bounds__(kSortBlock) void prefill_scatter_kernel(ItemSource src, const uint32_t *__restrict__ block_base,
-                                                                     uint32_t *__restrict__ sorted_token,
-                                                                     uint32_t *__restrict__ sorted_out_row) {
-    // an item's place inside its block's share of its expert = the items of the same expert in front of it: those in
-    // the waves in front (per-wave counts in LDS) plus those in lower lanes of its own wave (a mask built from one
-    // ballot per bit of the expert number)
-    __shared__ uint32_t wave_cnt[kSortBlock / 64][FFMOE_MAX_EXPERTS];
+template <int kScanKeep>
+__global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad,
+                                                                    uint32_t *__restrict__ block_cnt,
+                                                                    PrefillPlan *__restrict__ plan,
+                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles,
+                                                                    uint32_t tile_shift) {
+    plan_experts<kScanKeep>(n_blocks, n_experts, e_pad, block_cnt, plan, tiles, max_tiles, tile_shift);
+}
+
+// The lanes of the wave whose item has this lane's expert: a mask built from one ballot per bit of the expert number.
+__device__ __forceinline__ unsigned long long same_expert(uint32_t e) {
     static_assert(FFMOE_MAX_EXPERTS <= 256, "eight ballots tell the experts apart");
-    const uint32_t i = blockIdx.x * kSortBlock + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t c = threadIdx.x; c < (kSortBlock / 64) * FFMOE_MAX_EXPERTS; c += kSortBlock) (&wave_cnt[0][0])[c] = 0;
-    const uint32_t e = item_expert(src, i);
-    const bool valid = e != 0xFFFFFFFFu;
-    unsigned long long same = __ballot(valid);
+    unsigned long long same = __ballot(e != 0xFFFFFFFFu);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
         const bool bit = (e >> b) & 1u;
         const unsigned long long with = __ballot(bit);
         same &= bit ? with : ~with;
     }
-    const uint32_t in_front = __popcll(same & ((1ull << lane) - 1ull));
-    __syncthreads();
-    if (valid && in_front == 0) wave_cnt[wave][e] = __popcll(same);
-    __syncthreads();
-    if (!valid) return;
-    uint32_t rank = in_front;
-    for (uint32_t v = 0; v < wave; ++v) rank += wave_cnt[v][e];
-    const uint32_t pos = block_base[(size_t)blockIdx.x * src.n_experts + e] + rank;
+    return same;
+}
+
+__device__ __forceinline__ void place_item(const ItemSource &src, uint32_t i, uint32_t pos, uint32_t *__restrict__ sorted_token,
+                                           uint32_t *__restrict__ sorted_out_row) {
     uint32_t token, out_row;
     if (src.pairs) {
         const ffmoe_pair p = src.pairs[i];
@@ -246,6 +243,76 @@ __global__ __launch_bounds__(kSortBlock) void prefill_scatter_kernel(ItemSource 
     }
     sorted_token[pos] = token;
     sorted_out_row[pos] = out_row;
+}
+
+// A chunk of few items in one launch: the three kernels' work by one block, the waves in place of the sort blocks - wave w has a
+// contiguous run of items, 64 at a time, and counts them in LDS; an item's place is what its wave counted before it. Same
+// order. Bound: latencies one behind the other, and 1.6 us per 1,024 items, which is why it ends at kSortKeep of them: a call with
+// three launches | with one, top-8 of 128, 37 rows 101.5 us | 99, 301 rows 133.7 | 131.9, 512 rows 160.9 | 161.2, 1,000 rows 191 | 196.
+constexpr int kSortWaves = kScanThreads / 64, kSortKeep = 3;
+__global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource src, uint32_t e_pad, PrefillPlan *__restrict__ plan,
+                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles,
+                                                                    uint32_t tile_shift, uint32_t *__restrict__ sorted_token,
+                                                                    uint32_t *__restrict__ sorted_out_row) {
+    __shared__ uint32_t sorted[kSortKeep * kScanThreads];
+    __shared__ uint32_t cnt[kSortWaves * FFMOE_MAX_EXPERTS];        // [wave][expert]: items counted so far, then the wave's base
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t runs = (src.n_items + kScanThreads - 1) / kScanThreads, first = wave * runs * 64 + lane;
+    uint32_t e[kSortKeep], rank[kSortKeep];
+#pragma unroll
+    for (int u = 0; u < kSortKeep; ++u) e[u] = (uint32_t)u < runs ? item_expert(src, first + u * 64) : 0xFFFFFFFFu;
+    for (uint32_t c = threadIdx.x; c < kSortWaves * src.n_experts; c += kScanThreads) cnt[c] = 0;
+    __syncthreads();
+    uint32_t *const own = cnt + wave * src.n_experts;
+#pragma unroll
+    for (int u = 0; u < kSortKeep; ++u) {
+        if ((uint32_t)u < runs) {
+            const unsigned long long same = same_expert(e[u]);
+            const uint32_t in_front = __popcll(same & ((1ull << lane) - 1ull));
+            // (a wave's LDS instructions run in order: the counts as they are in front of this run, then with it)
+            if (e[u] != 0xFFFFFFFFu) rank[u] = own[e[u]] + in_front;
+            __builtin_amdgcn_wave_barrier();
+            if (e[u] != 0xFFFFFFFFu && in_front == 0) atomicAdd(&own[e[u]], (uint32_t)__popcll(same));
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    __syncthreads();
+    const uint32_t n_pairs = plan_experts<4>(kSortWaves, src.n_experts, e_pad, cnt, plan, tiles, max_tiles, tile_shift);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSortKeep; ++u)
+        if ((uint32_t)u < runs && e[u] != 0xFFFFFFFFu) {
+            const uint32_t i = first + u * 64;
+            sorted[own[e[u]] + rank[u]] = src.pairs ? src.pairs[i].token * src.top_k + src.pairs[i].rank : i;
+        }
+    __syncthreads();
+    // in order in LDS, then out in whole lines
+    for (uint32_t p = threadIdx.x; p < n_pairs; p += kScanThreads) {
+        const uint32_t out_row = sorted[p];
+        sorted_token[p] = out_row / src.top_k;
+        sorted_out_row[p] = out_row;
+    }
+}
+
+__global__ __launch_bounds__(kSortBlock) void prefill_scatter_kernel(ItemSource src, const uint32_t *__restrict__ block_base,
+                                                                     uint32_t *__restrict__ sorted_token,
+                                                                     uint32_t *__restrict__ sorted_out_row) {
+    // an item's place inside its block's share of its expert = the items of the same expert in front of it: those in
+    // the waves in front (per-wave counts in LDS) plus those in lower lanes of its own wave
+    __shared__ uint32_t wave_cnt[kSortBlock / 64][FFMOE_MAX_EXPERTS];
+    const uint32_t i = blockIdx.x * kSortBlock + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t c = threadIdx.x; c < (kSortBlock / 64) * FFMOE_MAX_EXPERTS; c += kSortBlock) (&wave_cnt[0][0])[c] = 0;
+    const uint32_t e = item_expert(src, i);
+    const bool valid = e != 0xFFFFFFFFu;
+    const unsigned long long same = same_expert(e);
+    const uint32_t in_front = __popcll(same & ((1ull << lane) - 1ull));
+    __syncthreads();
+    if (valid && in_front == 0) wave_cnt[wave][e] = __popcll(same);
+    __syncthreads();
+    if (!valid) return;
+    uint32_t rank = in_front;
+    for (uint32_t v = 0; v < wave; ++v) rank += wave_cnt[v][e];
+    place_item(src, i, block_base[(size_t)blockIdx.x * src.n_experts + e] + rank, sorted_token, sorted_out_row);
 }
 
 // A dense FFN's chunk needs no sort: one expert, route r = row r. One launch writes what the three above would: the
@@ -1329,14 +1396,19 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
         hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, dense_rows, sc.plan, sc.tiles, sc.sorted_token,
                            sc.sorted_out_row);
     } else {
-        hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
         uint32_t e_pad = 1;
         while (e_pad < n_experts) e_pad <<= 1;          // n_experts <= FFMOE_MAX_EXPERTS = 256 <= kScanThreads
-        const uint32_t run = (n_blocks + kScanThreads / e_pad - 1) / (kScanThreads / e_pad);     // sort blocks per thread
-        hipLaunchKernelGGL((run <= 16 ? prefill_scan_kernel<16> : prefill_scan_kernel<32>), dim3(1), dim3(kScanThreads), 0, s, n_blocks,
-                           n_experts, e_pad, sc.block_cnt, sc.plan, sc.tiles, sc.max_tiles, tile_shift);
-        hipLaunchKernelGGL(prefill_scatter_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt, sc.sorted_token,
-                           sc.sorted_out_row);
+        if (src.n_items <= (uint32_t)kSortKeep * kScanThreads) {
+            hipLaunchKernelGGL(prefill_sort_kernel, dim3(1), dim3(kScanThreads), 0, s, src, e_pad, sc.plan, sc.tiles, sc.max_tiles, tile_shift,
+                               sc.sorted_token, sc.sorted_out_row);
+        } else {
+            hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
+            const uint32_t run = (n_blocks + kScanThreads / e_pad - 1) / (kScanThreads / e_pad);     // sort blocks per thread
+            hipLaunchKernelGGL((run <= 16 ? prefill_scan_kernel<16> : prefill_scan_kernel<32>), dim3(1), dim3(kScanThreads), 0, s, n_blocks,
+                               n_experts, e_pad, sc.block_cnt, sc.plan, sc.tiles, sc.max_tiles, tile_shift);
+            hipLaunchKernelGGL(prefill_scatter_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt, sc.sorted_token,
+                               sc.sorted_out_row);
+        }
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

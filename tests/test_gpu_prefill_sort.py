@@ -1,0 +1,46 @@
+"""The prefill's sort of routes in one launch (3,072 items and fewer) and in three: the same rows, bit for bit, from a chunk and from its
+beginning on either side of the line, counts per expert, routes of weight zero and experts past the last left out. Run on
+the GPU box: pytest -m gpu."""
+import numpy as np
+import pytest
+
+from helpers import make_layer, to_ff_offsets
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("e,k,cuts", [(128, 8, (1, 7, 8, 9, 128, 129, 383, 384)), (256, 2, (31, 32, 33, 511, 512, 513, 1535, 1536)),
+                                      (3, 1, (3000, 3071, 3072)), (5, 3, (1024,)), (200, 4, (255, 256, 257, 768))])
+def test_one_launch_sorts_as_three_do(oracle, e, k, cuts):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, t = 128, 64, 3072 // k + 5
+    rng, pool, _ = make_layer(oracle, 3 + e, d, f, e, align=1)
+    idx = np.stack([rng.permutation(e)[:k] for _ in range(t)]).astype(np.uint32)
+    w = rng.uniform(0.2, 1.0, (t, k)).astype(np.float32)
+    w[rng.random((t, k)) < 0.05] = 0
+    ctx = ff.Context(d, f, e, k, n_layers=1, max_tokens=t)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(torch.bfloat16).cuda()
+        gi, gw = torch.from_numpy(idx.view(np.int32)).cuda(), torch.from_numpy(w).to(torch.bfloat16).cuda()
+        def counts(n, routes):
+            live = (w[:n] > 0) & (routes[:n] < e)
+            return np.bincount(routes[:n][live], minlength=e)
+
+        whole = ctx.prefill(0, x, gi, gw)                       # 3,072 + 5 k items: three launches
+        assert torch.isfinite(whole.float()).all() and whole.abs().max() > 0
+        assert np.array_equal(ctx.prefill_stats()[2], counts(t, idx))
+        for n in cuts:                                          # (the same products as the whole chunk's: equal bit for bit)
+            part = ctx.prefill(0, x[:n], gi[:n].contiguous(), gw[:n].contiguous())
+            assert np.array_equal(ctx.prefill_stats()[2], counts(n, idx)), n
+            assert torch.equal(part, whole[:n]), n
+        past = idx.copy()
+        past[rng.random((t, k)) < 0.2] = e + 3
+        for n in (cuts[-1], t):
+            ctx.prefill(0, x[:n], torch.from_numpy(past[:n].view(np.int32)).cuda(), gw[:n].contiguous())
+            n_pairs, _, got = ctx.prefill_stats()
+            assert np.array_equal(got, counts(n, past)) and n_pairs == got.sum(), n
+    finally:
+        ctx.close()
