@@ -359,7 +359,7 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
 // wave multiplies its weights with), 26 LDS reads and one barrier. Run back to back the card also lowers its clock under it.
 // Weights through LDS instead (a wave expands a tile for all waves to read) costs the same however the waves split a block:
 // 215 to 235 us where this takes 183; 64 weight rows x 128 pairs per wave, every tile expanded twice, 209. Gate/up and down of a
-// 3,072-row chunk 222 + 115 -> 183 + 110 us, of 8,192 skewed rows 7.5 % less per layer, of 1,000 FP16 rows 144 + 78 -> 112 + 80; 256 pairs in each of 128
+// 3,072-row chunk 222 + 115 -> 183 + 110 us, of 8,192 skewed rows 7.5 % less per layer, of 1,000 FP16 rows 144 + 78 -> 114 + 68; 256 pairs in each of 128
 // experts 275 + 133 -> 216 + 137 us (1,200 TFLOP/s in gate/up). A second pass of bf16 products by the vendor's library on ready-made
 // weights reaches 1,250 on this card.
 // GATE_UP: A rows are gathered token rows of x; streams are gate / up; out = the activations, stored in the order the
@@ -386,13 +386,13 @@ constexpr uint32_t kFragBytes = kWave * 16;                 // one matrix operan
 constexpr uint32_t kGemmABytes = kBM / 16 * 2 * kFragBytes;
 constexpr uint32_t kGemmWBytes = kTileBytes + 2 * kTileScaleBytes;            // packed tile of one wave (a 64-lane load brings the scales twice)
 constexpr uint32_t kGemmWAt = kRingA * kGemmABytes, kGemmRowAt = kGemmWAt + kRingW * kGemmTiles * kGemmWBytes;
-// (down product: the pairs' output rows and largest scales, two items' worth, and the block scales of the groups of A)
-constexpr uint32_t kGemmRowBytes = kBM * 4, kGemmLargestAt = kGemmRowAt + 2 * kGemmRowBytes, kGemmRelAt = kGemmLargestAt + 2 * kGemmRowBytes;
+// (down product: the pairs' output rows and largest scales, two items' worth)
+constexpr uint32_t kGemmRowBytes = kBM * 4, kGemmLargestAt = kGemmRowAt + 2 * kGemmRowBytes;
 // the epilogues work in the buffer of the item's last group of A: the next item's first two are in the others
 constexpr int kTurnBlocks = 3;                              // 16-pair blocks that a wave turns at a time
 constexpr uint32_t kGemmTurnRow = 2 * kTileRows * 2 + 16, kGemmTurnBytes = 16 * kGemmTurnRow;
 static_assert(kGemmTiles * kTurnBlocks * kGemmTurnBytes <= kGemmABytes && kGemmTiles * kBM * 4 <= kGemmABytes, "staging rows or peaks fit a buffer");
-constexpr uint32_t gemm_lds_bytes(bool gate_up, bool f16) { return gate_up ? kGemmRowAt : f16 ? kGemmRelAt + kRingA * kGemmRowBytes : kGemmLargestAt; }
+constexpr uint32_t gemm_lds_bytes(bool gate_up, bool f16) { return gate_up ? kGemmRowAt : f16 ? kGemmLargestAt + 2 * kGemmRowBytes : kGemmLargestAt; }
 
 // One M-tile x N-block, and what a wave needs to ask for its rows: `from` = GATE_UP: in bytes from the first row's start (WIDE, where
 // the rows span 4 GiB or more: in 16-byte pieces); else: in KiB, wave-uniform.
@@ -422,9 +422,9 @@ constexpr int gemm_queue(int nm, int most) {
 // F16: the reference's FP16 prefill (prefill.metal:581-598,685-702,723-777): FP16 rows against FP16 tile weights
 // half(fma(q, scale, bias)), fp32 sums; the activations between the two GEMMs are FP16 with a power-of-two scale per
 // pair and 64-wide block of F (`act_scale[pair][block]`; the block's largest magnitude lands below 2^14), so values
-// past FP16's range keep FP16's relative precision; the down GEMM brings every block of a pair to the pair's largest
-// scale as it takes it in (exact unless a value falls below FP16's normal range relative to that largest) and
-// applies that scale to the pair's sums.
+// past FP16's range keep FP16's relative precision; a pass between the two brings every block of a pair to the pair's largest
+// scale (exact unless a value falls below FP16's normal range relative to that largest) and the down GEMM applies that scale
+// to the pair's sums.
 // Where a wave is in the rings, as byte offsets into LDS: they turn on from one item to the next.
 struct GemmRings {
     uint32_t cur, next, before;           // A of the group at hand, of the next one, of the one before (and of the group after the next)
@@ -443,14 +443,7 @@ struct GemmRings {
 
 // The loads of one group: the k-th KiB of a wave's share of A, its packed tile (k = 0) and that tile's scales (k = 1).
 template <bool GATE_UP, bool F16, bool WIDE>
-__device__ __forceinline__ void gemm_load_a(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, const float *__restrict__ act_scale,
-                                            uint32_t grp, uint32_t at, uint32_t rel_buf, int k) {
-    if (F16 && !GATE_UP && k == 0) {
-        // the scales of four 16-pair blocks (the second four waves repeat the first's, so that all count alike)
-        const uint32_t block = min(4 * (gw.wave & 3) + (gw.lane >> 4), (it.tile.rows - 1) / 16);
-        global_to_lds_4(act_scale + ((size_t)(it.act_block0 + block) * gw.n_groups + grp) * 16 + (gw.lane & 15),
-                        lds_base + kGemmRelAt + rel_buf * kGemmRowBytes + (gw.wave & 3) * (kWave * 4));
-    }
+__device__ __forceinline__ void gemm_load_a(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, uint32_t grp, uint32_t at, int k) {
     const uint32_t to = lds_base + at + (gw.wave + kGemmTiles * k) * kFragBytes;
     if constexpr (GATE_UP && WIDE) global_to_lds_16(gw.a + grp * kGroup + (size_t)it.from[k] * 8, to);
     else if constexpr (GATE_UP) global_to_lds_16(gw.a + grp * kGroup, it.from[k], to);
@@ -462,8 +455,7 @@ __device__ __forceinline__ void gemm_load_w(uint32_t lane, const uint8_t *w_tile
 }
 // what an item's first step counts on: two groups of A, as many packed tiles as the ring holds
 template <bool GATE_UP, bool F16, bool WIDE>
-__device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, const GemmRings &rings,
-                                         const float *__restrict__ act_scale) {
+__device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, const GemmRings &rings) {
 #pragma unroll
     for (uint32_t grp = 0; grp < kRingW; ++grp) {
         const bool live = grp < rings.depth;
@@ -476,7 +468,7 @@ __device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it,
 #pragma unroll
             for (int k = 0; k < kMaxLoads; ++k)
                 if ((uint32_t)k < it.loads)
-                    gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, act_scale, grp, grp ? rings.next : rings.cur, (grp ? rings.next : rings.cur) / kGemmABytes, k);
+                    gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, grp, grp ? rings.next : rings.cur, k);
         }
     }
 }
@@ -486,8 +478,7 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
                                           uint8_t *__restrict__ lds, uint32_t lds_base, const uint32_t *__restrict__ sorted_out_row,
                                           uint16_t *__restrict__ out, float *__restrict__ act_scale, uint4 *__restrict__ dump = nullptr) {
     constexpr int NA = NM > 0 ? NM : 1;
-    constexpr int kQueue = gemm_queue(NA, F16 ? 4 : 8);     // (FP16 has the block scales and their products in registers besides)
-    constexpr bool kScaled = F16 && !GATE_UP;               // a pair's blocks come with scales of their own
+    constexpr int kQueue = gemm_queue(NA, 8);
     const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4, n_groups = gw.n_groups;
     const uint32_t tile = it.nb * kGemmTiles + wave;        // this wave's arena tile
     if constexpr (!GATE_UP) {
@@ -535,14 +526,12 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
 #pragma unroll
     for (int i = 0; i < NA; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     uint4 xq[kQueue];
-    uint32_t rq[kQueue];
     // fragment f (k-half f / NM of 16-pair block f % NM) of a group
     const uint32_t at0 = GATE_UP ? j * 128 + 16 * (jq ^ (j & 7)) : lane * 16;
     auto read_a = [&](uint32_t from, int f) __attribute__((always_inline)) {
         const int half = f / NA, i = f % NA;
         const uint32_t at = GATE_UP ? at0 ^ (64 * half) : at0 + half * kFragBytes;
         xq[f % kQueue] = *reinterpret_cast<const uint4 *>(lds + from + i * (2 * kFragBytes) + at);
-        if constexpr (kScaled) rq[f % kQueue] = *reinterpret_cast<const uint32_t *>(lds + kGemmRelAt + (from / kGemmABytes) * kGemmRowBytes + (i * 16 + j) * 4);
     };
     // One step = one group, its k-halves one after the other: the products with the four pieces of the next operand set's
     // expansion between them (a scheduling fence behind each product keeps them there) and the fragments of A kQueue - 1 ahead.
@@ -583,13 +572,6 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
                     if (ahead < 2 * NM) read_a(rings.cur, ahead);
                     else read_a(rings.next, ahead - 2 * NM);
                     x = xq[f % kQueue];
-                    if constexpr (kScaled) {
-                        const f16x2 r2 = __builtin_bit_cast(f16x2, rq[f % kQueue]);
-                        x.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.x) * r2);
-                        x.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.y) * r2);
-                        x.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.z) * r2);
-                        x.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x.w) * r2);
-                    }
                 }
 #pragma unroll
                 for (int st = 0; st < 2; ++st) {
@@ -600,12 +582,12 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
                     if (half == 1 && kSteady) {
 #pragma unroll
                         for (int k = 0; k < LOADS; ++k)
-                            if (at == max((k + 1) * kUnits / (LOADS + 1) - 1, 0)) gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, act_scale, grp + 2, rings.before, rings.before / kGemmABytes, k);
+                            if (at == max((k + 1) * kUnits / (LOADS + 1) - 1, 0)) gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, grp + 2, rings.before, k);
                     } else if (half == 1) {
 #pragma unroll
                         for (int k = 0; k < kMaxLoads; ++k)
                             if (at == max((k + 1) * kUnits / (kMaxLoads + 1) - 1, 0) && run_on && (uint32_t)k < next_item.loads)
-                                gemm_load_a<GATE_UP, F16, WIDE>(gw, next_item, lds_base, act_scale, grp + 2 - n_groups, rings.before, rings.before / kGemmABytes, k);
+                                gemm_load_a<GATE_UP, F16, WIDE>(gw, next_item, lds_base, grp + 2 - n_groups, rings.before, k);
                     } else {
 #pragma unroll
                         for (int k = 0; k < 2; ++k)
@@ -649,7 +631,7 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
     }
     lds_barrier();                      // nobody reads the last group's A any more
     uint8_t *const stage = lds + rings.before;
-    if (n_groups == 1 && next_item.valid) gemm_ask<GATE_UP, F16, WIDE>(gw, next_item, lds_base, rings, act_scale);
+    if (n_groups == 1 && next_item.valid) gemm_ask<GATE_UP, F16, WIDE>(gw, next_item, lds_base, rings);
 
     // epilogue: lane (j, jq) holds pair j of every 16-pair block, weight rows 4 jq .. 4 jq + 3 of both row blocks
     if constexpr (GATE_UP) {
@@ -843,7 +825,7 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
     rings.cur = 0, rings.next = kGemmABytes, rings.before = 2 * kGemmABytes;
     rings.slot = rings.first_slot = kGemmWAt + gw.wave * kGemmWBytes;
     rings.end_slot = rings.first_slot + rings.depth * (kGemmTiles * kGemmWBytes);
-    gemm_ask<GATE_UP, F16, WIDE>(gw, it, lds_base, rings, act_scale);
+    gemm_ask<GATE_UP, F16, WIDE>(gw, it, lds_base, rings);
     vmem_barrier<0>();
     for (uint32_t r = 1;; ++r) {
         const GemmItem next = item_at(r);
@@ -950,7 +932,6 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         from[0] = gw.a + (size_t)gw.act_block0 * n_groups * (2 * kWave * 8) + (tid & 127) * 8;
     }
     u32x4_t stage[kPieces];        // (a native vector type: it stays in registers)
-    float rel[kPieces];
     auto load_a = [&](uint32_t chunk) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < kPieces; ++k) {
@@ -960,7 +941,6 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
             } else {
                 const uint32_t grp = min(chunk * CHUNK + 2 * k % CHUNK + (tid >> 7), last);
                 stage[k] = *reinterpret_cast<const u32x4_t *>(from[0] + ((size_t)(2 * k / CHUNK) * n_groups + grp) * (2 * kWave * 8));
-                if constexpr (F16) rel[k] = act_scale[((size_t)(gw.act_block0 + 2 * k / CHUNK) * n_groups + grp) * 16 + (tid & 15)];
             }
         }
     };
@@ -971,15 +951,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
                 const uint32_t row = row0 + kPassRows * k;
                 lds[buf * kBuf + ((row >> 4) * kFrags + (p >> 2)) * kWave + (p & 3) * 16 + ((row + p) & 15)] = __builtin_bit_cast(uint4, stage[k]);
             } else {
-                uint4 v = __builtin_bit_cast(uint4, stage[k]);
-                if constexpr (F16) {
-                    const f16x2 r2 = __builtin_bit_cast(f16x2, rel[k]);
-                    v.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.x) * r2);
-                    v.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.y) * r2);
-                    v.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.z) * r2);
-                    v.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v.w) * r2);
-                }
-                lds[buf * kBuf + 256 * k + tid] = v;
+                lds[buf * kBuf + 256 * k + tid] = __builtin_bit_cast(uint4, stage[k]);
             }
         }
     };
@@ -1197,25 +1169,50 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_
 #undef FFMOE_STREAM
 }
 
-// Between the two GEMMs of the FP16 prefill: a pair's block scales divided by its largest (powers of two: exact), the
-// largest itself stored behind the table at [n_pairs * blocks + pair] - what prefill_routed_down_tensorops computes per
-// threadgroup into `relative` and `pair_scale` (prefill.metal:731-741), done once per pair here.
-// One block per M-tile, one thread per pair of it.
-__global__ __launch_bounds__(kBM) void prefill_pair_scale_kernel(const PrefillPlan *__restrict__ plan,
-                                                                 const PrefillTile *__restrict__ tiles, uint32_t groups,
-                                                                 uint32_t act_blocks, float *__restrict__ act_scale) {
-    const uint32_t ti = blockIdx.x;
-    if (ti >= plan->n_tiles) return;
-    const PrefillTile tile = tiles[ti];
-    if (threadIdx.x >= tile.rows) return;
-    const uint32_t block = tile.row_start / 16 + tile.order + threadIdx.x / 16, j = threadIdx.x % 16;
-    float *s = act_scale + (size_t)block * groups * 16 + j;
+// Between the two GEMMs of the FP16 prefill: a pair's blocks of 64 activations times their scales over its largest (powers of two),
+// in place, and the largest behind the table at [n_pairs * blocks + pair] - what prefill_routed_down_tensorops does per
+// threadgroup with `relative` and `pair_scale` as it takes the rows in (prefill.metal:731-741). Done there, every wave of the
+// down products scaled every operand of its tile again: 8,000 pairs of 704 over 128 experts, down 82 us and this pass, scales
+// only, 7 -> 68 + 10; the call with 62, 125 and 192 pairs per expert 215 -> 208, 301 -> 289 and 396 -> 375 us.
+// A wave per 16-pair block; a pair's blocks that have its largest scale stay as they are. Bound: memory's latency.
+constexpr int kPairBlocks = 2;                              // of a block
+__global__ __launch_bounds__(64 * kPairBlocks) void prefill_pair_scale_kernel(const PrefillPlan *__restrict__ plan,
+                                                                              const PrefillTile *__restrict__ tiles, uint32_t groups,
+                                                                              uint32_t act_blocks, float *__restrict__ act_scale,
+                                                                              uint16_t *__restrict__ acts) {
+    if (blockIdx.x >= plan->n_tiles) return;
+    const PrefillTile tile = tiles[blockIdx.x];
+    const uint32_t lane = threadIdx.x & 63, j = lane & 15, jq = lane >> 4, in_tile = blockIdx.y * kPairBlocks + (threadIdx.x >> 6);
+    if (in_tile * 16 >= tile.rows) return;
+    const bool live = in_tile * 16 + j < tile.rows;
+    const uint32_t block = tile.row_start / 16 + tile.order + in_tile;
+    const float *const s = act_scale + (size_t)block * groups * 16 + j;
     float largest = 0.0f;
-    for (uint32_t b = 0; b < groups; ++b) largest = fmaxf(largest, s[b * 16]);
+    for (uint32_t b = jq; b < groups; b += 4) largest = fmaxf(largest, s[b * 16]);
+    largest = fmaxf(largest, __shfl_xor(largest, 16, 64));
+    largest = fmaxf(largest, __shfl_xor(largest, 32, 64));
     const float inv = 1.0f / largest;          // a scale is 2^(e - 14) with e >= -100: never zero
-    // kept as the FP16 pair that the down products multiply by
-    for (uint32_t b = 0; b < groups; ++b) s[b * 16] = __uint_as_float(Act<true>::pack(s[b * 16] * inv, s[b * 16] * inv));
-    act_scale[(size_t)act_blocks * groups * 16 + block * 16 + j] = largest;
+    uint4 *const a = reinterpret_cast<uint4 *>(acts) + (size_t)block * groups * (2 * kWave) + lane;
+    constexpr int kAhead = 6;
+    for (uint32_t b0 = 0; b0 < groups; b0 += kAhead) {
+        uint4 v[kAhead][2];
+        float rel[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) rel[u] = live && b0 + u < groups ? s[(b0 + u) * 16] * inv : 1.0f;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (__ballot(rel[u] != 1.0f)) v[u][0] = a[(b0 + u) * (2 * kWave)], v[u][1] = a[(b0 + u) * (2 * kWave) + kWave];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (rel[u] == 1.0f) continue;
+            const f16x2 r2 = __builtin_bit_cast(f16x2, Act<true>::pack(rel[u], rel[u]));
+            auto times = [&](uint32_t x) __attribute__((always_inline)) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x) * r2); };
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                a[(b0 + u) * (2 * kWave) + h * kWave] = uint4{times(v[u][h].x), times(v[u][h].y), times(v[u][h].z), times(v[u][h].w)};
+        }
+    }
+    if (live && jq == 0) act_scale[(size_t)act_blocks * groups * 16 + block * 16 + j] = largest;
 }
 
 // h2[t][c] = bf16(sum_r w[t][r] * partial[t][r][c]) over the routes the sort kept, fma in rank order
@@ -1309,7 +1306,7 @@ uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts, uint32_t d, ui
 // The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths): tiles of 32 rows while the gate/up
 // launch is one round (four blocks per compute unit on the XCD with the most N-blocks), or while a chunk's products are few
 // enough that it cost less than the GEMMs at 256 rows per tile did; at most kDenseTileStreamRows. With tiles of fewer rows the
-// GEMMs are now the faster ones from some 640 rows on (2,816 -> 2,112, 897 rows 62 us, FP16 85, where 896 streamed ones take 78
+// GEMMs are now the faster ones from some 640 rows on (2,816 -> 2,112, 897 rows 62 us, FP16 81, where 896 streamed ones take 78
 // and 98), but their weights are rounded to 16 bits and the streamed ones' are not: a chunk that had the smaller error keeps it.
 // us at 32 | 256 rows per tile, bf16 (FP16): 2,816 -> 2,112, 512 rows 54 | 78 (71 | 107), 800 rows 69 | 79 (88 | 108); 2,816 ->
 // 2,816, 672 rows 70 | 87, 896 rows 94 | 88 (114 | 121); 4,096 -> 2,816, 672 rows 96 | 106, 896 rows 129 | 108 (147 | 142).
@@ -1323,8 +1320,8 @@ uint32_t dense_tile_shift(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, ui
 // Rows per M-tile of a dense FFN's GEMMs: 16 n, n chosen so that the items fill their last round. A compute unit takes (10 + n) / 10 of
 // about 1,000 cycles per group of an item and the time of some six groups around them; the lists' last N-blocks are counted as
 // full ones. 2,816 -> 2,112 -> 2,816, us of the call at 256 rows per tile | the rule's: 102 | 62 at 897 rows (n = 4), 104 | 82 at
-// 2,048 (9), 112 | 103 at 3,072 (13), 170 | 147 at 4,096 (12), 292 | 259 at 8,192 (13); FP16 inputs 144 | 85, 148 | 113, 154 | 141,
-// 220 | 188 and 367 | 323. Of n = 6..16 each, the rule's is the fastest at these sizes or within 3% of it.
+// 2,048 (9), 112 | 103 at 3,072 (13), 170 | 147 at 4,096 (12), 292 | 259 at 8,192 (13); FP16 inputs now 81, 105, 132,
+// 179 and 311. Of n = 6..16 each, the rule's is the fastest at these sizes or within 3% of it.
 uint32_t dense_tile_rows(uint32_t t, const ArenaGeom &g, uint32_t n_cus) {
     uint32_t best = kBM;
     uint64_t least = ~0ull;
@@ -1437,7 +1434,8 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     else FFMOE_GEMM(true, x, x_stride, sc.acts, gemm_gu);
     timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
     if (f16)
-        hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap), dim3(kBM), 0, s, sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale);
+        hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap, ((streamed ? 1u << tile_shift : kBM) / 16 + kPairBlocks - 1) / kPairBlocks), dim3(64 * kPairBlocks), 0, s,
+                           sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale, sc.acts);
     if (streamed) FFMOE_STREAM(false, sc.acts, g.f, partials, nb_dn);
     else FFMOE_GEMM(false, sc.acts, g.f, partials, gemm_dn);
 #undef FFMOE_GEMM
