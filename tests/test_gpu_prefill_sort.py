@@ -44,3 +44,24 @@ def test_one_launch_sorts_as_three_do(oracle, e, k, cuts):
             assert np.array_equal(got, counts(n, past)) and n_pairs == got.sum(), n
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("t,k,d,skip", [(1, 1, 8, 0), (3, 8, 2816, 0), (33, 8, 72, 0), (5, 9, 64, 0), (7, 17, 1000, 0), (5, 3, 13, 0), (9, 8, 64, 1), (300, 2, 8, 0)])
+def test_reduce_of_rows_by_pieces_and_by_elements(oracle, act, t, k, d, skip):
+    # 16-byte pieces where width and addresses allow, elements elsewhere: the oracle's fma in rank order, bit for bit
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    dt, kind = (torch.bfloat16, oracle.BF16) if act == "bf16" else (torch.float16, oracle.FP16)
+    rng = np.random.default_rng(t * 100 + k)
+    ctx = ff.Context(64, 64, 4, 1, n_layers=1, max_tokens=16, act_dtype=act)
+    try:
+        flat = torch.from_numpy(rng.normal(0, 1, t * k * d + skip).astype(np.float32)).to(dt).cuda()
+        partials = flat[skip:].view(t, k, d)
+        w = torch.from_numpy(rng.normal(0, 1, (t, k)).astype(np.float32)).to(dt).cuda()
+        bits = lambda a: a.view(torch.int16).cpu().numpy().view(np.uint16)
+        got = bits(ctx.reduce_token_major(partials, w))
+        assert np.array_equal(got, oracle.reduce_token_major(bits(partials), kind, bits(w), kind))
+    finally:
+        ctx.close()
