@@ -177,38 +177,42 @@ __device__ __forceinline__ void global_to_lds_4(const void *base, uint32_t offse
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory");
 }
 
-// xor-butterfly sum across the 64 lanes (masks 32,16,8,4,2,1): every lane ends with the same value, and
-// every addition has the operands v[i] and v[i ^ mask] - the order the CPU oracle restates. The partners
-// come through register-to-register lane moves (gfx950 row swaps for 32 and 16, DPP rotations and quad
-// permutations below that) at a few cycles a step; __shfl_xor goes through the LDS crossbar at more than
-// a hundred, six times in a row on the critical path of every row reduction.
-__device__ __forceinline__ float wave_butterfly_sum(float v) {
+// The steps of the butterfly below inside groups of N = 16 or 4 lanes (masks N / 2 .. 1).
+template <int N> __device__ __forceinline__ float row_butterfly_sum(float v) {
+    static_assert(N == 16 || N == 4, "a row or a quad");
     auto dpp = [](float x, auto ctrl, auto banks, float old) {
         return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(old), (int)__float_as_uint(x),
                                                                       decltype(ctrl)::value, 0xF, decltype(banks)::value, false));
     };
     using std::integral_constant;
-    // 32: the swap leaves (lower half, lower half) and (upper half, upper half) in the two registers
-    auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    // 16: the same with the odd rows of one register and the even rows of the other
-    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    // 8: rotation by half a row
-    v = v + dpp(v, integral_constant<int, 0x128>{}, integral_constant<int, 0xF>{}, v);
-    // 4: lanes 0-3 and 8-11 of a row take from four lanes up (rotate right by 12), the others from four down
-    float p = dpp(v, integral_constant<int, 0x12C>{}, integral_constant<int, 0x5>{}, v);
-    p = dpp(v, integral_constant<int, 0x124>{}, integral_constant<int, 0xA>{}, p);
-    v = v + p;
+    if constexpr (N == 16) {
+        // 8: rotation by half a row
+        v = v + dpp(v, integral_constant<int, 0x128>{}, integral_constant<int, 0xF>{}, v);
+        // 4: lanes 0-3 and 8-11 of a row take from four lanes up (rotate right by 12), the others from four down
+        float p = dpp(v, integral_constant<int, 0x12C>{}, integral_constant<int, 0x5>{}, v);
+        p = dpp(v, integral_constant<int, 0x124>{}, integral_constant<int, 0xA>{}, p);
+        v = v + p;
+    }
     // 2 and 1: permutations inside each quad
     v = v + dpp(v, integral_constant<int, 0x4E>{}, integral_constant<int, 0xF>{}, v);
     v = v + dpp(v, integral_constant<int, 0xB1>{}, integral_constant<int, 0xF>{}, v);
     return v;
 }
 
-// The same sums (same operands in every addition) through the LDS crossbar: for kernels that reduce many
-// independent values per wave and have the vector ALU busy with other work, where throughput counts and the
-// latency of a step does not.
+// xor-butterfly sum across the 64 lanes (masks 32,16,8,4,2,1): every lane ends with the same value, and
+// every addition has the operands v[i] and v[i ^ mask] - the order the CPU oracle restates. The partners
+// come through register-to-register lane moves (gfx950 row swaps for 32 and 16, DPP rotations and quad
+// permutations below that) at a few cycles a step; __shfl_xor goes through the LDS crossbar at more than
+// a hundred, six times in a row on the critical path of every row reduction.
+__device__ __forceinline__ float wave_butterfly_sum(float v) {
+    // 32: the swap leaves (lower half, lower half) and (upper half, upper half) in the two registers
+    auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    // 16: the same with the odd rows of one register and the even rows of the other
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    return row_butterfly_sum<16>(v);
+}
 __device__ __forceinline__ float wave_butterfly_sum_shuffle(float v) {
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, 64);

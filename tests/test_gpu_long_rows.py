@@ -184,3 +184,20 @@ def test_choices_that_need_no_scratch_order_no_streams(ctx, torch):
         early = sum(event.query() for event in done)
     assert early, "the short rows waited for the other stream's work"
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("count", [2, 63, 64, 65, 127, 1025, 1088, 1089, 2049, 7168, 7169])
+def test_greedy_choice_where_waves_run_out(ctx, oracle, torch, count):
+    # rows whose last values only some of a block's waves have, and those only some lanes
+    rng = np.random.default_rng(count)
+    rows = rng.normal(0, 3, (4, count)).astype(np.float32)
+    rows[1, count - 1] = 50.0
+    rows[2, : count - 1] = np.nan
+    rows[3, :] = -np.inf
+    logits = torch.from_numpy(rows).cuda()
+    for cap in (0.0, 30.0):
+        want_pos, want_conf = oracle.greedy_choice_rows(rows, cap)
+        pos, conf = ctx.argmax_rows(logits, softcap=cap)
+        assert np.array_equal(pos.cpu().numpy().astype(np.uint32), want_pos.astype(np.uint32))
+        assert np.abs(conf.cpu().numpy() - want_conf).max() <= 1e-5
+        assert np.array_equal(ctx.argmax_rows(logits, softcap=cap, want_conf=False).cpu().numpy(), pos.cpu().numpy())
