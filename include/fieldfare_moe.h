@@ -432,8 +432,8 @@ int ffmoe_upload_expert_parts(ffmoe_ctx *ctx, uint32_t layer, uint32_t expert, c
 
 /* y[t] = down( bf16( gelu_tanh(gate x[t]) * (up x[t]) ) ) for every row, weight 1, no routing: the
  * shared expert. Needs a context created with n_experts = 1 and top_k = 1 (f = the shared width).
- * Rows <= 16 run the streaming kernels of ffmoe_verify; 17 to 384 rows the resident-matrix GEMV on the expert's arena
- * tiles, a grid row per 16 input rows (when d and f fit that kernel: <= FFMOE_MATRIX_MAX_N); more rows the grouped GEMMs
+ * Rows <= 16 run the streaming kernels of ffmoe_verify; 17 to 384 rows the resident-matrix products on the expert's
+ * arena tiles in bands of input rows (when d and f fit that kernel: <= FFMOE_MATRIX_MAX_N); more rows the grouped GEMMs
  * of ffmoe_prefill (the reference switches from its per-token GEMV loop to batched GEMMs at 32 tokens). Replaces
  * SharedExpertInt4.encode (Kernels/MoE/SharedExpertInt4.swift:32-89, kernel shared_gate_up_act_int4,
  * Metal/MoE/moe.metal:548-570) and PrefillSharedExpert.encodeBlock
@@ -490,7 +490,7 @@ int ffmoe_layer_tail_routed(ffmoe_ctx *ctx, void *stream, const uint16_t *route_
  * context with n_experts = 1 and top_k = 1, d and f multiples of 64 up to FFMOE_MATRIX_MAX_N. The layer is then kept as
  * a gated gate/up matrix and a down matrix of nibble planes (ffmoe_matrix_create_int8_glu / _int8) owned by the
  * context, and ffmoe_dense_ffn, ffmoe_route_verify_shared and ffmoe_layer_tail_routed_shared serve it like a 4-bit
- * layer: ffmoe_dense_ffn runs the two GEMV passes, a grid row per 16 rows, or from 192 rows on (when the context's
+ * layer: ffmoe_dense_ffn runs the two matrix products (beyond 16 rows in bands of input rows), or from 192 rows on (when the context's
  * max_tokens reaches that) two dense GEMMs of rocBLAS on hi + lo rows of the weights, kept in the activation type for
  * that purpose (4 more bytes per weight; that form is not meant for stream capture: the library may allocate workspace
  * on its first call), or from 640 rows on (up to 1,024 at narrow widths; likewise) two GEMMs of its own on the integer
@@ -554,8 +554,8 @@ int ffmoe_rmsnorm(ffmoe_ctx *ctx, void *stream, const uint16_t *x, uint32_t x_st
  * (ffmoe_prefill, ffmoe_prefill_pairs, ffmoe_dense_ffn beyond 16 rows) follow the reference's FP16 tiles
  * (Metal/Prefill/prefill.metal:581-598,685-702,723-777): FP16 rows against tile weights half(fma(q, scale, bias)), fp32
  * sums, and the activations between the two GEMMs FP16 with a power-of-two scale per pair and 64-wide block of the
- * intermediate size, so that values past FP16's range keep FP16's relative precision; the down GEMM brings a
- * pair's blocks to the pair's largest scale as it reads them and applies that scale to the pair's sums. In FFMOE_FP16 input rows must be 16-byte aligned with strides
+ * intermediate size, so that values past FP16's range keep FP16's relative precision; a pass between the
+ * GEMMs brings a pair's blocks to the pair's largest scale and the down GEMM applies that scale to the pair's sums. In FFMOE_FP16 input rows must be 16-byte aligned with strides
  * that are multiples of 8 wherever a call accepts less otherwise (router, GEMV). Set it before the
  * first compute call; switching waits for the device. May allocate (once). */
 int ffmoe_set_activation_dtype(ffmoe_ctx *ctx, int dtype, char **err);
