@@ -1292,6 +1292,9 @@ __global__ void prefill_dump_plan_kernel(uint32_t expert, PrefillPlan *plan, Pre
 // 40 pairs 66 | 72 | 70 (76 | 87 | 83); 16 experts, 2,816 x 704, 48 pairs 54 | 55 | 54 (61 | 67 | 63). 64 experts, 1,024 x 512:
 // 32 pairs 39 | 38 | 42 (49 | 45 | 48), 48 pairs 51 | 45 | 45 (57 | 53 | 51); 64 experts, 1,536 x 768, 48 pairs 77 | 71 | 74 (85 | 80 |
 // 84); 256 experts, 512 x 256, 28 pairs 48 | 49 | 52, 40 pairs 59 | 56 | 53 (64 | 65 | 59).
+// (The third figures are the four-wave GEMMs' that the line was drawn by; with a wave per arena tile they cross, at the first shape, at
+// 44 pairs in FP16 - 42 pairs 182 | 184, 48 pairs 192 | 190 - and at some 40 in bf16, where the streamed weights are not rounded to 16
+// bits: a chunk that had the smaller error keeps it.)
 // Skewed routes move nothing: at the first shape with Zipf popularity of exponent 0.6, 1.1 and 1.6 the streaming form wins at
 // every size up to 48 pairs (448 rows 146 | 159 | 166 against 186 | 201 | 196 for the GEMMs, 768 rows 192 | 201 | 212 against 225 |
 // 226 | 232). Tiles of 16 pairs gain nothing over 32 (37 rows: 99), tiles of 128 lose everywhere (1,000 rows: 227, two waves per
