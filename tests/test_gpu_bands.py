@@ -1,6 +1,6 @@
 """Dense FFNs of 17 rows to a few hundred in bands of input rows: a row has the bits of the 16-row pass (8 bits) and of the same row
 in any other chunk (4 bits), in every split of K and number of row blocks per band, at K of one group and of no multiple of the
-splits, tile counts that fill no block, both activation types. Run on the GPU box: pytest -m gpu."""
+splits, tile counts that fill no block, both activation types. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,7 +1,7 @@
 """The prefill's grouped GEMMs: M-tiles of every number of 16-pair blocks (and one, two and no pairs past a block), plans whose
 largest tile is at most half a tile (deeper rings of packed tiles), K of one group, of fewer and of more than the rings hold,
 N-blocks that are full, half full and a quarter full, fewer and more items than compute units, both activation types; rows that
-span more than 4 GiB. Run on the GPU box: pytest -m gpu."""
+span more than 4 GiB. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

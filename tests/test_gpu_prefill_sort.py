@@ -1,6 +1,5 @@
 """The prefill's sort of routes in one launch (3,072 items and fewer) and in three: the same rows, bit for bit, from a chunk and from its
-beginning on either side of the line, counts per expert, routes of weight zero and experts past the last left out. Run on
-the GPU box: pytest -m gpu."""
+beginning on either side of the line, counts per expert, routes of weight zero and experts past the last left out. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 
