@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -20,6 +21,9 @@ using namespace ffmoe;
 struct ffmoe_layer {
     bool experts_loaded = false;
     std::vector<bool> part_loaded;  // experts uploaded one at a time (ffmoe_upload_expert_parts)
+    // experts with weight scales of 2^104 and more, and whether there is one (an upload of the whole layer tells for all together)
+    std::vector<bool> large_scales;
+    bool any_large_scale = false;
     void *router_w = nullptr;       // bf16 or float [E][D]
     int router_is_f32 = 0;
     uint16_t *effective_scale = nullptr;
@@ -442,10 +446,14 @@ int ffmoe_upload_layer(ffmoe_ctx *ctx, uint32_t layer, const void *blobs, size_t
         src = staging;
     }
     hipError_t e = launch_repack_layer(nullptr, src, stride, *offsets, sh.n_experts, ctx->geom,
-                                       ctx->arena + (size_t)layer * ctx->layer_bytes);
+                                       ctx->arena + (size_t)layer * ctx->layer_bytes, &ctx->pf.plan->large_scales);
     if (e == hipSuccess) e = hipDeviceSynchronize();
+    uint32_t large = 0;
+    if (e == hipSuccess) e = hipMemcpy(&large, &ctx->pf.plan->large_scales, sizeof large, hipMemcpyDeviceToHost);
     if (staging) (void)hipFree(staging);
     if (e != hipSuccess) return fail(err, FFMOE_ERR_RUNTIME, "re-tiling layer %u failed: %s", layer, hipGetErrorString(e));
+    ctx->layers[layer].large_scales.assign(sh.n_experts, large != 0);
+    ctx->layers[layer].any_large_scale = large != 0;
     drop_int8_form(ctx->layers[layer]);
     ctx->layers[layer].experts_loaded = true;
     return FFMOE_OK;
@@ -500,13 +508,19 @@ int ffmoe_upload_expert_parts(ffmoe_ctx *ctx, uint32_t layer, uint32_t expert, c
     const ffmoe_offsets offsets = {off[0], off[1], off[2], off[3], off[4], off[5], off[6], off[7], off[8]};
     if (e == hipSuccess)
         e = launch_repack_layer(nullptr, staging, total, offsets, 1, ctx->geom,
-                                ctx->arena + (size_t)layer * ctx->layer_bytes + (size_t)expert * ctx->geom.expert_bytes);
+                                ctx->arena + (size_t)layer * ctx->layer_bytes + (size_t)expert * ctx->geom.expert_bytes,
+                                &ctx->pf.plan->large_scales);
     if (e == hipSuccess) e = hipDeviceSynchronize();
+    uint32_t large = 0;
+    if (e == hipSuccess) e = hipMemcpy(&large, &ctx->pf.plan->large_scales, sizeof large, hipMemcpyDeviceToHost);
     (void)hipFree(staging);
     if (e != hipSuccess)
         return fail(err, FFMOE_ERR_RUNTIME, "upload of expert %u of layer %u failed: %s", expert, layer, hipGetErrorString(e));
     ffmoe_layer &l = ctx->layers[layer];
     drop_int8_form(l);      // the layer is 4-bit from here on
+    if (l.large_scales.size() != sh.n_experts) l.large_scales.assign(sh.n_experts, false);
+    l.large_scales[expert] = large != 0;
+    l.any_large_scale = std::find(l.large_scales.begin(), l.large_scales.end(), true) != l.large_scales.end();
     if (l.part_loaded.size() != sh.n_experts) l.part_loaded.assign(sh.n_experts, false);
     l.part_loaded[expert] = true;
     bool all = true;
@@ -799,7 +813,7 @@ static int prefill_common(ffmoe_ctx *ctx, void *stream, uint32_t layer, const ui
     claim_scratch(ctx, stream);
     FF_HIP(launch_prefill(static_cast<hipStream_t>(stream), ctx->arena + (size_t)layer * ctx->layer_bytes, ctx->geom,
                           ctx->shape.n_experts, ctx->shape.top_k, x, x_stride, t, idx, w, pairs, n_pairs, y, partials,
-                          ctx->pf, &ctx->timer, ctx->n_cus, ctx->f16, dense));
+                          ctx->pf, &ctx->timer, ctx->n_cus, ctx->f16, dense, ctx->layers[layer].any_large_scale));
     return FFMOE_OK;
 }
 
@@ -827,7 +841,7 @@ int ffmoe_prefill_dump_tiles(ffmoe_ctx *ctx, void *stream, uint32_t layer, uint3
     if (out_bytes < need) return fail(err, FFMOE_ERR_INVALID, "output holds %zu bytes, the fragments take %zu", out_bytes, need);
     claim_scratch(ctx, stream);
     FF_HIP(launch_prefill_dump_tiles(static_cast<hipStream_t>(stream), ctx->arena + (size_t)layer * ctx->layer_bytes, ctx->geom,
-                                     expert, gate_up != 0, ctx->pf, out, ctx->f16));
+                                     expert, gate_up != 0, ctx->pf, out, ctx->f16, ctx->layers[layer].any_large_scale));
     return FFMOE_OK;
 }
 

@@ -12,6 +12,7 @@ constexpr int kGroup = 64;     // MLX-affine group size (Infrastructure/ModelIO/
 constexpr int kWave = 64;      // CDNA wavefront
 constexpr int kTileRows = 16;  // weight rows per arena tile = MFMA 16x16x32 column block
 constexpr int kTileBytes = 1024;   // one arena tile: 64 lanes x 16 B (two 16-row x 64-k nibble blocks)
+constexpr uint32_t kLargeScale = (127 + 104) << 7;     // bf16 bits of 2^104: from here on, infinities and NaN included, 2^24 times a weight's scale is no fp32 number
 constexpr int kTileScaleBytes = 128;  // 16 rows x 4 bf16 (scale/bias of the two blocks)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -48,21 +49,6 @@ __device__ __forceinline__ float gelu_tanh_fast(float x) {
 // eight k-slots and position m + 4 holds element 2m + 1, so that ((w >> 4m) & 0x000F000F) is the
 // 16-bit pair (element 2m, element 2m + 1) with no cross-lane or cross-register shuffling.
 //
-// dequant8_bf16: the eight nibbles as bf16(fma(q, scale, bias)) - the reference's 16-bit tile weight
-// (Metal/Prefill/prefill.metal:581-590 with half replaced by bfloat as Metal/TensorCore/tensorops.metal:267).
-// q * scale is exact in fp32 (4-bit x 8-bit significands), so fma and mul-then-add agree.
-__device__ __forceinline__ uint4 dequant8_bf16(uint32_t w, float scale, float bias) {
-    // even nibbles / odd nibbles as bytes; the empty asm keeps the two masks as written so that each
-    // byte converts with one v_cvt_f32_ubyteN instead of a bit-field extract plus a convert
-    uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-    asm("" : "+v"(lo), "+v"(hi));
-    uint4 r;
-    r.x = pack_bf16x2(__builtin_fmaf((float)(lo & 0xFFu), scale, bias), __builtin_fmaf((float)((lo >> 16) & 0xFFu), scale, bias));
-    r.y = pack_bf16x2(__builtin_fmaf((float)(hi & 0xFFu), scale, bias), __builtin_fmaf((float)((hi >> 16) & 0xFFu), scale, bias));
-    r.z = pack_bf16x2(__builtin_fmaf((float)((lo >> 8) & 0xFFu), scale, bias), __builtin_fmaf((float)(lo >> 24), scale, bias));
-    r.w = pack_bf16x2(__builtin_fmaf((float)((hi >> 8) & 0xFFu), scale, bias), __builtin_fmaf((float)(hi >> 24), scale, bias));
-    return r;
-}
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -105,6 +91,23 @@ template <> struct Act<true> {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
 };
+
+// The eight nibbles of a dword, in arena order, as 16-bit fma(q, scale, bias) - the reference's tile weight
+// (Metal/Prefill/prefill.metal:581-590; bf16: half replaced by bfloat as Metal/TensorCore/tensorops.metal:267).
+// q * scale is exact in fp32 (4-bit x 8-bit significands), so fma and mul-then-add agree.
+template <bool F16>
+__device__ __forceinline__ uint4 dequant8(uint32_t w, float scale, float bias) {
+    // even nibbles / odd nibbles as bytes; the empty asm keeps the two masks as written so that each
+    // byte converts with one v_cvt_f32_ubyteN instead of a bit-field extract plus a convert
+    uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+    asm("" : "+v"(lo), "+v"(hi));
+    uint4 r;
+    r.x = Act<F16>::pack(__builtin_fmaf((float)(lo & 0xFFu), scale, bias), __builtin_fmaf((float)((lo >> 16) & 0xFFu), scale, bias));
+    r.y = Act<F16>::pack(__builtin_fmaf((float)(hi & 0xFFu), scale, bias), __builtin_fmaf((float)((hi >> 16) & 0xFFu), scale, bias));
+    r.z = Act<F16>::pack(__builtin_fmaf((float)((lo >> 8) & 0xFFu), scale, bias), __builtin_fmaf((float)(lo >> 24), scale, bias));
+    r.w = Act<F16>::pack(__builtin_fmaf((float)((hi >> 8) & 0xFFu), scale, bias), __builtin_fmaf((float)(hi >> 24), scale, bias));
+    return r;
+}
 
 // The eight nibbles of a dword as 16-bit values offset + q in the activation type (128 + q as bf16: 0x4300 | q
 // is exact, the bf16 ulp at 128 is 1). The matrix unit then accumulates sum (offset + q) x; the caller removes

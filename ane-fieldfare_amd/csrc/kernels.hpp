@@ -101,7 +101,8 @@ struct PrefillTile {
     uint32_t order;                       // the tile's number in row order (the tile list itself runs from the largest tile down)
 };
 struct PrefillPlan {
-    uint32_t n_pairs, n_tiles, pad[2];
+    uint32_t n_pairs, n_tiles;
+    uint32_t large_scales, pad;     // large_scales: an upload's, not a chunk's (launch_repack_layer)
     uint32_t expert_count[FFMOE_MAX_EXPERTS];
     uint32_t expert_offset[FFMOE_MAX_EXPERTS + 1];
 };
@@ -158,9 +159,9 @@ struct SharedExpert {
 constexpr uint32_t kSharedChunkGroups = 11;      // = kRing of the streaming kernels
 inline uint32_t shared_chunks(const ArenaGeom &g) { return (g.gf + kSharedChunkGroups - 1) / kSharedChunkGroups; }
 
-// repack.hip
+// repack.hip. *large_scales is cleared, then set where a scale of the experts is a large one
 hipError_t launch_repack_layer(hipStream_t s, const uint8_t *blobs, size_t stride, ffmoe_offsets off,
-                               uint32_t n_experts, ArenaGeom g, uint8_t *arena_layer);
+                               uint32_t n_experts, ArenaGeom g, uint8_t *arena_layer, uint32_t *large_scales);
 hipError_t launch_dequant_expert(hipStream_t s, const uint8_t *arena_expert, ArenaGeom g, int which,
                                  uint16_t *out);
 
@@ -255,12 +256,17 @@ hipError_t launch_dense8_rows(hipStream_t s, const uint16_t *x, uint32_t x_strid
 hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t stored_rows, uint32_t n, bool gated, const void *ops, uint32_t t,
                               void *out, uint32_t out_stride, bool f16, uint32_t n_cus);
 
-// prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr.
-// Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
+// prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr. large_scales: the
+// layer has weight scales of 2^104 and more. Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,
                           const uint16_t *x, uint32_t x_stride, uint32_t t, const uint32_t *idx, const uint16_t *w,
                           const ffmoe_pair *pairs, uint32_t n_pairs_in, uint16_t *y, uint16_t *partials_out,
-                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16 = false, bool dense = false);
+                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16 = false, bool dense = false,
+                          bool large_scales = false);
+
+// prefill_large.hip: either product (gate/up, else down) of the M-tiles in sc.tiles, `tile_cap` of them at most; `dump` as below
+hipError_t launch_prefill_large_scale(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, bool gate_up, uint32_t tile_cap, const uint16_t *a,
+                                      uint32_t a_stride, uint16_t *out, PrefillScratch sc, bool f16, void *dump = nullptr);
 
 // Test hook: the weight fragments of one expert's gate/up (or down) tiles as the grouped GEMM's matrix instructions
 // receive them: [N-block][group][fragment 0..15][lane] x 16 bytes, `prefill_dump_fragments` fragments in all.
@@ -268,7 +274,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
 // stream and k = 32 * (k-half) + 8 * (l / 16) .. + 7 of the group.
 uint32_t prefill_dump_fragments(const ArenaGeom &g, bool gate_up);
 hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t expert, bool gate_up,
-                                     PrefillScratch sc, void *dump, bool f16 = false);
+                                     PrefillScratch sc, void *dump, bool f16 = false, bool large_scales = false);
 
 // epilogue.hip: row-wise steps either side of the MoE stage
 hipError_t launch_post_attn_setup(hipStream_t s, uint16_t *hidden, uint32_t hidden_stride, const uint16_t *attn,

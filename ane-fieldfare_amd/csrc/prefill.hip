@@ -496,8 +496,8 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
         sraw = *reinterpret_cast<const uint2 *>(at + kTileBytes + j * 8);
     };
     // Expansion: bits 0..3 and 4..7 of each half of a dword are FP16 subnormals q 2^-24 and q 2^-20 as they lie, and one
-    // v_fma_mix_f32 takes such a half with fp32 scale (times 2^24, 2^20: exact) and bias: 17 vector instructions for eight
-    // weights instead of 23 with byte conversions, the same fp32 value to the bit.
+    // v_fma_mix_f32 takes such a half with fp32 scale (times 2^24, 2^20: exact below 2^104, and layers with larger ones do not come
+    // here) and bias: 17 vector instructions for eight weights instead of 23 with byte conversions, the same fp32 value to the bit.
     float s24[2], s20[2], bias[2];
     auto take_scales = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -1351,10 +1351,13 @@ uint32_t prefill_dump_fragments(const ArenaGeom &g, bool gate_up) {
 }
 
 hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t expert, bool gate_up,
-                                     PrefillScratch sc, void *dump, bool f16) {
+                                     PrefillScratch sc, void *dump, bool f16, bool large_scales) {
     if (f16 && !sc.act_scale) return hipErrorInvalidValue;
     hipLaunchKernelGGL(prefill_dump_plan_kernel, dim3(1), dim3(1), 0, s, expert, sc.plan, sc.tiles, sc.sorted_token,
                        sc.sorted_out_row);
+    if (large_scales)
+        return launch_prefill_large_scale(s, arena_layer, g, gate_up, 1, gate_up ? sc.partials : sc.acts, g.d, gate_up ? sc.acts : sc.partials, sc, f16,
+                                          dump);
     // the pair's input row is whatever row 0 of the scratch holds: only the weight side is looked at
 #define FFMOE_DUMP(GU, H, A, STRIDE, OUT, NB)                                                                              \
     hipLaunchKernelGGL((prefill_gemm_kernel<GU, H, false, true>), dim3((NB) * 8), dim3(64 * kGemmTiles), 0, s, arena_layer, g, sc.plan, sc.tiles,  \
@@ -1373,7 +1376,7 @@ hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, 
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,
                           const uint16_t *x, uint32_t x_stride, uint32_t t, const uint32_t *idx, const uint16_t *w,
                           const ffmoe_pair *pairs, uint32_t n_pairs_in, uint16_t *y, uint16_t *partials_out,
-                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16, bool dense) {
+                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16, bool dense, bool large_scales) {
     // dense: the caller vouches for a dense FFN's chunk - one expert, top_k = 1, every row routed to it at weight 1
     dense = dense && n_experts == 1 && top_k == 1 && !pairs && !y;
     timer->begin(s);
@@ -1433,13 +1436,17 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
     hipLaunchKernelGGL(stream_kernel<GU>(tile_shift, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
                        sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major, act_scale, act_blocks)
-    if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);
+    if (large_scales) {
+        if ((e = launch_prefill_large_scale(s, arena_layer, g, true, tile_cap, x, x_stride, sc.acts, sc, f16)) != hipSuccess) return e;
+    } else if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);
     else FFMOE_GEMM(true, x, x_stride, sc.acts, gemm_gu);
     timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
     if (f16)
         hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap, ((streamed ? 1u << tile_shift : kBM) / 16 + kPairBlocks - 1) / kPairBlocks), dim3(64 * kPairBlocks), 0, s,
                            sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale, sc.acts);
-    if (streamed) FFMOE_STREAM(false, sc.acts, g.f, partials, nb_dn);
+    if (large_scales) {
+        if ((e = launch_prefill_large_scale(s, arena_layer, g, false, tile_cap, sc.acts, g.f, partials, sc, f16)) != hipSuccess) return e;
+    } else if (streamed) FFMOE_STREAM(false, sc.acts, g.f, partials, nb_dn);
     else FFMOE_GEMM(false, sc.acts, g.f, partials, gemm_dn);
 #undef FFMOE_GEMM
 #undef FFMOE_STREAM

@@ -52,7 +52,7 @@ __device__ __forceinline__ uint16_t load_u16(const uint8_t *p) { return (uint16_
 // (A = row a, B = row a + 16).
 __global__ __launch_bounds__(256) void repack_kernel(const uint8_t *__restrict__ blobs, size_t stride,
                                                      ffmoe_offsets off, uint32_t n_experts, ArenaGeom g,
-                                                     uint8_t *__restrict__ arena) {
+                                                     uint8_t *__restrict__ arena, uint32_t *__restrict__ large_scales) {
     const size_t gu_tiles = (size_t)g.gu_rb * g.gd;
     const size_t dn_tiles = (size_t)g.dn_rbp * g.gf;
     const size_t tiles_per_expert = gu_tiles + dn_tiles;
@@ -104,6 +104,7 @@ __global__ __launch_bounds__(256) void repack_kernel(const uint8_t *__restrict__
             sc.x = (uint32_t)load_u16(sa + ia) | ((uint32_t)load_u16(ba + ia) << 16);
             sc.y = (uint32_t)load_u16(sb + ib) | ((uint32_t)load_u16(bb + ib) << 16);
             reinterpret_cast<uint2 *>(scale_dst)[i] = sc;
+            if ((sc.x & 0x7FFFu) >= kLargeScale || (sc.y & 0x7FFFu) >= kLargeScale) *large_scales = 1;
         }
     }
 }
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(256) void dequant_expert_kernel(const uint8_t *__re
         const uint32_t lane = jq * 16 + i;
         const uint32_t w = reinterpret_cast<const uint32_t *>(tiles + tile * kTileBytes)[lane * 4 + dword];
         const uint32_t sb = reinterpret_cast<const uint32_t *>(scales + tile * kTileScaleBytes)[i * 2 + (dword >> 1)];
-        const uint4 v = dequant8_bf16(w, bf16lo_to_f32(sb), bf16hi_to_f32(sb));
+        const uint4 v = dequant8<false>(w, bf16lo_to_f32(sb), bf16hi_to_f32(sb));
         *reinterpret_cast<uint4 *>(out + (size_t)row * cols + k0) = v;
     }
 }
@@ -146,10 +147,12 @@ __global__ __launch_bounds__(256) void dequant_expert_kernel(const uint8_t *__re
 }  // namespace
 
 hipError_t launch_repack_layer(hipStream_t s, const uint8_t *blobs, size_t stride, ffmoe_offsets off,
-                               uint32_t n_experts, ArenaGeom g, uint8_t *arena_layer) {
+                               uint32_t n_experts, ArenaGeom g, uint8_t *arena_layer, uint32_t *large_scales) {
+    const hipError_t e = hipMemsetAsync(large_scales, 0, sizeof *large_scales, s);
+    if (e != hipSuccess) return e;
     const size_t total = (size_t)n_experts * ((size_t)g.gu_rb * g.gd + (size_t)g.dn_rbp * g.gf) * kWave;
     const uint32_t blocks = (uint32_t)((total + 255) / 256 < 65535 * 8 ? (total + 255) / 256 : 65535 * 8);
-    hipLaunchKernelGGL(repack_kernel, dim3(blocks), dim3(256), 0, s, blobs, stride, off, n_experts, g, arena_layer);
+    hipLaunchKernelGGL(repack_kernel, dim3(blocks), dim3(256), 0, s, blobs, stride, off, n_experts, g, arena_layer, large_scales);
     return hipGetLastError();
 }
 
