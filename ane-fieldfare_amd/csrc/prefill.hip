@@ -473,9 +473,10 @@ __device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it,
     }
 }
 
+// (lds is not __restrict__: the loads write the same memory through lds_base)
 template <bool GATE_UP, int NM, int LOADS, bool F16, bool WIDE, bool DUMP>
 __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it, const GemmItem &next_item, GemmRings &rings, const ArenaGeom &g,
-                                          uint8_t *__restrict__ lds, uint32_t lds_base, const uint32_t *__restrict__ sorted_out_row,
+                                          uint8_t *lds, uint32_t lds_base, const uint32_t *__restrict__ sorted_out_row,
                                           uint16_t *__restrict__ out, float *__restrict__ act_scale, uint4 *__restrict__ dump = nullptr) {
     constexpr int NA = NM > 0 ? NM : 1;
     constexpr int kQueue = gemm_queue(NA, 8);
