@@ -333,7 +333,7 @@ int ffmoe_create(int device, const ffmoe_shape *shape, ffmoe_ctx **out, char **e
     // prefill scratch: sort tables, pair lists, activations and per-route rows for max_tokens tokens
     ctx->max_pairs = (shape->max_tokens > FFMOE_MAX_VERIFY_ROWS ? shape->max_tokens : FFMOE_MAX_VERIFY_ROWS) * shape->top_k;
     const size_t sort_blocks = (ctx->max_pairs + 255) / 256;
-    ctx->pf.max_tiles = prefill_max_tiles(ctx->max_pairs, shape->n_experts);
+    ctx->pf.max_tiles = prefill_max_tiles(ctx->max_pairs, shape->n_experts, ctx->geom, ctx->n_cus);
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&ctx->pf.block_cnt), sort_blocks * shape->n_experts * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&ctx->pf.plan), sizeof(PrefillPlan));
     if (e == hipSuccess) e = hipMemset(ctx->pf.plan, 0, sizeof(PrefillPlan));

@@ -233,14 +233,18 @@ hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t strid
                               uint32_t *out, float *out_conf, SampleScratch sc);
 
 // The most pairs per expert, on average, at which a prefill chunk takes the streaming product, and the M-tiles that a
-// scratch for `max_pairs` pairs has to hold: that product's tiles go down to 32 pairs (prefill_tile_shift, prefill.hip).
+// scratch for `max_pairs` pairs has to hold: that product's tiles go down to 32 pairs, the GEMMs' to as many as there are compute
+// units (prefill_tile_form, gemm_tile_rows in prefill.hip).
 constexpr uint32_t kPrefillStreamPairs = 48;
 constexpr uint32_t kDenseTileStreamRows = 896;       // and the most rows at which a dense FFN's chunk does
-inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts) {
+inline uint32_t prefill_max_tiles(uint32_t max_pairs, uint32_t n_experts, const ArenaGeom &g, uint32_t n_cus) {
     const uint32_t whole = max_pairs / FFMOE_PREFILL_TILE_M;
     // tiles of 32 pairs or more up to 48 per expert: 1.5 n_experts full ones at most; a dense FFN's down to 64 rows beyond the streamed
     const uint32_t dense = kDenseTileStreamRows / 32 > max_pairs / 64 ? kDenseTileStreamRows / 32 : max_pairs / 64;
-    const uint32_t small = n_experts == 1 ? dense : kPrefillStreamPairs * n_experts / 32;
+    uint32_t small = n_experts == 1 ? dense : kPrefillStreamPairs * n_experts / 32;
+    // full tiles of the GEMMs below 256 pairs
+    const uint32_t items = (n_cus + n_cus / 16) / ((g.gu_rb + 7) / 8) + 1, most = items < max_pairs / 32 ? items : max_pairs / 32;
+    if (small < most) small = most;
     return (whole > small ? whole : small) + n_experts + 1;
 }
 

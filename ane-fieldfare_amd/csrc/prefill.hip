@@ -25,6 +25,14 @@ namespace ffmoe {
 namespace {
 
 constexpr int kSortBlock = 256;
+// Pairs per M-tile, a multiple of 16 up to kBM, and what divides by it: n * `divide` >> 32 is n / rows for every n where rows is a
+// power of two, and up to 2^24 otherwise.
+struct TileRows {
+    uint32_t rows, divide;
+    __host__ __device__ explicit TileRows(uint32_t r) : rows(r), divide((uint32_t)(((1ull << 32) + r - 1) / r)) {}
+    __device__ __forceinline__ uint32_t whole(uint32_t n) const { return __umulhi(n, divide); }
+    __device__ __forceinline__ uint32_t rest(uint32_t n) const { return n - whole(n) * rows; }
+};
 constexpr int kBM = FFMOE_PREFILL_TILE_M;   // pairs per M-tile
 constexpr int kTilesPerBlock = 4;           // arena tiles (of 16 + 16 rows) per N-block
 
@@ -73,8 +81,7 @@ constexpr int kScanThreads = 1024;
 template <int kScanKeep>
 __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad, uint32_t *__restrict__ block_cnt,
                                              PrefillPlan *__restrict__ plan, PrefillTile *__restrict__ tiles, uint32_t max_tiles,
-                                             uint32_t tile_shift) {
-    const uint32_t bm = 1u << tile_shift;        // pairs per M-tile
+                                             TileRows bm) {
     __shared__ uint32_t total[FFMOE_MAX_EXPERTS];
     __shared__ uint32_t offset[FFMOE_MAX_EXPERTS + 1];
     __shared__ uint32_t tile_off[FFMOE_MAX_EXPERTS + 1];
@@ -115,7 +122,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
     if (threadIdx.x < FFMOE_MAX_EXPERTS) {
         const uint32_t i = threadIdx.x, lane = i & 63, wv = i >> 6;
         const uint32_t n = i < n_experts ? total[i] : 0;
-        const unsigned long long own = ((unsigned long long)((n + bm - 1) >> tile_shift) << 32) | n;
+        const unsigned long long own = ((unsigned long long)bm.whole(n + bm.rows - 1) << 32) | n;
         unsigned long long inc = own;
 #pragma unroll
         for (int sh = 1; sh < 64; sh <<= 1) {
@@ -141,7 +148,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
             unsigned long long all = ex;
             if (i != n_experts) {
                 const uint32_t n = total[i];
-                all += ((unsigned long long)((n + bm - 1) >> tile_shift) << 32) | n;
+                all += ((unsigned long long)bm.whole(n + bm.rows - 1) << 32) | n;
                 offset[n_experts] = (uint32_t)all;
                 tile_off[n_experts] = (uint32_t)(all >> 32);
             }
@@ -157,11 +164,11 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
     // anywhere in the expert order). Where an expert's shorter tile goes takes a look at every other expert's: the
     // threads of an expert share that out (one thread alone is a chain of two thousand instructions).
     if (live) {
-        const uint32_t rest = (total[e] & (bm - 1)), per_o = (e_pad + chunks - 1) / chunks;
+        const uint32_t rest = bm.rest(total[e]), per_o = (e_pad + chunks - 1) / chunks;
         const uint32_t o_lo = min(e_pad, ch * per_o), o_hi = min(e_pad, o_lo + per_o);
         uint32_t all = 0, in_front = 0, above = 0;
         for (uint32_t o = o_lo; o < o_hi; ++o) {
-            const uint32_t r = (total[o] & (bm - 1));          // experts past n_experts hold zero
+            const uint32_t r = bm.rest(total[o]);              // experts past n_experts hold zero
             const uint32_t has = r != 0 ? 1u : 0u;
             all += has;
             in_front += has & (o < e ? 1u : 0u);
@@ -191,7 +198,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
     plan->expert_offset[e] = offset[e];
     plan->expert_count[e] = total[e];
     // a tile keeps its number in row order, which places its activation blocks
-    const uint32_t nt = (total[e] + bm - 1) >> tile_shift, n_full = total[e] >> tile_shift;
+    const uint32_t nt = bm.whole(total[e] + bm.rows - 1), n_full = bm.whole(total[e]);
     const uint32_t shorter_tiles = shorter[0][e], shorter_in_front = shorter[1][e], ranked_above = shorter[2][e];
     const uint32_t full_in_front = tile_off[e] - shorter_in_front, full_tiles = tile_off[n_experts] - shorter_tiles;
     for (uint32_t i = 0; i < nt; ++i) {
@@ -199,8 +206,8 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
         if (ti < max_tiles) {
             PrefillTile tl;
             tl.expert = e;
-            tl.row_start = offset[e] + i * bm;
-            tl.rows = min(bm, total[e] - i * bm);
+            tl.row_start = offset[e] + i * bm.rows;
+            tl.rows = min(bm.rows, total[e] - i * bm.rows);
             tl.order = tile_off[e] + i;
             tiles[ti] = tl;
         }
@@ -213,8 +220,8 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
                                                                     uint32_t *__restrict__ block_cnt,
                                                                     PrefillPlan *__restrict__ plan,
                                                                     PrefillTile *__restrict__ tiles, uint32_t max_tiles,
-                                                                    uint32_t tile_shift) {
-    plan_experts<kScanKeep>(n_blocks, n_experts, e_pad, block_cnt, plan, tiles, max_tiles, tile_shift);
+                                                                    TileRows bm) {
+    plan_experts<kScanKeep>(n_blocks, n_experts, e_pad, block_cnt, plan, tiles, max_tiles, bm);
 }
 
 // The lanes of the wave whose item has this lane's expert: a mask built from one ballot per bit of the expert number.
@@ -252,7 +259,7 @@ __device__ __forceinline__ void place_item(const ItemSource &src, uint32_t i, ui
 constexpr int kSortWaves = kScanThreads / 64, kSortKeep = 3;
 __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource src, uint32_t e_pad, PrefillPlan *__restrict__ plan,
                                                                     PrefillTile *__restrict__ tiles, uint32_t max_tiles,
-                                                                    uint32_t tile_shift, uint32_t *__restrict__ sorted_token,
+                                                                    TileRows bm, uint32_t *__restrict__ sorted_token,
                                                                     uint32_t *__restrict__ sorted_out_row) {
     __shared__ uint32_t sorted[kSortKeep * kScanThreads];
     __shared__ uint32_t cnt[kSortWaves * FFMOE_MAX_EXPERTS];        // [wave][expert]: items counted so far, then the wave's base
@@ -277,7 +284,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
         }
     }
     __syncthreads();
-    const uint32_t n_pairs = plan_experts<4>(kSortWaves, src.n_experts, e_pad, cnt, plan, tiles, max_tiles, tile_shift);
+    const uint32_t n_pairs = plan_experts<4>(kSortWaves, src.n_experts, e_pad, cnt, plan, tiles, max_tiles, bm);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kSortKeep; ++u)
@@ -1281,7 +1288,46 @@ __global__ void prefill_dump_plan_kernel(uint32_t expert, PrefillPlan *plan, Pre
     sorted_out_row[0] = 0;
 }
 
-// Pairs per M-tile, as a shift: below 8 (256 pairs) the chunk goes through prefill_stream_kernel. The line is drawn by the
+// Pairs per M-tile of the grouped GEMMs: 256, or fewer where the gate/up items of the whole chunk then still run at once, a
+// compute unit each - few experts leave most units idle otherwise. From the chunk's size alone: an expert's pairs are taken as
+// normal about the mean with its root as deviation, so it has `full` whole tiles on average and one more with the rest. What
+// an item takes is what dense_tile_rows has measured; where the down product's items take two rounds, the second begins on the
+// units that had the smallest of the first. (Simulated for 19 shapes of 2 to 256 experts at 49 to 2,000 pairs per expert: 1 %
+// off the best on average, worse than 256 pairs at two points.) Router table to combined rows, us at 256 pairs | the rule's, bf16
+// (FP16): 8 experts of 4,096 x 1,536, 96 pairs each 86 | 68 (105 | 92), 192 pairs 108 | 89 (130 | 105); 8 of 2,048 x 704, 256 pairs
+// 75 | 49 (88 | 61); 16 of 2,816 x 704, 192 pairs 82 | 75 (97 | 86). (Blocks of four waves, two to a unit, as the GEMMs had them
+// before, took 80, 103, 68 and 84 there, in FP16 96, 122, 80 and 94.)
+uint32_t gemm_tile_rows(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g, uint32_t n_cus, uint32_t max_tiles) {
+    const float mean = (float)n_items / n_experts, dev = sqrtf(mean), cus = (float)n_cus;
+    const float nb_gu = (float)((g.gu_rb + kGemmTiles - 1) / kGemmTiles), nb_dn = (float)((g.dn_rbp + kGemmTiles - 1) / kGemmTiles);
+    if (n_items / (float)kBM * nb_gu > cus || n_experts * nb_gu > cus) return kBM;
+    uint32_t best = kBM;
+    float least = 0.0f;
+    for (uint32_t rows = kBM; rows >= 32; rows -= 16) {
+        float full = 0.0f, variance = 0.0f;
+        for (float r = (float)rows; r < mean + 4 * dev; r += rows) {
+            const float p = 0.5f * erfcf((r - mean) / (1.41421356f * dev));
+            full += p, variance += p * (1 - p);
+        }
+        // (of a chunk's tiles, the number that three in five chunks stay below)
+        const float tiles = n_experts * (full + 1) + 0.5f * sqrtf(n_experts * variance) - 0.3f;
+        if (rows < kBM && (tiles * nb_gu > cus || n_items / rows + n_experts >= max_tiles)) continue;
+        const float rest = fmaxf(mean - full * rows, 0.5f * dev), size_full = 10 + rows / 16.0f, size_rest = 10 + ceilf(rest / 16);
+        const float largest = full > 0.02f ? size_full : 10 + ceilf(fminf((float)rows, mean + 2 * dev) / 16);
+        auto rounds = [&](float nb) {
+            const float n_full = n_experts * full * nb, n = n_full + n_experts * nb;
+            if (tiles * nb <= cus) return largest;
+            if (n > 2 * cus) return fmaxf(largest, (n_full * size_full + n_experts * nb * size_rest) / cus + 0.5f * size_full);
+            if (n_full > cus) return 2 * size_full;
+            return fmaxf(largest, n + n_full > 2 * cus ? size_full + size_rest : 2 * size_rest);
+        };
+        const float cost = rounds(nb_gu) * (g.gd + 6) + rounds(nb_dn) * (g.gf + 6);
+        if (rows == kBM || cost < least * (best == kBM ? 0.99f : 1.0f)) least = cost, best = rows;
+    }
+    return best;
+}
+
+// Form and pairs per M-tile of a routed chunk. The line between prefill_stream_kernel and the GEMMs is drawn by the
 // pairs per expert on average, from the chunk's size alone: the counts themselves are only known on the device, and a pair
 // list's rows do not depend on how many of the chunk's pairs it names. Up to 28 the streaming product wins at every width.
 // Beyond, up to 48: tiles of 32 pairs still where a tile from every expert would not fill the chip (its blocks then run at once,
@@ -1300,25 +1346,17 @@ __global__ void prefill_dump_plan_kernel(uint32_t expert, PrefillPlan *plan, Pre
 // every size up to 48 pairs (448 rows 146 | 159 | 166 against 186 | 201 | 196 for the GEMMs, 768 rows 192 | 201 | 212 against 225 |
 // 226 | 232). Tiles of 16 pairs gain nothing over 32 (37 rows: 99), tiles of 128 lose everywhere (1,000 rows: 227, two waves per
 // SIMD).
-uint32_t prefill_tile_shift(uint32_t n_items, uint32_t n_experts, uint32_t d, uint32_t n_nblocks, uint32_t n_cus, bool f16) {
-    if (n_items <= 28 * n_experts) return 5;
-    if (n_items > kPrefillStreamPairs * n_experts) return 8;
-    if (n_nblocks * n_experts <= n_cus) return 5;
-    return n_items <= 32 * n_experts || d >= (f16 ? 1536u : 1024u) ? 6 : 8;
-}
-
-// The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths): tiles of 32 rows while the gate/up
-// launch is one round (four blocks per compute unit on the XCD with the most N-blocks), or while a chunk's products are few
-// enough that it cost less than the GEMMs at 256 rows per tile did; at most kDenseTileStreamRows. With tiles of fewer rows the
-// GEMMs are now the faster ones from some 640 rows on (2,816 -> 2,112, 897 rows 62 us, FP16 81, where 896 streamed ones take 78
-// and 98), but their weights are rounded to 16 bits and the streamed ones' are not: a chunk that had the smaller error keeps it.
-// us at 32 | 256 rows per tile, bf16 (FP16): 2,816 -> 2,112, 512 rows 54 | 78 (71 | 107), 800 rows 69 | 79 (88 | 108); 2,816 ->
-// 2,816, 672 rows 70 | 87, 896 rows 94 | 88 (114 | 121); 4,096 -> 2,816, 672 rows 96 | 106, 896 rows 129 | 108 (147 | 142).
-// Streamed tiles of 64 gain nothing (2,816 -> 2,112, 700 rows 71 | 66 at 32).
-uint32_t dense_tile_shift(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, bool f16) {
-    if (t > kDenseTileStreamRows) return 8;
-    const bool one_round = (n_nblocks + 7) / 8 * ((t + 31) / 32) <= 4 * (n_cus / 8);
-    return one_round || (uint64_t)t * g.d * g.f <= (f16 ? 9600000000ull : 6600000000ull) ? 5 : 8;
+struct TileForm {
+    bool streamed;
+    uint32_t rows;
+};
+TileForm prefill_tile_form(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, uint32_t max_tiles, bool f16) {
+    if (n_items <= 28 * n_experts) return {true, 32};
+    if (n_items <= kPrefillStreamPairs * n_experts) {
+        if (n_nblocks * n_experts <= n_cus) return {true, 32};
+        if (n_items <= 32 * n_experts || g.d >= (f16 ? 1536u : 1024u)) return {true, 64};
+    }
+    return {false, gemm_tile_rows(n_items, n_experts, g, n_cus, max_tiles)};
 }
 
 // Rows per M-tile of a dense FFN's GEMMs: 16 n, n chosen so that the items fill their last round. A compute unit takes (10 + n) / 10 of
@@ -1338,9 +1376,23 @@ uint32_t dense_tile_rows(uint32_t t, const ArenaGeom &g, uint32_t n_cus) {
     return best;
 }
 
+// The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths): tiles of 32 rows while the gate/up
+// launch is one round (four blocks per compute unit on the XCD with the most N-blocks), or while a chunk's products are few
+// enough that it cost less than the GEMMs at 256 rows per tile did; at most kDenseTileStreamRows. With tiles of fewer rows the
+// GEMMs are now the faster ones from some 640 rows on (2,816 -> 2,112, 897 rows 62 us, FP16 81, where 896 streamed ones take 78
+// and 98), but their weights are rounded to 16 bits and the streamed ones' are not: a chunk that had the smaller error keeps it.
+// us at 32 | 256 rows per tile, bf16 (FP16): 2,816 -> 2,112, 512 rows 54 | 78 (71 | 107), 800 rows 69 | 79 (88 | 108); 2,816 ->
+// 2,816, 672 rows 70 | 87, 896 rows 94 | 88 (114 | 121); 4,096 -> 2,816, 672 rows 96 | 106, 896 rows 129 | 108 (147 | 142).
+// Streamed tiles of 64 gain nothing (2,816 -> 2,112, 700 rows 71 | 66 at 32).
+TileForm dense_tile_form(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, bool f16) {
+    const bool one_round = (n_nblocks + 7) / 8 * ((t + 31) / 32) <= 4 * (n_cus / 8);
+    if (t <= kDenseTileStreamRows && (one_round || (uint64_t)t * g.d * g.f <= (f16 ? 9600000000ull : 6600000000ull))) return {true, 32};
+    return {false, dense_tile_rows(t, g, n_cus)};
+}
+
 template <bool GATE_UP>
-auto stream_kernel(uint32_t tile_shift, bool f16) {
-    if (tile_shift == 5) return f16 ? prefill_stream_kernel<GATE_UP, 2, true, 4> : prefill_stream_kernel<GATE_UP, 2, false, 4>;
+auto stream_kernel(uint32_t tile_rows, bool f16) {
+    if (tile_rows == 32) return f16 ? prefill_stream_kernel<GATE_UP, 2, true, 4> : prefill_stream_kernel<GATE_UP, 2, false, 4>;
     return f16 ? prefill_stream_kernel<GATE_UP, 4, true, 3> : prefill_stream_kernel<GATE_UP, 4, false, 3>;
 }
 
@@ -1392,24 +1444,24 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     if (src.n_items == 0) return hipSuccess;
     const uint32_t n_blocks = (src.n_items + kSortBlock - 1) / kSortBlock;
     const uint32_t nb_gu = (g.gu_rb + kTilesPerBlock - 1) / kTilesPerBlock, nb_dn = (g.dn_rbp + kTilesPerBlock - 1) / kTilesPerBlock;
-    const uint32_t tile_shift =
-        dense ? dense_tile_shift(t, g, nb_gu, n_cus, f16) : prefill_tile_shift(max(src.n_items, t * top_k), n_experts, g.d, nb_gu, n_cus, f16);
-    const bool streamed = tile_shift < 8;
-    const uint32_t dense_rows = dense && !streamed ? dense_tile_rows(t, g, n_cus) : 1u << tile_shift;
+    const TileForm form = dense ? dense_tile_form(t, g, nb_gu, n_cus, f16)
+                                : prefill_tile_form(max(src.n_items, t * top_k), n_experts, g, nb_gu, n_cus, sc.max_tiles, f16);
+    const bool streamed = form.streamed;
+    const uint32_t tile_rows = form.rows;
     if (dense) {
-        hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, dense_rows, sc.plan, sc.tiles, sc.sorted_token,
+        hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_rows, sc.plan, sc.tiles, sc.sorted_token,
                            sc.sorted_out_row);
     } else {
         uint32_t e_pad = 1;
         while (e_pad < n_experts) e_pad <<= 1;          // n_experts <= FFMOE_MAX_EXPERTS = 256 <= kScanThreads
         if (src.n_items <= (uint32_t)kSortKeep * kScanThreads) {
-            hipLaunchKernelGGL(prefill_sort_kernel, dim3(1), dim3(kScanThreads), 0, s, src, e_pad, sc.plan, sc.tiles, sc.max_tiles, tile_shift,
+            hipLaunchKernelGGL(prefill_sort_kernel, dim3(1), dim3(kScanThreads), 0, s, src, e_pad, sc.plan, sc.tiles, sc.max_tiles, TileRows(tile_rows),
                                sc.sorted_token, sc.sorted_out_row);
         } else {
             hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
             const uint32_t run = (n_blocks + kScanThreads / e_pad - 1) / (kScanThreads / e_pad);     // sort blocks per thread
             hipLaunchKernelGGL((run <= 16 ? prefill_scan_kernel<16> : prefill_scan_kernel<32>), dim3(1), dim3(kScanThreads), 0, s, n_blocks,
-                               n_experts, e_pad, sc.block_cnt, sc.plan, sc.tiles, sc.max_tiles, tile_shift);
+                               n_experts, e_pad, sc.block_cnt, sc.plan, sc.tiles, sc.max_tiles, TileRows(tile_rows));
             hipLaunchKernelGGL(prefill_scatter_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt, sc.sorted_token,
                                sc.sorted_out_row);
         }
@@ -1417,7 +1469,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     timer->mark(s, FFMOE_K_PREFILL_SORT);
-    const uint32_t tile_cap = min(sc.max_tiles, dense ? (t + dense_rows - 1) / dense_rows : (src.n_items >> tile_shift) + n_experts);
+    const uint32_t tile_cap = min(sc.max_tiles, dense ? (t + tile_rows - 1) / tile_rows : src.n_items / tile_rows + n_experts);
     const uint32_t tile_slots = (tile_cap + 7) / 8 * 8;
     if (f16 && !sc.act_scale) return hipErrorInvalidValue;      // allocated when the context was switched to FP16
     // grid: (N-blocks x tile slots) in either order of the kernel's block map
@@ -1435,7 +1487,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
                        arena_layer, g, sc.plan, sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, nb_major,    \
                        act_scale, act_blocks, nullptr)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
-    hipLaunchKernelGGL(stream_kernel<GU>(tile_shift, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
+    hipLaunchKernelGGL(stream_kernel<GU>(tile_rows, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
                        sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major, act_scale, act_blocks)
     if (large_scales) {
         if ((e = launch_prefill_large_scale(s, arena_layer, g, true, tile_cap, x, x_stride, sc.acts, sc, f16)) != hipSuccess) return e;
@@ -1443,7 +1495,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     else FFMOE_GEMM(true, x, x_stride, sc.acts, gemm_gu);
     timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
     if (f16)
-        hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap, ((streamed ? 1u << tile_shift : kBM) / 16 + kPairBlocks - 1) / kPairBlocks), dim3(64 * kPairBlocks), 0, s,
+        hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap, (tile_rows / 16 + kPairBlocks - 1) / kPairBlocks), dim3(64 * kPairBlocks), 0, s,
                            sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale, sc.acts);
     if (large_scales) {
         if ((e = launch_prefill_large_scale(s, arena_layer, g, false, tile_cap, sc.acts, g.f, partials, sc, f16)) != hipSuccess) return e;
