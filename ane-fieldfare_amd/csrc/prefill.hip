@@ -402,7 +402,7 @@ static_assert(kGemmTiles * kTurnBlocks * kGemmTurnBytes <= kGemmABytes && kGemmT
 constexpr uint32_t gemm_lds_bytes(bool gate_up, bool f16) { return gate_up ? kGemmRowAt : f16 ? kGemmLargestAt + 2 * kGemmRowBytes : kGemmLargestAt; }
 
 // One M-tile x N-block, and what a wave needs to ask for its rows: `from` = GATE_UP: in bytes from the first row's start (WIDE, where
-// the rows span 4 GiB or more: in 16-byte pieces); else: in KiB, wave-uniform.
+// the rows span 4 GiB or more: the row); else: in KiB, wave-uniform.
 struct GemmItem {
     bool valid;
     uint32_t parity;                      // of its number among the block's
@@ -448,11 +448,13 @@ struct GemmRings {
     }
 };
 
+// The 16-byte piece of its row's 128 bytes that a lane brings.
+__device__ __forceinline__ uint32_t gemm_row_piece(uint32_t lane) { return (lane & 7) ^ (lane >> 3); }
 // The loads of one group: the k-th KiB of a wave's share of A, its packed tile (k = 0) and that tile's scales (k = 1).
 template <bool GATE_UP, bool F16, bool WIDE>
 __device__ __forceinline__ void gemm_load_a(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, uint32_t grp, uint32_t at, int k) {
     const uint32_t to = lds_base + at + (gw.wave + kGemmTiles * k) * kFragBytes;
-    if constexpr (GATE_UP && WIDE) global_to_lds_16(gw.a + grp * kGroup + (size_t)it.from[k] * 8, to);
+    if constexpr (GATE_UP && WIDE) global_to_lds_16(gw.a + grp * kGroup + (size_t)it.from[k] * gw.a_stride + gemm_row_piece(gw.lane) * 8, to);
     else if constexpr (GATE_UP) global_to_lds_16(gw.a + grp * kGroup, it.from[k], to);
     else global_to_lds_16(gw.a + ((size_t)it.from[k] + 2 * grp) * (kWave * 8), gw.lane * 16, to);
 }
@@ -814,7 +816,8 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
             const uint32_t piece = gw.wave + kGemmTiles * k;
             if constexpr (GATE_UP) {
                 const uint32_t row = min(piece * 8 + (gw.lane >> 3), it.tile.rows - 1);
-                it.from[k] = (sorted_token[it.tile.row_start + row] * (gw.a_stride / 8) + ((gw.lane & 7) ^ (gw.lane >> 3))) * (WIDE ? 1u : 16u);
+                const uint32_t token = sorted_token[it.tile.row_start + row];
+                it.from[k] = WIDE ? token : (token * (gw.a_stride / 8) + gemm_row_piece(gw.lane)) * 16u;
             } else {
                 it.from[k] = __builtin_amdgcn_readfirstlane((it.act_block0 + min(piece >> 1, last_block)) * gw.n_groups * 2 + (piece & 1));
             }

@@ -75,13 +75,15 @@ def test_tiles_by_the_number_of_items(oracle, act, d, f, counts):
     test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts)
 
 
-@pytest.mark.parametrize("act", ["bf16", "fp16"])
-def test_rows_that_span_four_gigabytes(oracle, act):
-    # 99 rows of 2^25 elements' stride: a row's place does not fit 32 bits
+@pytest.mark.parametrize("act,stride", [("bf16", 1 << 24), ("bf16", 1 << 25), ("fp16", 1 << 25), ("bf16", 360_000_000), ("fp16", 360_000_000)])
+def test_rows_that_span_four_gigabytes(oracle, act, stride):
+    # 99 rows 32 MiB apart: a place past 2 GiB; 64 MiB: a row's place in bytes does not fit 32 bits; 720 MB apart: nor does the one in 16-byte pieces
     import torch
     import fieldfare_moe as ff
     ff.lib()
-    d, f, e, t, stride = 256, 192, 2, 99, 1 << 25
+    d, f, e, t = 256, 192, 2, 99
+    if torch.cuda.mem_get_info()[0] < t * stride * 2 + (4 << 30):
+        pytest.skip("the card's free memory does not hold the rows")
     rng, pool, _ = make_layer(oracle, 9, d, f, e, align=1)
     ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=t, act_dtype=act)
     try:
@@ -92,9 +94,14 @@ def test_rows_that_span_four_gigabytes(oracle, act):
         w = torch.from_numpy(rng.uniform(0.2, 1.0, (t, 1)).astype(np.float32)).to(dt).cuda()
         far = torch.empty(((t - 1) * stride + d,), dtype=dt, device="cuda").as_strided((t, d), (stride, 1))
         far.copy_(x)
-        assert torch.equal(ctx.prefill(0, far, idx, w), ctx.prefill(0, x, idx, w))
+        near = ctx.prefill(0, x, idx, w)
+        assert torch.isfinite(near).all() and near.abs().max() > 0
+        ctx.prefill(0, -x, idx, w)                              # (nothing of the rows stays in the scratch)
+        assert torch.equal(ctx.prefill(0, far, idx, w, out=torch.full_like(near, float("nan"))), near)
     finally:
         ctx.close()
+        far = None
+        torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
