@@ -31,7 +31,6 @@ struct TileRows {
     uint32_t rows, divide;
     __host__ __device__ explicit TileRows(uint32_t r) : rows(r), divide((uint32_t)(((1ull << 32) + r - 1) / r)) {}
     __device__ __forceinline__ uint32_t whole(uint32_t n) const { return __umulhi(n, divide); }
-    __device__ __forceinline__ uint32_t rest(uint32_t n) const { return n - whole(n) * rows; }
 };
 constexpr int kBM = FFMOE_PREFILL_TILE_M;   // pairs per M-tile
 constexpr int kTilesPerBlock = 4;           // arena tiles (of 16 + 16 rows) per N-block
@@ -82,7 +81,7 @@ template <int kScanKeep>
 __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad, uint32_t *__restrict__ block_cnt,
                                              PrefillPlan *__restrict__ plan, PrefillTile *__restrict__ tiles, uint32_t max_tiles,
                                              TileRows bm) {
-    __shared__ uint32_t total[FFMOE_MAX_EXPERTS];
+    __shared__ uint32_t total[FFMOE_MAX_EXPERTS], last_rows[FFMOE_MAX_EXPERTS];    // pairs, and those past the whole tiles
     __shared__ uint32_t offset[FFMOE_MAX_EXPERTS + 1];
     __shared__ uint32_t tile_off[FFMOE_MAX_EXPERTS + 1];
     __shared__ uint32_t part[kScanThreads];                 // [chunk][e_pad]: chunk sums, then chunk bases
@@ -122,7 +121,9 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
     if (threadIdx.x < FFMOE_MAX_EXPERTS) {
         const uint32_t i = threadIdx.x, lane = i & 63, wv = i >> 6;
         const uint32_t n = i < n_experts ? total[i] : 0;
-        const unsigned long long own = ((unsigned long long)bm.whole(n + bm.rows - 1) << 32) | n;
+        const uint32_t whole = bm.whole(n), rest = n - whole * bm.rows;
+        last_rows[i] = rest;
+        const unsigned long long own = ((unsigned long long)(whole + (rest != 0 ? 1u : 0u)) << 32) | n;
         unsigned long long inc = own;
 #pragma unroll
         for (int sh = 1; sh < 64; sh <<= 1) {
@@ -148,7 +149,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
             unsigned long long all = ex;
             if (i != n_experts) {
                 const uint32_t n = total[i];
-                all += ((unsigned long long)bm.whole(n + bm.rows - 1) << 32) | n;
+                all += ((unsigned long long)(bm.whole(n) + (last_rows[i] != 0 ? 1u : 0u)) << 32) | n;
                 offset[n_experts] = (uint32_t)all;
                 tile_off[n_experts] = (uint32_t)(all >> 32);
             }
@@ -164,11 +165,11 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
     // anywhere in the expert order). Where an expert's shorter tile goes takes a look at every other expert's: the
     // threads of an expert share that out (one thread alone is a chain of two thousand instructions).
     if (live) {
-        const uint32_t rest = bm.rest(total[e]), per_o = (e_pad + chunks - 1) / chunks;
+        const uint32_t rest = last_rows[e], per_o = (e_pad + chunks - 1) / chunks;
         const uint32_t o_lo = min(e_pad, ch * per_o), o_hi = min(e_pad, o_lo + per_o);
         uint32_t all = 0, in_front = 0, above = 0;
         for (uint32_t o = o_lo; o < o_hi; ++o) {
-            const uint32_t r = bm.rest(total[o]);              // experts past n_experts hold zero
+            const uint32_t r = last_rows[o];                   // experts past n_experts hold zero
             const uint32_t has = r != 0 ? 1u : 0u;
             all += has;
             in_front += has & (o < e ? 1u : 0u);
@@ -198,7 +199,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
     plan->expert_offset[e] = offset[e];
     plan->expert_count[e] = total[e];
     // a tile keeps its number in row order, which places its activation blocks
-    const uint32_t nt = bm.whole(total[e] + bm.rows - 1), n_full = bm.whole(total[e]);
+    const uint32_t n_full = bm.whole(total[e]), nt = n_full + (last_rows[e] != 0 ? 1u : 0u);
     const uint32_t shorter_tiles = shorter[0][e], shorter_in_front = shorter[1][e], ranked_above = shorter[2][e];
     const uint32_t full_in_front = tile_off[e] - shorter_in_front, full_tiles = tile_off[n_experts] - shorter_tiles;
     for (uint32_t i = 0; i < nt; ++i) {
