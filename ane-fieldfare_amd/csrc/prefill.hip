@@ -1308,8 +1308,8 @@ uint32_t gemm_tile_rows(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g
     uint32_t best = kBM;
     float least = 0.0f;
     for (uint32_t rows = kBM; rows >= 32; rows -= 16) {
-        float full = 0.0f, variance = 0.0f;
-        for (float r = (float)rows; r < mean + 4 * dev; r += rows) {
+        float full = floorf(fmaxf(mean - 4 * dev, 0.0f) / rows), variance = 0.0f;       // (every expert has these)
+        for (float r = (full + 1) * rows; r < mean + 4 * dev; r += rows) {
             const float p = 0.5f * erfcf((r - mean) / (1.41421356f * dev));
             full += p, variance += p * (1 - p);
         }
