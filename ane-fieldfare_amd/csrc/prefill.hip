@@ -1186,45 +1186,68 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_
 // threadgroup with `relative` and `pair_scale` as it takes the rows in (prefill.metal:731-741). Done there, every wave of the
 // down products scaled every operand of its tile again: 8,000 pairs of 704 over 128 experts, down 82 us and this pass, scales
 // only, 7 -> 68 + 10; the call with 62, 125 and 192 pairs per expert 215 -> 208, 301 -> 289 and 396 -> 375 us.
-// A wave per 16-pair block; a pair's blocks that have its largest scale stay as they are. Bound: memory's latency.
-constexpr int kPairBlocks = 2;                              // of a block
-__global__ __launch_bounds__(64 * kPairBlocks) void prefill_pair_scale_kernel(const PrefillPlan *__restrict__ plan,
-                                                                              const PrefillTile *__restrict__ tiles, uint32_t groups,
-                                                                              uint32_t act_blocks, float *__restrict__ act_scale,
-                                                                              uint16_t *__restrict__ acts) {
+// PARTS waves per 16 pairs, each with every PARTS-th block of 64: the wave's first activations are on their way while the scales are
+// read, whose largest meet in LDS. Where any of the 16 pairs is off its largest all of them are stored (times one: the same), as
+// whole lines. Bound: memory's latency with few pairs, its rate with many. One wave per 16 pairs, skipping lanes | this: one expert,
+// 512 rows, width 2,816 19.9 | 6.3 us, width 2,112 15.7 | 5.2, the call 55.3 | 41; 3,072 rows top-8 of 128 of width 704 17.5 | 14.6.
+// A layer of width 256 has nothing to share out and keeps one wave: 65,536 pairs, PARTS 4 | 2 | 1 14.3 | 12.6 | 11.8 us. There,
+// with few columns in the down product (512), scaling in the products took 7 us less in all (of 135); at 2,816 columns it took more.
+constexpr int kPairWaves = 4;                               // of a block
+template <int PARTS>
+__global__ __launch_bounds__(64 * kPairWaves) void prefill_pair_scale_kernel(const PrefillPlan *__restrict__ plan,
+                                                                             const PrefillTile *__restrict__ tiles, uint32_t groups,
+                                                                             uint32_t act_blocks, float *__restrict__ act_scale,
+                                                                             uint16_t *__restrict__ acts) {
+    __shared__ float peaks[kPairWaves][16];
     if (blockIdx.x >= plan->n_tiles) return;
     const PrefillTile tile = tiles[blockIdx.x];
-    const uint32_t lane = threadIdx.x & 63, j = lane & 15, jq = lane >> 4, in_tile = blockIdx.y * kPairBlocks + (threadIdx.x >> 6);
-    if (in_tile * 16 >= tile.rows) return;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = wave % PARTS, j = lane & 15, jq = lane >> 4;
+    const uint32_t in_tile = blockIdx.y * (kPairWaves / PARTS) + wave / PARTS;
+    if (in_tile * 16 >= tile.rows) return;                  // (PARTS = 4: the whole block)
     const bool live = in_tile * 16 + j < tile.rows;
     const uint32_t block = tile.row_start / 16 + tile.order + in_tile;
     const float *const s = act_scale + (size_t)block * groups * 16 + j;
-    float largest = 0.0f;
-    for (uint32_t b = jq; b < groups; b += 4) largest = fmaxf(largest, s[b * 16]);
-    largest = fmaxf(largest, __shfl_xor(largest, 16, 64));
-    largest = fmaxf(largest, __shfl_xor(largest, 32, 64));
-    const float inv = 1.0f / largest;          // a scale is 2^(e - 14) with e >= -100: never zero
     uint4 *const a = reinterpret_cast<uint4 *>(acts) + (size_t)block * groups * (2 * kWave) + lane;
-    constexpr int kAhead = 6;
-    for (uint32_t b0 = 0; b0 < groups; b0 += kAhead) {
-        uint4 v[kAhead][2];
-        float rel[kAhead];
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) rel[u] = live && b0 + u < groups ? s[(b0 + u) * 16] * inv : 1.0f;
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u)
-            if (__ballot(rel[u] != 1.0f)) v[u][0] = a[(b0 + u) * (2 * kWave)], v[u][1] = a[(b0 + u) * (2 * kWave) + kWave];
+    constexpr int kAhead = PARTS == 1 ? 4 : 3;
+    uint4 v[kAhead][2];
+    float own[kAhead];
+    auto load = [&](uint32_t b0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {
-            if (rel[u] == 1.0f) continue;
-            const f16x2 r2 = __builtin_bit_cast(f16x2, Act<true>::pack(rel[u], rel[u]));
+            const uint32_t b = min(b0 + u * PARTS, groups - 1);            // past the last: read, not used
+            v[u][0] = a[b * (2 * kWave)], v[u][1] = a[b * (2 * kWave) + kWave];
+            own[u] = s[b * 16];
+        }
+    };
+    load(part);
+    float largest = 0.0f;
+#pragma unroll 4
+    for (uint32_t b = part * 4 + jq; b < groups; b += 4 * PARTS) largest = fmaxf(largest, s[b * 16]);
+    largest = fmaxf(largest, __shfl_xor(largest, 16, 64));
+    largest = fmaxf(largest, __shfl_xor(largest, 32, 64));
+    if constexpr (PARTS > 1) {
+        static_assert(PARTS == kPairWaves, "the waves of a block meet");
+        if (jq == 0) peaks[wave][j] = largest;
+        lds_barrier();
+#pragma unroll
+        for (int w = 0; w < PARTS; ++w) largest = fmaxf(largest, peaks[w][j]);
+    }
+    const float inv = 1.0f / largest;          // a scale is 2^(e - 14) with e >= -100: never zero
+    for (uint32_t b0 = part; b0 < groups; b0 += kAhead * PARTS) {
+        if (b0 != part) load(b0);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t b = b0 + u * PARTS;
+            const float rel = live ? own[u] * inv : 1.0f;
+            if (b >= groups || !__ballot(rel != 1.0f)) continue;
+            const f16x2 r2 = __builtin_bit_cast(f16x2, Act<true>::pack(rel, rel));
             auto times = [&](uint32_t x) __attribute__((always_inline)) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, x) * r2); };
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                a[(b0 + u) * (2 * kWave) + h * kWave] = uint4{times(v[u][h].x), times(v[u][h].y), times(v[u][h].z), times(v[u][h].w)};
+                a[b * (2 * kWave) + h * kWave] = uint4{times(v[u][h].x), times(v[u][h].y), times(v[u][h].z), times(v[u][h].w)};
         }
     }
-    if (live && jq == 0) act_scale[(size_t)act_blocks * groups * 16 + block * 16 + j] = largest;
+    if (live && jq == 0 && part == 0) act_scale[(size_t)act_blocks * groups * 16 + block * 16 + j] = largest;
 }
 
 // h2[t][c] = bf16(sum_r w[t][r] * partial[t][r][c]) over the routes the sort kept, fma in rank order
@@ -1498,9 +1521,12 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     } else if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);
     else FFMOE_GEMM(true, x, x_stride, sc.acts, gemm_gu);
     timer->mark(s, FFMOE_K_PREFILL_GATE_UP);
-    if (f16)
-        hipLaunchKernelGGL(prefill_pair_scale_kernel, dim3(tile_cap, (tile_rows / 16 + kPairBlocks - 1) / kPairBlocks), dim3(64 * kPairBlocks), 0, s,
+    if (f16) {
+        const bool one = g.gf <= 4;
+        hipLaunchKernelGGL((one ? prefill_pair_scale_kernel<1> : prefill_pair_scale_kernel<kPairWaves>),
+                           dim3(tile_cap, one ? (tile_rows / 16 + kPairWaves - 1) / kPairWaves : tile_rows / 16), dim3(64 * kPairWaves), 0, s,
                            sc.plan, sc.tiles, g.gf, sc.act_blocks, sc.act_scale, sc.acts);
+    }
     if (large_scales) {
         if ((e = launch_prefill_large_scale(s, arena_layer, g, false, tile_cap, sc.acts, g.f, partials, sc, f16)) != hipSuccess) return e;
     } else if (streamed) FFMOE_STREAM(false, sc.acts, g.f, partials, nb_dn);
