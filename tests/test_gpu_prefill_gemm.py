@@ -66,11 +66,11 @@ def test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts):
 
 
 # Tiles of fewer than 256 pairs, where few experts leave compute units idle: of 128, 64 and 32 pairs, all of a chunk in one expert (as
-# many tiles as there can be), one expert; and whole tiles on long gate/up rings, which take more items than there are units.
+# many tiles as there can be), one expert, no more than a uniform chunk's experts have (80); and whole tiles on long gate/up rings, which take more items than there are units.
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,f,counts", [(320, 1536, (192, 130, 256, 257, 128, 1, 0, 300)), (320, 1536, (0, 0, 1300, 0, 0, 3, 0, 0)),
                                         (320, 1536, (63, 64, 65, 31, 96, 129, 0, 128)), (192, 320, (1000, 24)), (192, 320, (31, 32, 33, 65, 96, 97)),
-                                        (448, 384, (700,)), (448, 384, (290,)), (192, 704, LONG), (1408, 704, LONG)])
+                                        (448, 384, (700,)), (448, 384, (290,)), (192, 1536, (700,) + 15 * (9,)), (192, 1536, (1900,) + 39 * (5,)), (192, 704, LONG), (1408, 704, LONG)])
 def test_tiles_by_the_number_of_items(oracle, act, d, f, counts):
     test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts)
 
