@@ -199,6 +199,12 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     const uint32_t g_last = g1 > g0 ? g1 - 1 : n_groups - 1;
     const TileSource src = make_tile_source(tiles, (size_t)n_tiles * n_groups * kTileBytes, scales,
                                             (size_t)n_tiles * n_groups * kTileScaleBytes);
+    // 17 to 32 input rows of the plain 16-bit form: grid row 1 takes those past the 16th and reads the weights again, then from the caches
+    if (!(Y_F32 || GREEDY || PLANES8 || GLU)) {
+        x += (size_t)blockIdx.y * FFMOE_MAX_VERIFY_ROWS * x_stride;
+        y_ = reinterpret_cast<uint16_t *>(y_) + (size_t)blockIdx.y * FFMOE_MAX_VERIFY_ROWS * y_stride;
+        rows = min((uint32_t)FFMOE_MAX_VERIFY_ROWS, rows - blockIdx.y * FFMOE_MAX_VERIFY_ROWS);
+    }
     WeightRing ring;
 #pragma unroll
     for (int u = 0; u < kRing; ++u) ring_fill(ring, u, src, rb0 * n_groups + min(g0 + u, g_last), lane);
@@ -680,7 +686,11 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
     const uint32_t n_tiles = (planes8 || glu == 2) ? (m + 15) / 16 : (m + 31) / 32;      // glu == 1: pairs of tiles
     if (rows == 0 || rows > (1u << 20) || (rows > FFMOE_MAX_VERIFY_ROWS ? y_f32 : glu == 2)) return hipErrorInvalidValue;
     const uint32_t all_tiles = glu == 1 ? 2 * n_tiles : n_tiles;
-    if (rows > FFMOE_MAX_VERIFY_ROWS) {
+    // 17 to 32 rows of the plain 4-bit form: beyond 24 groups the GEMV's two grid rows, all of whose weights are on their way at once,
+    // beat the band's chain of groups. Gate/up in a band, then down bands | GEMV, us at 17 rows: 2,816 columns out, K of 1,024 12.3 | 13.3,
+    // 1,408 13.2 | 13.5, 1,600 13.6 | 13.5, 2,112 14.5 | 13.5, 2,816 15.4 | 14.0; 512 out, K of 1,792 10.1 | 10.0, 2,816 11.7 | 10.4.
+    const bool twice = rows > FFMOE_MAX_VERIFY_ROWS && rows <= 2 * FFMOE_MAX_VERIFY_ROWS && glu == 0 && !planes8 && n / kGroup > 6 * kKSplit;
+    if (rows > FFMOE_MAX_VERIFY_ROWS && !twice) {
         const BandShape shape = band_shape(rows, all_tiles, n / kGroup, n_cus);
         const uint32_t bands = ((rows + 15) / 16 + shape.blocks - 1) / shape.blocks, per_block = kBandWaves / shape.parts;
         const dim3 grid((bands * ((all_tiles + per_block - 1) / per_block) + 7) / 8 * 8);
@@ -707,7 +717,9 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
 #undef FFMOE_BAND
         return hipGetLastError();
     }
-    const dim3 grid(min(2 * n_cus, n_tiles));
+    // (two grid rows: a multiple of 8 blocks per row keeps a tile on one XCD, blocks go to the XCDs round robin, and its L2 serves the
+    // second; blocks past the tile count leave at once)
+    const dim3 grid(twice ? (min(2 * n_cus, n_tiles) + 7) / 8 * 8 : min(2 * n_cus, n_tiles), twice ? 2 : 1);
 #define FFMOE_MGEMV(Y, H, P, G)                                                                                             \
     hipLaunchKernelGGL((matrix_gemv_kernel<Y, H, false, false, P, G>), grid, dim3(256), 0, s, tiles, scales, m, n / kGroup, x, x_stride, \
                        rows, y, y_stride)

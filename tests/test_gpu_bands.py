@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(64, 64, (17, 33, 191)), (320, 192, (31, 64, 190)), (576, 2816, (17, 40, 97, 129, 161, 191)), (2816, 576, (18, 47, 129, 191)),
-          (2816, 2816, (17, 33, 49, 65, 81, 97, 129, 145, 177, 191)), (192, 1472, (100, 191))]
+          (2816, 2816, (17, 32, 33, 49, 65, 81, 97, 129, 145, 177, 191)), (192, 1472, (100, 191)), (64, 1536, (17, 32, 33)), (192, 1600, (17, 32, 33))]
 
 
 def _context(ff, oracle, torch, act, d, f, bits, cap):
