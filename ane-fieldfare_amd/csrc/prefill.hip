@@ -1189,7 +1189,7 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_
 // PARTS waves per 16 pairs, each with every PARTS-th block of 64: the wave's first activations are on their way while the scales are
 // read, whose largest meet in LDS. Where any of the 16 pairs is off its largest all of them are stored (times one: the same), as
 // whole lines. Bound: memory's latency with few pairs, its rate with many. One wave per 16 pairs, skipping lanes | this: one expert,
-// 512 rows, width 2,816 19.9 | 6.3 us, width 2,112 15.7 | 5.2, the call 55.3 | 41; 3,072 rows top-8 of 128 of width 704 17.5 | 14.6.
+// 512 rows, width 2,816 19.9 | 6.3 us, width 2,112 15.7 | 5.2, the calls 55.3 | 42.3 and 69.5 | 57.9; 3,072 rows top-8 of 128 of width 704 17.5 | 14.6.
 // A layer of width 256 has nothing to share out and keeps one wave: 65,536 pairs, PARTS 4 | 2 | 1 14.3 | 12.6 | 11.8 us. There,
 // with few columns in the down product (512), scaling in the products took 7 us less in all (of 135); at 2,816 columns it took more.
 constexpr int kPairWaves = 4;                               // of a block

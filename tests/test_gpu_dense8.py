@@ -1,6 +1,6 @@
 """The 8-bit dense layer's GEMMs on integer operands (640 rows and more): ragged row tiles either side of the tile sizes, an
 output width that fills half a block of columns, widths of an odd number of groups, both activation types, inputs with a large
-common part (so that the bias columns carry most of a sum), rows that overflow. Run on the GPU box: pytest -m gpu."""
+common part (so that the bias columns carry most of a sum), rows that overflow. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ def _gelu(x):
 
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
-# the last four: 64-row tiles in both products, 128 in the plain one alone, in the gated one alone, in both
+# K of one group to 44, output widths of a quarter of a 256-row block to eleven blocks
 @pytest.mark.parametrize("d,f,t", [(128, 64, 640), (192, 320, 641), (64, 704, 703), (192, 1472, 1088), (448, 192, 1089), (2816, 128, 1153),
                                    (192, 2816, 1025), (2112, 2112, 1217)])
 def test_rows_against_float64(oracle, act, d, f, t):
@@ -171,6 +171,8 @@ def test_tiles_of_the_row_count(oracle, act, d, f, rows):
         unit = 2.0 ** (-8 if act == "bf16" else -11)         # the bound of test_rows_against_float64
         assert np.all(np.abs(y[some].float().cpu().numpy() - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
         for n in rows:
-            assert torch.equal(ctx.dense_ffn(0, x[:n].cuda()), y[:n]), n
+            # (after rows of NaN through the scratch and into NaN: what is not written is not equal)
+            ctx.dense_ffn(0, torch.full_like(x, float("nan")).cuda())
+            assert torch.equal(ctx.dense_ffn(0, x[:n].cuda(), out=torch.full_like(y[:n], float("nan"))), y[:n]), n
     finally:
         ctx.close()

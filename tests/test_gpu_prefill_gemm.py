@@ -1,5 +1,5 @@
 """The prefill's grouped GEMMs: M-tiles of every number of 16-pair blocks (and one, two and no pairs past a block), plans whose
-largest tile is at most half a tile (deeper rings of packed tiles), K of one group, of fewer and of more than the rings hold,
+largest tile is at most half a tile, K of one group, of fewer and of more than the rings hold,
 N-blocks that are full, half full and a quarter full, fewer and more items than compute units, both activation types; rows that
 span more than 4 GiB. Needs a GPU: pytest -m gpu."""
 import numpy as np
@@ -125,6 +125,8 @@ def test_dense_tiles_of_the_row_count(oracle, act, d, f, rows):
         some = np.r_[0:200, t - 200:t]
         _check(oracle, pool, 1, np.zeros((len(some), 1), np.uint32), x[some], torch.ones((len(some), 1), dtype=dt), y.float().cpu().numpy()[some], act)
         for n in rows:
-            assert torch.equal(ctx.dense_ffn(0, x[:n].cuda()), y[:n]), n
+            # (after rows of NaN through the scratch and into NaN: what is not written is not equal)
+            ctx.dense_ffn(0, torch.full_like(x, float("nan")).cuda())
+            assert torch.equal(ctx.dense_ffn(0, x[:n].cuda(), out=torch.full_like(y[:n], float("nan"))), y[:n]), n
     finally:
         ctx.close()

@@ -1,5 +1,6 @@
 """The prefill's sort of routes in one launch (3,072 items and fewer) and in three: the same rows, bit for bit, from a chunk and from its
-beginning on either side of the line, counts per expert, routes of weight zero and experts past the last left out. Needs a GPU: pytest -m gpu."""
+beginning on either side of the line and from lists of pairs, counts per expert, routes of weight zero and experts past the last left
+out. What a call does not write is NaN. (The order of an expert's pairs shows in no result.) Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 
@@ -28,19 +29,42 @@ def test_one_launch_sorts_as_three_do(oracle, e, k, cuts):
             live = (w[:n] > 0) & (routes[:n] < e)
             return np.bincount(routes[:n][live], minlength=e)
 
-        whole = ctx.prefill(0, x, gi, gw)                       # 3,072 + 5 k items: three launches
+        def rows(n, routes, weights):
+            # whatever a lost or doubled route leaves unwritten is NaN: the routes' rows in the scratch and the output rows
+            ctx.prefill(0, torch.full_like(x, float("nan")), gi, torch.ones_like(gw))
+            y = ctx.prefill(0, x[:n], routes[:n].contiguous(), weights[:n].contiguous(), out=torch.full_like(x[:n], float("nan")))
+            return y, ctx.prefill_stats()
+
+        whole, stats = rows(t, gi, gw)                          # 3,072 + 5 k items: three launches
         assert torch.isfinite(whole.float()).all() and whole.abs().max() > 0
-        assert np.array_equal(ctx.prefill_stats()[2], counts(t, idx))
+        assert np.array_equal(stats[2], counts(t, idx))
         for n in cuts:                                          # (the same products as the whole chunk's: equal bit for bit)
-            part = ctx.prefill(0, x[:n], gi[:n].contiguous(), gw[:n].contiguous())
-            assert np.array_equal(ctx.prefill_stats()[2], counts(n, idx)), n
+            part, stats = rows(n, gi, gw)
+            assert np.array_equal(stats[2], counts(n, idx)), n
             assert torch.equal(part, whole[:n]), n
-        past = idx.copy()
-        past[rng.random((t, k)) < 0.2] = e + 3
+        # experts past the last: as if the routes had weight zero
+        lost = rng.random((t, k)) < 0.2
+        past = torch.from_numpy(np.where(lost, e + 3, idx).astype(np.int32)).cuda()
+        less = gw.masked_fill(torch.from_numpy(lost).cuda(), 0)
         for n in (cuts[-1], t):
-            ctx.prefill(0, x[:n], torch.from_numpy(past[:n].view(np.int32)).cuda(), gw[:n].contiguous())
-            n_pairs, _, got = ctx.prefill_stats()
-            assert np.array_equal(got, counts(n, past)) and n_pairs == got.sum(), n
+            got, (n_pairs, _, per_expert) = rows(n, past, gw)
+            assert np.array_equal(per_expert, counts(n, np.where(lost, e + 3, idx))) and n_pairs == per_expert.sum(), n
+            assert torch.equal(got, rows(n, gi, less)[0]), n
+        # a list of pairs in any order, its first 3,072 (one launch) and all of it (three): the rows that are listed, no others
+        token, rank = (v.reshape(-1) for v in np.divmod(rng.permutation(t * k), k))
+        lists = np.stack([token, np.where((w > 0) & ~lost, idx, e + 3)[token, rank], rank, np.zeros_like(token)], 1).astype(np.int32)
+        kept = torch.from_numpy(lists[:, 1] < e).cuda()
+        got = []
+        for n in (t * k, 3072):
+            ctx.prefill(0, torch.full_like(x, float("nan")), gi, torch.ones_like(gw))
+            out = torch.full((t * k, d), float("nan"), dtype=x.dtype, device="cuda")
+            ctx.prefill_pairs(0, x, torch.from_numpy(lists[:n].copy()).cuda(), t, out)
+            assert np.array_equal(ctx.prefill_stats()[2], np.bincount(lists[:n, 1], minlength=e + 4)[:e]), n
+            got.append(out[torch.from_numpy(token * k + rank).cuda()])      # in the list's order
+        all_rows, first = got
+        assert torch.isfinite(all_rows[kept]).all() and torch.isnan(all_rows[~kept]).all()
+        assert torch.equal(first[:3072][kept[:3072]], all_rows[:3072][kept[:3072]])
+        assert torch.isnan(first[3072:]).all() and torch.isnan(first[:3072][~kept[:3072]]).all()
     finally:
         ctx.close()
 
