@@ -40,11 +40,11 @@ struct ffmoe_layer {
 };
 
 // From this many rows on an 8-bit dense layer goes through the library's dense GEMM on hi / lo rows instead of the resident-matrix
-// products (drawn where those were a pass per 16 rows, and kept with the bits on either side: 2,816 -> 2,112 -> 2,816, 190 rows 43 us
-// in bands of rows, 66 in passes; the GEMM form 50 us at 128, 58 at 192, 67 at 256).
+// products (drawn where those were a pass per 16 rows, and kept with the bits on either side: 2,816 -> 2,112 -> 2,816, in bands of rows
+// 35 us at 160, 38 at 191, where passes took 66; the GEMM form 48 at 250, 52 at 384, 61 at 512).
 constexpr uint32_t kGemm8MinRows = 192;
 // Up to this many rows a 4-bit dense layer takes the resident-matrix products on its arena tiles (bands of input rows) instead of
-// the grouped products: 2,816 -> 2,112 -> 2,816, 301 rows 39 us against 41 in bf16 and 58 in FP16, 384 rows 46 against 45 and 63.
+// the grouped products: 2,816 -> 2,112 -> 2,816, 301 rows 32 us against 41 in bf16 and 47 in FP16, 384 rows 39 against 46 and 51.
 // The rows of a chunk and of a part of it are equal bit for bit up to here.
 constexpr uint32_t kDenseStreamMaxRows = 384;
 

@@ -48,7 +48,6 @@ __device__ __forceinline__ float gelu_tanh_fast(float x) {
 // Arena nibble order inside one dword: nibble position m (m = 0..3) holds element 2m of the lane's
 // eight k-slots and position m + 4 holds element 2m + 1, so that ((w >> 4m) & 0x000F000F) is the
 // 16-bit pair (element 2m, element 2m + 1) with no cross-lane or cross-register shuffling.
-//
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -216,6 +215,9 @@ __device__ __forceinline__ float wave_butterfly_sum(float v) {
     v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     return row_butterfly_sum<16>(v);
 }
+// The same sums (same operands in every addition) through the LDS crossbar: for kernels that reduce many
+// independent values per wave and have the vector ALU busy with other work, where throughput counts and the
+// latency of a step does not.
 __device__ __forceinline__ float wave_butterfly_sum_shuffle(float v) {
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, 64);

@@ -312,8 +312,9 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
 // the products and their sums one behind the other), beyond that the products and the sums themselves, a third of the products
 // being the inputs' own sums, which every wave makes anew. Kept out, as they change nothing: the sums between the products or
 // behind six of them, with and without a raised wave priority. 2,816 -> 2,112 -> 2,816, 4 bits, us of gate/up + down with the GEMV's
-// passes of 16 rows | now: 17 rows 10 + 7 | 9 + 8, 96 rows 17 + 12 | 12 + 10, 190 rows 28 + 18 | 17 + 12, 301 rows 39 + 24 | 22 +
-// 17, 384 rows 46 + 29 | 25 + 20; 8 bits, 37 rows 14 + 13 | 14 + 10, 190 rows 36 + 30 | 25 + 20.
+// passes of 16 rows | now: 96 rows 14 + 11 | 10 + 9, 190 rows 25 + 17 | 16 + 11, 301 rows 37 + 23 | 22 + 13, 384 rows 44 + 29 | 25 +
+// 17 (17 rows 7.7 + 5.8 | 7.5 + 6.7: the down product of up to 32 keeps the passes, launch_matrix_gemv); 8 bits, 17 rows 10.8 + 7.4 | 9.3
+// + 6.8, 37 rows 11.5 + 11.1 | 11.6 + 8.5, 190 rows 34 + 29 | 25 + 16.
 constexpr int kBandWaves = 8, kBandMax = 5;
 template <int PARTS, int R> struct Band {
     static constexpr int tiles = kBandWaves / PARTS, slices = kKSplit / PARTS;

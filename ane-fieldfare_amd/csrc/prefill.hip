@@ -256,7 +256,9 @@ __device__ __forceinline__ void place_item(const ItemSource &src, uint32_t i, ui
 // A chunk of few items in one launch: the three kernels' work by one block, the waves in place of the sort blocks - wave w has a
 // contiguous run of items, 64 at a time, and counts them in LDS; an item's place is what its wave counted before it. Same
 // order. Bound: latencies one behind the other, and 1.6 us per 1,024 items, which is why it ends at kSortKeep of them: a call with
-// three launches | with one, top-8 of 128, 37 rows 101.5 us | 99, 301 rows 133.7 | 131.9, 512 rows 160.9 | 161.2, 1,000 rows 191 | 196.
+// three launches | with one, top-8 of 128, 37 rows 101.5 us | 99, 384 rows 130.2 | 128.6, 512 rows 160.9 | 161.2, 1,000 rows 191 | 196.
+// At 3,072 items one launch is the faster in every shape timed: top-8 of 64 45.5 | 43.5, of 256 39.9 | 39.2, top-4 of 32 and of 60
+// 87.4 | 85.2 and 74.3 | 72.2, top-2 of 16 75.9 | 73.7, top-1 of 4 62.8 | 60.7; at 1,024 items by 3 to 4 us.
 constexpr int kSortWaves = kScanThreads / 64, kSortKeep = 3;
 __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource src, uint32_t e_pad, PrefillPlan *__restrict__ plan,
                                                                     PrefillTile *__restrict__ tiles, uint32_t max_tiles,
@@ -746,7 +748,8 @@ __device__ __forceinline__ bool prefill_block(uint32_t n_nblocks, bool nb_major,
     return true;
 }
 
-// F16: a context in FP16 mode - FP16 rows in, FP16 tiles, block-scaled FP16 activations, FP16 per-route rows out
+// F16: a context in FP16 mode - FP16 rows in, FP16 tiles, block-scaled FP16 activations, FP16 per-route rows out. (The FP16 gate/up
+// kernel is 12 registers over its 256; what it spills is reloaded outside the loop over groups.)
 // A block per compute unit, which works off its share of the XCD's items one after the other: an item's first loads then travel
 // during the epilogue of the one before.
 template <bool GATE_UP, bool F16 = false, bool WIDE = false, bool DUMP = false>
@@ -886,10 +889,10 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Grouped product for chunks whose experts hold few pairs each (a short prompt): same tiles, same N-blocks and same
-// activation layout as the GEMM above, another way through them. There the expansion to 16-bit weights (some 120 vector
-// instructions per 1 KiB tile, whatever the pairs) bounds the launch below about 50 pairs per expert: 90 us for the
-// 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s. Here a wave owns one arena tile row for the whole of K, streams its
+// Grouped product for chunks whose experts hold few pairs each (a short prompt): the GEMM's tiles and activation layout, N-blocks of
+// four arena tiles, another way through them. There the expansion to 16-bit weights (68 vector instructions per 1 KiB tile of
+// a wave, whatever the pairs, in front of its products) bounds the launch below about 50 pairs per expert: with the GEMMs that this
+// form was built beside, 90 us for the 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s. Here a wave owns one arena tile row for the whole of K, streams its
 // packed tiles through a ring of four and multiplies them in the offset form of the decode kernels (stream.hpp): about 75
 // vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. The pairs' rows go through LDS in
 // operand order, two groups at a time in two buffers, so that every wave of the block reads the same fragments and the

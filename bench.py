@@ -91,7 +91,7 @@ def clocks_under_load(burst, torch):
         seen = [(current(c + "/pp_dpm_sclk"), current(c + "/pp_dpm_mclk"), c) for c in cards]
         torch.cuda.synchronize()
         mhz = lambda v: int("".join(ch for ch in (v or "0") if ch.isdigit()) or 0)
-        sclk, mclk, card = max(seen, key=lambda r: mhz(r[0]))       # the busy card, should the box show several
+        sclk, mclk, card = max(seen, key=lambda r: mhz(r[0]))       # the busy card, should the machine show several
         pick = {"sclk": sclk, "mclk": mclk}
         caps = glob.glob(card + "/hwmon/hwmon*/power1_cap")
         if caps:
@@ -992,8 +992,8 @@ def main():
     cpu = None
     if not args.no_cpu:
         # The CPU oracle (a C restatement of the reference's Swift test-support CPU path: dequantise, then multiply)
-        # on the box's host cores, bounded samples of the same workloads. Threads: the box's share of its host (16 for
-        # one GPU; OMP_NUM_THREADS says so), whatever the OS shows.
+        # on the host's cores, bounded samples of the same workloads. Threads: what one GPU has of its host (16 for
+        # it; OMP_NUM_THREADS says so), whatever the OS shows.
         from concurrent.futures import ThreadPoolExecutor
         o_off, _ = oracle.layout_offsets(D, F, align=16)
         pool = oracle.ExpertPool(host_layer0, o_off, STRIDE, D, F)

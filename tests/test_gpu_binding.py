@@ -1,4 +1,4 @@
-"""The native half of the Python binding where it meets the device: errors and threads. Run on the GPU box: pytest -m gpu."""
+"""The native half of the Python binding where it meets the device: errors and threads. Needs a GPU: pytest -m gpu."""
 import pytest
 
 pytestmark = pytest.mark.gpu

@@ -1,5 +1,5 @@
 """Post-attention setup and layer tail through the C ABI: bit-exact against the CPU oracle (which pins this
-build's summation order), on the reference tests' seeds, strides and sentinels. Run on the GPU box: pytest -m gpu."""
+build's summation order), on the reference tests' seeds, strides and sentinels. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,6 +1,6 @@
 """A context in FP16 mode (FFMOE_FP16, the reference's text-path activation type) through the C ABI against
 the CPU oracle run with dtype = FP16: router, decode / verify, prefill, per-route rows, GEMV, the steps
-either side. Run on the GPU box: pytest -m gpu."""
+either side. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

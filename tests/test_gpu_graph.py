@@ -1,7 +1,7 @@
 """The hot-path entry points only enqueue kernels (no allocation, no memset, no synchronisation), so a caller
 may capture them into a HIP graph. A captured chain of layers is replayed several times, with eager work and
 synchronisations of the same context between the replays, and every replay must equal the eager result bit for bit.
-Run on the GPU box: pytest -m gpu."""
+Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

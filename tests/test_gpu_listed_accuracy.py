@@ -1,5 +1,5 @@
 """The listed GEMV's fp32 logits against float64: no further off than dot products on the vector unit left them (a relative
-error of 8.6e-7 in bf16, 1.6e-5 in FP16 at 2,816 columns). Run on the GPU box: pytest -m gpu."""
+error of 8.6e-7 in bf16, 1.6e-5 in FP16 at 2,816 columns). Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,5 +1,5 @@
 """The forms that split long rows of logits over many blocks (sampled and greedy choice) and the matrix-unit form of the
-reference-layout GEMV, at the edges of their ranges, against the CPU oracle. Run on the GPU box: pytest -m gpu."""
+reference-layout GEMV, at the edges of their ranges, against the CPU oracle. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,5 +1,5 @@
 """Resident INT4 matrix (LM head): re-tiling, multi-row GEMV and greedy choice against the CPU oracle,
-through the C ABI. Run on the GPU box: pytest -m gpu."""
+through the C ABI. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

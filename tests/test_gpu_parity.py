@@ -1,4 +1,4 @@
-"""HIP kernels against the CPU oracle, through the C ABI (ctypes). Run on the GPU box: pytest -m gpu."""
+"""HIP kernels against the CPU oracle, through the C ABI (ctypes). Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

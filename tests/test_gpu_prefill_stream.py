@@ -1,6 +1,6 @@
 """The prefill's streaming product (chunks whose experts hold few pairs): experts with 0, 1 and every count around a 16-pair
 block, around a tile of 32 and of 64 pairs, K of whole and of ragged chunks, output columns that do not fill an N-block, both
-activation types, and the line between it and the grouped GEMMs. Run on the GPU box: pytest -m gpu."""
+activation types, and the line between it and the grouped GEMMs. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

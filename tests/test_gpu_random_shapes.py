@@ -1,7 +1,7 @@
 """Shapes drawn at random (fixed seeds, so every run sees the same cases): ragged row counts, expert counts that are no
 multiple of anything, top_k from 1 to 8, hidden and intermediate sizes from 128 up - through the router, the verify
 block (both forms), the prefill chunk and the dense FFN, each against the CPU oracle to the bar of the fixed-shape
-tests. Run on the GPU box: pytest -m gpu."""
+tests. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,6 +1,6 @@
 """Router routes of a short prompt either side of the row count from which the prefill router runs in two passes (160, less
 where many experts meet few columns: in bf16 after 73 at 256 x 128 and 150 at 2,048 x 128): the same routes and weights,
-bit for bit, as the pinned sums of all logits. Run on the GPU box: pytest -m gpu."""
+bit for bit, as the pinned sums of all logits. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,7 +1,7 @@
 """Odd shapes through the C ABI against the CPU oracle: hidden / intermediate sizes that are not multiples of a
 wave's K-slice, a single 64-wide group, expert counts that are not powers of two, fewer experts than top-k
 slots, one route per token - for the router, the <= 16-row expert path and the grouped-GEMM path alike.
-Run on the GPU box: pytest -m gpu."""
+Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 

@@ -1,5 +1,5 @@
 """Dense (shared-expert) FFN through the C ABI against the CPU oracle: the single-row operator, its
-multi-row and batched forms, and the upload from separate projections. Run on the GPU box: pytest -m gpu."""
+multi-row and batched forms, and the upload from separate projections. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 
@@ -87,7 +87,7 @@ def test_shared_expert_rows(ff, oracle, torch, d, f, t):
 @pytest.mark.parametrize("d,f,t", [(128, 64, 17), (2816, 2112, 32), (256, 192, 23), (2816, 2112, 100), (192, 1472, 256),
                                    (64, 64, 255), (128, 64, 384), (3072, 192, 20)])
 def test_shared_expert_17_to_384_rows_stream_the_arena_tiles(ff, oracle, torch, d, f, t):
-    # a short prompt or a chunk's ragged end: the resident-matrix GEMV on the expert's arena tiles, a grid row per 16 input
+    # a short prompt or a chunk's ragged end: the resident-matrix products on the expert's arena tiles, in bands of input
     # rows ((3072, 192): wider than that kernel's ring, the grouped GEMMs take it). Rows against the reference; a row of
     # the block against the row run alone (the <= 16-row kernels: the same sums in another order, so to a rounding step);
     # the block split anywhere gives the same rows bit for bit.
@@ -301,7 +301,7 @@ def _int8_reference_rows(oracle, parts, x_bits):
                                     (192, 1472, 200), (2816, 2112, 256), (64, 64, 192)])
 def test_dense_ffn_on_an_int8_layer(ff, oracle, torch, d, fs, t):
     # the 8-bit shared expert as a layer of the dense context: ffmoe_dense_ffn equals the gated matrix + down matrix calls
-    # bit for bit (it runs the same two kernels, a grid row per 16 rows) and follows the reference's rows; from 192 rows on
+    # bit for bit (up to 16 rows the same two kernels, then bands of rows with the same sums) and follows the reference's rows; from 192 rows on
     # it runs the library's dense GEMM on hi / lo rows of the weights instead, which sums in another order: the same rows
     # to the rounding of a sum
     g = oracle.seed_tree_key(0x1A8, f"dense-int8-d{d}-fs{fs}-t{t}")
