@@ -11,7 +11,7 @@
 // order the reference's comparator produces (PrefillMoEGrouping.swift:66-75). Only integer counting uses
 // LDS atomics; every position comes from prefix sums, so the result does not depend on timing.
 //
-// GEMM: items of one M-tile of up to 256 same-expert pairs x 256 weight rows, a block per compute unit walking a list of them. Every
+// GEMM: items of one M-tile of up to 256 same-expert pairs x 256 weight rows, one or two blocks per compute unit walking lists of them. Every
 // wave expands its own arena tile to bf16(fma(q, scale, bias)) - the reference's 16-bit tile weight (prefill.metal:581-590) - in
 // the register layout v_mfma_f32_16x16x32_bf16 wants; the pairs' inputs and the packed tiles go from global memory straight into LDS.
 // fp32 accumulation; GELU-tanh(gate) * up in the epilogue.
@@ -363,13 +363,14 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
 //      from memory straight into LDS, kRingW groups ahead.
 //   Pairs: a 64-wide group of their rows goes from memory straight into LDS as well (three buffers), and every wave reads each
 //      16-pair fragment once and multiplies it with its two row blocks.
-// One block of eight waves per compute unit walks a list of such items (prefill_gemm_kernel), the loads running on from one to the next.
+// A block of eight waves per compute unit, or two where tiles have up to 128 pairs (GemmLds), walks a list of such items
+// (prefill_gemm_kernel), the loads running on from one to the next.
 // What bounds it: 192 pairs per expert make 48 matrix instructions per wave and group, i.e. 1,536 cycles of a SIMD's matrix unit
 // of the 2,150 that a group takes; beside them 82 vector instructions (the expansion, 68 of them, shrinks with every pair a
 // wave multiplies its weights with), 26 LDS reads and one barrier. Run back to back the card also lowers its clock under it.
 // Weights through LDS instead (a wave expands a tile for all waves to read) costs the same however the waves split a block:
 // 215 to 235 us where this takes 183; 64 weight rows x 128 pairs per wave, every tile expanded twice, 209. Gate/up and down of a
-// 3,072-row chunk 222 + 115 -> 183 + 110 us, of 8,192 skewed rows 7.5 % less per layer, of 1,000 FP16 rows 144 + 78 -> 114 + 68; 256 pairs in each of 128
+// 3,072-row chunk 222 + 115 -> 183 + 110 us, of 8,192 skewed rows 7.5 % less per layer, of 1,000 FP16 rows 144 + 78 -> 114 + 68 (102 + 59 with two blocks per unit); 256 pairs in each of 128
 // experts 275 + 133 -> 216 + 137 us (1,200 TFLOP/s in gate/up). A second pass of bf16 products by the vendor's library on ready-made
 // weights reaches 1,250 on this card.
 // GATE_UP: A rows are gathered token rows of x; streams are gate / up; out = the activations, stored in the order the
@@ -390,28 +391,37 @@ struct GemmWave {
 };
 
 constexpr int kGemmTiles = 8;                               // arena tiles per N-block = waves per block
-constexpr int kRingA = 3, kRingW = 5;                       // groups of A, and of packed tiles at most, in LDS
-constexpr int kMaxLoads = kBM / 64;                         // KiB of A per wave and group, a whole M-tile
 constexpr uint32_t kFragBytes = kWave * 16;                 // one matrix operand of a wave
-constexpr uint32_t kGemmABytes = kBM / 16 * 2 * kFragBytes;
 constexpr uint32_t kGemmWBytes = kTileBytes + 2 * kTileScaleBytes;            // packed tile of one wave (a 64-lane load brings the scales twice)
-constexpr uint32_t kGemmWAt = kRingA * kGemmABytes, kGemmRowAt = kGemmWAt + kRingW * kGemmTiles * kGemmWBytes;
-// (down product: the pairs' output rows and largest scales, two items' worth)
-constexpr uint32_t kGemmRowBytes = kBM * 4, kGemmLargestAt = kGemmRowAt + 2 * kGemmRowBytes;
-// the epilogues work in the buffer of the item's last group of A: the next item's first two are in the others
-constexpr int kTurnBlocks = 3;                              // 16-pair blocks that a wave turns at a time
 constexpr uint32_t kGemmTurnRow = 2 * kTileRows * 2 + 16, kGemmTurnBytes = 16 * kGemmTurnRow;
-static_assert(kGemmTiles * kTurnBlocks * kGemmTurnBytes <= kGemmABytes && kGemmTiles * kBM * 4 <= kGemmABytes, "staging rows or peaks fit a buffer");
-constexpr uint32_t gemm_lds_bytes(bool gate_up, bool f16) { return gate_up ? kGemmRowAt : f16 ? kGemmLargestAt + 2 * kGemmRowBytes : kGemmLargestAt; }
+// A block whose tiles have up to 64 LC pairs. Tiles of up to 128 leave registers (128 per wave) and LDS for two such blocks per compute
+// unit: four waves per SIMD have more to issue while one waits for the matrix unit, LDS or a barrier. Gate/up and down of 1,000 rows,
+// 62 pairs per expert, 99 + 62 us with one block | 89 + 51 with two; a wave then is picked for an instruction in 87 % of its SIMD's issue
+// slots, 77 % before. Beyond 128 pairs a wave's sums take the registers of two.
+template <int LC>
+struct GemmLds {
+    static constexpr int kBlocks = LC == 2 ? 2 : 1;                     // of a compute unit
+    static constexpr int kRingA = 3, kRingW = LC == 2 ? 3 : 5;          // groups of A, and of packed tiles at most
+    static constexpr uint32_t kABytes = 4 * LC * 2 * kFragBytes;
+    static constexpr uint32_t kWAt = kRingA * kABytes, kRowAt = kWAt + kRingW * kGemmTiles * kGemmWBytes;
+    // (down product: the pairs' output rows and largest scales, two items' worth)
+    static constexpr uint32_t kRowBytes = 64 * LC * 4, kLargestAt = kRowAt + 2 * kRowBytes;
+    // the epilogues work in the buffer of the item's last group of A: the next item's first two are in the others
+    static constexpr int kTurnBlocks = LC == 2 ? 1 : 3;                 // 16-pair blocks that a wave turns at a time
+    static constexpr uint32_t bytes(bool gate_up, bool f16) { return gate_up ? kRowAt : f16 ? kLargestAt + 2 * kRowBytes : kLargestAt; }
+    static_assert(kGemmTiles * kTurnBlocks * kGemmTurnBytes <= kABytes && kGemmTiles * 64 * LC * 4 <= kABytes, "staging rows or peaks fit a buffer");
+    static_assert(kBlocks * (kLargestAt + 2 * kRowBytes) <= 160 * 1024, "a compute unit's LDS");
+};
 
 // One M-tile x N-block, and what a wave needs to ask for its rows: `from` = GATE_UP: in bytes from the first row's start (WIDE, where
 // the rows span 4 GiB or more: the row); else: in KiB, wave-uniform.
+template <int LC>
 struct GemmItem {
     bool valid;
     uint32_t parity;                      // of its number among the block's
     PrefillTile tile;
     uint32_t nb, act_block0, loads;
-    uint32_t from[kMaxLoads];
+    uint32_t from[LC];
     const uint8_t *w_tiles, *w_scales;    // this wave's arena tile
 };
 
@@ -454,8 +464,8 @@ struct GemmRings {
 // The 16-byte piece of its row's 128 bytes that a lane brings.
 __device__ __forceinline__ uint32_t gemm_row_piece(uint32_t lane) { return (lane & 7) ^ (lane >> 3); }
 // The loads of one group: the k-th KiB of a wave's share of A, its packed tile (k = 0) and that tile's scales (k = 1).
-template <bool GATE_UP, bool F16, bool WIDE>
-__device__ __forceinline__ void gemm_load_a(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, uint32_t grp, uint32_t at, int k) {
+template <bool GATE_UP, bool F16, bool WIDE, int LC>
+__device__ __forceinline__ void gemm_load_a(const GemmWave &gw, const GemmItem<LC> &it, uint32_t lds_base, uint32_t grp, uint32_t at, int k) {
     const uint32_t to = lds_base + at + (gw.wave + kGemmTiles * k) * kFragBytes;
     if constexpr (GATE_UP && WIDE) global_to_lds_16(gw.a + grp * kGroup + (size_t)it.from[k] * gw.a_stride + gemm_row_piece(gw.lane) * 8, to);
     else if constexpr (GATE_UP) global_to_lds_16(gw.a + grp * kGroup, it.from[k], to);
@@ -466,10 +476,10 @@ __device__ __forceinline__ void gemm_load_w(uint32_t lane, const uint8_t *w_tile
     else global_to_lds_4(w_scales, lane * 4 % kTileScaleBytes, to + kTileBytes);
 }
 // what an item's first step counts on: two groups of A, as many packed tiles as the ring holds
-template <bool GATE_UP, bool F16, bool WIDE>
-__device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it, uint32_t lds_base, const GemmRings &rings) {
+template <bool GATE_UP, bool F16, bool WIDE, int LC>
+__device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem<LC> &it, uint32_t lds_base, const GemmRings &rings) {
 #pragma unroll
-    for (uint32_t grp = 0; grp < kRingW; ++grp) {
+    for (uint32_t grp = 0; grp < (uint32_t)GemmLds<LC>::kRingW; ++grp) {
         const bool live = grp < rings.depth;
         const uint32_t to = lds_base + rings.first_slot + grp * kGemmTiles * kGemmWBytes;
         if (live) {
@@ -478,28 +488,126 @@ __device__ __forceinline__ void gemm_ask(const GemmWave &gw, const GemmItem &it,
         }
         if (grp < 2 && live) {
 #pragma unroll
-            for (int k = 0; k < kMaxLoads; ++k)
+            for (int k = 0; k < LC; ++k)
                 if ((uint32_t)k < it.loads)
                     gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, grp, grp ? rings.next : rings.cur, k);
         }
     }
 }
 
+// What an item leaves. Nobody reads the last group of A any more; `stage` is its buffer.
+template <bool GATE_UP, int NM, bool F16, bool DUMP, int LC>
+__device__ __forceinline__ void gemm_epilogue(const GemmWave &gw, const GemmItem<LC> &it, const ArenaGeom &g, const uint8_t *lds, uint8_t *stage, uint32_t tile,
+                                              uint32_t lane, f32x4 (&acc)[NM > 0 ? NM : 1][2], uint16_t *__restrict__ out, float *__restrict__ act_scale) {
+    using L = GemmLds<LC>;
+    constexpr int NA = NM > 0 ? NM : 1;
+    const uint32_t wave = gw.wave, j = lane & 15, jq = lane >> 4;
+    // lane (j, jq) holds pair j of every 16-pair block, weight rows 4 jq .. 4 jq + 3 of both row blocks
+    if constexpr (GATE_UP) {
+        // this wave's arena tile is k = 16 (tile % 4) .. + 15 of group tile / 4 of F: k-half tile / 2 % 2, operand lane
+        // (j, 2 (tile % 2) + jq / 2), values 4 (jq % 2) .. + 3 of that lane's eight
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][0][r] = gelu_tanh_fast(acc[i][0][r]) * acc[i][1][r];
+        if constexpr (F16) {
+            // a pair's 64 activations of a group sit in the four lanes (j, 0..3) of four waves: their largest magnitude
+            // peak < 2^e goes to 2^14 (frexp / ldexp as prefill.metal:689-702)
+            float *peaks = reinterpret_cast<float *>(stage);                // [wave][pair]
+#pragma unroll
+            for (int i = 0; i < NM; ++i) {
+                float peak = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) peak = fmaxf(peak, fabsf(acc[i][0][r]));
+                peak = fmaxf(peak, __shfl_xor(peak, 16, 64));
+                peak = fmaxf(peak, __shfl_xor(peak, 32, 64));
+                if (jq == 0) peaks[wave * (16 * NM) + 16 * i + j] = peak;
+            }
+            lds_barrier();
+#pragma unroll
+            for (int i = 0; i < NM; ++i) {
+                float peak = 0.0f;
+#pragma unroll
+                for (uint32_t v = 0; v < 4; ++v) peak = fmaxf(peak, peaks[((wave & 4) + v) * (16 * NM) + 16 * i + j]);
+                int e = 0;
+                (void)frexpf(peak, &e);
+                e = max(e, -100);                                   // 2^(14 - e) stays finite for a block of denormal size
+                const float to_half = ldexpf(1.0f, 14 - e);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][0][r] *= to_half;
+                if (jq == 0 && (wave & 3) == 0 && 16 * i + j < it.tile.rows)
+                    act_scale[((size_t)(it.act_block0 + i) * g.gf + tile / kTilesPerBlock) * 16 + j] = ldexpf(1.0f, e - 14);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            if (16 * i + j >= it.tile.rows) continue;
+            uint16_t *oblk = out + (((size_t)(it.act_block0 + i) * g.gf + tile / kTilesPerBlock) * 2 + (tile >> 1 & 1)) * (kWave * 8);
+            *reinterpret_cast<uint2 *>(oblk + (((tile & 1) * 2 + (jq >> 1)) * 16 + j) * 8 + (jq & 1) * 4) =
+                make_uint2(Act<F16>::pack(acc[i][0][0], acc[i][0][1]), Act<F16>::pack(acc[i][0][2], acc[i][0][3]));
+        }
+        return;
+    }
+    // Down projection: a 16-pair block of this wave's columns is 16 rows x 64 B. Each wave turns its blocks through a private piece
+    // of LDS, so that four lanes store 64 contiguous bytes of a row, instead of 8-byte pieces 32 B apart per instruction.
+    uint8_t *turn = stage + wave * (L::kTurnBlocks * kGemmTurnBytes);
+    const uint32_t row = lane >> 2, chunk = lane & 3;                           // read side
+#pragma unroll
+    for (int i0 = 0; i0 < NM; i0 += L::kTurnBlocks) {
+#pragma unroll
+        for (int i = i0; i < i0 + L::kTurnBlocks && i < NM; ++i) {
+            float pair_largest = 1.0f;
+            if constexpr (F16) pair_largest = *reinterpret_cast<const float *>(lds + L::kLargestAt + it.parity * L::kRowBytes + (16 * i + j) * 4);
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                f32x4 v = acc[i][st];
+                if constexpr (F16) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] *= pair_largest;         // the pair's sums back to their scale
+                }
+                *reinterpret_cast<uint2 *>(turn + (i - i0) * kGemmTurnBytes + j * kGemmTurnRow + st * 32 + 8 * jq) =
+                    make_uint2(Act<F16>::pack(v[0], v[1]), Act<F16>::pack(v[2], v[3]));
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint4 v[L::kTurnBlocks];
+        uint32_t orow[L::kTurnBlocks];
+#pragma unroll
+        for (int i = i0; i < i0 + L::kTurnBlocks && i < NM; ++i) {
+            v[i - i0] = *reinterpret_cast<const uint4 *>(turn + (i - i0) * kGemmTurnBytes + row * kGemmTurnRow + 16 * chunk);
+            orow[i - i0] = *reinterpret_cast<const uint32_t *>(lds + L::kRowAt + it.parity * L::kRowBytes + (16 * i + row) * 4);
+        }
+#pragma unroll
+        for (int i = i0; i < i0 + L::kTurnBlocks && i < NM; ++i)
+            if (16 * i + row < it.tile.rows && (!DUMP || tile < gw.n_arena_tiles)) *reinterpret_cast<uint4 *>(out + (size_t)orow[i - i0] * g.d + tile * (2 * kTileRows) + 8 * chunk) = v[i - i0];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
 // (lds is not __restrict__: the loads write the same memory through lds_base)
-template <bool GATE_UP, int NM, int LOADS, bool F16, bool WIDE, bool DUMP>
-__device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it, const GemmItem &next_item, GemmRings &rings, const ArenaGeom &g,
+template <bool GATE_UP, int NM, int LOADS, bool F16, bool WIDE, bool DUMP, int LC>
+__device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem<LC> &it, const GemmItem<LC> &next_item, GemmRings &rings, const ArenaGeom &g,
                                           uint8_t *lds, uint32_t lds_base, const uint32_t *__restrict__ sorted_out_row,
                                           uint16_t *__restrict__ out, float *__restrict__ act_scale, uint4 *__restrict__ dump = nullptr) {
+    using L = GemmLds<LC>;
     constexpr int NA = NM > 0 ? NM : 1;
-    constexpr int kQueue = gemm_queue(NA, 8);
-    const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4, n_groups = gw.n_groups;
+    constexpr int kQueue = gemm_queue(NA, L::kBlocks == 1 ? 8 : WIDE && NM > 6 ? 2 : 4);
+    // (the lane's number is taken anew here and for the epilogue: what the compiler derives from it for every tile height it would
+    // otherwise compute in front of the list of items and keep in scratch memory)
+    uint32_t lane = gw.lane;
+    asm volatile("" : "+v"(lane));
+    const uint32_t wave = gw.wave, j = lane & 15, jq = lane >> 4, n_groups = gw.n_groups;
     const uint32_t tile = it.nb * kGemmTiles + wave;        // this wave's arena tile
     if constexpr (!GATE_UP) {
-        // the pairs' output rows (and largest scales), for the epilogue; waves 4.. repeat what waves 0..3 bring
-        const uint32_t pair = min((wave & 3) * kWave + lane, it.tile.rows - 1);
-        global_to_lds_4(sorted_out_row + it.tile.row_start + pair, lds_base + kGemmRowAt + it.parity * kGemmRowBytes + (wave & 3) * (kWave * 4));
+        // the pairs' output rows (and largest scales), for the epilogue; waves LC.. repeat what waves 0..LC - 1 bring
+        const uint32_t pair = min((wave % LC) * kWave + lane, it.tile.rows - 1);
+        global_to_lds_4(sorted_out_row + it.tile.row_start + pair, lds_base + L::kRowAt + it.parity * L::kRowBytes + (wave % LC) * (kWave * 4));
         if constexpr (F16)
-            global_to_lds_4(act_scale + (size_t)gw.act_blocks * g.gf * 16 + it.act_block0 * 16 + pair, lds_base + kGemmLargestAt + it.parity * kGemmRowBytes + (wave & 3) * (kWave * 4));
+            global_to_lds_4(act_scale + (size_t)gw.act_blocks * g.gf * 16 + it.act_block0 * 16 + pair, lds_base + L::kLargestAt + it.parity * L::kRowBytes + (wave % LC) * (kWave * 4));
     }
     uint4 wraw = {0, 0, 0, 0};
     uint2 sraw = {0, 0};
@@ -552,9 +660,12 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
     // last fragments' reads then run ahead into that group, and the buffer of the group before is filled again.
     // What a step asks for goes out between its products: all at once, the waves queue for the address unit (11 ns per KiB of
     // rows) in front of their products. Behind an item's last group comes the next item's first, so that its packed tiles and, in
-    // the last two steps, its A are on their way before this one ends; without a next item the packed tiles of this one once more.
-    const bool run_on = next_item.valid && n_groups > 1;
-    const uint8_t *const next_w_tiles = next_item.valid ? next_item.w_tiles : it.w_tiles, *const next_w_scales = next_item.valid ? next_item.w_scales : it.w_scales;
+    // the last two steps, its A are on their way before this one ends; without a next item this one's once more. (The last two steps
+    // ask for a whole tile's rows, whatever the items have: behind a branch the compiler moves a step's products, and keeps all their
+    // operands until there.)
+    GemmItem<LC> next = it;
+    if (next_item.valid) next = next_item;
+    const uint8_t *const next_w_tiles = next.w_tiles, *const next_w_scales = next.w_scales;
     uint32_t own_w = n_groups - rings.depth;                        // groups of this item whose packed tiles are still to be asked for
     const uint8_t *ask_tiles = own_w ? it.w_tiles + rings.depth * kTileBytes : next_w_tiles;
     const uint8_t *ask_scales = own_w ? it.w_scales + rings.depth * kTileScaleBytes : next_w_scales;
@@ -565,8 +676,7 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
         for (int half = 0; half < 2; ++half) {
             if (half == 1) {
                 if (DUMP) vmem_barrier<0>();
-                else if (kSteady || run_on) vmem_barrier<2>();      // (the packed tile asked for in the first half)
-                else vmem_barrier<0>();
+                else vmem_barrier<2>();                             // (the packed tile asked for in the first half)
                 if (NM > 0) read_w(rings.next_slot());
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -598,13 +708,13 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
                             if (at == max((k + 1) * kUnits / (LOADS + 1) - 1, 0)) gemm_load_a<GATE_UP, F16, WIDE>(gw, it, lds_base, grp + 2, rings.before, k);
                     } else if (half == 1) {
 #pragma unroll
-                        for (int k = 0; k < kMaxLoads; ++k)
-                            if (at == max((k + 1) * kUnits / (kMaxLoads + 1) - 1, 0) && run_on && (uint32_t)k < next_item.loads)
-                                gemm_load_a<GATE_UP, F16, WIDE>(gw, next_item, lds_base, grp + 2 - n_groups, rings.before, k);
+                        for (int k = 0; k < LC; ++k)
+                            if (at == max((k + 1) * kUnits / (LC + 1) - 1, 0))
+                                gemm_load_a<GATE_UP, F16, WIDE>(gw, next, lds_base, min(grp + 2 - n_groups, n_groups - 1), rings.before, k);
                     } else {
 #pragma unroll
                         for (int k = 0; k < 2; ++k)
-                            if (at == max((k + 1) * kUnits / 3 - 1, 0) && (kSteady || run_on))     // (this group's went to registers in the step before)
+                            if (at == max((k + 1) * kUnits / 3 - 1, 0))      // (this group's went to registers in the step before)
                                 gemm_load_w(lane, ask_tiles, ask_scales, lds_base + rings.slot, k);
                     }
                     if (NM > 0) {
@@ -646,90 +756,9 @@ __device__ __forceinline__ void gemm_wave(const GemmWave &gw, const GemmItem &it
     uint8_t *const stage = lds + rings.before;
     if (n_groups == 1 && next_item.valid) gemm_ask<GATE_UP, F16, WIDE>(gw, next_item, lds_base, rings);
 
-    // epilogue: lane (j, jq) holds pair j of every 16-pair block, weight rows 4 jq .. 4 jq + 3 of both row blocks
-    if constexpr (GATE_UP) {
-        // this wave's arena tile is k = 16 (tile % 4) .. + 15 of group tile / 4 of F: k-half tile / 2 % 2, operand lane
-        // (j, 2 (tile % 2) + jq / 2), values 4 (jq % 2) .. + 3 of that lane's eight
-#pragma unroll
-        for (int i = 0; i < NA; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][0][r] = gelu_tanh_fast(acc[i][0][r]) * acc[i][1][r];
-        if constexpr (F16) {
-            // a pair's 64 activations of a group sit in the four lanes (j, 0..3) of four waves: their largest magnitude
-            // peak < 2^e goes to 2^14 (frexp / ldexp as prefill.metal:689-702)
-            float *peaks = reinterpret_cast<float *>(stage);                // [wave][pair]
-#pragma unroll
-            for (int i = 0; i < NM; ++i) {
-                float peak = 0.0f;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) peak = fmaxf(peak, fabsf(acc[i][0][r]));
-                peak = fmaxf(peak, __shfl_xor(peak, 16, 64));
-                peak = fmaxf(peak, __shfl_xor(peak, 32, 64));
-                if (jq == 0) peaks[wave * (16 * NM) + 16 * i + j] = peak;
-            }
-            lds_barrier();
-#pragma unroll
-            for (int i = 0; i < NM; ++i) {
-                float peak = 0.0f;
-#pragma unroll
-                for (uint32_t v = 0; v < 4; ++v) peak = fmaxf(peak, peaks[((wave & 4) + v) * (16 * NM) + 16 * i + j]);
-                int e = 0;
-                (void)frexpf(peak, &e);
-                e = max(e, -100);                                   // 2^(14 - e) stays finite for a block of denormal size
-                const float to_half = ldexpf(1.0f, 14 - e);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[i][0][r] *= to_half;
-                if (jq == 0 && (wave & 3) == 0 && 16 * i + j < it.tile.rows)
-                    act_scale[((size_t)(it.act_block0 + i) * g.gf + tile / kTilesPerBlock) * 16 + j] = ldexpf(1.0f, e - 14);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NM; ++i) {
-            if (16 * i + j >= it.tile.rows) continue;
-            uint16_t *oblk = out + (((size_t)(it.act_block0 + i) * g.gf + tile / kTilesPerBlock) * 2 + (tile >> 1 & 1)) * (kWave * 8);
-            *reinterpret_cast<uint2 *>(oblk + (((tile & 1) * 2 + (jq >> 1)) * 16 + j) * 8 + (jq & 1) * 4) =
-                make_uint2(Act<F16>::pack(acc[i][0][0], acc[i][0][1]), Act<F16>::pack(acc[i][0][2], acc[i][0][3]));
-        }
-        return;
-    }
-    // Down projection: a 16-pair block of this wave's columns is 16 rows x 64 B. Each wave turns its blocks through a private piece
-    // of LDS, so that four lanes store 64 contiguous bytes of a row, instead of 8-byte pieces 32 B apart per instruction.
-    uint8_t *turn = stage + wave * (kTurnBlocks * kGemmTurnBytes);
-    const uint32_t row = lane >> 2, chunk = lane & 3;                           // read side
-#pragma unroll
-    for (int i0 = 0; i0 < NM; i0 += kTurnBlocks) {
-#pragma unroll
-        for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i) {
-            float pair_largest = 1.0f;
-            if constexpr (F16) pair_largest = *reinterpret_cast<const float *>(lds + kGemmLargestAt + it.parity * kGemmRowBytes + (16 * i + j) * 4);
-#pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                f32x4 v = acc[i][st];
-                if constexpr (F16) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] *= pair_largest;         // the pair's sums back to their scale
-                }
-                *reinterpret_cast<uint2 *>(turn + (i - i0) * kGemmTurnBytes + j * kGemmTurnRow + st * 32 + 8 * jq) =
-                    make_uint2(Act<F16>::pack(v[0], v[1]), Act<F16>::pack(v[2], v[3]));
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        uint4 v[kTurnBlocks];
-        uint32_t orow[kTurnBlocks];
-#pragma unroll
-        for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i) {
-            v[i - i0] = *reinterpret_cast<const uint4 *>(turn + (i - i0) * kGemmTurnBytes + row * kGemmTurnRow + 16 * chunk);
-            orow[i - i0] = *reinterpret_cast<const uint32_t *>(lds + kGemmRowAt + it.parity * kGemmRowBytes + (16 * i + row) * 4);
-        }
-#pragma unroll
-        for (int i = i0; i < i0 + kTurnBlocks && i < NM; ++i)
-            if (16 * i + row < it.tile.rows && (!DUMP || tile < gw.n_arena_tiles)) *reinterpret_cast<uint4 *>(out + (size_t)orow[i - i0] * g.d + tile * (2 * kTileRows) + 8 * chunk) = v[i - i0];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
+    uint32_t out_lane = gw.lane;
+    asm volatile("" : "+v"(out_lane));
+    gemm_epilogue<GATE_UP, NM, F16, DUMP, LC>(gw, it, g, lds, stage, tile, out_lane, acc, out, act_scale);
 }
 
 // Consecutive block ids go to consecutive XCDs. Many experts: all N-blocks of an M-tile share an XCD (its L2 holds
@@ -748,12 +777,11 @@ __device__ __forceinline__ bool prefill_block(uint32_t n_nblocks, bool nb_major,
     return true;
 }
 
-// F16: a context in FP16 mode - FP16 rows in, FP16 tiles, block-scaled FP16 activations, FP16 per-route rows out. (The FP16 gate/up
-// kernel is 12 registers over its 256; what it spills is reloaded outside the loop over groups.)
-// A block per compute unit, which works off its share of the XCD's items one after the other: an item's first loads then travel
+// F16: a context in FP16 mode - FP16 rows in, FP16 tiles, block-scaled FP16 activations, FP16 per-route rows out.
+// A block works off its share of the XCD's items one after the other: an item's first loads then travel
 // during the epilogue of the one before.
-template <bool GATE_UP, bool F16 = false, bool WIDE = false, bool DUMP = false>
-__global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
+template <bool GATE_UP, bool F16, bool WIDE, int LC, bool DUMP = false>
+__global__ __launch_bounds__(64 * kGemmTiles, 2 * GemmLds<LC>::kBlocks) void prefill_gemm_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
                                                                           const PrefillPlan *__restrict__ plan,
                                                                           const PrefillTile *__restrict__ tiles,
                                                                           const uint32_t *__restrict__ sorted_token,
@@ -762,7 +790,8 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
                                                                           uint16_t *__restrict__ out, bool nb_major,
                                                                           float *__restrict__ act_scale, uint32_t act_blocks,
                                                                           uint4 *__restrict__ dump = nullptr) {
-    __shared__ __align__(16) uint8_t lds[gemm_lds_bytes(GATE_UP, F16)];
+    using L = GemmLds<LC>;
+    __shared__ __align__(16) uint8_t lds[L::bytes(GATE_UP, F16)];
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     GemmWave gw;
     gw.lane = threadIdx.x & 63;
@@ -785,7 +814,7 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
     const uint32_t n_items = nb_major ? (uint32_t)((uint64_t)all * (xcd + 1) / 8) - first : tiles_x * n_nb + (over + 7 - xcd) / 8;
     // round r of this block: the rounds run forth and back over the blocks, so that who had a large item gets a small one
     auto item_at = [&](uint32_t r) __attribute__((always_inline)) {
-        GemmItem it;
+        GemmItem<LC> it;
         const uint32_t q = r * per_xcd + (r & 1 ? per_xcd - 1 - mine : mine);
         it.valid = q < n_items;
         it.parity = r & 1;
@@ -816,7 +845,7 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
         // at piece c ^ (r % 8) of the row, so that the sixteen rows of a fragment read fall on different banks. else: the
         // activations are stored fragment by fragment.
 #pragma unroll
-        for (int k = 0; k < kMaxLoads; ++k) {
+        for (int k = 0; k < LC; ++k) {
             const uint32_t piece = gw.wave + kGemmTiles * k;
             if constexpr (GATE_UP) {
                 const uint32_t row = min(piece * 8 + (gw.lane >> 3), it.tile.rows - 1);
@@ -833,27 +862,26 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2) void prefill_gemm_kernel(const 
         it.w_scales = expert_base + (GATE_UP ? g.gu_scales_off : g.dn_scales_off) + (size_t)at * kTileScaleBytes;
         return it;
     };
-    GemmItem it = item_at(0);
+    GemmItem<LC> it = item_at(0);
     if (!it.valid) return;
     GemmRings rings;
-    rings.depth = min((uint32_t)kRingW, gw.n_groups);
-    rings.cur = 0, rings.next = kGemmABytes, rings.before = 2 * kGemmABytes;
-    rings.slot = rings.first_slot = kGemmWAt + gw.wave * kGemmWBytes;
+    rings.depth = min((uint32_t)L::kRingW, gw.n_groups);
+    rings.cur = 0, rings.next = L::kABytes, rings.before = 2 * L::kABytes;
+    rings.slot = rings.first_slot = L::kWAt + gw.wave * kGemmWBytes;
     rings.end_slot = rings.first_slot + rings.depth * (kGemmTiles * kGemmWBytes);
     gemm_ask<GATE_UP, F16, WIDE>(gw, it, lds_base, rings);
     vmem_barrier<0>();
     for (uint32_t r = 1;; ++r) {
-        const GemmItem next = item_at(r);
+        const GemmItem<LC> next = item_at(r);
         const uint32_t n_mb = (it.tile.rows + 15) / 16;
         // (the test's tiles past the last, up to a set of four, are the last once more)
         const uint32_t owned = DUMP ? (gw.n_arena_tiles + kTilesPerBlock - 1) / kTilesPerBlock * kTilesPerBlock : gw.n_arena_tiles;
         const bool owns = it.nb * kGemmTiles + gw.wave < owned;
         // (waves that own no tile take part in the loads and the barriers, which are the same in all instantiations of one LOADS)
-#define FFMOE_GEMM_WAVE(N, L) gemm_wave<GATE_UP, N, L, F16, WIDE, DUMP>(gw, it, next, rings, g, lds, lds_base, sorted_out_row, out, act_scale, dump)
+#define FFMOE_GEMM_WAVE(N, K) if constexpr (K <= LC) gemm_wave<GATE_UP, N, K, F16, WIDE, DUMP, LC>(gw, it, next, rings, g, lds, lds_base, sorted_out_row, out, act_scale, dump)
         if constexpr (DUMP) {
             // the test launch runs one pair
-            if (owns) FFMOE_GEMM_WAVE(1, 1);
-            else FFMOE_GEMM_WAVE(0, 1);
+            if (owns) { FFMOE_GEMM_WAVE(1, 1); } else { FFMOE_GEMM_WAVE(0, 1); }
         } else if (!owns) {
             switch ((n_mb + 3) / 4) {
                 case 1: FFMOE_GEMM_WAVE(0, 1); break;
@@ -1336,7 +1364,13 @@ uint32_t gemm_tile_rows(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g
     // (73 | 62), 96 pairs 78 | 73 (78 | 74); 32 of 2,048 x 1,024, 62 pairs 82 | 74 (79 | 75); uniform routes within 1 %. Not where the
     // chip is full, where it expands the heavy experts' weights more often: 128 experts of 2,816 x 704, 62 pairs 211 | 248.
     const uint32_t most = n_experts * nb_gu <= 2 * cus ? (uint32_t)fminf((float)kBM, ceilf((mean + 4 * dev) / 16) * 16) : kBM;
-    if (n_items / (float)kBM * nb_gu > cus || n_experts * nb_gu > cus) return most;
+    // Where the chip is full, 128, of which a compute unit works at two tiles at a time (GemmLds), as long as that holds nearly all of a
+    // uniform chunk's experts whole; beyond, the second tiles' expansions cost more. us at 256 | 128, bf16 (FP16): 128 experts of
+    // 2,816 x 704, 850 rows (53 pairs each) 182 | 164 (199 | 181), 1,000 179 | 167 (204 | 191), 1,500 (94) 214 | 203 (246 | 238), 1,792 (112)
+    // 241 | 238 (275 | 272), 2,000 (125) 261 | 260 (289 | 299); Zipf of exponent 1.1, 1,000 rows 217 | 191 (236 | 216), 1,700 273 | 253 (305 |
+    // 283), 3,072 (192) 377 | 386; 64 experts of 2,048 x 1,408, 94 pairs 152 | 140 (177 | 164), 112 171 | 165 (197 | 192), 141 188 | 210;
+    // 256 of 512 x 256, 47 pairs 53 | 49 (62 | 58), Zipf 63 | 55 (73 | 64).
+    if (n_items / (float)kBM * nb_gu > cus || n_experts * nb_gu > cus) return mean + 1.5f * dev <= 128 ? (most < 128 ? most : 128) : most;
     uint32_t best = most;
     float least = 0.0f;
     for (uint32_t rows = most; rows >= 32; rows -= 16) {
@@ -1449,7 +1483,7 @@ hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, 
                                           dump);
     // the pair's input row is whatever row 0 of the scratch holds: only the weight side is looked at
 #define FFMOE_DUMP(GU, H, A, STRIDE, OUT, NB)                                                                              \
-    hipLaunchKernelGGL((prefill_gemm_kernel<GU, H, false, true>), dim3((NB) * 8), dim3(64 * kGemmTiles), 0, s, arena_layer, g, sc.plan, sc.tiles,  \
+    hipLaunchKernelGGL((prefill_gemm_kernel<GU, H, false, 4, true>), dim3((NB) * 8), dim3(64 * kGemmTiles), 0, s, arena_layer, g, sc.plan, sc.tiles,  \
                        sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, false, sc.act_scale, sc.act_blocks, static_cast<uint4 *>(dump))
     if (gate_up) {
         const uint32_t nb = (g.gu_rb + kGemmTiles - 1) / kGemmTiles;
@@ -1517,11 +1551,17 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     const uint32_t act_blocks = f16 ? sc.act_blocks : 0u;
     // (a row's address is 32 bits from the first row's where that reaches the last)
     const bool wide = (uint64_t)t * x_stride * 2 > 0xFFFFFFFFull;
-#define FFMOE_GEMM(GU, A, STRIDE, OUT, NB)                                                                                    \
-    hipLaunchKernelGGL((GU && wide ? (f16 ? prefill_gemm_kernel<GU, true, GU> : prefill_gemm_kernel<GU, false, GU>)                    \
-                                   : (f16 ? prefill_gemm_kernel<GU, true> : prefill_gemm_kernel<GU, false>)), dim3(8 * min((n_cus + 7) / 8, tile_slots * (NB))), dim3(64 * kGemmTiles), 0, s, \
+#define FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, LC)                                                                             \
+    hipLaunchKernelGGL((GU && wide ? (f16 ? prefill_gemm_kernel<GU, true, GU, LC> : prefill_gemm_kernel<GU, false, GU, LC>)   \
+                                   : (f16 ? prefill_gemm_kernel<GU, true, false, LC> : prefill_gemm_kernel<GU, false, false, LC>)), \
+                       dim3(8 * min((GemmLds<LC>::kBlocks * n_cus + 7) / 8, tile_slots * (NB))), dim3(64 * kGemmTiles), 0, s, \
                        arena_layer, g, sc.plan, sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, nb_major,    \
                        act_scale, act_blocks, nullptr)
+#define FFMOE_GEMM(GU, A, STRIDE, OUT, NB)                                                                                    \
+    do {                                                                                                                      \
+        if (tile_rows <= 128) FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, 2);                                                       \
+        else FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, 4);                                                                        \
+    } while (0)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
     hipLaunchKernelGGL(stream_kernel<GU>(tile_rows, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
                        sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major, act_scale, act_blocks)

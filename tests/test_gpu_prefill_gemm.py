@@ -75,6 +75,36 @@ def test_tiles_by_the_number_of_items(oracle, act, d, f, counts):
     test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts)
 
 
+# Chunks that fill the chip in tiles of at most 128 pairs, two blocks per compute unit: the edges of 16-pair blocks and of one and two
+# tiles, tall and flat layers, a last N-block that is half full. The same rows three times over take tiles of 256: the same bits.
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,counts", [(192, 704, 8 * (1, 16, 47, 64, 127, 128, 129, 0)), (64, 640, 8 * (17, 33, 80, 81, 96, 112, 113, 0)),
+                                        (512, 704, 7 * (31, 65, 48, 97, 95, 100, 63) + (257, 15))])
+def test_tiles_of_half_the_pairs(oracle, act, d, f, counts):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    e, t = len(counts), sum(counts)
+    assert 48 * e < t <= 112 * e and 3 * t > 130 * e
+    rng, pool, _ = make_layer(oracle, 51 + d, d, f, e, align=1)
+    idx = np.repeat(np.arange(e, dtype=np.uint32), counts)
+    rng.shuffle(idx)
+    ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=3 * t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt)
+        w = torch.from_numpy(rng.uniform(0.2, 1.0, (t, 1)).astype(np.float32)).to(dt)
+        gx, gi, gw = x.cuda(), torch.from_numpy(idx[:, None].view(np.int32)).cuda(), w.cuda()
+        tall = ctx.prefill(0, gx.repeat(3, 1), gi.repeat(3, 1), gw.repeat(3, 1))
+        ctx.prefill(0, torch.full_like(gx, float("nan")), gi, gw)           # (nothing of the rows stays in the scratch)
+        y = ctx.prefill(0, gx, gi, gw, out=torch.full_like(gx, float("nan")))
+        _check(oracle, pool, e, idx[:, None], x, w, y.float().cpu().numpy(), act)
+        assert all(torch.equal(tall[k * t:(k + 1) * t], y) for k in range(3))
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("act,stride", [("bf16", 1 << 24), ("bf16", 1 << 25), ("fp16", 1 << 25), ("bf16", 360_000_000), ("fp16", 360_000_000)])
 def test_rows_that_span_four_gigabytes(oracle, act, stride):
     # 99 rows 32 MiB apart: a place past 2 GiB; 64 MiB: a row's place in bytes does not fit 32 bits; 720 MB apart: nor does the one in 16-byte pieces
