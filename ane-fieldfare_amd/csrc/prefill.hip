@@ -921,12 +921,17 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2 * GemmLds<LC>::kBlocks) void pre
 // four arena tiles, another way through them. There the expansion to 16-bit weights (68 vector instructions per 1 KiB tile of
 // a wave, whatever the pairs, in front of its products) bounds the launch below about 50 pairs per expert: with the GEMMs that this
 // form was built beside, 90 us for the 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s. Here a wave owns one arena tile row for the whole of K, streams its
-// packed tiles through a ring of four and multiplies them in the offset form of the decode kernels (stream.hpp): about 75
-// vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. The pairs' rows go through LDS in
+// packed tiles through a ring of four and multiplies them in the offset form of the decode kernels (stream.hpp): about 52
+// vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. The biases (and the offset's correction)
+// of four groups are one fp32 product per 16 pairs - the groups' input sums by the scales' second halves, K of 4 - and the
+// sums are made once per block, each wave its share, instead of once per wave: per 16 pairs, tile and group 88 cycles of the matrix
+// unit instead of 96, 8 vector instructions instead of 16. 128 experts of 2,816 x 704, top-8, router table to combined rows, us before | now:
+// 301 rows 122 | 118, 384 rows 136 | 128, 700 rows 178 | 172 (FP16 131 | 126, 141 | 132, 187 | 184); a dense 2,816 -> 2,112 FFN of 700 rows
+// 67 | 63; 20 pairs per expert and fewer wait for the weights' bytes and keep their times. The pairs' rows go through LDS in
 // operand order, two groups at a time in two buffers, so that every wave of the block reads the same fragments and the
 // registers hold one chunk's 16-byte pieces in flight; the weights stay in flight across the barriers. Gate/up of 37 rows
-// 90 -> 56 us (4.7 TB/s), of 301 rows 103 -> 65. What bounds it then is the weights' bytes (32 pairs per tile) and the matrix and
-// vector instructions together (64).
+// 90 -> 56 us (4.7 TB/s). What bounds it then is the weights' bytes (32 pairs per tile) and the matrix and vector instructions
+// together (64).
 // A pair's arithmetic does not depend on its tile: any two launches of this kernel give the same row bit for bit.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kStreamDepth = 4;                                             // weight tiles in flight per wave
@@ -1017,25 +1022,54 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
 #pragma unroll
     for (int m = 0; m < NM; ++m) tot[m].a = tot[m].b = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // The groups' input sums: of a chunk's 16-pair blocks and groups every wave takes its share, as one value per pair in LDS
+    // ([quad of groups % 2][16-pair block][group of the quad][pair]: the lane order of the bias product's operand).
+    float *const sums = reinterpret_cast<float *>(lds + 2 * kBuf);
+    constexpr int kSums = (NM + 1) / 2;                   // 16-pair blocks per wave, of one of the chunk's two groups
+    static_assert(CHUNK == 2 && kStreamDepth == 4, "two waves per group of a chunk; a quad of groups per bias product");
+    auto sum_up = [&](uint32_t buf, uint32_t quad, int first) __attribute__((always_inline)) {
+        const int gl = wave & 1;
+#pragma unroll
+        for (int k = 0; k < kSums; ++k) {
+            const int m = min((int)(wave >> 1) + 2 * k, NM - 1);
+            const f32x4 sx = group_input_sum<F16>(frag(buf, m, 2 * gl), frag(buf, m, 2 * gl + 1));
+            if (j == 0) *reinterpret_cast<f32x4 *>(sums + (((quad & 1) * NM + m) * 4 + first + gl) * 16 + 4 * jq) = sx;
+        }
+    };
+    // a quad's scale and bias pairs as the lane's group of it has them
+    uint2 quad_s = {0u, 0u};
+    auto add_bias = [&](uint32_t quad, auto whole) __attribute__((always_inline)) {
+        float ta = bf16hi_to_f32(quad_s.x), tb = bf16hi_to_f32(quad_s.y);
+        if constexpr (!F16) {
+            ta = __builtin_fmaf(-Act<F16>::kOffset, bf16lo_to_f32(quad_s.x), ta);
+            tb = __builtin_fmaf(-Act<F16>::kOffset, bf16lo_to_f32(quad_s.y), tb);
+        }
+        const bool live = decltype(whole)::value || 4 * quad + jq < n_groups;
+        if (!live) ta = tb = 0.0f;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const float sx = live ? sums[((quad & 1) * NM + m) * kWave + lane] : 0.0f;
+            tot[m].a = __builtin_amdgcn_mfma_f32_16x16x4f32(sx, ta, tot[m].a, 0, 0, 0);
+            tot[m].b = __builtin_amdgcn_mfma_f32_16x16x4f32(sx, tb, tot[m].b, 0, 0, 0);
+        }
+    };
+
     auto step = [&](uint32_t buf, int gl, int u, uint32_t refill) __attribute__((always_inline)) {
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         const uint4 tile = ring_t[u];
         const uint2 sc = ring_s[u];
+        if (u == 0 || jq == (uint32_t)u) quad_s = sc;
         fill(u, refill);
         const uint4 wa0 = unpack8_stream<F16>(tile.x), wa1 = unpack8_stream<F16>(tile.y);
         const uint4 wb0 = unpack8_stream<F16>(tile.z), wb1 = unpack8_stream<F16>(tile.w);
-        float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y), ta = bf16hi_to_f32(sc.x), tb = bf16hi_to_f32(sc.y);
+        float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y);
         if constexpr (F16) {
             sa *= FineNibble<true>::kUnit;
             sb *= FineNibble<true>::kUnit;
-        } else {
-            ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ta);
-            tb = __builtin_fmaf(-Act<F16>::kOffset, sb, tb);
         }
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             const uint4 x0 = frag(buf, m, 2 * gl), x1 = frag(buf, m, 2 * gl + 1);
-            const f32x4 sx = group_input_sum<F16>(x0, x1);
             f32x4 aa = Act<F16>::mfma(x0, wa0, zero);
             aa = Act<F16>::mfma(x1, wa1, aa);
             f32x4 ab = Act<F16>::mfma(x0, wb0, zero);
@@ -1043,11 +1077,9 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 tot[m].a[r] = __builtin_fmaf(sa, aa[r], tot[m].a[r]);
-                tot[m].a[r] = __builtin_fmaf(ta, sx[r], tot[m].a[r]);
                 tot[m].b[r] = __builtin_fmaf(sb, ab[r], tot[m].b[r]);
-                tot[m].b[r] = __builtin_fmaf(tb, sx[r], tot[m].b[r]);
             }
-            // pinned: left alone, the compiler collects the scale-and-bias arithmetic of several groups and carries all
+            // pinned: left alone, the compiler collects the scales' arithmetic of several groups and carries all
             // their matrix results there, which does not fit the register budget
 #pragma unroll
             for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(tot[m].a[r]), "+v"(tot[m].b[r]));
@@ -1068,6 +1100,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         const uint32_t buf = c & 1;
         store_a(buf ^ 1);               // (past the last chunk: a buffer nobody reads)
         load_a(min(c + 2, n_chunks - 1));
+        sum_up(buf, c >> 1, kFirst);    // (of a group past the last: not used)
 #pragma unroll
         for (int gl = 0; gl < CHUNK; ++gl) {
             const uint32_t grp = c * CHUNK + gl;
@@ -1083,9 +1116,13 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     for (; (c + 2) * CHUNK <= n_groups; c += 2) {
         chunk(c, Even{}, Whole{});
         chunk(c + 1, Odd{}, Whole{});
+        add_bias(c >> 1, Whole{});
     }
-    if (c < n_chunks) chunk(c, Even{}, Part{});
-    if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
+    if (c < n_chunks) {
+        chunk(c, Even{}, Part{});
+        if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
+        add_bias(c >> 1, Part{});
+    }
 
     // lane (j, jq) holds, per stream, weight row j of the tile row for pairs 4 jq .. 4 jq + 3 of every 16-pair block. The
     // last chunk ended with a barrier: the LDS is free.
@@ -1178,7 +1215,7 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_
                                                                     const uint16_t *__restrict__ a, uint32_t a_stride,
                                                                     uint16_t *__restrict__ out, uint32_t n_nblocks, bool nb_major,
                                                                     float *__restrict__ act_scale, uint32_t act_blocks) {
-    __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave];
+    __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave + 2 * MAX_NM * kWave / 4];
     static_assert(16 * MAX_NM * kStreamStageRow <= sizeof(lds), "the down epilogue's rows fit");
     uint32_t ti, nb;
     if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;

@@ -66,6 +66,34 @@ def test_tile_edges_against_the_oracle(oracle, act, d, f, scale):
         ctx.close()
 
 
+# 1 to 5 groups of K in each product: a quad of groups short of three, two, one and none, and one group past it
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f", [(64, 128), (192, 64), (256, 192), (320, 256), (128, 320)])
+def test_a_row_without_bounds_stays_alone(oracle, act, d, f):
+    # an infinity or a NaN in a row (also in the last group, the one that loads past the end repeat): the others keep their bits
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    rng, pool, _ = make_layer(oracle, 3 * d + f, d, f, 4, align=1)
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    t = 20
+    x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt)
+    idx = torch.from_numpy(np.stack([rng.permutation(4) for _ in range(t)]).astype(np.int32)).cuda()
+    w = torch.full((t, 4), 0.25).to(dt).cuda()
+    bad = x.clone()
+    bad[3, d - 1], bad[17, 0] = float("inf"), float("nan")
+    ctx = ff.Context(d, f, 4, 4, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        y = ctx.prefill(0, x.cuda(), idx, w).cpu()
+        z = ctx.prefill(0, bad.cuda(), idx, w).cpu()
+        rest = [r for r in range(t) if r not in (3, 17)]
+        assert torch.isfinite(y.float()).all() and torch.equal(y[rest].view(torch.int16), z[rest].view(torch.int16))
+        assert not torch.isfinite(z[[3, 17]].float()).any()
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("t", [47, 48, 49])
 def test_the_line_to_the_grouped_gemms(oracle, t):
     # four experts, top-4: t pairs each; 48 per expert is the last chunk that streams. Either side to the same bar.
