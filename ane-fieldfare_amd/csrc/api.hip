@@ -623,7 +623,7 @@ int ffmoe_router(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t *r
                      static_cast<const uint4 *>(l.router_frag), l.router_norm_max};
     claim_scratch(ctx, stream);
     FF_HIP(launch_router(static_cast<hipStream_t>(stream), rw, router_x, x_stride, t, ctx->shape.n_experts,
-                         ctx->shape.d, ctx->shape.top_k, out_logits ? out_logits : ctx->logits, out_idx, out_w, &ctx->timer,
+                         ctx->shape.d, ctx->shape.top_k, out_logits ? out_logits : ctx->logits, out_idx, out_w, ctx->n_cus, &ctx->timer,
                          ctx->f16, out_logits != nullptr, ctx->logits));
     return FFMOE_OK;
 }

@@ -168,7 +168,7 @@ hipError_t launch_dequant_expert(hipStream_t s, const uint8_t *arena_expert, Are
 // router.hip
 hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uint32_t x_stride, uint32_t t,
                          uint32_t n_experts, uint32_t d, uint32_t top_k, float *logits, uint32_t *out_idx,
-                         uint16_t *out_w, KernelTimer *timer, bool f16 = false, bool want_logits = true,
+                         uint16_t *out_w, uint32_t n_cus, KernelTimer *timer, bool f16 = false, bool want_logits = true,
                          float *scratch = nullptr);
 // `frag`: E * d bf16 values, the weights in matrix-operand order (needs d % 32 == 0 and E % 16 == 0)
 hipError_t launch_router_fragments(hipStream_t s, const uint16_t *w, uint32_t n_experts, uint32_t d, void *frag);

@@ -16,15 +16,15 @@ namespace ffmoe {
 namespace {
 
 // Whether a prompt of t rows takes the form below where the two-pass form could serve. The two passes of the prefill form are
-// chains of round trips, 6.3 us + 30 ns per expert + 3.2 ns per column (FP16 rows 4.4) however few the rows; one block per
+// chains of round trips, 6.2 us + 12.5 ns per expert + 1.75 ns per column (FP16 rows 6.8 and 2.1) however few the rows; one block per
 // expert and four rows costs the router's weights once more from the caches for every four rows, 5.5 us + 0.58 ns per row and
-// expert whatever the columns (fitted at 8 tables). Two-pass form | this one, us, bf16: 2,816 x 128, 17 rows
-// 18.9 | 7.6, 64 rows 19.3 | 10.6, 128 rows 19.3 | 15.1, 160 rows 19.4 | 17.3; 2,048 x 128, 128 rows 16.3 | 14.9, 160 rows
-// 16.5 | 17.1; 1,024 x 64, 160 rows 11.7 | 11.3; 256 x 128, 64 rows 10.6 | 10.1, 128 rows 10.7 | 14.5; 512 x 16, 160 rows
-// 7.9 | 7.1; FP16, 2,816 x 128, 160 rows 22.8 | 17.4; 2,048 x 128, 160 rows 18.5 | 17.0; 256 x 128, 128 rows 11.9 | 14.5. Same
+// expert whatever the columns (fitted at 10 tables). Two-pass form | this one, us, bf16: 2,816 x 128, 17 rows
+// 12.6 | 7.6, 64 rows 13.0 | 10.7, 80 rows 12.9 | 11.8, 100 rows 12.9 | 13.4, 160 rows 13.0 | 17.2; 2,048 x 128, 64 rows 11.5 |
+// 10.5, 80 rows 11.4 | 11.6; 1,024 x 64, 80 rows 8.7 | 8.7; 256 x 128, 48 rows 8.9 | 9.2; 512 x 16, 160 rows
+// 7.6 | 7.1; FP16, 2,816 x 128, 100 rows 14.7 | 13.5, 130 rows 14.8 | 15.6; 2,048 x 128, 80 rows 12.9 | 11.7. Same
 // pinned sums: same routes bit for bit.
 bool router_small_rows(uint32_t t, uint32_t n_experts, uint32_t d, bool f16) {      // (in units of 20 ps)
-    return t <= 160 && 29u * n_experts * t <= 40000u + 1500u * n_experts + (f16 ? 220u : 160u) * d;
+    return t <= 160 && 29u * n_experts * t <= (f16 ? 65000u : 35000u) + 625u * n_experts + (f16 ? 105u : 88u) * d;
 }
 
 // Decode / verify / short-prompt router logits. grid = (E, ceil(T / 4)); the four waves of a block are the
@@ -210,9 +210,9 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const float *logits, co
 // fma alone); only the selected experts' logits have to be the pinned ones.
 //   1. router_approx_kernel: every logit on the matrix unit (bf16 products are exact, the fp32 sum runs in
 //      whatever order the unit uses), plus the squared norm of every row.
-//   2. router_exact_topk_kernel, one wave per token. Let a_e be the approximate and p_e the pinned logit of expert e, and
+//   2. router_exact_topk_kernel, one to four waves per token. Let a_e be the approximate and p_e the pinned logit of expert e, and
 //      B >= |a_e - p_e|. An expert among the pinned top k has a_e >= v_k - 2 B, v_k the k-th largest approximate logit:
-//      were a_e below that, the k experts with a >= v_k would all have p >= a - B > a_e + B >= p_e. The wave computes
+//      were a_e below that, the k experts with a >= v_k would all have p >= a - B > a_e + B >= p_e. It computes
 //      the pinned logit of every expert above that threshold (eight or nine at 128 experts) and selects among them
 //      with the same code as the other router kernels. A row with a non-finite value anywhere takes every expert as
 //      a candidate.
@@ -226,10 +226,8 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const float *logits, co
 // FP16 rows enter the approximate pass as two bf16 halves per value (split_f16x8: exact), which doubles its
 // instructions and its rounding count; the pinned sums widen them to fp32 as every other kernel does.
 // Needs: bf16 weights, no per-input scale, d a multiple of 256 up to 4096, E a multiple of 16 up to 128
-// (the four waves of a block of the approximate pass hold two 16-expert fragments each).
+// (the four waves of a block of the approximate pass hold two 16-expert fragments each, or up to four waves one each).
 // ---------------------------------------------------------------------------------------------------
-constexpr int kApproxFrags = 2;                      // 16-row operand fragments of token rows per block of the approximate pass
-constexpr int kApproxTok = 16 * kApproxFrags;
 constexpr int kApproxKParts = 4;        // K is cut into parts, one block each; the pass that follows adds the parts' sums
 
 // Router weights in matrix-operand order: frag[(h * E/16 + n) * 64 + lane] = the eight values
@@ -242,16 +240,21 @@ __global__ __launch_bounds__(256) void router_frag_kernel(const uint16_t *__rest
     frag[i] = *reinterpret_cast<const uint4 *>(w + (size_t)(16 * n + (lane & 15)) * d + 32 * h + 8 * (lane >> 4));
 }
 
-// One block = 32 token rows x one quarter of K x all experts, four waves: wave nq takes a quarter of the experts'
-// 16-column fragments (NF of them) against both 16-row fragments of the block's rows, with four k-steps of operands in
+// One block = 16 FRAGS token rows x one quarter of K x all experts: wave nq takes NF of the experts'
+// 16-column fragments against the 16-row fragments of the block's rows, with DEPTH k-steps of operands in
 // flight. Every block reads its quarter of the weights once, so what the pass moves through the second-level cache is
-// (rows / 32) x the weights - the time of this pass is that traffic and the round trips it is made of, not its
-// arithmetic; 16 rows per block with K inside the block moved twice as much on three quarters of the compute units.
-// Block 4 b + q leaves the sums of K quarter q for rows 32 b .. 32 b + 31 in approx[q] and the rows' squares in
+// (rows / 16 FRAGS) x the weights - the time of this pass is that traffic and the round trips it is made of, not its
+// arithmetic. With few rows the round trips decide: blocks of 16 rows with six steps in flight (eight where a wave has one
+// fragment); with many the traffic: 32 rows and four. Router of 2,816 x 128, us of the call at 32 | 16 rows per block: 301 rows 16.0 |
+// 13.8, 1,000 rows 21.6 | 19.6, 2,000 rows 30.6 | 29.6, 3,072 rows 41.2 | 41.4, 8,192 rows 91.7 | 96.8; FP16, whose rows are split in
+// every block, 19.1 | 15.3, 24.9 | 21.2, 33.3 | 31.4, 46.4 | 44.2, 102 | 104 (all with four waves per token in the second pass; one fragment
+// per wave and eight waves, 16 rows: 13.9, 19.6, 31.0, 43.8). 3,072 rows, bf16, of 4,096 x 128 38 | 40. Up to 1,024 columns a quarter of K
+// is at most eight steps, and the traffic decides earlier: 512 x 32, 900 rows 8.6 | 8.2, 1,400 rows 8.7 | 8.9, FP16 2,000 rows 10.0 | 10.7.
+// Block 4 b + q leaves the sums of K quarter q for its rows in approx[q] and the rows' squares in
 // xnorm2[q]; the reader adds them as (q0 + q1) + (q2 + q3). The loop body has no branch: the compiler then counts the
 // loads in flight exactly and waits for the oldest step only (behind a branch it waits for all of them, and the pass is
 // one round trip per step).
-constexpr int kApproxDepth = 4;
+static bool approx_few_rows(uint32_t t, uint32_t d, bool f16) { return t <= (d <= 1024 ? 1024u : f16 ? 3072u : 2048u); }
 
 // Eight FP16 values as two sets of eight bf16 values whose sums are the FP16 values exactly (eleven significant bits =
 // the leading eight + the remaining three), so that FP16 rows meet the bf16 weights on the bf16 matrix instruction with
@@ -273,54 +276,54 @@ __device__ __forceinline__ void split_f16x8(const uint4 &v, uint4 &lead, uint4 &
     rest = uint4{b[0], b[1], b[2], b[3]};
 }
 
-template <int NF, bool F16>
+template <int NF, int FRAGS, int DEPTH, bool F16>
 __global__ __launch_bounds__(256) void router_approx_kernel(const uint4 *__restrict__ wfrag, const uint16_t *__restrict__ x,
                                                             uint32_t x_stride, uint32_t t, uint32_t t_pad, uint32_t n_experts,
                                                             uint32_t d, float *__restrict__ approx, float *__restrict__ xnorm2) {
     const uint32_t lane = threadIdx.x & 63, nq = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t kq = blockIdx.x % kApproxKParts, t0 = (blockIdx.x / kApproxKParts) * kApproxTok;
+    const uint32_t kq = blockIdx.x % kApproxKParts, t0 = (blockIdx.x / kApproxKParts) * (16 * FRAGS);
     const uint32_t j = lane & 15, jq = lane >> 4;
     const uint32_t nfrag = n_experts / 16, nh = d / 32;
     const uint32_t h0 = kq * nh / kApproxKParts, h1 = (kq + 1) * nh / kApproxKParts, span = h1 - h0;
     const uint32_t n0 = nq * NF;                       // this wave's fragments: n0 .. n0 + NF - 1 (those below nfrag)
     // the rows are loaded four neighbouring lanes per 64 contiguous bytes (row lane / 4, chunk lane % 4: 16 requests per
     // instruction instead of 64) and turned into the operand layout (lane (j, jq): row j, chunk jq) by cross-lane moves
-    const uint16_t *xr[kApproxFrags];
+    const uint16_t *xr[FRAGS];
 #pragma unroll
-    for (int f = 0; f < kApproxFrags; ++f) xr[f] = x + (size_t)min(t0 + 16 * f + (lane >> 2), t - 1) * x_stride + 8 * (lane & 3);
+    for (int f = 0; f < FRAGS; ++f) xr[f] = x + (size_t)min(t0 + 16 * f + (lane >> 2), t - 1) * x_stride + 8 * (lane & 3);
     const int pull = (int)((4 * j + jq) * 4);
     const uint4 *wf = wfrag + lane;
-    f32x4 acc[kApproxFrags][NF];
-    float x2[kApproxFrags];
+    f32x4 acc[FRAGS][NF];
+    float x2[FRAGS];
 #pragma unroll
-    for (int f = 0; f < kApproxFrags; ++f) {
+    for (int f = 0; f < FRAGS; ++f) {
         x2[f] = 0.0f;
 #pragma unroll
         for (int n = 0; n < NF; ++n) acc[f][n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    uint4 a_q[kApproxDepth][kApproxFrags], b_q[kApproxDepth][NF];
+    uint4 a_q[DEPTH][FRAGS], b_q[DEPTH][NF];
     // step i of this block = k-step h0 + i; past the end it repeats the last step and enters with zero rows
     auto fetch = [&](int slot, uint32_t i) {
         const uint32_t h = h0 + min(i, span - 1);
 #pragma unroll
-        for (int f = 0; f < kApproxFrags; ++f) a_q[slot][f] = *reinterpret_cast<const uint4 *>(xr[f] + 32 * h);
+        for (int f = 0; f < FRAGS; ++f) a_q[slot][f] = *reinterpret_cast<const uint4 *>(xr[f] + 32 * h);
 #pragma unroll
         for (int n = 0; n < NF; ++n) b_q[slot][n] = wf[((size_t)h * nfrag + min(n0 + n, nfrag - 1)) * 64];
     };
     if (span) {
 #pragma unroll
-        for (int u = 0; u < kApproxDepth; ++u) fetch(u, u);
-        for (uint32_t ib = 0; ib < span; ib += kApproxDepth) {
+        for (int u = 0; u < DEPTH; ++u) fetch(u, u);
+        for (uint32_t ib = 0; ib < span; ib += DEPTH) {
 #pragma unroll
-            for (int u = 0; u < kApproxDepth; ++u) {
-                uint4 a[kApproxFrags], b[NF];
+            for (int u = 0; u < DEPTH; ++u) {
+                uint4 a[FRAGS], b[NF];
 #pragma unroll
-                for (int f = 0; f < kApproxFrags; ++f) a[f] = a_q[u][f];
+                for (int f = 0; f < FRAGS; ++f) a[f] = a_q[u][f];
 #pragma unroll
                 for (int n = 0; n < NF; ++n) b[n] = b_q[u][n];
-                fetch(u, ib + u + kApproxDepth);
+                fetch(u, ib + u + DEPTH);
 #pragma unroll
-                for (int f = 0; f < kApproxFrags; ++f) {
+                for (int f = 0; f < FRAGS; ++f) {
                     a[f].x = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)a[f].x);
                     a[f].y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)a[f].y);
                     a[f].z = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)a[f].z);
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(256) void router_approx_kernel(const uint4 *__restr
         }
     }
 #pragma unroll
-    for (int f = 0; f < kApproxFrags; ++f) {
+    for (int f = 0; f < FRAGS; ++f) {
         // the row's squares over this part of K: the four k-chunk lanes of a row
         x2[f] += __shfl_xor(x2[f], 16, 64);
         x2[f] += __shfl_xor(x2[f], 32, 64);
@@ -384,8 +387,12 @@ __device__ __forceinline__ float sum_k_parts(const float *__restrict__ p, size_t
 
 constexpr int kExactSteps = 4;          // d <= 4096: k = 1024 i + 256 s + 4 lane + j, i < 4
 
-// STEPS: 1024-wide steps of the pinned order that d needs; CHUNK: candidates whose rows are requested together.
-template <int STEPS, int CHUNK, bool F16>
+// STEPS: 1024-wide steps of the pinned order that d needs; CHUNK: candidates whose rows are requested together; PARTS: waves of a
+// block that share a token. A wave is a chain: its token's sums, the threshold, two or three round trips for the candidates' rows, their
+// sums, the select. While the tokens leave waves idle, PARTS of them do the first of it alike and a PARTS-th of the candidates each.
+// 2,816 x 128, us of the call at 1 | 2 | 4: 301 rows 20.3 | 17.5 | 16.0, 700 rows 21.4 | 19.4 | 17.1, 850 rows 21.1 | 19.7 | 21.0, 1,400
+// rows 24.8 | 22.4 | 25.7, 2,000 rows 25.3 | 28.7 | 30.6: four while three blocks per compute unit hold all, two while those do.
+template <int STEPS, int CHUNK, int PARTS, bool F16>
 __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_t *__restrict__ w, const uint16_t *__restrict__ x,
                                                                    uint32_t x_stride, uint32_t t, uint32_t n_experts, uint32_t d,
                                                                    uint32_t top_k, const float *__restrict__ approx,
@@ -393,8 +400,11 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
                                                                    float bound_per_norm,
                                                                    const uint16_t *__restrict__ per_expert_scale,
                                                                    uint32_t *__restrict__ out_idx, uint16_t *__restrict__ out_w) {
-    const uint32_t lane = threadIdx.x & 63, tok = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (tok >= t) return;
+    static_assert(4 % PARTS == 0, "a block of four waves");
+    __shared__ uint32_t keys[PARTS == 1 ? 1 : 4][PARTS == 1 ? 1 : 128];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t part = wave % PARTS, my_tok = blockIdx.x * (4 / PARTS) + wave / PARTS, tok = min(my_tok, t - 1);
+    if (PARTS == 1 && my_tok >= t) return;  // (else past the last: the last again, not stored, for the barrier)
     // the token's row, as the pinned order walks it: element j of (step i, sub-accumulator s) = x[1024 i + 256 s + 4 lane + j]
     const uint16_t *xr = x + (size_t)tok * x_stride;
     float xf[STEPS][4][4];
@@ -442,6 +452,16 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
     unsigned long long m0 = __ballot(lane < n_experts && (everyone || a[0] >= threshold));
     unsigned long long m1 = __ballot(64 + lane < n_experts && (everyone || a[1] >= threshold));
     uint32_t exact0 = 0u, exact1 = 0u;      // the pinned logits of this lane's two experts, as keys of the select
+    if constexpr (PARTS > 1) {
+        // every PARTS-th candidate is this wave's
+        auto share = [&](unsigned long long m, uint32_t before) __attribute__((always_inline)) {
+            const unsigned long long below = lane ? m << (64 - lane) : 0ull;
+            return __ballot((m >> lane & 1) && (before + __popcll(below)) % PARTS == part);
+        };
+        const uint32_t first = __popcll(m0);
+        m0 = share(m0, 0);
+        m1 = share(m1, first);
+    }
     // The candidates CHUNK at a time: all rows of a chunk are requested before the first sum runs, so a token pays a
     // few round trips to the weights instead of one per candidate.
     while (m0 | m1) {
@@ -489,6 +509,13 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
             if (e[q] == 64u + lane) exact1 = k_;
         }
     }
+    if constexpr (PARTS > 1) {
+        keys[wave][lane] = exact0, keys[wave][64 + lane] = exact1;
+        __syncthreads();
+        if (part || my_tok >= t) return;
+#pragma unroll
+        for (int q = 1; q < PARTS; ++q) exact0 = max(exact0, keys[wave + q][lane]), exact1 = max(exact1, keys[wave + q][64 + lane]);
+    }
     TopkRow tr;
     tr.key[0] = exact0, tr.key[1] = exact1, tr.key[2] = 0u, tr.key[3] = 0u;
     topk_select<2>(tr, top_k, lane);
@@ -499,7 +526,7 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
 
 hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uint32_t x_stride, uint32_t t,
                          uint32_t n_experts, uint32_t d, uint32_t top_k, float *logits, uint32_t *out_idx,
-                         uint16_t *out_w, KernelTimer *timer, bool f16, bool want_logits, float *scratch) {
+                         uint16_t *out_w, uint32_t n_cus, KernelTimer *timer, bool f16, bool want_logits, float *scratch) {
     timer->begin(s);
     const bool x_aligned = (reinterpret_cast<uintptr_t>(x) % 8 == 0) && (x_stride % 4 == 0);
     if (f16 && !x_aligned) return hipErrorInvalidValue;     // FP16 rows come 8-byte aligned (checked at the boundary)
@@ -525,13 +552,21 @@ hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uin
         // approximate logits of every expert on the matrix unit, the pinned ones only where the select can tell
         const uint32_t t_pad = (t + 63) & ~63u;
         float *xnorm2 = scratch, *approx = scratch + (size_t)kApproxKParts * t_pad;
-        const dim3 agrid((t + kApproxTok - 1) / kApproxTok * kApproxKParts);
-        const uint32_t per_wave = (n_experts / 16 + 3) / 4;       // fragments per wave: the four N quarters cover all of them
-#define FFMOE_APPROX(NF, H)                                                                                            \
-    hipLaunchKernelGGL((router_approx_kernel<NF, H>), agrid, dim3(256), 0, s, rw.w_frag, x, x_stride, t, t_pad, n_experts, d,  \
-                       approx, xnorm2)
-        if (f16) { if (per_wave <= 1) FFMOE_APPROX(1, true); else FFMOE_APPROX(2, true); }
-        else { if (per_wave <= 1) FFMOE_APPROX(1, false); else FFMOE_APPROX(2, false); }
+        const uint32_t nfrag = n_experts / 16;
+        const bool few = approx_few_rows(t, d, f16), paired = nfrag > 4;       // (two fragments per wave where four waves with one do not reach)
+#define FFMOE_APPROX(NF, FRAGS, DEPTH, H)                                                                                   \
+    hipLaunchKernelGGL((router_approx_kernel<NF, FRAGS, DEPTH, H>), dim3((t + 16 * FRAGS - 1) / (16 * FRAGS) * kApproxKParts), dim3(64 * ((nfrag + NF - 1) / NF)),  \
+                       0, s, rw.w_frag, x, x_stride, t, t_pad, n_experts, d, approx, xnorm2)
+#define FFMOE_APPROX_AS(H)                                                    \
+    do {                                                                      \
+        if (paired) {                                                         \
+            if (few) FFMOE_APPROX(2, 1, 6, H); else FFMOE_APPROX(2, 2, 4, H); \
+        } else {                                                              \
+            if (few) FFMOE_APPROX(1, 1, 8, H); else FFMOE_APPROX(1, 2, 4, H); \
+        }                                                                     \
+    } while (0)
+        if (f16) FFMOE_APPROX_AS(true); else FFMOE_APPROX_AS(false);
+#undef FFMOE_APPROX_AS
 #undef FFMOE_APPROX
         timer->mark(s, FFMOE_K_ROUTER_LOGITS);
         // 2 B per unit of ||x||: the rounding counts of the two sums (see above), 1 % on top for the norms' own rounding
@@ -539,15 +574,15 @@ hipError_t launch_router(hipStream_t s, RouterWeights rw, const uint16_t *x, uin
         // (FP16 rows enter as two bf16 halves: two instructions, 66 additions, per 32 elements)
         const float approx_roundings = (f16 ? 66.0f : 33.0f) * (float)(d / 128) + 2.0f, pinned_roundings = 4.0f * ((d + 1023) / 1024) + 8.0f;
         const float bound_per_norm = 2.02f * (approx_roundings * 0x1p-23f + pinned_roundings * 0x1p-24f) * rw.w_norm_max;
-#define FFMOE_EXACT_AS(STEPS, CHUNK, H)                                                                                    \
-    hipLaunchKernelGGL((router_exact_topk_kernel<STEPS, CHUNK, H>), dim3((t + 3) / 4), dim3(256), 0, s,                      \
-                       static_cast<const uint16_t *>(rw.w), x, x_stride, t, n_experts, d, top_k, approx, xnorm2, t_pad,        \
-                       bound_per_norm,                                                                                      \
-                       rw.per_expert_scale, out_idx, out_w)
-#define FFMOE_EXACT(STEPS, CHUNK)                                     \
-    do {                                                              \
-        if (f16) FFMOE_EXACT_AS(STEPS, CHUNK, true);                  \
-        else FFMOE_EXACT_AS(STEPS, CHUNK, false);                     \
+#define FFMOE_EXACT_AS(STEPS, CHUNK, PARTS)                                                                                   \
+    hipLaunchKernelGGL((f16 ? router_exact_topk_kernel<STEPS, CHUNK, PARTS, true> : router_exact_topk_kernel<STEPS, CHUNK, PARTS, false>), \
+                       dim3((t * PARTS + 3) / 4), dim3(256), 0, s, static_cast<const uint16_t *>(rw.w), x, x_stride, t, n_experts, d, top_k, \
+                       approx, xnorm2, t_pad, bound_per_norm, rw.per_expert_scale, out_idx, out_w)
+#define FFMOE_EXACT(STEPS, CHUNK)                                      \
+    do {                                                               \
+        if (t <= 3 * n_cus) FFMOE_EXACT_AS(STEPS, CHUNK, 4);           \
+        else if (t <= 6 * n_cus) FFMOE_EXACT_AS(STEPS, CHUNK, 2);      \
+        else FFMOE_EXACT_AS(STEPS, CHUNK, 1);                          \
     } while (0)
         if (d <= 1024) FFMOE_EXACT(1, 4); else if (d <= 2048) FFMOE_EXACT(2, 4); else if (d <= 3072) FFMOE_EXACT(3, 4); else FFMOE_EXACT(4, 2);
 #undef FFMOE_EXACT

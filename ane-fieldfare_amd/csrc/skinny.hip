@@ -1244,7 +1244,7 @@ hipError_t launch_verify_as(hipStream_t s, const uint8_t *arena_layer, ArenaGeom
                       route->router_x_stride % 4 == 0;
     if (route && !fuse) {
         const hipError_t e = launch_router(s, route->rw, route->router_x, route->router_x_stride, t, n_experts, g.d, top_k,
-                                           route->logits, const_cast<uint32_t *>(idx), const_cast<uint16_t *>(w), timer, F16);
+                                           route->logits, const_cast<uint32_t *>(idx), const_cast<uint16_t *>(w), n_cus, timer, F16);
         if (e != hipSuccess) return e;
     }
     timer->begin(s);

@@ -405,6 +405,41 @@ def test_prefill_router_fast_form_other_widths(oracle, torch, d, e):
     ctx.close()
 
 
+# rows just past where the two-pass form begins, the last and first row of a block of 16 and of 32, four, two and one wave per token (3 and
+# 6 tokens per compute unit), and the lines between blocks of 16 and of 32 rows (1,024 rows; past 1,024 columns 2,048, FP16 3,072)
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,e,t", [(256, 128, 57), (256, 80, 769), (256, 16, 1024), (256, 64, 1537), (512, 128, 1025), (1280, 48, 3073),
+                                   (2816, 128, 161), (2816, 112, 767), (3072, 128, 770), (2048, 64, 1536), (1280, 80, 2047), (1280, 128, 2049)])
+def test_prefill_router_two_pass_rows(oracle, torch, act, d, e, t):
+    """Every split of the two-pass router over waves and blocks: routes and weights bit for bit those of the form that computes
+    every pinned logit, with exact ties, experts one bf16 step apart, rows of huge and zero norm and rows without bounds (all
+    experts become candidates) at the front, in the middle and at the end."""
+    import fieldfare_moe as ff
+    ff.lib()
+    k = 8
+    rng = np.random.default_rng(d + e + t)
+    bits = oracle.bf16_bits(rng.normal(0, 0.02, (e, d)).astype(np.float32))
+    bits[5] = bits[3]
+    bits[e - 1] = bits[e - 2]
+    bits[7] = bits[6]
+    bits[7, 17] ^= 1
+    x = rng.normal(0, 1, (t, d)).astype(np.float32)
+    x[1], x[2], x[t // 2 + 1], x[t - 2] = x[1] * 1e3, 0.0, x[t // 2 + 1] * 1e-3, x[t - 2] * 200.0
+    x[4, d - 1], x[t // 2, 0], x[t - 1, d // 2] = np.inf, np.nan, -np.inf
+    x[8:12] = oracle.bf16_to_float(bits[6])[None] * 30          # the near-equal pair at the top
+    ctx = ff.Context(d, 64, e, k, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_router_bf16(0, bits)
+        xt = torch.from_numpy(x).to(torch.bfloat16 if act == "bf16" else torch.float16).cuda()
+        idx_fast, w_fast = ctx.router(0, xt)
+        idx_ref, w_ref, _ = ctx.router(0, xt, want_logits=True)
+        torch.cuda.synchronize()
+        assert np.array_equal(idx_fast.cpu().numpy(), idx_ref.cpu().numpy())
+        assert np.array_equal(bits_of(w_fast), bits_of(w_ref))
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,e,t", [(512, 96, 359), (256, 128, 65), (2816, 128, 1000)])
 def test_prefill_router_fast_form_at_the_context_row_limit(oracle, torch, act, d, e, t):
