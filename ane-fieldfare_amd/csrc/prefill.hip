@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kSortBlock) void prefill_hist_kernel(ItemSource src
     if (threadIdx.x < src.n_experts) block_cnt[(size_t)blockIdx.x * src.n_experts + threadIdx.x] = cnt[threadIdx.x];
 }
 
-// For a block of 1024 threads: per expert, turn the per-block counts (in memory or LDS) into per-block bases, then lay out the
+// One block of 1024 threads: per expert, turn the per-block counts into per-block bases, then lay out the
 // experts one after the other and cut each into M-tiles. Thread (expert e, chunk c) owns a contiguous run
 // of sort blocks, so the counts of a whole column are in flight at once and - up to kScanKeep per thread -
 // stay in registers between the summing pass and the pass that writes the bases.
@@ -78,9 +78,11 @@ constexpr int kScanThreads = 1024;
 // a run was read twice; short runs pay for the longer unrolled passes, 443.1 against 441.4 us for a plugin chunk of 3,079 rows)
 
 template <int kScanKeep>
-__device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad, uint32_t *__restrict__ block_cnt,
-                                             PrefillPlan *__restrict__ plan, PrefillTile *__restrict__ tiles, uint32_t max_tiles,
-                                             TileRows bm) {
+__global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad,
+                                                                    uint32_t *__restrict__ block_cnt,
+                                                                    PrefillPlan *__restrict__ plan,
+                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles,
+                                                                    TileRows bm) {
     __shared__ uint32_t total[FFMOE_MAX_EXPERTS], last_rows[FFMOE_MAX_EXPERTS];    // pairs, and those past the whole tiles
     __shared__ uint32_t offset[FFMOE_MAX_EXPERTS + 1];
     __shared__ uint32_t tile_off[FFMOE_MAX_EXPERTS + 1];
@@ -182,8 +184,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
         }
     }
     __syncthreads();
-    const uint32_t n_pairs = offset[n_experts];
-    if (!live) return n_pairs;
+    if (!live) return;
     uint32_t run = offset[e] + part[threadIdx.x];
 #pragma unroll
     for (int u = 0; u < kScanKeep; ++u) {
@@ -195,7 +196,7 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
         block_cnt[(size_t)b * n_experts + e] = run;
         run += c;
     }
-    if (ch != 0) return n_pairs;
+    if (ch != 0) return;
     plan->expert_offset[e] = offset[e];
     plan->expert_count[e] = total[e];
     // a tile keeps its number in row order, which places its activation blocks
@@ -213,16 +214,6 @@ __device__ __forceinline__ uint32_t plan_experts(uint32_t n_blocks, uint32_t n_e
             tiles[ti] = tl;
         }
     }
-    return n_pairs;
-}
-
-template <int kScanKeep>
-__global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_blocks, uint32_t n_experts, uint32_t e_pad,
-                                                                    uint32_t *__restrict__ block_cnt,
-                                                                    PrefillPlan *__restrict__ plan,
-                                                                    PrefillTile *__restrict__ tiles, uint32_t max_tiles,
-                                                                    TileRows bm) {
-    plan_experts<kScanKeep>(n_blocks, n_experts, e_pad, block_cnt, plan, tiles, max_tiles, bm);
 }
 
 // The lanes of the wave whose item has this lane's expert: a mask built from one ballot per bit of the expert number.
@@ -253,54 +244,117 @@ __device__ __forceinline__ void place_item(const ItemSource &src, uint32_t i, ui
     sorted_out_row[pos] = out_row;
 }
 
-// A chunk of few items in one launch: the three kernels' work by one block, the waves in place of the sort blocks - wave w has a
-// contiguous run of items, 64 at a time, and counts them in LDS; an item's place is what its wave counted before it. Same
-// order. Bound: latencies one behind the other, and 1.6 us per 1,024 items, which is why it ends at kSortKeep of them: a call with
-// three launches | with one, top-8 of 128, 37 rows 101.5 us | 99, 384 rows 130.2 | 128.6, 512 rows 160.9 | 161.2, 1,000 rows 191 | 196.
-// At 3,072 items one launch is the faster in every shape timed: top-8 of 64 45.5 | 43.5, of 256 39.9 | 39.2, top-4 of 32 and of 60
-// 87.4 | 85.2 and 74.3 | 72.2, top-2 of 16 75.9 | 73.7, top-1 of 4 62.8 | 60.7; at 1,024 items by 3 to 4 us.
-constexpr int kSortWaves = kScanThreads / 64, kSortKeep = 3;
-__global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource src, uint32_t e_pad, PrefillPlan *__restrict__ plan,
+// The three kernels' work in one launch, a block per expert: every block counts all items in LDS, marks its own expert's as it goes,
+// and knows after that where its expert's pairs and tiles begin - sums over the counts, no block waits for another. Wave w of a
+// block has a contiguous run of items, 64 at a time, eight loads in flight; an item's place is its expert's beginning and what its wave
+// and the waves in front hold of it. Same order as the three.
+// Bound: few items, latencies one behind the other; many, the counting, 27 cycles for a wave's 64 items, which every block does anew.
+// Call of a layer of 64 x 64, top-8 of 128, us: up to 3,072 items one block did the three kernels' work, that | this: 296 items 16.8 |
+// 14.3, 2,408 items 20.2 | 16.8; beyond, the three | this: 4,096 items 22.5 | 17.6, 8,000 items 23.6 | 17.7, 16,000 items 25.2 | 21.1,
+// 24,576 items 27.5 | 25.0 (Zipf routes 28.9 | 26.6), 32,768 items 28.9 | 29.3, 65,536 items 40 | 48; top-8 of 256, whose scan is
+// longer, 24,576 items 33.3 | 25.7, 65,536 items 57 | 47; top-1 of 32, 16,000 items 23.5 | 20.9, 24,576 items 25.4 | 25.9. Without the
+// shared start (blocks that begin at items of their own): the same.
+constexpr int kSortRuns = 64;                               // items of a lane: a bit each
+static uint32_t sort_one_launch(uint32_t n_experts) { return n_experts > 128 ? kSortRuns * kScanThreads : n_experts > 32 ? 24576u : 20480u; }
+// (256 threads up to 2,048 items: fewer waves to meet)
+static uint32_t sort_threads(uint32_t n_items) { return n_items <= 2048 ? 256 : kScanThreads; }
+__global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource src, PrefillPlan *__restrict__ plan,
                                                                     PrefillTile *__restrict__ tiles, uint32_t max_tiles,
                                                                     TileRows bm, uint32_t *__restrict__ sorted_token,
                                                                     uint32_t *__restrict__ sorted_out_row) {
-    __shared__ uint32_t sorted[kSortKeep * kScanThreads];
-    __shared__ uint32_t cnt[kSortWaves * FFMOE_MAX_EXPERTS];        // [wave][expert]: items counted so far, then the wave's base
-    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t runs = (src.n_items + kScanThreads - 1) / kScanThreads, first = wave * runs * 64 + lane;
-    uint32_t e[kSortKeep], rank[kSortKeep];
-#pragma unroll
-    for (int u = 0; u < kSortKeep; ++u) e[u] = (uint32_t)u < runs ? item_expert(src, first + u * 64) : 0xFFFFFFFFu;
-    for (uint32_t c = threadIdx.x; c < kSortWaves * src.n_experts; c += kScanThreads) cnt[c] = 0;
+    __shared__ uint32_t cnt[FFMOE_MAX_EXPERTS], wave_own[kScanThreads / 64];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6, mine = blockIdx.x;
+    for (uint32_t c = threadIdx.x; c < FFMOE_MAX_EXPERTS; c += blockDim.x) cnt[c] = 0;
     __syncthreads();
-    uint32_t *const own = cnt + wave * src.n_experts;
+    const uint32_t runs = (src.n_items + blockDim.x - 1) / blockDim.x, first = wave * runs * 64 + lane;
+    unsigned long long own = 0ull;
+    constexpr uint32_t kAhead = 8;
+    for (uint32_t u0 = 0; u0 < runs; u0 += kAhead) {
+        uint32_t e[kAhead];
+        if (src.pairs) {
 #pragma unroll
-    for (int u = 0; u < kSortKeep; ++u) {
-        if ((uint32_t)u < runs) {
-            const unsigned long long same = same_expert(e[u]);
-            const uint32_t in_front = __popcll(same & ((1ull << lane) - 1ull));
-            // (a wave's LDS instructions run in order: the counts as they are in front of this run, then with it)
-            if (e[u] != 0xFFFFFFFFu) rank[u] = own[e[u]] + in_front;
-            __builtin_amdgcn_wave_barrier();
-            if (e[u] != 0xFFFFFFFFu && in_front == 0) atomicAdd(&own[e[u]], (uint32_t)__popcll(same));
-            __builtin_amdgcn_wave_barrier();
+            for (uint32_t u = 0; u < kAhead; ++u) {
+                const ffmoe_pair p = src.pairs[min(first + (u0 + u) * 64, src.n_items - 1)];
+                e[u] = p.token < src.t && p.rank < src.top_k ? p.expert : 0xFFFFFFFFu;
+            }
+        } else {
+            // zero-weight routes are dropped, as the reference's prefill does (RealForwardRunner.swift:1528-1530)
+            uint16_t w[kAhead];
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u) {
+                const uint32_t i = min(first + (u0 + u) * 64, src.n_items - 1);
+                e[u] = src.idx[i], w[u] = src.w[i];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u) e[u] = (w[u] & 0x7FFFu) != 0 ? e[u] : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            const bool valid = u0 + u < runs && first + (u0 + u) * 64 < src.n_items && e[u] < src.n_experts;
+            if (valid) atomicAdd(&cnt[e[u]], 1u);
+            own |= (unsigned long long)(valid && e[u] == mine) << ((u0 + u) & 63);
         }
     }
+    // (counts up to kSortRuns * kScanThreads: exact in fp32, as are the sums below)
+    const uint32_t n_wave = (uint32_t)wave_butterfly_sum((float)__popcll(own));
+    if (lane == 0) wave_own[wave] = n_wave;
     __syncthreads();
-    const uint32_t n_pairs = plan_experts<4>(kSortWaves, src.n_experts, e_pad, cnt, plan, tiles, max_tiles, bm);
-    __syncthreads();
+    uint32_t n[FFMOE_MAX_EXPERTS / 64];
+    float in_front = 0.0f;
 #pragma unroll
-    for (int u = 0; u < kSortKeep; ++u)
-        if ((uint32_t)u < runs && e[u] != 0xFFFFFFFFu) {
-            const uint32_t i = first + u * 64;
-            sorted[own[e[u]] + rank[u]] = src.pairs ? src.pairs[i].token * src.top_k + src.pairs[i].rank : i;
+    for (uint32_t k = 0; k < FFMOE_MAX_EXPERTS / 64; ++k) {
+        n[k] = cnt[64 * k + lane];                          // (experts past the last hold zero)
+        if (64 * k + lane < mine) in_front += (float)n[k];
+    }
+    const uint32_t row0 = (uint32_t)wave_butterfly_sum(in_front);
+    uint32_t pos = row0;
+    for (uint32_t v = 0; v < wave; ++v) pos += wave_own[v];
+    if (n_wave) {
+        for (uint32_t u = 0; u < runs; ++u) {
+            const unsigned long long with = __ballot((own >> u) & 1ull);
+            if ((own >> u) & 1ull) place_item(src, first + u * 64, pos + (uint32_t)__popcll(with & ((1ull << lane) - 1ull)), sorted_token, sorted_out_row);
+            pos += (uint32_t)__popcll(with);
         }
-    __syncthreads();
-    // in order in LDS, then out in whole lines
-    for (uint32_t p = threadIdx.x; p < n_pairs; p += kScanThreads) {
-        const uint32_t out_row = sorted[p];
-        sorted_token[p] = out_row / src.top_k;
-        sorted_out_row[p] = out_row;
+    }
+    if (wave != waves - 1) return;
+    // The tile list runs from the largest tile down: the full tiles in expert order, then every expert's last, shorter
+    // tile by its rows (ties in expert order). The GEMM grids walk the list eight tiles at a time, so the launches end
+    // with their shortest blocks instead of with whatever the last experts hold (a Zipf chunk's heavy experts sit
+    // anywhere in the expert order).
+    const uint32_t n_mine = cnt[mine], whole_mine = bm.whole(n_mine), rest_mine = n_mine - whole_mine * bm.rows;
+    float full_front = 0.0f, full = 0.0f, pairs = 0.0f;
+    uint32_t shorter_front = 0, shorter = 0, above = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < FFMOE_MAX_EXPERTS / 64; ++k) {
+        const uint32_t o = 64 * k + lane, whole = bm.whole(n[k]), rest = n[k] - whole * bm.rows;
+        const bool front = o < mine;
+        full += (float)whole, pairs += (float)n[k];
+        full_front += front ? (float)whole : 0.0f;
+        shorter += (uint32_t)__popcll(__ballot(rest != 0));
+        shorter_front += (uint32_t)__popcll(__ballot(rest != 0 && front));
+        above += (uint32_t)__popcll(__ballot(rest > rest_mine || (rest != 0 && rest == rest_mine && front)));
+    }
+    const uint32_t full_in_front = (uint32_t)wave_butterfly_sum(full_front), full_tiles = (uint32_t)wave_butterfly_sum(full);
+    // a tile keeps its number in row order, which places its activation blocks
+    for (uint32_t i = lane; i < whole_mine + (rest_mine != 0 ? 1u : 0u); i += 64) {
+        const uint32_t ti = i < whole_mine ? full_in_front + i : full_tiles + above;
+        if (ti < max_tiles) {
+            PrefillTile tl;
+            tl.expert = mine;
+            tl.row_start = row0 + i * bm.rows;
+            tl.rows = min(bm.rows, n_mine - i * bm.rows);
+            tl.order = full_in_front + shorter_front + i;
+            tiles[ti] = tl;
+        }
+    }
+    const uint32_t n_pairs = (uint32_t)wave_butterfly_sum(pairs);
+    if (lane != 0) return;
+    plan->expert_offset[mine] = row0;
+    plan->expert_count[mine] = n_mine;
+    if (mine == 0) {
+        plan->n_pairs = n_pairs;
+        plan->n_tiles = min(full_tiles + shorter, max_tiles);
+        plan->expert_offset[src.n_experts] = n_pairs;
     }
 }
 
@@ -1559,13 +1613,13 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
         hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_rows, sc.plan, sc.tiles, sc.sorted_token,
                            sc.sorted_out_row);
     } else {
-        uint32_t e_pad = 1;
-        while (e_pad < n_experts) e_pad <<= 1;          // n_experts <= FFMOE_MAX_EXPERTS = 256 <= kScanThreads
-        if (src.n_items <= (uint32_t)kSortKeep * kScanThreads) {
-            hipLaunchKernelGGL(prefill_sort_kernel, dim3(1), dim3(kScanThreads), 0, s, src, e_pad, sc.plan, sc.tiles, sc.max_tiles, TileRows(tile_rows),
-                               sc.sorted_token, sc.sorted_out_row);
+        if (src.n_items <= sort_one_launch(n_experts)) {
+            hipLaunchKernelGGL(prefill_sort_kernel, dim3(n_experts), dim3(sort_threads(src.n_items)), 0, s, src, sc.plan, sc.tiles, sc.max_tiles,
+                               TileRows(tile_rows), sc.sorted_token, sc.sorted_out_row);
         } else {
             hipLaunchKernelGGL(prefill_hist_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, src, sc.block_cnt);
+            uint32_t e_pad = 1;
+            while (e_pad < n_experts) e_pad <<= 1;      // n_experts <= FFMOE_MAX_EXPERTS = 256 <= kScanThreads
             const uint32_t run = (n_blocks + kScanThreads / e_pad - 1) / (kScanThreads / e_pad);     // sort blocks per thread
             hipLaunchKernelGGL((run <= 16 ? prefill_scan_kernel<16> : prefill_scan_kernel<32>), dim3(1), dim3(kScanThreads), 0, s, n_blocks,
                                n_experts, e_pad, sc.block_cnt, sc.plan, sc.tiles, sc.max_tiles, TileRows(tile_rows));

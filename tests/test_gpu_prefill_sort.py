@@ -88,3 +88,41 @@ def test_reduce_of_rows_by_pieces_and_by_elements(oracle, act, t, k, d, skip):
         assert np.array_equal(got, oracle.reduce_token_major(bits(partials), kind, bits(w), kind))
     finally:
         ctx.close()
+
+
+# the last item count of one launch and the first of three (20,480, 24,576 and 65,536 items with up to 32, 128 and 256 experts), runs of 64
+# items per wave that end inside a group of eight loads, and the few items that 256 threads sort (2,048)
+@pytest.mark.parametrize("e,k,line,cuts", [(24, 2, 20480, (1023, 1025, 4500, 10240)), (33, 3, 24576, (682, 683, 2731, 8192)), (250, 8, 65536, (255, 257, 4097, 8192))])
+def test_one_launch_at_its_line(oracle, e, k, line, cuts):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, t = 64, 64, line // k + 3
+    rng, pool, _ = make_layer(oracle, 5 + e, d, f, e, align=1)
+    idx = np.argsort(rng.random((t, e)) - np.linspace(0, 0.6, e) * (rng.random((t, 1)) < 0.5), axis=1)[:, :k].astype(np.uint32)     # uneven
+    w = rng.uniform(0.2, 1.0, (t, k)).astype(np.float32)
+    w[rng.random((t, k)) < 0.05] = 0
+    ctx = ff.Context(d, f, e, k, n_layers=1, max_tokens=t)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(torch.bfloat16).cuda()
+        gi, gw = torch.from_numpy(idx.view(np.int32)).cuda(), torch.from_numpy(w).to(torch.bfloat16).cuda()
+
+        def rows(n):
+            # what a lost or doubled route leaves unwritten is NaN
+            ctx.prefill(0, torch.full_like(x, float("nan")), gi, torch.ones_like(gw))
+            y = ctx.prefill(0, x[:n], gi[:n].contiguous(), gw[:n].contiguous(), out=torch.full_like(x[:n], float("nan")))
+            n_pairs, n_tiles, counts = ctx.prefill_stats()
+            assert np.array_equal(counts, np.bincount(idx[:n][w[:n] > 0], minlength=e)) and n_pairs == counts.sum(), n
+            assert n_tiles == int(np.sum((counts + ff.PREFILL_TILE_M - 1) // ff.PREFILL_TILE_M)), n
+            return y
+
+        whole = rows(t)                                         # three launches
+        assert torch.isfinite(whole.float()).all() and whole.abs().max() > 0
+        assert torch.equal(rows(line // k), whole[:line // k])  # one launch, the same products
+        for n in cuts:                                          # (in the streaming product's range to its own bits: rounded weights elsewhere)
+            part = rows(n)
+            close = (part.float() - whole[:n].float()).abs() <= 2.0 ** -6 * whole[:n].float().abs() + 2.0 ** -6 * whole.float().abs().max()
+            assert close.all(), n
+    finally:
+        ctx.close()
