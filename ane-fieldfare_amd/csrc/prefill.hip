@@ -296,10 +296,10 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
             const bool valid = u0 + u < runs && first + (u0 + u) * 64 < src.n_items && e[u] < src.n_experts;
             uint32_t same = 1;
             bool adds = valid;
-            if (src.pairs || src.top_k == 1) {
-                // lists come sorted by expert, and neighbouring rows may agree: 64 lanes at one counter would take turns, so the first of a
-                // row of equals adds for all (8,000 pairs in order: 14.7 -> 7.4 us)
-                const uint32_t key = valid ? e[u] : 0xFFFFFFFFu, before = __shfl_up(key, 1, 64);
+            if (src.pairs) {
+                // lists come sorted by expert: 64 lanes at one counter would take turns, so the first of a row of equals adds for all
+                // (8,000 pairs in order: 14.7 -> 7.4 us; a table of top-1 routes, 20,480 random ones, would take 3 us more so)
+                const uint32_t key = valid ? e[u] : 0xFFFFFFFFu, before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0x138, 0xf, 0xf, false);    // (wave_shr:1)
                 const unsigned long long heads = __ballot(lane == 0 || key != before) >> lane >> 1;
                 adds = valid && (lane == 0 || key != before);
                 same = heads ? (uint32_t)__builtin_ctzll(heads) + 1 : 64 - lane;
