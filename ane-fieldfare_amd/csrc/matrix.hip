@@ -308,27 +308,31 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
 // GLU == 2: a 4-bit tile's stream A holds 16 rows of a gate projection and its stream B the same rows of the up projection - the
 // expert arena's gate/up tiles - and `m` counts the outputs gelu_tanh(gate . x) * (up . x), both sums fp32 in front of the
 // activation as in the expert kernels (moe.metal:496). GLU == 1 and PLANES8 as in the GEMV.
-// Bound: up to some 100 rows the chain of groups of one item (0.36 us each at one block of rows: the barrier, the expansion,
+// Four parts run two blocks per compute unit (four waves per SIMD, 128 registers, half the LDS, chunks of one group): what one block's
+// chain waits for the other fills. With one: 37 rows 14.3 us for both launches, now 12.9; 160 rows 23.3 | 20.8, 301 rows 32.0 | 28.7; 8 bits 19.4
+// | 16.9 and, 160 rows, 34.0 | 29.1. Two parts keep one: their chains are twice as long, their sums twice the registers.
+// Bound: up to some 100 rows the chain of groups of one item (the barrier, the expansion,
 // the products and their sums one behind the other), beyond that the products and the sums themselves, a third of the products
 // being the inputs' own sums, which every wave makes anew. Kept out, as they change nothing: the sums between the products or
 // behind six of them, with and without a raised wave priority. 2,816 -> 2,112 -> 2,816, 4 bits, us of gate/up + down with the GEMV's
 // passes of 16 rows | now: 96 rows 14 + 11 | 10 + 9, 190 rows 25 + 17 | 16 + 11, 301 rows 37 + 23 | 22 + 13, 384 rows 44 + 29 | 25 +
-// 17 (17 rows 7.7 + 5.8 | 7.5 + 6.7: the down product of up to 32 keeps the passes, launch_matrix_gemv); 8 bits, 17 rows 10.8 + 7.4 | 9.3
-// + 6.8, 37 rows 11.5 + 11.1 | 11.6 + 8.5, 190 rows 34 + 29 | 25 + 16.
+// 17 (17 rows 7.7 + 5.8 | 7.5 + 6.7: wide down products of up to 32 keep the passes, launch_matrix_gemv); 8 bits, 17 rows 10.8 + 7.4 | 9.3
+// + 6.8, 37 rows 11.5 + 11.1 | 11.6 + 8.5, 190 rows 34 + 29 | 25 + 16 (all with one block per unit).
 constexpr int kBandWaves = 8, kBandMax = 5;
 template <int PARTS, int R> struct Band {
     static constexpr int tiles = kBandWaves / PARTS, slices = kKSplit / PARTS;
-    static constexpr int groups = R <= 3 ? 2 : 1;                                   // of a chunk
+    static constexpr int blocks = PARTS / 2;                                        // per compute unit: PARTS waves per SIMD
+    static constexpr int groups = R <= 3 && blocks == 1 ? 2 : 1;                    // of a chunk
     static constexpr int scale_loads = (slices * kRing * kTileScaleBytes + 1023) / 1024;
     static constexpr uint32_t x_bytes = PARTS * R * 2048, group_bytes = x_bytes + kBandWaves * kTileBytes;
     static constexpr uint32_t scales_at = 0, ring_at = kBandWaves * scale_loads * 1024, chunk_bytes = groups * group_bytes;
-    static constexpr int room = (int)((160 * 1024 - ring_at) / chunk_bytes), depth = room < 6 ? room : 6;
+    static constexpr int room = (int)((160 * 1024 / blocks - ring_at) / chunk_bytes), depth = room < 6 ? room : 6;
     static constexpr uint32_t bytes = ring_at + depth * chunk_bytes;
     static constexpr int x_loads = (2 * R + tiles - 1) / tiles, loads = groups * (x_loads + 1);     // per wave and chunk
 };
 
 template <bool F16, bool PLANES8, int GLU, int PARTS, int R>
-__global__ __launch_bounds__(64 * kBandWaves, 2) void matrix_band_kernel(const uint8_t *__restrict__ tiles, const uint8_t *__restrict__ scales,
+__global__ __launch_bounds__(64 * kBandWaves, PARTS) void matrix_band_kernel(const uint8_t *__restrict__ tiles, const uint8_t *__restrict__ scales,
                                                                          uint32_t m, uint32_t n_groups, const uint16_t *__restrict__ x,
                                                                          uint32_t x_stride, uint32_t rows, uint16_t *__restrict__ y,
                                                                          uint32_t y_stride) {
@@ -644,10 +648,11 @@ size_t matrix_tiles_bytes(uint32_t m, uint32_t n, bool planes8) {
 size_t matrix_scales_bytes(uint32_t m, uint32_t n, bool planes8) {
     return (size_t)(planes8 ? (m + 15) / 16 : (m + 31) / 32) * (n / kGroup) * kTileScaleBytes;
 }
-// Parts of K per block and 16-row blocks per band: the pair whose rounds of items over the compute units cost least, an item's
-// time being 5 us + 0.18 us per group of its chain and (row block + 1). 2,816 -> 2 x 2,112 gated, 4 bits, us at parts.blocks: 37 rows
-// 4.1 9, 4.3 14, 2.1 13; 96 rows 4.1 17 (two rounds), 4.2 12, 2.1 14; 190 rows 4.3 25, 2.2 17, 2.3 22; 301 rows 4.3 26, 2.3 22, 2.4
-// 25; 384 rows 2.3 38, 2.4 25. Any gives the same bits.
+// Parts of K per block and 16-row blocks per band: the pair that costs least by what was measured, in units of 0.18 us. Four parts, two
+// blocks per compute unit: a unit's first block takes 14 and 1.3 R per group of its chain, the second beside it 6 and 0.9 R. Two parts,
+// one block, twice the chain: 12 and R + 0.7 per group. 2,816 -> 2 x 2,112 gated, then 2,112 -> 2,816 in the same shape, 4 bits, us at
+// parts.blocks: 37 rows 4.1 12.9, 4.2 16.4; 64 rows 4.1 15.6, 4.2 16.6; 96 rows 4.1 18.1, 4.2 16.9; 160 rows 4.1 22.6, 4.2 21.5, 4.3
+// 26.7; 240 rows 4.1 29.4, 4.2 30.1, 4.3 27.2, 2.3 35; 384 rows 4.2 41.7, 4.3 40.2, 2.4 42.2. Any gives the same bits.
 struct BandShape {
     uint32_t parts, blocks;
 };
@@ -656,9 +661,10 @@ static BandShape band_shape(uint32_t rows, uint32_t n_tiles, uint32_t n_groups, 
     BandShape best = {2, kBandMax};
     uint64_t least = ~0ull;
     for (uint32_t parts = 4; parts >= 2; parts -= 2)
-        for (uint32_t r = 1; r <= (parts == 4 ? 3u : (uint32_t)kBandMax); ++r) {
+        for (uint32_t r = parts == 4 ? 1 : 2; r <= (parts == 4 ? 3u : (uint32_t)kBandMax); ++r) {
             const uint32_t per_block = kBandWaves / parts, items = (row_blocks + r - 1) / r * ((n_tiles + per_block - 1) / per_block);
-            const uint64_t cost = (uint64_t)((items + n_cus - 1) / n_cus) * (28 + kKSplit / parts * per * (1 + r));
+            const uint64_t on_each = (items + n_cus - 1) / n_cus;
+            const uint64_t cost = parts == 4 ? (on_each + 1) / 2 * (14 + 13 * per * r / 10) + on_each / 2 * (6 + 9 * per * r / 10) : on_each * (12 + per * (20 * r + 14) / 10);
             if (cost < least) least = cost, best = BandShape{parts, r};
         }
     return best;
@@ -687,10 +693,11 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
     const uint32_t n_tiles = (planes8 || glu == 2) ? (m + 15) / 16 : (m + 31) / 32;      // glu == 1: pairs of tiles
     if (rows == 0 || rows > (1u << 20) || (rows > FFMOE_MAX_VERIFY_ROWS ? y_f32 : glu == 2)) return hipErrorInvalidValue;
     const uint32_t all_tiles = glu == 1 ? 2 * n_tiles : n_tiles;
-    // 17 to 32 rows of the plain 4-bit form: beyond 24 groups the GEMV's two grid rows, all of whose weights are on their way at once,
-    // beat the band's chain of groups. Gate/up in a band, then down bands | GEMV, us at 17 rows: 2,816 columns out, K of 1,024 12.3 | 13.3,
-    // 1,408 13.2 | 13.5, 1,600 13.6 | 13.5, 2,112 14.5 | 13.5, 2,816 15.4 | 14.0; 512 out, K of 1,792 10.1 | 10.0, 2,816 11.7 | 10.4.
-    const bool twice = rows > FFMOE_MAX_VERIFY_ROWS && rows <= 2 * FFMOE_MAX_VERIFY_ROWS && glu == 0 && !planes8 && n / kGroup > 6 * kKSplit;
+    // 17 to 32 rows of the plain 4-bit form: beyond 32 groups the GEMV's two grid rows, all of whose weights are on their way at once,
+    // beat the band's chain of groups. Gate/up in a band, then down bands | GEMV, us at 17 rows: 2,816 columns out, K of
+    // 1,600 12.0 | 12.4, 1,792 12.1 | 12.6, 2,112 12.8 | 12.6, 2,816 13.6 | 13.0; 1,024 out, 1,920 9.9 | 10.1; 512 out, 1,792 8.8 | 9.3, 2,816
+    // 10.3 | 9.7.
+    const bool twice = rows > FFMOE_MAX_VERIFY_ROWS && rows <= 2 * FFMOE_MAX_VERIFY_ROWS && glu == 0 && !planes8 && n / kGroup > 8 * kKSplit;
     if (rows > FFMOE_MAX_VERIFY_ROWS && !twice) {
         const BandShape shape = band_shape(rows, all_tiles, n / kGroup, n_cus);
         const uint32_t bands = ((rows + 15) / 16 + shape.blocks - 1) / shape.blocks, per_block = kBandWaves / shape.parts;
@@ -709,7 +716,6 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
             case 4 * 8 + 1: FFMOE_BAND(4, 1); break;
             case 4 * 8 + 2: FFMOE_BAND(4, 2); break;
             case 4 * 8 + 3: FFMOE_BAND(4, 3); break;
-            case 2 * 8 + 1: FFMOE_BAND(2, 1); break;
             case 2 * 8 + 2: FFMOE_BAND(2, 2); break;
             case 2 * 8 + 3: FFMOE_BAND(2, 3); break;
             case 2 * 8 + 4: FFMOE_BAND(2, 4); break;
