@@ -39,14 +39,29 @@ struct ffmoe_layer {
     uint8_t *gate_up8_ops = nullptr, *down8_ops = nullptr;
 };
 
-// From this many rows on an 8-bit dense layer goes through the library's dense GEMM on hi / lo rows instead of the resident-matrix
-// products (drawn where those were a pass per 16 rows, and kept with the bits on either side: 2,816 -> 2,112 -> 2,816, in bands of rows
-// 35 us at 160, 38 at 191, where passes took 66; the GEMM form 48 at 250, 52 at 384, 61 at 512).
+// From this many rows on an 8-bit dense layer may go through the library's dense GEMM on hi / lo rows instead of the resident-matrix
+// products; it does where that is the faster by what was measured, in units of 0.18 us: the library's GEMMs with their epilogues 31 us
+// and 9 per 10^9 of rows x d x f, as they come (2,816 -> 2,112, us at 192, 208, 224, 240, 256, 301, 384 rows 47, 44, 51, 46, 55, 48, 51; in bands
+// 38, 38, 39, 42, 46, 51, 64), the bands their cost. 2,048 -> 1,408, GEMM | bands: 192 rows 36 | 23, 301 rows 34 | 29, 448 rows 42 | 37, 480
+// rows 41 | 43; 1,024 -> 512: 192 rows 31 | 9.5, 480 rows 31 | 14. Beyond 512 rows only narrow layers': 704 -> 2,816, 560 rows 39 | 44, 192 -> 320 32 | 8.
+// FP16 keeps the line: its offset form has 4.17e-4 against 64 bits where the hi / lo rows have 4.16e-4 (192 rows of 2,816 -> 2,112; bf16 3.3e-3 both).
 constexpr uint32_t kGemm8MinRows = 192;
+static bool bands8_serve(uint32_t t, uint32_t d, uint32_t f, bool f16, uint32_t n_cus) {
+    const uint64_t products = (uint64_t)t * d * f;
+    return t < kGemm8MinRows || (!f16 && (t <= 512 || products <= 500000000) && band_pair_cost(t, d, f, true, n_cus) <= 152 + products / 20000000);
+}
 // Up to this many rows a 4-bit dense layer takes the resident-matrix products on its arena tiles (bands of input rows) instead of
-// the grouped products: 2,816 -> 2,112 -> 2,816, 301 rows 32 us against 41 in bf16 and 47 in FP16, 384 rows 39 against 46 and 51.
-// The rows of a chunk and of a part of it are equal bit for bit up to here.
-constexpr uint32_t kDenseStreamMaxRows = 384;
+// the grouped products: 2,816 -> 2,112 -> 2,816, 301 rows 29 us against 41 in bf16 and 47 in FP16, 384 rows 39 against 46 and 51.
+// The rows of a chunk and of a part of it are equal bit for bit up to here. bf16 stays with them up to kDenseBandMaxRows rows where the
+// grouped products, 8 us, 0.31 per group of d and f and 5.8 per 10^9 of rows x d x f, would take longer: grouped | bands, 2,816 -> 2,112, 400
+// rows 46 | 41, 512 rows 52 | 44, 700 rows 62 | 56, 768 rows 63 | 68; 2,816 -> 2,816, 512 rows 55 | 53, 560 rows 61 | 69; 2,048 -> 1,408, 400 rows
+// 30 | 26, 832 rows 39 | 36; 1,024 -> 512, 400 rows 17 | 10, 896 rows 18 | 15. (FP16 leaves: past the line the activations have block scales.)
+constexpr uint32_t kDenseStreamMaxRows = 384, kDenseBandMaxRows = kDenseTileStreamRows;
+static bool bands4_serve(uint32_t t, uint32_t d, uint32_t f, bool f16, uint32_t n_cus) {
+    if (t <= kDenseStreamMaxRows) return true;
+    if (f16 || t > kDenseBandMaxRows) return false;
+    return 100 * band_pair_cost(t, d, f, false, n_cus) <= 2000 + 172 * (uint64_t)((d + f) / 64) + (uint64_t)t * d * f / 310000;
+}
 
 // A resident matrix: the re-tiled copy of one [m][n] INT4 weight plus the scratch of its greedy choice.
 struct ffmoe_matrix {
@@ -873,7 +888,7 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
             ctx->timer.finish();
             return FFMOE_OK;
         }
-        if (t >= kGemm8MinRows && l.gate_up8_hilo) {
+        if (l.gate_up8_hilo && !bands8_serve(t, ctx->shape.d, ctx->shape.f, ctx->f16, ctx->n_cus)) {
             // many rows: two dense GEMMs of the library on the hi / lo rows (fp32 sums), each followed by the pass that adds
             // a weight row's two columns and rounds as the streaming form does
             const uint32_t f = ctx->shape.f, d = ctx->shape.d;
@@ -917,7 +932,8 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
     if (t <= FFMOE_MAX_VERIFY_ROWS)
         return verify_common(ctx, stream, layer, x, x_stride, t, ctx->dense_idx, ctx->dense_w, nullptr, nullptr, y, err, nullptr,
                              nullptr, true);
-    if (t <= kDenseStreamMaxRows && matrix_shape_ok(ctx->shape.d) && matrix_shape_ok(ctx->shape.f) && ctx->shape.f % 16 == 0) {
+    if (matrix_shape_ok(ctx->shape.d) && matrix_shape_ok(ctx->shape.f) && ctx->shape.f % 16 == 0 &&
+        bands4_serve(t, ctx->shape.d, ctx->shape.f, ctx->f16, ctx->n_cus)) {
         // 17 rows to a few hundred (a short prompt, a chunk's ragged end): below the row count at which the grouped GEMMs'
         // fixed cost (the weights' expansion per M-tile) is paid back, the resident-matrix GEMV streams the expert's arena
         // tiles as they lie - a gate/up tile's two streams are a gate and an up row block, a down tile is a plain 4-bit

@@ -207,6 +207,7 @@ struct SampleScratch {
 size_t matrix_tiles_bytes(uint32_t m, uint32_t n, bool planes8 = false);
 size_t matrix_scales_bytes(uint32_t m, uint32_t n, bool planes8 = false);
 bool matrix_shape_ok(uint32_t n);
+uint64_t band_pair_cost(uint32_t rows, uint32_t d, uint32_t f, bool planes8, uint32_t n_cus);
 hipError_t launch_matrix_repack(hipStream_t s, const uint8_t *w, const uint16_t *scales, const uint16_t *biases,
                                 uint32_t m, uint32_t n, uint8_t *tiles_out, uint8_t *scales_out, bool planes8 = false);
 hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t *scales, uint32_t m, uint32_t n,

@@ -655,19 +655,25 @@ size_t matrix_scales_bytes(uint32_t m, uint32_t n, bool planes8) {
 // 26.7; 240 rows 4.1 29.4, 4.2 30.1, 4.3 27.2, 2.3 35; 384 rows 4.2 41.7, 4.3 40.2, 2.4 42.2. Any gives the same bits.
 struct BandShape {
     uint32_t parts, blocks;
+    uint64_t cost;
 };
 static BandShape band_shape(uint32_t rows, uint32_t n_tiles, uint32_t n_groups, uint32_t n_cus) {
     const uint32_t row_blocks = (rows + 15) / 16, per = (n_groups + kKSplit - 1) / kKSplit;
-    BandShape best = {2, kBandMax};
-    uint64_t least = ~0ull;
+    BandShape best = {2, kBandMax, ~0ull};
     for (uint32_t parts = 4; parts >= 2; parts -= 2)
         for (uint32_t r = parts == 4 ? 1 : 2; r <= (parts == 4 ? 3u : (uint32_t)kBandMax); ++r) {
             const uint32_t per_block = kBandWaves / parts, items = (row_blocks + r - 1) / r * ((n_tiles + per_block - 1) / per_block);
             const uint64_t on_each = (items + n_cus - 1) / n_cus;
             const uint64_t cost = parts == 4 ? (on_each + 1) / 2 * (14 + 13 * per * r / 10) + on_each / 2 * (6 + 9 * per * r / 10) : on_each * (12 + per * (20 * r + 14) / 10);
-            if (cost < least) least = cost, best = BandShape{parts, r};
+            if (cost < best.cost) best = BandShape{parts, r, cost};
         }
     return best;
+}
+// What a gated product d -> f and a plain one back take in bands, in the same units (0.18 us; two launches are some 24 more).
+uint64_t band_pair_cost(uint32_t rows, uint32_t d, uint32_t f, bool planes8, uint32_t n_cus) {
+    const uint32_t f_tiles = (f + 15) / 16;
+    return band_shape(rows, planes8 ? 2 * f_tiles : f_tiles, d / kGroup, n_cus).cost +
+           band_shape(rows, planes8 ? (d + 15) / 16 : (d + 31) / 32, f / kGroup, n_cus).cost;
 }
 bool matrix_shape_ok(uint32_t n) { return n % kGroup == 0 && (n / kGroup + kKSplit - 1) / kKSplit <= (uint32_t)kRing; }
 

@@ -55,3 +55,28 @@ def test_4_bit_rows_equal_other_chunks(oracle, act, d, f, rows):
             assert torch.equal(ctx.dense_ffn(0, x[384 - t:]), want[384 - t:]), t
     finally:
         ctx.close()
+
+
+# more rows than the line below which bands always serve: where they are the faster (narrow layers) a row keeps the bits that it has in
+# chunks below the line; where the other form is (rows past the last of a shape's range) it comes within both forms' roundings of them
+@pytest.mark.parametrize("d,f,bits,rows", [(1024, 512, 4, (385, 512, 896)), (2816, 704, 4, (385, 640)), (192, 320, 4, (400, 895, 897)), (2816, 2816, 4, (400, 560)),
+                                           (1024, 512, 8, (192, 301, 511)), (192, 320, 8, (192, 639)), (2048, 1408, 8, (192, 448)), (2816, 2112, 8, (192, 208, 240, 301))])
+def test_rows_past_the_lines(oracle, d, f, bits, rows):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    past = {(192, 320, 4): 896, (2816, 2816, 4): 512, (2816, 2112, 8): 240}.get((d, f, bits), max(rows))
+    ctx, x = _context(ff, oracle, torch, "bf16", d, f, bits, max(rows))
+    try:
+        want = torch.cat([ctx.dense_ffn(0, x[r:r + 160]).clone() for r in range(0, max(rows), 160)])
+        assert torch.isfinite(want).all() and want.abs().max() > 0
+        for t in rows:
+            got = ctx.dense_ffn(0, x[:t])
+            if t <= past:
+                assert torch.equal(got, want[:t]), t
+            else:
+                # one rounding of the weights or of each activation more on either side (2^-9 of a term), and the rows' own (2^-9): within
+                # 2^-6 of the largest row
+                assert (got.float() - want[:t].float()).abs().max() <= 2.0 ** -6 * want.float().abs().max(), t
+    finally:
+        ctx.close()
