@@ -494,12 +494,6 @@ __global__ __launch_bounds__(64 * kBandWaves, PARTS) void matrix_band_kernel(con
     }
 }
 
-// The wave's largest key: by its upper half, then by the lower one of those that have it.
-__device__ __forceinline__ unsigned long long wave_max_key(unsigned long long k) {
-    const uint32_t hi = wave_max_u32((uint32_t)(k >> 32)), lo = wave_max_u32((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
-    return (unsigned long long)hi << 32 | lo;
-}
-
 // The block's largest key, the same in every thread (WAVES: 4 or 16; a wave's lanes hold all waves' keys several times over).
 template <int WAVES>
 __device__ __forceinline__ unsigned long long block_max_key(unsigned long long k, unsigned long long *s_k) {
@@ -510,10 +504,6 @@ __device__ __forceinline__ unsigned long long block_max_key(unsigned long long k
 }
 
 // The block's softmax pair, the same in every thread: the largest value first, then the sums relative to it. (No NaN comes here.)
-__device__ __forceinline__ float wave_max_f32(float v) {
-    const uint32_t u = wave_max_u32(orderable(v));
-    return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
-}
 template <int WAVES>
 __device__ __forceinline__ SoftmaxAcc block_softmax(SoftmaxAcc a, float2 *s_p) {
     float m = wave_max_f32(a.m);

@@ -26,6 +26,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "topk.hpp"
 
 namespace ffmoe {
 namespace {
@@ -75,8 +76,7 @@ struct SampleShared {
 };
 
 __device__ __forceinline__ float block_max_f(float v, SampleShared &sh) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    v = wave_max_f32(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) sh.red_f[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -87,8 +87,7 @@ __device__ __forceinline__ float block_max_f(float v, SampleShared &sh) {
 
 // sum in a fixed order: lanes by xor-butterfly, then the waves one after the other
 __device__ __forceinline__ float block_sum_f(float v, SampleShared &sh) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v = wave_butterfly_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) sh.red_f[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -99,11 +98,7 @@ __device__ __forceinline__ float block_sum_f(float v, SampleShared &sh) {
 
 // two sums side by side
 __device__ __forceinline__ float2 block_sum_f2(float2 v, SampleShared &sh) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        v.x += __shfl_xor(v.x, o, 64);
-        v.y += __shfl_xor(v.y, o, 64);
-    }
+    v = make_float2(wave_butterfly_sum(v.x), wave_butterfly_sum(v.y));
     float2 *red = reinterpret_cast<float2 *>(sh.red_k);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
@@ -117,12 +112,7 @@ __device__ __forceinline__ float2 block_sum_f2(float2 v, SampleShared &sh) {
 }
 
 __device__ __forceinline__ unsigned long long block_max_k(unsigned long long v, SampleShared &sh) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long other = ((unsigned long long)(uint32_t)__shfl_xor((int)(v >> 32), o, 64) << 32) |
-                                         (uint32_t)__shfl_xor((int)(uint32_t)v, o, 64);
-        v = other > v ? other : v;
-    }
+    v = wave_max_key(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) sh.red_k[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -238,13 +228,8 @@ __device__ __forceinline__ void sample_finish(SampleShared &sh, const SampleRule
             e = expf((v[u] - top) * invT);
             mine = ((unsigned long long)sample_key(v[u] * invT + sample_gumbel(seed, key, ids ? ids[at[u]] : at[u])) << 32) | (0xFFFFFFFFu - rank);
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            e += __shfl_xor(e, o, 64);
-            const unsigned long long other = __shfl_xor(mine, o, 64);
-            mine = other > mine ? other : mine;
-        }
-        esum += e;
+        mine = wave_max_key(mine);
+        esum += wave_butterfly_sum(e);
         best = mine > best ? mine : best;
     }
     if (lane == 0) {
@@ -407,7 +392,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float
 
 // ---- long rows: one sweep by many blocks, then one block per row -------------------------------------------------
 // Bound: the sweep is instruction issue (one tanhf and one expf, or the noise's two logf and 64-bit products, per logit),
-// spread over 128 blocks per full-vocabulary row; the second launch is a chain of LDS round trips.
+// spread over 128 blocks per full-vocabulary row; the second launch is a chain of round trips to memory and LDS, which is why its
+// reductions are register moves: 262,144 logits, the 64 largest, 5.2 + 12.1 us with shuffles and the bound found bit by bit, now 4.8 + 10.9.
 static_assert(kSampleMaxSegments <= kSampleThreads, "the finishing launches bring one segment per thread");
 constexpr int kScanThreads = 256, kScanPer = kSampleSegment / kScanThreads;
 static_assert(kSampleSegment % kScanThreads == 0 && kSampleGroup == 64, "a wave's load is one group");
@@ -435,26 +421,23 @@ __global__ __launch_bounds__(kScanThreads) void sample_scan_kernel(const float *
     if constexpr (TRUNCATED) {
         float sum = 0.0f;
         uint32_t finite = 0;
-        float top[kScanPer];
+        uint32_t top[kScanPer];
 #pragma unroll
         for (int u = 0; u < kScanPer; ++u) {
-            top[u] = c[u];
+            top[u] = c[u] == -INFINITY ? 0u : sample_key(c[u]);
             if (c[u] != -INFINITY) {
                 sum += expf(c[u] - cap);
                 ++finite;
             }
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-            for (int u = 0; u < kScanPer; ++u) top[u] = fmaxf(top[u], __shfl_xor(top[u], o, 64));
-            sum += __shfl_xor(sum, o, 64);
-            finite += (uint32_t)__shfl_xor((int)finite, o, 64);
-        }
+        for (int u = 0; u < kScanPer; ++u) top[u] = wave_max_u32(top[u]);
+        sum = wave_butterfly_sum(sum);
+        finite = (uint32_t)wave_butterfly_sum((float)finite);
         uint32_t *keys = sc.group_keys + (size_t)r * kSampleMaxGroups + seg * (kSampleSegment / kSampleGroup);
 #pragma unroll
         for (int u = 0; u < kScanPer; ++u)
-            if (lane == 0) keys[u * (kScanThreads / 64) + wave] = top[u] == -INFINITY ? 0u : sample_key(top[u]);
+            if (lane == 0) keys[u * (kScanThreads / 64) + wave] = top[u];
         if (lane == 0) {
             s_f[wave] = sum;
             s_n[wave] = finite;
@@ -475,8 +458,7 @@ __global__ __launch_bounds__(kScanThreads) void sample_scan_kernel(const float *
         float m = -INFINITY;
 #pragma unroll
         for (int u = 0; u < kScanPer; ++u) m = fmaxf(m, c[u]);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        m = wave_max_f32(m);
         if (lane == 0) s_f[wave] = m;
         __syncthreads();
         for (int w = 0; w < kScanThreads / 64; ++w) m = fmaxf(m, s_f[w]);
@@ -492,12 +474,8 @@ __global__ __launch_bounds__(kScanThreads) void sample_scan_kernel(const float *
             const unsigned long long k = ((unsigned long long)sample_key(g) << 32) | (0xFFFFFFFFu - i);
             best = k > best ? k : best;
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            sum += __shfl_xor(sum, o, 64);
-            const unsigned long long other = __shfl_xor(best, o, 64);
-            best = other > best ? other : best;
-        }
+        sum = wave_butterfly_sum(sum);
+        best = wave_max_key(best);
         if (lane == 0) {
             s_f[wave] = sum;
             s_k[wave] = best;
@@ -547,7 +525,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
     __shared__ SampleShared sh;
     __shared__ __align__(16) unsigned long long cand[kPickMaxCands];          // key << 32 | ~index: larger value first, then lower index
     __shared__ uint32_t group_list[kPickMaxGroups];
-    __shared__ uint32_t n_list, n_cand;
+    __shared__ uint32_t n_list, n_cand, reach_of[2][kSampleWaves];
     const uint32_t r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float *row = logits + (size_t)r * stride;
     const uint32_t n_groups = n_seg * (kSampleSegment / kSampleGroup);       // groups past the row's end hold key 0
@@ -572,30 +550,34 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
         return;
     }
     const uint32_t want = min(p.top_k, finite);
-    // A bound that at least `want` groups reach, found by wave 0 on the threads' largest keys (a lower bound of the groups'
-    // own want-th largest), bit by bit from the top until it leaves out most of the others.
+    // A bound that at least `want` groups reach, found on the threads' largest keys (a lower bound of the groups' own want-th
+    // largest), four bits at a time from the top until it leaves out most of the others: each of the sixteen waves counts for one
+    // value of the four. (Bit by bit by one wave it was 2 of the launch's 11.5 us.)
     uint32_t most = 0;
 #pragma unroll
     for (int s = 0; s < kPickSlots; ++s) most = max(most, keys[s]);
     sh.hist[tid] = most;
     __syncthreads();
-    if (wave == 0) {
-        uint32_t held[kSampleWaves];
+    static_assert(kSampleWaves == 16, "a wave per value of four bits");
+    uint32_t held[kSampleWaves];
 #pragma unroll
-        for (int s = 0; s < kSampleWaves; ++s) held[s] = sh.hist[64 * s + lane];
-        uint32_t low = 0, reach = kSampleThreads;
+    for (int s = 0; s < kSampleWaves; ++s) held[s] = sh.hist[64 * s + lane];
+    uint32_t low = 0, reach = kSampleThreads;
 #pragma unroll 1
-        for (int bit = 31; bit >= 0 && reach > want + want / 2; --bit) {
-            const uint32_t at = low | (1u << bit);
-            uint32_t c = 0;
+    for (int shift = 28; shift >= 0 && reach > want + want / 2; shift -= 4) {
+        const uint32_t at = low | (wave << shift);
+        uint32_t c = 0;
 #pragma unroll
-            for (int s = 0; s < kSampleWaves; ++s) c += __popcll(__ballot(held[s] >= at));
-            if (c >= want) low = at, reach = c;
-        }
-        if (lane == 0) sh.bin = max(low, 1u);      // fewer finite groups than `want`: every finite logit is a candidate
+        for (int s = 0; s < kSampleWaves; ++s) c += __popcll(__ballot(held[s] >= at));
+        uint32_t *const counts = reach_of[(shift >> 2) & 1];
+        if (lane == 0) counts[wave] = c;
+        __syncthreads();
+        c = counts[lane & 15];                                  // (wave 0's value is the bound so far: at least `want` reach it)
+        const int most_of = 31 - __builtin_clz((uint32_t)__ballot(c >= want) & 0xFFFFu);
+        low |= (uint32_t)most_of << shift;
+        reach = (uint32_t)__builtin_amdgcn_readlane((int)c, most_of);
     }
-    __syncthreads();
-    const uint32_t bound = sh.bin;
+    const uint32_t bound = max(low, 1u);           // fewer finite groups than `want`: every finite logit is a candidate
     const uint32_t key = sample_position_key(p, key_offset, r);
     // The candidates are first told apart by their raw value: `raw_low` is below every logit whose capped value reaches the
     // bound (the inverse of the cap at the bound less a few thousand times tanhf's error), so that the cap itself is
