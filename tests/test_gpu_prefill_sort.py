@@ -1,5 +1,5 @@
-"""The prefill's sort of routes in one launch (3,072 items and fewer) and in three: the same rows, bit for bit, from a chunk and from its
-beginning on either side of the line and from lists of pairs, counts per expert, routes of weight zero and experts past the last left
+"""The prefill's sort of routes in one launch and (past 20,480 to 65,536 items) in three: the same rows, bit for bit, from a chunk and from its
+beginning, on one side of the line and on either, and from lists of pairs, counts per expert, routes of weight zero and experts past the last left
 out. What a call does not write is NaN. (The order of an expert's pairs shows in no result.) Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
@@ -35,7 +35,7 @@ def test_one_launch_sorts_as_three_do(oracle, e, k, cuts):
             y = ctx.prefill(0, x[:n], routes[:n].contiguous(), weights[:n].contiguous(), out=torch.full_like(x[:n], float("nan")))
             return y, ctx.prefill_stats()
 
-        whole, stats = rows(t, gi, gw)                          # 3,072 + 5 k items: three launches
+        whole, stats = rows(t, gi, gw)                          # 3,072 + 5 k items
         assert torch.isfinite(whole.float()).all() and whole.abs().max() > 0
         assert np.array_equal(stats[2], counts(t, idx))
         for n in cuts:                                          # (the same products as the whole chunk's: equal bit for bit)
@@ -50,7 +50,7 @@ def test_one_launch_sorts_as_three_do(oracle, e, k, cuts):
             got, (n_pairs, _, per_expert) = rows(n, past, gw)
             assert np.array_equal(per_expert, counts(n, np.where(lost, e + 3, idx))) and n_pairs == per_expert.sum(), n
             assert torch.equal(got, rows(n, gi, less)[0]), n
-        # a list of pairs in any order, its first 3,072 (one launch) and all of it (three): the rows that are listed, no others
+        # a list of pairs in any order, its first 3,072 and all of it: the rows that are listed, no others
         token, rank = (v.reshape(-1) for v in np.divmod(rng.permutation(t * k), k))
         lists = np.stack([token, np.where((w > 0) & ~lost, idx, e + 3)[token, rank], rank, np.zeros_like(token)], 1).astype(np.int32)
         kept = torch.from_numpy(lists[:, 1] < e).cuda()
@@ -124,5 +124,37 @@ def test_one_launch_at_its_line(oracle, e, k, line, cuts):
             part = rows(n)
             close = (part.float() - whole[:n].float()).abs() <= 2.0 ** -6 * whole[:n].float().abs() + 2.0 ** -6 * whole.float().abs().max()
             assert close.all(), n
+    finally:
+        ctx.close()
+
+
+# 256 threads (2,048 pairs and fewer) and 1,024, runs of 64 pairs that end in one expert, in several and in pairs that are left out
+@pytest.mark.parametrize("e,k,n", [(128, 8, 8000), (128, 8, 2048), (3, 2, 2049), (200, 1, 130), (7, 4, 63), (1, 1, 700)])
+def test_lists_sorted_by_expert(oracle, e, k, n):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, t = 64, 64, (n + k - 1) // k + 40
+    rng, pool, _ = make_layer(oracle, 9 + e, d, f, e, align=1)
+    idx = np.stack([rng.permutation(e)[:k] for _ in range(t)])
+    token, rank = (v.reshape(-1) for v in np.divmod(rng.permutation(t * k)[:n], k))
+    lists = np.stack([token, idx[token, rank], rank, np.zeros_like(token)], 1).astype(np.int32)
+    out_of_range = rng.random(n) < 0.05
+    lists[out_of_range, rng.integers(0, 3)] += 1 << 20          # a token, an expert or a rank past the last
+    in_order = lists[np.argsort(lists[:, 1], kind="stable")]
+    ctx = ff.Context(d, f, e, k, n_layers=1, max_tokens=t)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(torch.bfloat16).cuda()
+        got = []
+        for pairs in (lists, in_order):
+            out = torch.full((t * k, d), float("nan"), dtype=x.dtype, device="cuda")
+            ctx.prefill_pairs(0, x, torch.from_numpy(pairs.copy()).cuda(), t, out)
+            n_pairs, _, counts = ctx.prefill_stats()
+            assert n_pairs == n - out_of_range.sum() and np.array_equal(counts, np.bincount(lists[~out_of_range, 1], minlength=e))
+            got.append(out.view(torch.int16))
+        assert torch.equal(got[0], got[1])                       # NaN where nothing is written, on both
+        written = torch.isfinite(out).all(1).cpu().numpy()
+        assert np.array_equal(np.flatnonzero(written), np.sort((token * k + rank)[~out_of_range]))
     finally:
         ctx.close()
