@@ -99,7 +99,7 @@ struct ffmoe_ctx {
     bool f16 = false;                // activations are FP16 (ffmoe_set_activation_dtype)
     // the 8-bit dense layers' GEMM form: the library handle and the fp32 sums [max_tokens][max(4 f, 2 d)]
     rocblas_handle blas = nullptr;
-    float *gemm8_sums = nullptr;                                // fewer rows than dense8_min_rows
+    float *gemm8_sums = nullptr;                                // (of fewer rows than dense8_min_rows)
     uint8_t *dense8_x = nullptr, *dense8_acts = nullptr;        // the integer form's inputs as operands, max_tokens rows
     SampleScratch sample{};          // what the sampled choice over long rows leaves between its two launches
     KernelTimer timer;

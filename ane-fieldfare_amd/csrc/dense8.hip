@@ -395,10 +395,14 @@ uint32_t n_blocks_of(uint32_t stored_rows) { return (stored_rows / 16 + kTilesN 
 // library's two take 22 us and 12.5 us per 1,000 rows and 10^6 weights of a projection: the lines cross where rows * d f / 10^6 is 68
 // times the groups of both products less 2,000 (fitted at 18 widths, GPU time, when a group of the chain took 0.7 us). A group is
 // 0.5 us now and the forms cross lower: library form | this one, us: 2,816 -> 2,112, 704 rows 76 | 56, 3,072 rows 248 | 140; 2,816 ->
-// 704, 1,024 rows 55 | 45; 1,024 -> 2,816, 1,024 rows 67 | 50. The line stays: a chunk keeps the form, and with it the bits, that
-// it had. Not below 640 rows, where the forms met at the widest, nor beyond 1,024, where the narrowest (2,816 -> 256) still
+// 704, 1,024 rows 55 | 45; 1,024 -> 2,816, 1,024 rows 67 | 50. The line of narrow layers stays: a chunk keeps the form, and with it the
+// bits, that it had. Wide ones change at 385 rows, where the library's form takes a step up: 2,816 -> 2,112, 301 rows 47 | 48, 384 rows 50 | 49,
+// 400 rows 65 | 49, 448 rows 68 | 50, 639 rows 63 | 50 (FP16 alike; errors against 64 bits equal: 3.32e-3, FP16 4.16e-4), those from
+// 2.8 * 10^6 weights of a projection at 560: 2,816 -> 1,024, 448 rows 40 | 41, 560 rows 45 | 42; 1,728 -> 1,664, 400 rows 37 | 38, 560 rows 44 | 38.
+// Narrower, 2,816 -> 704, 560 rows 38 | 40. Else not below 640 rows, where the forms met at the widest, nor beyond 1,024, where the narrowest (2,816 -> 256) still
 // crossed, but in a call that the library's own 41 us on the host bound.
 uint32_t dense8_min_rows(uint32_t d, uint32_t f) {
+    if ((uint64_t)d * f >= 2800000) return (uint64_t)d * f >= 4000000 ? 385 : 560;
     const uint32_t groups = all_groups_of(d) + all_groups_of(f);
     const uint64_t line = groups * 68ull <= 2000ull ? 0 : (groups * 68ull - 2000ull) * 1000000ull / ((uint64_t)d * f);
     return (uint32_t)(line < 640 ? 640 : line > 1024 ? 1024 : line);

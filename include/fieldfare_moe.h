@@ -490,10 +490,10 @@ int ffmoe_layer_tail_routed(ffmoe_ctx *ctx, void *stream, const uint16_t *route_
  * context with n_experts = 1 and top_k = 1, d and f multiples of 64 up to FFMOE_MATRIX_MAX_N. The layer is then kept as
  * a gated gate/up matrix and a down matrix of nibble planes (ffmoe_matrix_create_int8_glu / _int8) owned by the
  * context, and ffmoe_dense_ffn, ffmoe_route_verify_shared and ffmoe_layer_tail_routed_shared serve it like a 4-bit
- * layer: ffmoe_dense_ffn runs the two matrix products (beyond 16 rows in bands of input rows), or from 192 rows on (when the context's
- * max_tokens reaches that) two dense GEMMs of rocBLAS on hi + lo rows of the weights, kept in the activation type for
+ * layer: ffmoe_dense_ffn runs the two matrix products (beyond 16 rows in bands of input rows), or from 192 rows on (bf16: where bands are
+ * not the faster; when the context's max_tokens reaches that) two dense GEMMs of rocBLAS on hi + lo rows of the weights, kept in the activation type for
  * that purpose (4 more bytes per weight; that form is not meant for stream capture: the library may allocate workspace
- * on its first call), or from 640 rows on (up to 1,024 at narrow widths; likewise) two GEMMs of its own on the integer
+ * on its first call), or from 385 rows on (up to 1,024 at narrow widths; likewise) two GEMMs of its own on the integer
  * weights (2 more bytes per weight; these can be captured), with the same roundings (gate and up are rounded to 16 bits in front of the
  * activation, as the reference's fused kernel does, dequant_int8.metal:131-136). A layer is served in the width of
  * its latest upload: a later ffmoe_upload_layer / ffmoe_upload_expert_parts of the layer drops the 8-bit form. Blocking. */
