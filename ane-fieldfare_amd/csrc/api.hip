@@ -24,6 +24,7 @@ struct ffmoe_layer {
     // experts with weight scales of 2^104 and more, and whether there is one (an upload of the whole layer tells for all together)
     std::vector<bool> large_scales;
     bool any_large_scale = false;
+    bool large_scales8 = false;     // the 8-bit layer has one
     void *router_w = nullptr;       // bf16 or float [E][D]
     int router_is_f32 = 0;
     uint16_t *effective_scale = nullptr;
@@ -44,6 +45,8 @@ struct ffmoe_layer {
 // and 9 per 10^9 of rows x d x f, as they come (2,816 -> 2,112, us at 192, 208, 224, 240, 256, 301, 384 rows 47, 44, 51, 46, 55, 48, 51; in bands
 // 38, 38, 39, 42, 46, 51, 64), the bands their cost. 2,048 -> 1,408, GEMM | bands: 192 rows 36 | 23, 301 rows 34 | 29, 448 rows 42 | 37, 480
 // rows 41 | 43; 1,024 -> 512: 192 rows 31 | 9.5, 480 rows 31 | 14. Beyond 512 rows only narrow layers': 704 -> 2,816, 560 rows 39 | 44, 192 -> 320 32 | 8.
+// Layers with weight scales of 2^104 and more leave the bands from here on: 2,048 times a scale (the high nibbles' offset) swamps what
+// the other groups add and is infinite from 2^117 on, where the hi / lo rows hold the weight itself.
 // FP16 keeps the line: its offset form has 4.17e-4 against 64 bits where the hi / lo rows have 4.16e-4 (192 rows of 2,816 -> 2,112; bf16 3.3e-3 both).
 constexpr uint32_t kGemm8MinRows = 192;
 static bool bands8_serve(uint32_t t, uint32_t d, uint32_t f, bool f16, uint32_t n_cus) {
@@ -56,6 +59,7 @@ static bool bands8_serve(uint32_t t, uint32_t d, uint32_t f, bool f16, uint32_t 
 // grouped products, 8 us, 0.31 per group of d and f and 5.8 per 10^9 of rows x d x f, would take longer: grouped | bands, 2,816 -> 2,112, 400
 // rows 46 | 41, 512 rows 52 | 44, 700 rows 62 | 56, 768 rows 63 | 68; 2,816 -> 2,816, 512 rows 55 | 53, 560 rows 61 | 69; 2,048 -> 1,408, 400 rows
 // 30 | 26, 832 rows 39 | 36; 1,024 -> 512, 400 rows 17 | 10, 896 rows 18 | 15. (FP16 leaves: past the line the activations have block scales.)
+// A layer with weight scales of 2^104 and more is not for the bands: 128 times such a scale swamps the sums beside it (prefill_large.hip).
 constexpr uint32_t kDenseStreamMaxRows = 384, kDenseBandMaxRows = kDenseTileStreamRows;
 static bool bands4_serve(uint32_t t, uint32_t d, uint32_t f, bool f16, uint32_t n_cus) {
     if (t <= kDenseStreamMaxRows) return true;
@@ -888,7 +892,7 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
             ctx->timer.finish();
             return FFMOE_OK;
         }
-        if (l.gate_up8_hilo && !bands8_serve(t, ctx->shape.d, ctx->shape.f, ctx->f16, ctx->n_cus)) {
+        if (l.gate_up8_hilo && (l.large_scales8 ? t >= kGemm8MinRows : !bands8_serve(t, ctx->shape.d, ctx->shape.f, ctx->f16, ctx->n_cus))) {
             // many rows: two dense GEMMs of the library on the hi / lo rows (fp32 sums), each followed by the pass that adds
             // a weight row's two columns and rounds as the streaming form does
             const uint32_t f = ctx->shape.f, d = ctx->shape.d;
@@ -932,7 +936,7 @@ int ffmoe_dense_ffn(ffmoe_ctx *ctx, void *stream, uint32_t layer, const uint16_t
     if (t <= FFMOE_MAX_VERIFY_ROWS)
         return verify_common(ctx, stream, layer, x, x_stride, t, ctx->dense_idx, ctx->dense_w, nullptr, nullptr, y, err, nullptr,
                              nullptr, true);
-    if (matrix_shape_ok(ctx->shape.d) && matrix_shape_ok(ctx->shape.f) && ctx->shape.f % 16 == 0 &&
+    if (!ctx->layers[layer].any_large_scale && matrix_shape_ok(ctx->shape.d) && matrix_shape_ok(ctx->shape.f) && ctx->shape.f % 16 == 0 &&
         bands4_serve(t, ctx->shape.d, ctx->shape.f, ctx->f16, ctx->n_cus)) {
         // 17 rows to a few hundred (a short prompt, a chunk's ragged end): below the row count at which the grouped GEMMs'
         // fixed cost (the weights' expansion per M-tile) is paid back, the resident-matrix GEMV streams the expert's arena
@@ -1311,6 +1315,15 @@ int ffmoe_upload_expert_parts_int8(ffmoe_ctx *ctx, uint32_t layer, const ffmoe_p
     drop_int8_form(l);
     l.gate_up8 = gu;
     l.down8 = dn;
+    uint32_t large = 0;
+    hipError_t el = launch_matrix8_large_scales(nullptr, gu->scales, matrix_scales_bytes(2 * sh.f, sh.d, true), dn->scales,
+                                                matrix_scales_bytes(sh.d, sh.f, true), &ctx->pf.plan->large_scales);
+    if (el == hipSuccess) el = hipMemcpy(&large, &ctx->pf.plan->large_scales, sizeof large, hipMemcpyDeviceToHost);
+    if (el != hipSuccess) {
+        drop_int8_form(l);
+        return fail(err, FFMOE_ERR_RUNTIME, "the scales of the 8-bit layer: %s", hipGetErrorString(el));
+    }
+    l.large_scales8 = large != 0;
     if (sh.max_tokens >= kGemm8MinRows) {
         // large row counts go through the library's dense GEMM on hi / lo rows of the activation type
         if (!ctx->blas && rocblas_create_handle(&ctx->blas) != rocblas_status_success) {

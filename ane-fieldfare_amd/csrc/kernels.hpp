@@ -210,6 +210,8 @@ bool matrix_shape_ok(uint32_t n);
 uint64_t band_pair_cost(uint32_t rows, uint32_t d, uint32_t f, bool planes8, uint32_t n_cus);
 hipError_t launch_matrix_repack(hipStream_t s, const uint8_t *w, const uint16_t *scales, const uint16_t *biases,
                                 uint32_t m, uint32_t n, uint8_t *tiles_out, uint8_t *scales_out, bool planes8 = false);
+// *large: cleared, then set where a scale of two 8-bit matrices as stored is a large one (kLargeScale)
+hipError_t launch_matrix8_large_scales(hipStream_t s, const uint8_t *a, size_t a_bytes, const uint8_t *b, size_t b_bytes, uint32_t *large);
 hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t *scales, uint32_t m, uint32_t n,
                               const uint16_t *x, uint32_t x_stride, uint32_t rows, void *y, uint32_t y_stride,
                               bool y_f32, uint32_t n_cus, bool f16 = false, bool planes8 = false, int glu = 0);

@@ -116,6 +116,12 @@ __global__ __launch_bounds__(256) void repack_matrix8_kernel(const uint8_t *__re
     }
 }
 
+// Eight bytes of an 8-bit matrix's scales (16 s and b, s and 0) per thread.
+__global__ __launch_bounds__(256) void large_scales8_kernel(const uint2 *__restrict__ scales, size_t count, uint32_t *__restrict__ large) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < count && (scales[i].y & 0x7FFFu) >= kLargeScale) *large = 1;
+}
+
 // Greedy choice per row: the largest finite value wins, ties go to the lowest index, NaN and +-inf never
 // win; a row with no candidate yields index 0 (Metal/Sampling/logit.metal:689-720, 916-921). Two stages: the
 // GEMV's blocks each leave the winner of the weight rows they walked, then one block per input row picks
@@ -677,6 +683,16 @@ hipError_t launch_matrix_repack(hipStream_t s, const uint8_t *w, const uint16_t 
     else
         hipLaunchKernelGGL(repack_matrix_kernel, dim3(blocks), dim3(256), 0, s, w, reinterpret_cast<const uint8_t *>(scales),
                            reinterpret_cast<const uint8_t *>(biases), m, n, tiles_out, scales_out);
+    return hipGetLastError();
+}
+
+hipError_t launch_matrix8_large_scales(hipStream_t s, const uint8_t *a, size_t a_bytes, const uint8_t *b, size_t b_bytes, uint32_t *large) {
+    const hipError_t e = hipMemsetAsync(large, 0, sizeof *large, s);
+    if (e != hipSuccess) return e;
+    for (int k = 0; k < 2; ++k) {
+        const size_t count = (k ? b_bytes : a_bytes) / sizeof(uint2);
+        hipLaunchKernelGGL(large_scales8_kernel, dim3((uint32_t)((count + 255) / 256)), dim3(256), 0, s, reinterpret_cast<const uint2 *>(k ? b : a), count, large);
+    }
     return hipGetLastError();
 }
 

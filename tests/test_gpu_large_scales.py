@@ -1,4 +1,4 @@
-"""Prefill chunks of layers with INT4 weight scales from 2^104 up: what a form that carries 2^24 on the scale would turn into
+"""Prefill and dense chunks of layers with weight scales from 2^104 up: what a form that carries 2^24 on the scale would turn into
 infinities and NaN is as finite here as q * scale + bias is - whole groups with q = 0 under such a scale (their weights are the
 biases), and in bf16 groups whose inputs are as small as the scale is large. Needs a GPU: pytest -m gpu."""
 import numpy as np
@@ -30,10 +30,10 @@ def _part(oracle, rng, rows, cols, tiny):
     return W, oracle.bf16_bits(scale), oracle.bf16_bits(bias.astype(np.float32))
 
 
-def _layer(oracle, seed, act):
+def _layer(oracle, seed, act, e=E):
     rng = np.random.default_rng(seed)
     tiny = act == "bf16"            # (FP16 has neither such weights nor such inputs)
-    parts = [tuple(_part(oracle, rng, rows, cols, tiny and cols == D) for rows, cols in ((F, D), (F, D), (D, F))) for _ in range(E)]
+    parts = [tuple(_part(oracle, rng, rows, cols, tiny and cols == D) for rows, cols in ((F, D), (F, D), (D, F))) for _ in range(e)]
     return rng, oracle.pool_from_parts(parts, D, F, 1, None)
 
 
@@ -61,6 +61,73 @@ def test_chunks_against_the_oracle(oracle, act, t):
         y = ctx.prefill(0, x.cuda(), torch.from_numpy(idx.view(np.int32)).cuda(), w.cuda()).float().cpu().numpy()
         assert np.isfinite(y).all()
         _check(oracle, pool, E, idx, x, w, y, act)
+    finally:
+        ctx.close()
+
+
+# a dense FFN's chunk where bands of rows serve other layers of these widths (in bf16 up to 896 rows, in FP16 up to 384) and beyond
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("t", [17, 100, 384, 385, 640, 896, 897])
+def test_dense_chunks_against_the_oracle(oracle, act, t):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    rng, pool = _layer(oracle, t, act, 1)
+    ctx = ff.Context(D, F, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        x = _rows(torch, rng, t, act)
+        y = ctx.dense_ffn(0, x.cuda()).float().cpu().numpy()
+        assert np.isfinite(y).all()
+        _check(oracle, pool, 1, np.zeros((t, 1), np.uint32), x, torch.ones((t, 1), dtype=x.dtype), y, act)
+    finally:
+        ctx.close()
+
+
+def _part8(oracle, rng, rows, cols):
+    """8-bit weights around a zero point of 128, but in every third row group 0 is q = 0 under scales of 2^104 .. 2^123."""
+    W = rng.integers(0, 256, size=(rows, cols), dtype=np.uint8)
+    scale = np.abs(rng.normal(0, 0.001, size=(rows, cols // 64))).astype(np.float32)
+    bias = -128.0 * oracle.bf16_to_float(oracle.bf16_bits(scale)) + rng.normal(0, 1e-3, size=scale.shape).astype(np.float32)
+    some = np.arange(0, rows, 3)
+    W[some, :64] = 0
+    scale[some, 0] = np.exp2(104.0 + some % 20)
+    bias[some, 0] = rng.normal(0, 0.02, size=len(some))
+    return W, oracle.bf16_bits(scale), oracle.bf16_bits(bias.astype(np.float32))
+
+
+# 8 bits: from 192 rows on, where bf16 chunks of other layers of these widths stay in bands up to 639
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("t", [192, 300, 512, 639, 640])
+def test_8_bit_dense_chunks_against_float64(oracle, act, t):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    rng = np.random.default_rng(t)
+    parts = tuple(_part8(oracle, rng, rows, cols) for rows, cols in ((F, D), (F, D), (D, F)))
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    x = torch.from_numpy(rng.normal(0, 1, (t, D)).astype(np.float32)).to(dt)
+    ctx = ff.Context(D, F, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_expert_parts(0, 0, *parts, int8=True)
+        y = ctx.dense_ffn(0, x.cuda()).double().cpu().numpy()
+        g, u, dn = (oracle.dequantize_int8(*p).astype(np.float64) for p in parts)
+        rnd = lambda a: torch.from_numpy(a).to(torch.float32).to(dt).double().numpy()
+        gate, up = rnd(x.double().numpy() @ g.T), rnd(x.double().numpy() @ u.T)
+        a = rnd(rnd(0.5 * gate * (1 + np.tanh(0.7978845608028654 * (gate + 0.044715 * gate ** 3)))) * up)
+        ref, spread = a @ dn.T, np.abs(a) @ np.abs(dn.T)
+        # one unit of gate, up and the activation each through the down product, where an fp32 sum near a rounding's middle goes the
+        # other way; then the output's own half unit
+        unit = 2.0 ** (-8 if act == "bf16" else -11)
+        assert np.isfinite(y).all() and np.all(np.abs(y - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
+        # and the same layer replaced by one without such scales: the bits of a context that never had one
+        plain = tuple((W, np.minimum(S, oracle.bf16_bits(np.float32([0.01]))[0]), B) for W, S, B in parts)
+        ctx.upload_expert_parts(0, 0, *plain, int8=True)
+        z = ctx.dense_ffn(0, x.cuda())
+        other = ff.Context(D, F, 1, 1, n_layers=1, max_tokens=t, act_dtype=act)
+        other.upload_expert_parts(0, 0, *plain, int8=True)
+        assert torch.equal(other.dense_ffn(0, x.cuda()), z)
+        other.close()
     finally:
         ctx.close()
 
