@@ -989,12 +989,14 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2 * GemmLds<LC>::kBlocks) void pre
 // a wave, whatever the pairs, in front of its products) bounds the launch below about 50 pairs per expert: with the GEMMs that this
 // form was built beside, 90 us for the 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s. Here a wave owns one arena tile row for the whole of K, streams its
 // packed tiles through a ring of four and multiplies them in the offset form of the decode kernels (stream.hpp): about 52
-// vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. The biases (and the offset's correction)
-// of four groups are one fp32 product per 16 pairs - the groups' input sums by the scales' second halves, K of 4 - and the
-// sums are made once per block, each wave its share, instead of once per wave: per 16 pairs, tile and group 88 cycles of the matrix
-// unit instead of 96, 8 vector instructions instead of 16. 128 experts of 2,816 x 704, top-8, router table to combined rows, us before | now:
-// 301 rows 122 | 118, 384 rows 136 | 128, 700 rows 178 | 172 (FP16 131 | 126, 141 | 132, 187 | 184); a dense 2,816 -> 2,112 FFN of 700 rows
-// 67 | 63; 20 pairs per expert and fewer wait for the weights' bytes and keep their times. The pairs' rows go through LDS in
+// vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. From two 16-pair blocks on the groups' input
+// sums are made once per block of waves, each wave its share, and come in by outer products on the matrix unit: per 16 pairs, tile and
+// group 80 cycles of it instead of 96, and 8 vector instructions instead of 16, for one more barrier per 128 columns. The sums
+// are the same and the order is a group's scale, then its bias (with the offset's correction): four groups' biases as one product of K = 4 would
+// be 2 to 4 % faster again, but carries 128 times four groups' inputs in a sum at once, which is two bits less of it. 128 experts of
+// 2,816 x 704, top-8, router table to combined rows, us with every wave's own sums | so: 301 rows 115.7 | 113.6, 448 rows 135.5 | 131.1,
+// 576 rows 152.6 | 148.1, 736 rows 170.7 | 165.7 (FP16 123.7 | 121.9, 138.2 | 133.1, 159.4 | 156.8, 180.9 | 175.8); 64 of 320 x 192, 30
+// pairs each, 17.8 | 18.4. The pairs' rows go through LDS in
 // operand order, two groups at a time in two buffers, so that every wave of the block reads the same fragments and the
 // registers hold one chunk's 16-byte pieces in flight; the weights stay in flight across the barriers. Gate/up of 37 rows
 // 90 -> 56 us (4.7 TB/s). What bounds it then is the weights' bytes (32 pairs per tile) and the matrix and vector instructions
@@ -1029,6 +1031,8 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4, tid = threadIdx.x;
     const uint32_t n_groups = gw.n_groups, last = n_groups - 1;
     const uint32_t n_chunks = (n_groups + CHUNK - 1) / CHUNK;
+    static_assert(16 * NM * kStreamStageRow <= 2 * kBuf * sizeof(uint4), "the down epilogue's rows fit in front of the sums");
+    static_assert(NM * 2 * kWave * sizeof(uint4) + 4 * 16 * NM * sizeof(float) <= 2 * kBuf * sizeof(uint4), "so do the activations and the peaks");
 
     // Where this thread's pieces of a chunk come from and go to.
     // GATE_UP: row tid / kRowPieces + kPassRows k of the tile, piece tid % kRowPieces of its contiguous bytes; in LDS piece p of row r sits
@@ -1085,71 +1089,73 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         ring_t[u] = make_uint4(t.x, t.y, t.z, t.w);
         ring_s[u] = make_uint2(s.x, s.y);
     };
-    TwoStreamAcc tot[NM];
+    // the sums of two 16-pair blocks: stream a and stream b of each, as the bias product's result has them
+    constexpr int kPairs = (NM + 1) / 2;
+    f32x16 tot[kPairs];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) tot[m].a = tot[m].b = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < kPairs; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[i][r] = 0.0f;
 
-    // The groups' input sums: of a chunk's 16-pair blocks and groups every wave takes its share, as one value per pair in LDS
-    // ([quad of groups % 2][16-pair block][group of the quad][pair]: the lane order of the bias product's operand).
+    // The groups' input sums, a value per pair in LDS ([chunk % 2][16-pair block][group of the chunk][pair]): every wave makes its
+    // share of a chunk's while the block is at the chunk before. (Of one 16-pair block every wave makes its own: two instructions
+    // against a barrier, 37 rows of 128 experts 104.6 | 102.1 us.)
     float *const sums = reinterpret_cast<float *>(lds + 2 * kBuf);
+    constexpr bool kShared = NM > 1;
     constexpr int kSums = (NM + 1) / 2;                   // 16-pair blocks per wave, of one of the chunk's two groups
-    static_assert(CHUNK == 2 && kStreamDepth == 4, "two waves per group of a chunk; a quad of groups per bias product");
-    auto sum_up = [&](uint32_t buf, uint32_t quad, int first) __attribute__((always_inline)) {
+    static_assert(CHUNK == 2, "two waves per group of a chunk");
+    auto sum_up = [&](uint32_t buf, int slot) __attribute__((always_inline)) {
         const int gl = wave & 1;
 #pragma unroll
         for (int k = 0; k < kSums; ++k) {
             const int m = min((int)(wave >> 1) + 2 * k, NM - 1);
             const f32x4 sx = group_input_sum<F16>(frag(buf, m, 2 * gl), frag(buf, m, 2 * gl + 1));
-            if (j == 0) *reinterpret_cast<f32x4 *>(sums + (((quad & 1) * NM + m) * 4 + first + gl) * 16 + 4 * jq) = sx;
-        }
-    };
-    // a quad's scale and bias pairs as the lane's group of it has them
-    uint2 quad_s = {0u, 0u};
-    auto add_bias = [&](uint32_t quad, auto whole) __attribute__((always_inline)) {
-        float ta = bf16hi_to_f32(quad_s.x), tb = bf16hi_to_f32(quad_s.y);
-        if constexpr (!F16) {
-            ta = __builtin_fmaf(-Act<F16>::kOffset, bf16lo_to_f32(quad_s.x), ta);
-            tb = __builtin_fmaf(-Act<F16>::kOffset, bf16lo_to_f32(quad_s.y), tb);
-        }
-        const bool live = decltype(whole)::value || 4 * quad + jq < n_groups;
-        if (!live) ta = tb = 0.0f;
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            const float sx = live ? sums[((quad & 1) * NM + m) * kWave + lane] : 0.0f;
-            tot[m].a = __builtin_amdgcn_mfma_f32_16x16x4f32(sx, ta, tot[m].a, 0, 0, 0);
-            tot[m].b = __builtin_amdgcn_mfma_f32_16x16x4f32(sx, tb, tot[m].b, 0, 0, 0);
+            if (j == 0) *reinterpret_cast<f32x4 *>(sums + ((slot * NM + m) * CHUNK + gl) * 16 + 4 * jq) = sx;
         }
     };
 
-    auto step = [&](uint32_t buf, int gl, int u, uint32_t refill) __attribute__((always_inline)) {
+    auto step = [&](uint32_t buf, int slot, int gl, int u, uint32_t refill) __attribute__((always_inline)) {
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         const uint4 tile = ring_t[u];
         const uint2 sc = ring_s[u];
-        if (u == 0 || jq == (uint32_t)u) quad_s = sc;
         fill(u, refill);
         const uint4 wa0 = unpack8_stream<F16>(tile.x), wa1 = unpack8_stream<F16>(tile.y);
         const uint4 wb0 = unpack8_stream<F16>(tile.z), wb1 = unpack8_stream<F16>(tile.w);
-        float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y);
+        float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y), ta = bf16hi_to_f32(sc.x), tb = bf16hi_to_f32(sc.y);
         if constexpr (F16) {
             sa *= FineNibble<true>::kUnit;
             sb *= FineNibble<true>::kUnit;
+        } else {
+            ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ta);
+            tb = __builtin_fmaf(-Act<F16>::kOffset, sb, tb);
         }
+        const float bias = jq & 1 ? tb : ta;
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
+            f32x16 &t = tot[m / 2];
+            const int at = 8 * (m & 1);
             const uint4 x0 = frag(buf, m, 2 * gl), x1 = frag(buf, m, 2 * gl + 1);
+            f32x4 sx = zero;
+            if (!kShared) sx = group_input_sum<F16>(x0, x1);
             f32x4 aa = Act<F16>::mfma(x0, wa0, zero);
             aa = Act<F16>::mfma(x1, wa1, aa);
             f32x4 ab = Act<F16>::mfma(x0, wb0, zero);
             ab = Act<F16>::mfma(x1, wb1, ab);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                tot[m].a[r] = __builtin_fmaf(sa, aa[r], tot[m].a[r]);
-                tot[m].b[r] = __builtin_fmaf(sb, ab[r], tot[m].b[r]);
+                t[at + r] = __builtin_fmaf(sa, aa[r], t[at + r]);
+                t[at + 4 + r] = __builtin_fmaf(sb, ab[r], t[at + 4 + r]);
+                if (!kShared) t[at + r] = __builtin_fmaf(ta, sx[r], t[at + r]), t[at + 4 + r] = __builtin_fmaf(tb, sx[r], t[at + 4 + r]);
+            }
+            if (kShared && (m & 1) == 0 && m + 1 < NM) continue;
+            // four outer products of 16 sums by 16 biases, lane (j, jq) has both for block jq: t + bias * sum, rounded once as by an fma
+            if (kShared) {
+                const float both = sums[((slot * NM + (m & ~1)) * CHUNK + gl) * 16 + (m & 1 ? (lane >> 5) * (CHUNK * 16) : 0) + j];
+                t = __builtin_amdgcn_mfma_f32_16x16x1f32(both, bias, t, 0, 0, 0);
             }
             // pinned: left alone, the compiler collects the scales' arithmetic of several groups and carries all
             // their matrix results there, which does not fit the register budget
-#pragma unroll
-            for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(tot[m].a[r]), "+v"(tot[m].b[r]));
+            asm volatile("" : "+v"(t));
         }
     };
 
@@ -1159,21 +1165,24 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     store_a(0);
     load_a(min(1u, n_chunks - 1));
     lds_barrier();
+    if constexpr (kShared) {
+        sum_up(0, 0);
+        lds_barrier();
+    }
     // chunk c from LDS buffer c % 2; chunk c + 1 goes from registers into the other one, chunk c + 2 into the registers.
-    // One barrier per chunk: the stores of chunk c + 1 in front of their reads, the reads of chunk c in front of the stores of
-    // chunk c + 2 into the same buffer.
+    // Two barriers per chunk (one where no sums are shared). In its middle: the stores of chunk c + 1 in front of its sums; at its end: the sums and stores in
+    // front of their reads, the reads of chunk c in front of the stores of chunk c + 2 into the same buffer.
     auto chunk = [&](uint32_t c, auto parity, auto whole) __attribute__((always_inline)) {
-        constexpr int kFirst = decltype(parity)::value * CHUNK;
-        const uint32_t buf = c & 1;
-        store_a(buf ^ 1);               // (past the last chunk: a buffer nobody reads)
+        constexpr int kParity = decltype(parity)::value;
+        store_a(kParity ^ 1);           // (past the last chunk: a buffer nobody reads)
         load_a(min(c + 2, n_chunks - 1));
-        sum_up(buf, c >> 1, kFirst);    // (of a group past the last: not used)
 #pragma unroll
         for (int gl = 0; gl < CHUNK; ++gl) {
             const uint32_t grp = c * CHUNK + gl;
-            if (decltype(whole)::value || grp < n_groups) step(buf, gl, (kFirst + gl) % kStreamDepth, grp + kStreamDepth);
+            if (decltype(whole)::value || grp < n_groups) step(kParity, kParity, gl, (kParity * CHUNK + gl) % kStreamDepth, grp + kStreamDepth);
+            if (kShared || gl == CHUNK - 1) lds_barrier();
+            if (kShared && gl == 0) sum_up(kParity ^ 1, kParity ^ 1);      // (of a group past the last: not used)
         }
-        lds_barrier();
     };
     using Even = std::integral_constant<int, 0>;
     using Odd = std::integral_constant<int, 1>;
@@ -1183,13 +1192,9 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     for (; (c + 2) * CHUNK <= n_groups; c += 2) {
         chunk(c, Even{}, Whole{});
         chunk(c + 1, Odd{}, Whole{});
-        add_bias(c >> 1, Whole{});
     }
-    if (c < n_chunks) {
-        chunk(c, Even{}, Part{});
-        if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
-        add_bias(c >> 1, Part{});
-    }
+    if (c < n_chunks) chunk(c, Even{}, Part{});
+    if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
 
     // lane (j, jq) holds, per stream, weight row j of the tile row for pairs 4 jq .. 4 jq + 3 of every 16-pair block. The
     // last chunk ended with a barrier: the LDS is free.
@@ -1199,7 +1204,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
 #pragma unroll
         for (int m = 0; m < NM; ++m)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) h[m][r] = gelu_tanh_fast(tot[m].a[r]) * tot[m].b[r];
+            for (int r = 0; r < 4; ++r) h[m][r] = gelu_tanh_fast(tot[m / 2][8 * (m & 1) + r]) * tot[m / 2][8 * (m & 1) + 4 + r];
         if constexpr (F16) {
             // the block scale of a pair's 64 activations, as in gemm_wave's epilogue: sixteen lanes hold a quarter of them
             float *peaks = reinterpret_cast<float *>(lds + NM * 2 * kWave);             // [wave][pair]
@@ -1248,7 +1253,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t pair = 16 * m + 4 * jq + r;
-            float va = tot[m].a[r], vb = tot[m].b[r];
+            float va = tot[m / 2][8 * (m & 1) + r], vb = tot[m / 2][8 * (m & 1) + 4 + r];
             if constexpr (F16) {
                 const float largest = act_scale[(size_t)gw.act_blocks * g.gf * 16 + (gw.act_block0 + m) * 16 + 4 * jq + r];
                 va *= largest;
@@ -1282,8 +1287,7 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_
                                                                     const uint16_t *__restrict__ a, uint32_t a_stride,
                                                                     uint16_t *__restrict__ out, uint32_t n_nblocks, bool nb_major,
                                                                     float *__restrict__ act_scale, uint32_t act_blocks) {
-    __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave + 2 * MAX_NM * kWave / 4];
-    static_assert(16 * MAX_NM * kStreamStageRow <= sizeof(lds), "the down epilogue's rows fit");
+    __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave + 2 * MAX_NM * kStreamChunk * 16 / 4];
     uint32_t ti, nb;
     if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;
     GemmWave gw;

@@ -66,6 +66,61 @@ def test_tile_edges_against_the_oracle(oracle, act, d, f, scale):
         ctx.close()
 
 
+def _exact_part(oracle, rows, cols, one_hot):
+    """4-bit weights, scale 1 and bias 0, with q = 1 at column one_hot[row] and 0 elsewhere."""
+    q = np.zeros((rows, cols), np.uint8)
+    q[np.arange(rows), one_hot] = 1
+    unit = oracle.bf16_bits(np.ones((rows, cols // 64), np.float32))
+    return (q[:, ::2] | q[:, 1::2] << 4), unit, np.zeros_like(unit)
+
+
+# one, two and (wide layers, tiles of 64 pairs) up to four 16-pair blocks per tile
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,counts", [(256, 64, (9, 20, 32, 33)), (320, 128, (16, 17, 28, 1)), (1024, 704, 3 * (9, 20, 33, 40, 48, 49, 60, 16))])
+@pytest.mark.parametrize("small", [0, 1, 3])
+def test_a_small_group_beside_large_ones(oracle, act, d, f, counts, small):
+    """One group of the up projection adds an odd whole number v, every other one nothing: q = 0 and bias 0 under scales of 2^7 and
+    inputs of 8. There a bf16 sum is v + 2^23 for a moment (128 * 2^7 * 512), whole numbers that fp32 holds - not so v + 2^24,
+    which two such groups at once would make. gate = 16 = gelu(16), down picks one activation per column: the rows are 16 v exactly."""
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    e, t, rng = len(counts), sum(counts), np.random.default_rng(d + small)
+    assert 0 < t <= 48 * e
+    cols = 64 * small + np.arange(1, 17)
+    parts, v_of = [], []
+    for _ in range(e):
+        gate = _exact_part(oracle, f, d, np.full(f, 64 * small))
+        gate[1][:] = oracle.bf16_bits(np.float32([16.0]))[0]
+        q = np.zeros((f, d), np.uint8)
+        q[:, cols] = rng.integers(0, 16, (f, 16))
+        q[:, 64 * small] = 1 - q[:, cols].sum(1) % 2 + 14 * (rng.random(f) < 0.5)                       # makes the sum odd
+        scale = np.full((f, d // 64), 128.0, np.float32)
+        scale[:, small] = 1.0
+        up = (q[:, ::2] | q[:, 1::2] << 4), oracle.bf16_bits(scale), np.zeros((f, d // 64), np.uint16)
+        parts.append((gate, up, _exact_part(oracle, d, f, np.arange(d) % f)))
+        v_of.append(q[:, 64 * small:64 * small + 17].astype(np.int64))
+    idx = _routes(rng, counts, e)
+    x = np.full((t, d), 8.0, np.float32)
+    x[:, 64 * small:64 * small + 64] = 0
+    x[:, 64 * small] = 1                                    # column 0 of the group: every row's
+    pick = 2 * rng.integers(0, 2, (t, 16))                  # the others: 0 or 2, so that v stays odd where q of column 0 is
+    x[:, cols] = pick
+    ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        pool = oracle.pool_from_parts(parts, d, f, 1, None)
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        y = ctx.prefill(0, torch.from_numpy(x).to(dt).cuda(), torch.from_numpy(idx.view(np.int32)).cuda(), torch.ones((t, 1), dtype=dt).cuda())
+        row_x = np.concatenate([np.ones((t, 1), np.int64), pick], 1)
+        v = np.einsum("tk,tfk->tf", row_x, np.stack([v_of[i] for i in idx[:, 0]]))
+        # (a whole number of more than 8 significant bits is rounded once, as the activation)
+        want = torch.from_numpy(16.0 * v).to(torch.float32).to(dt).double().numpy()[:, np.arange(d) % f]
+        assert np.array_equal(y.double().cpu().numpy(), want)
+    finally:
+        ctx.close()
+
+
 # 1 to 5 groups of K in each product: a quad of groups short of three, two, one and none, and one group past it
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,f", [(64, 128), (192, 64), (256, 192), (320, 256), (128, 320)])
