@@ -1478,7 +1478,11 @@ uint32_t gemm_tile_rows(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g
     // 241 | 238 (275 | 272), 2,000 (125) 261 | 260 (289 | 299); Zipf of exponent 1.1, 1,000 rows 217 | 191 (236 | 216), 1,700 273 | 253 (305 |
     // 283), 3,072 (192) 377 | 386; 64 experts of 2,048 x 1,408, 94 pairs 152 | 140 (177 | 164), 112 171 | 165 (197 | 192), 141 188 | 210;
     // 256 of 512 x 256, 47 pairs 53 | 49 (62 | 58), Zipf 63 | 55 (73 | 64).
-    if (n_items / (float)kBM * nb_gu > cus || n_experts * nb_gu > cus) return mean + 1.5f * dev <= 128 ? (most < 128 ? most : 128) : most;
+    if (n_items / (float)kBM * nb_gu > cus || n_experts * nb_gu > cus) {
+        // (`most` and 256 fit every scratch, 128 where its tiles, one more than the whole ones per expert, do)
+        const bool halves = mean + 1.5f * dev <= 128 && n_items / 128 + n_experts < max_tiles;
+        return halves && most > 128 ? 128 : most;
+    }
     uint32_t best = most;
     float least = 0.0f;
     for (uint32_t rows = most; rows >= 32; rows -= 16) {

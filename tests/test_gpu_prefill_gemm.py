@@ -75,8 +75,8 @@ def test_tiles_by_the_number_of_items(oracle, act, d, f, counts):
     test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts)
 
 
-# Chunks that fill the chip in tiles of at most 128 pairs, two blocks per compute unit: the edges of 16-pair blocks and of one and two
-# tiles, tall and flat layers, a last N-block that is half full. The same rows three times over take tiles of 256: the same bits.
+# Chunks of more than one round in tiles of 96 and 112 pairs, two blocks per compute unit: the edges of 16-pair blocks, experts that such a
+# tile does not hold, tall and flat layers, a last N-block that is half full. The same rows three times over take larger tiles: the same bits.
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,f,counts", [(192, 704, 8 * (1, 16, 47, 64, 127, 128, 129, 0)), (64, 640, 8 * (17, 33, 80, 81, 96, 112, 113, 0)),
                                         (512, 704, 7 * (31, 65, 48, 97, 95, 100, 63) + (257, 15))])
@@ -103,6 +103,17 @@ def test_tiles_of_half_the_pairs(oracle, act, d, f, counts):
         assert all(torch.equal(tall[k * t:(k + 1) * t], y) for k in range(3))
     finally:
         ctx.close()
+
+
+# Layers of more than two rounds of items (576 or 640 gate/up N-blocks for 256 units), where a chunk of up to some 112 pairs per expert is cut
+# at 128: one pair around a 16-pair block, around one tile and two; every expert one pair past a tile, as many tiles as there can be.
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,f,counts", [(128, 704, 12 * (112, 113, 127, 128, 129, 96, 60, 81)), (64, 640, 16 * (257, 112, 113, 128, 127, 129, 1, 17)),
+                                        (64, 704, 48 * (129, 81))])
+def test_tiles_of_128_pairs_where_the_chip_is_full(oracle, act, d, f, counts):
+    e, t = len(counts), sum(counts)
+    assert e * ((f // 16 + 7) // 8) > 2 * 256 and 48 * e < t and t / e + 1.5 * (t / e) ** 0.5 <= 128
+    test_tiles_and_rings_against_the_oracle(oracle, act, d, f, counts)
 
 
 @pytest.mark.parametrize("act,stride", [("bf16", 1 << 24), ("bf16", 1 << 25), ("fp16", 1 << 25), ("bf16", 360_000_000), ("fp16", 360_000_000)])
