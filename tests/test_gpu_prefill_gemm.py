@@ -145,6 +145,41 @@ def test_rows_that_span_four_gigabytes(oracle, act, stride):
         torch.cuda.empty_cache()
 
 
+# Rows 8 and 4 MiB apart, 5 to 7.4 GB in all, of nine experts with 288 gate/up N-blocks: about 67 pairs per expert in tiles of 112, about 98 in
+# tiles of 128 (with 113, 127, 128 and more), about 150 in tiles of 208.
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("counts,stride", [((112, 97, 80, 64, 48, 33, 100, 40, 26), 1 << 22), ((128, 113, 127, 112, 129, 80, 97, 64, 33), 1 << 22),
+                                           ((208, 193, 177, 145, 129, 209, 113, 96, 80), 1 << 21)])
+def test_far_rows_in_tiles_of_every_height(oracle, act, counts, stride):
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, e, t = 128, 4096, len(counts), sum(counts)
+    assert t * stride * 2 > 1 << 32 and t > 48 * e and e * f // 128 > 256
+    if torch.cuda.mem_get_info()[0] < t * stride * 2 + (4 << 30):
+        pytest.skip("the card's free memory does not hold the rows")
+    rng, pool, _ = make_layer(oracle, 13, d, f, e, align=1)
+    idx = np.repeat(np.arange(e, dtype=np.uint32), counts)
+    rng.shuffle(idx)
+    ctx = ff.Context(d, f, e, 1, n_layers=1, max_tokens=t, act_dtype=act)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(dt)
+        w = torch.from_numpy(rng.uniform(0.2, 1.0, (t, 1)).astype(np.float32)).to(dt)
+        gx, gi, gw = x.cuda(), torch.from_numpy(idx[:, None].view(np.int32)).cuda(), w.cuda()
+        far = torch.empty(((t - 1) * stride + d,), dtype=dt, device="cuda").as_strided((t, d), (stride, 1))
+        far.copy_(gx)
+        near = ctx.prefill(0, gx, gi, gw)
+        _check(oracle, pool, e, idx[:, None], x, w, near.float().cpu().numpy(), act)
+        ctx.prefill(0, -gx, gi, gw)                             # (nothing of the rows stays in the scratch)
+        assert torch.equal(ctx.prefill(0, far, gi, gw, out=torch.full_like(near, float("nan"))), near)
+    finally:
+        ctx.close()
+        far = None
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,f,rows", [(704, 1408, (897, 1025, 1500, 1601, 2049, 2300, 2800, 3000, 3600, 4000, 4400, 5000)),
                                       (1408, 1408, (913, 1700, 4801, 5000, 5600))])
