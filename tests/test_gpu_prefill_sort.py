@@ -1,6 +1,6 @@
-"""The prefill's sort of routes in one launch and (past 20,480 to 65,536 items) in three: the same rows, bit for bit, from a chunk and from its
+"""The prefill's sort of routes in one launch (up to 20,480 to 65,536 items) and in three: the same rows, bit for bit, from a chunk and from its
 beginning, on one side of the line and on either, and from lists of pairs, counts per expert, routes of weight zero and experts past the last left
-out. What a call does not write is NaN. (The order of an expert's pairs shows in no result.) Needs a GPU: pytest -m gpu."""
+out (on either side of the line). What a call does not write is NaN. (The order of an expert's pairs shows in no result.) Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("e,k,cuts", [(128, 8, (1, 7, 8, 9, 128, 129, 383, 384)), (256, 2, (31, 32, 33, 511, 512, 513, 1535, 1536)),
                                       (3, 1, (3000, 3071, 3072)), (5, 3, (1024,)), (200, 4, (255, 256, 257, 768))])
-def test_one_launch_sorts_as_three_do(oracle, e, k, cuts):
+def test_chunks_and_their_beginnings(oracle, e, k, cuts):
     import torch
     import fieldfare_moe as ff
     ff.lib()
@@ -128,6 +128,55 @@ def test_one_launch_at_its_line(oracle, e, k, line, cuts):
         ctx.close()
 
 
+@pytest.mark.parametrize("e,k,line", [(24, 2, 20480), (33, 3, 24576), (250, 8, 65536)])
+def test_lists_and_lost_routes_past_the_line(oracle, e, k, line):
+    """What the three launches leave out and what they take: a list in any order, the same in order, its first part in one launch; a table
+    with experts past the last against the same with weight zero."""
+    import torch
+    import fieldfare_moe as ff
+    ff.lib()
+    d, f, t = 64, 64, line // k + 3
+    rng, pool, _ = make_layer(oracle, 15 + e, d, f, e, align=1)
+    idx = np.argsort(rng.random((t, e)), axis=1)[:, :k].astype(np.int64)
+    token, rank = (v.reshape(-1) for v in np.divmod(rng.permutation(t * k), k))
+    lists = np.stack([token, idx[token, rank], rank, np.zeros_like(token)], 1).astype(np.int32)
+    lost = rng.random(t * k) < 0.05
+    lists[np.flatnonzero(lost), rng.integers(0, 3, lost.sum())] += 1 << 20          # each a token, an expert or a rank past the last
+    in_order = lists[np.argsort(lists[:, 1], kind="stable")]
+    ctx = ff.Context(d, f, e, k, n_layers=1, max_tokens=t)
+    try:
+        ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+        x = torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).to(torch.bfloat16).cuda()
+
+        def rows(pairs, kept):
+            out = torch.full((t * k, d), float("nan"), dtype=x.dtype, device="cuda")
+            ctx.prefill_pairs(0, x, torch.from_numpy(pairs.copy()).cuda(), t, out)
+            n_pairs, _, counts = ctx.prefill_stats()
+            assert n_pairs == kept.sum() and np.array_equal(counts, np.bincount(lists[:len(kept)][kept, 1], minlength=e))
+            return out.view(torch.int16)
+
+        assert t * k > line
+        three, sorted_three, one = rows(lists, ~lost), rows(in_order, ~lost), rows(lists[:line], ~lost[:line])
+        assert torch.equal(three, sorted_three)                 # NaN where nothing is written, on both
+        place = torch.from_numpy(token * k + rank).cuda()
+        written = torch.isfinite(three.view(x.dtype)[place]).all(1).cpu().numpy()
+        assert np.array_equal(written, ~lost)
+        assert torch.equal(one[place[:line]], three[place[:line]]) and torch.isnan(one.view(x.dtype)[place[line:]]).all()
+
+        gone = rng.random((t, k)) < 0.2
+        past = torch.from_numpy(np.where(gone, e + rng.integers(0, 1 << 20, (t, k)), idx).astype(np.int32)).cuda()
+        plain, w = torch.from_numpy(idx.astype(np.int32)).cuda(), torch.from_numpy(rng.uniform(0.2, 1.0, (t, k)).astype(np.float32)).to(x.dtype)
+        less, w = w.masked_fill(torch.from_numpy(gone), 0).cuda(), w.cuda()
+        for n in (t, line // k):                                # three launches, one
+            ctx.prefill(0, torch.full_like(x, float("nan")), plain, torch.ones_like(w))
+            got = ctx.prefill(0, x[:n], past[:n].contiguous(), w[:n].contiguous(), out=torch.full_like(x[:n], float("nan")))
+            n_pairs, _, counts = ctx.prefill_stats()
+            assert n_pairs == (~gone[:n]).sum() and np.array_equal(counts, np.bincount(idx[:n][~gone[:n]], minlength=e)), n
+            assert torch.isfinite(got.float()).all() and torch.equal(got, ctx.prefill(0, x[:n], plain[:n].contiguous(), less[:n].contiguous())), n
+    finally:
+        ctx.close()
+
+
 # 256 threads (2,048 pairs and fewer) and 1,024, runs of 64 pairs that end in one expert, in several and in pairs that are left out
 @pytest.mark.parametrize("e,k,n", [(128, 8, 8000), (128, 8, 2048), (3, 2, 2049), (200, 1, 130), (7, 4, 63), (1, 1, 700)])
 def test_lists_sorted_by_expert(oracle, e, k, n):
@@ -140,7 +189,7 @@ def test_lists_sorted_by_expert(oracle, e, k, n):
     token, rank = (v.reshape(-1) for v in np.divmod(rng.permutation(t * k)[:n], k))
     lists = np.stack([token, idx[token, rank], rank, np.zeros_like(token)], 1).astype(np.int32)
     out_of_range = rng.random(n) < 0.05
-    lists[out_of_range, rng.integers(0, 3)] += 1 << 20          # a token, an expert or a rank past the last
+    lists[np.flatnonzero(out_of_range), rng.integers(0, 3, out_of_range.sum())] += 1 << 20          # each a token, an expert or a rank past the last
     in_order = lists[np.argsort(lists[:, 1], kind="stable")]
     ctx = ff.Context(d, f, e, k, n_layers=1, max_tokens=t)
     try:
