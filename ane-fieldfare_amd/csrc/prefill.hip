@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
                 token[u] = p.token, e[u] = p.expert, rank[u] = p.rank;
             }
 #pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u) e[u] = (token[u] < src.t) & (rank[u] < src.top_k) ? e[u] : 0xFFFFFFFFu;
+            for (uint32_t u = 0; u < kAhead; ++u) e[u] = ((token[u] < src.t) & (rank[u] < src.top_k)) ? e[u] : 0xFFFFFFFFu;
         } else {
             // zero-weight routes are dropped, as the reference's prefill does (RealForwardRunner.swift:1528-1530)
             uint16_t w[kAhead];
