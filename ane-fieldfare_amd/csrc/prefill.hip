@@ -255,7 +255,16 @@ __device__ __forceinline__ void place_item(const ItemSource &src, uint32_t i, ui
 // longer, 24,576 items 33.3 | 25.7, 65,536 items 57 | 47; top-1 of 32, 16,000 items 23.5 | 20.9, 24,576 items 25.4 | 25.9. Without the
 // shared start (blocks that begin at items of their own): the same.
 constexpr int kSortRuns = 64;                               // items of a lane: a bit each
-static uint32_t sort_one_launch(uint32_t n_experts) { return n_experts > 128 ? kSortRuns * kScanThreads : n_experts > 32 ? 24576u : 20480u; }
+// Up to how many items one launch sorts: where it crosses the three, later with skewed tables (whose lanes meet at the three launches'
+// counters too) than with uniform ones, earlier with lists in order (which cost the three few turns). Three | one, us: lists, top-1 of 4
+// 20,000 pairs 23.7 | 22.6, top-2 of 16 16,000 19.8 | 19.4, 18,000 20.1 | 21.5, top-4 of 48 18,000 18.9 | 20.4, top-8 of 128 18,000 20.2 | 20.8,
+// 24,500 20.9 | 22.0; tables, uniform (Zipf), top-2 of 24 18,000 23.0 | 23.1 (25.9 | 24.9), 20,000 23.4 | 23.9 (26.3 | 26.1), top-4 of 48
+// 20,000 23.2 | 23.8 (25.3 | 25.2), 24,500 23.9 | 25.8 (26.4 | 27.4), top-8 of 128 24,500 25.9 | 25.5 (27.0 | 27.1).
+static uint32_t sort_one_launch(const ItemSource &src) {
+    if (src.n_experts > 128) return kSortRuns * kScanThreads;
+    if (src.pairs) return src.n_experts > 4 ? 16384u : 20480u;
+    return src.n_experts > 64 ? 24576u : 20480u;
+}
 // (256 threads up to 2,048 items: fewer waves to meet)
 static uint32_t sort_threads(uint32_t n_items) { return n_items <= 2048 ? 256 : kScanThreads; }
 __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource src, PrefillPlan *__restrict__ plan,
@@ -1634,7 +1643,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
         hipLaunchKernelGGL(prefill_dense_plan_kernel, dim3(n_blocks), dim3(kSortBlock), 0, s, t, tile_rows, sc.plan, sc.tiles, sc.sorted_token,
                            sc.sorted_out_row);
     } else {
-        if (src.n_items <= sort_one_launch(n_experts)) {
+        if (src.n_items <= sort_one_launch(src)) {
             hipLaunchKernelGGL(prefill_sort_kernel, dim3(n_experts), dim3(sort_threads(src.n_items)), 0, s, src, sc.plan, sc.tiles, sc.max_tiles,
                                TileRows(tile_rows), sc.sorted_token, sc.sorted_out_row);
         } else {

@@ -1,4 +1,4 @@
-"""The prefill's sort of routes in one launch (up to 20,480 to 65,536 items) and in three: the same rows, bit for bit, from a chunk and from its
+"""The prefill's sort of routes in one launch (up to 16,384 to 65,536 items) and in three: the same rows, bit for bit, from a chunk and from its
 beginning, on one side of the line and on either, and from lists of pairs, counts per expert, routes of weight zero and experts past the last left
 out (on either side of the line). What a call does not write is NaN. (The order of an expert's pairs shows in no result.) Needs a GPU: pytest -m gpu."""
 import numpy as np
@@ -90,9 +90,9 @@ def test_reduce_of_rows_by_pieces_and_by_elements(oracle, act, t, k, d, skip):
         ctx.close()
 
 
-# the last item count of one launch and the first of three (20,480, 24,576 and 65,536 items with up to 32, 128 and 256 experts), runs of 64
-# items per wave that end inside a group of eight loads, and the few items that 256 threads sort (2,048)
-@pytest.mark.parametrize("e,k,line,cuts", [(24, 2, 20480, (1023, 1025, 4500, 10240)), (33, 3, 24576, (682, 683, 2731, 8192)), (250, 8, 65536, (255, 257, 4097, 8192))])
+# the last item count of one launch and the first of three (20,480 items with up to 64 experts, 24,576 with up to 128 and 65,536 beyond)
+# and past it, runs of 64 items per wave that end inside a group of eight loads, and the few items that 256 threads sort (2,048)
+@pytest.mark.parametrize("e,k,line,cuts", [(64, 4, 20480, (682, 683, 5120)), (65, 3, 24576, (8191, 8192)), (128, 1, 24576, (2047, 2049, 24576)), (24, 2, 20480, (1023, 1025, 4500, 10240)), (33, 3, 24576, (682, 683, 2731, 8192)), (250, 8, 65536, (255, 257, 4097, 8192))])
 def test_one_launch_at_its_line(oracle, e, k, line, cuts):
     import torch
     import fieldfare_moe as ff
@@ -119,7 +119,7 @@ def test_one_launch_at_its_line(oracle, e, k, line, cuts):
 
         whole = rows(t)                                         # three launches
         assert torch.isfinite(whole.float()).all() and whole.abs().max() > 0
-        assert torch.equal(rows(line // k), whole[:line // k])  # one launch, the same products
+        assert torch.equal(rows(line // k), whole[:line // k])  # one launch where the line is this table's, the same products
         for n in cuts:                                          # (in the streaming product's range to its own bits: rounded weights elsewhere)
             part = rows(n)
             close = (part.float() - whole[:n].float()).abs() <= 2.0 ** -6 * whole[:n].float().abs() + 2.0 ** -6 * whole.float().abs().max()
@@ -128,7 +128,8 @@ def test_one_launch_at_its_line(oracle, e, k, line, cuts):
         ctx.close()
 
 
-@pytest.mark.parametrize("e,k,line", [(24, 2, 20480), (33, 3, 24576), (250, 8, 65536)])
+# (lists: one launch up to 20,480 pairs with up to four experts, 16,384 with up to 128, 65,536 beyond)
+@pytest.mark.parametrize("e,k,line", [(4, 2, 20480), (5, 2, 16384), (128, 3, 16384), (24, 2, 20480), (33, 3, 24576), (250, 8, 65536)])
 def test_lists_and_lost_routes_past_the_line(oracle, e, k, line):
     """What the three launches leave out and what they take: a list in any order, the same in order, its first part in one launch; a table
     with experts past the last against the same with weight zero."""
