@@ -22,8 +22,10 @@ namespace {
 // 12.6 | 7.6, 64 rows 13.0 | 10.7, 80 rows 12.9 | 11.8, 100 rows 12.9 | 13.4, 160 rows 13.0 | 17.2; 2,048 x 128, 64 rows 11.5 |
 // 10.5, 80 rows 11.4 | 11.6; 1,024 x 64, 80 rows 8.7 | 8.7; 256 x 128, 48 rows 8.9 | 9.2; 512 x 16, 160 rows
 // 7.6 | 7.1; FP16, 2,816 x 128, 100 rows 14.7 | 13.5, 130 rows 14.8 | 15.6; 2,048 x 128, 80 rows 12.9 | 11.7. Same
-// pinned sums: same routes bit for bit.
+// pinned sums: same routes bit for bit. Neither pass is shorter than its launch: narrow tables' two took 9.0 us (FP16 9.7) where the
+// above says 7: 32 x 512, 128 rows 9.0 | 8.7, 160 rows 9.1 | 9.3 (FP16 9.8 | 9.2); 16 x 256, 160 rows 9.0 | 8.1.
 bool router_small_rows(uint32_t t, uint32_t n_experts, uint32_t d, bool f16) {      // (in units of 20 ps)
+    if (t <= 160 && n_experts * t <= (f16 ? 5120u : 4096u)) return true;
     return t <= 160 && 29u * n_experts * t <= (f16 ? 65000u : 35000u) + 625u * n_experts + (f16 ? 105u : 88u) * d;
 }
 

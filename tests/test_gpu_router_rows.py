@@ -1,5 +1,6 @@
 """Router routes of a short prompt either side of the row count from which the prefill router runs in two passes (160, less
-where many experts meet few columns: in bf16 after 73 at 256 x 128 and 150 at 2,048 x 128): the same routes and weights,
+where many experts meet few columns: after 37 at 256 x 128 and 79 at 2,048 x 128, in FP16 46 and 96; narrow tables after 4,096 rows x
+experts, in FP16 5,120): the same routes and weights,
 bit for bit, as the pinned sums of all logits. Needs a GPU: pytest -m gpu."""
 import numpy as np
 import pytest
@@ -11,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,e,t", [(2816, 128, 17), (2816, 128, 160), (2816, 128, 161), (1024, 16, 160), (4096, 128, 163),
-                                   (256, 128, 73), (256, 128, 74), (256, 128, 78), (2048, 128, 150), (2048, 128, 151)])
+                                   (256, 128, 73), (256, 128, 74), (256, 128, 78), (2048, 128, 150), (2048, 128, 151),
+                                   (256, 128, 37), (256, 128, 38), (256, 128, 46), (256, 128, 47), (2048, 128, 79), (2048, 128, 80), (2048, 128, 96), (2048, 128, 97), (512, 32, 128), (512, 32, 129), (512, 32, 160), (512, 32, 161), (256, 16, 160)])
 def test_routes_either_side_of_the_two_pass_line(oracle, act, d, e, t):
     import torch
     import fieldfare_moe as ff
