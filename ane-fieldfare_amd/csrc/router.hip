@@ -404,8 +404,8 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
                                                                    uint32_t *__restrict__ out_idx, uint16_t *__restrict__ out_w) {
     static_assert(4 % PARTS == 0, "a block of four waves");
     __shared__ uint32_t keys[PARTS == 1 ? 1 : 4][PARTS == 1 ? 1 : 128];
-    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t part = wave % PARTS, my_tok = blockIdx.x * (4 / PARTS) + wave / PARTS, tok = min(my_tok, t - 1);
+    const uint32_t lane = threadIdx.x & 63, wave = PARTS == 1 ? threadIdx.x >> 6 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t part = wave % PARTS, my_tok = blockIdx.x * (4 / PARTS) + wave / PARTS, tok = PARTS == 1 ? my_tok : min(my_tok, t - 1);
     if (PARTS == 1 && my_tok >= t) return;  // (else past the last: the last again, not stored, for the barrier)
     // the token's row, as the pinned order walks it: element j of (step i, sub-accumulator s) = x[1024 i + 256 s + 4 lane + j]
     const uint16_t *xr = x + (size_t)tok * x_stride;
