@@ -1554,7 +1554,8 @@ TileForm prefill_tile_form(uint32_t n_items, uint32_t n_experts, const ArenaGeom
 // about 1,000 cycles per group of an item and the time of some six groups around them; the lists' last N-blocks are counted as
 // full ones. 2,816 -> 2,112 -> 2,816, us of the call at 256 rows per tile | the rule's: 102 | 62 at 897 rows (n = 4), 104 | 82 at
 // 2,048 (9), 112 | 103 at 3,072 (13), 170 | 147 at 4,096 (12), 292 | 259 at 8,192 (13); FP16 inputs now 81, 105, 132,
-// 179 and 311. Of n = 6..16 each, the rule's is the fastest at these sizes or within 3% of it.
+// 179 and 311. Of n = 6..16 each, the rule's was the fastest at these sizes or within 3% of it. (All with one block per unit; up to 128 rows
+// two of them run beside each other now: at 897 rows 52, FP16 66.)
 uint32_t dense_tile_rows(uint32_t t, const ArenaGeom &g, uint32_t n_cus) {
     uint32_t best = kBM;
     uint64_t least = ~0ull;
@@ -1672,6 +1673,15 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     const uint32_t act_blocks = f16 ? sc.act_blocks : 0u;
     // (a row's address is 32 bits from the first row's where that reaches the last)
     const bool wide = (uint64_t)t * x_stride * 2 > 0xFFFFFFFFull;
+    // Tiles of up to 128 pairs run two blocks to a compute unit (GemmLds), also where a launch has no more items than units and every block
+    // is alone: the shorter start and end of an item are worth 1 to 8 % there. Not tiles of 112 pairs (FP16: 96 and 112) over 40 groups and
+    // more: alone, the longer rings and queues win. us of the call with two blocks | one, dense: 4,096 -> 1,408, FP16, 1,536 rows (96 each)
+    // 84.7 | 79.5, 2,048 rows (128) 91 | 95; 2,816 -> 2,816, FP16, 897 rows (96) 84.1 | 81.6, 1,200 rows (112) 92.5 | 89.5, bf16 77.4 | 75.9; 2,816 -> 704,
+    // FP16, 2,048 rows (96) 60.5 | 56.5; 2,048 -> 1,408, 1,536 rows (80) 44.3 | 45.2; 1,024 -> 512, 897 rows (64) 23.5 | 24.5, FP16 30.2 | 31.3. 8 experts
+    // of 4,096 x 1,536, 192 pairs each (112) 89.1 | 87.6, FP16 107.5 | 103.9, 96 pairs each (64), FP16, 78.5 | 80.1.
+    const auto two_blocks = [&](uint32_t groups, uint32_t n_nb) {
+        return tile_rows <= 128 && (groups < 40 || tile_cap * n_nb > n_cus || tile_rows <= (f16 ? 80u : 96u) || tile_rows == 128);
+    };
 #define FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, LC)                                                                             \
     hipLaunchKernelGGL((GU && wide ? (f16 ? prefill_gemm_kernel<GU, true, GU, LC> : prefill_gemm_kernel<GU, false, GU, LC>)   \
                                    : (f16 ? prefill_gemm_kernel<GU, true, false, LC> : prefill_gemm_kernel<GU, false, false, LC>)), \
@@ -1680,7 +1690,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
                        act_scale, act_blocks, nullptr)
 #define FFMOE_GEMM(GU, A, STRIDE, OUT, NB)                                                                                    \
     do {                                                                                                                      \
-        if (tile_rows <= 128) FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, 2);                                                       \
+        if (two_blocks(GU ? g.gd : g.gf, NB)) FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, 2);                                       \
         else FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, 4);                                                                        \
     } while (0)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \

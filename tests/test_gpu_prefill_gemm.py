@@ -182,10 +182,10 @@ def test_far_rows_in_tiles_of_every_height(oracle, act, counts, stride):
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 @pytest.mark.parametrize("d,f,rows", [(704, 1408, (897, 1025, 1500, 1601, 2049, 2300, 2800, 3000, 3600, 4000, 4400, 5000)),
-                                      (1408, 1408, (913, 1700, 4801, 5000, 5600))])
+                                      (1408, 1408, (913, 1700, 4801, 5000, 5600)), (2816, 704, (1200, 2048, 3000, 4096))])
 def test_dense_tiles_of_the_row_count(oracle, act, d, f, rows):
-    """A dense FFN's tiles have as many rows as fill the last round of blocks (64 to 256): the largest chunk against 64-bit products,
-    every other one, cut elsewhere, to the same bits."""
+    """A dense FFN's tiles have as many rows as fill the last round of blocks (64 to 256; over 2,560 columns and more, tiles of 96 and 112 rows run
+    a block per compute unit): the largest chunk against 64-bit products, every other one, cut elsewhere, to the same bits."""
     import torch
     import fieldfare_moe as ff
     ff.lib()
