@@ -397,7 +397,7 @@ uint32_t n_blocks_of(uint32_t stored_rows) { return (stored_rows / 16 + kTilesN 
 // 0.5 us now and the forms cross lower: library form | this one, us: 2,816 -> 2,112, 704 rows 76 | 56, 3,072 rows 248 | 140; 2,816 ->
 // 704, 1,024 rows 55 | 45; 1,024 -> 2,816, 1,024 rows 67 | 50. The line of narrow layers stays: a chunk keeps the form, and with it the
 // bits, that it had. Wide ones change at 385 rows, where the library's form takes a step up: 2,816 -> 2,112, 301 rows 47 | 48, 384 rows 50 | 49,
-// 400 rows 65 | 49, 448 rows 68 | 50, 639 rows 63 | 50 (FP16 alike; errors against 64 bits equal: 3.32e-3, FP16 4.16e-4), those from
+// 400 rows 65 | 49, 448 rows 68 | 50, 639 rows 63 | 50; 2,816 -> 1,600, 385 rows 50 | 45, 512 rows 53 | 46; 2,304 -> 1,792 46 | 42, 51 | 42; 2,048 -> 2,048 46 | 41, 49 | 42 (FP16 alike; errors against 64 bits equal: 3.32e-3, FP16 4.16e-4), those from
 // 2.8 * 10^6 weights of a projection at 560: 2,816 -> 1,024, 448 rows 40 | 41, 560 rows 45 | 42; 1,728 -> 1,664, 400 rows 37 | 38, 560 rows 44 | 38.
 // Narrower, 2,816 -> 704, 560 rows 38 | 40. Else not below 640 rows, where the forms met at the widest, nor beyond 1,024, where the narrowest (2,816 -> 256) still
 // crossed, but in a call that the library's own 41 us on the host bound.

@@ -690,11 +690,11 @@ def main():
             fl = 2.0 * 3 * D * FS * TPs
             shared[f"rows{TPs}"] = {"us": round(tp_ * 1e6, 1), "TFLOPs": round(fl / tp_ / 1e12, 1),
                                     "frac_mfma_peak": round(fl / tp_ / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4)}
-            # the 8-bit layer at many rows: a 16-bit matrix element cannot hold q * s + b of an 8-bit q; from 640 rows on the
-            # GEMMs multiply by the integers q and bring scale and bias in with the sums
+            # the 8-bit layer at many rows: a 16-bit matrix element cannot hold q * s + b of an 8-bit q; from 385 rows on (at
+            # this width) the GEMMs multiply by the integers q and bring scale and bias in with the sums
             tp8 = timed(lambda: int8_step(xps, yps), 24, warm=24)
             shared["int8"][f"rows{TPs}"] = {"us": round(tp8 * 1e6, 1),
-                                            "form": "GEMMs on integer weights" if TPs >= 640 else "below the integer GEMMs' row count",
+                                            "form": "GEMMs on integer weights" if TPs >= 385 else "below the integer GEMMs' row count",
                                             "TFLOPs": round(fl / tp8 / 1e12, 1)}
             del xps, yps
         extra["shared_expert"] = shared

@@ -1,4 +1,4 @@
-"""The 8-bit dense layer's GEMMs on integer operands (640 rows and more): ragged row tiles either side of the tile sizes, an
+"""The 8-bit dense layer's GEMMs on integer operands (640 rows and more, wide layers from 560 or 385 on): ragged row tiles either side of the tile sizes, an
 output width that fills half a block of columns, widths of an odd number of groups, both activation types, inputs with a large
 common part (so that the bias columns carry most of a sum), rows that overflow. Needs a GPU: pytest -m gpu."""
 import numpy as np
@@ -16,7 +16,7 @@ def _gelu(x):
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
 # K of one group to 44, output widths of a quarter of a 256-row block to eleven blocks
 @pytest.mark.parametrize("d,f,t", [(128, 64, 640), (192, 320, 641), (64, 704, 703), (192, 1472, 1088), (448, 192, 1089), (2816, 128, 1153),
-                                   (192, 2816, 1025), (2112, 2112, 1217)])
+                                   (192, 2816, 1025), (2112, 2112, 1217), (2816, 2112, 386), (2816, 2112, 543), (2816, 1024, 561)])
 def test_rows_against_float64(oracle, act, d, f, t):
     import torch
     import fieldfare_moe as ff
@@ -42,7 +42,8 @@ def test_rows_against_float64(oracle, act, d, f, t):
         assert np.all(np.abs(yf - ref) <= 1.1 * unit * (4 * spread + np.abs(ref)))
         assert cosine(yf, ref) > 0.99999 and rel_err(yf, ref) < (1e-2 if act == "bf16" else 1.5e-3)
         # a row does not depend on the rows beside it (both tile sizes sum in one order)
-        first = 1024 if t > 1024 else 640                    # from 1,024 rows on every width takes this form
+        # from 1,024 rows on every width takes this form, those here from 640 on, wide ones from 560 or 385 on
+        first = 1024 if t > 1024 else 640 if t >= 640 else 560 if d * f < 4000000 else 385
         part = ctx.dense_ffn(0, x[:first].cuda()).float().cpu().numpy()
         assert np.array_equal(part, yf[:first])
         # other rows are untouched by one that is not finite
@@ -90,7 +91,7 @@ def test_the_form_follows_the_activation_type(oracle):
         ctx.close()
 
 
-@pytest.mark.parametrize("d,f,line", [(2816, 128, 1024), (1024, 1984, 689), (128, 192, 640)])
+@pytest.mark.parametrize("d,f,line", [(2816, 128, 1024), (1024, 1984, 689), (128, 192, 640), (2816, 2112, 385), (2816, 1024, 560)])
 def test_the_line_to_the_library_form(oracle, d, f, line):
     # the row before and the row after the line that the widths draw, in a context for more rows and in one for the row before alone
     import torch
