@@ -1098,19 +1098,19 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         ring_t[u] = make_uint4(t.x, t.y, t.z, t.w);
         ring_s[u] = make_uint2(s.x, s.y);
     };
-    // the sums of two 16-pair blocks: stream a and stream b of each, as the bias product's result has them
+    // the sums of two 16-pair blocks (or of the one): stream a and stream b of each, as the bias product's result has them
+    constexpr bool kShared = NM > 1;
     constexpr int kPairs = (NM + 1) / 2;
-    f32x16 tot[kPairs];
+    float __attribute__((ext_vector_type(kShared ? 16 : 8))) tot[kPairs];
 #pragma unroll
     for (int i = 0; i < kPairs; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tot[i][r] = 0.0f;
+        for (int r = 0; r < (kShared ? 16 : 8); ++r) tot[i][r] = 0.0f;
 
     // The groups' input sums, a value per pair in LDS ([chunk % 2][16-pair block][group of the chunk][pair]): every wave makes its
     // share of a chunk's while the block is at the chunk before. (Of one 16-pair block every wave makes its own: two instructions
     // against a barrier, 37 rows of 128 experts 104.6 | 102.1 us.)
     float *const sums = reinterpret_cast<float *>(lds + 2 * kBuf);
-    constexpr bool kShared = NM > 1;
     constexpr int kSums = (NM + 1) / 2;                   // 16-pair blocks per wave, of one of the chunk's two groups
     static_assert(CHUNK == 2, "two waves per group of a chunk");
     auto sum_up = [&](uint32_t buf, int slot) __attribute__((always_inline)) {
@@ -1141,7 +1141,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         const float bias = jq & 1 ? tb : ta;
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-            f32x16 &t = tot[m / 2];
+            auto &t = tot[m / 2];
             const int at = 8 * (m & 1);
             const uint4 x0 = frag(buf, m, 2 * gl), x1 = frag(buf, m, 2 * gl + 1);
             f32x4 sx = zero;
@@ -1158,7 +1158,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
             }
             if (kShared && (m & 1) == 0 && m + 1 < NM) continue;
             // four outer products of 16 sums by 16 biases, lane (j, jq) has both for block jq: t + bias * sum, rounded once as by an fma
-            if (kShared) {
+            if constexpr (kShared) {
                 const float both = sums[((slot * NM + (m & ~1)) * CHUNK + gl) * 16 + (m & 1 ? (lane >> 5) * (CHUNK * 16) : 0) + j];
                 t = __builtin_amdgcn_mfma_f32_16x16x1f32(both, bias, t, 0, 0, 0);
             }
