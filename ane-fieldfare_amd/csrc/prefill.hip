@@ -1568,7 +1568,8 @@ uint32_t dense_tile_rows(uint32_t t, const ArenaGeom &g, uint32_t n_cus) {
     return best;
 }
 
-// The same for a dense FFN's chunk that no GEMV took (beyond 384 rows at the model's widths): tiles of 32 rows while the gate/up
+// The same for a dense FFN's chunk that no bands took (at the model's widths FP16 beyond 384 rows, bf16 at 561 to 654 and beyond 704, where
+// their rounds cost more; d or f beyond the bands' widths from 17 rows on): tiles of 32 rows while the gate/up
 // launch is one round (four blocks per compute unit on the XCD with the most N-blocks), or while a chunk's products are few
 // enough that it cost less than the GEMMs at 256 rows per tile did; at most kDenseTileStreamRows. With tiles of fewer rows the
 // GEMMs are now the faster ones from some 640 rows on (2,816 -> 2,112, 897 rows 62 us, FP16 81, where 896 streamed ones take 78

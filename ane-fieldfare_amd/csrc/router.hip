@@ -393,7 +393,9 @@ constexpr int kExactSteps = 4;          // d <= 4096: k = 1024 i + 256 s + 4 lan
 // block that share a token. A wave is a chain: its token's sums, the threshold, two or three round trips for the candidates' rows, their
 // sums, the select. While the tokens leave waves idle, PARTS of them do the first of it alike and a PARTS-th of the candidates each.
 // 2,816 x 128, us of the call at 1 | 2 | 4: 301 rows 20.3 | 17.5 | 16.0, 700 rows 21.4 | 19.4 | 17.1, 850 rows 21.1 | 19.7 | 21.0, 1,400
-// rows 24.8 | 22.4 | 25.7, 2,000 rows 25.3 | 28.7 | 30.6: four while three blocks per compute unit hold all, two while those do.
+// rows 24.8 | 22.4 | 25.7, 2,000 rows 25.3 | 28.7 | 30.6: four while three blocks per compute unit hold all, two while those do. (Three is what the registers of
+// 2,049 columns and more allow; narrower tables, which hold four and eight, take the same line and are the faster too, us at 1 | the line's: 512 x
+// 128, 700 rows 12.1 | 10.8, 1,400 rows 14.2 | 13.3; 1,024 x 64, 12.8 | 10.4, 14.0 | 13.2; 256 x 16, 11.0 | 9.6, 11.5 | 10.7; 4,096 x 128, 26.4 | 19.6, 30.5 | 28.1.)
 template <int STEPS, int CHUNK, int PARTS, bool F16>
 __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_t *__restrict__ w, const uint16_t *__restrict__ x,
                                                                    uint32_t x_stride, uint32_t t, uint32_t n_experts, uint32_t d,

@@ -31,7 +31,6 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// One wave: candidate e lives in lane e % 64, slot e / 64 (E <= 256). top_k rounds of a wave-wide
 // The wave's largest key: by its upper half, then by the lower one of those that have it.
 __device__ __forceinline__ unsigned long long wave_max_key(unsigned long long k) {
     const uint32_t hi = wave_max_u32((uint32_t)(k >> 32)), lo = wave_max_u32((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
@@ -43,6 +42,7 @@ __device__ __forceinline__ float wave_max_f32(float v) {
     return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
 }
 
+// One wave: candidate e lives in lane e % 64, slot e / 64 (E <= 256). top_k rounds of a wave-wide
 // argmax over the total order (score desc, index asc): the largest score by wave_max_u32, then the lowest
 // index that holds it by ballots, slot by slot. Scores <= -inf and NaN are never taken; empty rounds give
 // (index 0, -inf) and weight 0 (moe.metal:194-236). The weights: lane i takes exp(score_i - max) and the

@@ -433,8 +433,9 @@ int ffmoe_upload_expert_parts(ffmoe_ctx *ctx, uint32_t layer, uint32_t expert, c
 /* y[t] = down( bf16( gelu_tanh(gate x[t]) * (up x[t]) ) ) for every row, weight 1, no routing: the
  * shared expert. Needs a context created with n_experts = 1 and top_k = 1 (f = the shared width).
  * Rows <= 16 run the streaming kernels of ffmoe_verify; 17 to 384 rows (bf16: up to 896 where that is the faster) the
- * resident-matrix products on the expert's arena tiles in bands of input rows (when d and f fit that kernel:
- * <= FFMOE_MATRIX_MAX_N); more rows the grouped products of ffmoe_prefill (the reference switches from its per-token GEMV loop to batched GEMMs at 32 tokens). Replaces
+ * resident-matrix products on the expert's arena tiles in bands of input rows (when d and f fit that kernel,
+ * <= FFMOE_MATRIX_MAX_N, and no weight scale of the layer is 2^104 or more); more rows the grouped products of
+ * ffmoe_prefill (the reference switches from its per-token GEMV loop to batched GEMMs at 32 tokens). Replaces
  * SharedExpertInt4.encode (Kernels/MoE/SharedExpertInt4.swift:32-89, kernel shared_gate_up_act_int4,
  * Metal/MoE/moe.metal:548-570) and PrefillSharedExpert.encodeBlock
  * (Kernels/Prefill/MoE/PrefillSharedExpert.swift:94-137). Gate and up stay fp32 in front of the
@@ -490,8 +491,9 @@ int ffmoe_layer_tail_routed(ffmoe_ctx *ctx, void *stream, const uint16_t *route_
  * context with n_experts = 1 and top_k = 1, d and f multiples of 64 up to FFMOE_MATRIX_MAX_N. The layer is then kept as
  * a gated gate/up matrix and a down matrix of nibble planes (ffmoe_matrix_create_int8_glu / _int8) owned by the
  * context, and ffmoe_dense_ffn, ffmoe_route_verify_shared and ffmoe_layer_tail_routed_shared serve it like a 4-bit
- * layer: ffmoe_dense_ffn runs the two matrix products (beyond 16 rows in bands of input rows), or from 192 rows on (bf16: where bands are
- * not the faster; when the context's max_tokens reaches that) two dense GEMMs of rocBLAS on hi + lo rows of the weights, kept in the activation type for
+ * layer: ffmoe_dense_ffn runs the two matrix products (beyond 16 rows in bands of input rows), or from 192 rows on (bf16:
+ * where bands are not the faster or a weight scale is 2^104 or more; when the context's max_tokens reaches that) two dense
+ * GEMMs of rocBLAS on hi + lo rows of the weights, kept in the activation type for
  * that purpose (4 more bytes per weight; that form is not meant for stream capture: the library may allocate workspace
  * on its first call), or from 385 rows on (up to 1,024 at narrow widths; likewise) two GEMMs of its own on the integer
  * weights (2 more bytes per weight; these can be captured), with the same roundings (gate and up are rounded to 16 bits in front of the
