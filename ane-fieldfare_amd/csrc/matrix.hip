@@ -174,14 +174,19 @@ __device__ __forceinline__ SoftmaxAcc softmax_shuffle(const SoftmaxAcc &a, int m
 // leaves the softmax pair of the sums it finished in conf_part[row * gridDim.x + block].
 // PLANES8: the matrix is an 8-bit one stored as two nibble planes (above): a tile is 16 rows, an output the sum of its
 // two streams.
-template <bool Y_F32, bool F16, bool GREEDY = false, bool CONF = false, bool PLANES8 = false, int GLU = 0>
+// FEW (up to four input rows of the plain form): input row t is operand row 4 t, so that one of a lane's four sums is all there is to
+// keep up, and each operand lane loads its own bytes: the lanes of a row ask for the same ones, there is nothing to turn through LDS.
+// 1 row, us without | so: 16,384 x 1,408 6.7 | 5.9, 16,384 x 2,816 7.2 | 6.8, 262,144 x 2,816 76.5 | 74.9 (5.5 TB/s).
+template <bool Y_F32, bool F16, bool GREEDY = false, bool CONF = false, bool PLANES8 = false, int GLU = 0, bool FEW = false>
 __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__restrict__ tiles,
                                                              const uint8_t *__restrict__ scales, uint32_t m,
                                                              uint32_t n_groups, const uint16_t *__restrict__ x,
                                                              uint32_t x_stride, uint32_t rows, void *__restrict__ y_,
                                                              uint32_t y_stride, float2 *__restrict__ conf_part = nullptr,
                                                              float softcap = 0.0f) {
-    __shared__ float s_red[2][kKSplit][8][64];
+    constexpr int kSums = FEW ? 1 : 4;
+    __shared__ float s_red[2][kKSplit][2 * kSums][64];
+    static_assert(!FEW || !(GREEDY || PLANES8 || GLU), "few rows of the plain form");
     static_assert(!(PLANES8 && GREEDY), "the greedy choice is built for the 4-bit head only");
     static_assert((GLU == 1) ? PLANES8 : true, "tile pairs are the 8-bit planes' gated form");
     // GLU == 1: tiles 2 p and 2 p + 1 hold rows 16 p ... 16 p + 15 of a gate and of an up projection; a block takes whole
@@ -217,13 +222,17 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     // the input rows of this wave's K-slice: requested as 64-byte pieces (four lanes per row), then turned into the
     // operand layout - with 16 rows the operand layout itself would make every lane of every load a request of its own
     uint4 x0[kRing], x1[kRing];
-    load_token_rows(x, x_stride, rows, lane, KSlice{g0, ng, g_last}, x0, x1);
-    turn_token_rows(lane, x0, x1);
+    if constexpr (FEW) {
+        load_few_rows(x, x_stride, rows, lane, KSlice{g0, ng, g_last}, x0, x1);
+    } else {
+        load_token_rows(x, x_stride, rows, lane, KSlice{g0, ng, g_last}, x0, x1);
+        turn_token_rows(lane, x0, x1);
+    }
     // per group: the sum of its inputs per token column, once for all the tile rows this wave walks
     f32x4 sx[kRing];
 #pragma unroll
     for (int u = 0; u < kRing; ++u) sx[u] = group_input_sum<F16>(x0[u], x1[u]);
-    const uint32_t my_row = 4 * jq + ks;        // the input row this lane finishes
+    const uint32_t my_row = FEW ? jq : 4 * jq + ks;        // the input row this lane finishes (FEW: a wave finishes one stream, waves 2 and 3 none)
     float *y32 = reinterpret_cast<float *>(y_);
     uint16_t *y16 = reinterpret_cast<uint16_t *>(y_);
     unsigned long long best = 0ull;
@@ -237,14 +246,26 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), lane);
+            ring_step<F16, true, kSums>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), lane);
         const int buf = (rb - rb0) & 1;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < kSums; ++r) {
             s_red[buf][ks][r][lane] = tot.a[r];
-            s_red[buf][ks][4 + r][lane] = tot.b[r];
+            s_red[buf][ks][kSums + r][lane] = tot.b[r];
         }
         lds_barrier();
+        if constexpr (FEW) {
+            if (ks > 1) continue;
+            float v = s_red[buf][0][ks][lane];
+#pragma unroll
+            for (int o = 1; o < kKSplit; ++o) v += s_red[buf][o][ks][lane];
+            const uint32_t row = (rb * 2 + ks) * kTileRows + j;
+            if (my_row < rows && row < m) {
+                if (Y_F32) y32[(size_t)my_row * y_stride + row] = v;
+                else y16[(size_t)my_row * y_stride + row] = Act<F16>::round(v);
+            }
+            continue;
+        }
         float va = s_red[buf][0][ks][lane], vb = s_red[buf][0][4 + ks][lane];
 #pragma unroll
         for (int o = 1; o < kKSplit; ++o) {
@@ -302,6 +323,71 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
             if (j == 0 && my_row < rows) conf_part[(size_t)my_row * gridDim.x + blockIdx.x] = make_float2(soft.m, soft.s);
         }
     }
+}
+
+// The plain 4-bit form for matrices of few tiles: a block takes ONE of a tile's two streams, 16 weight rows, so that twice as many
+// compute units share the steps and each wave issues half of them; what the GEMV keeps per group for the tiles to come is not kept.
+// FEW as in the GEMV. Every sum has the GEMV's operands in its order, so an output's bits do not depend on the form.
+// What bounds it: a launch (3.2 us with one step in it) and a round trip. Before, turning the inputs was 88 exchanges through LDS per wave
+// and the eleven steps some 70 instructions each on one compute unit in six. 1,408 x 2,816, us back to back, the GEMV | so: 1 row 5.8 | 3.7,
+// 16 rows 5.8 | 4.3; 8,192 x 2,816, 1 row 5.9 | 4.9.
+template <bool Y_F32, bool F16, bool FEW>
+__global__ __launch_bounds__(256, 2) void matrix_gemv_half_kernel(const uint8_t *__restrict__ tiles, const uint8_t *__restrict__ scales, uint32_t m,
+                                                                  uint32_t n_groups, const uint16_t *__restrict__ x, uint32_t x_stride,
+                                                                  uint32_t rows, void *__restrict__ y_, uint32_t y_stride) {
+    constexpr int kSums = FEW ? 1 : 4;
+    __shared__ float s_red[kKSplit][kSums][64];
+    const uint32_t n_tiles = (m + 31) / 32;
+    const uint32_t tile = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7), half = blockIdx.x >> 3 & 1;      // (a tile's halves on one XCD)
+    if (tile >= n_tiles) return;
+    const uint32_t lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, jq = lane >> 4;
+    const KSlice k = k_slice(n_groups, ks);
+    const uint8_t *const my_tiles = tiles + (size_t)tile * n_groups * kTileBytes + lane * 16 + half * 8;
+    const uint8_t *const my_scales = scales + (size_t)tile * n_groups * kTileScaleBytes + j * 8 + half * 4;
+    uint2 w[kRing];
+    uint32_t sb[kRing];
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) {
+        const uint32_t grp = min(k.g0 + u, k.g_last);
+        w[u] = *reinterpret_cast<const uint2 *>(my_tiles + (size_t)grp * kTileBytes);
+        sb[u] = *reinterpret_cast<const uint32_t *>(my_scales + (size_t)grp * kTileScaleBytes);
+    }
+    uint4 x0[kRing], x1[kRing];
+    if constexpr (FEW) {
+        load_few_rows(x, x_stride, rows, lane, k, x0, x1);
+    } else {
+        load_token_rows(x, x_stride, rows, lane, k, x0, x1);
+        turn_token_rows(lane, x0, x1);
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    float tot[kSums];
+#pragma unroll
+    for (int r = 0; r < kSums; ++r) tot[r] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) {
+        const uint32_t sc = (uint32_t)u < k.ng ? sb[u] : 0u;
+        const f32x4 sx = group_input_sum<F16>(x0[u], x1[u]);
+        f32x4 acc = Act<F16>::mfma(x0[u], unpack8_offset<F16>(w[u].x), zero);
+        acc = Act<F16>::mfma(x1[u], unpack8_offset<F16>(w[u].y), acc);
+        const float s = bf16lo_to_f32(sc), t = __builtin_fmaf(-Act<F16>::kOffset, s, bf16hi_to_f32(sc));
+#pragma unroll
+        for (int r = 0; r < kSums; ++r) {
+            tot[r] = __builtin_fmaf(s, acc[r], tot[r]);
+            tot[r] = __builtin_fmaf(t, sx[r], tot[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kSums; ++r) s_red[ks][r][lane] = tot[r];
+    lds_barrier();
+    if (FEW && ks != 0) return;
+    const uint32_t r = FEW ? 0 : ks;
+    float v = s_red[0][r][lane];
+#pragma unroll
+    for (int o = 1; o < kKSplit; ++o) v += s_red[o][r][lane];
+    const uint32_t row = FEW ? jq : 4 * jq + ks, col = tile * 2 * kTileRows + half * kTileRows + j;
+    if (row >= rows || col >= m) return;
+    if (Y_F32) reinterpret_cast<float *>(y_)[(size_t)row * y_stride + col] = v;
+    else reinterpret_cast<uint16_t *>(y_)[(size_t)row * y_stride + col] = Act<F16>::round(v);
 }
 
 // The same sums for more than 16 input rows, 16 R of them per block: there the GEMV's grid rows each read the weights and every
@@ -736,11 +822,26 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
 #undef FFMOE_BAND
         return hipGetLastError();
     }
+    // Half a tile per block while those run at once: three such blocks per compute unit with few rows (135 registers), and, with the
+    // inputs to be turned in every one of them, not many more than one otherwise. us back to back with whole tiles | halves, N = 2,816: 1
+    // row, 8,192 out 5.9 | 4.9, 12,288 out 7.1 | 6.1 (12,320 in whole tiles of few rows 6.7), 16,384 out 6.8 | 7.4; 5 rows, 4,100 out 5.9 | 5.4, 5,632 out 5.7 |
+    // 5.6, 8,200 out 6.8 | 7.2; 16 rows, 4,100 out 5.9 | 5.6, 5,632 out 5.8 | 5.9, 10,000 out 7.4 | 7.8.
+    if (!planes8 && glu == 0 && rows <= FFMOE_MAX_VERIFY_ROWS && (rows <= 4 ? 2 * n_tiles <= 3 * n_cus : 8 * n_tiles <= 5 * n_cus)) {
+        const dim3 halves((n_tiles + 7) / 8 * 16);
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, halves, dim3(256), 0, s, tiles, scales, m, n / kGroup, x, x_stride, rows, y, y_stride); };
+        auto pick = [&](auto few) {
+            constexpr bool FEW = decltype(few)::value;
+            if (f16) { if (y_f32) launch(matrix_gemv_half_kernel<true, true, FEW>); else launch(matrix_gemv_half_kernel<false, true, FEW>); }
+            else { if (y_f32) launch(matrix_gemv_half_kernel<true, false, FEW>); else launch(matrix_gemv_half_kernel<false, false, FEW>); }
+        };
+        if (rows <= 4) pick(std::true_type{}); else pick(std::false_type{});
+        return hipGetLastError();
+    }
     // (two grid rows: a multiple of 8 blocks per row keeps a tile on one XCD, blocks go to the XCDs round robin, and its L2 serves the
     // second; blocks past the tile count leave at once)
     const dim3 grid(twice ? (min(2 * n_cus, n_tiles) + 7) / 8 * 8 : min(2 * n_cus, n_tiles), twice ? 2 : 1);
-#define FFMOE_MGEMV(Y, H, P, G)                                                                                             \
-    hipLaunchKernelGGL((matrix_gemv_kernel<Y, H, false, false, P, G>), grid, dim3(256), 0, s, tiles, scales, m, n / kGroup, x, x_stride, \
+#define FFMOE_MGEMV(Y, H, P, ...)                                                                                           \
+    hipLaunchKernelGGL((matrix_gemv_kernel<Y, H, false, false, P, __VA_ARGS__>), grid, dim3(256), 0, s, tiles, scales, m, n / kGroup, x, x_stride, \
                        rows, y, y_stride)
     if (glu == 1) {
         if (f16) { if (y_f32) FFMOE_MGEMV(true, true, true, 1); else FFMOE_MGEMV(false, true, true, 1); }
@@ -748,6 +849,9 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
     } else if (planes8) {
         if (f16) { if (y_f32) FFMOE_MGEMV(true, true, true, 0); else FFMOE_MGEMV(false, true, true, 0); }
         else { if (y_f32) FFMOE_MGEMV(true, false, true, 0); else FFMOE_MGEMV(false, false, true, 0); }
+    } else if (rows <= 4) {
+        if (f16) { if (y_f32) FFMOE_MGEMV(true, true, false, 0, true); else FFMOE_MGEMV(false, true, false, 0, true); }
+        else { if (y_f32) FFMOE_MGEMV(true, false, false, 0, true); else FFMOE_MGEMV(false, false, false, 0, true); }
     } else {
         if (f16) { if (y_f32) FFMOE_MGEMV(true, true, false, 0); else FFMOE_MGEMV(false, true, false, 0); }
         else { if (y_f32) FFMOE_MGEMV(true, false, false, 0); else FFMOE_MGEMV(false, false, false, 0); }

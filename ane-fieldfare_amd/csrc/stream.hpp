@@ -63,7 +63,8 @@ __device__ __forceinline__ f32x4 group_input_sum(const uint4 &x0, const uint4 &x
 
 // Consume ring slot u against the resident token operand (`sx` = its group_input_sum), then start the load
 // that refills the slot (REFILL = false: a wave that walks one tile row only has nothing to refill).
-template <bool F16 = false, bool REFILL = true>
+// SUMS: of the lane's four results, how many are kept up.
+template <bool F16 = false, bool REFILL = true, int SUMS = 4>
 __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, const uint4 &x0, const uint4 &x1,
                                           const f32x4 &sx, TwoStreamAcc &tot, const TileSource &src,
                                           uint32_t next_tile_index, uint32_t lane) {
@@ -80,7 +81,7 @@ __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, co
     const float sb = bf16lo_to_f32(sc.y), bb = bf16hi_to_f32(sc.y);
     const float ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ba), tb = __builtin_fmaf(-Act<F16>::kOffset, sb, bb);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < SUMS; ++r) {
         tot.a[r] = __builtin_fmaf(sa, acc_a[r], tot.a[r]);
         tot.a[r] = __builtin_fmaf(ta, sx[r], tot.a[r]);
         tot.b[r] = __builtin_fmaf(sb, acc_b[r], tot.b[r]);
@@ -108,6 +109,20 @@ __device__ __forceinline__ KSlice k_slice(uint32_t groups, uint32_t ks) {
 __device__ __forceinline__ void load_token_rows(const uint16_t *__restrict__ x, uint32_t x_stride, uint32_t rows,
                                                 uint32_t lane, const KSlice &k, uint4 (&x0)[kRing], uint4 (&x1)[kRing]) {
     const uint16_t *xrow = x + (size_t)min(lane >> 2, rows - 1) * x_stride + 8 * (lane & 3);
+#pragma unroll
+    for (int u = 0; u < kRing; ++u) {
+        const bool live = (uint32_t)u < k.ng;
+        const uint32_t gg = min(k.g0 + u, k.g_last);
+        x0[u] = live ? *reinterpret_cast<const uint4 *>(xrow + gg * kGroup) : uint4{0, 0, 0, 0};
+        x1[u] = live ? *reinterpret_cast<const uint4 *>(xrow + gg * kGroup + 32) : uint4{0, 0, 0, 0};
+    }
+}
+
+// Up to four rows straight in the operand layout, row t as operand row 4 t (and 4 t + 1 .. + 3, whose results nobody keeps): the
+// lanes of a row and quarter ask for the same 16 bytes, so an instruction is as many requests of 64 bytes as there are rows.
+__device__ __forceinline__ void load_few_rows(const uint16_t *__restrict__ x, uint32_t x_stride, uint32_t rows, uint32_t lane,
+                                              const KSlice &k, uint4 (&x0)[kRing], uint4 (&x1)[kRing]) {
+    const uint16_t *xrow = x + (size_t)min((lane & 15) >> 2, rows - 1) * x_stride + 8 * (lane >> 4);
 #pragma unroll
     for (int u = 0; u < kRing; ++u) {
         const bool live = (uint32_t)u < k.ng;
