@@ -28,45 +28,55 @@ struct Row8 {
     float v[8];
 };
 
-// Rows are in the context's activation type (F16: FP16, else bf16); norm weights are always bf16 (loadw8).
-template <bool VEC, bool F16>
-__device__ __forceinline__ Row8 load8(const uint16_t *__restrict__ row, uint32_t chunk) {
+// Rows are in the context's activation type (F16: FP16, else bf16); norm weights are always bf16.
+template <bool VEC>
+__device__ __forceinline__ uint4 load_raw8(const uint16_t *__restrict__ row, uint32_t chunk) {
+    if (VEC) return reinterpret_cast<const uint4 *>(row)[chunk];
+    const uint16_t *p = row + 8 * chunk;
+    return make_uint4(p[0] | (uint32_t)p[1] << 16, p[2] | (uint32_t)p[3] << 16, p[4] | (uint32_t)p[5] << 16, p[6] | (uint32_t)p[7] << 16);
+}
+
+template <bool F16>
+__device__ __forceinline__ Row8 widen8(const uint4 &q) {
     Row8 r;
-    if (VEC) {
-        const uint4 q = reinterpret_cast<const uint4 *>(row)[chunk];
-        r.v[0] = Act<F16>::lo(q.x); r.v[1] = Act<F16>::hi(q.x);
-        r.v[2] = Act<F16>::lo(q.y); r.v[3] = Act<F16>::hi(q.y);
-        r.v[4] = Act<F16>::lo(q.z); r.v[5] = Act<F16>::hi(q.z);
-        r.v[6] = Act<F16>::lo(q.w); r.v[7] = Act<F16>::hi(q.w);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) r.v[e] = Act<F16>::widen(row[8 * chunk + e]);
-    }
+    r.v[0] = Act<F16>::lo(q.x); r.v[1] = Act<F16>::hi(q.x);
+    r.v[2] = Act<F16>::lo(q.y); r.v[3] = Act<F16>::hi(q.y);
+    r.v[4] = Act<F16>::lo(q.z); r.v[5] = Act<F16>::hi(q.z);
+    r.v[6] = Act<F16>::lo(q.w); r.v[7] = Act<F16>::hi(q.w);
     return r;
 }
 
-template <bool VEC>
-__device__ __forceinline__ Row8 loadw8(const uint16_t *__restrict__ row, uint32_t chunk) {
-    return load8<VEC, false>(row, chunk);
+template <bool VEC, bool F16>
+__device__ __forceinline__ Row8 load8(const uint16_t *__restrict__ row, uint32_t chunk) {
+    return widen8<F16>(load_raw8<VEC>(row, chunk));
+}
+
+// A value on its way to 16 bits is an fp32 number first, as in the reference: left alone, the compiler makes a product and its rounding
+// to FP16 one v_fma_mixlo_f16, which rounds once (some 5 of 100,000 values off by one bit).
+template <bool F16>
+__device__ __forceinline__ float as_f32(float x) {
+    if (F16) asm("" : "+v"(x));
+    return x;
+}
+template <bool F16>
+__device__ __forceinline__ float round16(float x) { return Act<F16>::widen(Act<F16>::round(as_f32<F16>(x))); }
+
+template <bool F16>
+__device__ __forceinline__ uint4 pack8(const Row8 &r) {
+    auto pair = [&](int e) { return Act<F16>::pack(as_f32<F16>(r.v[e]), as_f32<F16>(r.v[e + 1])); };
+    return make_uint4(pair(0), pair(2), pair(4), pair(6));
 }
 
 template <bool VEC, bool F16>
 __device__ __forceinline__ void store8(uint16_t *__restrict__ row, uint32_t chunk, const Row8 &r) {
     if (VEC) {
-        uint4 q;
-        q.x = Act<F16>::pack(r.v[0], r.v[1]);
-        q.y = Act<F16>::pack(r.v[2], r.v[3]);
-        q.z = Act<F16>::pack(r.v[4], r.v[5]);
-        q.w = Act<F16>::pack(r.v[6], r.v[7]);
-        reinterpret_cast<uint4 *>(row)[chunk] = q;
+        reinterpret_cast<uint4 *>(row)[chunk] = pack8<F16>(r);
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) row[8 * chunk + e] = Act<F16>::round(r.v[e]);
+        for (int e = 0; e < 8; ++e) row[8 * chunk + e] = Act<F16>::round(as_f32<F16>(r.v[e]));
     }
 }
 
-template <bool F16>
-__device__ __forceinline__ float round16(float x) { return Act<F16>::widen(Act<F16>::round(x)); }
 
 // 1 / sqrt(mean of squares + eps) over the block's row; `slot` is a 4-float LDS area of its own
 __device__ __forceinline__ float block_rms_inv(const Row8 (&x)[kMaxChunks], uint32_t n_mine, uint32_t d, float eps,
@@ -78,7 +88,7 @@ __device__ __forceinline__ float block_rms_inv(const Row8 (&x)[kMaxChunks], uint
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(x[c].v[e], x[c].v[e], acc);
     acc = wave_butterfly_sum(acc);
-    if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = acc;
+    if ((threadIdx.x & 63) == 0 && threadIdx.x < kRowThreads) slot[threadIdx.x >> 6] = acc;
     __syncthreads();
     const float total = (slot[0] + slot[1]) + (slot[2] + slot[3]);
     return 1.0f / sqrtf(total / (float)d + eps);
@@ -101,9 +111,9 @@ __global__ __launch_bounds__(kRowThreads) void post_attn_setup_kernel(
         if ((uint32_t)c < n_mine) {
             a[c] = load8<VEC, F16>(arow, t + c * kRowThreads);
             h[c] = load8<VEC, F16>(hrow, t + c * kRowThreads);
-            w0[c] = loadw8<VEC>(w_post_attn, t + c * kRowThreads);
-            w1[c] = loadw8<VEC>(w_pre_ffn, t + c * kRowThreads);
-            w2[c] = loadw8<VEC>(w_pre_ffn2, t + c * kRowThreads);
+            w0[c] = load8<VEC, false>(w_post_attn, t + c * kRowThreads);
+            w1[c] = load8<VEC, false>(w_pre_ffn, t + c * kRowThreads);
+            w2[c] = load8<VEC, false>(w_pre_ffn2, t + c * kRowThreads);
         }
     const float attn_inv = block_rms_inv(a, n_mine, d, eps, s_sum[0]);
 #pragma unroll
@@ -148,25 +158,42 @@ struct RoutedRows {
     uint32_t shared_chunks, t;
 };
 
+// What a chunk of h2 (and of h1) is made of. The routes' weights and validity words come as one load each, a route per lane: read
+// where they are wanted, route after route, the words were eight scalar loads one behind the other.
+struct RoutedChunk {
+    f32x4 lo[8], hi[8], shared_lo[4], shared_hi[4];
+};
+
+__device__ __forceinline__ RoutedChunk load_routed(const RoutedRows &rr, uint32_t row, uint32_t d, uint32_t chunk) {
+    RoutedChunk in;
+#pragma unroll
+    for (uint32_t r = 0; r < 8; ++r) {
+        const float *src = rr.partials + (size_t)(row * rr.top_k + min(r, rr.top_k - 1)) * d + 8 * chunk;
+        in.lo[r] = *reinterpret_cast<const f32x4 *>(src);
+        in.hi[r] = *reinterpret_cast<const f32x4 *>(src + 4);
+    }
+    if (rr.shared_partials)
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const float *src = rr.shared_partials + ((size_t)min(c, rr.shared_chunks - 1) * rr.t + row) * d + 8 * chunk;
+            in.shared_lo[c] = *reinterpret_cast<const f32x4 *>(src);
+            in.shared_hi[c] = *reinterpret_cast<const f32x4 *>(src + 4);
+        }
+    return in;
+}
+
 template <bool F16>
-__device__ __forceinline__ Row8 shared_row8(const RoutedRows &rr, uint32_t row, uint32_t d, uint32_t chunk) {
+__device__ __forceinline__ Row8 shared_row8(const RoutedRows &rr, const RoutedChunk &in) {
     Row8 out;
 #pragma unroll
     for (int i = 0; i < 8; ++i) out.v[i] = 0.0f;
-    f32x4 lo[4], hi[4];
-#pragma unroll
-    for (uint32_t c = 0; c < 4; ++c) {
-        const float *src = rr.shared_partials + ((size_t)min(c, rr.shared_chunks - 1) * rr.t + row) * d + 8 * chunk;
-        lo[c] = *reinterpret_cast<const f32x4 *>(src);
-        hi[c] = *reinterpret_cast<const f32x4 *>(src + 4);
-    }
 #pragma unroll
     for (uint32_t c = 0; c < 4; ++c) {
         if (c < rr.shared_chunks) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                out.v[i] += lo[c][i];
-                out.v[4 + i] += hi[c][i];
+                out.v[i] += in.shared_lo[c][i];
+                out.v[4 + i] += in.shared_hi[c][i];
             }
         }
     }
@@ -175,30 +202,20 @@ __device__ __forceinline__ Row8 shared_row8(const RoutedRows &rr, uint32_t row, 
     return out;
 }
 
+// lane r: route r's weight bits and validity word (also where lane r itself has no chunk)
 template <bool F16>
-__device__ __forceinline__ Row8 combine8(const RoutedRows &rr, uint32_t row, uint32_t d, uint32_t chunk) {
-    float wv[8];
-    uint32_t valid[8];
-    f32x4 lo[8], hi[8];
-#pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) {
-        const uint32_t route = row * rr.top_k + min(r, rr.top_k - 1);
-        wv[r] = Act<F16>::widen(rr.w[route]);
-        valid[r] = rr.route_valid[route];
-        const float *src = rr.partials + (size_t)route * d + 8 * chunk;
-        lo[r] = *reinterpret_cast<const f32x4 *>(src);
-        hi[r] = *reinterpret_cast<const f32x4 *>(src + 4);
-    }
+__device__ __forceinline__ Row8 combine8(const RoutedChunk &in, uint32_t top_k, uint32_t weight, uint32_t valid) {
     Row8 out;
 #pragma unroll
     for (int i = 0; i < 8; ++i) out.v[i] = 0.0f;
 #pragma unroll
     for (uint32_t r = 0; r < 8; ++r) {
-        if (r < rr.top_k && valid[r] != 0) {
+        const float wv = Act<F16>::widen((uint16_t)__builtin_amdgcn_readlane((int)weight, (int)r));
+        if (r < top_k && __builtin_amdgcn_readlane((int)valid, (int)r) != 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                out.v[i] = __builtin_fmaf(wv[r], lo[r][i], out.v[i]);
-                out.v[4 + i] = __builtin_fmaf(wv[r], hi[r][i], out.v[4 + i]);
+                out.v[i] = __builtin_fmaf(wv, in.lo[r][i], out.v[i]);
+                out.v[4 + i] = __builtin_fmaf(wv, in.hi[r][i], out.v[4 + i]);
             }
         }
     }
@@ -210,8 +227,11 @@ __device__ __forceinline__ Row8 combine8(const RoutedRows &rr, uint32_t row, uin
 // NORMS: h1 arrives before its own norm (w_postffn1) and, when w_next is given, the norm of the new hidden
 // row under w_next goes to `normed` (the next layer's input norm): fused_layer_tail_norms
 // (Kernels/Fusions/FusedLayerTail.swift:74-117). h1 itself is left as it was found.
+// COMBINE: rows of more than 256 chunks have a thread per chunk for the combining, which is 24 loads of 16 bytes for one: those past the
+// 256th hand their chunks, rounded to 16 bits as they are, to the threads that own them in the order of the sums. 1 row of
+// 2,816, us per launch: both chunks by their owner, each behind its own chain of loads 5.9, so 4.6.
 template <bool VEC, bool NORMS, bool F16, bool COMBINE = false>
-__global__ __launch_bounds__(kRowThreads) void layer_tail_kernel(const uint16_t *__restrict__ h2, uint32_t h2_stride,
+__global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer_tail_kernel(const uint16_t *__restrict__ h2, uint32_t h2_stride,
                                                                  const uint16_t *__restrict__ h1, uint32_t h1_stride,
                                                                  uint16_t *__restrict__ hidden, uint32_t hidden_stride,
                                                                  const uint16_t *__restrict__ w_postffn2,
@@ -223,27 +243,63 @@ __global__ __launch_bounds__(kRowThreads) void layer_tail_kernel(const uint16_t 
                                                                  RoutedRows routed) {
     __shared__ float s_sum[4][4];
     const uint32_t row = blockIdx.x, t = threadIdx.x, chunks = d / 8;
-    const uint32_t n_mine = t < chunks ? (chunks - t + kRowThreads - 1) / kRowThreads : 0;
+    const uint32_t n_mine = t < min(chunks, (uint32_t)kRowThreads) ? (chunks - t + kRowThreads - 1) / kRowThreads : 0;
     uint16_t *hrow = hidden + (size_t)row * hidden_stride;
     Row8 a[kMaxChunks], h12[kMaxChunks], hv[kMaxChunks], wf1[kMaxChunks], wf2[kMaxChunks], wf[kMaxChunks], wn[kMaxChunks];
-#pragma unroll
-    for (int c = 0; c < kMaxChunks; ++c)
-        if ((uint32_t)c < n_mine) {
-            const uint32_t chunk = t + c * kRowThreads;
-            if (!COMBINE) a[c] = load8<VEC, F16>(h2 + (size_t)row * h2_stride, chunk);
-            if (!COMBINE || !routed.shared_partials) h12[c] = load8<VEC, F16>(h1 + (size_t)row * h1_stride, chunk);
-            hv[c] = load8<VEC, F16>(hrow, chunk);
-            wf2[c] = loadw8<VEC>(w_postffn2, chunk);
-            wf[c] = loadw8<VEC>(w_postffn, chunk);
-            if (NORMS) wf1[c] = loadw8<VEC>(w_postffn1, chunk);
-            if (NORMS && w_next) wn[c] = loadw8<VEC>(w_next, chunk);
-        }
-    if (COMBINE) {
+    if constexpr (COMBINE) {
+        // every load before the first use of one: converted beside their loads, a thread's chunks were a round trip each
+        __shared__ uint4 handed[2][kRowThreads];        // h2, h1: chunks 256 .. 511
+        const bool h1_given = !routed.shared_partials;
+        const uint32_t route = row * routed.top_k + min(t & 63, routed.top_k - 1);
+        const uint32_t weight = routed.w[route], valid = routed.route_valid[route];
+        uint4 h1_raw[kMaxChunks], h_raw[kMaxChunks], wf2_raw[kMaxChunks], wf_raw[kMaxChunks];
 #pragma unroll
         for (int c = 0; c < kMaxChunks; ++c)
             if ((uint32_t)c < n_mine) {
-                a[c] = combine8<F16>(routed, row, d, t + c * kRowThreads);
-                if (routed.shared_partials) h12[c] = shared_row8<F16>(routed, row, d, t + c * kRowThreads);
+                const uint32_t chunk = t + c * kRowThreads;
+                if (h1_given) h1_raw[c] = load_raw8<VEC>(h1 + (size_t)row * h1_stride, chunk);
+                h_raw[c] = load_raw8<VEC>(hrow, chunk);
+                wf2_raw[c] = load_raw8<VEC>(w_postffn2, chunk);
+                wf_raw[c] = load_raw8<VEC>(w_postffn, chunk);
+            }
+        uint4 h2_raw = {0, 0, 0, 0};
+        if (t < chunks) {
+            const RoutedChunk in = load_routed(routed, row, d, t);
+            h2_raw = pack8<F16>(combine8<F16>(in, routed.top_k, weight, valid));
+            uint4 h1_mine = {0, 0, 0, 0};
+            if (!h1_given) h1_mine = pack8<F16>(shared_row8<F16>(routed, in));
+            if (t < kRowThreads) {
+                if (!h1_given) h1_raw[0] = h1_mine;
+            } else {
+                handed[0][t - kRowThreads] = h2_raw;
+                handed[1][t - kRowThreads] = h1_mine;
+            }
+        }
+        __syncthreads();
+        if (n_mine > 1) {
+            a[1] = widen8<F16>(handed[0][t]);
+            if (!h1_given) h1_raw[1] = handed[1][t];
+        }
+        a[0] = widen8<F16>(h2_raw);
+#pragma unroll
+        for (int c = 0; c < kMaxChunks; ++c) {
+            h12[c] = widen8<F16>(h1_raw[c]);
+            hv[c] = widen8<F16>(h_raw[c]);
+            wf2[c] = widen8<false>(wf2_raw[c]);
+            wf[c] = widen8<false>(wf_raw[c]);
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < kMaxChunks; ++c)
+            if ((uint32_t)c < n_mine) {
+                const uint32_t chunk = t + c * kRowThreads;
+                a[c] = load8<VEC, F16>(h2 + (size_t)row * h2_stride, chunk);
+                h12[c] = load8<VEC, F16>(h1 + (size_t)row * h1_stride, chunk);
+                hv[c] = load8<VEC, F16>(hrow, chunk);
+                wf2[c] = load8<VEC, false>(w_postffn2, chunk);
+                wf[c] = load8<VEC, false>(w_postffn, chunk);
+                if (NORMS) wf1[c] = load8<VEC, false>(w_postffn1, chunk);
+                if (NORMS && w_next) wn[c] = load8<VEC, false>(w_next, chunk);
             }
     }
     if (NORMS) {
@@ -301,7 +357,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t *x,
     for (int c = 0; c < kMaxChunks; ++c)
         if ((uint32_t)c < n_mine) {
             a[c] = load8<VEC, F16>(x + (size_t)row * x_stride, t + c * kRowThreads);
-            wq[c] = loadw8<VEC>(w, t + c * kRowThreads);
+            wq[c] = load8<VEC, false>(w, t + c * kRowThreads);
         }
     const float inv = block_rms_inv(a, n_mine, d, eps, s_sum);
 #pragma unroll
@@ -351,7 +407,7 @@ hipError_t launch_layer_tail(hipStream_t s, const uint16_t *h2, uint32_t h2_stri
         // h2 is made from the un-combined rows (16-byte aligned fp32 rows: d % 8 == 0); the plain tail only
         const bool vec = (shared_partials || aligned16(h1, h1_stride)) && aligned16(hidden, hidden_stride) && aligned16(w_postffn2, 8) && aligned16(w_postffn, 8);
 #define FFMOE_TAILC(V, H)                                                                                             \
-    hipLaunchKernelGGL((layer_tail_kernel<V, false, H, true>), dim3(t), dim3(kRowThreads), 0, s, nullptr, 0u, h1, h1_stride, \
+    hipLaunchKernelGGL((layer_tail_kernel<V, false, H, true>), dim3(t), dim3(d / 8 > kRowThreads ? 2 * kRowThreads : kRowThreads), 0, s, nullptr, 0u, h1, h1_stride, \
                        hidden, hidden_stride, w_postffn2, w_postffn, d, eps, layer_scalar, nullptr, nullptr, nullptr, 0u, routed)
         if (f16) { if (vec) FFMOE_TAILC(true, true); else FFMOE_TAILC(false, true); }
         else { if (vec) FFMOE_TAILC(true, false); else FFMOE_TAILC(false, false); }

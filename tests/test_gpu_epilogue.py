@@ -207,3 +207,47 @@ def test_rmsnorm_reference_case_hidden_size(oracle, torch, act):
     rel = np.abs(got - ref).max() / np.abs(ref).max()
     assert rel < 5e-3, rel
     c.close()
+
+
+def test_fp16_rows_round_products_through_fp32(ctx, oracle, torch):
+    # enough rows that a product rounded to FP16 in one step, without the fp32 rounding in front, would show (5 values in 100,000)
+    rows, d = 301, 2816
+    g = np.random.default_rng(16)
+    hidden, attn, h2, h1 = (g.normal(0, 1, (rows, d)).astype(np.float16).view(np.uint16) for _ in range(4))
+    ws = [oracle.bf16_bits((0.5 + g.random(d)).astype(np.float32)) for _ in range(5)]
+    tw = [bf16_tensor(torch, w) for w in ws]
+    dev = lambda a: torch.from_numpy(a.view(np.float16).copy()).cuda()
+    import fieldfare_moe as ff
+    c = ff.Context(128, 64, 4, 2, n_layers=1, max_tokens=16, act_dtype="fp16")
+    th = dev(hidden)
+    got = (th,) + tuple(c.post_attn_setup(th, dev(attn), tw[0], tw[1], tw[2], eps=EPS, d=d))
+    ref = oracle.post_attn_setup(hidden, attn, ws[0], ws[1], ws[2], EPS, oracle.FP16)
+    for a, b in zip(got, ref):
+        assert np.array_equal(bits_of(a), b)
+    c.layer_tail(dev(h2), dev(h1), th, tw[3], tw[4], 0.875, EPS, d=d)
+    assert np.array_equal(bits_of(th), oracle.layer_tail(h2, h1, ref[0], ws[3], ws[4], 0.875, EPS, oracle.FP16))
+    assert np.array_equal(bits_of(c.rmsnorm(dev(attn), tw[0], EPS, d=d)), oracle.rmsnorm(attn, ws[0], EPS, oracle.FP16))
+    c.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,top_k", [(2048, 8), (2112, 3), (4096, 8), (128, 1)])
+def test_tail_of_uncombined_rows_equals_separate_steps(oracle, torch, d, top_k, act):
+    # the tail that combines the routes' rows itself: rows of up to 256 chunks of eight values, of just more and of the most
+    import fieldfare_moe as ff
+    from helpers import make_layer, to_ff_offsets
+    e, f, t = 8, 64, 5
+    rng, pool, router = make_layer(oracle, 9, d, f, e)
+    ctx = ff.Context(d, f, e, top_k, n_layers=1, max_tokens=16, act_dtype=act)
+    ctx.upload_layer(0, pool.bytes, pool.stride, to_ff_offsets(ff, pool.offsets))
+    ctx.upload_router_bf16(0, router)
+    make = lambda: torch.from_numpy(rng.normal(0, 1, (t, d)).astype(np.float32)).cuda().to(ctx.act)
+    x, h1, hidden = make(), make(), make()
+    w2, w1 = (bf16_tensor(torch, oracle.bf16_bits((0.5 + rng.random(d)).astype(np.float32))) for _ in range(2))
+    y, _, w = ctx.route_verify(0, x, x)
+    want = hidden.clone()
+    ctx.layer_tail(y, h1, want, w2, w1, 0.5)
+    _, _, w = ctx.route_verify(0, x, x, combine=False)
+    ctx.layer_tail_routed(w, h1, hidden, w2, w1, 0.5)
+    assert torch.equal(hidden.view(torch.int16), want.view(torch.int16))
+    ctx.close()
