@@ -150,110 +150,123 @@ __global__ __launch_bounds__(256) void gemv_int4_kernel(const uint8_t *__restric
     }
 }
 
-// The same product on the matrix unit, for n <= 4 * kRing * 64. A block takes 16 weight rows at a time, its four waves split
+// The same product on the matrix unit, for n <= kListedParts * kListedRing * 64. A block takes 16 weight rows at a time, its eight waves split
 // K; a group's product is v_mfma_f32_16x16x32 of the (up to 16) input rows with the nibbles as 16 + q (bf16) or as
 // subnormals (FP16: common.hpp), then s * acc + (b - 16 s) * sum x, as in the expert kernels (stream.hpp) but on the reference's row-major bytes: four
 // neighbouring lanes load the 32 bytes of a row's group (16 segments per request instead of 64) and ds_bpermute hands
 // each operand lane (row i, quarter q) its eight bytes, the values k = 16 q .. 16 q + 15 of the group. Nibble p of such a
 // dword is element p, so ((w >> 4 m) & 0x000F000F) pairs elements m and m + 4, and the input operand is paired the same way.
+// FEW (up to four input rows): input row t is operand row 4 t, so that one of a lane's four sums is all there is to keep up, and
+// each operand lane loads its own bytes - the lanes of a row ask for the same ones, nothing is turned through LDS.
 // Bound: latency - row id, weights, products and the merge are one chain per 16 rows, and a hot list of a few thousand
-// rows is one such chain per compute unit. 4,099 listed rows x 2,816, 16 input rows: 50.8 us with the vector ALU's dot
-// products (four passes of four input rows over the weights) -> 7.5 us;
-// 32,768 rows: 19 us. Error of a logit against 64 bits (2-norm): 1.7e-7 in bf16 and 4.9e-6 in FP16, where the dot products have
+// rows is one such chain per compute unit. So the input rows are asked for between the ids and the weights, which wait for
+// the ids, and eight waves take six groups each: with four, eleven each, a chain was twice as long and a block's registers left
+// two waves per SIMD. Listed rows x 2,816, us with four waves and the input rows behind the weights | so: 512 rows, 1 input row 6.4 | 4.8;
+// 4,099 rows, 1 input row 7.1 | 5.7, 16 input rows 7.4 | 6.2 (the vector unit's dot products: 50.8); 32,768 rows 17.7 | 16.8, 19.0 | 17.5.
+// Error of a logit against 64 bits (2-norm): 1.7e-7 in bf16 and 4.9e-6 in FP16, where the dot products have
 // 8.6e-7 and 1.6e-5, and 128 + q / 1024 + q on the matrix unit 1.0e-6 and 1.4e-5.
-template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16>
-__global__ __launch_bounds__(256, 2) void gemv_int4_mfma_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
-                                                                const uint16_t *__restrict__ biases, const uint16_t *__restrict__ x,
-                                                                void *__restrict__ y_, uint32_t m, uint32_t n_groups, uint32_t rows,
-                                                                uint32_t x_stride, uint32_t y_stride, const uint32_t *__restrict__ ids) {
-    __shared__ float s_red[2][kKSplit][4][64];
+constexpr int kListedParts = 8, kListedRing = 6;
+static_assert(kListedParts * kListedRing >= kKSplit * kRing, "every width up to FFMOE_MATRIX_MAX_N");
+template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16, bool FEW>
+__global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
+                                                                              const uint16_t *__restrict__ biases, const uint16_t *__restrict__ x,
+                                                                              void *__restrict__ y_, uint32_t m, uint32_t n_groups, uint32_t rows,
+                                                                              uint32_t x_stride, uint32_t y_stride, const uint32_t *__restrict__ ids) {
+    constexpr int kSums = FEW ? 1 : 4;
+    __shared__ float s_red[2][kListedParts][kSums][64];
     const uint32_t lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, jq = lane >> 4;                  // operand layout: row j, quarter jq
     const uint32_t lrow = lane >> 2, lq = lane & 3;                // load layout: row lrow, quarter lq
     const uint32_t n_blocks = (m + kTileRows - 1) / kTileRows;
-    const KSlice k = k_slice(n_groups, ks);
+    const uint32_t g0 = ks * n_groups / kListedParts, ng = (ks + 1) * n_groups / kListedParts - g0;
+    const uint32_t g_last = ng ? g0 + ng - 1 : min(g0, n_groups - 1);
     const size_t row_bytes = (size_t)n_groups * (kGroup / 2);
     auto id_of = [&](uint32_t rb) {
         const uint32_t o = min(rb * kTileRows + lrow, m - 1);
         return ids ? ids[o] : o;
     };
-    uint2 wt[kRing];
-    uint32_t sb[3];                                                 // scale | bias << 16 of groups g0 + 3 lq + 0 .. 2 of row lrow
+    uint2 wt[kListedRing];
+    uint32_t sb[2];                                                 // scale | bias << 16 of groups g0 + 2 lq + 0 .. 1 of row lrow
     auto load_w = [&](uint32_t row, int u) {
-        const uint8_t *p = w + row * row_bytes + (size_t)min(k.g0 + u, k.g_last) * (kGroup / 2) + 8 * lq;
+        const uint8_t *p = w + row * row_bytes + (size_t)min(g0 + u, g_last) * (kGroup / 2) + 8 * lq;
         if (ALIGNED) return *reinterpret_cast<const uint2 *>(p);
         const uint16_t *h = reinterpret_cast<const uint16_t *>(p);  // 2-byte alignment is guaranteed
         return make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
     };
     auto load_s = [&](uint32_t row, int v) {
-        const size_t at = (size_t)row * n_groups + min(k.g0 + 3 * lq + v, k.g_last);
+        const size_t at = (size_t)row * n_groups + min(g0 + 2 * lq + v, g_last);
         return (uint32_t)scales[at] | ((uint32_t)biases[at] << 16);
     };
     uint32_t rb = blockIdx.x;                                       // the grid has at most n_blocks blocks
-    uint32_t row = id_of(rb);
-#pragma unroll
-    for (int u = 0; u < kRing; ++u) wt[u] = load_w(row, u);
-#pragma unroll
-    for (int v = 0; v < 3; ++v) sb[v] = load_s(row, v);
-    uint32_t next_id = id_of(min(rb + gridDim.x, n_blocks - 1));
-
-    // the input rows of this wave's K-slice in operand order, paired like the nibbles, and their sum per group
-    uint4 x0[kRing], x1[kRing];
-    f32x4 sx[kRing];
+    uint32_t row = id_of(rb), next_id = id_of(min(rb + gridDim.x, n_blocks - 1));
+    // the input rows of this wave's K-slice
+    uint4 x0[kListedRing], x1[kListedRing];
     {
-        const uint16_t *xrow = x + (size_t)min(lrow, rows - 1) * x_stride + 16 * lq;
+        const uint32_t my = FEW ? j >> 2 : lrow, quarter = FEW ? jq : lq;
+        const uint16_t *xrow = x + (size_t)min(my, rows - 1) * x_stride + 16 * quarter;
 #pragma unroll
-        for (int u = 0; u < kRing; ++u) {
-            const bool live = (uint32_t)u < k.ng;
-            const uint16_t *p = xrow + min(k.g0 + u, k.g_last) * kGroup;
+        for (int u = 0; u < kListedRing; ++u) {
+            const bool live = (uint32_t)u < ng;
+            const uint16_t *p = xrow + min(g0 + u, g_last) * kGroup;
             x0[u] = live ? load_x8<X_ALIGNED>(p) : uint4{0, 0, 0, 0};
             x1[u] = live ? load_x8<X_ALIGNED>(p + 8) : uint4{0, 0, 0, 0};
         }
-        turn_token_rows(lane, x0, x1);
+    }
+#pragma unroll
+    for (int u = 0; u < kListedRing; ++u) wt[u] = load_w(row, u);
+#pragma unroll
+    for (int v = 0; v < 2; ++v) sb[v] = load_s(row, v);
+    // ... in operand order, paired like the nibbles, and their sum per group
+    f32x4 sx[kListedRing];
+    {
+        if constexpr (!FEW) turn_token_rows(lane, x0, x1);
         auto paired = [](const uint4 &d) {
             return uint4{(d.x & 0xFFFFu) | (d.z << 16), (d.x >> 16) | (d.z & 0xFFFF0000u),
                          (d.y & 0xFFFFu) | (d.w << 16), (d.y >> 16) | (d.w & 0xFFFF0000u)};
         };
 #pragma unroll
-        for (int u = 0; u < kRing; ++u) {
+        for (int u = 0; u < kListedRing; ++u) {
             x0[u] = paired(x0[u]);
             x1[u] = paired(x1[u]);
             sx[u] = group_input_sum<F16>(x0[u], x1[u]);
         }
     }
     const int pull = (int)((4 * j + jq) * 4);
-    const uint32_t my_row = 4 * jq + ks;                            // the input row this lane finishes
+    const uint32_t my_row = FEW ? jq : 4 * jq + ks;                 // the input row this lane finishes (waves kSums and up: none)
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     for (int buf = 0; rb < n_blocks; rb += gridDim.x, buf ^= 1) {
         row = next_id;
         next_id = id_of(min(rb + 2 * gridDim.x, n_blocks - 1));
-        f32x4 tot = zero;
+        float tot[kSums];
 #pragma unroll
-        for (int u = 0; u < kRing; ++u) {
+        for (int r = 0; r < kSums; ++r) tot[r] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kListedRing; ++u) {
             uint2 t;
             t.x = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].x);
             t.y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].y);
-            uint32_t sc = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((4 * j + u / 3) * 4), (int)sb[u % 3]);
-            if ((uint32_t)u >= k.ng) sc = 0;
+            uint32_t sc = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((4 * j + u / 2) * 4), (int)sb[u % 2]);
+            if ((uint32_t)u >= ng) sc = 0;
             wt[u] = load_w(row, u);                                 // the next 16 rows (past the last: these again)
             f32x4 acc = Act<F16>::mfma(x0[u], unpack8_fine<F16>(t.x), zero);
             acc = Act<F16>::mfma(x1[u], unpack8_fine<F16>(t.y), acc);
             const float s = bf16lo_to_f32(sc), b = bf16hi_to_f32(sc), su = s * FineNibble<F16>::kUnit;
             const float tb = __builtin_fmaf(-FineNibble<F16>::kOffset, s, b);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < kSums; ++r) {
                 tot[r] = __builtin_fmaf(su, acc[r], tot[r]);
                 tot[r] = __builtin_fmaf(tb, sx[u][r], tot[r]);
             }
         }
 #pragma unroll
-        for (int v = 0; v < 3; ++v) sb[v] = load_s(row, v);
+        for (int v = 0; v < 2; ++v) sb[v] = load_s(row, v);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s_red[buf][ks][r][lane] = tot[r];
+        for (int r = 0; r < kSums; ++r) s_red[buf][ks][r][lane] = tot[r];
         lds_barrier();
+        if (ks >= (uint32_t)kSums) continue;
         float v = s_red[buf][0][ks][lane];
 #pragma unroll
-        for (int o = 1; o < kKSplit; ++o) v += s_red[buf][o][ks][lane];
+        for (int o = 1; o < kListedParts; ++o) v += s_red[buf][o][ks][lane];
         const uint32_t out = rb * kTileRows + j;
         if (my_row < rows && out < m) {
             const size_t at = (size_t)my_row * y_stride + out;
@@ -268,14 +281,14 @@ __global__ __launch_bounds__(256, 2) void gemv_int4_mfma_kernel(const uint8_t *_
 hipError_t launch_gemv_int4(hipStream_t s, const uint8_t *w, const uint16_t *scales, const uint16_t *biases,
                             const uint16_t *x, void *y, uint32_t m, uint32_t n, uint32_t rows,
                             uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids, bool f16, uint32_t n_cus) {
-    if (n / kGroup <= (uint32_t)(kKSplit * kRing)) {
+    if (n <= FFMOE_MATRIX_MAX_N) {
         // every row count of such a width takes this form (the rows of a call equal single-row calls bit for bit)
         const dim3 blocks(min((m + kTileRows - 1) / kTileRows, 2 * n_cus));
         const bool wide_w = reinterpret_cast<uintptr_t>(w) % 8 == 0, wide_x = reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_stride % 8 == 0;
         if (f16 && !wide_x) return hipErrorInvalidValue;     // FP16 rows come 16-byte aligned (checked at the boundary)
 #define FFMOE_GEMVM(A, X, Y, H)                                                                                                     \
-    hipLaunchKernelGGL((gemv_int4_mfma_kernel<A, X, Y, H>), blocks, dim3(256), 0, s, w, scales, biases, x, y, m, n / kGroup, rows, x_stride, \
-                       y_stride, ids)
+    hipLaunchKernelGGL((rows <= 4 ? gemv_int4_mfma_kernel<A, X, Y, H, true> : gemv_int4_mfma_kernel<A, X, Y, H, false>), blocks,               \
+                       dim3(64 * kListedParts), 0, s, w, scales, biases, x, y, m, n / kGroup, rows, x_stride, y_stride, ids)
 #define FFMOE_GEMVM_X(A, Y)                                                                             \
     do {                                                                                                \
         if (f16) FFMOE_GEMVM(A, true, Y, true);                                                         \

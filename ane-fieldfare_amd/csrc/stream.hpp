@@ -132,7 +132,7 @@ __device__ __forceinline__ void load_few_rows(const uint16_t *__restrict__ x, ui
     }
 }
 
-__device__ __forceinline__ void turn_token_rows(uint32_t lane, uint4 (&x0)[kRing], uint4 (&x1)[kRing]) {
+template <int N> __device__ __forceinline__ void turn_token_rows(uint32_t lane, uint4 (&x0)[N], uint4 (&x1)[N]) {
     const uint32_t j = lane & 15, jq = lane >> 4;
     const int pull = (int)((4 * j + jq) * 4);       // operand lane (j, jq) takes what load lane 4 j + jq holds
     auto turn = [&](uint4 &v) {
@@ -142,7 +142,7 @@ __device__ __forceinline__ void turn_token_rows(uint32_t lane, uint4 (&x0)[kRing
         v.w = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)v.w);
     };
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) {
+    for (int u = 0; u < N; ++u) {
         turn(x0[u]);
         turn(x1[u]);
     }
