@@ -139,11 +139,18 @@ __device__ __forceinline__ unsigned long long argmax_key(float v, uint32_t i) {
 struct SoftmaxAcc {
     float m, s;      // m = -inf: nothing seen yet
 };
+// The divisions as reciprocals with a step of Newton's method each: 11 instructions for some 35, and no further off (the quotient's error is
+// below a unit in its last place, the second product and sum round once).
 __device__ __forceinline__ float capped(float v, float softcap) {
     if (!(softcap > 0.0f)) return v;
-    // tanh z = 1 - 2 / (exp(2 z) + 1); exp saturates to inf / 0 cleanly, so large |z| give +-1
-    const float z = v / softcap;
-    return softcap * (1.0f - 2.0f / (__expf(2.0f * z) + 1.0f));
+    // tanh z = 1 - 2 / (exp(2 z) + 1); from z = 40 on (and where v / softcap is no number any more) that is 1
+    const float inv = 1.0f / softcap;
+    float z = fminf(fmaxf(v * inv, -40.0f), 40.0f);
+    z = fminf(__builtin_fmaf(__builtin_fmaf(-z, softcap, v), inv, z), 40.0f);
+    const float d = __expf(2.0f * z) + 1.0f;
+    float r = __builtin_amdgcn_rcpf(d);
+    r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+    return __builtin_fmaf(-2.0f * softcap, r, softcap);
 }
 __device__ __forceinline__ void softmax_take(SoftmaxAcc &a, float v, float softcap) {
     if (!(__builtin_fabsf(v) < INFINITY)) return;          // non-finite logits take no part (they never win either)
@@ -586,26 +593,28 @@ __global__ __launch_bounds__(64 * kBandWaves, PARTS) void matrix_band_kernel(con
     }
 }
 
-// The block's largest key, the same in every thread (WAVES: 4 or 16; a wave's lanes hold all waves' keys several times over).
+// The block's largest key and, if it is wanted, its softmax pair (the largest value first, then the sums relative to it; no NaN comes
+// here), for the threads of its first wave: the others are told to leave. WAVES: 4 or 16; a wave's lanes hold all waves' several times over.
 template <int WAVES>
-__device__ __forceinline__ unsigned long long block_max_key(unsigned long long k, unsigned long long *s_k) {
-    k = wave_max_key(k);
-    if ((threadIdx.x & 63) == 0) s_k[threadIdx.x >> 6] = k;
+__device__ __forceinline__ bool block_choice(unsigned long long &best, SoftmaxAcc &soft, bool conf, unsigned long long *s_k, float2 *s_p) {
+    best = wave_max_key(best);
+    if (conf) {
+        const float m = wave_max_f32(soft.m);
+        soft = SoftmaxAcc{m, wave_butterfly_sum(soft.m > -INFINITY ? soft.s * __expf(soft.m - m) : 0.0f)};
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_k[threadIdx.x >> 6] = best;
+        s_p[threadIdx.x >> 6] = make_float2(soft.m, soft.s);
+    }
     __syncthreads();
-    return wave_max_key(s_k[threadIdx.x & (WAVES - 1)]);
-}
-
-// The block's softmax pair, the same in every thread: the largest value first, then the sums relative to it. (No NaN comes here.)
-template <int WAVES>
-__device__ __forceinline__ SoftmaxAcc block_softmax(SoftmaxAcc a, float2 *s_p) {
-    float m = wave_max_f32(a.m);
-    float s = wave_butterfly_sum(a.m > -INFINITY ? a.s * __expf(a.m - m) : 0.0f);
-    if ((threadIdx.x & 63) == 0) s_p[threadIdx.x >> 6] = make_float2(m, s);
-    __syncthreads();
+    if (threadIdx.x >= 64) return false;
     const float2 own = s_p[threadIdx.x & (WAVES - 1)];
-    m = wave_max_f32(own.x);
-    s = row_butterfly_sum<WAVES>(own.x > -INFINITY ? own.y * __expf(own.x - m) : 0.0f);
-    return SoftmaxAcc{m, s};
+    best = wave_max_key(s_k[threadIdx.x & (WAVES - 1)]);
+    if (conf) {
+        const float m = wave_max_f32(own.x);
+        soft = SoftmaxAcc{m, row_butterfly_sum<WAVES>(own.x > -INFINITY ? own.y * __expf(own.x - m) : 0.0f)};
+    }
+    return true;
 }
 
 // The winner's value from its key (argmax_key is a bijection on the finite values).
@@ -635,12 +644,9 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const unsigned long l
             soft = softmax_merge(soft, SoftmaxAcc{q.x, q.y});
         }
     }
-    best = block_max_key<4>(best, s_k);
-    if (threadIdx.x == 0) out[row] = best ? 0xFFFFFFFFu - (uint32_t)best : 0u;
-    if (out_conf) {
-        soft = block_softmax<4>(soft, s_p);
-        if (threadIdx.x == 0) out_conf[row] = winner_confidence(best, soft, softcap);
-    }
+    if (!block_choice<4>(best, soft, out_conf != nullptr, s_k, s_p) || threadIdx.x != 0) return;
+    out[row] = best ? 0xFFFFFFFFu - (uint32_t)best : 0u;
+    if (out_conf) out_conf[row] = winner_confidence(best, soft, softcap);
 }
 
 // argmax_rows_f32 (Metal/Sampling/logit.metal:946-1010): the greedy choice over rows of fp32 logits that are in
@@ -650,7 +656,8 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const unsigned long l
 // winners argmax_merge_kernel joins. A thread requests eight values before it looks at the first, and adds their
 // exponentials relative to the largest of the eight (value by value it was a chain of exponentials: 16 rows of 4,099 took
 // 10.4 us with 256 threads each, 6.2 us so; 5.2 with waves that skip what lies past the row's end and reductions by register moves
-// instead of through the LDS crossbar; 16 rows of 32,768 in segments: 4.9 + 3.9 us).
+// instead of through the LDS crossbar; 4.6 with caps that divide by reciprocals and one barrier for both reductions; one row of 512 3.3 -> 2.7,
+// of 4,099 4.6 -> 3.8; 16 rows of 32,768 in segments: 4.0 + 2.6 us).
 constexpr int kArgmaxThreads = 1024, kArgmaxBatch = 8;
 constexpr uint32_t kArgmaxOneBlock = 8192;
 
@@ -668,7 +675,7 @@ __global__ __launch_bounds__(THREADS) void argmax_rows_kernel(const float *__res
         float v[kArgmaxBatch];
 #pragma unroll
         for (int u = 0; u < kArgmaxBatch; ++u) v[u] = base + u * THREADS < hi ? row[base + u * THREADS] : NAN;
-        // (a wave past the row's end skips what it does not have: the caps' divisions are what a block of 1,024 threads spends its time on)
+        // (a wave past the row's end skips what it does not have: the caps and exponentials are what a block of 1,024 threads spends its time on)
         const uint32_t wave_base = __builtin_amdgcn_readfirstlane(base & ~63u);
         float m = soft.m;
 #pragma unroll
@@ -691,9 +698,7 @@ __global__ __launch_bounds__(THREADS) void argmax_rows_kernel(const float *__res
             soft = SoftmaxAcc{m, sum};
         }
     }
-    best = block_max_key<THREADS / 64>(best, s_k);
-    if (out_conf) soft = block_softmax<THREADS / 64>(soft, s_p);
-    if (threadIdx.x != 0) return;
+    if (!block_choice<THREADS / 64>(best, soft, out_conf != nullptr, s_k, s_p) || threadIdx.x != 0) return;
     if (segments) {
         SampleSegment seg{};
         seg.best = best;
@@ -713,10 +718,9 @@ __global__ __launch_bounds__(256) void argmax_merge_kernel(const SampleSegment *
     SampleSegment mine{};
     mine.top = -INFINITY;
     if (threadIdx.x < n_seg) mine = segments[(size_t)blockIdx.x * kSampleMaxSegments + threadIdx.x];
-    const unsigned long long best = block_max_key<4>(mine.best, s_k);
+    unsigned long long best = mine.best;
     SoftmaxAcc soft{mine.top, mine.sum};
-    if (out_conf) soft = block_softmax<4>(soft, s_p);
-    if (threadIdx.x != 0) return;
+    if (!block_choice<4>(best, soft, out_conf != nullptr, s_k, s_p) || threadIdx.x != 0) return;
     out[blockIdx.x] = best ? 0xFFFFFFFFu - (uint32_t)best : 0xFFFFFFFFu;
     if (out_conf) out_conf[blockIdx.x] = winner_confidence(best, soft, softcap);
 }
