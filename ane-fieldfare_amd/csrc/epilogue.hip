@@ -8,7 +8,9 @@
 // reference stages rows in threadgroup memory); a row is read once and written once: HBM-bound.
 // Every input row and every weight vector of a launch is requested before the first reduction, so a launch is one
 // memory round trip and its block reductions (a load issued behind a reduction is another dependent round trip, and
-// at 16 rows these kernels are nothing but their round trips).
+// at 16 rows these kernels are nothing but their round trips); no value is converted before the last of a thread's requests
+// is out (beside its load it was waited for, and the second chunk of a row went out a round trip later: setup of 1 row of 2,816 3.16 us, now
+// 3.04; tail of 3,072 rows 16.0 | 15.5, of 8,192 33.1 | 31.3).
 //
 // Summation order of the squares (the reference's simd_sum leaves it open): thread t owns the 8-element
 // chunks t, t + 256, ... and adds their squares in index order with fmaf; the wave meets in a
@@ -44,11 +46,6 @@ __device__ __forceinline__ Row8 widen8(const uint4 &q) {
     r.v[4] = Act<F16>::lo(q.z); r.v[5] = Act<F16>::hi(q.z);
     r.v[6] = Act<F16>::lo(q.w); r.v[7] = Act<F16>::hi(q.w);
     return r;
-}
-
-template <bool VEC, bool F16>
-__device__ __forceinline__ Row8 load8(const uint16_t *__restrict__ row, uint32_t chunk) {
-    return widen8<F16>(load_raw8<VEC>(row, chunk));
 }
 
 // A value on its way to 16 bits is an fp32 number first, as in the reference: left alone, the compiler makes a product and its rounding
@@ -105,16 +102,26 @@ __global__ __launch_bounds__(kRowThreads) void post_attn_setup_kernel(
     const uint32_t n_mine = t < chunks ? (chunks - t + kRowThreads - 1) / kRowThreads : 0;
     uint16_t *hrow = hidden + (size_t)row * hidden_stride;
     const uint16_t *arow = attn + (size_t)row * attn_stride;
-    Row8 a[kMaxChunks], h[kMaxChunks], w0[kMaxChunks], w1[kMaxChunks], w2[kMaxChunks];
+    uint4 a_raw[kMaxChunks], h_raw[kMaxChunks], w0_raw[kMaxChunks], w1_raw[kMaxChunks], w2_raw[kMaxChunks];
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c)
         if ((uint32_t)c < n_mine) {
-            a[c] = load8<VEC, F16>(arow, t + c * kRowThreads);
-            h[c] = load8<VEC, F16>(hrow, t + c * kRowThreads);
-            w0[c] = load8<VEC, false>(w_post_attn, t + c * kRowThreads);
-            w1[c] = load8<VEC, false>(w_pre_ffn, t + c * kRowThreads);
-            w2[c] = load8<VEC, false>(w_pre_ffn2, t + c * kRowThreads);
+            const uint32_t chunk = t + c * kRowThreads;
+            a_raw[c] = load_raw8<VEC>(arow, chunk);
+            h_raw[c] = load_raw8<VEC>(hrow, chunk);
+            w0_raw[c] = load_raw8<VEC>(w_post_attn, chunk);
+            w1_raw[c] = load_raw8<VEC>(w_pre_ffn, chunk);
+            w2_raw[c] = load_raw8<VEC>(w_pre_ffn2, chunk);
         }
+    Row8 a[kMaxChunks], h[kMaxChunks], w0[kMaxChunks], w1[kMaxChunks], w2[kMaxChunks];
+#pragma unroll
+    for (int c = 0; c < kMaxChunks; ++c) {
+        a[c] = widen8<F16>(a_raw[c]);
+        h[c] = widen8<F16>(h_raw[c]);
+        w0[c] = widen8<false>(w0_raw[c]);
+        w1[c] = widen8<false>(w1_raw[c]);
+        w2[c] = widen8<false>(w2_raw[c]);
+    }
     const float attn_inv = block_rms_inv(a, n_mine, d, eps, s_sum[0]);
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c)
@@ -289,18 +296,29 @@ __global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer
             wf[c] = widen8<false>(wf_raw[c]);
         }
     } else {
+        uint4 a_raw[kMaxChunks], h1_raw[kMaxChunks], h_raw[kMaxChunks], wf2_raw[kMaxChunks], wf_raw[kMaxChunks], wf1_raw[kMaxChunks], wn_raw[kMaxChunks];
 #pragma unroll
         for (int c = 0; c < kMaxChunks; ++c)
             if ((uint32_t)c < n_mine) {
                 const uint32_t chunk = t + c * kRowThreads;
-                a[c] = load8<VEC, F16>(h2 + (size_t)row * h2_stride, chunk);
-                h12[c] = load8<VEC, F16>(h1 + (size_t)row * h1_stride, chunk);
-                hv[c] = load8<VEC, F16>(hrow, chunk);
-                wf2[c] = load8<VEC, false>(w_postffn2, chunk);
-                wf[c] = load8<VEC, false>(w_postffn, chunk);
-                if (NORMS) wf1[c] = load8<VEC, false>(w_postffn1, chunk);
-                if (NORMS && w_next) wn[c] = load8<VEC, false>(w_next, chunk);
+                a_raw[c] = load_raw8<VEC>(h2 + (size_t)row * h2_stride, chunk);
+                h1_raw[c] = load_raw8<VEC>(h1 + (size_t)row * h1_stride, chunk);
+                h_raw[c] = load_raw8<VEC>(hrow, chunk);
+                wf2_raw[c] = load_raw8<VEC>(w_postffn2, chunk);
+                wf_raw[c] = load_raw8<VEC>(w_postffn, chunk);
+                if (NORMS) wf1_raw[c] = load_raw8<VEC>(w_postffn1, chunk);
+                if (NORMS) wn_raw[c] = load_raw8<VEC>(w_next ? w_next : w_postffn1, chunk);
             }
+#pragma unroll
+        for (int c = 0; c < kMaxChunks; ++c) {
+            a[c] = widen8<F16>(a_raw[c]);
+            h12[c] = widen8<F16>(h1_raw[c]);
+            hv[c] = widen8<F16>(h_raw[c]);
+            wf2[c] = widen8<false>(wf2_raw[c]);
+            wf[c] = widen8<false>(wf_raw[c]);
+            if (NORMS) wf1[c] = widen8<false>(wf1_raw[c]);
+            if (NORMS) wn[c] = widen8<false>(wn_raw[c]);
+        }
     }
     if (NORMS) {
         const float inv_h1 = block_rms_inv(h12, n_mine, d, eps, s_sum[2]);
@@ -352,13 +370,19 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t *x,
     __shared__ float s_sum[4];
     const uint32_t row = blockIdx.x, t = threadIdx.x, chunks = d / 8;
     const uint32_t n_mine = t < chunks ? (chunks - t + kRowThreads - 1) / kRowThreads : 0;
-    Row8 a[kMaxChunks], wq[kMaxChunks];
+    uint4 a_raw[kMaxChunks], w_raw[kMaxChunks];
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c)
         if ((uint32_t)c < n_mine) {
-            a[c] = load8<VEC, F16>(x + (size_t)row * x_stride, t + c * kRowThreads);
-            wq[c] = load8<VEC, false>(w, t + c * kRowThreads);
+            a_raw[c] = load_raw8<VEC>(x + (size_t)row * x_stride, t + c * kRowThreads);
+            w_raw[c] = load_raw8<VEC>(w, t + c * kRowThreads);
         }
+    Row8 a[kMaxChunks], wq[kMaxChunks];
+#pragma unroll
+    for (int c = 0; c < kMaxChunks; ++c) {
+        a[c] = widen8<F16>(a_raw[c]);
+        wq[c] = widen8<false>(w_raw[c]);
+    }
     const float inv = block_rms_inv(a, n_mine, d, eps, s_sum);
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c)
