@@ -93,10 +93,10 @@ __device__ __forceinline__ float block_rms_inv(const Row8 (&x)[kMaxChunks], uint
 
 template <bool VEC, bool F16>
 __global__ __launch_bounds__(kRowThreads) void post_attn_setup_kernel(
-    uint16_t *__restrict__ hidden, uint32_t hidden_stride, const uint16_t *__restrict__ attn, uint32_t attn_stride,
-    uint16_t *__restrict__ dense_x, uint32_t dense_stride, uint16_t *__restrict__ routed_x, uint32_t routed_stride,
-    uint16_t *__restrict__ router_x, uint32_t router_stride, const uint16_t *__restrict__ w_post_attn,
-    const uint16_t *__restrict__ w_pre_ffn, const uint16_t *__restrict__ w_pre_ffn2, uint32_t d, float eps) {
+    uint16_t *__restrict__ hidden, const uint16_t *__restrict__ attn, const uint16_t *__restrict__ w_post_attn, uint32_t hidden_stride,
+    uint32_t attn_stride, uint32_t d, float eps, const uint16_t *__restrict__ w_pre_ffn, const uint16_t *__restrict__ w_pre_ffn2,
+    uint16_t *__restrict__ dense_x, uint16_t *__restrict__ routed_x, uint16_t *__restrict__ router_x, uint32_t dense_stride,
+    uint32_t routed_stride, uint32_t router_stride) {
     __shared__ float s_sum[2][4];
     const uint32_t row = blockIdx.x, t = threadIdx.x, chunks = d / 8;
     const uint32_t n_mine = t < chunks ? (chunks - t + kRowThreads - 1) / kRowThreads : 0;
@@ -238,12 +238,11 @@ __device__ __forceinline__ Row8 combine8(const RoutedChunk &in, uint32_t top_k, 
 // 256th hand their chunks, rounded to 16 bits as they are, to the threads that own them in the order of the sums. 1 row of
 // 2,816, us per launch: both chunks by their owner, each behind its own chain of loads 5.9, so 4.6.
 template <bool VEC, bool NORMS, bool F16, bool COMBINE = false>
-__global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer_tail_kernel(const uint16_t *__restrict__ h2, uint32_t h2_stride,
-                                                                 const uint16_t *__restrict__ h1, uint32_t h1_stride,
-                                                                 uint16_t *__restrict__ hidden, uint32_t hidden_stride,
+__global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer_tail_kernel(const uint16_t *__restrict__ h1, uint16_t *__restrict__ hidden,
                                                                  const uint16_t *__restrict__ w_postffn2,
-                                                                 const uint16_t *__restrict__ w_postffn, uint32_t d,
-                                                                 float eps, float layer_scalar,
+                                                                 const uint16_t *__restrict__ w_postffn,
+                                                                 const uint16_t *__restrict__ h2, uint32_t h2_stride, uint32_t h1_stride,
+                                                                 uint32_t hidden_stride, uint32_t d, float eps, float layer_scalar,
                                                                  const uint16_t *__restrict__ w_postffn1,
                                                                  const uint16_t *__restrict__ w_next,
                                                                  uint16_t *__restrict__ normed, uint32_t normed_stride,
@@ -257,8 +256,6 @@ __global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer
         // every load before the first use of one: converted beside their loads, a thread's chunks were a round trip each
         __shared__ uint4 handed[2][kRowThreads];        // h2, h1: chunks 256 .. 511
         const bool h1_given = !routed.shared_partials;
-        const uint32_t route = row * routed.top_k + min(t & 63, routed.top_k - 1);
-        const uint32_t weight = routed.w[route], valid = routed.route_valid[route];
         uint4 h1_raw[kMaxChunks], h_raw[kMaxChunks], wf2_raw[kMaxChunks], wf_raw[kMaxChunks];
 #pragma unroll
         for (int c = 0; c < kMaxChunks; ++c)
@@ -269,6 +266,8 @@ __global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer
                 wf2_raw[c] = load_raw8<VEC>(w_postffn2, chunk);
                 wf_raw[c] = load_raw8<VEC>(w_postffn, chunk);
             }
+        const uint32_t route = row * routed.top_k + min(t & 63, routed.top_k - 1);
+        const uint32_t weight = routed.w[route], valid = routed.route_valid[route];
         uint4 h2_raw = {0, 0, 0, 0};
         if (t < chunks) {
             const RoutedChunk in = load_routed(routed, row, d, t);
@@ -409,9 +408,8 @@ hipError_t launch_post_attn_setup(hipStream_t s, uint16_t *hidden, uint32_t hidd
                      aligned16(routed_x, routed_stride) && aligned16(router_x, router_stride) && aligned16(w_post_attn, 8) &&
                      aligned16(w_pre_ffn, 8) && aligned16(w_pre_ffn2, 8);
 #define FFMOE_SETUP(V, H)                                                                                                  \
-    hipLaunchKernelGGL((post_attn_setup_kernel<V, H>), dim3(t), dim3(kRowThreads), 0, s, hidden, hidden_stride, attn, attn_stride, \
-                       dense_x, dense_stride, routed_x, routed_stride, router_x, router_stride, w_post_attn, w_pre_ffn,       \
-                       w_pre_ffn2, d, eps)
+    hipLaunchKernelGGL((post_attn_setup_kernel<V, H>), dim3(t), dim3(kRowThreads), 0, s, hidden, attn, w_post_attn, hidden_stride, attn_stride, \
+                       d, eps, w_pre_ffn, w_pre_ffn2, dense_x, routed_x, router_x, dense_stride, routed_stride, router_stride)
     if (f16) { if (vec) FFMOE_SETUP(true, true); else FFMOE_SETUP(false, true); }
     else { if (vec) FFMOE_SETUP(true, false); else FFMOE_SETUP(false, false); }
 #undef FFMOE_SETUP
@@ -431,8 +429,8 @@ hipError_t launch_layer_tail(hipStream_t s, const uint16_t *h2, uint32_t h2_stri
         // h2 is made from the un-combined rows (16-byte aligned fp32 rows: d % 8 == 0); the plain tail only
         const bool vec = (shared_partials || aligned16(h1, h1_stride)) && aligned16(hidden, hidden_stride) && aligned16(w_postffn2, 8) && aligned16(w_postffn, 8);
 #define FFMOE_TAILC(V, H)                                                                                             \
-    hipLaunchKernelGGL((layer_tail_kernel<V, false, H, true>), dim3(t), dim3(d / 8 > kRowThreads ? 2 * kRowThreads : kRowThreads), 0, s, nullptr, 0u, h1, h1_stride, \
-                       hidden, hidden_stride, w_postffn2, w_postffn, d, eps, layer_scalar, nullptr, nullptr, nullptr, 0u, routed)
+    hipLaunchKernelGGL((layer_tail_kernel<V, false, H, true>), dim3(t), dim3(d / 8 > kRowThreads ? 2 * kRowThreads : kRowThreads), 0, s, h1, hidden, \
+                       w_postffn2, w_postffn, nullptr, 0u, h1_stride, hidden_stride, d, eps, layer_scalar, nullptr, nullptr, nullptr, 0u, routed)
         if (f16) { if (vec) FFMOE_TAILC(true, true); else FFMOE_TAILC(false, true); }
         else { if (vec) FFMOE_TAILC(true, false); else FFMOE_TAILC(false, false); }
 #undef FFMOE_TAILC
@@ -444,12 +442,12 @@ hipError_t launch_layer_tail(hipStream_t s, const uint16_t *h2, uint32_t h2_stri
 #define FFMOE_TAIL(V, N)                                                                                              \
     do {                                                                                                              \
         if (f16)                                                                                                      \
-            hipLaunchKernelGGL((layer_tail_kernel<V, N, true>), dim3(t), dim3(kRowThreads), 0, s, h2, h2_stride, h1, h1_stride, \
-                               hidden, hidden_stride, w_postffn2, w_postffn, d, eps, layer_scalar, w_postffn1, w_next, normed, \
+            hipLaunchKernelGGL((layer_tail_kernel<V, N, true>), dim3(t), dim3(kRowThreads), 0, s, h1, hidden, w_postffn2, \
+                               w_postffn, h2, h2_stride, h1_stride, hidden_stride, d, eps, layer_scalar, w_postffn1, w_next, normed, \
                                normed_stride, routed);                                                                \
         else                                                                                                          \
-            hipLaunchKernelGGL((layer_tail_kernel<V, N, false>), dim3(t), dim3(kRowThreads), 0, s, h2, h2_stride, h1, h1_stride, \
-                               hidden, hidden_stride, w_postffn2, w_postffn, d, eps, layer_scalar, w_postffn1, w_next, normed, \
+            hipLaunchKernelGGL((layer_tail_kernel<V, N, false>), dim3(t), dim3(kRowThreads), 0, s, h1, hidden, w_postffn2, \
+                               w_postffn, h2, h2_stride, h1_stride, hidden_stride, d, eps, layer_scalar, w_postffn1, w_next, normed, \
                                normed_stride, routed);                                                                \
     } while (0)
     if (vec) { if (norms) FFMOE_TAIL(true, true); else FFMOE_TAIL(true, false); }

@@ -1288,14 +1288,12 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
 
 // MAX_NM: 16-pair blocks of the largest tile the plan cut
 template <bool GATE_UP, int MAX_NM, bool F16, int WAVES>
-__global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
-                                                                    const PrefillPlan *__restrict__ plan,
-                                                                    const PrefillTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const PrefillPlan *__restrict__ plan, const PrefillTile *__restrict__ tiles,
+                                                                    uint32_t n_nblocks, bool nb_major, const uint8_t *__restrict__ arena_layer,
                                                                     const uint32_t *__restrict__ sorted_token,
-                                                                    const uint32_t *__restrict__ sorted_out_row,
-                                                                    const uint16_t *__restrict__ a, uint32_t a_stride,
-                                                                    uint16_t *__restrict__ out, uint32_t n_nblocks, bool nb_major,
-                                                                    float *__restrict__ act_scale, uint32_t act_blocks) {
+                                                                    const uint16_t *__restrict__ a, uint32_t a_stride, uint32_t act_blocks,
+                                                                    ArenaGeom g, const uint32_t *__restrict__ sorted_out_row,
+                                                                    uint16_t *__restrict__ out, float *__restrict__ act_scale) {
     __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave + 2 * MAX_NM * kStreamChunk * 16 / 4];
     uint32_t ti, nb;
     if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;
@@ -1699,8 +1697,8 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
         else FFMOE_GEMM_LC(GU, A, STRIDE, OUT, NB, 4);                                                                        \
     } while (0)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
-    hipLaunchKernelGGL(stream_kernel<GU>(tile_rows, f16), dim3(grid_of(NB)), dim3(256), 0, s, arena_layer, g, sc.plan,  \
-                       sc.tiles, sc.sorted_token, sc.sorted_out_row, A, STRIDE, OUT, NB, nb_major, act_scale, act_blocks)
+    hipLaunchKernelGGL(stream_kernel<GU>(tile_rows, f16), dim3(grid_of(NB)), dim3(256), 0, s, sc.plan, sc.tiles, NB,    \
+                       nb_major, arena_layer, sc.sorted_token, A, STRIDE, act_blocks, g, sc.sorted_out_row, OUT, act_scale)
     if (large_scales) {
         if ((e = launch_prefill_large_scale(s, arena_layer, g, true, tile_cap, x, x_stride, sc.acts, sc, f16)) != hipSuccess) return e;
     } else if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);

@@ -611,13 +611,12 @@ __device__ __forceinline__ void lone_wave_keys(const void *__restrict__ router_w
 
 template <bool W_F32, bool F16, int SHARED>
 __global__ __launch_bounds__(256, 2) void route_gate_up_persistent(
-    const uint8_t *__restrict__ arena_layer, ArenaGeom g, uint32_t top_k, uint32_t n_experts, const void *__restrict__ router_w,
-    const uint16_t *__restrict__ effective_scale, const uint16_t *__restrict__ per_expert_scale,
-    const uint16_t *__restrict__ router_x, uint32_t router_x_stride, uint32_t rows, RouteMail *__restrict__ mail,
-    unsigned long long poll_ticks,
-    uint32_t *__restrict__ out_idx, uint16_t *__restrict__ out_w, VerifyPlan *__restrict__ plan,
-    const uint16_t *__restrict__ x, uint32_t x_stride, uint16_t *__restrict__ acts, SharedArg<SHARED, SharedGateUp> sh,
-    uint32_t prefetch_blocks) {
+    RouteMail *__restrict__ mail, const void *__restrict__ router_w, const uint16_t *__restrict__ router_x,
+    const uint16_t *__restrict__ effective_scale, uint32_t router_x_stride, uint32_t rows, uint32_t n_experts, uint32_t top_k,
+    uint32_t d, uint32_t prefetch_blocks, const uint16_t *__restrict__ x, uint32_t x_stride, ArenaGeom g,
+    const uint8_t *__restrict__ arena_layer, const uint16_t *__restrict__ per_expert_scale, unsigned long long poll_ticks,
+    uint32_t *__restrict__ out_idx, uint16_t *__restrict__ out_w, VerifyPlan *__restrict__ plan, uint16_t *__restrict__ acts,
+    SharedArg<SHARED, SharedGateUp> sh) {
     __shared__ GateUpMerge s_red;
     __shared__ PlanScratch ps;
     float(*s_part)[kChunkTokens][64] = reinterpret_cast<float(*)[kChunkTokens][64]>(&s_red[0][0][0][0]);   // 4 KiB of the 16
@@ -632,7 +631,7 @@ __global__ __launch_bounds__(256, 2) void route_gate_up_persistent(
         const uint32_t e = item % n_experts, t0 = (item / n_experts) * kChunkTokens;
         const uint32_t t_end = min(rows, t0 + kChunkTokens);
         float acc[kChunkTokens] = {0.f, 0.f, 0.f, 0.f};
-        accumulate_sub<W_F32, F16 ? 2 : 1>(router_w, effective_scale, router_x, router_x_stride, e, g.d, ks, lane, t0, t_end - 1, acc);
+        accumulate_sub<W_F32, F16 ? 2 : 1>(router_w, effective_scale, router_x, router_x_stride, e, d, ks, lane, t0, t_end - 1, acc);
         if (item != blockIdx.x) __syncthreads();      // the previous item's partials have been read
 #pragma unroll
         for (int r = 0; r < kChunkTokens; ++r) s_part[ks][r][lane] = acc[r];
@@ -726,7 +725,7 @@ __global__ __launch_bounds__(256, 2) void route_gate_up_persistent(
                 // the row's logits are not coming (a block that makes them is not running): this wave makes them itself
                 if (lane == 0 && ks == 1) atomicAdd(&mail->faults, 1u);
                 uint32_t keys[kChunkTokens][4];
-                lone_wave_keys<W_F32, F16>(router_w, effective_scale, router_x, router_x_stride, n_experts, g.d, row, row, lane, keys);
+                lone_wave_keys<W_F32, F16>(router_w, effective_scale, router_x, router_x_stride, n_experts, d, row, row, lane, keys);
 #pragma unroll
                 for (int c = 0; c < 4; ++c) tr.key[c] = keys[0][c];
                 break;
@@ -769,7 +768,7 @@ __global__ __launch_bounds__(256, 2) void route_gate_up_persistent(
                 const uint32_t my_row = threadIdx.x / top_k, my_rank = threadIdx.x % top_k;
                 for (uint32_t t0 = r_first; t0 <= r_last; t0 += kChunkTokens) {
                     uint32_t keys[kChunkTokens][4];
-                    lone_wave_keys<W_F32, F16>(router_w, effective_scale, router_x, router_x_stride, n_experts, g.d, t0,
+                    lone_wave_keys<W_F32, F16>(router_w, effective_scale, router_x, router_x_stride, n_experts, d, t0,
                                                min(t0 + kChunkTokens - 1, rows - 1), lane, keys);
 #pragma unroll
                     for (int i = 0; i < kChunkTokens; ++i) {
@@ -831,11 +830,10 @@ struct SharedDown {
 };
 
 template <bool OUT_BF16, bool F16, bool SHARED>
-__global__ __launch_bounds__(256, 5) void skinny_down_lds(const uint8_t *__restrict__ arena_layer, ArenaGeom g,
-                                                          const VerifyPlan *__restrict__ plan,
-                                                          const uint16_t *__restrict__ acts,
+__global__ __launch_bounds__(256, 5) void skinny_down_lds(const VerifyPlan *__restrict__ plan, const uint16_t *__restrict__ acts,
+                                                          const uint8_t *__restrict__ arena_layer, RouteMail *mail, uint32_t parts,
                                                           float *__restrict__ partials_f32,
-                                                          uint16_t *__restrict__ partials_bf16, uint32_t parts, RouteMail *mail,
+                                                          uint16_t *__restrict__ partials_bf16, ArenaGeom g,
                                                           SharedArg<SHARED, SharedDown> sh_arg) {
     SharedDown sh{nullptr, g, nullptr, nullptr, 0xFFFFFFFFu, 0u, nullptr, nullptr};
     if constexpr (SHARED) sh = sh_arg;
@@ -1294,11 +1292,10 @@ hipError_t launch_verify_as(hipStream_t s, const uint8_t *arena_layer, ArenaGeom
             blocks = (blocks + 7) / 8 * 8 + prefetch_blocks;       // the spare blocks start on XCD 0 (blocks go to XCDs round robin)
         }
 #define FFMOE_ROUTE_GU(WF, SH)                                                                                              \
-    hipLaunchKernelGGL((route_gate_up_persistent<WF, F16, SH>), dim3(blocks), dim3(256), 0, s, arena_layer, g, top_k, n_experts, \
-                       route->rw.w, route->rw.effective_scale, route->rw.per_expert_scale, route->router_x,                  \
-                       route->router_x_stride, t, route->mail, route->poll_ticks, const_cast<uint32_t *>(idx),                \
-                       const_cast<uint16_t *>(w), plan,                                                                     \
-                       x, x_stride, acts, shared_arg<SH>(sh_gu), prefetch_blocks)
+    hipLaunchKernelGGL((route_gate_up_persistent<WF, F16, SH>), dim3(blocks), dim3(256), 0, s, route->mail, route->rw.w,         \
+                       route->router_x, route->rw.effective_scale, route->router_x_stride, t, n_experts, top_k, g.d, prefetch_blocks, \
+                       x, x_stride, g, arena_layer, route->rw.per_expert_scale, route->poll_ticks, const_cast<uint32_t *>(idx),  \
+                       const_cast<uint16_t *>(w), plan, acts, shared_arg<SH>(sh_gu))
         if (shared8) { if (route->rw.w_is_f32) FFMOE_ROUTE_GU(true, 2); else FFMOE_ROUTE_GU(false, 2); }
         else if (shared) { if (route->rw.w_is_f32) FFMOE_ROUTE_GU(true, 1); else FFMOE_ROUTE_GU(false, 1); }
         else { if (route->rw.w_is_f32) FFMOE_ROUTE_GU(true, 0); else FFMOE_ROUTE_GU(false, 0); }
@@ -1359,11 +1356,11 @@ hipError_t launch_verify_as(hipStream_t s, const uint8_t *arena_layer, ArenaGeom
                                      : dim3((g.dn_rbp + 3) / 4, slots);
 #define FFMOE_DOWN(BF)                                                                                                \
     if (dn_whole && shared)                                                                                           \
-        hipLaunchKernelGGL((skinny_down_lds<BF, F16, true>), dn_grid, dim3(256), 0, s, arena_layer, g, plan, acts,    \
-                           partials_f32, partials_bf16, dn_parts, rows_only ? mail : nullptr, sh_dn);                  \
+        hipLaunchKernelGGL((skinny_down_lds<BF, F16, true>), dn_grid, dim3(256), 0, s, plan, acts, arena_layer,         \
+                           rows_only ? mail : nullptr, dn_parts, partials_f32, partials_bf16, g, sh_dn);                    \
     else if (dn_whole)                                                                                                \
-        hipLaunchKernelGGL((skinny_down_lds<BF, F16, false>), dn_grid, dim3(256), 0, s, arena_layer, g, plan, acts,   \
-                           partials_f32, partials_bf16, dn_parts, rows_only ? mail : nullptr, NoSharedExpert{});       \
+        hipLaunchKernelGGL((skinny_down_lds<BF, F16, false>), dn_grid, dim3(256), 0, s, plan, acts, arena_layer,         \
+                           rows_only ? mail : nullptr, dn_parts, partials_f32, partials_bf16, g, NoSharedExpert{});         \
     else if (dn_ksplit && dense_ksplit)                                                                               \
         hipLaunchKernelGGL((skinny_down_ksplit_persistent<BF, F16, true>), dn_grid, dim3(256), 0, s, arena_layer, g,  \
                            plan, acts, partials_f32, partials_bf16, t);                                               \
