@@ -1132,26 +1132,29 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *__restrict__ 
     const uint32_t tok = blockIdx.y;
     if (mail && blockIdx.x == 0 && tok == 0 && threadIdx.x == 0) advance_epoch(mail);      // the routing launch of this call has read it
     const uint32_t c = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (c >= d) return;
-    // One round trip: the routes' weights and validity and all eight rows are requested together. A row the plan
+    // One round trip: the routes' weights and validity, all eight rows and the residual are requested together. A row the plan
     // skipped was never written and may hold anything: it is loaded like the others and dropped by the select below
-    // (its address is inside the buffer either way), instead of being asked for only once its validity has arrived.
-    float wv[8];
-    uint32_t valid[8];
+    // (its address is inside the buffer either way), instead of being asked for only once its validity has arrived. Weights and
+    // validity come as one load each, a route per lane (the token is the block's: read route by route they were scalar loads that
+    // the compiler put behind the rows); without a residual the first row's bytes stand in for it. A verify step of
+    // 16 rows of 2,816 49.3 us, so 49.0.
+    const uint32_t my_route = tok * top_k + min(threadIdx.x & 63, top_k - 1);
+    const uint32_t w_lane = w[my_route], valid_lane = plan->route_valid[my_route];
+    if (c >= d) return;
     f32x4 p[8];
 #pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) {
-        const uint32_t route = tok * top_k + min(r, top_k - 1);
-        wv[r] = Act<F16>::widen(w[route]);
-        valid[r] = plan->route_valid[route];
-        p[r] = *reinterpret_cast<const f32x4 *>(partials + (size_t)route * d + c);
-    }
+    for (uint32_t r = 0; r < 8; ++r) p[r] = *reinterpret_cast<const f32x4 *>(partials + (size_t)(tok * top_k + min(r, top_k - 1)) * d + c);
+    const uint2 rv = *(residual ? reinterpret_cast<const uint2 *>(residual + (size_t)tok * d + c)
+                                : reinterpret_cast<const uint2 *>(partials + (size_t)tok * top_k * d + c));
+    float wv[8];
     bool live[8];
 #pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) live[r] = r < top_k && valid[r] != 0;
+    for (uint32_t r = 0; r < 8; ++r) {
+        wv[r] = Act<F16>::widen((uint16_t)__builtin_amdgcn_readlane((int)w_lane, (int)r));
+        live[r] = r < top_k && __builtin_amdgcn_readlane((int)valid_lane, (int)r) != 0;
+    }
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     if (residual) {
-        const uint2 rv = *reinterpret_cast<const uint2 *>(residual + (size_t)tok * d + c);
         acc[0] = Act<F16>::lo(rv.x); acc[1] = Act<F16>::hi(rv.x);
         acc[2] = Act<F16>::lo(rv.y); acc[3] = Act<F16>::hi(rv.y);
     }
