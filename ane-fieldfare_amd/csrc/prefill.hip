@@ -1537,13 +1537,21 @@ uint32_t gemm_tile_rows(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g
 // bits: a chunk that had the smaller error keeps it.)
 // Skewed routes move nothing: at the first shape with Zipf popularity of exponent 0.6, 1.1 and 1.6 the streaming form wins at
 // every size up to 48 pairs (448 rows 146 | 159 | 166 against 186 | 201 | 196 for the GEMMs, 768 rows 192 | 201 | 212 against 225 |
-// 226 | 232). Tiles of 16 pairs gain nothing over 32 (37 rows: 99), tiles of 128 lose everywhere (1,000 rows: 227, two waves per
-// SIMD).
+// 226 | 232). Tiles of 128 lose everywhere (1,000 rows: 227, two waves per SIMD).
+// Tiles of 16 pairs leave room for six blocks per compute unit (80 registers; FP16's epilogue does not fit them, and five blocks gain
+// nothing): up to some five pairs per expert, where a tile from every expert is more blocks than four per unit and no more than six. Then
+// a launch is one round instead of one and a part of one. us of the call at 32 | 16, bf16: 128 experts of 2,816 x 704, 17 rows 69.9 | 65.3,
+// 24 rows 86 | 80.5, 37 rows 92.9 | 92.6, 64 rows 99.8 | 97.2, Zipf of exponent 1.1 48 rows 77.9 | 73.5, 80 rows 93.5 | 91.4, 128 rows (8
+// pairs) 100.7 | 105.3; 64 of 2,048 x 1,408, 17 rows 58.7 | 56.4, 40 rows 67.6 | 66.9; 80 of 4,096 x 1,024, top-4, 80 rows 122 | 114. Past six
+// blocks 256 of 2,816 x 704, 40 rows 125 | 127.5, 256 of 1,024 x 512, Zipf, 120 rows 44.0 | 46.0; below four 8 of 4,096 x 1,536, top-2, 18 rows
+// 33.3 | 34.9, 64 of 2,048 x 704, Zipf, 64 rows 43.2 | 44.2.
 struct TileForm {
     bool streamed;
     uint32_t rows;
 };
 TileForm prefill_tile_form(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, uint32_t max_tiles, bool f16) {
+    // (a scratch holds 2.5 tiles per expert)
+    if (!f16 && n_items <= 5 * n_experts && n_nblocks * n_experts > 4 * n_cus && n_nblocks * n_experts <= 6 * n_cus) return {true, 16};
     if (n_items <= 28 * n_experts) return {true, 32};
     if (n_items <= kPrefillStreamPairs * n_experts) {
         if (n_nblocks * n_experts <= n_cus) return {true, 32};
@@ -1587,6 +1595,7 @@ TileForm dense_tile_form(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, uin
 
 template <bool GATE_UP>
 auto stream_kernel(uint32_t tile_rows, bool f16) {
+    if (tile_rows == 16) return prefill_stream_kernel<GATE_UP, 1, false, 6>;           // (bf16 alone: prefill_tile_form)
     if (tile_rows == 32) return f16 ? prefill_stream_kernel<GATE_UP, 2, true, 4> : prefill_stream_kernel<GATE_UP, 2, false, 4>;
     return f16 ? prefill_stream_kernel<GATE_UP, 4, true, 3> : prefill_stream_kernel<GATE_UP, 4, false, 3>;
 }

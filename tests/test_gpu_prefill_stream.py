@@ -20,13 +20,13 @@ def _routes(rng, counts, e):
 
 # d, f: (groups of d, groups of f) = whole pairs of chunks, one ragged chunk, three groups past a pair; 320 columns = 2.5 N-blocks
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
-@pytest.mark.parametrize("d,f,scale", [(256, 128, 1), (320, 192, 1), (448, 64, 2), (64, 704, 2), (320, 704, 1.5)])
+@pytest.mark.parametrize("d,f,scale", [(256, 128, 1), (320, 192, 1), (448, 64, 2), (64, 704, 2), (320, 704, 1.5), (192, 576, 9)])
 def test_tile_edges_against_the_oracle(oracle, act, d, f, scale):
     import torch
     import fieldfare_moe as ff
     ff.lib()
     # scale 1: 44 pairs per expert on average, 2: 22 (tiles of 32); 1.5: 29.5 and eleven N-blocks, more blocks than compute
-    # units (tiles of 64)
+    # units (tiles of 64); 9: 4.9 pairs and nine N-blocks, a tile of each expert between four and six blocks per unit (bf16: tiles of 16)
     e = int(len(COUNTS) * scale)
     counts = np.array(COUNTS + (0,) * (e - len(COUNTS)))
     rng, pool, _ = make_layer(oracle, 77 + d, d, f, e, align=1)
