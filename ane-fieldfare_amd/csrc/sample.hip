@@ -75,6 +75,26 @@ struct SampleShared {
     uint32_t n_above, bin, above;
 };
 
+// How many lanes below this one have their bit set.
+__device__ __forceinline__ uint32_t lanes_in_front(unsigned long long mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Lane l: the sum over lanes 0 .. l (register moves; a shift by __shfl_up is a trip through LDS at each of the six steps).
+__device__ __forceinline__ float wave_running_sum(float v) {
+    auto from = [](float x, auto ctrl, auto rows) {
+        return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), decltype(ctrl)::value, decltype(rows)::value, 0xF, false));
+    };
+    using std::integral_constant;
+    v += from(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});   // row_shr:1, 2, 4, 8: sums inside a row of 16
+    v += from(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+    v += from(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+    v += from(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+    v += from(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});   // row_bcast:15 into rows 1 and 3
+    v += from(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});   // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 __device__ __forceinline__ float block_max_f(float v, SampleShared &sh) {
     v = wave_max_f32(v);
     __syncthreads();
@@ -174,8 +194,14 @@ __device__ __forceinline__ void sample_finish(SampleShared &sh, const SampleRule
         at[u] = sh.sorted_i[rank];
     }
     const float top = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(v[0])));
-    float share[kSlots], incl[kSlots];
+    float share[kSlots], incl[kSlots], score[kSlots];
     float so_far = 0.0f;
+    // (also of those that the prefix leaves out: beside its chain instead of behind it)
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+        if (64u * u >= n) break;
+        score[u] = v[u] * invT + sample_gumbel(seed, key, ids ? ids[at[u]] : at[u]);
+    }
 #pragma unroll
     for (int u = 0; u < kSlots; ++u) {
         share[u] = 64u * u + lane < n ? expf(v[u] - p.softcap) / total1 : 0.0f;
@@ -184,13 +210,8 @@ __device__ __forceinline__ void sample_finish(SampleShared &sh, const SampleRule
 #pragma unroll
     for (int u = 0; u < kSlots; ++u) {
         if (64u * u >= n) break;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const float up = __shfl_up(incl[u], o, 64);
-            if (lane >= (uint32_t)o) incl[u] += up;
-        }
-        incl[u] += so_far;
-        so_far = __shfl(incl[u], 63, 64);
+        incl[u] = wave_running_sum(incl[u]) + so_far;
+        so_far = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(incl[u]), 63));
     }
     // The prefix is defined by the running sum that takes the shares one after the other. Two orders of adding <= 256
     // positive shares that add to at most about 1 differ by less than 256 * 2^-24 * 2: where no prefix sum comes closer to
@@ -226,7 +247,7 @@ __device__ __forceinline__ void sample_finish(SampleShared &sh, const SampleRule
         unsigned long long mine = 0ull;
         if (rank < keep) {
             e = expf((v[u] - top) * invT);
-            mine = ((unsigned long long)sample_key(v[u] * invT + sample_gumbel(seed, key, ids ? ids[at[u]] : at[u])) << 32) | (0xFFFFFFFFu - rank);
+            mine = ((unsigned long long)sample_key(score[u]) << 32) | (0xFFFFFFFFu - rank);
         }
         mine = wave_max_key(mine);
         esum += wave_butterfly_sum(e);
@@ -393,7 +414,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(const float
 // ---- long rows: one sweep by many blocks, then one block per row -------------------------------------------------
 // Bound: the sweep is instruction issue (one tanhf and one expf, or the noise's two logf and 64-bit products, per logit),
 // spread over 128 blocks per full-vocabulary row; the second launch is a chain of round trips to memory and LDS, which is why its
-// reductions are register moves: 262,144 logits, the 64 largest, 5.2 + 12.1 us with shuffles and the bound found bit by bit, now 4.8 + 10.9.
+// reductions are register moves: 262,144 logits, the 64 largest, 5.2 + 12.1 us with shuffles and the bound found bit by bit, then 4.6 +
+// 9.8, now 4.6 + 8.2: a wave takes its places in a list with one atomic (one per slot: 1.1 us), the raw bound is one wave's, the running sum
+// of the shares register moves with the noise beside it. The stages then, of 8.2: keys and sums 1.2, bound 2.0, list 0.8, candidates 1.6, caps
+// and ranks 0.9, draw 0.9.
 static_assert(kSampleMaxSegments <= kSampleThreads, "the finishing launches bring one segment per thread");
 constexpr int kScanThreads = 256, kScanPer = kSampleSegment / kScanThreads;
 static_assert(kSampleSegment % kScanThreads == 0 && kSampleGroup == 64, "a wave's load is one group");
@@ -552,7 +576,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
     const uint32_t want = min(p.top_k, finite);
     // A bound that at least `want` groups reach, found on the threads' largest keys (a lower bound of the groups' own want-th
     // largest), four bits at a time from the top until it leaves out most of the others: each of the sixteen waves counts for one
-    // value of the four. (Bit by bit by one wave it was 2 of the launch's 11.5 us.)
+    // value of the four, from the first bits in which any two differ. (Bit by bit by one wave it was 2 of the launch's 11.5 us.)
     uint32_t most = 0;
 #pragma unroll
     for (int s = 0; s < kPickSlots; ++s) most = max(most, keys[s]);
@@ -562,9 +586,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
     uint32_t held[kSampleWaves];
 #pragma unroll
     for (int s = 0; s < kSampleWaves; ++s) held[s] = sh.hist[64 * s + lane];
-    uint32_t low = 0, reach = kSampleThreads;
+    // the bits that all of them share need no counting (a row's largest values have their upper eight or so in common)
+    const uint32_t one = (uint32_t)__builtin_amdgcn_readfirstlane((int)held[0]);
+    uint32_t differ = 0, reach = kSampleThreads;
+#pragma unroll
+    for (int s = 0; s < kSampleWaves; ++s) differ |= held[s] ^ one;
+    differ = wave_max_u32(differ);                              // its highest bit is the highest in which any two differ
+    const int top = differ ? (31 - __builtin_clz(differ)) & ~3 : -4;
+    uint32_t low = top < 28 ? one >> (top + 4) << (top + 4) : 0u;
 #pragma unroll 1
-    for (int shift = 28; shift >= 0 && reach > want + want / 2; shift -= 4) {
+    for (int shift = top; shift >= 0 && reach > want + want / 2; shift -= 4) {
         const uint32_t at = low | (wave << shift);
         uint32_t c = 0;
 #pragma unroll
@@ -582,23 +613,38 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
     // The candidates are first told apart by their raw value: `raw_low` is below every logit whose capped value reaches the
     // bound (the inverse of the cap at the bound less a few thousand times tanhf's error), so that the cap itself is
     // computed once per candidate and not for the other 63 logits of its group.
-    float raw_low = -FLT_MAX;
-    if (bound > 1u) {
-        const float at = __uint_as_float((bound & 0x80000000u) ? (bound & 0x7FFFFFFFu) : ~bound) / p.softcap;
-        const float z = fminf(at - 1e-4f * fabsf(at) - 1e-6f, 0.9999f);
-        if (z > -0.9999f) raw_low = p.softcap * atanhf(z);
+    // (One wave makes it for all, beside the others' lists.)
+    if (wave == kSampleWaves - 1) {
+        float low_of = -FLT_MAX;
+        if (bound > 1u) {
+            const float at = __uint_as_float((bound & 0x80000000u) ? (bound & 0x7FFFFFFFu) : ~bound) / p.softcap;
+            const float z = fminf(at - 1e-4f * fabsf(at) - 1e-6f, 0.9999f);
+            if (z > -0.9999f) low_of = p.softcap * atanhf(z);
+        }
+        if (lane == 0) sh.red_f[0] = low_of;
     }
+    // (a wave takes its places in a list all at once: one after the other the counter's answers were a chain of round trips to LDS)
+    {
+        unsigned long long mask[kPickSlots];
+        uint32_t n = 0;
 #pragma unroll
-    for (int s = 0; s < kPickSlots; ++s) {
-        const unsigned long long mask = __ballot(keys[s] >= bound);
-        if (mask == 0ull) continue;
-        uint32_t first = 0;
-        if (lane == 0) first = atomicAdd(&n_list, (uint32_t)__popcll(mask));
-        first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-        if (keys[s] >= bound && first < kPickMaxGroups) group_list[first] = s * kSampleThreads + tid;
+        for (int s = 0; s < kPickSlots; ++s) mask[s] = __ballot(keys[s] >= bound), n += (uint32_t)__popcll(mask[s]);
+        if (n) {
+            uint32_t first = 0;
+            if (lane == 0) first = atomicAdd(&n_list, n);
+            first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+#pragma unroll
+            for (int s = 0; s < kPickSlots; ++s) {
+                if (mask[s] == 0ull) continue;
+                const uint32_t place = first + lanes_in_front(mask[s]);
+                if (keys[s] >= bound && place < kPickMaxGroups) group_list[place] = s * kSampleThreads + tid;
+                first += (uint32_t)__popcll(mask[s]);
+            }
+        }
     }
     __syncthreads();
     const uint32_t listed = n_list;
+    const float raw_low = sh.red_f[0];
     bool fits = listed <= kPickMaxGroups;
     if (fits) {
         constexpr int kAhead = 8;
@@ -611,15 +657,20 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(const float
                 at[u] = li < listed ? group_list[li] * kSampleGroup + lane : 0xFFFFFFFFu;
                 v[u] = at[u] < count ? row[at[u]] : NAN;
             }
+            unsigned long long mask[kAhead];
+            uint32_t n = 0;
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) mask[u] = __ballot(v[u] >= raw_low && v[u] <= FLT_MAX), n += (uint32_t)__popcll(mask[u]);
+            if (n == 0) continue;
+            uint32_t first = 0;
+            if (lane == 0) first = atomicAdd(&n_cand, n);
+            first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) {
-                const bool take = v[u] >= raw_low && v[u] <= FLT_MAX;
-                const unsigned long long mask = __ballot(take);
-                if (mask == 0ull) continue;
-                uint32_t first = 0;
-                if (lane == 0) first = atomicAdd(&n_cand, (uint32_t)__popcll(mask));
-                first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-                if (take && first < kPickMaxCands) cand[first] = ((unsigned long long)__float_as_uint(v[u]) << 32) | (0xFFFFFFFFu - at[u]);
+                if (mask[u] == 0ull) continue;
+                const uint32_t place = first + lanes_in_front(mask[u]);
+                if ((mask[u] >> lane & 1ull) && place < kPickMaxCands) cand[place] = ((unsigned long long)__float_as_uint(v[u]) << 32) | (0xFFFFFFFFu - at[u]);
+                first += (uint32_t)__popcll(mask[u]);
             }
         }
         __syncthreads();

@@ -45,6 +45,27 @@ def test_sampled_choice_at_the_edges_of_the_split_form(ctx, oracle, torch, count
     assert (np.abs(prob[same] - want_prob[same]) <= 1e-5 + 2e-3 * want_prob[same]).all(), (prob, want_prob)
 
 
+# what the groups' largest have in common: all bits, all but the last, all but the sign and more, a whole row in one group
+@pytest.mark.parametrize("count", [16384, 65536, 65600])
+def test_sampled_choice_where_group_maxima_share_their_bits(ctx, oracle, torch, count):
+    rng = np.random.default_rng(count)
+    rows = np.full((5, count), -9.0, np.float32)
+    rows[0, ::64] = 2.5
+    rows[1, ::64] = np.where(rng.random((count + 63) // 64) < 0.5, np.float32(2.5), np.nextafter(np.float32(2.5), np.float32(3)))
+    rows[2, ::64] = rng.choice(np.float32([-1.5, 1.5]), (count + 63) // 64)
+    rows[3, :] = -np.inf
+    rows[3, 640:660] = rng.normal(0, 2, 20)
+    rows[4, ::64] = np.float32(2.0) + rng.random((count + 63) // 64).astype(np.float32) * np.float32(0.01)
+    want_tok, want_prob, gap = oracle.sample_rows(rows, 0.9, 0.9, 48, key_base=7, softcap=30.0, seed=3)
+    tok, prob = ctx.sample_rows(torch.from_numpy(rows).cuda(), 0.9, 30.0, 3, key_base=7, top_k=48, top_p=0.9)
+    tok, prob = tok.cpu().numpy().astype(np.uint32), prob.cpu().numpy().astype(np.float64)
+    clear = gap > 1e-4                                         # log and tanh of the two machines differ by less
+    assert clear.sum() >= 4 and np.array_equal(tok[clear], want_tok[clear]), (tok, want_tok, gap)
+    # (as above)
+    same = tok == want_tok
+    assert (np.abs(prob[same] - want_prob[same]) <= 1e-5 + 2e-3 * want_prob[same]).all(), (prob, want_prob)
+
+
 @pytest.mark.parametrize("count", [1, 1023, 8192, 8193, 10241, 262144])
 def test_greedy_choice_over_long_rows(ctx, oracle, torch, count):
     rng = np.random.default_rng(count)
