@@ -375,11 +375,11 @@ __global__ __launch_bounds__(256) void router_approx_kernel(const uint4 *__restr
     }
 }
 
-// What the approximate pass left per part of K, added pairwise (a tree of log2(parts) levels; all loads first).
-__device__ __forceinline__ float sum_k_parts(const float *__restrict__ p, size_t part_stride) {
+// What the approximate pass left per part of K, added pairwise (a tree of log2(parts) levels).
+__device__ __forceinline__ float sum_k_parts(const float (&p)[kApproxKParts]) {
     float v[kApproxKParts];
 #pragma unroll
-    for (int q = 0; q < kApproxKParts; ++q) v[q] = p[q * part_stride];
+    for (int q = 0; q < kApproxKParts; ++q) v[q] = p[q];
 #pragma unroll
     for (int w = 1; w < kApproxKParts; w *= 2)
 #pragma unroll
@@ -396,6 +396,12 @@ constexpr int kExactSteps = 4;          // d <= 4096: k = 1024 i + 256 s + 4 lan
 // rows 24.8 | 22.4 | 25.7, 2,000 rows 25.3 | 28.7 | 30.6: four while three blocks per compute unit hold all, two while those do. (Three is what the registers of
 // 2,049 columns and more allow; narrower tables, which hold four and eight, take the same line and are the faster too, us at 1 | the line's: 512 x
 // 128, 700 rows 12.1 | 10.8, 1,400 rows 14.2 | 13.3; 1,024 x 64, 12.8 | 10.4, 14.0 | 13.2; 256 x 16, 11.0 | 9.6, 11.5 | 10.7; 4,096 x 128, 26.4 | 19.6, 30.5 | 28.1.)
+// What a wave waits for and issues has become less since the lines were drawn (the token's row came in front of its approximate logits, each
+// load behind a branch of its own; the k-th logit and the ranks were eight rounds of a wave-wide maximum each; the reductions stood one behind the
+// other). us of the call, so | now: 100 rows 12.3 | 11.0, 301 rows 13.1 | 11.7, 900 rows 16.7 | 14.7, 1,500 rows 21.2 | 18.9, 3,072 rows 30.6 |
+// 27.5, FP16 33.4 | 30.7; 4,096 x 128, 1,000 rows 17.3 | 15.3; 1,024 x 64 10.0 | 9.6. In cycles of a wave at 301 rows: its loads 1,100, sums 700, k-th logit
+// 1,200, candidates 800, their rows 2,000 and sums 2,000, ranks and weights 1,500. Bound: that chain, from some 1,500 rows on the vector instructions
+// (two per weight and product).
 template <int STEPS, int CHUNK, int PARTS, bool F16>
 __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_t *__restrict__ w, const uint16_t *__restrict__ x,
                                                                    uint32_t x_stride, uint32_t t, uint32_t n_experts, uint32_t d,
@@ -409,52 +415,65 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
     const uint32_t lane = threadIdx.x & 63, wave = PARTS == 1 ? threadIdx.x >> 6 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t part = wave % PARTS, my_tok = blockIdx.x * (4 / PARTS) + wave / PARTS, tok = PARTS == 1 ? my_tok : min(my_tok, t - 1);
     if (PARTS == 1 && my_tok >= t) return;  // (else past the last: the last again, not stored, for the barrier)
-    // the token's row, as the pinned order walks it: element j of (step i, sub-accumulator s) = x[1024 i + 256 s + 4 lane + j]
+    // d is a multiple of 256 past the whole steps in front of the last: a (step, sub-accumulator) pair is inside the row for every lane
+    // or for none, and only the last step's later three have to be asked about
+    auto inside = [&](int i, int s_) __attribute__((always_inline)) { return i < STEPS - 1 || s_ == 0 || 1024u * i + 256u * s_ < d; };
+    // the parts of the approximate logits (at most 128 experts: the lane's candidates are experts lane and 64 + lane) and the token's row,
+    // as the pinned order walks it: element j of (step i, sub-accumulator s) = x[1024 i + 256 s + 4 lane + j]; all asked for together
     const uint16_t *xr = x + (size_t)tok * x_stride;
-    float xf[STEPS][4][4];
-    {
-        uint2 xraw[STEPS][4];
+    float parts_of[2][kApproxKParts], norm_of[kApproxKParts];
+    uint2 xraw[STEPS][4];
 #pragma unroll
-        for (int i = 0; i < STEPS; ++i)
+    for (int q = 0; q < kApproxKParts; ++q) {
 #pragma unroll
-            for (int s_ = 0; s_ < 4; ++s_) {
-                // d is a multiple of 256: a (step, sub-accumulator) pair is inside the row for every lane or for none
-                const uint32_t k = 1024 * i + 256 * s_;
-                xraw[i][s_] = k < d ? *reinterpret_cast<const uint2 *>(xr + k + 4 * lane) : make_uint2(0u, 0u);
-            }
-#pragma unroll
-        for (int i = 0; i < STEPS; ++i)
-#pragma unroll
-            for (int s_ = 0; s_ < 4; ++s_) {
-                xf[i][s_][0] = Act<F16>::lo(xraw[i][s_].x), xf[i][s_][1] = Act<F16>::hi(xraw[i][s_].x);
-                xf[i][s_][2] = Act<F16>::lo(xraw[i][s_].y), xf[i][s_][3] = Act<F16>::hi(xraw[i][s_].y);
-            }
+        for (int c = 0; c < 2; ++c) parts_of[c][q] = approx[((size_t)q * t_pad + tok) * n_experts + min(c * 64 + lane, n_experts - 1)];
+        norm_of[q] = xnorm2[(size_t)q * t_pad + tok];
     }
-    // at most 128 experts: the lane's candidates are experts lane and 64 + lane
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+        for (int s_ = 0; s_ < 4; ++s_)
+            if (inside(i, s_)) xraw[i][s_] = *reinterpret_cast<const uint2 *>(xr + 1024 * i + 256 * s_ + 4 * lane);
     float a[2];
     bool odd = false;       // a value that is not finite
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         const uint32_t e = c * 64 + lane;
-        a[c] = e < n_experts ? sum_k_parts(approx + (size_t)tok * n_experts + e, (size_t)t_pad * n_experts) : -INFINITY;
+        a[c] = e < n_experts ? sum_k_parts(parts_of[c]) : -INFINITY;
         odd = odd || (e < n_experts && !(fabsf(a[c]) < INFINITY));
     }
     // 2 B: see the comment above; the absolute term covers products the matrix unit may flush to zero
-    const float norm2 = sum_k_parts(xnorm2 + tok, t_pad);
+    const float norm2 = sum_k_parts(norm_of);
     const float bound = bound_per_norm * sqrtf(norm2) + 1e-30f;
     const bool everyone = __any(odd) || !(bound < INFINITY);
-    // v_k, the k-th largest approximate logit (equal values leave together, which can only lower it)
+    // v_k, the k-th largest approximate logit: a round of a wave-wide maximum per rank (equal values leave together, which can only lower
+    // it), or, where that chain is the longer, the upper 18 bits of its key two by two (what the others could leave out is a candidate
+    // in twenty tokens)
     uint32_t key0 = a[0] > -INFINITY ? orderable(a[0]) : 0u, key1 = a[1] > -INFINITY ? orderable(a[1]) : 0u;
     uint32_t kth = 0;
-    for (uint32_t r = 0; r < top_k; ++r) {
-        kth = wave_max_u32(max(key0, key1));
-        if (key0 == kth) key0 = 0u;
-        if (key1 == kth) key1 = 0u;
+    if (top_k <= 4) {
+        for (uint32_t r = 0; r < top_k; ++r) {
+            kth = wave_max_u32(max(key0, key1));
+            if (key0 == kth) key0 = 0u;
+            if (key1 == kth) key1 = 0u;
+        }
+    } else {
+#pragma unroll
+        for (int bit = 30; bit >= 14; bit -= 2) {
+            uint32_t reach[4];
+#pragma unroll
+            for (uint32_t v = 1; v < 4; ++v) {
+                const uint32_t at = kth | v << bit;
+                reach[v] = (uint32_t)(__popcll(__ballot(key0 >= at)) + __popcll(__ballot(key1 >= at)));
+            }
+            kth |= (reach[3] >= top_k ? 3u : reach[2] >= top_k ? 2u : reach[1] >= top_k ? 1u : 0u) << bit;
+        }
     }
     const float v_k = kth ? __uint_as_float((kth & 0x80000000u) ? (kth & 0x7FFFFFFFu) : ~kth) : -INFINITY;
     const float threshold = v_k - bound;        // -inf when fewer than k candidates exist: everyone is in
     unsigned long long m0 = __ballot(lane < n_experts && (everyone || a[0] >= threshold));
     unsigned long long m1 = __ballot(64 + lane < n_experts && (everyone || a[1] >= threshold));
+    const unsigned long long all0 = m0, all1 = m1;
     uint32_t exact0 = 0u, exact1 = 0u;      // the pinned logits of this lane's two experts, as keys of the select
     if constexpr (PARTS > 1) {
         // every PARTS-th candidate is this wave's
@@ -466,6 +485,15 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
         m0 = share(m0, 0);
         m1 = share(m1, first);
     }
+    float xf[STEPS][4][4];
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+        for (int s_ = 0; s_ < 4; ++s_)
+            if (inside(i, s_)) {
+                xf[i][s_][0] = Act<F16>::lo(xraw[i][s_].x), xf[i][s_][1] = Act<F16>::hi(xraw[i][s_].x);
+                xf[i][s_][2] = Act<F16>::lo(xraw[i][s_].y), xf[i][s_][3] = Act<F16>::hi(xraw[i][s_].y);
+            }
     // The candidates CHUNK at a time: all rows of a chunk are requested before the first sum runs, so a token pays a
     // few round trips to the weights instead of one per candidate.
     while (m0 | m1) {
@@ -482,24 +510,25 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
             } else {
                 e[q] = 0xFFFFFFFFu;
             }
-            const uint16_t *wr = w + (size_t)(e[q] == 0xFFFFFFFFu ? 0u : e[q]) * d;
+            if (e[q] == 0xFFFFFFFFu) continue;
+            const uint16_t *wr = w + (size_t)e[q] * d;
 #pragma unroll
             for (int i = 0; i < STEPS; ++i)
 #pragma unroll
-                for (int s_ = 0; s_ < 4; ++s_) {
-                    const uint32_t k = 1024 * i + 256 * s_;
-                    wq[q][i][s_] = k < d && e[q] != 0xFFFFFFFFu ? *reinterpret_cast<const uint2 *>(wr + k + 4 * lane) : make_uint2(0u, 0u);
-                }
+                for (int s_ = 0; s_ < 4; ++s_)
+                    if (inside(i, s_)) wq[q][i][s_] = *reinterpret_cast<const uint2 *>(wr + 1024 * i + 256 * s_ + 4 * lane);
         }
+        float v[CHUNK];
 #pragma unroll
         for (int q = 0; q < CHUNK; ++q) {
+            v[q] = 0.0f;
             if (e[q] == 0xFFFFFFFFu) continue;
             float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < STEPS; ++i)
 #pragma unroll
                 for (int s_ = 0; s_ < 4; ++s_) {
-                    if (1024u * i + 256u * s_ < d) {
+                    if (inside(i, s_)) {
                         const uint2 wv = wq[q][i][s_];
                         acc[s_] = __builtin_fmaf(bf16lo_to_f32(wv.x), xf[i][s_][0], acc[s_]);
                         acc[s_] = __builtin_fmaf(bf16hi_to_f32(wv.x), xf[i][s_][1], acc[s_]);
@@ -507,8 +536,14 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
                         acc[s_] = __builtin_fmaf(bf16hi_to_f32(wv.y), xf[i][s_][3], acc[s_]);
                     }
                 }
-            const float v = wave_butterfly_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
-            const uint32_t k_ = v > -INFINITY ? orderable(v) : 0u;
+            v[q] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        }
+        // (the chunk's reductions beside each other)
+#pragma unroll
+        for (int q = 0; q < CHUNK; ++q) v[q] = wave_butterfly_sum(v[q]);
+#pragma unroll
+        for (int q = 0; q < CHUNK; ++q) {
+            const uint32_t k_ = v[q] > -INFINITY ? orderable(v[q]) : 0u;
             if (e[q] == lane) exact0 = k_;
             if (e[q] == 64u + lane) exact1 = k_;
         }
@@ -522,7 +557,7 @@ __global__ __launch_bounds__(256, 3) void router_exact_topk_kernel(const uint16_
     }
     TopkRow tr;
     tr.key[0] = exact0, tr.key[1] = exact1, tr.key[2] = 0u, tr.key[3] = 0u;
-    topk_select<2>(tr, top_k, lane);
+    few_topk_select(tr, all0, all1, top_k, lane);
     topk_store(tr, per_expert_scale, top_k, out_idx + (size_t)tok * top_k, out_w + (size_t)tok * top_k, lane, F16);
 }
 

@@ -112,6 +112,31 @@ __device__ __forceinline__ void topk_select(TopkRow &t, uint32_t top_k, uint32_t
     topk_weights(t, mine, max_s, top_k);
 }
 
+// The select of one wave that knows its row's few candidates (bits of `m0`: experts 0 .. 63, of `m1`: 64 .. 127; every other key is 0).
+// A candidate's rank is how many have a larger key, or an equal one and a lower index: three ballots and a lane's two moves per
+// candidate where topk_select has a chain of forty instructions per rank. Same routes, same weights.
+__device__ __forceinline__ void few_topk_select(TopkRow &t, unsigned long long m0, unsigned long long m1, uint32_t top_k, uint32_t lane) {
+    uint32_t got = 0;       // lane i: the key of rank i
+    t.idx = 0;
+    auto take = [&](uint32_t ko, uint32_t rank, uint32_t e) __attribute__((always_inline)) {
+        if (lane == rank && rank < top_k && ko != 0u) got = ko, t.idx = e;
+    };
+    for (; m0; m0 &= m0 - 1) {
+        const uint32_t l = (uint32_t)__builtin_ctzll(m0), ko = (uint32_t)__builtin_amdgcn_readlane((int)t.key[0], (int)l);
+        const unsigned long long front = (1ull << l) - 1ull;
+        take(ko, (uint32_t)__popcll((__ballot(t.key[0] >= ko) & front) | (__ballot(t.key[0] > ko) & ~front)) + (uint32_t)__popcll(__ballot(t.key[1] > ko)), l);
+    }
+    for (; m1; m1 &= m1 - 1) {
+        const uint32_t l = (uint32_t)__builtin_ctzll(m1), ko = (uint32_t)__builtin_amdgcn_readlane((int)t.key[1], (int)l);
+        const unsigned long long front = (1ull << l) - 1ull;
+        take(ko, (uint32_t)__popcll(__ballot(t.key[0] >= ko)) + (uint32_t)__popcll((__ballot(t.key[1] >= ko) & front) | (__ballot(t.key[1] > ko) & ~front)), 64u + l);
+    }
+    // recover the score from the key: orderable() is a bijection
+    const float mine = got ? __uint_as_float((got & 0x80000000u) ? (got & 0x7FFFFFFFu) : ~got) : -INFINITY;
+    const float max_s = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(mine), 0));
+    topk_weights(t, mine, max_s, top_k);
+}
+
 // The same select by the four waves of a block together (moe.metal:186-237 ranks with a SIMD-wide pass as well):
 // instead of top_k dependent rounds of a wave-wide maximum, every candidate's rank is COUNTED - how many candidates
 // have a larger key - and the candidates of rank < top_k go to their places. Every wave holds the row's keys (t.key,
