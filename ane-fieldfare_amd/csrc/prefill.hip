@@ -1412,7 +1412,8 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const uint16_t *__
     // One round trip: the routes' weights, experts and rows are requested together. A dropped route's row was never written
     // and may hold anything: it is loaded like the others (its place is inside the buffer) and its sums are passed by. Asked for
     // behind their weights and experts the rows were a second round trip: 301 rows of 8 x 2,816 6.0 us, now 4.9; 3,072 rows 28.6 | 25.0
-    // (6.2 TB/s; 8,192 rows, which no cache holds, 84.8 | 83.3).
+    // (6.2 TB/s; 8,192 rows, which no cache holds, 84.8 | 83.3). The rows are read once, and said to be so: 8,192 rows 79.3 -> 62.0
+    // (6.7 TB/s), 3,072 rows 23.0 either way.
     uint16_t wbits[8];
     uint32_t expert[8];
     uint4 p[8];
@@ -1421,7 +1422,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const uint16_t *__
         const uint32_t route = tok * top_k + min(r, top_k - 1);
         wbits[r] = w[route];
         expert[r] = idx[route];
-        p[r] = *reinterpret_cast<const uint4 *>(partials + (size_t)route * d + c);
+        p[r] = __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(partials + (size_t)route * d + c)));
     }
     float wv[8];
     bool live[8];
