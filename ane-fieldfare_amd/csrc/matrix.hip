@@ -184,7 +184,8 @@ __device__ __forceinline__ SoftmaxAcc softmax_shuffle(const SoftmaxAcc &a, int m
 // FEW (up to four input rows of the plain form): input row t is operand row 4 t, so that one of a lane's four sums is all there is to
 // keep up, and each operand lane loads its own bytes: the lanes of a row ask for the same ones, there is nothing to turn through LDS.
 // 1 row, us without | so: 16,384 x 1,408 6.7 | 5.9, 16,384 x 2,816 7.2 | 6.8, 262,144 x 2,816 76.5 | 74.9 (5.5 TB/s).
-template <bool Y_F32, bool F16, bool GREEDY = false, bool CONF = false, bool PLANES8 = false, int GLU = 0, bool FEW = false>
+// ONCE: the matrix is more than the memory side's cache holds (kReadOnce).
+template <bool Y_F32, bool F16, bool GREEDY = false, bool CONF = false, bool PLANES8 = false, int GLU = 0, bool FEW = false, bool ONCE = false>
 __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__restrict__ tiles,
                                                              const uint8_t *__restrict__ scales, uint32_t m,
                                                              uint32_t n_groups, const uint16_t *__restrict__ x,
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     }
     WeightRing ring;
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) ring_fill(ring, u, src, rb0 * n_groups + min(g0 + u, g_last), lane);
+    for (int u = 0; u < kRing; ++u) ring_fill<ONCE>(ring, u, src, rb0 * n_groups + min(g0 + u, g_last), lane);
     // the input rows of this wave's K-slice: requested as 64-byte pieces (four lanes per row), then turned into the
     // operand layout - with 16 rows the operand layout itself would make every lane of every load a request of its own
     uint4 x0[kRing], x1[kRing];
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16, true, kSums>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), lane);
+            ring_step<F16, true, kSums, ONCE>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), lane);
         const int buf = (rb - rb0) & 1;
 #pragma unroll
         for (int r = 0; r < kSums; ++r) {
@@ -850,15 +851,21 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
     if (glu == 1) {
         if (f16) { if (y_f32) FFMOE_MGEMV(true, true, true, 1); else FFMOE_MGEMV(false, true, true, 1); }
         else { if (y_f32) FFMOE_MGEMV(true, false, true, 1); else FFMOE_MGEMV(false, false, true, 1); }
-    } else if (planes8) {
-        if (f16) { if (y_f32) FFMOE_MGEMV(true, true, true, 0); else FFMOE_MGEMV(false, true, true, 0); }
-        else { if (y_f32) FFMOE_MGEMV(true, false, true, 0); else FFMOE_MGEMV(false, false, true, 0); }
-    } else if (rows <= 4) {
-        if (f16) { if (y_f32) FFMOE_MGEMV(true, true, false, 0, true); else FFMOE_MGEMV(false, true, false, 0, true); }
-        else { if (y_f32) FFMOE_MGEMV(true, false, false, 0, true); else FFMOE_MGEMV(false, false, false, 0, true); }
     } else {
-        if (f16) { if (y_f32) FFMOE_MGEMV(true, true, false, 0); else FFMOE_MGEMV(false, true, false, 0); }
-        else { if (y_f32) FFMOE_MGEMV(true, false, false, 0); else FFMOE_MGEMV(false, false, false, 0); }
+        auto pick = [&](auto once) {
+            constexpr bool O = decltype(once)::value;
+            if (planes8) {
+                if (f16) { if (y_f32) FFMOE_MGEMV(true, true, true, 0, false, O); else FFMOE_MGEMV(false, true, true, 0, false, O); }
+                else { if (y_f32) FFMOE_MGEMV(true, false, true, 0, false, O); else FFMOE_MGEMV(false, false, true, 0, false, O); }
+            } else if (rows <= 4) {
+                if (f16) { if (y_f32) FFMOE_MGEMV(true, true, false, 0, true, O); else FFMOE_MGEMV(false, true, false, 0, true, O); }
+                else { if (y_f32) FFMOE_MGEMV(true, false, false, 0, true, O); else FFMOE_MGEMV(false, false, false, 0, true, O); }
+            } else {
+                if (f16) { if (y_f32) FFMOE_MGEMV(true, true, false, 0, false, O); else FFMOE_MGEMV(false, true, false, 0, false, O); }
+                else { if (y_f32) FFMOE_MGEMV(true, false, false, 0, false, O); else FFMOE_MGEMV(false, false, false, 0, false, O); }
+            }
+        };
+        if (!twice && (size_t)n_tiles * (n / kGroup) * kTileBytes > kMemoryCacheBytes) pick(std::true_type{}); else pick(std::false_type{});
     }
 #undef FFMOE_MGEMV
     return hipGetLastError();
@@ -1016,8 +1023,9 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
     const dim3 grid(greedy_segments(m, n_cus));
     float2 *conf_part = reinterpret_cast<float2 *>(partials + (size_t)FFMOE_MAX_VERIFY_ROWS * grid.x);
 #define FFMOE_GREEDY(H, C)                                                                                                  \
-    hipLaunchKernelGGL((matrix_gemv_kernel<true, H, true, C>), grid, dim3(256), 0, s, tiles, scales, m, n / kGroup, x, x_stride, \
-                       rows, partials, 0u, conf_part, softcap)
+    hipLaunchKernelGGL((once ? matrix_gemv_kernel<true, H, true, C, false, 0, false, true> : matrix_gemv_kernel<true, H, true, C>), grid, dim3(256), 0, s, \
+                       tiles, scales, m, n / kGroup, x, x_stride, rows, partials, 0u, conf_part, softcap)
+    const bool once = (size_t)((m + 31) / 32) * (n / kGroup) * kTileBytes > kMemoryCacheBytes;
     if (f16) { if (out_conf) FFMOE_GREEDY(true, true); else FFMOE_GREEDY(true, false); }
     else { if (out_conf) FFMOE_GREEDY(false, true); else FFMOE_GREEDY(false, false); }
 #undef FFMOE_GREEDY

@@ -38,13 +38,21 @@ __device__ __forceinline__ TileSource make_tile_source(const uint8_t *tiles, siz
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-// `tile_index` = index of the 1 KiB tile inside the region (wave-uniform).
+// For tiles that no other block reads and no cache holds until the next call: the load's non-temporal bit. The memory side's cache has
+// 256 MB; a sweep of more pushes its own lines out before they are wanted again, and is the faster when it leaves none there: the
+// head's 415 MB, one input row, with the draw behind it 89.0 -> 79.8 us, greedy 84.7 -> 78.4; the layer of a 37-row prompt (a chunk's 390 MB of experts)
+// 126.1 -> 116.2, of 301 rows 177 -> 169.6. Below that the next call finds the lines: 158 MB 26.5 us, so 28.1; 25 MB 6.9 | 8.7; 155 MB of experts 57 | 65.5.
+constexpr int kReadOnce = 2;
+constexpr size_t kMemoryCacheBytes = 256u << 20;
+
+// `tile_index` = index of the 1 KiB tile inside the region (wave-uniform). ONCE: see kReadOnce.
+template <bool ONCE = false>
 __device__ __forceinline__ void ring_fill(WeightRing &ring, int u, const TileSource &src, uint32_t tile_index,
                                           uint32_t lane) {
     // the index is wave-uniform by contract; pinning it to a scalar register spares the waterfall loop the
     // compiler emits whenever it happened to compute a uniform value in a vector register
     tile_index = __builtin_amdgcn_readfirstlane(tile_index);
-    const u32x4_t t = __builtin_amdgcn_raw_buffer_load_b128(src.tiles, (int)(lane * 16u), (int)(tile_index * kTileBytes), 0);
+    const u32x4_t t = __builtin_amdgcn_raw_buffer_load_b128(src.tiles, (int)(lane * 16u), (int)(tile_index * kTileBytes), ONCE ? kReadOnce : 0);
     const u32x2_t s = __builtin_amdgcn_raw_buffer_load_b64(src.scales, (int)((lane & 15u) * 8u),
                                                            (int)(tile_index * kTileScaleBytes), 0);
     ring.t[u] = make_uint4(t.x, t.y, t.z, t.w);
@@ -64,7 +72,7 @@ __device__ __forceinline__ f32x4 group_input_sum(const uint4 &x0, const uint4 &x
 // Consume ring slot u against the resident token operand (`sx` = its group_input_sum), then start the load
 // that refills the slot (REFILL = false: a wave that walks one tile row only has nothing to refill).
 // SUMS: of the lane's four results, how many are kept up.
-template <bool F16 = false, bool REFILL = true, int SUMS = 4>
+template <bool F16 = false, bool REFILL = true, int SUMS = 4, bool ONCE = false>
 __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, const uint4 &x0, const uint4 &x1,
                                           const f32x4 &sx, TwoStreamAcc &tot, const TileSource &src,
                                           uint32_t next_tile_index, uint32_t lane) {
@@ -72,7 +80,7 @@ __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, co
     const uint4 tile = ring.t[u];
     uint2 sc = ring.s[u];
     if (!live) sc = make_uint2(0u, 0u);
-    if (REFILL) ring_fill(ring, u, src, next_tile_index, lane);
+    if (REFILL) ring_fill<ONCE>(ring, u, src, next_tile_index, lane);
     f32x4 acc_a = Act<F16>::mfma(x0, unpack8_offset<F16>(tile.x), zero);
     acc_a = Act<F16>::mfma(x1, unpack8_offset<F16>(tile.y), acc_a);
     f32x4 acc_b = Act<F16>::mfma(x0, unpack8_offset<F16>(tile.z), zero);

@@ -1,0 +1,33 @@
+"""Matrices and layers of more bytes than the memory side's cache holds: their weights are read with another cache hint, in kernels of
+their own. Same bits as the forms without it. Needs a GPU: pytest -m gpu."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N = 2112                                            # 262,144 x 2,112 in 4 bits, 131,072 x 2,112 in 8: 277 MB
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+def test_rows_of_a_large_matrix(act):
+    import torch
+    import fieldfare_moe as ff
+    from fieldfare_moe import synthetic as syn
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    ctx = ff.Context(256, 128, 8, 8, n_layers=1, max_tokens=16, act_dtype=act)
+    try:
+        m = 262144
+        parts = syn.synth_matrix_gpu(torch, gen, m, N)
+        head = ctx.matrix(*parts, greedy=True)
+        x = torch.randn((16, N), device="cuda", generator=gen).to(dt)
+        at = torch.tensor([0, 31, 32, 4097, 131071, 200000, m - 33, m - 1], device="cuda")
+        few = ctx.matrix(*[p[at].contiguous() for p in parts])
+        for rows in (1, 4, 5, 16):
+            y = head.gemv(x[:rows], f32_out=True)
+            assert torch.equal(y[:, at], few.gemv(x[:rows], f32_out=True))
+            assert torch.equal(head.gemv(x[:rows])[:, at], few.gemv(x[:rows]))
+            best, _ = head.greedy_conf(x[:rows], softcap=30.0)
+            assert torch.equal(best.to(torch.int64), y.argmax(1))
+    finally:
+        ctx.close()
