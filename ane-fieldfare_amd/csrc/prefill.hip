@@ -1025,7 +1025,7 @@ __device__ __forceinline__ uint4 unpack8_stream(uint32_t w) {
     else return unpack8_offset<false>(w);
 }
 
-template <bool GATE_UP, int NM, bool F16>
+template <bool GATE_UP, int NM, bool F16, bool ONCE>
 __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom &g, const TileSource &src, uint32_t tile0,
                                             uint4 *__restrict__ lds, const uint32_t *__restrict__ sorted_token,
                                             const uint32_t *__restrict__ sorted_out_row, uint16_t *__restrict__ out,
@@ -1093,7 +1093,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     uint2 ring_s[kStreamDepth];
     auto fill = [&](int u, uint32_t grp) __attribute__((always_inline)) {
         const uint32_t tile = __builtin_amdgcn_readfirstlane(tile0 + min(grp, last));
-        const u32x4_t t = __builtin_amdgcn_raw_buffer_load_b128(src.tiles, (int)(lane * 16u), (int)(tile * kTileBytes), 0);
+        const u32x4_t t = __builtin_amdgcn_raw_buffer_load_b128(src.tiles, (int)(lane * 16u), (int)(tile * kTileBytes), ONCE ? kReadOnce : 0);
         const u32x2_t s = __builtin_amdgcn_raw_buffer_load_b64(src.scales, (int)(j * 8u), (int)(tile * kTileScaleBytes), 0);
         ring_t[u] = make_uint4(t.x, t.y, t.z, t.w);
         ring_s[u] = make_uint2(s.x, s.y);
@@ -1286,10 +1286,11 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     }
 }
 
-// MAX_NM: 16-pair blocks of the largest tile the plan cut
+// MAX_NM: 16-pair blocks of the largest tile the plan cut. `read_once`: the chunk's experts are more than the memory side's cache holds
+// (stream.hpp). A whole tile is no reader of that kind: its expert may have others, on the same XCD (700 Zipf routes of exponent 1.1 with every tile so: 2 % slower).
 template <bool GATE_UP, int MAX_NM, bool F16, int WAVES>
 __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const PrefillPlan *__restrict__ plan, const PrefillTile *__restrict__ tiles,
-                                                                    uint32_t n_nblocks, bool nb_major, const uint8_t *__restrict__ arena_layer,
+                                                                    uint32_t n_nblocks, bool nb_major, bool read_once, const uint8_t *__restrict__ arena_layer,
                                                                     const uint32_t *__restrict__ sorted_token,
                                                                     const uint16_t *__restrict__ a, uint32_t a_stride, uint32_t act_blocks,
                                                                     ArenaGeom g, const uint32_t *__restrict__ sorted_out_row,
@@ -1315,9 +1316,12 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const Prefil
     const TileSource src = make_tile_source(expert_base + (GATE_UP ? g.gu_tiles_off : g.dn_tiles_off), n_tiles * kTileBytes,
                                             expert_base + (GATE_UP ? g.gu_scales_off : g.dn_scales_off), n_tiles * kTileScaleBytes);
     const uint32_t tile0 = at * gw.n_groups;
+    const bool once = read_once && __builtin_amdgcn_readfirstlane(gw.tile.rows) < 16 * MAX_NM;
 #define FFMOE_STREAM(N)                                                                                                      \
-    if constexpr (N <= MAX_NM)                                                                                               \
-        stream_tile<GATE_UP, N, F16>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale)
+    if constexpr (N <= MAX_NM) {                                                                                             \
+        if (once) stream_tile<GATE_UP, N, F16, true>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale);  \
+        else stream_tile<GATE_UP, N, F16, false>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale);      \
+    }
     switch (__builtin_amdgcn_readfirstlane((gw.tile.rows + 15) / 16)) {
         case 1: FFMOE_STREAM(1); break;
         case 2: FFMOE_STREAM(2); break;
@@ -1686,6 +1690,8 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     const uint32_t act_blocks = f16 ? sc.act_blocks : 0u;
     // (a row's address is 32 bits from the first row's where that reaches the last)
     const bool wide = (uint64_t)t * x_stride * 2 > 0xFFFFFFFFull;
+    // (as many experts as the chunk's routes can reach)
+    const bool read_once = (size_t)min(src.n_items, n_experts) * g.expert_bytes > kMemoryCacheBytes;
     // Tiles of up to 128 pairs run two blocks to a compute unit (GemmLds), also where a launch has no more items than units and every block
     // is alone: the shorter start and end of an item are worth 1 to 8 % there. Not tiles of 112 pairs (FP16: 96 and 112) over 40 groups and
     // more: alone, the longer rings and queues win. us of the call with two blocks | one, dense: 4,096 -> 1,408, FP16, 1,536 rows (96 each)
@@ -1708,7 +1714,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     } while (0)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
     hipLaunchKernelGGL(stream_kernel<GU>(tile_rows, f16), dim3(grid_of(NB)), dim3(256), 0, s, sc.plan, sc.tiles, NB,    \
-                       nb_major, arena_layer, sc.sorted_token, A, STRIDE, act_blocks, g, sc.sorted_out_row, OUT, act_scale)
+                       nb_major, read_once, arena_layer, sc.sorted_token, A, STRIDE, act_blocks, g, sc.sorted_out_row, OUT, act_scale)
     if (large_scales) {
         if ((e = launch_prefill_large_scale(s, arena_layer, g, true, tile_cap, x, x_stride, sc.acts, sc, f16)) != hipSuccess) return e;
     } else if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);

@@ -31,3 +31,28 @@ def test_rows_of_a_large_matrix(act):
             assert torch.equal(best.to(torch.int64), y.argmax(1))
     finally:
         ctx.close()
+
+
+def test_short_chunk_of_a_large_layer():
+    # 128 experts of 2,816 x 704: a chunk that reaches them all beside parts of it that reach few
+    import torch
+    import fieldfare_moe as ff
+    from fieldfare_moe import synthetic as syn
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    for act in ("bf16", "fp16"):
+        ctx = ff.Context(syn.D, syn.F, syn.E, syn.K, n_layers=1, max_tokens=512, act_dtype=act)
+        try:
+            offsets, _ = syn.layout_offsets(syn.D, syn.F, align=16)
+            ctx.upload_layer(0, syn.synth_layer_gpu(torch, gen, offsets).view(-1), syn.STRIDE, offsets)
+            dt = torch.bfloat16 if act == "bf16" else torch.float16
+            for t in (40, 301, 500):                # tiles of 16 (bf16), 32 and 64 pairs; one expert with whole tiles
+                x = torch.randn((t, syn.D), device="cuda", generator=gen).to(dt)
+                idx = torch.topk(torch.rand((t, syn.E), device="cuda", generator=gen), syn.K, dim=1).indices.to(torch.int32)
+                idx[:, 0] = torch.where((idx[:, 1:] == 7).any(1), idx[:, 0], 7)
+                w = (torch.rand((t, syn.K), device="cuda", generator=gen) * 0.2 + 0.05).to(dt)
+                y = ctx.prefill(0, x, idx.contiguous(), w)
+                for part in (slice(0, 2), slice(t - 3, t)):
+                    assert torch.equal(ctx.prefill(0, x[part].contiguous(), idx[part].contiguous(), w[part].contiguous()), y[part])
+        finally:
+            ctx.close()
