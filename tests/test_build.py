@@ -15,6 +15,15 @@ def test_the_library_is_the_default_and_needs_no_torch():
     assert "binding.cpp" in both and "BINDING_HASH_PATH" in both and "libfieldfare_moe_hip.so" in both
 
 
+def test_a_change_of_flags_rebuilds_what_they_build():
+    # the digest beside each covers the Makefile: an object with the old flags would pass for one with the new
+    import fieldfare_moe as ff
+    lines = subprocess.run(["make", "-n", "-W", "Makefile", "-C", str(ff.CSRC), "PYTHON=false", "all"], capture_output=True, text=True).stdout
+    for source in ff.CSRC.glob("*.hip"):
+        assert f"-c {source.name} -o {source.stem}.o" in lines, source.name
+    assert "binding.cpp -o" in lines
+
+
 def test_a_module_for_another_torch_is_stale(monkeypatch):
     import torch
     import fieldfare_moe as ff
