@@ -12,6 +12,8 @@
 // 4-bit ones: q = 16 h + l, so w = (16 s) h + b + s l. A tile then holds rows 16 p + l % 16 twice - stream A their
 // high nibbles with scale 16 s (exact: a power of two) and bias b, stream B their low nibbles with scale s and bias
 // 0 - and an output is the sum of its two streams. Same bytes as the 8-bit matrix, same stream, same speed.
+#include <cfloat>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "stream.hpp"
@@ -140,17 +142,18 @@ struct SoftmaxAcc {
     float m, s;      // m = -inf: nothing seen yet
 };
 // The divisions as reciprocals with a step of Newton's method each: 11 instructions for some 35, and no further off (the quotient's error is
-// below a unit in its last place, the second product and sum round once).
+// below a unit in its last place, the second product and sum round once). Every positive cap has a place: the reciprocal of one below 2^-128
+// is held to a number (0 stays 0), and it is r that is doubled, not the cap, which may be the largest number there is.
 __device__ __forceinline__ float capped(float v, float softcap) {
     if (!(softcap > 0.0f)) return v;
     // tanh z = 1 - 2 / (exp(2 z) + 1); from z = 40 on (and where v / softcap is no number any more) that is 1
-    const float inv = 1.0f / softcap;
+    const float inv = fminf(1.0f / softcap, FLT_MAX);
     float z = fminf(fmaxf(v * inv, -40.0f), 40.0f);
     z = fminf(__builtin_fmaf(__builtin_fmaf(-z, softcap, v), inv, z), 40.0f);
     const float d = __expf(2.0f * z) + 1.0f;
     float r = __builtin_amdgcn_rcpf(d);
     r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
-    return __builtin_fmaf(-2.0f * softcap, r, softcap);
+    return __builtin_fmaf(-softcap, r + r, softcap);
 }
 __device__ __forceinline__ void softmax_take(SoftmaxAcc &a, float v, float softcap) {
     if (!(__builtin_fabsf(v) < INFINITY)) return;          // non-finite logits take no part (they never win either)

@@ -182,6 +182,20 @@ def test_argmax_rows_choice_and_confidence(ctx, oracle, torch, softcap):
     assert np.array_equal(only.cpu().numpy().astype(np.uint32), want_tok)
 
 
+@pytest.mark.parametrize("softcap", [3.4e38, 1.8e38, 1e-36, 1e-39, 1e-44])
+def test_caps_at_the_ends_of_the_range(ctx, oracle, torch, softcap):
+    # caps whose double or whose reciprocal is no fp32 number; logits of the cap's size, either sign, zero among them
+    rng = np.random.default_rng(43)
+    rows = (softcap * rng.uniform(-0.9, 0.9, (3, 700))).astype(np.float32)
+    rows[0, 5] = 0.0
+    rows[1, :] = 0.0
+    rows[2, ::2] = 0.0
+    want_tok, want_conf = oracle.greedy_choice_rows(rows, float(np.float32(softcap)))
+    tok, conf = ctx.argmax_rows(torch.from_numpy(rows).cuda(), softcap=softcap)
+    assert np.array_equal(tok.cpu().numpy().astype(np.uint32), want_tok)
+    assert np.abs(conf.cpu().numpy() - want_conf).max() <= 1e-5 + 1e-4 * want_conf.max()
+
+
 def test_greedy_conf_and_hot_vocabulary_choice(ctx, oracle, torch):
     # LMHeadChainInt4.encodeGreedyRows with its confidence output, and encodeHotGreedyRows (LMHeadChainInt4.swift:
     # 94-186): the choice over the listed rows of the head, mapped back through the list, equals the full head's
