@@ -1403,41 +1403,42 @@ __global__ __launch_bounds__(64 * kPairWaves) void prefill_pair_scale_kernel(con
 // h2[t][c] = bf16(sum_r w[t][r] * partial[t][r][c]) over the routes the sort kept, fma in rank order
 // (prefill.metal:544-565); dropped routes (zero weight, expert out of range) add nothing, which equals
 // the reference's zero-filled partial rows without having to clear 138 MB first.
-template <bool F16>
+// TOP_K rows per token and no more, and of those the live ones: what a thread does not ask for is worth more than the round trip that asking
+// for all eight places beside the weights and experts saves. us, 8,192 rows of 2,816, all live | half lost | seven eighths lost, so: top-8 64.5 | 37.6 |
+// 15.3, top-2 21.3 | 14.5 | 10.6, top-1 15.0 | 11.3 | 9.8; all eight at once 61.5 | 61.5 | 65.5, 36.6 | 36.5 | 35.4, 30.2 | 31.2 | 31.4. 3,072 rows, top-8
+// 23.1 | 14.0 | 7.3 (23.2 | 25.1 | 26); 301 rows 4.1 (4.3). The rows are read once, and said to be so: 8,192 rows, top-8, 91 without. Bound: the rows'
+// bytes (6.4 TB/s at 8,192 rows, 6.7 from the caches at 3,072).
+template <bool F16, int TOP_K>
 __global__ __launch_bounds__(256) void prefill_combine_kernel(const uint16_t *__restrict__ partials,
-                                                              const uint16_t *__restrict__ w,
-                                                              const uint32_t *__restrict__ idx, uint32_t n_experts,
-                                                              uint32_t top_k, uint32_t d, uint32_t t,
+                                                              const uint16_t *__restrict__ w, const uint32_t *__restrict__ idx,
+                                                              uint32_t n_experts, uint32_t d, uint32_t t,
                                                               uint16_t *__restrict__ y) {
     // one thread per 16-byte piece of an output row, pieces numbered across rows so that every block is full
     const uint32_t pieces = d / 8, piece = blockIdx.x * 256 + threadIdx.x;
     const uint32_t tok = piece / pieces, c = (piece % pieces) * 8;
     if (tok >= t) return;
-    // One round trip: the routes' weights, experts and rows are requested together. A dropped route's row was never written
-    // and may hold anything: it is loaded like the others (its place is inside the buffer) and its sums are passed by. Asked for
-    // behind their weights and experts the rows were a second round trip: 301 rows of 8 x 2,816 6.0 us, now 4.9; 3,072 rows 28.6 | 25.0
-    // (6.2 TB/s; 8,192 rows, which no cache holds, 84.8 | 83.3). The rows are read once, and said to be so: 8,192 rows 79.3 -> 62.0
-    // (6.7 TB/s), 3,072 rows 23.0 either way.
-    uint16_t wbits[8];
-    uint32_t expert[8];
-    uint4 p[8];
+    uint16_t wbits[TOP_K];
+    uint32_t expert[TOP_K];
 #pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) {
-        const uint32_t route = tok * top_k + min(r, top_k - 1);
-        wbits[r] = w[route];
-        expert[r] = idx[route];
-        p[r] = __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(partials + (size_t)route * d + c)));
+    for (uint32_t r = 0; r < TOP_K; ++r) {
+        wbits[r] = w[tok * TOP_K + r];
+        expert[r] = idx[tok * TOP_K + r];
     }
-    float wv[8];
-    bool live[8];
+    float wv[TOP_K];
+    bool live[TOP_K];
 #pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) {
-        live[r] = r < top_k && (wbits[r] & 0x7FFFu) != 0 && expert[r] < n_experts;
+    for (uint32_t r = 0; r < TOP_K; ++r) {
+        live[r] = (wbits[r] & 0x7FFFu) != 0 && expert[r] < n_experts;
         wv[r] = Act<F16>::widen(wbits[r]);
     }
+    uint4 p[TOP_K];
+#pragma unroll
+    for (uint32_t r = 0; r < TOP_K; ++r)
+        if (live[r])
+            p[r] = __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(partials + (size_t)(tok * TOP_K + r) * d + c)));
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (uint32_t r = 0; r < 8; ++r) {
+    for (uint32_t r = 0; r < TOP_K; ++r) {
         if (live[r]) {
             const uint32_t pw[4] = {p[r].x, p[r].y, p[r].z, p[r].w};
 #pragma unroll
@@ -1736,12 +1737,22 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     if (e != hipSuccess) return e;
     timer->mark(s, FFMOE_K_PREFILL_DOWN);
     if (y) {
-        if (f16)
-            hipLaunchKernelGGL(prefill_combine_kernel<true>, dim3((t * (g.d / 8) + 255) / 256), dim3(256), 0, s, partials, w, idx,
-                               n_experts, top_k, g.d, t, y);
-        else
-            hipLaunchKernelGGL(prefill_combine_kernel<false>, dim3((t * (g.d / 8) + 255) / 256), dim3(256), 0, s, partials, w, idx,
-                               n_experts, top_k, g.d, t, y);
+        auto launch = [&](auto k) {
+            constexpr int K = decltype(k)::value;
+            hipLaunchKernelGGL((f16 ? prefill_combine_kernel<true, K> : prefill_combine_kernel<false, K>), dim3((t * (g.d / 8) + 255) / 256), dim3(256), 0, s,
+                               partials, w, idx, n_experts, g.d, t, y);
+        };
+        using std::integral_constant;
+        switch (top_k) {
+            case 1: launch(integral_constant<int, 1>{}); break;
+            case 2: launch(integral_constant<int, 2>{}); break;
+            case 3: launch(integral_constant<int, 3>{}); break;
+            case 4: launch(integral_constant<int, 4>{}); break;
+            case 5: launch(integral_constant<int, 5>{}); break;
+            case 6: launch(integral_constant<int, 6>{}); break;
+            case 7: launch(integral_constant<int, 7>{}); break;
+            default: launch(integral_constant<int, 8>{}); break;        // (top_k <= 8: checked where a context is made)
+        }
         timer->mark(s, FFMOE_K_PREFILL_COMBINE);
     }
     timer->finish();
