@@ -832,7 +832,7 @@ static int prefill_common(ffmoe_ctx *ctx, void *stream, uint32_t layer, const ui
     claim_scratch(ctx, stream);
     FF_HIP(launch_prefill(static_cast<hipStream_t>(stream), ctx->arena + (size_t)layer * ctx->layer_bytes, ctx->geom,
                           ctx->shape.n_experts, ctx->shape.top_k, x, x_stride, t, idx, w, pairs, n_pairs, y, partials,
-                          ctx->pf, &ctx->timer, ctx->n_cus, ctx->f16, dense, ctx->layers[layer].any_large_scale));
+                          ctx->pf, &ctx->timer, ctx->n_cus, ctx->shape.n_layers, ctx->f16, dense, ctx->layers[layer].any_large_scale));
     return FFMOE_OK;
 }
 

@@ -101,8 +101,8 @@ struct PrefillTile {
     uint32_t order;                       // the tile's number in row order (the tile list itself runs from the largest tile down)
 };
 struct PrefillPlan {
-    uint32_t n_pairs, n_tiles;
-    uint32_t large_scales, pad;     // large_scales: an upload's, not a chunk's (launch_repack_layer)
+    uint32_t n_pairs, n_tiles, live_experts;      // live_experts: those with a pair
+    uint32_t large_scales;          // an upload's, not a chunk's (launch_repack_layer)
     uint32_t expert_count[FFMOE_MAX_EXPERTS];
     uint32_t expert_offset[FFMOE_MAX_EXPERTS + 1];
 };
@@ -264,11 +264,11 @@ hipError_t launch_dense8_gemm(hipStream_t s, const void *weights, uint32_t store
                               void *out, uint32_t out_stride, bool f16, uint32_t n_cus);
 
 // prefill.hip: routes come from (idx, w) [t][top_k], or from an explicit pair list when `pairs` != nullptr. large_scales: the
-// layer has weight scales of 2^104 and more. Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
+// layer has weight scales of 2^104 and more; n_layers: of the context, one of which this is. Writes y [t][d] (combined) when y != nullptr; un-weighted bf16 rows go to partials_out or to scratch.
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,
                           const uint16_t *x, uint32_t x_stride, uint32_t t, const uint32_t *idx, const uint16_t *w,
                           const ffmoe_pair *pairs, uint32_t n_pairs_in, uint16_t *y, uint16_t *partials_out,
-                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16 = false, bool dense = false,
+                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, uint32_t n_layers, bool f16 = false, bool dense = false,
                           bool large_scales = false);
 
 // prefill_large.hip: either product (gate/up, else down) of the M-tiles in sc.tiles, `tile_cap` of them at most; `dump` as below

@@ -88,6 +88,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
     __shared__ uint32_t tile_off[FFMOE_MAX_EXPERTS + 1];
     __shared__ uint32_t part[kScanThreads];                 // [chunk][e_pad]: chunk sums, then chunk bases
     __shared__ unsigned long long scan_own[FFMOE_MAX_EXPERTS], wave_sum[FFMOE_MAX_EXPERTS / 64];
+    __shared__ uint32_t wave_live[FFMOE_MAX_EXPERTS / 64];
     __shared__ uint32_t shorter[3][FFMOE_MAX_EXPERTS];      // per expert: shorter tiles in all, in front of it, ranked above its own
     const uint32_t e = threadIdx.x % e_pad, ch = threadIdx.x / e_pad, chunks = kScanThreads / e_pad;
     const uint32_t per = (n_blocks + chunks - 1) / chunks;
@@ -132,7 +133,8 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
             const unsigned long long up = __shfl_up(inc, sh, 64);
             if (lane >= (uint32_t)sh) inc += up;
         }
-        if (lane == 63) wave_sum[wv] = inc;
+        const uint32_t with_pairs = (uint32_t)__popcll(__ballot(n != 0));
+        if (lane == 63) wave_sum[wv] = inc, wave_live[wv] = with_pairs;
         scan_own[i] = inc - own;
     }
     __syncthreads();
@@ -157,6 +159,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_scan_kernel(uint32_t n_b
             }
             plan->n_pairs = (uint32_t)all;
             plan->n_tiles = min((uint32_t)(all >> 32), max_tiles);
+            plan->live_experts = wave_live[0] + wave_live[1] + wave_live[2] + wave_live[3];
             plan->expert_offset[n_experts] = (uint32_t)all;
         }
     }
@@ -345,13 +348,14 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
     // anywhere in the expert order).
     const uint32_t n_mine = cnt[mine], whole_mine = bm.whole(n_mine), rest_mine = n_mine - whole_mine * bm.rows;
     float full_front = 0.0f, full = 0.0f, pairs = 0.0f;
-    uint32_t shorter_front = 0, shorter = 0, above = 0;
+    uint32_t shorter_front = 0, shorter = 0, above = 0, with_pairs = 0;
 #pragma unroll
     for (uint32_t k = 0; k < FFMOE_MAX_EXPERTS / 64; ++k) {
         const uint32_t o = 64 * k + lane, whole = bm.whole(n[k]), rest = n[k] - whole * bm.rows;
         const bool front = o < mine;
         full += (float)whole, pairs += (float)n[k];
         full_front += front ? (float)whole : 0.0f;
+        with_pairs += (uint32_t)__popcll(__ballot(n[k] != 0));
         shorter += (uint32_t)__popcll(__ballot(rest != 0));
         shorter_front += (uint32_t)__popcll(__ballot(rest != 0 && front));
         above += (uint32_t)__popcll(__ballot(rest > rest_mine || (rest != 0 && rest == rest_mine && front)));
@@ -376,6 +380,7 @@ __global__ __launch_bounds__(kScanThreads) void prefill_sort_kernel(ItemSource s
     if (mine == 0) {
         plan->n_pairs = n_pairs;
         plan->n_tiles = min(full_tiles + shorter, max_tiles);
+        plan->live_experts = with_pairs;
         plan->expert_offset[src.n_experts] = n_pairs;
     }
 }
@@ -425,6 +430,7 @@ __global__ __launch_bounds__(kSortBlock) void prefill_dense_plan_kernel(uint32_t
     if (i == 0) {
         plan->n_pairs = t;
         plan->n_tiles = n_tiles;
+        plan->live_experts = 1;
         plan->expert_count[0] = t;
         plan->expert_offset[0] = 0;
         plan->expert_offset[1] = t;
@@ -1286,11 +1292,13 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     }
 }
 
-// MAX_NM: 16-pair blocks of the largest tile the plan cut. `read_once`: the chunk's experts are more than the memory side's cache holds
-// (stream.hpp). A whole tile is no reader of that kind: its expert may have others, on the same XCD (700 Zipf routes of exponent 1.1 with every tile so: 2 % slower).
+// MAX_NM: 16-pair blocks of the largest tile the plan cut. `once_from`: with so many live experts or more the weights are read as data that no
+// cache holds until the next call (read_once_experts), by tiles that are not whole: most are their expert's only one; the short one behind an
+// expert's whole tiles reads so as well, which costs nothing in a layer that comes from memory (301 rows on 40 experts, three layers in turn, 83.5 us,
+// 85.3 without; 700 Zipf rows of exponent 1.1 173.5 | 178). Not whole tiles, whose experts have others (the same Zipf rows with every tile so: 2 % slower).
 template <bool GATE_UP, int MAX_NM, bool F16, int WAVES>
 __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const PrefillPlan *__restrict__ plan, const PrefillTile *__restrict__ tiles,
-                                                                    uint32_t n_nblocks, bool nb_major, bool read_once, const uint8_t *__restrict__ arena_layer,
+                                                                    uint32_t n_nblocks, bool nb_major, uint32_t once_from, const uint8_t *__restrict__ arena_layer,
                                                                     const uint32_t *__restrict__ sorted_token,
                                                                     const uint16_t *__restrict__ a, uint32_t a_stride, uint32_t act_blocks,
                                                                     ArenaGeom g, const uint32_t *__restrict__ sorted_out_row,
@@ -1316,7 +1324,7 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const Prefil
     const TileSource src = make_tile_source(expert_base + (GATE_UP ? g.gu_tiles_off : g.dn_tiles_off), n_tiles * kTileBytes,
                                             expert_base + (GATE_UP ? g.gu_scales_off : g.dn_scales_off), n_tiles * kTileScaleBytes);
     const uint32_t tile0 = at * gw.n_groups;
-    const bool once = read_once && __builtin_amdgcn_readfirstlane(gw.tile.rows) < 16 * MAX_NM;
+    const bool once = __builtin_amdgcn_readfirstlane(gw.tile.rows) < 16 * MAX_NM && plan->live_experts >= once_from;
 #define FFMOE_STREAM(N)                                                                                                      \
     if constexpr (N <= MAX_NM) {                                                                                             \
         if (once) stream_tile<GATE_UP, N, F16, true>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale);  \
@@ -1461,6 +1469,7 @@ __global__ void prefill_dump_plan_kernel(uint32_t expert, PrefillPlan *plan, Pre
                                          uint32_t *sorted_out_row) {
     plan->n_pairs = 1;
     plan->n_tiles = 1;
+    plan->live_experts = 1;
     PrefillTile tl;
     tl.expert = expert;
     tl.row_start = 0;
@@ -1599,6 +1608,19 @@ TileForm dense_tile_form(uint32_t t, const ArenaGeom &g, uint32_t n_nblocks, uin
     return {false, dense_tile_rows(t, g, n_cus)};
 }
 
+// From how many live experts on a streamed chunk's weights are read once (kReadOnce): where those of all the context's layers, which a program
+// takes one after the other, are more than the memory side's cache holds - this layer's live experts, which the device alone knows, taken for every
+// layer's. Asked where the chunk's routes could reach more than the cache in this one layer. 128 experts of 2,816 x 704 (3.3 MB each), us of the call
+// without | with the hint. Three layers in turn: 24 rows, 40 live 46.8 | 42.5; 37 rows, 40 live 44.4 | 39.7, 80 live 66.9 | 57.8; 100 rows, 60 live 58.1 |
+// 53.1; 301 rows, 40 live 82.4 | 79.7, 110 live 103.0 | 96.6. One layer again and again, tiles of 32: 100 rows, 60 live 46.6 | 52.0, 80 live 58.1 | 61.0, 110 live
+// 91 | 82; 301 rows, 60 live 79.8 | 84.8, 80 live 83.2 | 89.9, 110 live 102 | 97.6. Tiles of 16, six blocks per unit, lose their lines from three
+// quarters of the cache on: 24 rows, 40 live 37.7 | 40.6, 58 live 48.3 | 48.5, 74 live 61.3 | 56.8; 37 rows, 50 live 45.3 | 46.5, 60 live 48.9 | 47.6, 79 live 61.4 | 57.6.
+uint32_t read_once_experts(uint32_t n_items, uint32_t n_experts, uint32_t n_layers, const ArenaGeom &g, uint32_t tile_rows) {
+    if ((size_t)min(n_items, n_experts) * g.expert_bytes <= kMemoryCacheBytes) return 0xFFFFFFFFu;
+    const size_t holds = tile_rows == 16 ? kMemoryCacheBytes / 4 * 3 : kMemoryCacheBytes;
+    return (uint32_t)(holds / ((size_t)n_layers * g.expert_bytes)) + 1;
+}
+
 template <bool GATE_UP>
 auto stream_kernel(uint32_t tile_rows, bool f16) {
     if (tile_rows == 16) return prefill_stream_kernel<GATE_UP, 1, false, 6>;           // (bf16 alone: prefill_tile_form)
@@ -1639,7 +1661,7 @@ hipError_t launch_prefill_dump_tiles(hipStream_t s, const uint8_t *arena_layer, 
 hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g, uint32_t n_experts, uint32_t top_k,
                           const uint16_t *x, uint32_t x_stride, uint32_t t, const uint32_t *idx, const uint16_t *w,
                           const ffmoe_pair *pairs, uint32_t n_pairs_in, uint16_t *y, uint16_t *partials_out,
-                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, bool f16, bool dense, bool large_scales) {
+                          PrefillScratch sc, KernelTimer *timer, uint32_t n_cus, uint32_t n_layers, bool f16, bool dense, bool large_scales) {
     // dense: the caller vouches for a dense FFN's chunk - one expert, top_k = 1, every row routed to it at weight 1
     dense = dense && n_experts == 1 && top_k == 1 && !pairs && !y;
     timer->begin(s);
@@ -1691,8 +1713,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     const uint32_t act_blocks = f16 ? sc.act_blocks : 0u;
     // (a row's address is 32 bits from the first row's where that reaches the last)
     const bool wide = (uint64_t)t * x_stride * 2 > 0xFFFFFFFFull;
-    // (as many experts as the chunk's routes can reach)
-    const bool read_once = (size_t)min(src.n_items, n_experts) * g.expert_bytes > kMemoryCacheBytes;
+    const uint32_t once_from = read_once_experts(src.n_items, n_experts, n_layers, g, tile_rows);
     // Tiles of up to 128 pairs run two blocks to a compute unit (GemmLds), also where a launch has no more items than units and every block
     // is alone: the shorter start and end of an item are worth 1 to 8 % there. Not tiles of 112 pairs (FP16: 96 and 112) over 40 groups and
     // more: alone, the longer rings and queues win. us of the call with two blocks | one, dense: 4,096 -> 1,408, FP16, 1,536 rows (96 each)
@@ -1715,7 +1736,7 @@ hipError_t launch_prefill(hipStream_t s, const uint8_t *arena_layer, ArenaGeom g
     } while (0)
 #define FFMOE_STREAM(GU, A, STRIDE, OUT, NB)                                                                                  \
     hipLaunchKernelGGL(stream_kernel<GU>(tile_rows, f16), dim3(grid_of(NB)), dim3(256), 0, s, sc.plan, sc.tiles, NB,    \
-                       nb_major, read_once, arena_layer, sc.sorted_token, A, STRIDE, act_blocks, g, sc.sorted_out_row, OUT, act_scale)
+                       nb_major, once_from, arena_layer, sc.sorted_token, A, STRIDE, act_blocks, g, sc.sorted_out_row, OUT, act_scale)
     if (large_scales) {
         if ((e = launch_prefill_large_scale(s, arena_layer, g, true, tile_cap, x, x_stride, sc.acts, sc, f16)) != hipSuccess) return e;
     } else if (streamed) FFMOE_STREAM(true, x, x_stride, sc.acts, nb_gu);

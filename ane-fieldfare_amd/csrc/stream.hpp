@@ -38,10 +38,11 @@ __device__ __forceinline__ TileSource make_tile_source(const uint8_t *tiles, siz
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-// For tiles that no other block reads and no cache holds until the next call: the load's non-temporal bit. The memory side's cache has
+// For tiles that no other block counts on and no cache holds until the next call: the load's non-temporal bit. The memory side's cache has
 // 256 MB; a sweep of more pushes its own lines out before they are wanted again, and is the faster when it leaves none there: the
 // head's 415 MB, one input row, with the draw behind it 89.0 -> 79.8 us, greedy 84.7 -> 78.4; the layer of a 37-row prompt (a chunk's 390 MB of experts)
-// 126.1 -> 116.2, of 301 rows 177 -> 169.6. Below that the next call finds the lines: 158 MB 26.5 us, so 28.1; 25 MB 6.9 | 8.7; 155 MB of experts 57 | 65.5.
+// 126.1 -> 116.2, of 301 rows 177 -> 169.6. Below that the next call finds the lines: a matrix of 158 MB 26.5 us, so 28.1; of 25 MB 6.9 | 8.7 (a
+// layer's experts: read_once_experts in prefill.hip).
 constexpr int kReadOnce = 2;
 constexpr size_t kMemoryCacheBytes = 256u << 20;
 

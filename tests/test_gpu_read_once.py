@@ -33,26 +33,61 @@ def test_rows_of_a_large_matrix(act):
         ctx.close()
 
 
-def test_short_chunk_of_a_large_layer():
-    # 128 experts of 2,816 x 704: a chunk that reaches them all beside parts of it that reach few
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("layers", [1, 2])
+def test_short_chunk_of_a_large_layer(act, layers):
+    # 128 experts of 2,816 x 704 (80 of them fill the memory side's cache, 40 where the context has two layers): a chunk that reaches
+    # them all, or 30, or 60, beside parts of it that could not reach as many as the cache holds
     import torch
     import fieldfare_moe as ff
     from fieldfare_moe import synthetic as syn
     gen = torch.Generator(device="cuda")
     gen.manual_seed(6)
-    for act in ("bf16", "fp16"):
-        ctx = ff.Context(syn.D, syn.F, syn.E, syn.K, n_layers=1, max_tokens=512, act_dtype=act)
-        try:
-            offsets, _ = syn.layout_offsets(syn.D, syn.F, align=16)
-            ctx.upload_layer(0, syn.synth_layer_gpu(torch, gen, offsets).view(-1), syn.STRIDE, offsets)
-            dt = torch.bfloat16 if act == "bf16" else torch.float16
-            for t in (40, 301, 500):                # tiles of 16 (bf16), 32 and 64 pairs; one expert with whole tiles
-                x = torch.randn((t, syn.D), device="cuda", generator=gen).to(dt)
-                idx = torch.topk(torch.rand((t, syn.E), device="cuda", generator=gen), syn.K, dim=1).indices.to(torch.int32)
+    ctx = ff.Context(syn.D, syn.F, syn.E, syn.K, n_layers=layers, max_tokens=512, act_dtype=act)
+    try:
+        offsets, _ = syn.layout_offsets(syn.D, syn.F, align=16)
+        for layer in range(layers):
+            ctx.upload_layer(layer, syn.synth_layer_gpu(torch, gen, offsets).view(-1), syn.STRIDE, offsets)
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        for t in (40, 301, 500):                    # tiles of 16 (bf16), 32 and 64 pairs; one expert with whole tiles
+            x = torch.randn((t, syn.D), device="cuda", generator=gen).to(dt)
+            for live in (syn.E, 60, 30):
+                idx = torch.topk(torch.rand((t, live), device="cuda", generator=gen), syn.K, dim=1).indices.to(torch.int32)
                 idx[:, 0] = torch.where((idx[:, 1:] == 7).any(1), idx[:, 0], 7)
+                idx = (idx * (syn.E // live)).contiguous()
                 w = (torch.rand((t, syn.K), device="cuda", generator=gen) * 0.2 + 0.05).to(dt)
-                y = ctx.prefill(0, x, idx.contiguous(), w)
+                y = ctx.prefill(layers - 1, x, idx, w)
+                n_pairs, _, counts = ctx.prefill_stats()
+                assert n_pairs == t * syn.K and (counts > 0).sum() == len(torch.unique(idx))
                 for part in (slice(0, 2), slice(t - 3, t)):
-                    assert torch.equal(ctx.prefill(0, x[part].contiguous(), idx[part].contiguous(), w[part].contiguous()), y[part])
-        finally:
-            ctx.close()
+                    assert torch.equal(ctx.prefill(layers - 1, x[part].contiguous(), idx[part].contiguous(), w[part].contiguous()), y[part])
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+def test_whole_and_lone_tiles_of_a_large_layer(act):
+    # experts whose pairs are one short, one whole, two whole and a whole and a short tile of 32, in a layer read once and in calls of
+    # few of its experts, whose tiles are the others' too
+    import torch
+    import fieldfare_moe as ff
+    from fieldfare_moe import synthetic as syn
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    ctx = ff.Context(syn.D, syn.F, syn.E, 1, n_layers=1, max_tokens=4096, act_dtype=act)
+    try:
+        offsets, _ = syn.layout_offsets(syn.D, syn.F, align=16)
+        ctx.upload_layer(0, syn.synth_layer_gpu(torch, gen, offsets).view(-1), syn.STRIDE, offsets)
+        counts = torch.tensor([(1, 31, 32, 33, 64, 16, 3, 0)[e % 8] for e in range(syn.E)])
+        t = int(counts.sum())
+        assert t <= 28 * syn.E                      # tiles of 32
+        idx = torch.repeat_interleave(torch.arange(syn.E), counts).to(torch.int32)[torch.randperm(t)].cuda()[:, None].contiguous()
+        dt = torch.bfloat16 if act == "bf16" else torch.float16
+        x = torch.randn((t, syn.D), device="cuda", generator=gen).to(dt)
+        w = (torch.rand((t, 1), device="cuda", generator=gen) * 0.2 + 0.05).to(dt)
+        y = ctx.prefill(0, x, idx, w)
+        for some in range(16):                      # eight experts at a time, one of each count
+            at = torch.nonzero(idx[:, 0] // 8 == some)[:, 0]
+            assert torch.equal(ctx.prefill(0, x[at].contiguous(), idx[at].contiguous(), w[at].contiguous()), y[at]), some
+    finally:
+        ctx.close()
