@@ -27,8 +27,43 @@ def test_rows_of_a_large_matrix(act):
             y = head.gemv(x[:rows], f32_out=True)
             assert torch.equal(y[:, at], few.gemv(x[:rows], f32_out=True))
             assert torch.equal(head.gemv(x[:rows])[:, at], few.gemv(x[:rows]))
-            best, _ = head.greedy_conf(x[:rows], softcap=30.0)
+            best, conf = head.greedy_conf(x[:rows], softcap=30.0)
             assert torch.equal(best.to(torch.int64), y.argmax(1))
+            # the winner's share of the capped logits' softmax: an exponential's argument is off by some units of 2^-24 of 60 (two caps of
+            # at most 30), 2e-5, and a sum of positive values by a unit for each of the few hundred that one place adds up, 4e-5
+            capped = 30.0 * torch.tanh(y.double() / 30.0)
+            want = torch.softmax(capped, 1).gather(1, best.to(torch.int64)[:, None])[:, 0]
+            assert ((conf.double() - want).abs() <= 1e-4 * want).all(), rows
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+def test_rows_of_a_large_8bit_matrix(act):
+    import torch
+    import fieldfare_moe as ff
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(8)
+    dt = torch.bfloat16 if act == "bf16" else torch.float16
+    ctx = ff.Context(256, 128, 8, 8, n_layers=1, max_tokens=16, act_dtype=act)
+    try:
+        m = 131072
+        w = torch.randint(0, 256, (m, N), dtype=torch.uint8, device="cuda", generator=gen)
+        s = (torch.randn((m, N // ff.GROUP), device="cuda", generator=gen) * 0.001).abs().to(torch.bfloat16)
+        b = (-128.0 * s.float() + torch.randn((m, N // ff.GROUP), device="cuda", generator=gen) * 1e-3).to(torch.bfloat16)
+        x = torch.randn((16, N), device="cuda", generator=gen).to(dt)
+        at = torch.tensor([0, 15, 16, 4097, 65535, 100000, m - 17, m - 1], device="cuda")
+        large = ctx.matrix_int8(w, s, b)
+        few = ctx.matrix_int8(*[p[at].contiguous() for p in (w, s, b)])
+        scale, bias = (p[at].double().repeat_interleave(ff.GROUP, 1) for p in (s, b))
+        want = x.double() @ (scale * w[at].double() + bias).T
+        for rows in (1, 4, 5, 16):
+            y = large.gemv(x[:rows], f32_out=True)
+            assert torch.equal(y[:, at], few.gemv(x[:rows], f32_out=True))
+            assert torch.equal(large.gemv(x[:rows])[:, at], few.gemv(x[:rows]))
+            # (the nibbles enter as 128 + q, 1024 + q in FP16, and spread by 4.6: four roundings of such a sum)
+            usual = 4 * ((1024 if act == "fp16" else 128) + 8) / 4.6 * 2.0 ** -24
+            assert (y[:, at].double() - want[:rows]).norm() <= usual * want[:rows].norm(), rows
     finally:
         ctx.close()
 
