@@ -186,8 +186,8 @@ __device__ __forceinline__ SoftmaxAcc softmax_shuffle(const SoftmaxAcc &a, int m
 // two streams.
 // FEW (up to four input rows of the plain form): input row t is operand row 4 t, so that one of a lane's four sums is all there is to
 // keep up, and each operand lane loads its own bytes: the lanes of a row ask for the same ones, there is nothing to turn through LDS.
-// 1 row, us without | so: 16,384 x 1,408 6.7 | 5.9, 16,384 x 2,816 7.2 | 6.8, 262,144 x 2,816 76.5 | 74.9 (5.5 TB/s).
-// ONCE: the matrix is more than the memory side's cache holds (kReadOnce).
+// 1 row, us without | so: 16,384 x 1,408 6.7 | 5.9, 16,384 x 2,816 7.2 | 6.8, 262,144 x 2,816 76.5 | 74.9.
+// ONCE: the matrix is more than the memory side's cache holds (kReadOnce); with it the last of those takes 66.6 (6.2 TB/s).
 template <bool Y_F32, bool F16, bool GREEDY = false, bool CONF = false, bool PLANES8 = false, int GLU = 0, bool FEW = false, bool ONCE = false>
 __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__restrict__ tiles,
                                                              const uint8_t *__restrict__ scales, uint32_t m,
@@ -868,7 +868,12 @@ hipError_t launch_matrix_gemv(hipStream_t s, const uint8_t *tiles, const uint8_t
                 else { if (y_f32) FFMOE_MGEMV(true, false, false, 0, false, O); else FFMOE_MGEMV(false, false, false, 0, false, O); }
             }
         };
-        if (!twice && (size_t)n_tiles * (n / kGroup) * kTileBytes > kMemoryCacheBytes) pick(std::true_type{}); else pick(std::false_type{});
+        // Read once from the memory side's cache on; 4 bits with more than four input rows, which take longer over their bytes, from a sixteenth more
+        // on. us without the hint | with, N = 2,112: 4 bits, 1 row, 270 MB 61.3 | 61.0, 277 MB 58.6 | 56.5, 338 MB 74.2 | 68.1; 16 rows, 270 MB 68.8 | 74.1,
+        // 277 MB 67.1 | 68.7, 290 MB 74.4 | 73.9, 338 MB 88.8 | 84.3; 8 bits, 1 row, 259 MB 55.0 | 53.3, 277 MB 62.1 | 60.2, 16 rows, 259 MB 56.0 | 55.9, 277 MB
+        // 65.9 | 65.8, 338 MB 86.6 | 81.1.
+        const size_t once_from = planes8 || rows <= 4 ? kMemoryCacheBytes : kMemoryCacheBytes / 16 * 17;
+        if (!twice && (size_t)n_tiles * (n / kGroup) * kTileBytes > once_from) pick(std::true_type{}); else pick(std::false_type{});
     }
 #undef FFMOE_MGEMV
     return hipGetLastError();
@@ -1028,6 +1033,7 @@ hipError_t launch_matrix_greedy(hipStream_t s, const uint8_t *tiles, const uint8
 #define FFMOE_GREEDY(H, C)                                                                                                  \
     hipLaunchKernelGGL((once ? matrix_gemv_kernel<true, H, true, C, false, 0, false, true> : matrix_gemv_kernel<true, H, true, C>), grid, dim3(256), 0, s, \
                        tiles, scales, m, n / kGroup, x, x_stride, rows, partials, 0u, conf_part, softcap)
+    // (16 rows, N = 2,112, us without the hint | with: 259 MB 62.7 | 62.8, 270 MB 69.6 | 70.4, 301 MB 76.2 | 75.4, 338 MB 84.8 | 82.8)
     const bool once = (size_t)((m + 31) / 32) * (n / kGroup) * kTileBytes > kMemoryCacheBytes;
     if (f16) { if (out_conf) FFMOE_GREEDY(true, true); else FFMOE_GREEDY(true, false); }
     else { if (out_conf) FFMOE_GREEDY(false, true); else FFMOE_GREEDY(false, false); }

@@ -4,11 +4,10 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-N = 2112                                            # 262,144 x 2,112 in 4 bits, 131,072 x 2,112 in 8: 277 MB
-
-
+# 262,144 rows in 4 bits, 131,072 in 8: 277 MB at 2,112 columns, where 4 bits are read so for up to four rows, and 294 MB at 2,240
+@pytest.mark.parametrize("N", [2112, 2240])
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
-def test_rows_of_a_large_matrix(act):
+def test_rows_of_a_large_matrix(act, N):
     import torch
     import fieldfare_moe as ff
     from fieldfare_moe import synthetic as syn
@@ -39,7 +38,7 @@ def test_rows_of_a_large_matrix(act):
 
 
 @pytest.mark.parametrize("act", ["bf16", "fp16"])
-def test_rows_of_a_large_8bit_matrix(act):
+def test_rows_of_a_large_8bit_matrix(act, N=2112):
     import torch
     import fieldfare_moe as ff
     gen = torch.Generator(device="cuda")
