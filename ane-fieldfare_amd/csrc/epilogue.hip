@@ -25,6 +25,10 @@ namespace {
 
 constexpr int kRowThreads = 256;
 constexpr int kMaxChunks = 2;        // D <= 4096: at most two 8-element chunks per thread
+// Up to how many rows the tail converts before its first reduction: four of its blocks run on a compute unit then, two with the norms. us, late |
+// early, 2,816 columns: 1 row 3.03 | 2.98, 100 rows 3.34 | 3.28, 301 rows 4.18 | 4.02, 1,000 rows 5.82 | 5.56 (3,072 rows 12.9 | 13.4); 4,096 columns, 1,000 rows
+// 6.66 | 6.27; with the norms 301 rows 5.84 | 5.66, 500 rows 6.19 | 6.02 (1,000 rows 9.2 | 9.8, 8,192 rows 41 | 57).
+constexpr uint32_t kEarlyRows = 1024, kEarlyNormRows = 512;
 
 struct Row8 {
     float v[8];
@@ -237,7 +241,9 @@ __device__ __forceinline__ Row8 combine8(const RoutedChunk &in, uint32_t top_k, 
 // COMBINE: rows of more than 256 chunks have a thread per chunk for the combining, which is 24 loads of 16 bytes for one: those past the
 // 256th hand their chunks, rounded to 16 bits as they are, to the threads that own them in the order of the sums. 1 row of
 // 2,816, us per launch: both chunks by their owner, each behind its own chain of loads 5.9, so 4.6.
-template <bool VEC, bool NORMS, bool F16, bool COMBINE = false>
+// EARLY: a thread's chunks are fp32 numbers, and only where it has them, before the first reduction, in 123 registers (171 with NORMS); else they stay
+// as they came, in 62 (74), and are converted behind each. The first is the shorter chain, the second more blocks per compute unit: kEarlyRows.
+template <bool VEC, bool NORMS, bool F16, bool COMBINE = false, bool EARLY = false>
 __global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer_tail_kernel(const uint16_t *__restrict__ h1, uint16_t *__restrict__ hidden,
                                                                  const uint16_t *__restrict__ w_postffn2,
                                                                  const uint16_t *__restrict__ w_postffn,
@@ -310,6 +316,7 @@ __global__ __launch_bounds__(COMBINE ? 2 * kRowThreads : kRowThreads) void layer
             }
 #pragma unroll
         for (int c = 0; c < kMaxChunks; ++c) {
+            if (EARLY && (uint32_t)c >= n_mine) break;
             a[c] = widen8<F16>(a_raw[c]);
             h12[c] = widen8<F16>(h1_raw[c]);
             hv[c] = widen8<F16>(h_raw[c]);
@@ -379,6 +386,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_kernel(const uint16_t *x,
     Row8 a[kMaxChunks], wq[kMaxChunks];
 #pragma unroll
     for (int c = 0; c < kMaxChunks; ++c) {
+        if ((uint32_t)c >= n_mine) break;       // (early: 51 registers, eight waves per SIMD either way; 1,000 rows of 2,816 3.48 -> 3.36 us)
         a[c] = widen8<F16>(a_raw[c]);
         wq[c] = widen8<false>(w_raw[c]);
     }
@@ -439,20 +447,21 @@ hipError_t launch_layer_tail(hipStream_t s, const uint16_t *h2, uint32_t h2_stri
     const bool vec = aligned16(h2, h2_stride) && aligned16(h1, h1_stride) && aligned16(hidden, hidden_stride) &&
                      aligned16(w_postffn2, 8) && aligned16(w_postffn, 8) &&
                      (!norms || (aligned16(w_postffn1, 8) && (!w_next || (aligned16(w_next, 8) && aligned16(normed, normed_stride)))));
+    // (as many rows as blocks of the early form that run at once)
+    const bool early = t <= (norms ? kEarlyNormRows : kEarlyRows);
+#define FFMOE_TAIL_AS(V, N, H, E)                                                                                     \
+    hipLaunchKernelGGL((layer_tail_kernel<V, N, H, false, E>), dim3(t), dim3(kRowThreads), 0, s, h1, hidden, w_postffn2, \
+                       w_postffn, h2, h2_stride, h1_stride, hidden_stride, d, eps, layer_scalar, w_postffn1, w_next, normed, \
+                       normed_stride, routed)
 #define FFMOE_TAIL(V, N)                                                                                              \
     do {                                                                                                              \
-        if (f16)                                                                                                      \
-            hipLaunchKernelGGL((layer_tail_kernel<V, N, true>), dim3(t), dim3(kRowThreads), 0, s, h1, hidden, w_postffn2, \
-                               w_postffn, h2, h2_stride, h1_stride, hidden_stride, d, eps, layer_scalar, w_postffn1, w_next, normed, \
-                               normed_stride, routed);                                                                \
-        else                                                                                                          \
-            hipLaunchKernelGGL((layer_tail_kernel<V, N, false>), dim3(t), dim3(kRowThreads), 0, s, h1, hidden, w_postffn2, \
-                               w_postffn, h2, h2_stride, h1_stride, hidden_stride, d, eps, layer_scalar, w_postffn1, w_next, normed, \
-                               normed_stride, routed);                                                                \
+        if (f16) { if (early) FFMOE_TAIL_AS(V, N, true, true); else FFMOE_TAIL_AS(V, N, true, false); }               \
+        else { if (early) FFMOE_TAIL_AS(V, N, false, true); else FFMOE_TAIL_AS(V, N, false, false); }                 \
     } while (0)
     if (vec) { if (norms) FFMOE_TAIL(true, true); else FFMOE_TAIL(true, false); }
     else { if (norms) FFMOE_TAIL(false, true); else FFMOE_TAIL(false, false); }
 #undef FFMOE_TAIL
+#undef FFMOE_TAIL_AS
     return hipGetLastError();
 }
 

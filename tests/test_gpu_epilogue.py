@@ -251,3 +251,32 @@ def test_tail_of_uncombined_rows_equals_separate_steps(oracle, torch, d, top_k, 
     ctx.layer_tail_routed(w, h1, hidden, w2, w1, 0.5)
     assert torch.equal(hidden.view(torch.int16), want.view(torch.int16))
     ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("d,pad", [(256, 0), (2048, 0), (2056, 0), (2816, 3), (4096, 0)])
+def test_tail_rows_do_not_depend_on_how_many_there_are(torch, d, pad, act):
+    # either side of 512 and of 1,024 rows, where the tail changes its form; rows in 16-byte order and (pad) not
+    import fieldfare_moe as ff
+    rng = torch.Generator(device="cuda")
+    rng.manual_seed(d + pad)
+    ctx = ff.Context(128, 64, 4, 2, n_layers=1, max_tokens=16, act_dtype=act)
+    try:
+        rnd = lambda *shape: torch.randn(shape, device="cuda", generator=rng)
+        rows = lambda: rnd(1025, d + pad).to(ctx.act)[:, :d]
+        h2, h1, hidden = rows(), rows(), rows()
+        w1, w2, w, w_next = (rnd(d).to(torch.bfloat16) for _ in range(4))
+        for norms in (False, True):
+            seen = None
+            for t in (1025, 1024, 513, 512, 1):
+                h = torch.empty((t, d + pad), device="cuda", dtype=ctx.act)[:, :d].copy_(hidden[:t])
+                if norms:
+                    out = (ctx.layer_tail_norms(h2[:t], h1[:t], h, w1, w2, w, 0.5, w_next=w_next, d=d), h)
+                else:
+                    ctx.layer_tail(h2[:t], h1[:t], h, w2, w, 0.5, d=d)
+                    out = (h,)
+                assert all(torch.isfinite(o.float()).all() for o in out)
+                seen = seen or out
+                assert all(torch.equal(o, s[:t]) for o, s in zip(out, seen)), (norms, t)
+    finally:
+        ctx.close()
