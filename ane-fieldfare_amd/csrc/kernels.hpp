@@ -236,7 +236,8 @@ hipError_t launch_argmax_rows(hipStream_t s, const float *logits, uint32_t strid
                               uint32_t *out, float *out_conf, SampleScratch sc);
 
 // The most pairs per expert, on average, at which a prefill chunk takes the streaming product, and the M-tiles that a
-// scratch for `max_pairs` pairs has to hold: that product's tiles go down to 32 pairs, the GEMMs' to as many as there are compute
+// scratch for `max_pairs` pairs has to hold: that product's tiles go down to 32 pairs, and to 16 where the experts have five on average or fewer
+// (5 / 16 n_experts full ones at most, and a shorter one per expert), the GEMMs' to as many as there are compute
 // units (prefill_tile_form, gemm_tile_rows in prefill.hip).
 constexpr uint32_t kPrefillStreamPairs = 48;
 constexpr uint32_t kDenseTileStreamRows = 896;       // and the most rows at which a dense FFN's chunk does

@@ -1565,7 +1565,7 @@ struct TileForm {
     uint32_t rows;
 };
 TileForm prefill_tile_form(uint32_t n_items, uint32_t n_experts, const ArenaGeom &g, uint32_t n_nblocks, uint32_t n_cus, uint32_t max_tiles, bool f16) {
-    // (a scratch holds 2.5 tiles per expert)
+    // (1.32 tiles per expert at most, of the 2.5 that a scratch holds)
     if (!f16 && n_items <= 5 * n_experts && n_nblocks * n_experts > 4 * n_cus && n_nblocks * n_experts <= 6 * n_cus) return {true, 16};
     if (n_items <= 28 * n_experts) return {true, 32};
     if (n_items <= kPrefillStreamPairs * n_experts) {
