@@ -1002,24 +1002,29 @@ __global__ __launch_bounds__(64 * kGemmTiles, 2 * GemmLds<LC>::kBlocks) void pre
 // Grouped product for chunks whose experts hold few pairs each (a short prompt): the GEMM's tiles and activation layout, N-blocks of
 // four arena tiles, another way through them. There the expansion to 16-bit weights (68 vector instructions per 1 KiB tile of
 // a wave, whatever the pairs, in front of its products) bounds the launch below about 50 pairs per expert: with the GEMMs that this
-// form was built beside, 90 us for the 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s. Here a wave owns one arena tile row for the whole of K, streams its
+// form was built beside, 90 us for the 260 MB of a 37-row chunk's gate/up weights, 2.9 TB/s (here 47). Here a wave owns one arena tile row for the whole of K, streams its
 // packed tiles through a ring of four and multiplies them in the offset form of the decode kernels (stream.hpp): about 52
 // vector instructions per tile at 32 pairs, no expansion in LDS, the weights un-rounded. From two 16-pair blocks on the groups' input
 // sums are made once per block of waves, each wave its share, and come in by outer products on the matrix unit: per 16 pairs, tile and
-// group 80 cycles of it instead of 96, and 8 vector instructions instead of 16, for one more barrier per 128 columns. The sums
+// group 80 cycles of it instead of 96, and 8 vector instructions instead of 16. The sums
 // are the same and the order is a group's scale, then its bias (with the offset's correction): four groups' biases as one product of K = 4 would
 // be 2 to 4 % faster again, but carries 128 times four groups' inputs in a sum at once, which is two bits less of it. 128 experts of
 // 2,816 x 704, top-8, router table to combined rows, us with every wave's own sums | so: 301 rows 115.7 | 113.6, 448 rows 135.5 | 131.1,
 // 576 rows 152.6 | 148.1, 736 rows 170.7 | 165.7 (FP16 123.7 | 121.9, 138.2 | 133.1, 159.4 | 156.8, 180.9 | 175.8); 64 of 320 x 192, 30
-// pairs each, 17.8 | 18.4. The pairs' rows go through LDS in
-// operand order, two groups at a time in two buffers, so that every wave of the block reads the same fragments and the
-// registers hold one chunk's 16-byte pieces in flight; the weights stay in flight across the barriers. Gate/up of 37 rows
-// 90 -> 56 us (4.7 TB/s). What bounds it then is the weights' bytes (32 pairs per tile) and the matrix and vector instructions
-// together (64).
+// pairs each, 17.8 | 18.4. The pairs' rows go straight into LDS, two groups at a time in a ring of four buffers (three for tiles of 64
+// pairs, whose LDS is three blocks'), as lines of 128 bytes with their pieces turned by the row, so that every wave of the block
+// reads the same fragments without conflicts and no register, store or address of theirs is on the waves' way; the weights stay in
+// flight across the barriers, of which there is one per two groups. A step asks for its fragments in front of the 28 instructions that unpack its
+// weights. (Rows through registers and two barriers, each fragment asked for where it is used: 248 vector instructions per four steps of
+// 32 pairs, now 229. Three layers in turn, us of gate/up + down: 93 experts with 19 pairs each 55.5 + 31.1, now 50.9 + 30.5; 128 with 32
+// 73.2 + 44.0 | 69.1 + 43.1, with 12 55.2 + 33.0 | 53.3 + 31.6, with 4 (tiles of 16) 48.5 + 29.7 | 48.9 + 28.4; a prompt of 301 rows 63.2 + 36.5 |
+// 60.0 + 36.7. The same order of a step with the rows still through registers spills them: 48 experts with 19 pairs 33 -> 44 us.) What
+// bounds it then is the weights' bytes (4.8 TB/s at 19 pairs with four blocks per unit) and the matrix and vector instructions
+// together (64 pairs).
 // A pair's arithmetic does not depend on its tile: any two launches of this kernel give the same row bit for bit.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kStreamDepth = 4;                                             // weight tiles in flight per wave
-constexpr int kStreamChunk = 2;                                             // groups whose rows are in LDS at a time, twice
+constexpr int kStreamChunk = 2;                                             // groups per buffer of rows, and per barrier
 constexpr uint32_t kStreamStageRow = 2 * kTilesPerBlock * kTileRows * 2 + 16;   // bytes: 128 output columns + padding
 
 // The eight nibbles of a dword as matrix operands. bf16: 128 + q, as in the decode kernels. FP16: the subnormal q * 2^-24. With
@@ -1031,68 +1036,55 @@ __device__ __forceinline__ uint4 unpack8_stream(uint32_t w) {
     else return unpack8_offset<false>(w);
 }
 
-template <bool GATE_UP, int NM, bool F16, bool ONCE>
+// LDS of a block whose tiles have up to MAX_NM 16-pair blocks: buffers of a chunk of the pairs' rows each, then the groups' input sums.
+template <int MAX_NM>
+struct StreamLds {
+    static constexpr int kBufs = MAX_NM <= 2 ? 4 : 3;                   // one in use, one whose sums are made, the others on their way
+    static constexpr uint32_t kGroupBytes = 16 * MAX_NM * kGroup * 2, kBufBytes = kStreamChunk * kGroupBytes;
+    static constexpr uint32_t kSumsAt = kBufs * kBufBytes, kBytes = kSumsAt + 2 * MAX_NM * kStreamChunk * 16 * 4;
+};
+
+template <bool GATE_UP, int NM, bool F16, bool ONCE, int MAX_NM>
 __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom &g, const TileSource &src, uint32_t tile0,
-                                            uint4 *__restrict__ lds, const uint32_t *__restrict__ sorted_token,
+                                            uint8_t *lds, uint32_t lds_base, const uint32_t *__restrict__ sorted_token,
                                             const uint32_t *__restrict__ sorted_out_row, uint16_t *__restrict__ out,
                                             float *__restrict__ act_scale) {
-    constexpr int CHUNK = kStreamChunk;
-    static_assert(2 * CHUNK % kStreamDepth == 0, "a group's ring slot follows from its place in a pair of chunks");
-    constexpr int kFrags = 2 * CHUNK;                     // operand fragments of a 16-pair block in a chunk
-    constexpr int kRowPieces = 8 * CHUNK;                 // 16-byte pieces of a row in a chunk
-    constexpr int kPassRows = 256 / kRowPieces;           // rows that the block's threads load at a time
-    constexpr int kPieces = 16 * NM / kPassRows;          // pieces of A per thread and chunk
-    constexpr int kBuf = NM * kFrags * kWave;             // one LDS buffer, in pieces
+    using L = StreamLds<MAX_NM>;
+    constexpr int CHUNK = kStreamChunk, kAhead = L::kBufs - 1;
+    static_assert(CHUNK == 2 && 2 * CHUNK % kStreamDepth == 0, "a group's ring slot follows from its place in a pair of chunks; two waves per group of a chunk");
+    constexpr uint32_t kGroupBytes = NM * 2048;           // a group of the tile's rows in LDS
     const uint32_t lane = gw.lane, wave = gw.wave, j = lane & 15, jq = lane >> 4, tid = threadIdx.x;
     const uint32_t n_groups = gw.n_groups, last = n_groups - 1;
     const uint32_t n_chunks = (n_groups + CHUNK - 1) / CHUNK;
-    static_assert(16 * NM * kStreamStageRow <= 2 * kBuf * sizeof(uint4), "the down epilogue's rows fit in front of the sums");
-    static_assert(NM * 2 * kWave * sizeof(uint4) + 4 * 16 * NM * sizeof(float) <= 2 * kBuf * sizeof(uint4), "so do the activations and the peaks");
+    static_assert(16 * NM * kStreamStageRow <= L::kSumsAt, "the down epilogue's rows fit in front of the sums");
+    static_assert(NM * 2 * kWave * sizeof(uint4) + 4 * 16 * NM * sizeof(float) <= L::kSumsAt, "so do the activations and the peaks");
 
-    // Where this thread's pieces of a chunk come from and go to.
-    // GATE_UP: row tid / kRowPieces + kPassRows k of the tile, piece tid % kRowPieces of its contiguous bytes; in LDS piece p of row r sits
-    // in fragment p / 4 at (p % 4, (r + p) % 16): the 16 pieces that 16 neighbouring lanes store then fall on 16
-    // different 16-byte columns, and so do the 16 rows that a fragment read takes.
-    // else: the activations are in fragment order already, the chunk of a 16-pair block is contiguous.
-    const uint16_t *from[GATE_UP ? kPieces : 1];
-    const uint32_t p = tid % kRowPieces, row0 = tid / kRowPieces;
-    if constexpr (GATE_UP) {
+    // The pairs' rows go straight into LDS, 1 KiB per load, NM loads per wave and chunk. GATE_UP: eight rows of 128 bytes (one group),
+    // eight neighbouring lanes per row; 16-byte piece c of row r lies at piece c ^ (r % 8), so that the sixteen rows of a fragment
+    // fall on different banks. else: the activations are in fragment order already.
+    const uint16_t *from[NM];
 #pragma unroll
-        for (int k = 0; k < kPieces; ++k) {
-            const uint32_t row = min(row0 + kPassRows * k, gw.tile.rows - 1);
-            from[k] = gw.a + (size_t)sorted_token[gw.tile.row_start + row] * gw.a_stride + (p & 7) * 8;
+    for (int k = 0; k < NM; ++k) {
+        const uint32_t piece = (wave + 4 * k) % (2 * NM);
+        if constexpr (GATE_UP) {
+            const uint32_t row = min(piece * 8 + (lane >> 3), gw.tile.rows - 1);
+            from[k] = gw.a + (size_t)sorted_token[gw.tile.row_start + row] * gw.a_stride + 8 * ((lane & 7) ^ (lane >> 3));
+        } else {
+            from[k] = gw.a + ((size_t)(gw.act_block0 + (piece >> 1)) * n_groups * 2 + (piece & 1)) * (kWave * 8) + lane * 8;
         }
-    } else {
-        from[0] = gw.a + (size_t)gw.act_block0 * n_groups * (2 * kWave * 8) + (tid & 127) * 8;
     }
-    u32x4_t stage[kPieces];        // (a native vector type: it stays in registers)
-    auto load_a = [&](uint32_t chunk) __attribute__((always_inline)) {
+    auto load_a = [&](uint32_t chunk, uint32_t buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < kPieces; ++k) {
-            if constexpr (GATE_UP) {
-                const uint32_t grp = min(chunk * CHUNK + (p >> 3), last);        // past the end: the last group again, never used
-                stage[k] = *reinterpret_cast<const u32x4_t *>(from[k] + grp * kGroup);
-            } else {
-                const uint32_t grp = min(chunk * CHUNK + 2 * k % CHUNK + (tid >> 7), last);
-                stage[k] = *reinterpret_cast<const u32x4_t *>(from[0] + ((size_t)(2 * k / CHUNK) * n_groups + grp) * (2 * kWave * 8));
-            }
+        for (int k = 0; k < NM; ++k) {
+            const uint32_t gl = (wave + 4 * k) / (2 * NM), piece = (wave + 4 * k) % (2 * NM);
+            const uint32_t grp = min(chunk * CHUNK + gl, last);         // past the end: the last group again, never used
+            global_to_lds_16(from[k] + (size_t)grp * (GATE_UP ? kGroup : 2 * kWave * 8), lds_base + buf + gl * kGroupBytes + piece * 1024);
         }
     };
-    auto store_a = [&](uint32_t buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < kPieces; ++k) {
-            if constexpr (GATE_UP) {
-                const uint32_t row = row0 + kPassRows * k;
-                lds[buf * kBuf + ((row >> 4) * kFrags + (p >> 2)) * kWave + (p & 3) * 16 + ((row + p) & 15)] = __builtin_bit_cast(uint4, stage[k]);
-            } else {
-                lds[buf * kBuf + 256 * k + tid] = __builtin_bit_cast(uint4, stage[k]);
-            }
-        }
-    };
-    // fragment f of 16-pair block m, this lane's 16 bytes of it
-    auto frag = [&](uint32_t buf, int m, int f) __attribute__((always_inline)) {
-        const uint32_t at = GATE_UP ? jq * 16 + ((j + jq + 4 * (f & 3)) & 15) : lane;
-        return lds[buf * kBuf + (m * kFrags + f) * kWave + at];
+    // fragment f of 16-pair block m, this lane's 16 bytes of it: k-half f % 2 of group f / 2 of the chunk whose buffer `at` and `at64` lie in
+    const uint32_t at0 = GATE_UP ? j * 128 + 16 * (jq ^ (j & 7)) : lane * 16, at1 = GATE_UP ? at0 ^ 64 : at0 + 1024;
+    auto frag = [&](uint32_t at, int m, int gl) __attribute__((always_inline)) {
+        return *reinterpret_cast<const uint4 *>(lds + at + gl * kGroupBytes + m * 2048);
     };
 
     uint4 ring_t[kStreamDepth];
@@ -1104,6 +1096,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         ring_t[u] = make_uint4(t.x, t.y, t.z, t.w);
         ring_s[u] = make_uint2(s.x, s.y);
     };
+    constexpr int kFillLoads = 2;
     // the sums of two 16-pair blocks (or of the one): stream a and stream b of each, as the bias product's result has them
     constexpr bool kShared = NM > 1;
     constexpr int kPairs = (NM + 1) / 2;
@@ -1116,24 +1109,46 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     // The groups' input sums, a value per pair in LDS ([chunk % 2][16-pair block][group of the chunk][pair]): every wave makes its
     // share of a chunk's while the block is at the chunk before. (Of one 16-pair block every wave makes its own: two instructions
     // against a barrier, 37 rows of 128 experts 104.6 | 102.1 us.)
-    float *const sums = reinterpret_cast<float *>(lds + 2 * kBuf);
+    float *const sums = reinterpret_cast<float *>(lds + L::kSumsAt);
     constexpr int kSums = (NM + 1) / 2;                   // 16-pair blocks per wave, of one of the chunk's two groups
-    static_assert(CHUNK == 2, "two waves per group of a chunk");
-    auto sum_up = [&](uint32_t buf, int slot) __attribute__((always_inline)) {
-        const int gl = wave & 1;
+    const uint32_t sum_gl = wave & 1;
+    auto sum_block = [&](int k) __attribute__((always_inline)) { return min((wave >> 1) + 2u * k, NM - 1u); };
+    uint4 sum_x[kSums][2];
+    auto sum_read = [&](uint32_t buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < kSums; ++k) {
-            const int m = min((int)(wave >> 1) + 2 * k, NM - 1);
-            const f32x4 sx = group_input_sum<F16>(frag(buf, m, 2 * gl), frag(buf, m, 2 * gl + 1));
-            if (j == 0) *reinterpret_cast<f32x4 *>(sums + ((slot * NM + m) * CHUNK + gl) * 16 + 4 * jq) = sx;
+            const uint32_t here = buf + sum_gl * kGroupBytes + sum_block(k) * 2048;
+            sum_x[k][0] = frag(at0 + here, 0, 0), sum_x[k][1] = frag(at1 + here, 0, 0);
+        }
+    };
+    auto sum_up = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kSums; ++k) {
+            const f32x4 sx = group_input_sum<F16>(sum_x[k][0], sum_x[k][1]);
+            if (j == 0) *reinterpret_cast<f32x4 *>(sums + ((slot * NM + sum_block(k)) * CHUNK + sum_gl) * 16 + 4 * jq) = sx;
         }
     };
 
-    auto step = [&](uint32_t buf, int slot, int gl, int u, uint32_t refill) __attribute__((always_inline)) {
+    // One group. What it reads of LDS is asked for in front of the unpacking, which covers the way; the ring's slot is filled again behind it,
+    // when its registers are free. NEXT >= 0: on the way the wave's share of the next chunk's sums, from buffer `next`, for that slot.
+    auto step = [&](uint32_t cur, uint32_t next_buf, int slot, int gl, int u, uint32_t refill, auto next_sums) __attribute__((always_inline)) {
+        constexpr int kNext = decltype(next_sums)::value;
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        uint4 x[2][2][2];                                   // of a pair of 16-pair blocks, and of the next pair
+        auto read_x = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                if (2 * i + q < NM) x[i & 1][q][0] = frag(cur + at0, 2 * i + q, gl), x[i & 1][q][1] = frag(cur + at1, 2 * i + q, gl);
+        };
+        read_x(0);
+        float both[kPairs];
+#pragma unroll
+        for (int i = 0; i < kPairs; ++i)
+            if (kShared) both[i] = sums[((slot * NM + 2 * i) * CHUNK + gl) * 16 + (2 * i + 1 < NM ? (lane >> 5) * (CHUNK * 16) : 0) + j];
+        if (kNext >= 0) sum_read(next_buf);
+        __builtin_amdgcn_sched_barrier(0);
         const uint4 tile = ring_t[u];
         const uint2 sc = ring_s[u];
-        fill(u, refill);
         const uint4 wa0 = unpack8_stream<F16>(tile.x), wa1 = unpack8_stream<F16>(tile.y);
         const uint4 wb0 = unpack8_stream<F16>(tile.z), wb1 = unpack8_stream<F16>(tile.w);
         float sa = bf16lo_to_f32(sc.x), sb = bf16lo_to_f32(sc.y), ta = bf16hi_to_f32(sc.x), tb = bf16hi_to_f32(sc.y);
@@ -1145,74 +1160,86 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
             tb = __builtin_fmaf(-Act<F16>::kOffset, sb, tb);
         }
         const float bias = jq & 1 ? tb : ta;
+        __builtin_amdgcn_sched_barrier(0);
+        fill(u, refill);
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            auto &t = tot[m / 2];
-            const int at = 8 * (m & 1);
-            const uint4 x0 = frag(buf, m, 2 * gl), x1 = frag(buf, m, 2 * gl + 1);
-            f32x4 sx = zero;
-            if (!kShared) sx = group_input_sum<F16>(x0, x1);
-            f32x4 aa = Act<F16>::mfma(x0, wa0, zero);
-            aa = Act<F16>::mfma(x1, wa1, aa);
-            f32x4 ab = Act<F16>::mfma(x0, wb0, zero);
-            ab = Act<F16>::mfma(x1, wb1, ab);
+        for (int i = 0; i < kPairs; ++i) {
+            auto &t = tot[i];
+            const int n = 2 * i + 1 < NM ? 2 : 1;
+            if (i + 1 < kPairs) read_x(i + 1);
+            f32x4 aa[2], ab[2], sx = zero;
+            if (!kShared) sx = group_input_sum<F16>(x[0][0][0], x[0][0][1]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                t[at + r] = __builtin_fmaf(sa, aa[r], t[at + r]);
-                t[at + 4 + r] = __builtin_fmaf(sb, ab[r], t[at + 4 + r]);
-                if (!kShared) t[at + r] = __builtin_fmaf(ta, sx[r], t[at + r]), t[at + 4 + r] = __builtin_fmaf(tb, sx[r], t[at + 4 + r]);
-            }
-            if (kShared && (m & 1) == 0 && m + 1 < NM) continue;
+            for (int q = 0; q < n; ++q) aa[q] = Act<F16>::mfma(x[i & 1][q][0], wa0, zero), ab[q] = Act<F16>::mfma(x[i & 1][q][0], wb0, zero);
+#pragma unroll
+            for (int q = 0; q < n; ++q) aa[q] = Act<F16>::mfma(x[i & 1][q][1], wa1, aa[q]), ab[q] = Act<F16>::mfma(x[i & 1][q][1], wb1, ab[q]);
+            if (i == 0 && kNext >= 0) sum_up(kNext);
+#pragma unroll
+            for (int q = 0; q < n; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    t[8 * q + r] = __builtin_fmaf(sa, aa[q][r], t[8 * q + r]);
+                    t[8 * q + 4 + r] = __builtin_fmaf(sb, ab[q][r], t[8 * q + 4 + r]);
+                    if (!kShared) t[r] = __builtin_fmaf(ta, sx[r], t[r]), t[4 + r] = __builtin_fmaf(tb, sx[r], t[4 + r]);
+                }
             // four outer products of 16 sums by 16 biases, lane (j, jq) has both for block jq: t + bias * sum, rounded once as by an fma
-            if constexpr (kShared) {
-                const float both = sums[((slot * NM + (m & ~1)) * CHUNK + gl) * 16 + (m & 1 ? (lane >> 5) * (CHUNK * 16) : 0) + j];
-                t = __builtin_amdgcn_mfma_f32_16x16x1f32(both, bias, t, 0, 0, 0);
-            }
+            if constexpr (kShared) t = __builtin_amdgcn_mfma_f32_16x16x1f32(both[i], bias, t, 0, 0, 0);
             // pinned: left alone, the compiler collects the scales' arithmetic of several groups and carries all
             // their matrix results there, which does not fit the register budget
             asm volatile("" : "+v"(t));
         }
     };
 
-    load_a(0);
+    // Chunk c lies in buffer c % kBufs. While the block is at it the loads of chunk c + kAhead go into the buffer of the chunk before, and
+    // (kShared) chunk c + 1 is there already, for its sums. One barrier per chunk, at its end: it waits for the loads of the chunk
+    // that is needed next, i.e. for all but those that every wave has asked for since, always the same number: chunk by chunk NM of rows, then
+    // one fill per group (the loads in front of the loop go out in that order too).
+    constexpr int kChunkFills = CHUNK * kFillLoads;
+    constexpr int kInFlight = kShared ? kChunkFills * (kAhead - 1) + NM * (kAhead - 2) : kChunkFills * kAhead + NM * (kAhead - 1);
+    static_assert(kStreamDepth == 2 * CHUNK, "two chunks' fills in front of the loop");
+    uint32_t cur = 0, next_buf = L::kBufBytes;
 #pragma unroll
-    for (int u = 0; u < kStreamDepth; ++u) fill(u, u);
-    store_a(0);
-    load_a(min(1u, n_chunks - 1));
-    lds_barrier();
+    for (int a = 0; a < kAhead; ++a) {
+        load_a(min((uint32_t)a, n_chunks - 1), a * L::kBufBytes);
+        if (a >= kAhead - 2)
+#pragma unroll
+            for (int q = 0; q < CHUNK; ++q) fill((a - (kAhead - 2)) * CHUNK + q, (a - (kAhead - 2)) * CHUNK + q);
+    }
+    // (the first chunk, and kShared the second: less is in flight behind the first than there will be)
+    ring_barrier<kShared ? (kAhead == 2 ? kChunkFills : 2 * kChunkFills + NM * (kAhead - 2)) : 2 * kChunkFills + NM * (kAhead - 1)>();
     if constexpr (kShared) {
-        sum_up(0, 0);
+        sum_read(0);
+        sum_up(0);
         lds_barrier();
     }
-    // chunk c from LDS buffer c % 2; chunk c + 1 goes from registers into the other one, chunk c + 2 into the registers.
-    // Two barriers per chunk (one where no sums are shared). In its middle: the stores of chunk c + 1 in front of its sums; at its end: the sums and stores in
-    // front of their reads, the reads of chunk c in front of the stores of chunk c + 2 into the same buffer.
     auto chunk = [&](uint32_t c, auto parity, auto whole) __attribute__((always_inline)) {
         constexpr int kParity = decltype(parity)::value;
-        store_a(kParity ^ 1);           // (past the last chunk: a buffer nobody reads)
-        load_a(min(c + 2, n_chunks - 1));
-#pragma unroll
-        for (int gl = 0; gl < CHUNK; ++gl) {
-            const uint32_t grp = c * CHUNK + gl;
-            if (decltype(whole)::value || grp < n_groups) step(kParity, kParity, gl, (kParity * CHUNK + gl) % kStreamDepth, grp + kStreamDepth);
-            if (kShared || gl == CHUNK - 1) lds_barrier();
-            if (kShared && gl == 0) sum_up(kParity ^ 1, kParity ^ 1);      // (of a group past the last: not used)
-        }
+        using Sums = std::integral_constant<int, kShared ? kParity ^ 1 : -1>;
+        using None = std::integral_constant<int, -1>;
+        const uint32_t before = cur ? cur - L::kBufBytes : kAhead * L::kBufBytes;
+        load_a(min(c + kAhead, n_chunks - 1), before);
+        step(cur, next_buf, kParity, 0, (kParity * CHUNK) % kStreamDepth, c * CHUNK + kStreamDepth, Sums{});      // (past the last chunk sums nobody uses)
+        if (decltype(whole)::value || c * CHUNK + 1 < n_groups)
+            step(cur, next_buf, kParity, 1, (kParity * CHUNK + 1) % kStreamDepth, c * CHUNK + 1 + kStreamDepth, None{});
+        ring_barrier<kInFlight>();
+        cur = next_buf;
+        next_buf = next_buf == kAhead * L::kBufBytes ? 0 : next_buf + L::kBufBytes;
     };
     using Even = std::integral_constant<int, 0>;
     using Odd = std::integral_constant<int, 1>;
     using Whole = std::integral_constant<bool, true>;
     using Part = std::integral_constant<bool, false>;
     uint32_t c = 0;
+#pragma nounroll
     for (; (c + 2) * CHUNK <= n_groups; c += 2) {
         chunk(c, Even{}, Whole{});
         chunk(c + 1, Odd{}, Whole{});
     }
     if (c < n_chunks) chunk(c, Even{}, Part{});
     if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
+    ring_barrier<0>();                  // no load is on its way into what follows, and nobody reads the last chunk any more
 
-    // lane (j, jq) holds, per stream, weight row j of the tile row for pairs 4 jq .. 4 jq + 3 of every 16-pair block. The
-    // last chunk ended with a barrier: the LDS is free.
+    // lane (j, jq) holds, per stream, weight row j of the tile row for pairs 4 jq .. 4 jq + 3 of every 16-pair block
     uint16_t *half = reinterpret_cast<uint16_t *>(lds);
     if constexpr (GATE_UP) {
         float h[NM][4];
@@ -1222,7 +1249,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
             for (int r = 0; r < 4; ++r) h[m][r] = gelu_tanh_fast(tot[m / 2][8 * (m & 1) + r]) * tot[m / 2][8 * (m & 1) + 4 + r];
         if constexpr (F16) {
             // the block scale of a pair's 64 activations, as in gemm_wave's epilogue: sixteen lanes hold a quarter of them
-            float *peaks = reinterpret_cast<float *>(lds + NM * 2 * kWave);             // [wave][pair]
+            float *peaks = reinterpret_cast<float *>(lds + NM * 2 * kFragBytes);        // [wave][pair]
 #pragma unroll
             for (int m = 0; m < NM; ++m)
 #pragma unroll
@@ -1258,11 +1285,11 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         lds_barrier();
         for (uint32_t i = tid; i < (uint32_t)NM * 2 * kWave; i += 256) {
             const uint32_t m = i / (2 * kWave), at = i % (2 * kWave);
-            *reinterpret_cast<uint4 *>(out + (((size_t)(gw.act_block0 + m) * g.gf + gw.nb) * 2 * kWave + at) * 8) = lds[i];
+            *reinterpret_cast<uint4 *>(out + (((size_t)(gw.act_block0 + m) * g.gf + gw.nb) * 2 * kWave + at) * 8) = reinterpret_cast<const uint4 *>(lds)[i];
         }
         return;
     }
-    uint8_t *rows = reinterpret_cast<uint8_t *>(lds);
+    uint8_t *rows = lds;
 #pragma unroll
     for (int m = 0; m < NM; ++m)
 #pragma unroll
@@ -1303,7 +1330,8 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const Prefil
                                                                     const uint16_t *__restrict__ a, uint32_t a_stride, uint32_t act_blocks,
                                                                     ArenaGeom g, const uint32_t *__restrict__ sorted_out_row,
                                                                     uint16_t *__restrict__ out, float *__restrict__ act_scale) {
-    __shared__ __align__(16) uint4 lds[2 * MAX_NM * 2 * kStreamChunk * kWave + 2 * MAX_NM * kStreamChunk * 16 / 4];
+    __shared__ __align__(16) uint8_t lds[StreamLds<MAX_NM>::kBytes];
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     uint32_t ti, nb;
     if (!prefill_block(n_nblocks, nb_major, ti, nb) || ti >= plan->n_tiles) return;
     GemmWave gw;
@@ -1327,8 +1355,8 @@ __global__ __launch_bounds__(256, WAVES) void prefill_stream_kernel(const Prefil
     const bool once = __builtin_amdgcn_readfirstlane(gw.tile.rows) < 16 * MAX_NM && plan->live_experts >= once_from;
 #define FFMOE_STREAM(N)                                                                                                      \
     if constexpr (N <= MAX_NM) {                                                                                             \
-        if (once) stream_tile<GATE_UP, N, F16, true>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale);  \
-        else stream_tile<GATE_UP, N, F16, false>(gw, g, src, tile0, lds, sorted_token, sorted_out_row, out, act_scale);      \
+        if (once) stream_tile<GATE_UP, N, F16, true, MAX_NM>(gw, g, src, tile0, lds, lds_base, sorted_token, sorted_out_row, out, act_scale);  \
+        else stream_tile<GATE_UP, N, F16, false, MAX_NM>(gw, g, src, tile0, lds, lds_base, sorted_token, sorted_out_row, out, act_scale);      \
     }
     switch (__builtin_amdgcn_readfirstlane((gw.tile.rows + 15) / 16)) {
         case 1: FFMOE_STREAM(1); break;

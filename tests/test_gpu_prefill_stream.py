@@ -66,6 +66,14 @@ def test_tile_edges_against_the_oracle(oracle, act, d, f, scale):
         ctx.close()
 
 
+# K of one to five chunks of two groups, the last one whole or ragged: every place at which the ring of row buffers can end, with four buffers
+# (tiles of up to 32 pairs) and with three (tiles of 64)
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("groups,f,scale", [(g, 128, 1) for g in (2, 6, 8, 9, 10)] + [(g, 704, 1.5) for g in (1, 2, 3, 4, 6, 7, 8)])
+def test_the_ring_of_row_buffers_ends_anywhere(oracle, act, groups, f, scale):
+    test_tile_edges_against_the_oracle(oracle, act, 64 * groups, f, scale)
+
+
 def _exact_part(oracle, rows, cols, one_hot):
     """4-bit weights, scale 1 and bias 0, with q = 1 at column one_hot[row] and 0 elsewhere."""
     q = np.zeros((rows, cols), np.uint8)
