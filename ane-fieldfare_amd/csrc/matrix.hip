@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     }
     WeightRing ring;
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) ring_fill<ONCE>(ring, u, src, rb0 * n_groups + min(g0 + u, g_last), lane);
+    for (int u = 0; u < kRing; ++u) ring_fill_here<ONCE>(ring, u, src, rb0 * n_groups + min(g0 + u, g_last), lane);
     // the input rows of this wave's K-slice: requested as 64-byte pieces (four lanes per row), then turned into the
     // operand layout - with 16 rows the operand layout itself would make every lane of every load a request of its own
     uint4 x0[kRing], x1[kRing];
@@ -251,13 +251,13 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     float gate_kept = 0.0f;
 
     for (uint32_t rb = rb0; rb < rb1; ++rb) {
-        const uint32_t next_row = min(rb + 1, rb1 - 1) * n_groups;
+        const uint32_t next_row = min(rb + 1, rb1 - 1) * n_groups, fill_lane = rb + 1 < rb1 || (size_t)n_tiles * n_groups >= kNoLaneTiles ? lane : no_lane(lane);
         TwoStreamAcc tot;
         tot.a = f32x4{0.f, 0.f, 0.f, 0.f};
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16, true, kSums, ONCE>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), lane);
+            ring_step<F16, true, kSums, ONCE>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), fill_lane);
         const int buf = (rb - rb0) & 1;
 #pragma unroll
         for (int r = 0; r < kSums; ++r) {

@@ -358,7 +358,7 @@ __device__ __forceinline__ void gate_up_rows(GateUpMerge &s_red, PlanScratch &ps
     WeightRing ring;
     if (has_rows) {
 #pragma unroll
-        for (int u = 0; u < kRing; ++u) ring_fill(ring, u, gu_src, rb0 * g.gd + min(g0 + u, g_last), lane);
+        for (int u = 0; u < kRing; ++u) ring_fill_here(ring, u, gu_src, rb0 * g.gd + min(g0 + u, g_last), lane);
     }
     if (!DENSE && plan_out) build_plan_routes(ps, n_routes, plan_out, route_expert);
     if (!has_rows) return;
@@ -378,14 +378,14 @@ __device__ __forceinline__ void gate_up_rows(GateUpMerge &s_red, PlanScratch &ps
     uint16_t *out_col = acts + (size_t)col * top_k * g.f + j;
 
     for (uint32_t rb = rb0; rb < rb1; ++rb) {
-        // the refill targets the next row block; past the last one it re-reads the current tiles (cache hits)
-        const uint32_t next_row = min(rb + 1, rb1 - 1) * g.gd;
+        // the refill targets the next row block
+        const uint32_t next_row = min(rb + 1, rb1 - 1) * g.gd, fill_lane = rb + 1 < rb1 ? lane : no_lane(lane);
         TwoStreamAcc tot;
         tot.a = f32x4{0.f, 0.f, 0.f, 0.f};
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, gu_src, next_row + min(g0 + u, g_last), lane);
+            ring_step<F16>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, gu_src, next_row + min(g0 + u, g_last), fill_lane);
         const int buf = (rb - rb0) & 1;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -450,19 +450,19 @@ __device__ __forceinline__ void shared_gate_up8_rows(GateUpMerge &s_red, const S
                                             (size_t)2 * pairs * gd * kTileScaleBytes);
     WeightRing ring;
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) ring_fill(ring, u, src, rb0 * gd + min(k.g0 + u, k.g_last), lane);
+    for (int u = 0; u < kRing; ++u) ring_fill_here(ring, u, src, rb0 * gd + min(k.g0 + u, k.g_last), lane);
     prepare_token_rows<F16>(lane, x0, x1, sx);
     const uint32_t col = 4 * jq + ks;       // the input row this lane finishes
     uint16_t *out_col = sh.acts + (size_t)col * sh.g.f + j;
     float gate_kept = 0.0f;
     for (uint32_t rb = rb0; rb < rb1; ++rb) {
-        const uint32_t next_row = min(rb + 1, rb1 - 1) * gd;
+        const uint32_t next_row = min(rb + 1, rb1 - 1) * gd, fill_lane = rb + 1 < rb1 ? lane : no_lane(lane);
         TwoStreamAcc tot;
         tot.a = f32x4{0.f, 0.f, 0.f, 0.f};
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16>(ring, u, (uint32_t)u < k.ng, x0[u], x1[u], sx[u], tot, src, next_row + min(k.g0 + u, k.g_last), lane);
+            ring_step<F16>(ring, u, (uint32_t)u < k.ng, x0[u], x1[u], sx[u], tot, src, next_row + min(k.g0 + u, k.g_last), fill_lane);
         const int buf = (rb - rb0) & 1;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -914,7 +914,7 @@ __global__ __launch_bounds__(256, 5) void skinny_down_lds(const VerifyPlan *__re
         const f32x4 sx = group_input_sum<F16>(x0, x1);
         // consume slot u % kDownDepth; the load that refills it (group u + kDownDepth) starts inside the step
         if (u + kDownDepth < kRing)
-            ring_step<F16, true>(ring, u % kDownDepth, live, x0, x1, sx, tot, src, tile0 + min((uint32_t)(u + kDownDepth), g_last), lane);
+            ring_step<F16, true, 4, false, false>(ring, u % kDownDepth, live, x0, x1, sx, tot, src, tile0 + min((uint32_t)(u + kDownDepth), g_last), lane);
         else
             ring_step<F16, false>(ring, u % kDownDepth, live, x0, x1, sx, tot, src, 0u, lane);
         // The running sums are pinned here: left alone, the compiler sinks the scale-and-bias arithmetic of every
@@ -980,7 +980,7 @@ __global__ __launch_bounds__(256, 2) void skinny_down_ksplit_persistent(const ui
                                             expert_base + g.dn_scales_off, (size_t)g.dn_rbp * g.gf * kTileScaleBytes);
     WeightRing ring;
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) ring_fill(ring, u, src, rb0 * g.gf + min(g0 + u, g_last), lane);
+    for (int u = 0; u < kRing; ++u) ring_fill_here(ring, u, src, rb0 * g.gf + min(g0 + u, g_last), lane);
     // a wide expert is a dense one: up to 16 distinct activation rows, fetched four lanes per 64 contiguous
     // bytes (slot lane / 4, chunk lane % 4) and turned into the operand layout by cross-lane moves
     // (with one or two rows the operand layout itself is as cheap to load, and needs no moves)
@@ -1017,13 +1017,13 @@ __global__ __launch_bounds__(256, 2) void skinny_down_ksplit_persistent(const ui
     const size_t out_base = (size_t)route_of(min(my_ts, n - 1)) * g.d;
 
     for (uint32_t rb = rb0; rb < rb1; ++rb) {
-        const uint32_t next_row = min(rb + 1, rb1 - 1) * g.gf;
+        const uint32_t next_row = min(rb + 1, rb1 - 1) * g.gf, fill_lane = rb + 1 < rb1 ? lane : no_lane(lane);
         TwoStreamAcc tot;
         tot.a = f32x4{0.f, 0.f, 0.f, 0.f};
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), lane);
+            ring_step<F16>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), fill_lane);
         const int buf = (rb - rb0) & 1;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {

@@ -60,6 +60,19 @@ __device__ __forceinline__ void ring_fill(WeightRing &ring, int u, const TileSou
     ring.s[u] = make_uint2(s.x, s.y);
 }
 
+// The same where it stands, before what follows: for the fills in front of a loop of ring_steps, whose waits count on the loads' order.
+template <bool ONCE = false>
+__device__ __forceinline__ void ring_fill_here(WeightRing &ring, int u, const TileSource &src, uint32_t tile_index, uint32_t lane) {
+    ring_fill<ONCE>(ring, u, src, tile_index, lane);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The lane of a refill that is not wanted: its tile's bytes lie 2 GiB further on, past the end of a region of less (kNoLaneTiles), and memory is
+// not asked for them. (Its scales, 128 bytes, are read and left.) The offset is the lane's own, which is held against what the descriptor has
+// left behind the tile's; with the tile's it stays below 4 GiB.
+constexpr uint32_t kNoLaneTiles = (1u << 31) / kTileBytes;
+__device__ __forceinline__ uint32_t no_lane(uint32_t lane) { return lane | 0x08000000u; }
+
 // Sum of a group's 64 inputs per token column, in the register layout of the matrix results: the product
 // with an all-ones operand. It depends on the token operand only, so a wave that walks several tile rows
 // with the same operand computes it once per group, not once per tile.
@@ -73,7 +86,14 @@ __device__ __forceinline__ f32x4 group_input_sum(const uint4 &x0, const uint4 &x
 // Consume ring slot u against the resident token operand (`sx` = its group_input_sum), then start the load
 // that refills the slot (REFILL = false: a wave that walks one tile row only has nothing to refill).
 // SUMS: of the lane's four results, how many are kept up.
-template <bool F16 = false, bool REFILL = true, int SUMS = 4, bool ONCE = false>
+// PIN: the refill stands behind the unpacking of its slot, and nowhere else. Left alone the compiler collects the refills of a whole tile row at its
+// end and waits for nearly all of them at the next one's start, so that a wave has its twelve KiB in flight a part of the time only: 262,144 x
+// 2,816, greedy with confidence, 16 rows 76.6 us, now 73.0; fp32 logits of 1 row 67.1 | 62.6, of 16 rows 82.5 | 76.2; verify block of 16 rows 48.6 | 47.9,
+// layer block of 1 row 28.4 | 28.1, of 5 FP16 rows 42.8 | 42.2. Not for a wave of one tile row, whose rows and weights
+// are better asked for as the compiler has it (skinny_down_lds: 5.9 us at 1 row, pinned 6.2 to 6.5). The last tile row's refills come with
+// no_lane (asked for once more, its tiles are the launch's last requests: layer block of 1 row 28.65); written as steps without a refill, behind a
+// branch, the compiler keeps both rows' operands and spills.
+template <bool F16 = false, bool REFILL = true, int SUMS = 4, bool ONCE = false, bool PIN = REFILL>
 __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, const uint4 &x0, const uint4 &x1,
                                           const f32x4 &sx, TwoStreamAcc &tot, const TileSource &src,
                                           uint32_t next_tile_index, uint32_t lane) {
@@ -81,11 +101,16 @@ __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, co
     const uint4 tile = ring.t[u];
     uint2 sc = ring.s[u];
     if (!live) sc = make_uint2(0u, 0u);
-    if (REFILL) ring_fill<ONCE>(ring, u, src, next_tile_index, lane);
-    f32x4 acc_a = Act<F16>::mfma(x0, unpack8_offset<F16>(tile.x), zero);
-    acc_a = Act<F16>::mfma(x1, unpack8_offset<F16>(tile.y), acc_a);
-    f32x4 acc_b = Act<F16>::mfma(x0, unpack8_offset<F16>(tile.z), zero);
-    acc_b = Act<F16>::mfma(x1, unpack8_offset<F16>(tile.w), acc_b);
+    if (REFILL && !PIN) ring_fill<ONCE>(ring, u, src, next_tile_index, lane);
+    const uint4 wa0 = unpack8_offset<F16>(tile.x), wa1 = unpack8_offset<F16>(tile.y), wb0 = unpack8_offset<F16>(tile.z), wb1 = unpack8_offset<F16>(tile.w);
+    if (PIN) {
+        __builtin_amdgcn_sched_barrier(0);
+        ring_fill_here<ONCE>(ring, u, src, next_tile_index, lane);
+    }
+    f32x4 acc_a = Act<F16>::mfma(x0, wa0, zero);
+    acc_a = Act<F16>::mfma(x1, wa1, acc_a);
+    f32x4 acc_b = Act<F16>::mfma(x0, wb0, zero);
+    acc_b = Act<F16>::mfma(x1, wb1, acc_b);
     const float sa = bf16lo_to_f32(sc.x), ba = bf16hi_to_f32(sc.x);
     const float sb = bf16lo_to_f32(sc.y), bb = bf16hi_to_f32(sc.y);
     const float ta = __builtin_fmaf(-Act<F16>::kOffset, sa, ba), tb = __builtin_fmaf(-Act<F16>::kOffset, sb, bb);
