@@ -187,7 +187,12 @@ __device__ __forceinline__ SoftmaxAcc softmax_shuffle(const SoftmaxAcc &a, int m
 // FEW (up to four input rows of the plain form): input row t is operand row 4 t, so that one of a lane's four sums is all there is to
 // keep up, and each operand lane loads its own bytes: the lanes of a row ask for the same ones, there is nothing to turn through LDS.
 // 1 row, us without | so: 16,384 x 1,408 6.7 | 5.9, 16,384 x 2,816 7.2 | 6.8, 262,144 x 2,816 76.5 | 74.9.
-// ONCE: the matrix is more than the memory side's cache holds (kReadOnce); with it the last of those takes 66.6 (6.2 TB/s).
+// ONCE: the matrix is more than the memory side's cache holds (kReadOnce); with it the last of those takes 66.6 (with the refills pinned and every
+// gridDim.x-th tile 60.7, 6.8 TB/s).
+// A block takes every gridDim.x-th tile (the gated form a range of pairs): what the chip reads and, above all, writes at a time lies together then. With
+// a range each, 512 blocks write 128-byte pieces of 16 rows 2 KiB apart, which are few of the caches' channels: 262,144 x 2,816, fp32 logits, us with
+// ranges | so: 1 row 62.9 | 60.7, 4 66.2 | 63.5, 8 70.9 | 67.2, 16 76.1 | 72.1, greedy with confidence, 1 row, 68.4 | 66.9 (stores to one small region 67; non-temporal or write-through ones, four tiles' at a time, or whole lines by half a wave
+// per row change nothing).
 template <bool Y_F32, bool F16, bool GREEDY = false, bool CONF = false, bool PLANES8 = false, int GLU = 0, bool FEW = false, bool ONCE = false>
 __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__restrict__ tiles,
                                                              const uint8_t *__restrict__ scales, uint32_t m,
@@ -203,11 +208,10 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     // GLU == 1: tiles 2 p and 2 p + 1 hold rows 16 p ... 16 p + 15 of a gate and of an up projection; a block takes whole
     // pairs, and `m` counts the outputs gelu_tanh(gate . x) * (up . x)
     const uint32_t n_tiles = GLU == 1 ? 2 * ((m + 15) / 16) : PLANES8 ? (m + 15) / 16 : (m + 31) / 32;
-    uint32_t rb0, rb1;
-    split_range(GLU == 1 ? n_tiles / 2 : n_tiles, gridDim.x, blockIdx.x, rb0, rb1);
+    uint32_t rb0 = blockIdx.x, rb1 = n_tiles, every = gridDim.x;
     if (GLU == 1) {
-        rb0 *= 2;
-        rb1 *= 2;
+        split_range(n_tiles / 2, gridDim.x, blockIdx.x, rb0, rb1);
+        rb0 *= 2, rb1 *= 2, every = 1;
     }
     if (rb0 >= rb1) {
         if (GREEDY && threadIdx.x < rows) reinterpret_cast<unsigned long long *>(y_)[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = 0ull;
@@ -250,15 +254,18 @@ __global__ __launch_bounds__(256, 2) void matrix_gemv_kernel(const uint8_t *__re
     SoftmaxAcc soft{-INFINITY, 0.0f};
     float gate_kept = 0.0f;
 
-    for (uint32_t rb = rb0; rb < rb1; ++rb) {
-        const uint32_t next_row = min(rb + 1, rb1 - 1) * n_groups, fill_lane = rb + 1 < rb1 || (size_t)n_tiles * n_groups >= kNoLaneTiles ? lane : no_lane(lane);
+    uint32_t buf = 1;
+    for (uint32_t rb = rb0; rb < rb1; rb += every) {
+        const bool more = rb + every < rb1;
+        const uint32_t next_row = (more ? rb + every : rb) * n_groups;
+        const uint32_t fill_lane = more || (size_t)n_tiles * n_groups >= kNoLaneTiles ? lane : no_lane(lane);
         TwoStreamAcc tot;
         tot.a = f32x4{0.f, 0.f, 0.f, 0.f};
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
             ring_step<F16, true, kSums, ONCE>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, next_row + min(g0 + u, g_last), fill_lane);
-        const int buf = (rb - rb0) & 1;
+        buf ^= 1u;
 #pragma unroll
         for (int r = 0; r < kSums; ++r) {
             s_red[buf][ks][r][lane] = tot.a[r];

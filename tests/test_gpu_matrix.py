@@ -65,6 +65,32 @@ def test_matrix_gemv_reference_shapes(ctx, oracle, torch, m, n, rows, off, src):
     mx.close()
 
 
+# 512 blocks (two per compute unit) with no, one, two or three tiles each: one short of a round, a round, one past it, and an odd end; 63 and 64 rows leave a
+# last tile short. n: one group (a block's three other waves have none), and eleven per wave
+@pytest.mark.parametrize("m,n", [(511 * 32, 64), (512 * 32, 128), (512 * 32 + 1, 64), (1031 * 32 + 5, 192), (1024 * 32 + 40, 2816)])
+@pytest.mark.parametrize("rows", [1, 4, 5, 16])
+def test_every_tile_once_whichever_block_takes_it(ctx, torch, m, n, rows):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + rows)
+    W = torch.randint(0, 256, (m, n // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    S, B = ((torch.randn((m, n // 64), device="cuda", generator=gen) * 0.02).to(torch.bfloat16) for _ in range(2))
+    x = torch.randn((rows, n), device="cuda", generator=gen).to(torch.bfloat16)
+    mx = ctx.matrix(W, S, B, greedy=True)
+    y = mx.gemv(x, f32_out=True)
+    q = torch.stack((W & 15, W >> 4), 2).reshape(m, n).double()
+    w = q * S.double().repeat_interleave(64, 1) + B.double().repeat_interleave(64, 1)
+    ref, spread = x.double() @ w.T, x.double().abs() @ (q * S.double().abs().repeat_interleave(64, 1) + B.double().abs().repeat_interleave(64, 1)).T
+    # fp32 sums of up to 2,816 products in the offset form (128 + q, so some 17 times the products' own magnitude), 2^-24 each
+    assert torch.all((y.double() - ref).abs() <= 17 * 2.0 ** -24 * 64 * spread + 1e-9)
+    assert torch.equal(mx.gemv(x), y.to(torch.bfloat16))
+    assert torch.equal(mx.greedy(x).long(), y.argmax(1))
+    # and the same bits as where its tiles lie in a matrix of their own
+    for lo, hi in ((0, 300), ((m - 300) // 32 * 32, m)):
+        part = ctx.matrix(W[lo:hi].contiguous(), S[lo:hi].contiguous(), B[lo:hi].contiguous())
+        assert torch.equal(part.gemv(x, f32_out=True), y[:, lo:hi])
+        part.close()
+    mx.close()
+
+
 def test_matrix_equals_raw_layout_gemv(ctx, oracle, torch):
     # the same weight through the reference-layout GEMV and through the resident tiles
     m, n, rows = 512, 1408, 5
