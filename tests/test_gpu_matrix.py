@@ -536,6 +536,24 @@ def test_final_row_head_matches_scalar_offset_path(ctx, oracle, torch):
 
 
 @pytest.mark.parametrize("act", ["fp16", "bf16"])
+@pytest.mark.parametrize("n", [64, 192, 1088, 2816])
+@pytest.mark.parametrize("m", [1, 17, 65])
+def test_table_rows_of_any_shape_and_place(ff, oracle, torch, act, n, m):
+    # every row of tables that end inside a tile of rows, from one group of columns to the widest, and rows past the end; the
+    # expression is exact in fp32 up to its last rounding, so the bits are the oracle's
+    g = np.random.default_rng(m * 4096 + n)
+    W, S, B = oracle.quantize_int4(g.uniform(-1.0, 1.0, (m, n)).astype(np.float32))
+    c = ff.Context(128, 64, 16, 8, n_layers=1, max_tokens=16, act_dtype=act)
+    table = c.matrix(W, S, B)
+    ids = np.concatenate([g.permutation(m), [m, (m + 31) // 32 * 32, 2**31 - 1]]).astype(np.int32)
+    got = bits_of(table.rows(torch.from_numpy(ids).cuda(), 7.5))
+    want = oracle.bits16(oracle.dequantize_int4(W, S, B) * np.float32(7.5), oracle.FP16 if act == "fp16" else oracle.BF16)
+    assert np.array_equal(got[:m], want[ids[:m]]) and not got[m:].any()
+    table.close()
+    c.close()
+
+
+@pytest.mark.parametrize("act", ["fp16", "bf16"])
 def test_embedding_rows_from_the_resident_table(ff, oracle, torch, act):
     # embedLookupInt4_withSqrtDScale_matchesReference (EmbedLookupTests.swift:24-62): same seed, label, table (16 x 128),
     # token 9 and scale sqrt(128); FP16 out as there (and bf16). The reference allows Tolerance.quantInt4; the kernel's
