@@ -253,9 +253,10 @@ __global__ __launch_bounds__(256) void router_frag_kernel(const uint16_t *__rest
 // per wave and eight waves, 16 rows: 13.9, 19.6, 31.0, 43.8). 3,072 rows, bf16, of 4,096 x 128 38 | 40. Up to 1,024 columns a quarter of K
 // is at most eight steps, and the traffic decides earlier: 512 x 32, 900 rows 8.6 | 8.2, 1,400 rows 8.7 | 8.9, FP16 2,000 rows 10.0 | 10.7.
 // Block 4 b + q leaves the sums of K quarter q for its rows in approx[q] and the rows' squares in
-// xnorm2[q]; the reader adds them as (q0 + q1) + (q2 + q3). The loop body has no branch: the compiler then counts the
-// loads in flight exactly and waits for the oldest step only (behind a branch it waits for all of them, and the pass is
-// one round trip per step).
+// xnorm2[q]; the reader adds them as (q0 + q1) + (q2 + q3). The loop body has no branch: the compiler then
+// collects a turn's DEPTH steps of requests and waits for them once per turn (behind a branch for each step's, and the pass is one round
+// trip per step). With the requests pinned step by step, which leaves DEPTH steps in flight throughout, the pass takes as long: 3,072
+// rows 14.0 us either way, 301 rows 6.7.
 static bool approx_few_rows(uint32_t t, uint32_t d, bool f16) { return t <= (d <= 1024 ? 1024u : f16 ? 3072u : 2048u); }
 
 // Eight FP16 values as two sets of eight bf16 values whose sums are the FP16 values exactly (eleven significant bits =
