@@ -162,18 +162,22 @@ __global__ __launch_bounds__(256) void gemv_int4_kernel(const uint8_t *__restric
 // rows is one such chain per compute unit. So the input rows are asked for between the ids and the weights, which wait for
 // the ids, and eight waves take six groups each: with four, eleven each, a chain was twice as long and a block's registers left
 // two waves per SIMD. Listed rows x 2,816, us with four waves and the input rows behind the weights | so: 512 rows, 1 input row 6.4 | 4.8;
-// 4,099 rows, 1 input row 7.1 | 5.7, 16 input rows 7.4 | 6.2 (the vector unit's dot products: 50.8); 32,768 rows 17.7 | 16.8, 19.0 | 17.5.
+// 4,099 rows, 1 input row 7.1 | 5.7, 16 input rows 7.4 | 6.2 (both shorter still, below; the vector unit's dot products: 50.8); 32,768 rows 17.7 | 16.8, 19.0 | 17.5.
 // Error of a logit against 64 bits (2-norm): 1.7e-7 in bf16 and 4.9e-6 in FP16, where the dot products have
 // 8.6e-7 and 1.6e-5, and 128 + q / 1024 + q on the matrix unit 1.0e-6 and 1.4e-5.
 constexpr int kListedParts = 8, kListedRing = 6;
 static_assert(kListedParts * kListedRing >= kKSplit * kRing, "every width up to FFMOE_MATRIX_MAX_N");
-template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16, bool FEW>
+// ONE: the launch has a block for every 16 rows, none of which takes others: it asks for no further weights, whose requests (the same rows
+// again) a block would have to wait for before it can end. Listed rows x 2,816, us with the
+// requests | so: 16 rows, 1 input row 4.06 | 3.77, 16 input rows 4.54 | 4.28; 1,408 rows 4.47 | 4.10, 5.03 | 4.71; 4,099 rows 6.0 | 5.24, 6.3 | 6.08; 8,192
+// rows 7.5 | 5.9, 7.4 | 6.75. Beyond, two blocks per compute unit go on to others (8,193 rows 6.75, 7.2: a block in 500 takes a second sixteen).
+template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16, bool FEW, bool ONE>
 __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
                                                                               const uint16_t *__restrict__ biases, const uint16_t *__restrict__ x,
                                                                               void *__restrict__ y_, uint32_t m, uint32_t n_groups, uint32_t rows,
                                                                               uint32_t x_stride, uint32_t y_stride, const uint32_t *__restrict__ ids) {
     constexpr int kSums = FEW ? 1 : 4;
-    __shared__ float s_red[2][kListedParts][kSums][64];
+    __shared__ float s_red[ONE ? 1 : 2][kListedParts][kSums][64];
     const uint32_t lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, jq = lane >> 4;                  // operand layout: row j, quarter jq
     const uint32_t lrow = lane >> 2, lq = lane & 3;                // load layout: row lrow, quarter lq
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
         return (uint32_t)scales[at] | ((uint32_t)biases[at] << 16);
     };
     uint32_t rb = blockIdx.x;                                       // the grid has at most n_blocks blocks
-    uint32_t row = id_of(rb), next_id = id_of(min(rb + gridDim.x, n_blocks - 1));
+    uint32_t row = id_of(rb), next_id = ONE ? 0u : id_of(min(rb + gridDim.x, n_blocks - 1));
     // the input rows of this wave's K-slice
     uint4 x0[kListedRing], x1[kListedRing];
     {
@@ -235,8 +239,10 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
     const uint32_t my_row = FEW ? jq : 4 * jq + ks;                 // the input row this lane finishes (waves kSums and up: none)
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     for (int buf = 0; rb < n_blocks; rb += gridDim.x, buf ^= 1) {
-        row = next_id;
-        next_id = id_of(min(rb + 2 * gridDim.x, n_blocks - 1));
+        if constexpr (!ONE) {
+            row = next_id;
+            next_id = id_of(min(rb + 2 * gridDim.x, n_blocks - 1));
+        }
         float tot[kSums];
 #pragma unroll
         for (int r = 0; r < kSums; ++r) tot[r] = 0.0f;
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
             t.y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].y);
             uint32_t sc = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((4 * j + u / 2) * 4), (int)sb[u % 2]);
             if ((uint32_t)u >= ng) sc = 0;
-            wt[u] = load_w(row, u);                                 // the next 16 rows (past the last: these again)
+            if constexpr (!ONE) wt[u] = load_w(row, u);             // the next 16 rows (past the last: these again)
             f32x4 acc = Act<F16>::mfma(x0[u], unpack8_fine<F16>(t.x), zero);
             acc = Act<F16>::mfma(x1[u], unpack8_fine<F16>(t.y), acc);
             const float s = bf16lo_to_f32(sc), b = bf16hi_to_f32(sc), su = s * FineNibble<F16>::kUnit;
@@ -258,12 +264,17 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
                 tot[r] = __builtin_fmaf(tb, sx[u][r], tot[r]);
             }
         }
+        if constexpr (!ONE) {
 #pragma unroll
-        for (int v = 0; v < 2; ++v) sb[v] = load_s(row, v);
+            for (int v = 0; v < 2; ++v) sb[v] = load_s(row, v);
+        }
 #pragma unroll
         for (int r = 0; r < kSums; ++r) s_red[buf][ks][r][lane] = tot[r];
         lds_barrier();
-        if (ks >= (uint32_t)kSums) continue;
+        if (ks >= (uint32_t)kSums) {
+            if constexpr (ONE) return;
+            continue;
+        }
         float v = s_red[buf][0][ks][lane];
 #pragma unroll
         for (int o = 1; o < kListedParts; ++o) v += s_red[buf][o][ks][lane];
@@ -273,6 +284,7 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
             if (Y_F32) reinterpret_cast<float *>(y_)[at] = v;
             else reinterpret_cast<uint16_t *>(y_)[at] = Act<F16>::round(v);
         }
+        if constexpr (ONE) return;
     }
 }
 
@@ -283,11 +295,14 @@ hipError_t launch_gemv_int4(hipStream_t s, const uint8_t *w, const uint16_t *sca
                             uint32_t x_stride, uint32_t y_stride, int y_f32, const uint32_t *ids, bool f16, uint32_t n_cus) {
     if (n <= FFMOE_MATRIX_MAX_N) {
         // every row count of such a width takes this form (the rows of a call equal single-row calls bit for bit)
-        const dim3 blocks(min((m + kTileRows - 1) / kTileRows, 2 * n_cus));
+        const uint32_t tiles = (m + kTileRows - 1) / kTileRows;
+        const dim3 blocks(min(tiles, 2 * n_cus));
+        const bool one = tiles <= 2 * n_cus;                 // a block for every 16 rows
         const bool wide_w = reinterpret_cast<uintptr_t>(w) % 8 == 0, wide_x = reinterpret_cast<uintptr_t>(x) % 16 == 0 && x_stride % 8 == 0;
         if (f16 && !wide_x) return hipErrorInvalidValue;     // FP16 rows come 16-byte aligned (checked at the boundary)
 #define FFMOE_GEMVM(A, X, Y, H)                                                                                                     \
-    hipLaunchKernelGGL((rows <= 4 ? gemv_int4_mfma_kernel<A, X, Y, H, true> : gemv_int4_mfma_kernel<A, X, Y, H, false>), blocks,               \
+    hipLaunchKernelGGL((rows <= 4 ? (one ? gemv_int4_mfma_kernel<A, X, Y, H, true, true> : gemv_int4_mfma_kernel<A, X, Y, H, true, false>)     \
+                                  : (one ? gemv_int4_mfma_kernel<A, X, Y, H, false, true> : gemv_int4_mfma_kernel<A, X, Y, H, false, false>)), blocks, \
                        dim3(64 * kListedParts), 0, s, w, scales, biases, x, y, m, n / kGroup, rows, x_stride, y_stride, ids)
 #define FFMOE_GEMVM_X(A, Y)                                                                             \
     do {                                                                                                \

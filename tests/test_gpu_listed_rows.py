@@ -39,3 +39,23 @@ def test_listed_forms_agree(m, n, shift, act):
         of[r] = y
         assert torch.equal(y, of[16][:r]), r       # whatever the form, a row's bits are the same
     ctx.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "fp16"])
+@pytest.mark.parametrize("rows", [1, 4, 5, 16])
+def test_a_block_for_every_sixteen_rows_or_not(act, rows):
+    # up to 32 weight rows per compute unit a block takes sixteen and ends, beyond it goes on to others: the same bits
+    import torch
+    import fieldfare_moe as ff
+    from fieldfare_moe import synthetic as syn
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows)
+    most = 32 * torch.cuda.get_device_properties(0).multi_processor_count
+    ctx = ff.Context(128, 64, 16, 8, n_layers=1, max_tokens=16, act_dtype=act)
+    W, S, B = syn.synth_matrix_gpu(torch, gen, most, 704)
+    ids = torch.randint(0, most, (most + 17,), device="cuda", generator=gen, dtype=torch.int32)
+    x = torch.randn((rows, 704), device="cuda", generator=gen).to(ctx.act)
+    whole = ctx.gemv_int4_listed(W, S, B, ids, x)
+    for m in (1, 16, 31, most - 15, most):
+        assert torch.equal(ctx.gemv_int4_listed(W, S, B, ids[:m].contiguous(), x), whole[:, :m]), m
+    ctx.close()
