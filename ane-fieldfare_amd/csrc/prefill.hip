@@ -1081,7 +1081,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
             global_to_lds_16(from[k] + (size_t)grp * (GATE_UP ? kGroup : 2 * kWave * 8), lds_base + buf + gl * kGroupBytes + piece * 1024);
         }
     };
-    // fragment f of 16-pair block m, this lane's 16 bytes of it: k-half f % 2 of group f / 2 of the chunk whose buffer `at` and `at64` lie in
+    // fragment f of 16-pair block m, this lane's 16 bytes of it: k-half f % 2 (at0, at1) of group f / 2 of a chunk
     const uint32_t at0 = GATE_UP ? j * 128 + 16 * (jq ^ (j & 7)) : lane * 16, at1 = GATE_UP ? at0 ^ 64 : at0 + 1024;
     auto frag = [&](uint32_t at, int m, int gl) __attribute__((always_inline)) {
         return *reinterpret_cast<const uint4 *>(lds + at + gl * kGroupBytes + m * 2048);
@@ -1130,8 +1130,9 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
     };
 
     // One group. What it reads of LDS is asked for in front of the unpacking, which covers the way; the ring's slot is filled again behind it,
-    // when its registers are free. NEXT >= 0: on the way the wave's share of the next chunk's sums, from buffer `next`, for that slot.
-    auto step = [&](uint32_t cur, uint32_t next_buf, int slot, int gl, int u, uint32_t refill, auto next_sums) __attribute__((always_inline)) {
+    // when its registers are free (`refills`: where it is wanted again). next_sums >= 0: on the way the wave's share of the next chunk's sums,
+    // from buffer `next_buf`, for that slot.
+    auto step = [&](uint32_t cur, uint32_t next_buf, int slot, int gl, int u, uint32_t refill, auto next_sums, auto refills) __attribute__((always_inline)) {
         constexpr int kNext = decltype(next_sums)::value;
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         uint4 x[2][2][2];                                   // of a pair of 16-pair blocks, and of the next pair
@@ -1161,7 +1162,7 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         }
         const float bias = jq & 1 ? tb : ta;
         __builtin_amdgcn_sched_barrier(0);
-        fill(u, refill);
+        if constexpr (decltype(refills)::value) fill(u, refill);
 #pragma unroll
         for (int i = 0; i < kPairs; ++i) {
             auto &t = tot[i];
@@ -1192,8 +1193,10 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
 
     // Chunk c lies in buffer c % kBufs. While the block is at it the loads of chunk c + kAhead go into the buffer of the chunk before, and
     // (kShared) chunk c + 1 is there already, for its sums. One barrier per chunk, at its end: it waits for the loads of the chunk
-    // that is needed next, i.e. for all but those that every wave has asked for since, always the same number: chunk by chunk NM of rows, then
-    // one fill per group (the loads in front of the loop go out in that order too).
+    // that is needed next, i.e. for all but those that every wave has asked for since: in the loop, and in front of it, always the same
+    // number, chunk by chunk NM of rows, then one fill per group. The last one or two chunks, behind the loop, have nothing left to ask for (their rows
+    // and weights went out kAhead chunks and kStreamDepth groups before), and their barriers wait for everything: a count over
+    // refills that nobody reads would be wrong, since the compiler drops them.
     constexpr int kChunkFills = CHUNK * kFillLoads;
     constexpr int kInFlight = kShared ? kChunkFills * (kAhead - 1) + NM * (kAhead - 2) : kChunkFills * kAhead + NM * (kAhead - 1);
     static_assert(kStreamDepth == 2 * CHUNK, "two chunks' fills in front of the loop");
@@ -1212,31 +1215,30 @@ __device__ __forceinline__ void stream_tile(const GemmWave &gw, const ArenaGeom 
         sum_up(0);
         lds_barrier();
     }
-    auto chunk = [&](uint32_t c, auto parity, auto whole) __attribute__((always_inline)) {
+    using Even = std::integral_constant<int, 0>;
+    using Odd = std::integral_constant<int, 1>;
+    using None = std::integral_constant<int, -1>;
+    // a chunk; `asks`: of the loop. Behind it a chunk's second group may be missing.
+    auto chunk = [&](uint32_t c, auto parity, auto asks) __attribute__((always_inline)) {
         constexpr int kParity = decltype(parity)::value;
+        constexpr bool kAsks = decltype(asks)::value;
         using Sums = std::integral_constant<int, kShared ? kParity ^ 1 : -1>;
-        using None = std::integral_constant<int, -1>;
-        const uint32_t before = cur ? cur - L::kBufBytes : kAhead * L::kBufBytes;
-        load_a(min(c + kAhead, n_chunks - 1), before);
-        step(cur, next_buf, kParity, 0, (kParity * CHUNK) % kStreamDepth, c * CHUNK + kStreamDepth, Sums{});      // (past the last chunk sums nobody uses)
-        if (decltype(whole)::value || c * CHUNK + 1 < n_groups)
-            step(cur, next_buf, kParity, 1, (kParity * CHUNK + 1) % kStreamDepth, c * CHUNK + 1 + kStreamDepth, None{});
-        ring_barrier<kInFlight>();
+        if constexpr (kAsks) load_a(min(c + kAhead, n_chunks - 1), cur ? cur - L::kBufBytes : kAhead * L::kBufBytes);
+        step(cur, next_buf, kParity, 0, (kParity * CHUNK) % kStreamDepth, c * CHUNK + kStreamDepth, Sums{}, asks);      // (past the last chunk sums nobody uses)
+        if (kAsks || c * CHUNK + 1 < n_groups)
+            step(cur, next_buf, kParity, 1, (kParity * CHUNK + 1) % kStreamDepth, c * CHUNK + 1 + kStreamDepth, None{}, asks);
+        ring_barrier<kAsks ? kInFlight : 0>();
         cur = next_buf;
         next_buf = next_buf == kAhead * L::kBufBytes ? 0 : next_buf + L::kBufBytes;
     };
-    using Even = std::integral_constant<int, 0>;
-    using Odd = std::integral_constant<int, 1>;
-    using Whole = std::integral_constant<bool, true>;
-    using Part = std::integral_constant<bool, false>;
     uint32_t c = 0;
 #pragma nounroll
     for (; (c + 2) * CHUNK <= n_groups; c += 2) {
-        chunk(c, Even{}, Whole{});
-        chunk(c + 1, Odd{}, Whole{});
+        chunk(c, Even{}, std::true_type{});
+        chunk(c + 1, Odd{}, std::true_type{});
     }
-    if (c < n_chunks) chunk(c, Even{}, Part{});
-    if (c + 1 < n_chunks) chunk(c + 1, Odd{}, Part{});
+    if (c < n_chunks) chunk(c, Even{}, std::false_type{});
+    if (c + 1 < n_chunks) chunk(c + 1, Odd{}, std::false_type{});
     ring_barrier<0>();                  // no load is on its way into what follows, and nobody reads the last chunk any more
 
     // lane (j, jq) holds, per stream, weight row j of the tile row for pairs 4 jq .. 4 jq + 3 of every 16-pair block
