@@ -159,24 +159,33 @@ __global__ __launch_bounds__(256) void gemv_int4_kernel(const uint8_t *__restric
 // FEW (up to four input rows): input row t is operand row 4 t, so that one of a lane's four sums is all there is to keep up, and
 // each operand lane loads its own bytes - the lanes of a row ask for the same ones, nothing is turned through LDS.
 // Bound: latency - row id, weights, products and the merge are one chain per 16 rows, and a hot list of a few thousand
-// rows is one such chain per compute unit. So the input rows are asked for between the ids and the weights, which wait for
-// the ids, and eight waves take six groups each: with four, eleven each, a chain was twice as long and a block's registers left
-// two waves per SIMD. Listed rows x 2,816, us with four waves and the input rows behind the weights | so: 512 rows, 1 input row 6.4 | 4.8;
-// 4,099 rows, 1 input row 7.1 | 5.7, 16 input rows 7.4 | 6.2 (both shorter still, below; the vector unit's dot products: 50.8); 32,768 rows 17.7 | 16.8, 19.0 | 17.5.
+// rows is one such chain per compute unit. So eight waves take six groups each: with four, eleven each, a chain was twice as long and
+// a block's registers left two waves per SIMD. Listed rows x 2,816, us with four waves | eight: 512 rows, 1 input row 6.4 | 4.8;
+// 4,099 rows, 1 input row 7.1 | 5.7, 16 input rows 7.4 | 6.2 (all shorter still, below; the vector unit's dot products: 50.8); 32,768 rows 17.7 | 16.8, 19.0 | 17.5.
+// EARLY (but for lists of more than a block per 16 rows with more than four input rows): the input rows are asked for while the ids are on their way, and
+// as soon as those are there the scales and all six groups of weights, in one burst in front of the input rows' turn and sums. Left alone the compiler asks
+// for the weights behind the sums and, ONE, two or three groups at a time where it uses them, each a round trip to memory. us so in front of it | now,
+// of lists that repeat and of rows that no cache holds: 16 rows, 1 input row 3.51 | 3.51 and 4.92 | 4.08, 16 input rows 4.09 | 4.04 and 5.00 | 4.54;
+// 512 rows 3.77 | 3.75 and 5.62 | 4.64, 4.31 | 4.28 and 5.60 | 5.23; 1,408 rows 3.79 | 3.77 and 6.09 | 5.16, 4.37 | 4.37 and 5.95 | 5.71; 4,099 rows 5.00 | 5.11
+// and 7.81 | 7.14, 5.92 | 6.03 and 8.11 | 8.25 (one unit of 256 has two blocks); 8,192 rows 6.08 | 6.02 and 10.68 | 9.97, 6.91 | 6.77 and 11.22 | 10.92; 16,384 rows,
+// 1 input row 11.26 | 10.74 and 17.9 | 17.4. There with 16 input rows, whose 16 segments per request keep the address unit busy, the weights behind the sums
+// are the faster: 11.0 and 19.2, in front of them 11.4 and 19.3.
 // Error of a logit against 64 bits (2-norm): 1.7e-7 in bf16 and 4.9e-6 in FP16, where the dot products have
 // 8.6e-7 and 1.6e-5, and 128 + q / 1024 + q on the matrix unit 1.0e-6 and 1.4e-5.
 constexpr int kListedParts = 8, kListedRing = 6;
 static_assert(kListedParts * kListedRing >= kKSplit * kRing, "every width up to FFMOE_MATRIX_MAX_N");
 // ONE: the launch has a block for every 16 rows, none of which takes others: it asks for no further weights, whose requests (the same rows
-// again) a block would have to wait for before it can end. Listed rows x 2,816, us with the
-// requests | so: 16 rows, 1 input row 4.06 | 3.77, 16 input rows 4.54 | 4.28; 1,408 rows 4.47 | 4.10, 5.03 | 4.71; 4,099 rows 6.0 | 5.24, 6.3 | 6.08; 8,192
-// rows 7.5 | 5.9, 7.4 | 6.75. Beyond, two blocks per compute unit go on to others (8,193 rows 6.75, 7.2: a block in 500 takes a second sixteen).
+// again) a block would have to wait for before it can end. Listed rows x 2,816, us with the requests (and the weights behind the sums) | so, of lists
+// that repeat and of rows that no cache holds: 16 rows, 1 input row 3.67 | 3.51 and 4.81 | 4.08, 16 input rows 4.26 | 4.04 and 5.14 | 4.54; 1,408 rows 4.16 | 3.77 and
+// 6.04 | 5.16, 4.74 | 4.37 and 6.41 | 5.71; 4,099 rows 5.87 | 5.11 and 8.26 | 7.14, 6.11 | 6.03 and 8.33 | 8.25; 8,192 rows 7.78 | 6.02 and 11.61 | 9.97, 7.76 | 6.77
+// and 12.37 | 10.92. Beyond, two blocks per compute unit go on to others.
 template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16, bool FEW, bool ONE>
 __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
                                                                               const uint16_t *__restrict__ biases, const uint16_t *__restrict__ x,
                                                                               void *__restrict__ y_, uint32_t m, uint32_t n_groups, uint32_t rows,
                                                                               uint32_t x_stride, uint32_t y_stride, const uint32_t *__restrict__ ids) {
     constexpr int kSums = FEW ? 1 : 4;
+    constexpr bool EARLY = FEW || ONE;                              // (without a branch from here to the first products)
     __shared__ float s_red[ONE ? 1 : 2][kListedParts][kSums][64];
     const uint32_t lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, jq = lane >> 4;                  // operand layout: row j, quarter jq
@@ -189,19 +198,30 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
         const uint32_t o = min(rb * kTileRows + lrow, m - 1);
         return ids ? ids[o] : o;
     };
-    uint2 wt[kListedRing];
-    uint32_t sb[2];                                                 // scale | bias << 16 of groups g0 + 2 lq + 0 .. 1 of row lrow
+    // As they come from memory: what a word is put together from stays apart until it is used, so that no load waits for one before it.
+    struct Words { uint32_t part[ALIGNED ? 2 : 4]; };               // ALIGNED: two words, else (2-byte alignment is guaranteed) their halves
+    Words wt[kListedRing];
+    uint2 first_sb[2];                                              // scale and bias of groups g0 + 2 lq + 0 .. 1 of row lrow
     auto load_w = [&](uint32_t row, int u) {
         const uint8_t *p = w + row * row_bytes + (size_t)min(g0 + u, g_last) * (kGroup / 2) + 8 * lq;
-        if (ALIGNED) return *reinterpret_cast<const uint2 *>(p);
-        const uint16_t *h = reinterpret_cast<const uint16_t *>(p);  // 2-byte alignment is guaranteed
-        return make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+        Words r;
+        if constexpr (ALIGNED) {
+            const uint2 v = *reinterpret_cast<const uint2 *>(p);
+            r.part[0] = v.x, r.part[1] = v.y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r.part[i] = reinterpret_cast<const uint16_t *>(p)[i];
+        }
+        return r;
     };
+    auto word = [](const Words &r, int i) { return ALIGNED ? r.part[i] : r.part[2 * i % 4] | (r.part[(2 * i + 1) % 4] << 16); };
     auto load_s = [&](uint32_t row, int v) {
         const size_t at = (size_t)row * n_groups + min(g0 + 2 * lq + v, g_last);
-        return (uint32_t)scales[at] | ((uint32_t)biases[at] << 16);
+        return make_uint2(scales[at], biases[at]);
     };
-    uint32_t rb = blockIdx.x;                                       // the grid has at most n_blocks blocks
+    auto pair = [](const uint2 &v) { return v.x | (v.y << 16); };
+    uint32_t rb = blockIdx.x;
+    if (EARLY && rb >= n_blocks) return;                            // (the grid has at most n_blocks blocks: the loop's first turn needs no test)
     uint32_t row = id_of(rb), next_id = ONE ? 0u : id_of(min(rb + gridDim.x, n_blocks - 1));
     // the input rows of this wave's K-slice
     uint4 x0[kListedRing], x1[kListedRing];
@@ -210,16 +230,18 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
         const uint16_t *xrow = x + (size_t)min(my, rows - 1) * x_stride + 16 * quarter;
 #pragma unroll
         for (int u = 0; u < kListedRing; ++u) {
-            const bool live = (uint32_t)u < ng;
             const uint16_t *p = xrow + min(g0 + u, g_last) * kGroup;
-            x0[u] = live ? load_x8<X_ALIGNED>(p) : uint4{0, 0, 0, 0};
-            x1[u] = live ? load_x8<X_ALIGNED>(p + 8) : uint4{0, 0, 0, 0};
+            const bool ask = EARLY || (uint32_t)u < ng;             // (EARLY: past the share its last group again, whose products are left out below)
+            x0[u] = ask ? load_x8<X_ALIGNED>(p) : uint4{0, 0, 0, 0};
+            x1[u] = ask ? load_x8<X_ALIGNED>(p + 8) : uint4{0, 0, 0, 0};
         }
     }
+    if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kListedRing; ++u) wt[u] = load_w(row, u);
 #pragma unroll
-    for (int v = 0; v < 2; ++v) sb[v] = load_s(row, v);
+    for (int v = 0; v < 2; ++v) first_sb[v] = load_s(row, v);
+    if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);
     // ... in operand order, paired like the nibbles, and their sum per group
     f32x4 sx[kListedRing];
     {
@@ -235,6 +257,8 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
             sx[u] = group_input_sum<F16>(x0[u], x1[u]);
         }
     }
+    if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);
+    uint32_t sb[2] = {pair(first_sb[0]), pair(first_sb[1])};
     const int pull = (int)((4 * j + jq) * 4);
     const uint32_t my_row = FEW ? jq : 4 * jq + ks;                 // the input row this lane finishes (waves kSums and up: none)
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -249,10 +273,10 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
 #pragma unroll
         for (int u = 0; u < kListedRing; ++u) {
             uint2 t;
-            t.x = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].x);
-            t.y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)wt[u].y);
+            t.x = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)word(wt[u], 0));
+            t.y = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)word(wt[u], 1));
             uint32_t sc = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((4 * j + u / 2) * 4), (int)sb[u % 2]);
-            if ((uint32_t)u >= ng) sc = 0;
+            if (!EARLY && (uint32_t)u >= ng) sc = 0;
             if constexpr (!ONE) wt[u] = load_w(row, u);             // the next 16 rows (past the last: these again)
             f32x4 acc = Act<F16>::mfma(x0[u], unpack8_fine<F16>(t.x), zero);
             acc = Act<F16>::mfma(x1[u], unpack8_fine<F16>(t.y), acc);
@@ -260,13 +284,13 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
             const float tb = __builtin_fmaf(-FineNibble<F16>::kOffset, s, b);
 #pragma unroll
             for (int r = 0; r < kSums; ++r) {
-                tot[r] = __builtin_fmaf(su, acc[r], tot[r]);
-                tot[r] = __builtin_fmaf(tb, sx[u][r], tot[r]);
+                const float sum = __builtin_fmaf(tb, sx[u][r], __builtin_fmaf(su, acc[r], tot[r]));
+                tot[r] = !EARLY || (uint32_t)u < ng ? sum : tot[r];
             }
         }
         if constexpr (!ONE) {
 #pragma unroll
-            for (int v = 0; v < 2; ++v) sb[v] = load_s(row, v);
+            for (int v = 0; v < 2; ++v) sb[v] = pair(load_s(row, v));
         }
 #pragma unroll
         for (int r = 0; r < kSums; ++r) s_red[buf][ks][r][lane] = tot[r];
