@@ -79,7 +79,8 @@ def test_every_tile_once_whichever_block_takes_it(ctx, torch, m, n, rows):
     q = torch.stack((W & 15, W >> 4), 2).reshape(m, n).double()
     w = q * S.double().repeat_interleave(64, 1) + B.double().repeat_interleave(64, 1)
     ref, spread = x.double() @ w.T, x.double().abs() @ (q * S.double().abs().repeat_interleave(64, 1) + B.double().abs().repeat_interleave(64, 1)).T
-    # fp32 sums of up to 2,816 products in the offset form (128 + q, so some 17 times the products' own magnitude), 2^-24 each
+    # fp32 sums in the offset form: a group's products are of 128 + q, so some 17 times their own magnitude, and are added one after the other at worst: 64
+    # roundings of 2^-24. (What the groups' and the waves' sums add, at most 15 roundings of the sums themselves, is a seventieth of that.)
     assert torch.all((y.double() - ref).abs() <= 17 * 2.0 ** -24 * 64 * spread + 1e-9)
     assert torch.equal(mx.gemv(x), y.to(torch.bfloat16))
     assert torch.equal(mx.greedy(x).long(), y.argmax(1))
@@ -87,6 +88,29 @@ def test_every_tile_once_whichever_block_takes_it(ctx, torch, m, n, rows):
     for lo, hi in ((0, 300), ((m - 300) // 32 * 32, m)):
         part = ctx.matrix(W[lo:hi].contiguous(), S[lo:hi].contiguous(), B[lo:hi].contiguous())
         assert torch.equal(part.gemv(x, f32_out=True), y[:, lo:hi])
+        part.close()
+    mx.close()
+
+
+def test_a_matrix_past_two_gib_of_tiles(ctx, torch):
+    # from 2 GiB on a tile's byte offset has its highest bit set, and the refills behind a block's last tile name it again instead of a place past the end:
+    # the first tiles, those around the 2 GiB and the last, against matrices of their own
+    n, m = 2816, 47_665 * 32 - 27
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    W = torch.randint(0, 256, (m, n // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    S, B = ((torch.randn((m, n // 64), device="cuda", generator=gen) * 0.02).to(torch.bfloat16) for _ in range(2))
+    mx = ctx.matrix(W, S, B, greedy=True)
+    edge = 2 ** 31 // (1024 * (n // 64)) * 32               # the tile row that the 2 GiB fall into
+    parts = [(lo, hi, ctx.matrix(W[lo:hi].contiguous(), S[lo:hi].contiguous(), B[lo:hi].contiguous()))
+             for lo, hi in ((0, 64), (edge - 64, edge + 96), ((m - 64) // 32 * 32, m))]
+    for rows in (1, 4, 5, 16):
+        x = torch.randn((rows, n), device="cuda", generator=gen).to(torch.bfloat16)
+        y = mx.gemv(x, f32_out=True)
+        for lo, hi, part in parts:
+            assert torch.equal(part.gemv(x, f32_out=True), y[:, lo:hi]), (rows, lo)
+        assert torch.equal(mx.gemv(x), y.to(torch.bfloat16))
+        assert torch.equal(mx.greedy(x).long(), y.argmax(1))
+    for _, _, part in parts:
         part.close()
     mx.close()
 
