@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(512, 1) void decode_down_combine_kernel(const uint8
         tot.b = tot.a;
 #pragma unroll
         for (int u = 0; u < kRing; ++u)
-            ring_step<F16>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, rb * ng + min((uint32_t)u, g_last), lane);
+            ring_step<F16, false>(ring, u, (uint32_t)u < ng, x0[u], x1[u], sx[u], tot, src, 0u, lane);      // (one tile row: no refills)
         if (jq == 0) {          // token column 0 sits in the first element of lanes 0..15
             s_row[r][j] = tot.a[0];
             s_row[r][kTileRows + j] = tot.b[0];

@@ -136,3 +136,13 @@ def test_the_listed_gemv_asks_for_its_weights_in_one_burst():
         assert not any("vmcnt" in op for op in front[at[0]:at[-1]]), name
         checked += 1
     assert checked == 36
+
+
+@pytest.mark.skipif(OBJDUMP is None, reason="needs llvm-objdump")
+def test_the_one_row_down_launch_refills_nothing():
+    # A wave of decode_down_combine_kernel walks one tile row: no slot of its ring is wanted twice. A refill named all the same is dropped by
+    # the compiler, but its fences stay and hold the arithmetic of a step in its place, for 218 registers instead of 176. What a wave cannot do
+    # without at once is eleven groups of weights (6 registers) and of its row (8), i.e. 154; 192 leaves room for addresses and sums.
+    for name, code in kernels("decode_down_combine_kernel").items():
+        registers = [int(n) for _, op, _ in code for n in re.findall(r"\bv\[?(?:\d+:)?(\d+)", op)]
+        assert max(registers) < 192, f"{name}: {max(registers) + 1} registers"
