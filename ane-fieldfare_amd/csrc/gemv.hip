@@ -163,22 +163,24 @@ __global__ __launch_bounds__(256) void gemv_int4_kernel(const uint8_t *__restric
 // a block's registers left two waves per SIMD. Listed rows x 2,816, us with four waves | eight: 512 rows, 1 input row 6.4 | 4.8;
 // 4,099 rows, 1 input row 7.1 | 5.7, 16 input rows 7.4 | 6.2 (all shorter still, below; the vector unit's dot products: 50.8); 32,768 rows 17.7 | 16.8, 19.0 | 17.5.
 // EARLY (but for lists of more than a block per 16 rows with more than four input rows): the input rows are asked for while the ids are on their way, and
-// as soon as those are there the scales and all six groups of weights, in one burst in front of the input rows' turn and sums. Left alone the compiler asks
-// for the weights behind the sums and, ONE, two or three groups at a time where it uses them, each a round trip to memory. us so in front of it | now,
-// of lists that repeat and of rows that no cache holds: 16 rows, 1 input row 3.51 | 3.51 and 4.92 | 4.08, 16 input rows 4.09 | 4.04 and 5.00 | 4.54;
-// 512 rows 3.77 | 3.75 and 5.62 | 4.64, 4.31 | 4.28 and 5.60 | 5.23; 1,408 rows 3.79 | 3.77 and 6.09 | 5.16, 4.37 | 4.37 and 5.95 | 5.71; 4,099 rows 5.00 | 5.11
-// and 7.81 | 7.14, 5.92 | 6.03 and 8.11 | 8.25 (one unit of 256 has two blocks); 8,192 rows 6.08 | 6.02 and 10.68 | 9.97, 6.91 | 6.77 and 11.22 | 10.92; 16,384 rows,
-// 1 input row 11.26 | 10.74 and 17.9 | 17.4. There with 16 input rows, whose 16 segments per request keep the address unit busy, the weights behind the sums
-// are the faster: 11.0 and 19.2, in front of them 11.4 and 19.3.
+// the scales and all six groups of weights in one burst: of up to four input rows as soon as the ids are there, of more once the input rows are
+// there too and turned, in front of their sums. (16 segments per request, they would stand behind the weights of the block's earlier waves in the unit's
+// cache, which keeps its order: 16 input rows, weights that no cache holds, us with the turn behind the burst | in front: 512 listed rows 4.45 | 4.28, 1,408 4.76 | 4.57,
+// 4,096 5.09 | 4.79, 4,099 6.50 | 6.32, 8,192 7.70 | 7.25. With up to four it is 4.36 behind and 4.42 in front at 1,408.) Left alone the compiler asks for
+// the weights behind the sums and, ONE, two or three groups at a time where it uses them, each a round trip to memory. Us of the call so | now,
+// of lists that repeat and of rows that no cache holds: 512 rows, 4 input rows 4.24 | 4.20 and 4.65 | 4.27, 16 input rows 4.40 | 4.22 and 4.86 | 4.28;
+// 1,408 rows 4.25 | 4.15 and 5.22 | 4.28, 4.42 | 4.22 and 5.26 | 4.57; 4,096 rows 4.17 | 4.15 and 5.47 | 4.55, 4.63 | 4.25 and 5.42 | 4.79. Where units have two
+// blocks, 4,099 rows (one unit) 4.68 | 4.93 and 5.83 | 5.48, 5.66 | 5.65 and 6.16 | 6.33, 5,120 rows 5.09 | 5.32 and 6.77 | 6.23, 6.08 | 6.07 and 6.95 | 6.95, 8,192
+// rows 5.43 | 5.38 and 7.05 | 6.53, 6.29 | 6.13 and 8.08 | 7.25. More than a block per 16 rows: 16,384 rows, 4 input rows 9.80 | 9.43 and 11.19 | 11.06, 32,768 rows 14.80 | 14.95 and
+// 17.67 | 17.17; with 16 input rows the weights behind the sums are the faster: 9.6 and 12.0, in front of them 10.1 and 12.6.
 // Error of a logit against 64 bits (2-norm): 1.7e-7 in bf16 and 4.9e-6 in FP16, where the dot products have
 // 8.6e-7 and 1.6e-5, and 128 + q / 1024 + q on the matrix unit 1.0e-6 and 1.4e-5.
 constexpr int kListedParts = 8, kListedRing = 6;
 static_assert(kListedParts * kListedRing >= kKSplit * kRing, "every width up to FFMOE_MATRIX_MAX_N");
 // ONE: the launch has a block for every 16 rows, none of which takes others: it asks for no further weights, whose requests (the same rows
-// again) a block would have to wait for before it can end. Listed rows x 2,816, us with the requests (and the weights behind the sums) | so, of lists
-// that repeat and of rows that no cache holds: 16 rows, 1 input row 3.67 | 3.51 and 4.81 | 4.08, 16 input rows 4.26 | 4.04 and 5.14 | 4.54; 1,408 rows 4.16 | 3.77 and
-// 6.04 | 5.16, 4.74 | 4.37 and 6.41 | 5.71; 4,099 rows 5.87 | 5.11 and 8.26 | 7.14, 6.11 | 6.03 and 8.33 | 8.25; 8,192 rows 7.78 | 6.02 and 11.61 | 9.97, 7.76 | 6.77
-// and 12.37 | 10.92. Beyond, two blocks per compute unit go on to others.
+// again) a block would have to wait for before it can end. Us of the call with the requests (and the weights behind the sums) | so, of lists that repeat and of
+// rows that no cache holds: 1,408 rows, 4 input rows 4.32 | 4.15 and 5.18 | 4.28, 16 input rows 4.75 | 4.22 and 5.49 | 4.57; 4,099 rows 5.68 | 4.93 and 6.25 | 5.48,
+// 5.91 | 5.65 and 6.29 | 6.33; 8,192 rows 7.10 | 5.38 and 8.20 | 6.53, 7.09 | 6.13 and 8.95 | 7.25. Beyond, two blocks per compute unit go on to others.
 template <bool ALIGNED, bool X_ALIGNED, bool Y_F32, bool F16, bool FEW, bool ONE>
 __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(const uint8_t *__restrict__ w, const uint16_t *__restrict__ scales,
                                                                               const uint16_t *__restrict__ biases, const uint16_t *__restrict__ x,
@@ -237,15 +239,16 @@ __global__ __launch_bounds__(64 * kListedParts, 4) void gemv_int4_mfma_kernel(co
         }
     }
     if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!FEW) turn_token_rows(lane, x0, x1);              // ... in operand order
+    if constexpr (!FEW && EARLY) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < kListedRing; ++u) wt[u] = load_w(row, u);
 #pragma unroll
     for (int v = 0; v < 2; ++v) first_sb[v] = load_s(row, v);
     if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);
-    // ... in operand order, paired like the nibbles, and their sum per group
+    // ... paired like the nibbles, and their sum per group
     f32x4 sx[kListedRing];
     {
-        if constexpr (!FEW) turn_token_rows(lane, x0, x1);
         auto paired = [](const uint4 &d) {
             return uint4{(d.x & 0xFFFFu) | (d.z << 16), (d.x >> 16) | (d.z & 0xFFFF0000u),
                          (d.y & 0xFFFFu) | (d.w << 16), (d.y >> 16) | (d.w & 0xFFFF0000u)};

@@ -123,7 +123,7 @@ def test_the_streaming_products_barriers_cover_the_rows_that_are_read_next():
 @pytest.mark.skipif(OBJDUMP is None, reason="needs llvm-objdump")
 def test_the_listed_gemv_asks_for_its_weights_in_one_burst():
     # gemv_int4_mfma_kernel<.., FEW, ONE>, but for the form of neither: six groups of weights and two scales and biases, none of which waits for another or
-    # for the input rows' products
+    # for the input rows' products. Of more than four input rows (not FEW) the burst stands behind the turn of all twelve pieces of 16 bytes.
     checked = 0
     for name, code in kernels("gemv_int4_mfma_kernel").items():
         few, one = re.search(r"ILb[01]ELb[01]ELb[01]ELb[01]ELb([01])ELb([01])E", name).groups()
@@ -134,6 +134,7 @@ def test_the_listed_gemv_asks_for_its_weights_in_one_burst():
         at = [i for i, op in enumerate(front) if re.match(r"global_load_(dwordx2|ushort) ", op)]
         assert len(at) == 10, f"{name}: {len(at)} of 10 requests in front of the first product"
         assert not any("vmcnt" in op for op in front[at[0]:at[-1]]), name
+        assert sum(op.startswith("ds_bpermute") for op in front[:at[0]]) == (0 if few == "1" else 48), name
         checked += 1
     assert checked == 36
 
