@@ -913,8 +913,8 @@ hipError_t launch_gelu_mul(hipStream_t s, const uint16_t *gate, uint32_t gate_st
 // copy, so that tied embeddings need no second table. One thread per two words of a tile that lie together
 // (lane 16 (k / 8 % 4) + row % 16, words 2 (row / 16 % 2) + (k / 32 % 2)), i.e. elements 8 jq ... + 7 of a group's halves, and the
 // row's scale pair. What bounds it is the memory's rate in requests: a row's 32 bytes per group lie in four lines and its scales in a
-// fifth. A thread per word asks for twice the requests and scale pairs of the same lines: 262,144 x 2,816, random ids, us so |
-// now: 301 rows 5.3 | 5.05, 3,072 rows 20.7 | 19.8, 8,192 rows 49.1 | 44.8; 1 row 1.8 and 5 FP16 rows 2.55 either way. An id past the
+// fifth. A thread per word asks for twice the requests and scale pairs of the same lines: 262,144 x 2,816, random ids of two tables in turn, us of
+// a call so | now: 1,000 rows 6.9 | 6.3, 3,072 rows 18.35 | 17.4, 8,192 rows 46.3 | 41.7; up to 301 rows 3.4 either way. An id past the
 // table gives a row of zeros.
 template <bool F16>
 __global__ __launch_bounds__(256) void matrix_rows_kernel(const uint8_t *__restrict__ tiles, const uint8_t *__restrict__ scales,

@@ -87,12 +87,14 @@ __device__ __forceinline__ f32x4 group_input_sum(const uint4 &x0, const uint4 &x
 // that refills the slot (REFILL = false: a wave that walks one tile row only has nothing to refill).
 // SUMS: of the lane's four results, how many are kept up.
 // PIN: the refill stands behind the unpacking of its slot, and nowhere else. Left alone the compiler collects the refills of a whole tile row at its
-// end and waits for nearly all of them at the next one's start, so that a wave has its twelve KiB in flight a part of the time only: 262,144 x
-// 2,816, greedy with confidence, 16 rows 76.6 us, now 73.0; fp32 logits of 1 row 67.1 | 62.6, of 16 rows 82.5 | 76.2; verify block of 16 rows 48.6 | 47.9,
-// layer block of 1 row 28.4 | 28.1, of 5 FP16 rows 42.8 | 42.2. Not for a wave of one tile row, whose rows and weights
-// are better asked for as the compiler has it (skinny_down_lds: 5.9 us at 1 row, pinned 6.2 to 6.5). The last tile row's refills come with
-// no_lane (asked for once more, its tiles are the launch's last requests: layer block of 1 row 28.65); written as steps without a refill, behind a
-// branch, the compiler keeps both rows' operands and spills.
+// end and waits for nearly all of them at the next one's start, so that a wave has its twelve KiB in flight a part of the time only. Us of a call as the compiler
+// has it | pinned, both builds in turn, weights of two heads or three layers in turn: 262,144 x 2,816, greedy with confidence, 16 rows 73.3 | 71.3; fp32 logits of
+// 1 row 64.2 | 60.8, of 16 rows 75.1 | 71.0; verify block of 16 rows 46.4 | 45.2, layer block of 1 row 28.9 | 28.3, of 5 FP16 rows 43.5 | 43.3 (three runs of a side
+// differ by 0.1, the heads' by 0.5); a dense FFN with skinny_down_ksplit_persistent alone changed, 48 layers in turn, 2,816 -> 2,112, 1 row 11.76 | 11.57,
+// 16 rows 12.67 | 12.55, 2,816 -> 2,816, 1 row 12.12 | 11.86. Not for a wave of one tile row, whose rows and weights are better asked for as the compiler has it
+// (skinny_down_lds: 5.9 us at 1 row, pinned 6.2 to 6.5) or which refills nothing (decode_down_combine_kernel: REFILL = false). The last tile row's refills come with
+// no_lane (asked for once more, its tiles are the launch's last requests: layer block of 1 row 28.7 | 28.3, a sampled head's row 74.9 | 73.0); written as steps
+// without a refill, behind a branch, the compiler keeps both rows' operands and spills.
 template <bool F16 = false, bool REFILL = true, int SUMS = 4, bool ONCE = false, bool PIN = REFILL>
 __device__ __forceinline__ void ring_step(WeightRing &ring, int u, bool live, const uint4 &x0, const uint4 &x1,
                                           const f32x4 &sx, TwoStreamAcc &tot, const TileSource &src,
